@@ -113,6 +113,25 @@ def test_linear(M, N, K, dtype):
     _close(out_s, wide[:, :K].double().cpu() @ w.double().T, 2e-6 if dtype == torch.float32 else 2e-5, "strided")
 
 
+@pytest.mark.parametrize("N,K", [(48, 16), (33, 7), (100, 260), (304, 2047), (2050, 520), (4096, 288), (16, 2304)])
+def test_linear_f32_rows_do_not_depend_on_their_number(N, K):
+    """float32: few rows on the streaming kernel, more on tiles of every size, K in parts, with remainders and without 16-byte
+    rows.  Every launch gives a row the same bits, and the sum of K products of float32 stays within K / 8 + 8 roundings of
+    terms of their root mean square."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(N + K)
+    M = 3100 if N < 64 or N >= 2048 else 700
+    x = torch.randn(M, K + 4, generator=g).to(DEV)[:, :K]
+    w = torch.randn(N, K, generator=g).to(DEV)
+    ref = x.double() @ w.double().T
+    whole = ops.linear(x, w)
+    bound = 2.0 ** -24 * (K / 8 + 8) * math.sqrt(K)
+    assert float((whole.double() - ref).abs().max()) < max(bound, 2.0 ** -22 * math.sqrt(K) * 4)
+    for m in (1, 2, 16, 17, 33, 64, 65, 97, 130, 260, 515, M):
+        if m <= M:
+            assert torch.equal(ops.linear(x[:m], w), whole[:m]), m
+
+
 @pytest.mark.parametrize("M,N,K", [(16, 33000, 2560), (10, 40000, 4096), (3, 33000, 512)])
 def test_linear_very_wide(M, N, K):
     """An output head's shape: thousands of groups of 16 columns; with many rows and a long K a block
