@@ -910,6 +910,43 @@ def test_attention_mfma_prompt_portions_and_mixed(nq, nkv, d, ps, window):
     _close(gen.reshape(T, nq, d), ref, ATTN_TOL, "generic attention on the same step")
 
 
+@pytest.mark.parametrize("cols", [None, 16, 128])
+@pytest.mark.parametrize("entries", [[(0, 37), (50, 13), (129, 1), (0, 1), (63, 2), (7, 170)], [(0, 1), (31, 1), (32, 1), (700, 1)]])
+@pytest.mark.parametrize("nq,nkv,d,ps,window,cap,sink", [
+    (4, 2, 16, 16, 0, 0, False), (8, 2, 32, 8, 24, 0, True), (6, 3, 48, 8, 0, 5.0, False), (32, 8, 128, 16, 0, 0, False),
+    (5, 5, 80, 32, 33, 0, False), (16, 8, 64, 4, 40, 0, True), (40, 2, 96, 8, 0, 0, False), (4, 1, 192, 16, 0, 0, True),
+    (20, 1, 256, 64, 70, 3.0, False)])
+def test_attention_f32(nq, nkv, d, ps, window, cap, sink, entries, cols):
+    """The matrix-core kernel in float32 against float64 softmaxes and the general kernel: prompts, portions behind a cached prefix,
+    single tokens (alone, and beside portions), every place that no token sees holding NaN.  A score of unit-variance rows is
+    a sum of d products and the output one of n weighted values: 4e-6 of the largest value covers both kernels."""
+    ops = _ops()
+    if cols == 128 and (d > 128 or all(n == 1 for _, n in entries)):
+        pytest.skip("no such block")
+    batch, kv, ks, vs, positions, token_req = _fake_step(entries, ps, nkv, d, torch.float32, seed=nq + d)
+    T = batch.num_tokens
+    held = torch.zeros(kv.k_cache.shape[0], ps, dtype=torch.bool)
+    for r, (P, n) in enumerate(entries):
+        for j in range(max(0, P - window + 1) if window else 0, P + n):
+            held[int(kv.block_tables[r, j // ps]), j % ps] = True
+    kv.k_cache.masked_fill_(~held[:, None, :, None].to(DEV), float("nan"))
+    kv.v_cache.masked_fill_(~held[:, None, None, :].to(DEV), float("nan"))
+    g = torch.Generator().manual_seed(2)
+    wide = torch.zeros(T, nq * d + 2 * nkv * d)
+    q = torch.randn(T, nq, d, generator=g)
+    wide[:, :nq * d] = q.reshape(T, nq * d)
+    sinks = torch.randn(nq, generator=g).to(DEV) if sink else None
+    scale = 1 / math.sqrt(d)
+    out = ops.attention_f32(wide.to(DEV), nq, nkv, d, kv, batch, window, scale, sinks, cap, cols=cols)
+    gen = ops.attention_generic(wide.to(DEV), nq, nkv, d, kv.k_cache, kv.v_cache, kv.block_tables, batch.token_req,
+                                batch.positions, window, scale, sinks=sinks, softcap=cap)
+    _close(out, gen.double(), 4e-6, "against the general kernel")
+    if not cap and not sink:
+        for r in range(len(entries)):
+            sel = (token_req == r).nonzero().flatten()
+            _close(out.reshape(T, nq, d)[sel], _attn_ref(q[sel], ks[r], vs[r], positions[sel], window, scale), 4e-6, f"row {r}")
+
+
 @pytest.mark.parametrize("bins,groups", [(None, None), (3, 2), (1, 2), (None, 1), (3, 1), (1, 1)])
 @pytest.mark.parametrize("nq,nkv,d,ps,window", [
     (32, 8, 128, 16, 0), (8, 2, 32, 8, 300), (6, 3, 48, 8, 0), (5, 1, 128, 32, 0), (40, 2, 96, 8, 77),

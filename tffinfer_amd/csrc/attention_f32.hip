@@ -1,0 +1,251 @@
+// Attention over the paged cache in float32 on the float32 matrix cores (v_mfma_f32_16x16x4_f32), for head sizes that
+// are multiples of 16 up to 128, 192 and 256, and pages of a power of two of at least four tokens: the path of the
+// 32-bit model.  Other sizes, and keys of blocks before a window, run on the general kernel (attention_generic.hip).
+//
+// A column is a (token, q head of the kv head's group) pair of one request, numbered token * G + head.  A wave takes
+// 16 NC columns; per step of 32 keys
+//   S^T = K Q^T      lane (column = l % 16, g = l / 16) gets the scores of keys 4 g .. 4 g + 3 of sixteen;
+//   softmax          running maximum m and sum l per column (two lane swaps a step), scores scaled after the product,
+//                    capped (c tanh(s / c)) if a cap is given, then masked: lo <= key <= position;
+//   O^T += V^T P^T   the probabilities lie in the registers as the MFMA wants them, the values come transposed from
+//                    their page, [element][slot]: four keys of an element are one 16-byte load.
+// Keys and values go from memory straight into the MFMA operands.  WK waves of a block share the columns' keys (step by
+// step in turn) and merge through LDS at the end, so that short prompts and decode steps fill the chip; WQ waves with
+// neighbouring columns walk the same keys, so that the CU's cache serves them.  With sinks, e^(sink - m) is one more
+// term of the denominator.
+// What bounds it: the matrix cores and the operands' way from L2 for prompts (2,048 tokens of 32 heads of 128 on 8 kv heads
+// 434 us = 79 TFLOP/s; the general kernel, a wave a token and head on the vector units, 43,960 us), the chain of a step for
+// few keys (two requests of 400 tokens decoding 18 us, 207 before; 401 + 230 tokens of 16 heads 29 us, 1,193 before).
+#include "common.h"
+#include "tffinfer_kernels.h"
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float af_floatx4;
+
+__device__ __forceinline__ af_floatx4 af_mfma16(const float4& a, const float4& b, af_floatx4 c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
+}
+
+template <int DF, int NC, int WQ, int WK>
+__global__ __launch_bounds__(64 * WQ * WK, 2) void attention_f32_kernel(
+    const float* __restrict__ q, int q_stride, float* __restrict__ out, const float* __restrict__ k_cache,
+    const float* __restrict__ v_cache, const int32_t* __restrict__ block_tables, int bt_stride,
+    const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ start_pos, const int32_t* __restrict__ work, int items,
+    int tiles, int nq, int nkv, int ps_shift, int window, float scale, const float* __restrict__ sinks, float softcap) {
+    constexpr int D = 16 * DF;
+    __shared__ af_floatx4 red_o[WK > 1 ? WQ * WK * NC * DF : 1][64];
+    __shared__ float red_ml[WK > 1 ? WQ * WK * NC : 1][2][16];
+    // heads fastest: the blocks of one kv head meet on one XCD when there are eight; the last columns, which see most
+    // keys, first
+    const int g_kv = blockIdx.x % nkv, item = items - 1 - (int)(blockIdx.x / nkv);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, wq = wv / WK, wk = wv % WK, r = lane & 15, g = lane >> 4;
+    const int G = nq / nkv, ps = 1 << ps_shift;
+    const int row = work ? work[2 * item] : item / tiles;
+    const int c0 = (work ? work[2 * item + 1] : item % tiles * (16 * NC * WQ)) + wq * 16 * NC;
+    const int t0 = cu_tokens[row], ncol = (cu_tokens[row + 1] - t0) * G, p0 = start_pos[row];
+    if (ncol <= 0) return;                                // (the whole block: a row without tokens)
+    const int32_t* bt = block_tables + (size_t)row * bt_stride;
+    const bool any = c0 < ncol;
+    // the wave's columns; those past the last one repeat it
+    int pos[NC], lo[NC];
+    size_t place[NC];
+    float4 qf[NC][DF];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int col = min(c0 + c * 16 + r, ncol - 1);
+        const int tok = col / G, head = g_kv * G + col - tok * G;
+        pos[c] = p0 + tok;
+        lo[c] = window > 0 ? max(0, pos[c] - window + 1) : 0;
+        place[c] = (size_t)(t0 + tok) * nq * D + (size_t)head * D;
+        const float* qp = q + (size_t)(t0 + tok) * q_stride + (size_t)head * D + 4 * g;
+#pragma unroll
+        for (int s = 0; s < DF; ++s) qf[c][s] = *reinterpret_cast<const float4*>(qp + 16 * s);
+    }
+    const int first_pos = p0 + c0 / G, last_pos = p0 + (min(c0 + 16 * NC, ncol) - 1) / G;
+    const int lo_min = window > 0 ? max(0, first_pos - window + 1) : 0;
+    const int lo_max = window > 0 ? max(0, last_pos - window + 1) : 0;
+    float m[NC], l[NC];
+    af_floatx4 o[NC][DF];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        m[c] = -INFINITY;
+        l[c] = 0.f;
+#pragma unroll
+        for (int s = 0; s < DF; ++s) o[c][s] = af_floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (any) {
+        for (int k = (lo_min & ~31) + 32 * wk; k <= last_pos; k += 32 * WK) {
+            af_floatx4 sc[NC][2];
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                const int key = min(k + 16 * f + r, last_pos);       // (never past what the request holds)
+                const float* kp = k_cache + (((size_t)bt[key >> ps_shift] * nkv + g_kv) * ps + (key & (ps - 1))) * D + 4 * g;
+                float4 kf[DF];
+#pragma unroll
+                for (int s = 0; s < DF; ++s) kf[s] = *reinterpret_cast<const float4*>(kp + 16 * s);
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    sc[c][f] = af_floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int s = 0; s < DF; ++s) sc[c][f] = af_mfma16(kf[s], qf[c][s], sc[c][f]);
+                }
+            }
+            const bool edge = k < lo_max || k + 31 > first_pos;       // some column does not see all of the step
+            float4 p[NC][2];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                float s[8], mx = -INFINITY;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    s[i] = sc[c][i >> 2][i & 3] * scale;
+                    if (softcap > 0.f) s[i] = softcap * tanhf(s[i] / softcap);
+                    if (edge) {
+                        const int key = k + 16 * (i >> 2) + 4 * g + (i & 3);
+                        if (key < lo[c] || key > pos[c]) s[i] = -INFINITY;
+                    }
+                    mx = fmaxf(mx, s[i]);
+                }
+                const float m_new = fmaxf(m[c], rows_max(mx));
+                const float ref = m_new == -INFINITY ? 0.f : m_new;   // (a column that has seen no key yet)
+                const float corr = expf(m[c] - ref);
+                m[c] = m_new;
+                float sum = 0.f, e[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    e[i] = expf(s[i] - ref);
+                    sum += e[i];
+                }
+                l[c] = l[c] * corr + sum;            // (the four lanes of a column add their parts at the end)
+#pragma unroll
+                for (int x = 0; x < DF; ++x) o[c][x] = o[c][x] * corr;
+                p[c][0] = make_float4(e[0], e[1], e[2], e[3]);
+                p[c][1] = make_float4(e[4], e[5], e[6], e[7]);
+            }
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                const int quad = k + 16 * f + 4 * g, key = min(quad, last_pos & ~3);
+                const float* vp = v_cache + ((size_t)bt[key >> ps_shift] * nkv + g_kv) * ps * D + (key & (ps - 1)) + (size_t)r * ps;
+                float4 vf[DF];
+#pragma unroll
+                for (int s = 0; s < DF; ++s) vf[s] = *reinterpret_cast<const float4*>(vp + (size_t)16 * s * ps);
+                if (edge) {      // slots that hold nothing of the request's may hold anything: 0 x NaN is not 0
+#pragma unroll
+                    for (int s = 0; s < DF; ++s) {
+                        vf[s].x = quad + 0 >= lo_min && quad + 0 <= last_pos ? vf[s].x : 0.f;
+                        vf[s].y = quad + 1 >= lo_min && quad + 1 <= last_pos ? vf[s].y : 0.f;
+                        vf[s].z = quad + 2 >= lo_min && quad + 2 <= last_pos ? vf[s].z : 0.f;
+                        vf[s].w = quad + 3 >= lo_min && quad + 3 <= last_pos ? vf[s].w : 0.f;
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+#pragma unroll
+                    for (int s = 0; s < DF; ++s) o[c][s] = af_mfma16(vf[s], p[c][f], o[c][s]);
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) l[c] = rows_sum(l[c]);
+    if (WK > 1) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if (g == 0) {
+                red_ml[wv * NC + c][0][r] = m[c];
+                red_ml[wv * NC + c][1][r] = l[c];
+            }
+#pragma unroll
+            for (int s = 0; s < DF; ++s) red_o[(wv * NC + c) * DF + s][lane] = o[c][s];
+        }
+        __syncthreads();
+        if (!any) return;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            float mm = -INFINITY, ll = 0.f, f[WK];
+#pragma unroll
+            for (int w = 0; w < WK; ++w) mm = fmaxf(mm, red_ml[(wq * WK + w) * NC + c][0][r]);
+#pragma unroll
+            for (int w = 0; w < WK; ++w) {
+                f[w] = expf(red_ml[(wq * WK + w) * NC + c][0][r] - mm);       // (some wave has seen the column's own key)
+                ll = fmaf(f[w], red_ml[(wq * WK + w) * NC + c][1][r], ll);
+            }
+            const int col = c0 + c * 16 + r;
+            if (sinks && col < ncol) ll += expf(sinks[g_kv * G + col % G] - mm);
+            const float inv = 1.0f / ll;
+            for (int s = wk; s < DF; s += WK) {
+                af_floatx4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int w = 0; w < WK; ++w) t = t + red_o[((wq * WK + w) * NC + c) * DF + s][lane] * f[w];
+                t = t * inv;
+                if (col < ncol) *reinterpret_cast<float4*>(out + place[c] + 16 * s + 4 * g) = make_float4(t[0], t[1], t[2], t[3]);
+            }
+        }
+        return;
+    }
+    if (!any) return;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int col = c0 + c * 16 + r;
+        if (col >= ncol) continue;
+        float ll = l[c];
+        if (sinks) ll += expf(sinks[g_kv * G + col % G] - m[c]);
+        const float inv = 1.0f / ll;
+#pragma unroll
+        for (int s = 0; s < DF; ++s) {
+            const af_floatx4 t = o[c][s] * inv;
+            *reinterpret_cast<float4*>(out + place[c] + 16 * s + 4 * g) = make_float4(t[0], t[1], t[2], t[3]);
+        }
+    }
+}
+
+TFF_API int tff_attention_f32_supported(int d, int page_size) {
+    const bool size = (d > 0 && d <= 128 && d % 16 == 0) || d == 192 || d == 256;
+    return size && page_size >= 4 && (page_size & (page_size - 1)) == 0;
+}
+
+// work: int32 [items, 2] (row, first column) of tiles of `cols` columns, or null: every row has `tiles` tiles from column
+// 0 on, items = rows * tiles.  cols 16: 4 waves share a tile's keys (8 with `alone`, for steps of one token a request);
+// 128: 4 waves of 32 columns each.
+TFF_API int tff_attention_f32(const void* q, int q_stride, void* out, const void* k_cache, const void* v_cache,
+                              const int32_t* block_tables, int bt_stride, const int32_t* cu_tokens, const int32_t* start_pos,
+                              const int32_t* work, int items, int tiles, int cols, int alone, int nq, int nkv, int d, int page_size,
+                              int num_pages, int window, float scale, const float* sinks, float softcap, tff_stream_t stream) {
+    TFF_REQUIRE(q && out && k_cache && v_cache && block_tables && cu_tokens && start_pos, "attention_f32: null pointer");
+    TFF_REQUIRE(tff_attention_f32_supported(d, page_size), "attention_f32: head size %d on pages of %d tokens", d, page_size);
+    TFF_REQUIRE(nq > 0 && nkv > 0 && nq % nkv == 0, "attention_f32: %d query heads are not a multiple of %d key heads", nq, nkv);
+    TFF_REQUIRE(num_pages > 0 && bt_stride > 0 && window >= 0 && q_stride >= nq * d && q_stride % 4 == 0,
+                "attention_f32: bad geometry pages=%d table stride=%d window=%d query rows of %d", num_pages, bt_stride, window, q_stride);
+    TFF_REQUIRE(((uintptr_t)q % 16) == 0 && ((uintptr_t)out % 16) == 0 && ((uintptr_t)k_cache % 16) == 0 &&
+                ((uintptr_t)v_cache % 16) == 0, "attention_f32: operands must be 16-byte aligned");
+    TFF_REQUIRE(items >= 0 && (work || tiles > 0) && (long)items * nkv < (1L << 31), "attention_f32: bad work");
+    TFF_REQUIRE(cols == 16 || (cols == 128 && work && d <= 128), "attention_f32: tiles of %d columns of %d", cols, d);
+    if (items == 0) return 0;
+    hipStream_t s = (hipStream_t)stream;
+    const int shift = __builtin_ctz(page_size);
+#define AF_LAUNCH(DF, NC, WQ, WK)                                                                                          \
+    attention_f32_kernel<DF, NC, WQ, WK><<<items * nkv, 64 * WQ * WK, 0, s>>>(                                             \
+        (const float*)q, q_stride, (float*)out, (const float*)k_cache, (const float*)v_cache, block_tables, bt_stride,      \
+        cu_tokens, start_pos, work, items, tiles, nq, nkv, shift, window, scale, sinks, softcap)
+#define AF_SIZE(DF)                                  \
+    case DF:                                         \
+        if (cols == 128) AF_LAUNCH(DF, 2, 4, 1);     \
+        else if (alone) AF_LAUNCH(DF, 1, 1, 8);      \
+        else AF_LAUNCH(DF, 1, 1, 4);                 \
+        break
+    switch (d / 16) {
+        AF_SIZE(1);
+        AF_SIZE(2);
+        AF_SIZE(3);
+        AF_SIZE(4);
+        AF_SIZE(5);
+        AF_SIZE(6);
+        AF_SIZE(7);
+        AF_SIZE(8);
+        case 12: AF_LAUNCH(12, 1, 1, 4); break;
+        default: AF_LAUNCH(16, 1, 1, 4); break;
+    }
+#undef AF_SIZE
+#undef AF_LAUNCH
+    return tff_check_launch("attention_f32");
+}

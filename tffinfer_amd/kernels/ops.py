@@ -529,6 +529,59 @@ def attention_generic(q: torch.Tensor, nq: int, nkv: int, d: int, k_cache: torch
     return out
 
 
+def attention_f32_supported(q: torch.Tensor, d: int, page_size: int) -> bool:
+    return (q.dtype == torch.float32 and q.data_ptr() % 16 == 0 and q.stride(0) % 4 == 0
+            and bool(_lib.load().tff_attention_f32_supported(int(d), int(page_size))))
+
+
+#: tiles of 16 columns x kv heads from which prompts take blocks of 128 columns (four waves that walk the same keys,
+#: two column tiles each) instead of blocks of 16 whose four waves share the keys: 4,096 tokens of 32 heads on 8 (8,192 tiles)
+#: 1,477 against 1,600 us, 2,048 tokens (4,096 tiles) 522 against 434
+F32_WIDE_TILES = 8192
+
+
+def attention_f32(q: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, window: int = 0, scale: float | None = None,
+                  sinks: torch.Tensor | None = None, softcap: float = 0.0, cols: int | None = None) -> torch.Tensor:
+    """float32 attention of the step's tokens on the float32 matrix cores; ``cols`` overrides the columns of a
+    block (16 or 128).  Otherwise as :func:`paged_attention`."""
+    _req(q, "attention q", torch.float32, 2)
+    T = q.shape[0]
+    if q.shape[1] < nq * d:
+        raise _lib.KernelError(f"attention q: rows of {q.shape[1]} hold fewer than nq*d = {nq * d}")
+    k_cache, v_cache = kv.k_cache, kv.v_cache
+    _req(k_cache, "k cache", q.dtype, 4)
+    _req(v_cache, "v cache", q.dtype, 4)
+    _check_cache(k_cache, v_cache, nkv, d, "attention")
+    bt = _req(kv.block_tables, "block tables", torch.int32, 2)
+    _req(batch.cu_tokens, "cu_tokens", torch.int32, 1)
+    _req(batch.start_pos, "start_pos", torch.int32, 1)
+    R = batch.num_reqs
+    if batch.cu_tokens.numel() != R + 1 or batch.start_pos.numel() != R or bt.shape[0] != R:
+        raise _lib.KernelError("attention: the step's tables do not describe the same number of requests")
+    if batch.num_tokens != T:
+        raise _lib.KernelError(f"attention: {T} query rows for a step of {batch.num_tokens} tokens")
+    _check_sinks(sinks, nq)
+    G = nq // nkv
+    if scale is None:
+        scale = 1.0 / math.sqrt(d)
+    out = torch.empty(T, nq * d, dtype=q.dtype, device=q.device)
+    work, tiles, alone = None, -(-G // 16), batch.max_new_tokens == 1
+    if alone:
+        items, cols = R * tiles, 16        # (no list: sizes come from the tables, a captured step serves any requests)
+    else:
+        if cols is None:
+            cu = batch.host_cu_tokens
+            count = sum(-(-(b - a) * G // 16) for a, b in zip(cu, cu[1:])) * nkv
+            cols = 128 if d <= 128 and count >= F32_WIDE_TILES else 16
+        work = _attention_work(batch, G, cols, q.device)
+        items = work.shape[0]
+    _lib.check(_lib.load().tff_attention_f32(
+        q.data_ptr(), q.stride(0), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), bt.data_ptr(), bt.stride(0),
+        batch.cu_tokens.data_ptr(), batch.start_pos.data_ptr(), _ptr(work), items, tiles, cols, 1 if alone else 0, nq, nkv, d,
+        k_cache.shape[2], k_cache.shape[0], int(window), float(scale), _ptr(sinks), float(softcap or 0.0), _stream()))
+    return out
+
+
 def _pool_table(kv, pool: int, window: int) -> torch.Tensor | None:
     """The step's table of the pages that hold the mean keys of blocks of ``pool`` tokens."""
     if not pool:
@@ -964,9 +1017,9 @@ def paged_attention(q: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, windo
                     scale: float | None = None, sinks: torch.Tensor | None = None,
                     softcap: float = 0.0, pool: int = 0) -> torch.Tensor:
     """Attention of a step's tokens over the cache view ``kv`` (k_cache,
-    v_cache, block_tables) with the step's ``batch``.  bfloat16 with a head
-    size the matrix-core kernel takes runs there; everything else (float32,
-    other head sizes) on the general kernel.  ``sinks`` (float32 [nq]): a
+    v_cache, block_tables) with the step's ``batch``.  A head size and page that
+    the matrix-core kernels (bfloat16, float32) take runs there; everything else
+    on the general kernel.  ``sinks`` (float32 [nq]): a
     number per query head whose exponential is one more term of the softmax's
     denominator, with no key and no value, not scaled.  ``softcap`` c > 0: the
     scaled scores are capped, s <- c tanh(s / c), before the mask.  ``pool`` P > 0 (with a window):
@@ -975,6 +1028,8 @@ def paged_attention(q: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, windo
     # (the matrix-core kernels cap scores at head sizes up to 192)
     if mfma_attention_supported(q.dtype, d, kv.k_cache.shape[2]) and not (softcap and d > 192):
         return attention_mfma(q, nq, nkv, d, kv, batch, window, scale, sinks=sinks, softcap=softcap, pool=pool)
+    if not pool and attention_f32_supported(q, d, kv.k_cache.shape[2]):
+        return attention_f32(q, nq, nkv, d, kv, batch, window, scale, sinks=sinks, softcap=softcap)
     return attention_generic(q, nq, nkv, d, kv.k_cache, kv.v_cache, kv.block_tables,
                              batch.token_req, batch.positions, window, scale, sinks=sinks, softcap=softcap, pool=pool,
                              pool_tables=_pool_table(kv, pool, int(window)))
@@ -2251,6 +2306,7 @@ OP_TABLE = {
     "qk_norm_rope_kv": qk_norm_rope_kv,
     "attention": paged_attention,
     "attention_generic": attention_generic,
+    "attention_f32": attention_f32,
     "attention_mfma": attention_mfma,
     "attention_decode_fused": attention_decode_fused,
     "qkv_attention": qkv_attention,
