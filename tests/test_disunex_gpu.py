@@ -121,6 +121,41 @@ def test_experts(dtype, E, top, width, ff, limit, T):
         assert torch.equal(alone[0], tiles[7])
 
 
+@pytest.mark.parametrize("T", [33, 300, 1700])
+@pytest.mark.parametrize("E,top,width,ff,gate,on_input,pad", [
+    (3, 1, 64, 64, True, False, 0), (5, 2, 192, 320, True, True, 64), (4, 2, 1216, 64, False, False, 8), (9, 4, 320, 448, False, True, 0),
+    (12, 3, 576, 200, True, False, 64), (6, 2, 72, 704, False, False, 0)])
+def test_experts_on_whole_lines(E, top, width, ff, gate, on_input, pad, T):
+    """Inner sizes in units of 64 (one of them, both, one unit and many; the last two cases mix the two kernels), output columns
+    that end inside a tile, an expert without pairs and one with most of them, padded rows.  Products of bfloat16 summed in
+    float32, the inner row rounded once: 2^-8 of the largest value covers both roundings."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(E + ff + T)
+    h = torch.randn(T, width, generator=g).bfloat16().to(DEV)
+    mats = [(torch.randn(E, *s, generator=g) * 0.1).bfloat16().to(DEV) for s in ((ff, width), (ff, width), (width, ff))]
+    score = torch.rand(T, E, generator=g)
+    score[:, 0] = -1.0                               # (nobody's expert, unless all are needed)
+    score[: T * 2 // 3, 1] = 2.0
+    idx = score.topk(top).indices.to(torch.int32).to(DEV)
+    wts = torch.rand(T, top, generator=g).to(DEV)
+    ref = torch.zeros(T, width, dtype=torch.float64, device=DEV)
+    for k in range(top):
+        for e in range(E):
+            t = (idx[:, k] == e).nonzero().flatten()
+            w = wts[t, k].double()[:, None]
+            G, U = (h[t].double() @ mats[m][e].double().T * (w if on_input else 1.0) for m in (0, 1))
+            y = G.clamp(max=0.7) * torch.sigmoid(1.702 * G.clamp(max=0.7)) * (U.clamp(-0.7, 0.7) + 1.0) if gate else U.clamp(min=0) ** 2
+            ref[t] += (1.0 if on_input else w) * (y @ mats[2][e].double().T)
+    pads = [torch.nn.functional.pad(m, (0, pad)).contiguous() for m in mats]
+    how = dict(up_offset=1.0 if gate else 0.0, weight_input=on_input, by_tiles=True)
+    run = lambda a, i, w: ops.as_tensor(ops.routed_experts(a, pads[0] if gate else None, pads[1], pads[2], i, w, 0.7 if gate else math.inf,        # noqa: E731
+                                                           1.702 if gate else 1.0, **how))
+    out = run(h, idx, wts)
+    assert float((out.double() - ref).abs().max()) < 2.0 ** -8 * float(ref.abs().max())
+    for n in (1, 40):                                # (another split into tiles, other tiles: the same bits)
+        assert torch.equal(run(h[:n].contiguous(), idx[:n].contiguous(), wts[:n].contiguous()), out[:n])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rank,rot,dims,ps,Dp", [(40, 8, 8, 16, 48), (24, 16, 16, 8, 48), (150, 10, 6, 16, 192),
                                                  (20, 6, 6, 32, 32), (11, 0, 0, 8, 16)])

@@ -14,10 +14,9 @@
 // Activations A [M, K] stay row-major.  The W tile is the MFMA's first operand,
 // so a lane ends up with 4 consecutive output columns of one row.
 #include "common.h"
+#include "mfma_tiles.h"
 #include "tffinfer_kernels.h"
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 __device__ __forceinline__ uint4 ld16(const bf16_t* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ bf16x8 as_frag(const uint4& v) { return *reinterpret_cast<const bf16x8*>(&v); }
@@ -83,11 +82,7 @@ __device__ __forceinline__ floatx4 bias4(const float* __restrict__ bias, int n, 
 // while one is worked on.
 // A wave waits for its own copies of the tile it is about to read
 // (s_waitcnt vmcnt), the barrier that follows makes the other waves' visible.
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* glb_ptr_t;
-
-constexpr int vmcnt_imm(int v) { return (v & 15) | (7 << 4) | (15 << 8) | ((v >> 4) << 14); }
-
 template <int WGM, int WGN, int WTM, int WTN, int STAGES, bool GLU, typename TC, int KPS = 2, bool EARLY = false>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bf16_async_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, TC* __restrict__ C, int M, int N,
@@ -373,27 +368,6 @@ static int launch_async_g(const bf16_t* A, const bf16_t* Wp, void* C, int M, int
 // tile t + NWS - 1; at the start of t it needs W tile t + 1 and the A unit of t + 1, issued in tile
 // t - NWS + 2 at the latest.  Copies complete in the order issued, so the wait is by count.
 // K a multiple of 64; a split of K takes whole units.
-__device__ __forceinline__ void mfma_acc(floatx4& c, const bf16x8& a, const bf16x8& b) {
-    // accumulate in place, in the accumulation registers, as the instruction itself says it: through
-    // the builtin the register allocator moves accumulators between the two files around every MFMA
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-}
-__device__ __forceinline__ void copy16_to_lds_sbase(unsigned long long base, unsigned lane_off, unsigned lds_wave_addr) {
-    // the address is a uniform base and a 32-bit offset per lane: walking k is scalar work
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds_wave_addr), "v"(lane_off), "s"(base)
-                 : "memory", "m0");
-}
-
-// The lane's index, taken where it is asked for: what the epilogue works out from it is then worked out
-// after the main loop, where there are registers for it, instead of before it and kept (or spilled) across.
-__device__ __forceinline__ int w4_lane() {
-    int lane;
-    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
-    return lane;
-}
-
 // A wave's 128 rows x OW column groups of results go out through LDS, so that a store instruction
 // writes whole rows instead of 16 rows x 8 or 16 bytes: a lane leaves its four columns of a row in
 // the wave's own region of LDS (rows padded by 16 bytes against bank conflicts) and takes 16 bytes

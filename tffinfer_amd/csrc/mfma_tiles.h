@@ -1,0 +1,32 @@
+// What the products of four waves a block share: operand types, MFMAs that accumulate in place, copies from global memory
+// into LDS by a uniform base, the wait for them by count.
+#pragma once
+#include "common.h"
+
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+// s_waitcnt's immediate that waits until at most v copies or loads of the wave are in flight
+constexpr int vmcnt_imm(int v) { return (v & 15) | (7 << 4) | (15 << 8) | ((v >> 4) << 14); }
+
+__device__ __forceinline__ void mfma_acc(floatx4& c, const bf16x8& a, const bf16x8& b) {
+    // accumulate in place, in the accumulation registers, as the instruction itself says it: through
+    // the builtin the register allocator moves accumulators between the two files around every MFMA
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void copy16_to_lds_sbase(unsigned long long base, unsigned lane_off, unsigned lds_wave_addr) {
+    // the address is a uniform base and a 32-bit offset per lane: walking k is scalar work
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds_wave_addr), "v"(lane_off), "s"(base)
+                 : "memory", "m0");
+}
+
+// The lane's index, taken where it is asked for: what the epilogue works out from it is then worked out
+// after the main loop, where there are registers for it, instead of before it and kept (or spilled) across.
+__device__ __forceinline__ int w4_lane() {
+    int lane;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+    return lane;
+}

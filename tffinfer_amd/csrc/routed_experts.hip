@@ -23,7 +23,10 @@
 // rows a power of two of bytes apart all come through one memory channel, so the loader puts a
 // little room behind each).
 #include "common.h"
+#include "mfma_tiles.h"
 #include "tffinfer_kernels.h"
+#include <math.h>
+#include <type_traits>
 
 // dot product of two rows of K elements by one wave (lanes stride through k, then a tree)
 template <typename TA, typename TB>
@@ -523,6 +526,193 @@ __global__ __launch_bounds__(256) void experts_tiles_kernel(
     }
 }
 
+// The same products for inner sizes in units of 64: both operands pass through LDS as whole cache lines, four waves, one to
+// a SIMD, with the LDS reads of the next 32 k and the copies of later units between the MFMAs of the present ones.  Block:
+// BM = 16 WTM WGM pairs x BN = 64 WTN / WGM weight rows.  What bounds the kernel above is the number of requests to L2 (operands as
+// 64-byte pieces of rows, 64 flops a byte on its 128 x 128 tile) and the waits between its barriers, which nothing overlaps.
+// Here a unit of 64 k is copied eight rows x 128 bytes at a time (lane i of a copy lands at byte 16 i and fetches row i / 8,
+// chunk (i % 8) ^ (i / 8), so that an operand's sixteen rows come back from different banks), the pairs' rows through
+// the tile's list; NS units lie in LDS, two are on their way.  GATE_UP: the tile's groups of 16 weight rows are gate
+// and up in turn, so a lane holds both sums of its outputs.  k ascends in steps of 32 for every pair as above: the same bits.
+// Unit u + 2 is copied during unit u, into the slot that unit u - 1 has left: its last operands were read, and had arrived
+// (lgkmcnt 0), before the barrier in the middle of unit u - 1.  At that barrier of unit u every wave's copies of unit u + 1 have
+// landed: all but the CP / 2 copies that it issued in the first half of unit u.
+// us for both products before / now: 32 experts, four a token, 4,096 x 1,536 gated, 2,048 tokens 883 / 578 (535 TFLOP/s; some 700 with
+// the tiles' padding), 150 tokens 273 / 262; 4,096 x 3,072 without a gate, 4,096 tokens 2,041 / 1,164; 16 experts, two a token, 2,048 x 2,048
+// without a gate, 512 tokens 130 / 86.
+template <int MODE, int WGM, int WTM, int WTN>
+__global__ __launch_bounds__(256) void experts_lines_kernel(
+    const bf16_t* __restrict__ a_rows, int a_row, const bf16_t* __restrict__ W0, const bf16_t* __restrict__ W1,
+    const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_rows, const int32_t* __restrict__ num_tiles,
+    const float* __restrict__ wts, int T, int top, int K, int N, float limit, float act_alpha, float up_offset,
+    bf16_t* __restrict__ y, float* __restrict__ out, int max_tiles, int col_blocks, int ldw, int weight_input) {
+    constexpr int NW = 4, NS = 3, WGN = NW / WGM;
+    constexpr int BM = WGM * WTM * 16, BN = WGN * WTN * 16;
+    constexpr int LPA = BM / 8 / NW, LPW = BN / 8 / NW, CP = LPA + LPW;      // a wave's copies of a unit
+    constexpr unsigned A_BYTES = BM * 128u, UNIT = (BM + BN) * 128u;
+    constexpr int NMF = WTM * WTN, RPM = NMF / (WTM + WTN), CPM = NMF / (CP / 2);
+    static_assert(RPM >= 1 && CPM >= 1 && CP % 2 == 0 && LPA >= 1, "the MFMAs of a k-tile hide its reads and copies");
+    static_assert(NS * UNIT <= 160 * 1024, "LDS");
+    __shared__ __attribute__((aligned(1024))) char smem[NS * UNIT];
+    // blocks to XCDs as above: one XCD sees all tiles of a column block, an expert's tiles next to each other
+    const int L = blockIdx.x, q8 = L >> 3;
+    const int tile = q8 % max_tiles, col_block = (q8 / max_tiles) * 8 + (L & 7);
+    if (tile >= num_tiles[0] || col_block >= col_blocks) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = WGM == 2 ? wave >> 1 : 0, wn = WGM == 2 ? wave & 1 : wave;
+    const int fr = lane & 15, fg = lane >> 4;
+    const int e = tile_expert[tile];
+    const int32_t* pairs = tile_rows + (size_t)tile * BM;
+    const int c0 = col_block * (MODE == 1 ? BN / 2 : BN);           // the block's first output
+
+    floatx4 acc[WTN][WTM];
+#pragma unroll
+    for (int i = 0; i < WTN; ++i)
+#pragma unroll
+        for (int j = 0; j < WTM; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    // what a wave copies of a unit: the pairs' rows, eight at a time, and the weight's
+    const unsigned chunk = (unsigned)(((lane & 7) ^ (lane >> 3)) * 16);
+    unsigned off[CP];
+    unsigned long long base[3];
+    base[0] = (unsigned long long)a_rows;
+    base[1] = (unsigned long long)(W0 + (size_t)e * N * ldw);
+    base[2] = MODE == 1 ? (unsigned long long)(W1 + (size_t)e * N * ldw) : base[1];
+#pragma unroll
+    for (int c = 0; c < LPA; ++c) {
+        const int p = max(pairs[(wave + NW * c) * 8 + (lane >> 3)], 0);      // (a place without a pair repeats pair 0, nobody reads it)
+        off[c] = (unsigned)(MODE != 0 ? p / top : p) * (unsigned)a_row * 2u + chunk;
+    }
+#pragma unroll
+    for (int c = 0; c < LPW; ++c) {
+        const int r0 = (wave + NW * c) * 8, grp = r0 >> 4, in = (r0 & 15) + (lane >> 3);
+        const int n = c0 + (MODE == 1 ? grp >> 1 : grp) * 16 + in;
+        off[LPA + c] = (unsigned)min(n, N - 1) * (unsigned)ldw * 2u + chunk;
+    }
+    const unsigned smem_addr = (unsigned)(size_t)(lds_ptr_t)smem;
+    const int nu = K >> 6;
+    int u_next = 0;                                   // the unit to copy next; past the end the last one once more
+    unsigned long long k_off = 0;
+    unsigned ws = 0;                                  // its slot
+#define EXL_COPY(c)                                                                                                 \
+    {                                                                                                               \
+        const int which = (c) < LPA ? 0 : (MODE == 1 && (((wave + NW * ((c) - LPA)) >> 1) & 1)) ? 2 : 1;             \
+        copy16_to_lds_sbase(base[which] + k_off, off[c],                                                            \
+                            smem_addr + ws + ((c) < LPA ? 0u : A_BYTES) + (unsigned)(wave + NW * ((c) < LPA ? (c) : (c) - LPA)) * 1024u); \
+    }
+#define EXL_ISSUED()                                                                                                \
+    {                                                                                                               \
+        if (u_next + 1 < nu) { ++u_next; k_off += 128ull; }                                                         \
+        ws = ws + UNIT == NS * UNIT ? 0u : ws + UNIT;                                                               \
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int c = 0; c < CP; ++c) EXL_COPY(c)
+        EXL_ISSUED()
+    }
+    // a lane's 16 bytes of an operand: row fr of 16, chunk h * 4 + fg of the row's 8
+    unsigned rd[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) rd[h] = (unsigned)(fr >> 3) * 1024u + (unsigned)(((fr & 7) * 8 + ((h * 4 + fg) ^ (fr & 7))) * 16);
+    const unsigned a_rd = (unsigned)(wm * WTM) * 2048u, w_rd = A_BYTES + (unsigned)(wn * WTN) * 2048u;
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(CP));
+    __syncthreads();
+    bf16x8 fw[2][WTN], fa[2][WTM];
+#pragma unroll
+    for (int i = 0; i < WTN; ++i) fw[0][i] = *reinterpret_cast<const bf16x8*>(smem + w_rd + rd[0] + i * 2048);
+#pragma unroll
+    for (int j = 0; j < WTM; ++j) fa[0][j] = *reinterpret_cast<const bf16x8*>(smem + a_rd + rd[0] + j * 2048);
+    unsigned rs = 0;                                  // the slot that the next operands are read from
+#define EXL_TILE(h)                                                                                                 \
+    {                                                                                                               \
+        if (h) {                                                                                                    \
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                                      \
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(CP / 2));                                                          \
+            asm volatile("s_barrier" ::: "memory");                                                                 \
+            rs = rs + UNIT == NS * UNIT ? 0u : rs + UNIT;                                                           \
+        }                                                                                                           \
+        const char* na = smem + rs + a_rd + rd[(h) ^ 1];                                                            \
+        const char* nw = smem + rs + w_rd + rd[(h) ^ 1];                                                            \
+        _Pragma("unroll") for (int i = 0; i < WTN; ++i)                                                             \
+            _Pragma("unroll") for (int j = 0; j < WTM; ++j) {                                                       \
+                const int q = i * WTM + j;                                                                          \
+                mfma_acc(acc[i][j], fw[h][i], fa[h][j]);                                                            \
+                if (q % RPM == RPM - 1 && q / RPM < WTN + WTM) {                                                    \
+                    const int x = q / RPM;                                                                          \
+                    if (x < WTM) fa[(h) ^ 1][x < WTM ? x : 0] = *reinterpret_cast<const bf16x8*>(na + x * 2048);    \
+                    else fw[(h) ^ 1][x >= WTM ? x - WTM : 0] = *reinterpret_cast<const bf16x8*>(nw + (x - WTM) * 2048); \
+                }                                                                                                   \
+                if (q % CPM == CPM - 1 && q / CPM < CP / 2) EXL_COPY((h) * (CP / 2) + q / CPM)                      \
+            }                                                                                                       \
+        if (h) EXL_ISSUED()                                                                                         \
+    }
+    for (int u = 0; u < nu; ++u) {
+        EXL_TILE(0)
+        EXL_TILE(1)
+    }
+#undef EXL_TILE
+#undef EXL_COPY
+#undef EXL_ISSUED
+    // every copy has landed, every operand has come back and the last MFMAs have written: LDS is free for the results
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+    __syncthreads();
+    // A wave's results go through its own part of LDS, so that its stores are whole pieces of a pair's row.
+    typedef typename std::conditional<MODE == 0, float, bf16_t>::type TO;
+    constexpr int OW = MODE == 1 ? WTN / 2 : WTN, EL = 16 / (int)sizeof(TO);
+    constexpr int RB = OW * 16 * (int)sizeof(TO), RBP = RB + 16, LPR = RB / 16, RPI = 64 / LPR;
+    constexpr int REGION = (int)(NS * UNIT / NW) & ~1023;
+    static_assert(WTM * 16 * RBP <= REGION && LPR <= 64 && (LPR & (LPR - 1)) == 0, "the wave's part holds its results");
+    char* region = smem + wave * REGION;
+    const int ln = w4_lane(), r = ln & 15, g = ln >> 4;
+#pragma unroll
+    for (int j = 0; j < WTM; ++j) {
+        __builtin_amdgcn_sched_barrier(0);
+        float w = 1.0f;
+        if (MODE == 0 ? !weight_input : weight_input != 0) {
+            const int p = pairs[(wm * WTM + j) * 16 + r];
+            w = p >= 0 ? wts[p] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < OW; ++i) {
+            char* dst = region + (j * 16 + r) * RBP + (i * 16 + g * 4) * (int)sizeof(TO);
+            float v[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if constexpr (MODE == 1) {
+                    const float gv = fminf(acc[2 * i][j][c] * w, limit);
+                    const float uv = fminf(fmaxf(acc[2 * i + 1][j][c] * w, -limit), limit);
+                    v[c] = gv * (1.0f / (1.0f + expf(-act_alpha * gv))) * (uv + up_offset);
+                } else if constexpr (MODE == 2) {
+                    const float u = fmaxf(acc[i][j][c] * w, 0.f);
+                    v[c] = u * u;
+                } else {
+                    v[c] = w * acc[i][j][c];
+                }
+            }
+            if constexpr (sizeof(TO) == 4) {
+                *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+                union { bf16_t h[4]; uint2 u; } pk;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) pk.h[c] = (bf16_t)v[c];
+                *reinterpret_cast<uint2*>(dst) = pk.u;
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int srow = ln / LPR, sch = ln % LPR, n = c0 + wn * OW * 16 + sch * EL;
+#pragma unroll 4
+    for (int t = 0; t < WTM * 16 / RPI; ++t) {
+        const int row = t * RPI + srow, p = pairs[wm * WTM * 16 + row];
+        const uint4 v = *reinterpret_cast<const uint4*>(region + row * RBP + sch * 16);
+        if (p < 0 || n >= N) continue;                // (N is a multiple of 8: a piece is whole or not there)
+        if constexpr (MODE == 0) *reinterpret_cast<uint4*>(out + ((size_t)(p % top) * T + p / top) * N + n) = v;
+        else *reinterpret_cast<uint4*>(y + (size_t)p * N + n) = v;
+    }
+}
+
 // The planes of the pairs whose expert has no matrices: out[k][t][:] = wts[t][k] * h[t][:].
 __global__ __launch_bounds__(256) void experts_identity_kernel(const bf16_t* __restrict__ h, int h_row,
                                                                const int32_t* __restrict__ idx, const float* __restrict__ wts,
@@ -561,10 +751,27 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
                 ((uintptr_t)Wd % 16) == 0 && ((uintptr_t)y % 16) == 0, "experts_by_tiles: operands must be 16-byte aligned");
     TFF_REQUIRE((long)T * top < (1L << 31) && max_tiles <= (1 << 20) && max_tiles >= (long)T * top / 64 + E,
                 "experts_by_tiles: %d tiles do not hold %d x %d pairs of %d experts", max_tiles, T, top, E);
-    // tiles of 128 pairs where an expert has a few hundred on average: every weight element fetched
-    // serves twice the flops, which is what bounds these products; the padding of an expert's last
-    // tile costs more with fewer pairs
-    const bool tall = (long)T * top >= 192L * E;
+    // Inner sizes in units of 64 run on whole cache lines, the others on 64-byte pieces.  (A lane's offset into the rows is 32 bits.)
+    const size_t limit32 = (size_t)1 << 32;
+    const bool h_near = (size_t)T * h_row * 2 < limit32, y_near = (size_t)T * top * ff * 2 < limit32;
+    const bool lines_up = width % 64 == 0 && h_near && (size_t)ff * ldw_in * 2 < limit32;
+    const bool lines_down = ff % 64 == 0 && y_near && (size_t)width * ldw_down * 2 < limit32;
+    // Tiles of 128 or of 64 pairs.  On 64-byte pieces: 128 where an expert has a few hundred pairs on average (every weight element
+    // fetched serves twice the flops; the padding of an expert's last tile costs more with fewer).  On whole lines a block is
+    // alone on its CU and a tile of 128 takes some 1.12 times as long as one of 64 (up to there both are their weight's stream), so
+    // what counts is how often the blocks go round the CUs.  us, 64 / 128: 32 experts, four a token, 4,096 x 1,536, 150 tokens 265 / 287,
+    // 512 tokens 328 / 301, 1,000 tokens 464 / 384; 16 experts, two a token, 2,048 x 1,024, 700 tokens 72 / 84, 1,000 tokens 117 / 85.
+    bool tall = (long)T * top >= 192L * E;
+    if (lines_up && lines_down) {
+        const double n = (double)T * top / E;
+        const int cb_up = (ff + (Wg ? 127 : 255)) / (Wg ? 128 : 256), cb_down = (width + 255) / 256;
+        double cost[2];
+        for (int i = 0; i < 2; ++i) {
+            const double tiles = E * fmax(1.0, n / (64 << i) + 0.5);      // (half of an expert's last tile is padding on average)
+            cost[i] = ceil(tiles * cb_up / 256) * width + ceil(tiles * cb_down / 256) * ff;
+        }
+        tall = cost[1] * 1.12 < cost[0];
+    }
     const int rows = tall ? 128 : 64;
     if (T == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
@@ -575,28 +782,39 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
     experts_sort_kernel<<<1, 1024, 0, s>>>(idx, T * top, E, rows, tile_expert, tile_rows, num_tiles);
     int rc = tff_check_launch("experts_sort");
     if (rc) return rc;
-    const int cb_up = Wg ? (ff + 63) / 64 : (ff + 127) / 128, cb_down = (width + 127) / 128;
-#define EXT_LAUNCH(GU, AFRV, CB, ...) experts_tiles_kernel<GU, AFRV><<<((CB) + 7) / 8 * 8 * max_tiles, 256, 0, s>>>(__VA_ARGS__)
-    if (!Wg && tall)
-        EXT_LAUNCH(2, 8, cb_up, (const bf16_t*)h, h_row, (const bf16_t*)Wu, nullptr, tile_expert, tile_rows,
-                   num_tiles, wts, T, top, width, ff, limit, act_alpha, up_offset, (bf16_t*)y, nullptr, max_tiles, cb_up, ldw_in, weight_input);
-    else if (!Wg)
-        EXT_LAUNCH(2, 4, cb_up, (const bf16_t*)h, h_row, (const bf16_t*)Wu, nullptr, tile_expert, tile_rows,
-                   num_tiles, wts, T, top, width, ff, limit, act_alpha, up_offset, (bf16_t*)y, nullptr, max_tiles, cb_up, ldw_in, weight_input);
-    else if (tall)
-        EXT_LAUNCH(1, 8, cb_up, (const bf16_t*)h, h_row, (const bf16_t*)Wg, (const bf16_t*)Wu, tile_expert, tile_rows,
-                   num_tiles, wts, T, top, width, ff, limit, act_alpha, up_offset, (bf16_t*)y, nullptr, max_tiles, cb_up, ldw_in, weight_input);
-    else
-        EXT_LAUNCH(1, 4, cb_up, (const bf16_t*)h, h_row, (const bf16_t*)Wg, (const bf16_t*)Wu, tile_expert, tile_rows,
-                   num_tiles, wts, T, top, width, ff, limit, act_alpha, up_offset, (bf16_t*)y, nullptr, max_tiles, cb_up, ldw_in, weight_input);
-    rc = tff_check_launch("experts_gate_up_tiles");
-    if (rc) return rc;
-    if (tall)
-        EXT_LAUNCH(0, 8, cb_down, (const bf16_t*)y, ff, (const bf16_t*)Wd, nullptr, tile_expert, tile_rows, num_tiles, wts,
-                   T, top, ff, width, limit, act_alpha, up_offset, nullptr, out, max_tiles, cb_down, ldw_down, weight_input);
-    else
-        EXT_LAUNCH(0, 4, cb_down, (const bf16_t*)y, ff, (const bf16_t*)Wd, nullptr, tile_expert, tile_rows, num_tiles, wts,
-                   T, top, ff, width, limit, act_alpha, up_offset, nullptr, out, max_tiles, cb_down, ldw_down, weight_input);
-#undef EXT_LAUNCH
+    const int up_mode = Wg ? 1 : 2;
+    const bf16_t *w0 = (const bf16_t*)(Wg ? Wg : Wu), *w1 = (const bf16_t*)(Wg ? Wu : nullptr);
+#define EX_ARGS_UP (const bf16_t*)h, h_row, w0, w1, tile_expert, tile_rows, num_tiles, wts, T, top, width, ff, limit, act_alpha, \
+                   up_offset, (bf16_t*)y, nullptr, max_tiles, cb, ldw_in, weight_input
+#define EX_ARGS_DOWN (const bf16_t*)y, ff, (const bf16_t*)Wd, nullptr, tile_expert, tile_rows, num_tiles, wts, T, top, ff, width, limit, \
+                     act_alpha, up_offset, nullptr, out, max_tiles, cb, ldw_down, weight_input
+#define EX_GRID (unsigned)((cb + 7) / 8 * 8 * max_tiles)
+#define EX_LINES(MODE, ...)                                                                                \
+    do {                                                                                                   \
+        if (tall) experts_lines_kernel<MODE, 2, 4, 8><<<EX_GRID, 256, 0, s>>>(__VA_ARGS__);                \
+        else experts_lines_kernel<MODE, 1, 4, 4><<<EX_GRID, 256, 0, s>>>(__VA_ARGS__);                     \
+    } while (0)
+#define EX_TILES(MODE, ...)                                                                                \
+    do {                                                                                                   \
+        if (tall) experts_tiles_kernel<MODE, 8><<<EX_GRID, 256, 0, s>>>(__VA_ARGS__);                      \
+        else experts_tiles_kernel<MODE, 4><<<EX_GRID, 256, 0, s>>>(__VA_ARGS__);                           \
+    } while (0)
+    {
+        const int out_cols = (lines_up ? 256 : 128) / (Wg ? 2 : 1), cb = (ff + out_cols - 1) / out_cols;
+        if (lines_up && up_mode == 1) EX_LINES(1, EX_ARGS_UP);
+        else if (lines_up) EX_LINES(2, EX_ARGS_UP);
+        else if (up_mode == 1) EX_TILES(1, EX_ARGS_UP);
+        else EX_TILES(2, EX_ARGS_UP);
+        rc = tff_check_launch("experts_gate_up_tiles");
+        if (rc) return rc;
+    }
+    const int cb = (width + (lines_down ? 255 : 127)) / (lines_down ? 256 : 128);
+    if (lines_down) EX_LINES(0, EX_ARGS_DOWN);
+    else EX_TILES(0, EX_ARGS_DOWN);
+#undef EX_ARGS_UP
+#undef EX_ARGS_DOWN
+#undef EX_GRID
+#undef EX_LINES
+#undef EX_TILES
     return tff_check_launch("experts_down_tiles");
 }
