@@ -95,3 +95,13 @@ def test_the_test_configurations_differ_from_each_other_in_every_size():
             assert len({m["dim"], m["rot_dim"], m["vdim"]}) >= 2         # never all three alike
         seen[name] = (cfg["width"], cfg["vocab"], cfg["postln_alpha"])
     assert len(set(seen.values())) == len(seen)
+
+
+def test_few_tokens_stream_their_experts_and_many_are_dealt_to_them():
+    """The rule between the two ways: one token never takes tiles, the choice turns once as the tokens grow, and with inner
+    sizes that are not in units of 64 at 32 tokens."""
+    from tffinfer_amd.kernels.ops import _experts_by_tiles
+    for E, top, width, ff in ((32, 4, 4096, 1536), (16, 2, 2048, 1024), (8, 8, 64, 64), (1, 1, 128, 4096), (256, 8, 7168, 2048), (4, 6, 256, 128)):
+        way = [_experts_by_tiles(T, top, E, width, ff, 3) for T in range(1, 4097)]
+        assert not way[0] and way[-1] and sum(a != b for a, b in zip(way, way[1:])) == 1
+    assert [T for T in range(1, 64) if _experts_by_tiles(T, 2, 8, 72, 64, 2)][0] == 32

@@ -1250,8 +1250,21 @@ def pad_expert_rows(w: torch.Tensor) -> torch.Tensor:
 
 
 #: tokens from which a step's (token, expert) pairs are dealt to their experts and run on the matrix
-#: cores; below, every pair streams its expert's rows itself, which is what few tokens are bound by
+#: cores, where the inner sizes are not in units of 64; below, every pair streams its expert's rows itself
 EXPERT_TILES_MIN_TOKENS = 32
+
+
+def _experts_by_tiles(T: int, top: int, E: int, width: int, ff: int, matrices: int) -> bool:
+    """Whether the pairs of ``T`` tokens are dealt to their experts.  With inner sizes in units of 64 by what the two ways take,
+    fitted to 1 to 31 tokens of five sizes: a pair streams its expert's matrices at 7.3 TB/s (experts that several
+    tokens chose come from a cache), the tiles read every chosen expert once at 7 TB/s and have a floor of the length of
+    a block.  32 experts, four a token, 4,096 x 1,536, us by pairs / tiles: 8 tokens 172 / 195, 12 tokens 238 / 206, 31 tokens
+    549 / 235; 16 experts, two a token, 2,048 x 1,024: 16 tokens 58 / 63, 24 tokens 84 / 66."""
+    if width % 64 or ff % 64:
+        return T >= EXPERT_TILES_MIN_TOKENS
+    size = matrices * width * ff * 2e-6
+    used = E * (1.0 - (1.0 - min(top, E) / E) ** T)
+    return 8.0 + 0.137 * T * top * size > 12.0 + 0.0105 * (width + ff) + 0.143 * used * size
 
 
 def routed_experts(h: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
@@ -1287,7 +1300,7 @@ def routed_experts(h: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_
     L = _lib.load()
     y = torch.empty(T * top, ff, dtype=h.dtype, device=h.device)
     if by_tiles is None:
-        by_tiles = T >= EXPERT_TILES_MIN_TOKENS
+        by_tiles = _experts_by_tiles(T, top, E, width, ff, 2 if w_gate is None else 3)
     if by_tiles and h.dtype == torch.bfloat16 and L.tff_experts_tiles_supported(width, ff, width):
         # many tokens: the pairs dealt to their experts, the products on the matrix cores; the result
         # comes as one plane per chosen expert, for the norm that follows to add up in their order
