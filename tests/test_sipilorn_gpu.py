@@ -197,6 +197,34 @@ def test_delta_rule_whole_and_in_portions(H, G, D, E, taps):
     assert float(state[1].abs().max()) == 0 and float(state[2].abs().max()) == 0
 
 
+@pytest.mark.parametrize("H,G,D,E,taps", [(2, 1, 64, 20, 4), (4, 4, 64, 64, 1), (6, 2, 128, 128, 3), (2, 2, 256, 36, 4)])
+@pytest.mark.parametrize("extreme", [False, True])
+def test_delta_rule_in_chunks_of_sixteen(H, G, D, E, taps, extreme):
+    """Portions long enough for the chunks (ending in a chunk's first, middle and last token, beside a portion of one and of three
+    tokens), then more tokens from the state they left, against the plain loop; ``extreme``: decays of zero (a whole row of states
+    forgotten) and of one, beta of zero and of one.  The bound is that of the token-by-token form."""
+    ops = _ops()
+    for first, rest in ((96, 5), (97, 130), (111, 1), (161, 96)):
+        T = first + rest
+        proj, conv, a_log, dt = _delta_case(T, H, G, D, E, taps, D + E + T)
+        C = 2 * G * D + H * E
+        if extreme:
+            g = torch.Generator().manual_seed(T)
+            proj[:, C:C + H] = 80.0 * torch.randint(-1, 2, (T, H), generator=g)
+            proj[:, C + H:C + 2 * H] = torch.where(torch.rand(T, H, generator=g) < 0.1, 4e3, -80.0)
+        ref = _plain_delta(proj, conv, a_log, dt, H, G, D, E)
+        row = H * E * D + (taps - 1) * C
+        row += -row % 4
+        state = torch.zeros(4, row, device=DEV)
+        dev = [x.to(DEV) for x in (conv, a_log, dt)]
+        few = torch.cat([proj[:first], proj[:1], proj[:3]]).to(DEV)
+        o = ops.gated_delta(few, *dev, state, _batch([first, 1, 3], [0, 0, 0], [2, 0, 3]), H, G, D, E)
+        assert _err(o[:first], ref[:first]) < 3e-5 and _err(o[first:first + 1], ref[:1]) < 3e-5 and _err(o[first + 1:], ref[:3]) < 3e-5
+        o = ops.gated_delta(proj[first:].to(DEV), *dev, state, _batch([rest], [first], [2]), H, G, D, E)
+        assert _err(o, ref[first:]) < 3e-5, (first, rest)
+        assert float(state[1].abs().max()) == 0
+
+
 @pytest.mark.parametrize("decode", [False, True])
 def test_a_value_written_far_back_is_read(decode):
     """Decay 1, beta 1, keys that are axes: the value written under an axis at the third token is what a query

@@ -110,7 +110,7 @@ __device__ __forceinline__ void gd_keep_inputs(const float* __restrict__ proj, s
 
 // One token of one value channel, on the row of sixteen lanes that shares the channel; lane s holds the key
 // channels s, s + 16, ... of S, k and q.  The same additions in the same order wherever it is used, so that a
-// sequence gives the same bits however it is cut into steps.
+// sequence gives the same bits however it is cut into steps of portions that are too short for chunks (below).
 template <int KPL>
 __device__ __forceinline__ float gd_token(float (&S)[KPL], const float (&kk)[KPL], const float (&qq)[KPL], float v, float beta,
                                           float g) {
@@ -326,6 +326,264 @@ TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ld
     else GD_LAUNCH(16);
 #undef GD_LAUNCH
     return tff_check_launch("gdelta_recurrence");
+}
+
+// ------------------------------------------------- long portions: chunks of sixteen tokens ---
+// For head sizes of 64, 128 and 256.  Within a chunk that starts from S0, with G_t = g_0 .. g_t and P_ts = g_(s+1) .. g_t,
+//
+//   (I + L) U = B (V - diag(G) K S0),   L_ts = beta_t P_ts (k_t . k_s), s < t;      S_t = G_t S0 + sum over s <= t of P_ts k_s u_s^T
+//   O = diag(G) Q S0 + A U,             A_ts = P_ts (q_t . k_s), s <= t
+//
+// so that a chunk is a handful of products on the float32 matrix cores (v_mfma_f32_16x16x4_f32) instead of sixteen steps that
+// wait for one another.  The P are products, not quotients: a decay of zero is a factor like any other.  (I + L)^-1 B and A do not
+// depend on S: gdelta_chunk_kernel forms them for all chunks at once, a wave per chunk and head (the inverse by forward
+// substitution, a lane a column; its elements are beta_s k_t' (product of reflections) k_s, at most 1 in size).
+// gdelta_scan_kernel walks the chunks of a request: a block per head and sixteen value channels, a wave a quarter of the key
+// channels, whose part of S stays in its accumulators; the waves' parts of K S0 and Q S0 meet in LDS, one barrier a chunk, and the
+// next chunk's operands are on their way meanwhile.  Accumulators are operands as they are: lane (column r, g) holds rows 4 g ..
+// 4 g + 3 of a product, which is where the next product's MFMA j wants row 4 g + j.
+// One token after the other took 0.25 us a token: 2,048 tokens of 32 heads of 128 x 128 in 515 us, now 17 + 196; 2,048 tokens of 4 heads
+// of 64 x 64 400 / 110; four requests of 901, 700, 430 and 300 tokens, with the preparation, 428 / 295.  The relative error against 64
+// bits is 1.3e-7 (1.2e-7 token by token).
+//
+// work: per chunk and head 16 x 16 of (I + L)^-1 B, 16 x 16 of A, 16 G, 16 P_15,s; the chunk that starts at token t of row r
+// lies at place t / 16 + r.
+#define GD_WORK 544
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gd_floatx4;
+
+__device__ __forceinline__ gd_floatx4 gd_mfma16(const float4& a, const gd_floatx4& b, gd_floatx4 c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[0], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[1], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[2], c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[3], c, 0, 0, 0);
+}
+
+// The same from zero in two chains of eight terms, which meet at the end: half the wait and a smaller error.
+__device__ __forceinline__ gd_floatx4 gd_mfma16_halves(const float4& a, const gd_floatx4& b) {
+    const gd_floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+    gd_floatx4 x = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[0], zero, 0, 0, 0);
+    gd_floatx4 y = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[2], zero, 0, 0, 0);
+    x = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[1], x, 0, 0, 0);
+    y = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[3], y, 0, 0, 0);
+    return x + y;
+}
+
+__global__ __launch_bounds__(64) void gdelta_chunk_kernel(const float* __restrict__ pre, const int32_t* __restrict__ cu_tokens,
+                                                          float* __restrict__ work, int H, int G, int D, int E) {
+    __shared__ float sl[16][17];
+    const int h = blockIdx.y, r = blockIdx.z, lane = threadIdx.x, c = lane & 15, g = lane >> 4;
+    const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0, first = blockIdx.x * 16;
+    if (first >= n) return;
+    const int C = 2 * G * D + H * E, gk = h / (H / G);
+    const size_t ldq = (size_t)C + 2 * H;
+    const int tok = first + c;                            // this lane's token as a row and as a column
+    const float* row = pre + (size_t)(t0 + min(tok, n - 1)) * ldq;
+    const float* kp = row + (size_t)(G + gk) * D + 4 * g;
+    const float* qp = row + (size_t)gk * D + 4 * g;
+    gd_floatx4 kk = {0.f, 0.f, 0.f, 0.f}, qk = {0.f, 0.f, 0.f, 0.f};
+    for (int d = 0; d < D; d += 32) {                     // (short chains, added up: a sum of D terms in one chain loses a bit more)
+        gd_floatx4 ks[2], qs[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float4 k4 = *reinterpret_cast<const float4*>(kp + d + 16 * i), q4 = *reinterpret_cast<const float4*>(qp + d + 16 * i);
+            const gd_floatx4 kb = {k4.x, k4.y, k4.z, k4.w};
+            ks[i] = gd_mfma16(k4, kb, gd_floatx4{0.f, 0.f, 0.f, 0.f});      // lane: k_t . k_s, s = c, t = 4 g + i
+            qs[i] = gd_mfma16(q4, kb, gd_floatx4{0.f, 0.f, 0.f, 0.f});
+        }
+        kk = kk + (ks[0] + ks[1]);
+        qk = qk + (qs[0] + qs[1]);
+    }
+    // (tokens past the portion's end: beta 0, no decay)
+    const float beta = tok < n ? row[C + h] : 0.f, dec = tok < n ? row[C + H + h] : 1.f;
+    // (in 64 bits: sixteen roundings of one factor would be one error of a whole row of the results)
+    double p[4] = {1., 1., 1., 1.}, gt = 1., pe = 1.;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const double x = (double)__shfl(dec, j, 64);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] *= (j > c && j <= 4 * g + i) ? x : 1.;
+        gt *= j <= c ? x : 1.;
+        pe *= j > c ? x : 1.;
+    }
+    float* w = work + ((size_t)((t0 + first) / 16 + r) * H + h) * GD_WORK;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int t = 4 * g + i;
+        const float bt = __shfl(beta, t, 64);
+        sl[t][c] = c < t ? bt * (float)p[i] * kk[i] : 0.f;
+        w[256 + t * 16 + c] = c <= t ? (float)p[i] * qk[i] : 0.f;
+    }
+    __syncthreads();
+    if (lane < 16) {
+        float x[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            float a = t == c ? 1.f : 0.f;
+#pragma unroll
+            for (int s = 0; s < t; ++s) a = fmaf(-sl[t][s], x[s], a);
+            x[t] = a;
+            w[t * 16 + c] = a * beta;
+        }
+        w[512 + c] = (float)gt;
+        w[528 + c] = (float)pe;
+    }
+}
+
+// WV waves of NT tiles of 16 key channels each (D = 16 WV NT).
+template <int NT, int WV>
+__global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __restrict__ pre, const float* __restrict__ proj, size_t ldp,
+                                                          float* __restrict__ state, size_t state_row, size_t tail_off, int taps,
+                                                          const int32_t* __restrict__ cu_tokens,
+                                                          const int32_t* __restrict__ state_slots, const float* __restrict__ work,
+                                                          float* __restrict__ o, int H, int G, int E) {
+    constexpr int D = 16 * WV * NT;
+    __shared__ gd_floatx4 part[2][2][WV][64];
+    const int h = blockIdx.x, r = blockIdx.z, j0 = blockIdx.y * 16;      // (a head's blocks on one XCD: they read the same keys and queries)
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+    const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0;
+    if (n <= 0) return;                                    // (the whole block: a request without tokens changes nothing)
+    const int C = 2 * G * D + H * E, gk = h / (H / G);
+    const size_t ldq = (size_t)C + 2 * H;
+    const bool live = j0 + c < E;
+    const int j = min(j0 + c, E - 1);
+    float* srow = state + (size_t)state_slots[r] * state_row;
+    float* sp = srow + ((size_t)h * E + j) * D + wv * 16 * NT + 4 * g;
+    gd_floatx4 S[NT];
+#pragma unroll
+    for (int m = 0; m < NT; ++m) S[m] = *reinterpret_cast<const gd_floatx4*>(sp + 16 * m);
+    struct Ops {
+        float4 k[NT], q[NT], inv, att, gt, pe;
+        float kt[NT][4], v[4];
+    } x0, x1, x2;
+    // Addresses are a uniform base and a lane's 32-bit offset that is the same for all chunks but the last, whose tokens past the
+    // portion's end repeat its last one (their u is zero): with one wave to a SIMD address arithmetic is time.
+    const unsigned wstep = (unsigned)H * GD_WORK * 4u, ld = (unsigned)ldq * 4u;
+    const int chunks = (n + 15) / 16, last = n - 1 - 16 * (chunks - 1);
+    const char* base = (const char*)(pre + (size_t)t0 * ldq);
+    const char* wbase = (const char*)(work + ((size_t)(t0 / 16 + r) * H + h) * GD_WORK);
+    const unsigned kcol = (unsigned)((G + gk) * D + wv * 16 * NT) * 4u, qcol = (unsigned)(gk * D + wv * 16 * NT) * 4u;
+    const unsigned vcol = (unsigned)(2 * G * D + h * E + j) * 4u;
+    const unsigned in_w = (unsigned)(c * 16 + 4 * g) * 4u, in_g = (unsigned)(4 * g) * 4u;
+    auto fetch = [&](int i, Ops& x) {
+        const int most = i + 1 < chunks ? 15 : last;
+        const char* b = base + (size_t)i * 16 * ld;
+        const char* w = wbase + (size_t)i * wstep;
+        const unsigned row = (unsigned)min(c, most) * ld + (unsigned)(4 * g) * 4u;
+#pragma unroll
+        for (int m = 0; m < NT; ++m) {
+            x.k[m] = *reinterpret_cast<const float4*>(b + (row + kcol + 64u * m));
+            x.q[m] = *reinterpret_cast<const float4*>(b + (row + qcol + 64u * m));
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const unsigned tr = (unsigned)min(4 * g + q, most) * ld;
+            x.v[q] = *reinterpret_cast<const float*>(b + (tr + vcol));
+#pragma unroll
+            for (int m = 0; m < NT; ++m) x.kt[m][q] = *reinterpret_cast<const float*>(b + (tr + kcol + 64u * m + 4u * c));
+        }
+        x.inv = *reinterpret_cast<const float4*>(w + in_w);
+        x.att = *reinterpret_cast<const float4*>(w + (in_w + 1024u));
+        x.gt = *reinterpret_cast<const float4*>(w + (in_g + 2048u));
+        x.pe = *reinterpret_cast<const float4*>(w + (in_g + 2112u));
+    };
+    // a chunk's operands are asked for two chunks ahead: a chunk takes less time than a load from far memory
+    int i = 0;
+    float* ocol = o + (size_t)t0 * H * E + (size_t)h * E + j;
+    auto meet = [&](const gd_floatx4 (&p)[WV][64]) {       // the waves' parts, added as a tree
+        gd_floatx4 v[WV];
+#pragma unroll
+        for (int w = 0; w < WV; ++w) v[w] = p[w][lane];
+#pragma unroll
+        for (int k = 1; k < WV; k *= 2)
+#pragma unroll
+            for (int w = 0; w < WV; w += 2 * k) v[w] = v[w] + v[w + k];
+        return v[0];
+    };
+    auto chunk = [&](const Ops& now, Ops& ahead) {
+        fetch(min(i + 2, chunks - 1), ahead);      // (past the end the last one again: with a condition the wait for a chunk would be one for all)
+        const int buf = i & 1;
+        gd_floatx4 x = gd_mfma16_halves(now.k[0], S[0]), y = gd_mfma16_halves(now.q[0], S[0]);
+#pragma unroll
+        for (int m = 1; m < NT; ++m) {
+            x = x + gd_mfma16_halves(now.k[m], S[m]);
+            y = y + gd_mfma16_halves(now.q[m], S[m]);
+        }
+        part[buf][0][wv][lane] = x;
+        part[buf][1][wv][lane] = y;
+        __syncthreads();          // (the other buffer was last read before this barrier)
+        x = meet(part[buf][0]);
+        const gd_floatx4 gt = {now.gt.x, now.gt.y, now.gt.z, now.gt.w};
+        gd_floatx4 v = {now.v[0], now.v[1], now.v[2], now.v[3]};
+        v = v - gt * x;
+        const gd_floatx4 u = gd_mfma16_halves(now.inv, v);
+        const float gend = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(now.gt.w), 48));      // G_15: the whole chunk's decay
+#pragma unroll
+        for (int m = 0; m < NT; ++m) {
+            const float4 kt = make_float4(now.kt[m][0] * now.pe.x, now.kt[m][1] * now.pe.y, now.kt[m][2] * now.pe.z, now.kt[m][3] * now.pe.w);
+            S[m] = gd_mfma16(kt, u, S[m] * gend);
+        }
+        if (wv == i % WV) {                               // the waves take turns at the outputs
+            y = meet(part[buf][1]);
+            y = gd_mfma16_halves(now.att, u) + gt * y;
+            float* op = ocol + (size_t)(16 * i + 4 * g) * H * E;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (live && 16 * i + 4 * g + q < n) op[(size_t)q * H * E] = y[q];
+        }
+        ++i;
+    };
+    fetch(0, x0);
+    fetch(min(1, chunks - 1), x1);
+    for (;;) {
+        chunk(x0, x2);
+        if (i >= chunks) break;
+        chunk(x1, x0);
+        if (i >= chunks) break;
+        chunk(x2, x1);
+        if (i >= chunks) break;
+    }
+    if (live) {
+#pragma unroll
+        for (int m = 0; m < NT; ++m) *reinterpret_cast<gd_floatx4*>(sp + 16 * m) = S[m];
+    }
+    if (blockIdx.y == 0) gd_keep_inputs(proj, ldp, srow + tail_off, taps, t0, n, h, gk, H, G, D, E);
+}
+
+TFF_API size_t tff_gdelta_chunks_workspace(int T, int R, int H) { return ((size_t)T / 16 + R + 1) * H * GD_WORK * sizeof(float); }
+
+TFF_API int tff_gdelta_chunks_supported(int D, int E, size_t state_row) {
+    return (D == 64 || D == 128 || D == 256) && E % 4 == 0 && state_row % 4 == 0;
+}
+
+// As tff_gdelta_recurrence, in chunks; max_tokens: the longest portion.  Every row's first 2 G D + H E + 2 H channels of pre are
+// a multiple of four long, and pre, state and work are 16-byte aligned.
+TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
+                                         size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* work,
+                                         float* o, int T, int R, int H, int G, int D, int E, int max_tokens, tff_stream_t stream) {
+    TFF_REQUIRE(pre && proj && state && cu_tokens && state_slots && work && o, "gdelta_chunks: null pointer");
+    TFF_REQUIRE(R >= 0 && H > 0 && G > 0 && H % G == 0 && E > 0 && taps >= 1 && taps <= GD_MAX_TAPS && T >= 0 && max_tokens > 0,
+                "gdelta_chunks: bad sizes heads=%d kv_heads=%d vdim=%d taps=%d", H, G, E, taps);
+    const size_t C = 2 * (size_t)G * D + (size_t)H * E;
+    TFF_REQUIRE(tff_gdelta_chunks_supported(D, E, state_row) && H % 2 == 0, "gdelta_chunks: heads of %d x %d, state rows of %zu", D, E, state_row);
+    TFF_REQUIRE(((uintptr_t)pre % 16) == 0 && ((uintptr_t)state % 16) == 0 && ((uintptr_t)work % 16) == 0,
+                "gdelta_chunks: operands must be 16-byte aligned");
+    TFF_REQUIRE(ldp >= C + 2 * (size_t)H && (size_t)H * E * D <= tail_off && tail_off + (size_t)(taps - 1) * C <= state_row,
+                "gdelta_chunks: rows of %zu or state rows of %zu are too short", ldp, state_row);
+    TFF_REQUIRE(H <= 65535 && R <= 65535, "gdelta_chunks: too many heads or requests");
+    TFF_REQUIRE((C + 2 * (size_t)H) * 17 < ((size_t)1 << 31), "gdelta_chunks: rows of %zu channels are too long", C);
+    if (R == 0) return 0;
+    hipStream_t s = (hipStream_t)stream;
+    gdelta_chunk_kernel<<<dim3((max_tokens + 15) / 16, H, R), 64, 0, s>>>(pre, cu_tokens, work, H, G, D, E);
+    if (int rc = tff_check_launch("gdelta_chunk")) return rc;
+    const dim3 grid(H, (E + 15) / 16, R);
+    TFF_REQUIRE(grid.y <= 65535, "gdelta_chunks: heads of %d value channels", E);
+#define GD_SCAN(NT, WV) gdelta_scan_kernel<NT, WV><<<grid, 64 * WV, 0, s>>>(pre, proj, ldp, state, state_row, tail_off, taps, cu_tokens, state_slots, work, o, H, G, E)
+    if (D == 64) GD_SCAN(1, 4);
+    else if (D == 128) GD_SCAN(2, 4);
+    else GD_SCAN(4, 4);
+#undef GD_SCAN
+    return tff_check_launch("gdelta_scan");
 }
 
 // One wave per (token, head): the head's E channels of o are divided by their root mean square, multiplied by

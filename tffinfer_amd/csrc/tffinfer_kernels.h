@@ -387,6 +387,15 @@ TFF_API int tff_gdelta_prep(const float* proj, size_t ldp, const float* wconv, i
 TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
                                   size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* o,
                                   int R, int H, int G, int D, int E, int max_tokens, tff_stream_t stream);
+// The same for long portions (max_tokens: the longest), in chunks of sixteen tokens on the float32 matrix cores: head sizes of
+// 64, 128 and 256, an even number of heads; work: tff_gdelta_chunks_workspace bytes.  A token's result depends on where its portion
+// began, beyond rounding it does not.
+TFF_API size_t tff_gdelta_chunks_workspace(int T, int R, int H);
+TFF_API int tff_gdelta_chunks_supported(int D, int E, size_t state_row);
+TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
+                                         size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* work,
+                                         float* o, int T, int R, int H, int G, int D, int E, int max_tokens, tff_stream_t stream);
+
 // out[t * out_row + h * E + e] = o[t, h, e] / sqrt(mean over e of o^2 + eps) * w[e] * silu(g[t * g_row + h * E + e]) * scale
 TFF_API int tff_head_norm_silu_gate(const float* o, const float* g, size_t g_row, const float* w, float eps, float scale,
                                     void* out, size_t out_row, int T, int H, int E, int out_dtype, tff_stream_t stream);
