@@ -820,6 +820,36 @@ def test_sample_ties_rows_off_alignment_and_batch_position():
         assert alone[0] == tok[r]
 
 
+@pytest.mark.parametrize("V", [16384, 16385, 20001, 151936])
+def test_sample_of_few_kept_tokens_is_that_of_the_passes(V):
+    """Rows with a small top_k by the maxima of their runs (few=True): the token that the passes over the row give, to the bit,
+    with top_p and min_p, over flat, peaked, tied, masked and broken rows, and where more is kept than fits."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(V)
+    rows = []
+    for scale in (0.0, 0.01, 1.0, 3.0, 30.0, 900.0):
+        rows += [torch.randn(V, generator=g) * scale for _ in range(5)]
+    tied = torch.randn(V, generator=g)
+    tied[torch.randperm(V, generator=g)[:700]] = 4.5                 # more ties at the top than candidates fit
+    rounded = (torch.randn(V, generator=g) * 4).round()
+    masked = torch.full((V,), float("-inf"))
+    masked[V - 3:] = torch.tensor([1.0, 0.5, 0.25])
+    broken = torch.randn(V, generator=g)
+    broken[7], broken[V - 1], broken[200:330] = float("nan"), float("inf"), float("nan")
+    nan = torch.randn(V, generator=g) * 2
+    nan[100:400] = float("nan")
+    rows += [tied, rounded, masked, broken, nan, torch.full((V,), float("-inf")), torch.arange(V).float() / V]
+    x = torch.stack(rows).to(DEV)
+    R = x.shape[0]
+    for k, p, mp, T, u in ((50, 0.95, 0.0, 0.8, 0.5), (1, 1.0, 0.0, 1.0, 0.9), (5, 0.3, 0.0, 2.5, 0.0), (100, 1.0, 0.02, 0.7, 0.999999),
+                           (256, 0.9, 0.0, 0.05, 0.31), (40, 0.0, 0.0, 1.0, 0.7), (20, 0.99, 1.5, 1.0, 0.2), (0, 0.9, 0.0, 1.0, 0.4),
+                           (130, 0.999, 0.0, 0.0, 0.6)):
+        num = lambda v, dt=torch.float32: torch.full((R,), v, dtype=dt, device=DEV)        # noqa: E731
+        us = (num(u) + torch.arange(R, device=DEV) * 0.017) % 1.0
+        args = (x, num(T), us, num(k, torch.int32), num(p), num(mp))
+        assert torch.equal(ops.sample(*args, few=True), ops.sample(*args)), (k, p, mp, T)
+
+
 def test_sample_refuses_a_vocabulary_beyond_its_layout():
     ops = _ops()
     from tffinfer_amd.kernels.lib import KernelError

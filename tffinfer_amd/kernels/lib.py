@@ -103,7 +103,7 @@ _SIGNATURES = {
     "tff_argmax_workspace_bytes": [_I, _I],
     "tff_argmax": [_P, _P, _I, _I, _P, _P],
     "tff_repetition_penalty": [_P, _I, _I, _P, _P, _P, _P],
-    "tff_sample": [_P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P],
+    "tff_sample": [_P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P],
     "tff_add_layernorm": [_P, _P, _I, _Z, _P, _I, _Z, _P, _P, _P, _F, _P, _P, _P, _F, _P, _P, _P, _F, _P, _P, _I, _I, _P, _I, _P, _Z,
                           _Z, _P, _P, _Z, _I, _P],
     "tff_input_conv": [_P, _P, _I, _P, _Z, _Z, _P, _I, _I, _P, _P, _P, _I, _I, _P],
