@@ -150,6 +150,44 @@ def test_recurrence_whole_and_in_portions(H, D):
         assert torch.equal(torch.cat(got, 0), whole)
 
 
+@pytest.mark.parametrize("H,D,portions", [(2, 64, (128,)), (3, 64, (129, 3, 250)), (1, 128, (145, 128)), (2, 128, (16, 15, 200))])
+def test_recurrence_in_chunks_of_sixteen(H, D, portions):
+    """Portions beside one another, the longest of 128 tokens and more, from states that are not zero, with rows
+    wider than the heads: against 64 bits, outputs, state and kept row; no other slot is touched.  A sum of some
+    D terms and a product of up to 16 decays, each kept to half a unit of 2^-23, stay under 16 such units."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(D + len(portions))
+    T, W, R = sum(portions), 8, len(portions)
+    wide = torch.randn(T, 4 * H * D, generator=g)
+    wide[:, 3 * H * D:] *= 3
+    w0 = torch.rand(H * D, generator=g) * 3.5 - 3
+    u = torch.randn(H * D, generator=g)
+    x = torch.randn(T, W, generator=g)
+    row = H * D * D + W
+    state = torch.randn(R + 2, row, generator=g)
+    start = state.clone().double()
+    dev, slots = wide.to(DEV), list(range(R, 0, -1))
+    state = state.to(DEV)
+    r, k, v, z = (dev[:, i * H * D:(i + 1) * H * D] for i in range(4))
+    o = ops.wkv_recurrence(r, k, v, z, w0.to(DEV), u.to(DEV), state, _batch(list(portions), [0] * R, slots), H, D, x=x.to(DEV),
+                           prev_off=H * D * D)
+    R64, K64, V64, Z64 = (t.double().view(T, H, D) for t in wide.split(H * D, 1))
+    w = torch.exp(-torch.exp(Z64 + w0.double().view(H, D)))
+    at = 0
+    for n, slot in zip(portions, slots):
+        S, out = start[slot, :H * D * D].view(H, D, D).clone(), []
+        for t in range(at, at + n):
+            kv = K64[t][:, :, None] * V64[t][:, None]
+            out.append((R64[t][:, :, None] * (S + u.double().view(H, D)[:, :, None] * kv)).sum(1))
+            S = w[t][:, :, None] * S + kv
+        assert _err(o[at:at + n], torch.stack(out).view(n, H * D)) < 16 * 2 ** -23
+        assert _err(state[slot, :H * D * D].view(H, D, D), S) < 16 * 2 ** -23
+        assert torch.equal(state[slot, H * D * D:].cpu(), x[at + n - 1])
+        at += n
+    for slot in (0, R + 1):
+        assert torch.equal(state[slot].cpu().double(), start[slot])
+
+
 @pytest.mark.parametrize("H,D", [(3, 8), (2, 40), (1, 128)])
 def test_norm_over_each_head_and_gate(H, D):
     ops = _ops()

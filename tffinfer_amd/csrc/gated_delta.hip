@@ -550,7 +550,7 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
     if (blockIdx.y == 0) gd_keep_inputs(proj, ldp, srow + tail_off, taps, t0, n, h, gk, H, G, D, E);
 }
 
-TFF_API size_t tff_gdelta_chunks_workspace(int T, int R, int H) { return ((size_t)T / 16 + R + 1) * H * GD_WORK * sizeof(float); }
+TFF_API size_t tff_gdelta_chunks_workspace_bytes(int T, int R, int H) { return ((size_t)T / 16 + R + 1) * H * GD_WORK * sizeof(float); }
 
 TFF_API int tff_gdelta_chunks_supported(int D, int E, size_t state_row) {
     return (D == 64 || D == 128 || D == 256) && E % 4 == 0 && state_row % 4 == 0;

@@ -16,6 +16,7 @@
 //   how the tokens were cut into steps beyond rounding (`long_portions` picks the form for prompts, whose
 //   sums run in another order than those of the form for single tokens).  The block of head 0 also
 //   leaves the portion's last row of x in the state.
+// tff_wkv_recurrence_chunks: the same in chunks of sixteen tokens on the float32 matrix cores, for heads of 64 and 128.
 // tff_head_norm_gate: out = o / sqrt(mean over the head of o^2 + eps) * weight * silu(g).
 // tff_tanh: out = tanh(in), float32 in, the activation type out.
 #include "common.h"
@@ -419,6 +420,258 @@ TFF_API int tff_wkv_recurrence(const float* r, const float* k, const float* v, c
 #undef WKV_WAVES
 #undef WKV_LAUNCH
     return tff_check_launch("wkv_recurrence");
+}
+
+// ------------------------------------------------- portions in chunks of sixteen tokens ---
+// For heads of 64 and 128.  Within a chunk that starts from S0, with F_t = w_0 .. w_(t-1) and P_ts = w_(s+1) .. w_(t-1) per key channel,
+//
+//   o_t = S0^T (F_t r_t) + sum over s < t of (sum over i of r_t[i] P_ts[i] k_s[i]) v_s + (sum over i of r_t[i] u[i] k_t[i]) v_t
+//   S  <- diag(w_0 .. w_15) S0 + sum over s of (w_(s+1) .. w_15 k_s) v_s^T
+//
+// No factor is a quotient (a running product of decays underflows): all are products of up to fifteen decays, formed where they are
+// used.  wkv_chunk_kernel works out what does not depend on S, a wave per chunk and head (lane (token, quarter of every sixteen channels);
+// the sums over channels for all pairs of tokens, walking s down from t while the product grows by one decay a step).
+// wkv_scan_kernel carries S through a request's chunks with products on the float32 matrix cores: a block per head and sixteen value
+// channels, a wave a quarter of the key channels with its part of S in its accumulators; the waves' parts of an output meet
+// in LDS.  S itself waits for one multiply-add a chunk.
+// A token after the other took 0.25 - 0.28 us a token, however wide the GPU: us, called from Python, before / now for 1,500 tokens of 64
+// heads of 64 374 / 92 (chunks 41, scan 47), of 16 heads of 128 652 / 110, of 4 heads of 64 297 / 62; four portions of 901, 700, 430 and
+// 300 tokens 280 / 129.  Relative error of the outputs against 64 bits 8.7e-8 / 6.7e-8 (heads of 128: 9.5e-8 / 6.8e-8).
+//
+// work: per chunk and head 16 rows of F_t r_t, 16 of w_(s+1) .. w_15 k_s, 16 x 16 weights of v, the chunk's decays; the chunk that
+// starts at token t of row r lies at place t / 16 + r.
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float wkv_floatx4;
+
+// from zero in two chains of eight terms that meet at the end: half the wait and a smaller error
+__device__ __forceinline__ wkv_floatx4 wkv_mfma16(const wkv_floatx4& a, const wkv_floatx4& b) {
+    const wkv_floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+    wkv_floatx4 x = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], b[0], zero, 0, 0, 0);
+    wkv_floatx4 y = __builtin_amdgcn_mfma_f32_16x16x4f32(a[2], b[2], zero, 0, 0, 0);
+    x = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], b[1], x, 0, 0, 0);
+    y = __builtin_amdgcn_mfma_f32_16x16x4f32(a[3], b[3], y, 0, 0, 0);
+    return x + y;
+}
+constexpr int wkv_work(int D) { return 33 * D + 256; }
+
+template <int D>
+__global__ __launch_bounds__(64) void wkv_chunk_kernel(const float* __restrict__ r, const float* __restrict__ k,
+                                                       const float* __restrict__ z, size_t row, const float* __restrict__ w0,
+                                                       const float* __restrict__ u, const int32_t* __restrict__ cu_tokens,
+                                                       float* __restrict__ work, int H) {
+    constexpr int M = D / 16, LDR = D + 4;
+    __shared__ __attribute__((aligned(16))) float ks[16 * LDR], ws[16 * LDR];
+    const int h = blockIdx.x, req = blockIdx.z, lane = threadIdx.x, c = lane & 15, g = lane >> 4;
+    const int t0 = cu_tokens[req], n = cu_tokens[req + 1] - t0, first = blockIdx.y * 16;
+    if (first >= n) return;
+    const bool live = first + c < n;                      // (tokens past the portion's end: no key, no decay)
+    const size_t at = (size_t)(t0 + min(first + c, n - 1)) * row + (size_t)h * D + 4 * g;
+    const float* up = u + (size_t)h * D + 4 * g;
+    const float* bp = w0 + (size_t)h * D + 4 * g;
+    wkv_floatx4 x[M], kk[M], w[M];
+    double own = 0.;                                      // r u k of the token itself
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        x[m] = *reinterpret_cast<const wkv_floatx4*>(r + at + 16 * m);
+        kk[m] = *reinterpret_cast<const wkv_floatx4*>(k + at + 16 * m);
+        w[m] = *reinterpret_cast<const wkv_floatx4*>(z + at + 16 * m);
+    }
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        const wkv_floatx4 b = *reinterpret_cast<const wkv_floatx4*>(bp + 16 * m), uu = *reinterpret_cast<const wkv_floatx4*>(up + 16 * m);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            w[m][e] = live ? expf(-expf(w[m][e] + b[e])) : 1.f;
+            kk[m][e] = live ? kk[m][e] : 0.f;
+            own = fma((double)x[m][e] * (double)uu[e], (double)kk[m][e], own);
+        }
+        *reinterpret_cast<wkv_floatx4*>(ks + c * LDR + 16 * m + 4 * g) = kk[m];
+        *reinterpret_cast<wkv_floatx4*>(ws + c * LDR + 16 * m + 4 * g) = w[m];
+    }
+    __syncthreads();
+    float* wp = work + ((size_t)((t0 + first) / 16 + req) * H + h) * wkv_work(D);
+    auto quarters = [](double a) {                        // the sum over the four lanes of a token
+        a += __shfl_xor(a, 16, 64);
+        return a + __shfl_xor(a, 32, 64);
+    };
+    own = quarters(own);
+    wkv_floatx4 att = {0.f, 0.f, 0.f, 0.f};
+    // (products and sums in 64 bits: up to fifteen roundings of a product would be seen in the results)
+    double p[M][4];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[m][e] = (double)x[m][e];
+#pragma unroll
+    for (int s = 15; s >= 0; --s) {
+        double a = 0.;
+        if (s < c) {
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const wkv_floatx4 y = *reinterpret_cast<const wkv_floatx4*>(ks + s * LDR + 16 * m + 4 * g);
+                const wkv_floatx4 d = *reinterpret_cast<const wkv_floatx4*>(ws + s * LDR + 16 * m + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    a = fma(p[m][e], (double)y[e], a);
+                    p[m][e] *= (double)d[e];
+                }
+            }
+        }
+        a = quarters(a);
+        if (s >> 2 == g) att[s & 3] = s < c ? (float)a : (s == c ? (float)own : 0.f);
+    }
+#pragma unroll
+    for (int m = 0; m < M; ++m) {                         // (p is r times all decays before its token by now)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[m][e] = (float)p[m][e];
+        *reinterpret_cast<wkv_floatx4*>(wp + c * D + 16 * m + 4 * g) = x[m];
+    }
+    *reinterpret_cast<wkv_floatx4*>(wp + 32 * D + c * 16 + 4 * g) = att;
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[m][e] = 1.;
+#pragma unroll
+    for (int j = 15; j > 0; --j)
+        if (j > c) {
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const wkv_floatx4 d = *reinterpret_cast<const wkv_floatx4*>(ws + j * LDR + 16 * m + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) p[m][e] *= (double)d[e];
+            }
+        }
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        wkv_floatx4 end;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            end[e] = (float)((double)w[m][e] * p[m][e]);
+            kk[m][e] = (float)((double)kk[m][e] * p[m][e]);
+        }
+        *reinterpret_cast<wkv_floatx4*>(wp + 16 * D + c * D + 16 * m + 4 * g) = kk[m];
+        if (c == 0) *reinterpret_cast<wkv_floatx4*>(wp + 32 * D + 256 + 16 * m + 4 * g) = end;
+    }
+}
+
+// Four waves of NT tiles of 16 key channels (D = 64 NT).  Four chunks between two barriers: after the barrier each wave has one
+// chunk's output to put together, so that no wave waits for another's.
+template <int NT>
+__global__ __launch_bounds__(256) void wkv_scan_kernel(const float* __restrict__ v, size_t row, float* __restrict__ state, size_t state_row,
+                                                       const int32_t* __restrict__ cu_tokens,
+                                                       const int32_t* __restrict__ state_slots, const float* __restrict__ work,
+                                                       float* __restrict__ o, int H, const float* __restrict__ x, int W, size_t prev_off) {
+    constexpr int D = 64 * NT;
+    __shared__ wkv_floatx4 part[2][4][4][64];              // by turns, chunk, wave
+    const int h = blockIdx.x, req = blockIdx.z, j0 = blockIdx.y * 16;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+    const int t0 = cu_tokens[req], n = cu_tokens[req + 1] - t0;
+    if (n <= 0) return;
+    float* srow = state + (size_t)state_slots[req] * state_row;
+    float* sp = srow + (size_t)h * D * D + (size_t)(wv * 16 * NT + 4 * g) * D + j0 + c;
+    wkv_floatx4 S[NT];
+#pragma unroll
+    for (int m = 0; m < NT; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[m][i] = sp[(size_t)(16 * m + i) * D];
+    struct Ops {
+        wkv_floatx4 r[NT], kt[NT], w[NT], v;
+    } ops[4];
+    // Addresses are a uniform base and a lane's 32-bit offset that is the same for all chunks but the last, whose tokens past the
+    // portion's end repeat its last one (their keys are zero).
+    const int chunks = (n + 15) / 16, last = n - 1 - 16 * (chunks - 1);
+    const char* wbase = (const char*)(work + ((size_t)(t0 / 16 + req) * H + h) * wkv_work(D));
+    const size_t wstep = (size_t)H * wkv_work(D) * 4;
+    const char* vbase = (const char*)(v + (size_t)t0 * row + (size_t)h * D + j0);
+    const unsigned ldv = (unsigned)row * 4u;
+    const unsigned in_r = (unsigned)(c * D + 4 * g + wv * 16 * NT) * 4u, in_k = (unsigned)(16 * D + 4 * g * D + c + wv * 16 * NT) * 4u;
+    const unsigned in_w = (unsigned)(32 * D + 256 + 4 * g + wv * 16 * NT) * 4u, in_a = (unsigned)(32 * D + c * 16 + 4 * g) * 4u;
+    auto fetch = [&](int i, Ops& q) {
+        const int most = i + 1 < chunks ? 15 : last;
+        const char* w = wbase + (size_t)i * wstep;
+        const char* vp = vbase + (size_t)i * 16 * ldv;
+#pragma unroll
+        for (int m = 0; m < NT; ++m) {
+            q.r[m] = *reinterpret_cast<const wkv_floatx4*>(w + (in_r + 64u * m));
+            q.w[m] = *reinterpret_cast<const wkv_floatx4*>(w + (in_w + 64u * m));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) q.kt[m][e] = *reinterpret_cast<const float*>(w + (in_k + (unsigned)(e * D + 16 * m) * 4u));
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            q.v[e] = *reinterpret_cast<const float*>(vp + ((unsigned)min(4 * g + e, most) * ldv + (unsigned)c * 4u));
+    };
+#pragma unroll
+    for (int a = 0; a < 4; ++a) fetch(min(a, chunks - 1), ops[a]);
+    int buf = 0;
+    for (int first = 0; first < chunks; first += 4, buf ^= 1) {
+        const int mine = first + wv;
+        const wkv_floatx4 att = *reinterpret_cast<const wkv_floatx4*>(wbase + (size_t)min(mine, chunks - 1) * wstep + in_a);
+        wkv_floatx4 vm = ops[0].v;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            Ops& now = ops[a];
+            if (a > 0 && wv == a) vm = now.v;
+            if (first + a < chunks) {
+                wkv_floatx4 y = wkv_mfma16(now.r[0], S[0]);
+#pragma unroll
+                for (int m = 1; m < NT; ++m) y = y + wkv_mfma16(now.r[m], S[m]);
+#pragma unroll
+                for (int m = 0; m < NT; ++m) {
+                    const wkv_floatx4 add = wkv_mfma16(now.kt[m], now.v);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) S[m][e] = fmaf(S[m][e], now.w[m][e], add[e]);
+                }
+                part[buf][a][wv][lane] = y;
+            }
+            fetch(min(first + 4 + a, chunks - 1), now);   // (past the end the last one again: a condition would make the waits exact for neither)
+        }
+        __syncthreads();                                  // (the other buffer was last read before this barrier)
+        if (mine < chunks) {
+            wkv_floatx4 y = (part[buf][wv][0][lane] + part[buf][wv][1][lane]) + (part[buf][wv][2][lane] + part[buf][wv][3][lane]);
+            y = wkv_mfma16(att, vm) + y;
+            float* op = o + (size_t)(t0 + 16 * mine + 4 * g) * H * D + (size_t)h * D + j0 + c;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (16 * mine + 4 * g + q < n) op[(size_t)q * H * D] = y[q];
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < NT; ++m)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sp[(size_t)(16 * m + e) * D] = S[m][e];
+    if (h == 0 && blockIdx.y == 0 && x) {
+        const float* lastx = x + (size_t)(t0 + n - 1) * W;
+        for (int e = tid; e < W; e += 256) srow[prev_off + e] = lastx[e];
+    }
+}
+
+TFF_API size_t tff_wkv_chunks_workspace_bytes(int T, int R, int H, int D) {
+    return ((size_t)T / 16 + R + 1) * H * wkv_work(D) * sizeof(float);
+}
+
+// As tff_wkv_recurrence, for heads of 64 and 128; max_tokens: the longest portion; row a multiple of 4 and r, k, z, w0, u and
+// work 16-byte aligned.
+TFF_API int tff_wkv_recurrence_chunks(const float* r, const float* k, const float* v, const float* z, size_t row, const float* w0,
+                                      const float* u, float* state, size_t state_row, const int32_t* cu_tokens,
+                                      const int32_t* state_slots, float* work, float* o, int T, int R, int H, int D, const float* x,
+                                      int W, size_t prev_off, int max_tokens, tff_stream_t stream) {
+    TFF_REQUIRE(r && k && v && z && w0 && u && state && cu_tokens && state_slots && work && o, "wkv_chunks: null pointer");
+    TFF_REQUIRE(R >= 0 && T >= 0 && H > 0 && max_tokens > 0 && (D == 64 || D == 128), "wkv_chunks: %d heads of %d (64 or 128)", H, D);
+    TFF_REQUIRE(row >= (size_t)H * D && row % 4 == 0 && (size_t)H * D * D <= state_row && (!x || prev_off + (size_t)W <= state_row),
+                "wkv_chunks: rows of %zu, state rows of %zu do not hold %d heads of %d", row, state_row, H, D);
+    TFF_REQUIRE(((uintptr_t)r % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)z % 16) == 0 && ((uintptr_t)w0 % 16) == 0 &&
+                ((uintptr_t)u % 16) == 0 && ((uintptr_t)work % 16) == 0, "wkv_chunks: operands must be 16-byte aligned");
+    TFF_REQUIRE(row < ((size_t)1 << 25), "wkv_chunks: rows of %zu are too long", row);
+    TFF_REQUIRE(R <= 65535 && max_tokens <= 16 * 65535, "wkv_chunks: too many requests or tokens");
+    if (R == 0) return 0;
+    hipStream_t s = (hipStream_t)stream;
+    const dim3 pieces(H, (max_tokens + 15) / 16, R), grid(H, D / 16, R);
+    if (D == 64) wkv_chunk_kernel<64><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, H);
+    else wkv_chunk_kernel<128><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, H);
+    if (int rc = tff_check_launch("wkv_chunk")) return rc;
+    if (D == 64) wkv_scan_kernel<1><<<grid, 256, 0, s>>>(v, row, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off);
+    else wkv_scan_kernel<2><<<grid, 256, 0, s>>>(v, row, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off);
+    return tff_check_launch("wkv_scan");
 }
 
 template <typename TO>

@@ -79,11 +79,13 @@ _SIGNATURES = {
     "tff_scale_rows": [_P, _F, _Z, _P],
     "tff_token_shift_mix": [_P, _P, _Z, _Z, _P, _I, _P, _P, _P, _P, _I, _I, _I, _P],
     "tff_wkv_recurrence": [_P, _P, _P, _P, _Z, _P, _P, _P, _Z, _P, _P, _P, _I, _I, _I, _P, _I, _Z, _I, _P],
+    "tff_wkv_chunks_workspace_bytes": [_I, _I, _I, _I],
+    "tff_wkv_recurrence_chunks": [_P, _P, _P, _P, _Z, _P, _P, _P, _Z, _P, _P, _P, _P, _I, _I, _I, _I, _P, _I, _Z, _I, _P],
     "tff_head_norm_gate": [_P, _P, _Z, _P, _F, _P, _I, _I, _I, _I, _P],
     "tff_tanh": [_P, _P, _Z, _I, _P],
     "tff_gdelta_prep": [_P, _Z, _P, _I, _P, _P, _P, _Z, _Z, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "tff_gdelta_recurrence": [_P, _P, _Z, _P, _Z, _Z, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
-    "tff_gdelta_chunks_workspace": [_I, _I, _I],
+    "tff_gdelta_chunks_workspace_bytes": [_I, _I, _I],
     "tff_gdelta_chunks_supported": [_I, _I, _Z],
     "tff_gdelta_recurrence_chunks": [_P, _P, _Z, _P, _Z, _Z, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "tff_head_norm_silu_gate": [_P, _P, _Z, _P, _F, _F, _P, _Z, _I, _I, _I, _I, _P],

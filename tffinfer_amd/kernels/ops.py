@@ -1028,7 +1028,8 @@ def paged_attention(q: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, windo
     # (the matrix-core kernels cap scores at head sizes up to 192)
     if mfma_attention_supported(q.dtype, d, kv.k_cache.shape[2]) and not (softcap and d > 192):
         return attention_mfma(q, nq, nkv, d, kv, batch, window, scale, sinks=sinks, softcap=softcap, pool=pool)
-    if not pool and attention_f32_supported(q, d, kv.k_cache.shape[2]):
+    if not pool and attention_f32_supported(q, d, kv.k_cache.shape[2]) \
+            and kv.k_cache.data_ptr() % 16 == 0 and kv.v_cache.data_ptr() % 16 == 0:
         return attention_f32(q, nq, nkv, d, kv, batch, window, scale, sinks=sinks, softcap=softcap)
     return attention_generic(q, nq, nkv, d, kv.k_cache, kv.v_cache, kv.block_tables,
                              batch.token_req, batch.positions, window, scale, sinks=sinks, softcap=softcap, pool=pool,
@@ -1414,6 +1415,12 @@ def token_shift_mix(x: torch.Tensor, state: torch.Tensor, prev_off: int, mu: tor
 WKV_LONG_PORTION = 16
 
 
+#: tokens of the longest portion from which heads of 64 and 128 run in chunks of sixteen on the matrix cores: two kernels and a
+#: workspace for one kernel.  Called from here, us for 96 tokens of 64 heads of 64 27 token by token, 22 - 29 in chunks; 128 33 / 23;
+#: 400 97 / 38
+WKV_CHUNKS_MIN_TOKENS = 128
+
+
 def wkv_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tensor, w0: torch.Tensor,
                    u: torch.Tensor, state: torch.Tensor, batch, H: int, D: int, x: torch.Tensor | None = None,
                    prev_off: int = 0) -> torch.Tensor:
@@ -1444,11 +1451,21 @@ def wkv_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.T
     o = torch.empty(T, HD, dtype=torch.float32, device=r.device)
     if T == 0:
         return o
+    longest = int(getattr(batch, "max_new_tokens", 0) or 0)
+    if longest >= WKV_CHUNKS_MIN_TOKENS and D in (64, 128) and r.stride(0) % 4 == 0 and r.stride(0) < 1 << 25 \
+            and all(t.data_ptr() % 16 == 0 for t in (r, k, z, w0, u)):
+        L = _lib.load()
+        work = torch.empty(L.tff_wkv_chunks_workspace_bytes(T, batch.num_reqs, H, D) // 4, dtype=torch.float32, device=r.device)
+        _lib.check(L.tff_wkv_recurrence_chunks(
+            r.data_ptr(), k.data_ptr(), v.data_ptr(), z.data_ptr(), r.stride(0), w0.data_ptr(), u.data_ptr(), state.data_ptr(), row,
+            batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), work.data_ptr(), o.data_ptr(), T, batch.num_reqs, H, D, _ptr(x), W,
+            int(prev_off), longest, _stream()))
+        return o
     _lib.check(_lib.load().tff_wkv_recurrence(r.data_ptr(), k.data_ptr(), v.data_ptr(), z.data_ptr(), r.stride(0),
                                               w0.data_ptr(), u.data_ptr(), state.data_ptr(), row,
                                               batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), o.data_ptr(),
                                               batch.num_reqs, H, D, _ptr(x), W, int(prev_off),
-                                              1 if getattr(batch, "max_new_tokens", 0) >= WKV_LONG_PORTION else 0, _stream()))
+                                              1 if longest >= WKV_LONG_PORTION else 0, _stream()))
     return o
 
 
@@ -2054,8 +2071,8 @@ def gated_delta(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, d
                                  state.data_ptr(), row, tail, batch.token_req.data_ptr(), batch.cu_tokens.data_ptr(),
                                  batch.state_slots.data_ptr(), pre.data_ptr(), T, H, G, D, E, stream))
     longest = int(getattr(batch, "max_new_tokens", 0) or 0)
-    if longest >= GDELTA_CHUNKS_MIN_TOKENS and H % 2 == 0 and L.tff_gdelta_chunks_supported(D, E, row):
-        work = torch.empty(L.tff_gdelta_chunks_workspace(T, batch.num_reqs, H) // 4, dtype=torch.float32, device=proj.device)
+    if longest >= GDELTA_CHUNKS_MIN_TOKENS and H % 2 == 0 and state.data_ptr() % 16 == 0 and L.tff_gdelta_chunks_supported(D, E, row):
+        work = torch.empty(L.tff_gdelta_chunks_workspace_bytes(T, batch.num_reqs, H) // 4, dtype=torch.float32, device=proj.device)
         _lib.check(L.tff_gdelta_recurrence_chunks(
             pre.data_ptr(), proj.data_ptr(), ldp, state.data_ptr(), row, tail, taps, batch.cu_tokens.data_ptr(),
             batch.state_slots.data_ptr(), work.data_ptr(), o.data_ptr(), T, batch.num_reqs, H, G, D, E, longest, stream))
