@@ -225,6 +225,29 @@ def test_delta_rule_in_chunks_of_sixteen(H, G, D, E, taps, extreme):
         assert float(state[1].abs().max()) == 0
 
 
+@pytest.mark.parametrize("H,G,D,E", [(2, 1, 64, 20), (4, 2, 128, 128), (2, 2, 256, 36), (4, 2, 16, 8)])
+def test_delta_rule_of_many_tokens_is_that_of_few(H, G, D, E):
+    """More tokens than the preparation takes one by one, in requests too short for the chunks, from states that are not zero:
+    the same bits as each request by itself, and the plain loop within the bound of that form."""
+    ops = _ops()
+    taps, ns = 4, [95, 1, 94, 2, 93, 95, 3, 90, 88, 60]
+    T = sum(ns)
+    proj, conv, a_log, dt = _delta_case(T, H, G, D, E, taps, D + E)
+    row = H * E * D + (taps - 1) * (2 * G * D + H * E)
+    row += -row % 4
+    dev, many = [x.to(DEV) for x in (conv, a_log, dt)], torch.zeros(len(ns), row, device=DEV)
+    first = many.normal_(generator=torch.Generator(device=DEV).manual_seed(D)).clone()
+    o = ops.gated_delta(proj.to(DEV), *dev, many, _batch(ns, [0] * len(ns), list(range(len(ns)))), H, G, D, E)
+    at = 0
+    for i, n in enumerate(ns):
+        one = ops.gated_delta(proj[at:at + n].to(DEV), *dev, first, _batch([n], [0], [i]), H, G, D, E)
+        assert torch.equal(one, o[at:at + n]) and torch.equal(first[i], many[i])
+        first[i].zero_()
+        again = ops.gated_delta(proj[at:at + n].to(DEV), *dev, first, _batch([n], [0], [i]), H, G, D, E)
+        assert _err(again, _plain_delta(proj[at:at + n], conv, a_log, dt, H, G, D, E)) < 3e-5
+        at += n
+
+
 @pytest.mark.parametrize("decode", [False, True])
 def test_a_value_written_far_back_is_read(decode):
     """Decay 1, beta 1, keys that are axes: the value written under an axis at the third token is what a query

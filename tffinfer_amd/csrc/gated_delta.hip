@@ -73,6 +73,89 @@ __global__ __launch_bounds__(64) void gdelta_prep_kernel(
     }
 }
 
+// The same for four taps and heads of whole float4, on rows of 16-byte alignment: LPT lanes share a head, four channels each, and a
+// group of them takes a run of RUN tokens, so that an input row is read RUN + 3 times by RUN tokens instead of four times
+// each, and the weights once a run.  A wave a token and head with 4-byte loads was bound by its instructions and by the turn of small
+// blocks: 2,048 tokens of 8,192 channels (134 MB to move, 22 us at the rate of a large copy) 92 us, now 37.  The convolution's four terms
+// and the factor of a unit vector, which a whole row of the results shares, are kept in 64 bits until they are rounded once.
+// A run is one token below GD_RUNS_FROM tokens, where waves count for more; the sums are the same: 1, 8 and 48 tokens 6.4, 5.3 and
+// 6.9 us before, 3.4, 4.4 and 5.4 now; 256 tokens 8.6 in runs of one, 11.9 in runs of four.
+#define GD_RUNS_FROM 512
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gd_floatx4;
+typedef __attribute__((__vector_size__(4 * sizeof(double)))) double gd_doublex4;
+
+template <int LPT, int RUN>
+__global__ __launch_bounds__(64) void gdelta_prep_runs_kernel(
+    const float* __restrict__ proj, size_t ldp, const float* __restrict__ wconv, const float* __restrict__ a_log,
+    const float* __restrict__ dt_bias, const float* __restrict__ state, size_t state_row, size_t tail_off,
+    const int32_t* __restrict__ token_req, const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ state_slots,
+    float* __restrict__ pre, int T, int H, int G, int D, int E) {
+    constexpr int GROUPS = 64 / LPT;
+    const int u = blockIdx.y, lane = threadIdx.x;
+    const int C = 2 * G * D + H * E;
+    const size_t ldq = (size_t)C + 2 * H;
+    if (u == 2 * G + H) {
+        const int first = blockIdx.x * GROUPS * RUN, count = min(GROUPS * RUN, T - first);
+        for (int x = lane; x < count * H; x += 64) {
+            const int t = first + x / H, h = x % H;
+            const float* row = proj + (size_t)t * ldp;
+            float* out = pre + (size_t)t * ldq;
+            const float b = row[C + h], a = row[C + H + h] + dt_bias[h];
+            const float sp = a > 20.f ? a : log1pf(expf(a));
+            out[C + h] = 1.0f / (1.0f + expf(-b));
+            out[C + H + h] = expf(-expf(a_log[h]) * sp);
+        }
+        return;
+    }
+    const int l = lane % LPT, t0 = (blockIdx.x * GROUPS + lane / LPT) * RUN;
+    const int n = u < 2 * G ? D : E, c0 = u < 2 * G ? u * D : 2 * G * D + (u - 2 * G) * E;
+    const bool live = 4 * l < n;
+    const int c = c0 + (live ? 4 * l : 0);
+    gd_floatx4 rows[RUN + 3];
+#pragma unroll
+    for (int q = 0; q < RUN + 3; ++q) {                 // (rows before the step and past it are read as its first and last and not used)
+        const int t = min(max(t0 - 3 + q, 0), T - 1);
+        rows[q] = *reinterpret_cast<const gd_floatx4*>(proj + (size_t)t * ldp + c);
+    }
+    gd_floatx4 w[4];                                       // by channel
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = *reinterpret_cast<const gd_floatx4*>(wconv + (size_t)(c + e) * 4);
+#pragma unroll
+    for (int q = 0; q < RUN; ++q) {
+        const int t = min(t0 + q, T - 1);
+        const int r = token_req[t], i = t - cu_tokens[r];  // the token's place in its request's portion
+        gd_floatx4 x[4] = {rows[q], rows[q + 1], rows[q + 2], rows[q + 3]};
+        if (i < 3) {                                       // inputs before the portion are the state's
+            const float* tail = state + (size_t)state_slots[r] * state_row + tail_off;
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                if (i - 3 + k < 0) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[k][e] = tail[(size_t)(i + k) * C + c + e];
+                }
+        }
+        gd_floatx4 y;
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            double acc = 0.;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc = fma((double)w[e][k], (double)x[k][e], acc);
+            y[e] = gd_silu((float)acc);
+            ss = fmaf(y[e], y[e], ss);
+        }
+        if (u < 2 * G) {
+            ss = live ? ss : 0.f;
+#pragma unroll
+            for (int m = 1; m < LPT; m *= 2) ss += __shfl_xor(ss, m, 64);
+            const double f = 1.0 / sqrt(((double)ss + 1e-6) * (u < G ? (double)D : 1.0));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = (float)((double)y[e] * f);
+        }
+        if (live && t0 + q < T) *reinterpret_cast<gd_floatx4*>(pre + (size_t)t * ldq + c) = y;
+    }
+}
+
 TFF_API int tff_gdelta_prep(const float* proj, size_t ldp, const float* wconv, int taps, const float* a_log,
                             const float* dt_bias, const float* state, size_t state_row, size_t tail_off,
                             const int32_t* token_req, const int32_t* cu_tokens, const int32_t* state_slots, float* pre,
@@ -87,6 +170,23 @@ TFF_API int tff_gdelta_prep(const float* proj, size_t ldp, const float* wconv, i
                 "gdelta_prep: rows of %zu or state rows of %zu are too short", ldp, state_row);
     TFF_REQUIRE(2 * G + H + 1 <= 65535, "gdelta_prep: too many heads");
     if (T == 0) return 0;
+    const int widest = D > E ? D : E;
+    if (taps == 4 && D % 4 == 0 && E % 4 == 0 && H % 2 == 0 && widest <= 256 && ldp % 4 == 0 && ((uintptr_t)proj % 16) == 0 &&
+        ((uintptr_t)wconv % 16) == 0 && ((uintptr_t)pre % 16) == 0) {
+#define GD_RUNS(LPT, RUN)                                                                                                     \
+    gdelta_prep_runs_kernel<LPT, RUN><<<dim3((T + 64 / LPT * RUN - 1) / (64 / LPT * RUN), 2 * G + H + 1), 64, 0,               \
+                                        (hipStream_t)stream>>>(proj, ldp, wconv, a_log, dt_bias, state, state_row, tail_off,   \
+                                                               token_req, cu_tokens, state_slots, pre, T, H, G, D, E)
+        if (T < GD_RUNS_FROM) {
+            if (widest <= 64) GD_RUNS(16, 1);
+            else if (widest <= 128) GD_RUNS(32, 1);
+            else GD_RUNS(64, 1);
+        } else if (widest <= 64) GD_RUNS(16, 4);
+        else if (widest <= 128) GD_RUNS(32, 4);
+        else GD_RUNS(64, 4);
+#undef GD_RUNS
+        return tff_check_launch("gdelta_prep_runs");
+    }
     gdelta_prep_kernel<<<dim3(T, 2 * G + H + 1), 64, 0, (hipStream_t)stream>>>(
         proj, ldp, wconv, taps, a_log, dt_bias, state, state_row, tail_off, token_req, cu_tokens, state_slots, pre, H, G, D, E);
     return tff_check_launch("gdelta_prep");
@@ -339,28 +439,22 @@ TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ld
 // depend on S: gdelta_chunk_kernel forms them for all chunks at once, a wave per chunk and head (the inverse by forward
 // substitution, a lane a column; its elements are beta_s k_t' (product of reflections) k_s, at most 1 in size).
 // gdelta_scan_kernel walks the chunks of a request: a block per head and sixteen value channels, a wave a quarter of the key
-// channels, whose part of S stays in its accumulators; the waves' parts of K S0 and Q S0 meet in LDS, one barrier a chunk, and the
-// next chunk's operands are on their way meanwhile.  Accumulators are operands as they are: lane (column r, g) holds rows 4 g ..
-// 4 g + 3 of a product, which is where the next product's MFMA j wants row 4 g + j.
-// One token after the other took 0.25 us a token: 2,048 tokens of 32 heads of 128 x 128 in 515 us, now 17 + 196; 2,048 tokens of 4 heads
-// of 64 x 64 400 / 110; four requests of 901, 700, 430 and 300 tokens, with the preparation, 428 / 295.  The relative error against 64
-// bits is 1.3e-7 (1.2e-7 token by token).
+// channels, whose part of S stays in its accumulators; the waves' parts of K S0 meet in LDS, one barrier a chunk (those of Q S0 once
+// every four chunks, for which the waves then put one output together each), and the next chunks' operands are on their way
+// meanwhile.  Accumulators are operands as they are: lane (column r, g) holds rows 4 g .. 4 g + 3 of a product, which is where the
+// next product's MFMA j wants row 4 g + j.
+// One token after the other took 0.25 us a token: 2,048 tokens of 32 heads of 128 x 128 in 540 us, now 21 + 188; with the preparation,
+// 2,048 tokens of 4 heads of 64 x 64 438 / 129, four requests of 901, 700, 430 and 300 tokens 420 / 245.  Relative error against 64
+// bits over 96 to 400 tokens, with the preparation: heads of 64 1.26e-7 before, 1.11e-7 now; of 128 1.18e-7, 1.02e-7; of 256
+// 1.02e-7, 0.97e-7.
 //
 // work: per chunk and head 16 x 16 of (I + L)^-1 B, 16 x 16 of A, 16 G, 16 P_15,s; the chunk that starts at token t of row r
 // lies at place t / 16 + r.
 #define GD_WORK 544
 
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gd_floatx4;
 
-__device__ __forceinline__ gd_floatx4 gd_mfma16(const float4& a, const gd_floatx4& b, gd_floatx4 c) {
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[0], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[1], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[2], c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[3], c, 0, 0, 0);
-}
-
-// The same from zero in two chains of eight terms, which meet at the end: half the wait and a smaller error.
-__device__ __forceinline__ gd_floatx4 gd_mfma16_halves(const float4& a, const gd_floatx4& b) {
+// From zero in two chains of eight terms, which meet at the end: half the wait and a smaller error.
+__device__ __forceinline__ gd_floatx4 gd_mfma16(const float4& a, const gd_floatx4& b) {
     const gd_floatx4 zero = {0.f, 0.f, 0.f, 0.f};
     gd_floatx4 x = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[0], zero, 0, 0, 0);
     gd_floatx4 y = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[2], zero, 0, 0, 0);
@@ -371,7 +465,7 @@ __device__ __forceinline__ gd_floatx4 gd_mfma16_halves(const float4& a, const gd
 
 __global__ __launch_bounds__(64) void gdelta_chunk_kernel(const float* __restrict__ pre, const int32_t* __restrict__ cu_tokens,
                                                           float* __restrict__ work, int H, int G, int D, int E) {
-    __shared__ float sl[16][17];
+    __shared__ double sl[16][17];
     const int h = blockIdx.y, r = blockIdx.z, lane = threadIdx.x, c = lane & 15, g = lane >> 4;
     const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0, first = blockIdx.x * 16;
     if (first >= n) return;
@@ -381,49 +475,49 @@ __global__ __launch_bounds__(64) void gdelta_chunk_kernel(const float* __restric
     const float* row = pre + (size_t)(t0 + min(tok, n - 1)) * ldq;
     const float* kp = row + (size_t)(G + gk) * D + 4 * g;
     const float* qp = row + (size_t)gk * D + 4 * g;
-    gd_floatx4 kk = {0.f, 0.f, 0.f, 0.f}, qk = {0.f, 0.f, 0.f, 0.f};
-    for (int d = 0; d < D; d += 32) {                     // (short chains, added up: a sum of D terms in one chain loses a bit more)
-        gd_floatx4 ks[2], qs[2];
+    // (in 64 bits all of it, here and below: what is rounded here is rounded in whole rows of the results.
+    // v_mfma_f64_16x16x4_f64 leaves lane (column c, g) the rows g + 4 i.)
+    gd_doublex4 kk = {0., 0., 0., 0.}, qk = {0., 0., 0., 0.};
+    for (int d = 0; d < D; d += 32) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const float4 k4 = *reinterpret_cast<const float4*>(kp + d + 16 * i), q4 = *reinterpret_cast<const float4*>(qp + d + 16 * i);
-            const gd_floatx4 kb = {k4.x, k4.y, k4.z, k4.w};
-            ks[i] = gd_mfma16(k4, kb, gd_floatx4{0.f, 0.f, 0.f, 0.f});      // lane: k_t . k_s, s = c, t = 4 g + i
-            qs[i] = gd_mfma16(q4, kb, gd_floatx4{0.f, 0.f, 0.f, 0.f});
+            const gd_floatx4 k4 = *reinterpret_cast<const gd_floatx4*>(kp + d + 16 * i), q4 = *reinterpret_cast<const gd_floatx4*>(qp + d + 16 * i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                kk = __builtin_amdgcn_mfma_f64_16x16x4f64((double)k4[e], (double)k4[e], kk, 0, 0, 0);      // k_t . k_s, s = c
+                qk = __builtin_amdgcn_mfma_f64_16x16x4f64((double)q4[e], (double)k4[e], qk, 0, 0, 0);
+            }
         }
-        kk = kk + (ks[0] + ks[1]);
-        qk = qk + (qs[0] + qs[1]);
     }
     // (tokens past the portion's end: beta 0, no decay)
     const float beta = tok < n ? row[C + h] : 0.f, dec = tok < n ? row[C + H + h] : 1.f;
-    // (in 64 bits: sixteen roundings of one factor would be one error of a whole row of the results)
     double p[4] = {1., 1., 1., 1.}, gt = 1., pe = 1.;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         const double x = (double)__shfl(dec, j, 64);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) p[i] *= (j > c && j <= 4 * g + i) ? x : 1.;
+        for (int i = 0; i < 4; ++i) p[i] *= (j > c && j <= g + 4 * i) ? x : 1.;
         gt *= j <= c ? x : 1.;
         pe *= j > c ? x : 1.;
     }
     float* w = work + ((size_t)((t0 + first) / 16 + r) * H + h) * GD_WORK;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int t = 4 * g + i;
+        const int t = g + 4 * i;
         const float bt = __shfl(beta, t, 64);
-        sl[t][c] = c < t ? bt * (float)p[i] * kk[i] : 0.f;
-        w[256 + t * 16 + c] = c <= t ? (float)p[i] * qk[i] : 0.f;
+        sl[t][c] = c < t ? (double)bt * p[i] * kk[i] : 0.;
+        w[256 + t * 16 + c] = c <= t ? (float)(p[i] * qk[i]) : 0.f;
     }
     __syncthreads();
     if (lane < 16) {
-        float x[16];
+        double x[16];
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
-            float a = t == c ? 1.f : 0.f;
+            double a = t == c ? 1. : 0.;
 #pragma unroll
-            for (int s = 0; s < t; ++s) a = fmaf(-sl[t][s], x[s], a);
+            for (int s = 0; s < t; ++s) a = fma(-sl[t][s], x[s], a);
             x[t] = a;
-            w[t * 16 + c] = a * beta;
+            w[t * 16 + c] = (float)(a * (double)beta);
         }
         w[512 + c] = (float)gt;
         w[528 + c] = (float)pe;
@@ -438,7 +532,7 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
                                                           const int32_t* __restrict__ state_slots, const float* __restrict__ work,
                                                           float* __restrict__ o, int H, int G, int E) {
     constexpr int D = 16 * WV * NT;
-    __shared__ gd_floatx4 part[2][2][WV][64];
+    __shared__ gd_floatx4 px[2][WV][64], py[2][WV][WV][64];      // parts of K S0 by turns; of Q S0 by turns and chunk
     const int h = blockIdx.x, r = blockIdx.z, j0 = blockIdx.y * 16;      // (a head's blocks on one XCD: they read the same keys and queries)
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
     const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0;
@@ -500,37 +594,49 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
             for (int w = 0; w < WV; w += 2 * k) v[w] = v[w] + v[w + k];
         return v[0];
     };
+    // The outputs hang off the chain from chunk to chunk: each wave puts one of WV chunks' together once all of them are through.
+    gd_floatx4 own_u = {0.f, 0.f, 0.f, 0.f}, own_gt = own_u;
+    float4 own_att = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto outputs = [&](int first) {
+        const int mine = first + wv;
+        if (mine >= chunks) return;
+        const gd_floatx4 y = gd_mfma16(own_att, own_u) + own_gt * meet(py[first / WV & 1][wv]);
+        float* op = ocol + (size_t)(16 * mine + 4 * g) * H * E;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (live && 16 * mine + 4 * g + q < n) op[(size_t)q * H * E] = y[q];
+    };
     auto chunk = [&](const Ops& now, Ops& ahead) {
         fetch(min(i + 2, chunks - 1), ahead);      // (past the end the last one again: with a condition the wait for a chunk would be one for all)
         const int buf = i & 1;
-        gd_floatx4 x = gd_mfma16_halves(now.k[0], S[0]), y = gd_mfma16_halves(now.q[0], S[0]);
+        gd_floatx4 x = gd_mfma16(now.k[0], S[0]), y = gd_mfma16(now.q[0], S[0]);
 #pragma unroll
         for (int m = 1; m < NT; ++m) {
-            x = x + gd_mfma16_halves(now.k[m], S[m]);
-            y = y + gd_mfma16_halves(now.q[m], S[m]);
+            x = x + gd_mfma16(now.k[m], S[m]);
+            y = y + gd_mfma16(now.q[m], S[m]);
         }
-        part[buf][0][wv][lane] = x;
-        part[buf][1][wv][lane] = y;
-        __syncthreads();          // (the other buffer was last read before this barrier)
-        x = meet(part[buf][0]);
+        px[buf][wv][lane] = x;
+        py[i / WV & 1][i % WV][wv][lane] = y;
+        __syncthreads();          // (the other buffers were last read before this barrier)
+        x = meet(px[buf]);
         const gd_floatx4 gt = {now.gt.x, now.gt.y, now.gt.z, now.gt.w};
         gd_floatx4 v = {now.v[0], now.v[1], now.v[2], now.v[3]};
         v = v - gt * x;
-        const gd_floatx4 u = gd_mfma16_halves(now.inv, v);
+        const gd_floatx4 u = gd_mfma16(now.inv, v);
         const float gend = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(now.gt.w), 48));      // G_15: the whole chunk's decay
 #pragma unroll
         for (int m = 0; m < NT; ++m) {
             const float4 kt = make_float4(now.kt[m][0] * now.pe.x, now.kt[m][1] * now.pe.y, now.kt[m][2] * now.pe.z, now.kt[m][3] * now.pe.w);
-            S[m] = gd_mfma16(kt, u, S[m] * gend);
-        }
-        if (wv == i % WV) {                               // the waves take turns at the outputs
-            y = meet(part[buf][1]);
-            y = gd_mfma16_halves(now.att, u) + gt * y;
-            float* op = ocol + (size_t)(16 * i + 4 * g) * H * E;
+            const gd_floatx4 add = gd_mfma16(kt, u);
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (live && 16 * i + 4 * g + q < n) op[(size_t)q * H * E] = y[q];
+            for (int e = 0; e < 4; ++e) S[m][e] = fmaf(S[m][e], gend, add[e]);
         }
+        if (wv == i % WV) {
+            own_u = u;
+            own_gt = gt;
+            own_att = now.att;
+        }
+        if (i % WV == WV - 1) outputs(i - (WV - 1));
         ++i;
     };
     fetch(0, x0);
@@ -543,6 +649,7 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
         chunk(x2, x1);
         if (i >= chunks) break;
     }
+    if (chunks % WV != 0) outputs(chunks - chunks % WV);
     if (live) {
 #pragma unroll
         for (int m = 0; m < NT; ++m) *reinterpret_cast<gd_floatx4*>(sp + 16 * m) = S[m];
