@@ -150,6 +150,29 @@ def test_recurrence_whole_and_in_portions(H, D):
         assert torch.equal(torch.cat(got, 0), whole)
 
 
+@pytest.mark.parametrize("group", [1, 255, 257, 512, 513, 1025, 2048, 2049, 2600])
+def test_output_norm_and_depth_at_the_edges_of_a_block(group):
+    """Groups around the sizes at which a thread has one element more, as a sum of planes; the sum over the depth of rows that
+    are whole float4 and of rows that are not.  A float32 sum of n terms in chains of n / 256 and a tree is within 2^-24 (n / 256 + 10)
+    of its size, the planes' and the levels' sums within 2^-24 of each addition: 32 times 2^-24 covers both."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(group)
+    n, groups, planes, levels = 3, 2, 5, 11
+    H = groups * group
+    d, x = torch.randn(planes, n, H, generator=g), torch.randn(n, H, generator=g)
+    w, hist, coef = torch.randn(H, generator=g), torch.randn(levels, n, H, generator=g), torch.rand(levels, generator=g)
+    resid = x.to(DEV)
+    ops.group_rmsnorm_add(resid, d.to(DEV), w.to(DEV), groups, 1e-6, None)
+    y = d.double().sum(0).view(n, groups, group)
+    y = (y / torch.sqrt((y * y).mean(-1, keepdim=True) + 1e-6)).view(n, H) * w.double() + x.double()
+    assert _err(resid, y) < 32 * 2 ** -24
+    at, deep = x.to(DEV), hist.to(DEV)
+    ops.depth_average(deep, levels, coef.to(DEV), at, torch.bfloat16)
+    want = (coef[:-1, None, None].double() * hist[:-1].double()).sum(0) + coef[-1].double() * x.double()
+    assert _err(at, want) < 32 * 2 ** -24
+    assert torch.equal(deep[-1].cpu(), x) and torch.equal(deep[:-1].cpu(), hist[:-1])
+
+
 @pytest.mark.parametrize("H,D,portions", [(2, 64, (128,)), (3, 64, (129, 3, 250)), (1, 128, (145, 128)), (2, 128, (16, 15, 200))])
 def test_recurrence_in_chunks_of_sixteen(H, D, portions):
     """Portions beside one another, the longest of 128 tokens and more, from states that are not zero, with rows
