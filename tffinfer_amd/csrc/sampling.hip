@@ -7,7 +7,8 @@
 // min_p are fields of its SamplingConfig (LLMSampler.h:55-63).  Here one block
 // works on one row of float32 logits.  Thresholds are found by a radix search
 // over the bit patterns of the unnormalised probabilities e_i = exp((l_i - max)/temp)
-// instead of a sort (histograms of 11, 11 and 8 bits: two passes over the row as a rule);
+// instead of a sort (histograms of 11, 11 and 8 bits: two passes over the row as a rule; under a small
+// top_k of a large vocabulary over the runs of the row alone whose maxima can be among its tokens);
 // sums that decide a threshold or the drawn index are sums of integers, so the same
 // row and the same uniform number give the same token in any batch.
 #include "common.h"

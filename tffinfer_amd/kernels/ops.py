@@ -1452,7 +1452,7 @@ def wkv_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.T
     if T == 0:
         return o
     longest = int(getattr(batch, "max_new_tokens", 0) or 0)
-    if longest >= WKV_CHUNKS_MIN_TOKENS and D in (64, 128) and r.stride(0) % 4 == 0 and r.stride(0) < 1 << 25 \
+    if WKV_CHUNKS_MIN_TOKENS <= longest < 1 << 20 and D in (64, 128) and r.stride(0) % 4 == 0 and r.stride(0) < 1 << 25 \
             and all(t.data_ptr() % 16 == 0 for t in (r, k, z, w0, u)):
         L = _lib.load()
         work = torch.empty(L.tff_wkv_chunks_workspace_bytes(T, batch.num_reqs, H, D) // 4, dtype=torch.float32, device=r.device)
