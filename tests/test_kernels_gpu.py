@@ -977,6 +977,28 @@ def test_attention_f32(nq, nkv, d, ps, window, cap, sink, entries, cols):
             _close(out.reshape(T, nq, d)[sel], _attn_ref(q[sel], ks[r], vs[r], positions[sel], window, scale), 4e-6, f"row {r}")
 
 
+@pytest.mark.parametrize("window", [1, 17, 40])
+@pytest.mark.parametrize("entries", [[(100, 9), (61, 1), (0, 70)], [(100, 1), (61, 1)]])
+def test_attention_f32_looks_up_no_page_before_the_window(entries, window):
+    """Entries of the table for pages that a window has given back name no page (-1): the general kernel does not look at
+    them, nor does this one, although it walks the keys in steps of 32.  The place that a page -1 would have holds NaN."""
+    ops = _ops()
+    nq, nkv, d, ps = 8, 2, 64, 8
+    batch, kv, ks, vs, positions, token_req = _fake_step(entries, ps, nkv, d, torch.float32, seed=window)
+    for name in ("k_cache", "v_cache"):
+        pages = getattr(kv, name)
+        guarded = torch.full((pages.shape[0] + 1, *pages.shape[1:]), float("nan"), device=DEV)
+        guarded[1:] = pages
+        setattr(kv, name, guarded[1:])
+    for r, (P, _) in enumerate(entries):
+        kv.block_tables[r, :max(0, P - window + 1) // ps] = -1
+    q = torch.randn(batch.num_tokens, nq, d, generator=torch.Generator().manual_seed(5))
+    out = ops.attention_f32(q.reshape(batch.num_tokens, nq * d).to(DEV), nq, nkv, d, kv, batch, window)
+    for r in range(len(entries)):
+        sel = (token_req == r).nonzero().flatten()
+        _close(out.reshape(-1, nq, d)[sel], _attn_ref(q[sel], ks[r], vs[r], positions[sel], window, 1 / math.sqrt(d)), 4e-6, f"row {r}")
+
+
 @pytest.mark.parametrize("bins,groups", [(None, None), (3, 2), (1, 2), (None, 1), (3, 1), (1, 1)])
 @pytest.mark.parametrize("nq,nkv,d,ps,window", [
     (32, 8, 128, 16, 0), (8, 2, 32, 8, 300), (6, 3, 48, 8, 0), (5, 1, 128, 32, 0), (40, 2, 96, 8, 77),

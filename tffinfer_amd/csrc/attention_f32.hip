@@ -80,7 +80,7 @@ __global__ __launch_bounds__(64 * WQ * WK, 2) void attention_f32_kernel(
             af_floatx4 sc[NC][2];
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
-                const int key = min(k + 16 * f + r, last_pos);       // (never past what the request holds)
+                const int key = min(max(k + 16 * f + r, lo_min), last_pos);      // (no page outside of what some column sees is looked up)
                 const float* kp = k_cache + (((size_t)bt[key >> ps_shift] * nkv + g_kv) * ps + (key & (ps - 1))) * D + 4 * g;
                 float4 kf[DF];
 #pragma unroll
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(64 * WQ * WK, 2) void attention_f32_kernel(
             }
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
-                const int quad = k + 16 * f + 4 * g, key = min(quad, last_pos & ~3);
+                const int quad = k + 16 * f + 4 * g, key = min(max(quad, lo_min & ~3), last_pos & ~3);
                 const float* vp = v_cache + ((size_t)bt[key >> ps_shift] * nkv + g_kv) * ps * D + (key & (ps - 1)) + (size_t)r * ps;
                 float4 vf[DF];
 #pragma unroll
