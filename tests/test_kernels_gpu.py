@@ -977,6 +977,45 @@ def test_attention_f32(nq, nkv, d, ps, window, cap, sink, entries, cols):
             _close(out.reshape(T, nq, d)[sel], _attn_ref(q[sel], ks[r], vs[r], positions[sel], window, scale), 4e-6, f"row {r}")
 
 
+@pytest.mark.parametrize("nq,nkv,d,ps,window,cap,sink", [
+    (4, 2, 16, 16, 0, 0, False), (8, 2, 32, 8, 24, 0, True), (32, 8, 128, 16, 0, 5.0, False), (5, 5, 80, 32, 33, 0, False),
+    (16, 8, 112, 4, 40, 0, True), (40, 2, 96, 8, 0, 0, False), (4, 1, 192, 16, 100, 0, True), (20, 1, 256, 64, 0, 3.0, False)])
+def test_attention_f32_gives_a_token_the_same_bits_in_any_step(nq, nkv, d, ps, window, cap, sink):
+    """A request beside others, alone, cut into portions, token by token, and in blocks of 16 and of 128 columns: the same bits."""
+    from types import SimpleNamespace
+    ops = _ops()
+    entries = [(0, 300), (513, 41), (260, 1), (0, 1), (31, 2)]
+    batch, kv, ks, vs, positions, token_req = _fake_step(entries, ps, nkv, d, torch.float32, seed=nq + d)
+    g = torch.Generator().manual_seed(3)
+    q = torch.randn(batch.num_tokens, nq * d, generator=g).to(DEV)
+    sinks = torch.randn(nq, generator=g).to(DEV) if sink else None
+
+    def step(parts, cols=None):
+        """parts: (request, its first token in the step above, tokens)."""
+        cu, start, rows = [0], [], []
+        for r, first, n in parts:
+            cu.append(cu[-1] + n)
+            start.append(entries[r][0] + first)
+            rows += list(range(batch.host_cu_tokens[r] + first, batch.host_cu_tokens[r] + first + n))
+        b = SimpleNamespace(num_reqs=len(parts), num_tokens=cu[-1], max_new_tokens=max(n for _, _, n in parts), host_cu_tokens=cu,
+                            host_start_pos=start, cu_tokens=torch.tensor(cu, dtype=torch.int32, device=DEV),
+                            start_pos=torch.tensor(start, dtype=torch.int32, device=DEV))
+        view = SimpleNamespace(k_cache=kv.k_cache, v_cache=kv.v_cache, block_tables=kv.block_tables[[r for r, _, _ in parts]].contiguous())
+        return ops.attention_f32(q[rows].contiguous(), nq, nkv, d, view, b, window, None, sinks, cap, cols=cols), rows
+
+    all_of = [(r, 0, n) for r, (_, n) in enumerate(entries)]
+    whole, _ = step(all_of)
+    ways = [[p] for p in all_of] + [[(0, a, n), (1, a // 8, 3)] for a, n in ((0, 7), (7, 129), (136, 33), (169, 131))]
+    ways += [[(0, t, 1), (1, 40, 1)] for t in (0, 31, 32, 170, 255, 256, 299)] + [[(1, t, 1), (2, 0, 1), (3, 0, 1)] for t in (0, 17, 40)]
+    for parts in ways:
+        got, rows = step(parts)
+        assert torch.equal(got, whole[rows]), parts
+    if d <= 128:
+        for parts in (all_of, [(0, 13, 200)], [(0, 0, 130), (1, 5, 30)]):
+            got, rows = step(parts, cols=128)
+            assert torch.equal(got, whole[rows]), parts
+
+
 @pytest.mark.parametrize("window", [1, 17, 40])
 @pytest.mark.parametrize("entries", [[(100, 9), (61, 1), (0, 70)], [(100, 1), (61, 1)]])
 def test_attention_f32_looks_up_no_page_before_the_window(entries, window):

@@ -123,12 +123,12 @@ TFF_API int tff_attention_generic(const void* q, int q_stride, void* out,
 // of a power of two of at least four tokens (tff_attention_f32_supported), without keys of blocks.  Row i's tokens are
 // cu_tokens[i] .. cu_tokens[i + 1] - 1 at positions from start_pos[i] on.  work: int32 [items, 2] (row, first column) of
 // tiles of `cols` columns (16, or 128 for head sizes up to 128), a column being a (token, q head of the group) pair
-// numbered token * group + head; or null: every row has `tiles` tiles of 16 from column 0 on.  alone: every row brings
-// one token (eight waves share its keys).
+// numbered token * group + head; or null: every row has `tiles` tiles of 16 from column 0 on.  A token's result is the same bits
+// whatever else the step holds and however its request was cut into portions.
 TFF_API int tff_attention_f32_supported(int d, int page_size);
 TFF_API int tff_attention_f32(const void* q, int q_stride, void* out, const void* k_cache, const void* v_cache,
                               const int32_t* block_tables, int bt_stride, const int32_t* cu_tokens, const int32_t* start_pos,
-                              const int32_t* work, int items, int tiles, int cols, int alone, int nq, int nkv, int d, int page_size,
+                              const int32_t* work, int items, int tiles, int cols, int nq, int nkv, int d, int page_size,
                               int num_pages, int window, float scale, const float* sinks, float softcap, tff_stream_t stream);
 
 // bfloat16 attention on the matrix cores.  A wave works on `cols_per_wave` (16)

@@ -534,10 +534,10 @@ def attention_f32_supported(q: torch.Tensor, d: int, page_size: int) -> bool:
             and bool(_lib.load().tff_attention_f32_supported(int(d), int(page_size))))
 
 
-#: tiles of 16 columns x kv heads from which prompts take blocks of 128 columns (four waves that walk the same keys,
-#: two column tiles each) instead of blocks of 16 whose four waves share the keys: 4,096 tokens of 32 heads on 8 (8,192 tiles)
-#: 1,477 against 1,600 us, 2,048 tokens (4,096 tiles) 522 against 434
-F32_WIDE_TILES = 8192
+#: tiles of 16 columns x kv heads from which a step takes blocks of 128 columns (four waves that walk the same keys, two column
+#: tiles each) instead of blocks of 16 whose waves share the keys; the results are the same bits.  us on 16 / 128, 32 heads of 128 on 8:
+#: 2,048 tokens (4,096 tiles) 441 / 493, 3,072 tokens 914 / 827, 4,096 tokens 1,553 / 1,437
+F32_WIDE_TILES = 6144
 
 
 def attention_f32(q: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, window: int = 0, scale: float | None = None,
@@ -577,7 +577,7 @@ def attention_f32(q: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, window:
         items = work.shape[0]
     _lib.check(_lib.load().tff_attention_f32(
         q.data_ptr(), q.stride(0), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), bt.data_ptr(), bt.stride(0),
-        batch.cu_tokens.data_ptr(), batch.start_pos.data_ptr(), _ptr(work), items, tiles, cols, 1 if alone else 0, nq, nkv, d,
+        batch.cu_tokens.data_ptr(), batch.start_pos.data_ptr(), _ptr(work), items, tiles, cols, nq, nkv, d,
         k_cache.shape[2], k_cache.shape[0], int(window), float(scale), _ptr(sinks), float(softcap or 0.0), _stream()))
     return out
 
