@@ -1016,6 +1016,31 @@ def test_attention_f32_gives_a_token_the_same_bits_in_any_step(nq, nkv, d, ps, w
             assert torch.equal(got, whole[rows]), parts
 
 
+@pytest.mark.parametrize("cols", [16, 128])
+@pytest.mark.parametrize("nq,nkv,d,ps,window", [(4, 2, 64, 16, 0), (5, 5, 128, 8, 24), (2, 1, 256, 16, 0)])
+def test_attention_f32_values_that_are_not_finite_reach_their_readers_only(nq, nkv, d, ps, window, cols):
+    """Infinities and NaN among the values: tokens that see none of them give the bits that they give without, the others
+    exactly what the general kernel gives: the same elements are +inf, -inf and NaN."""
+    ops = _ops()
+    if cols == 128 and d > 128:
+        pytest.skip("no such block")
+    entries = [(0, 130), (40, 70)]
+    batch, kv, ks, vs, positions, token_req = _fake_step(entries, ps, nkv, d, torch.float32, seed=d)
+    q = torch.randn(batch.num_tokens, nq * d, generator=torch.Generator().manual_seed(4)).to(DEV)
+    clean = ops.attention_f32(q, nq, nkv, d, kv, batch, window, cols=cols)
+    inf, nan = float("inf"), float("nan")
+    bad = [(0, 50, 3, inf), (0, 50, 7, -inf), (0, 77, 3, -inf), (0, 90, 9, nan), (0, 129, 5, inf), (1, 41, 2, nan), (1, 100, d - 1, inf)]
+    for r, j, e, x in bad:
+        kv.v_cache[kv.block_tables[r, j // ps], nkv - 1, e, j % ps] = x
+    out = ops.attention_f32(q, nq, nkv, d, kv, batch, window, cols=cols)
+    gen = ops.attention_generic(q, nq, nkv, d, kv.k_cache, kv.v_cache, kv.block_tables, batch.token_req, batch.positions, window,
+                                1 / math.sqrt(d))
+    fine = torch.isfinite(gen)
+    assert 0 < int((~fine).sum()) < gen.numel() // 4
+    assert torch.equal(out[fine], clean[fine])
+    assert torch.equal(out.nan_to_num(7.0, 8.0, 9.0)[~fine], gen.nan_to_num(7.0, 8.0, 9.0)[~fine])
+
+
 @pytest.mark.parametrize("window", [1, 17, 40])
 @pytest.mark.parametrize("entries", [[(100, 9), (61, 1), (0, 70)], [(100, 1), (61, 1)]])
 def test_attention_f32_looks_up_no_page_before_the_window(entries, window):

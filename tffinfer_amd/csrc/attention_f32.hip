@@ -34,6 +34,20 @@ __device__ __forceinline__ af_floatx4 af_mfma16(const float4& a, const float4& b
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
 }
 
+// The value of key j, zero if it lies outside of what the tile sees or is not finite, which `odd` then notes.
+__device__ __forceinline__ float af_finite(float v, int j, int lo, int hi, bool& odd) {
+    const bool in = j >= lo && j <= hi, fine = fabsf(v) < INFINITY;
+    odd |= in && !fine;
+    return in && fine ? v : 0.f;
+}
+// A value that is not finite as a number whose sums over up to 255 values tell how many of which kind there were, and what
+// such a sum stands for.
+__device__ __forceinline__ float af_kind(float v) { return v == INFINITY ? 1.f : v == -INFINITY ? 256.f : v != v ? 65536.f : 0.f; }
+__device__ __forceinline__ float af_sum_of_kinds(int n) {
+    const bool up = n & 255, down = n >> 8 & 255;
+    return n >> 16 || (up && down) ? __builtin_nanf("") : up ? INFINITY : down ? -INFINITY : 0.f;
+}
+
 // WAVES waves; SHARED: all with the same columns, each with PARTS / WAVES parts of the keys, else with columns of their own and all parts.
 template <int DF, int NC, int WAVES, bool SHARED, int PARTS>
 __global__ __launch_bounds__(64 * WAVES, 2) void attention_f32_kernel(
@@ -84,8 +98,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_f32_kernel(
 #pragma unroll
             for (int s = 0; s < DF; ++s) o[c][s] = af_floatx4{0.f, 0.f, 0.f, 0.f};
         }
-        const int first = lo_min >> 5;
-        for (int k = 32 * (first + ((part - first) & (PARTS - 1))); k <= last_pos; k += 32 * PARTS) {
+        const int first = lo_min >> 5, begin = 32 * (first + ((part - first) & (PARTS - 1)));
+        bool odd = false;
+        for (int k = begin; k <= last_pos; k += 32 * PARTS) {
             af_floatx4 sc[NC][2];
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
@@ -139,19 +154,46 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_f32_kernel(
                 float4 vf[DF];
 #pragma unroll
                 for (int s = 0; s < DF; ++s) vf[s] = *reinterpret_cast<const float4*>(vp + (size_t)16 * s * ps);
-                if (edge) {      // slots that hold nothing of the request's may hold anything: 0 x NaN is not 0
+                if (edge) {
+                    // Slots that hold nothing of the request's may hold anything, and 0 x NaN is not 0; nor may a value that is not
+                    // finite reach the columns that do not see its token.  Such values are left out, and follow below.
 #pragma unroll
                     for (int s = 0; s < DF; ++s) {
-                        vf[s].x = quad + 0 >= lo_min && quad + 0 <= last_pos ? vf[s].x : 0.f;
-                        vf[s].y = quad + 1 >= lo_min && quad + 1 <= last_pos ? vf[s].y : 0.f;
-                        vf[s].z = quad + 2 >= lo_min && quad + 2 <= last_pos ? vf[s].z : 0.f;
-                        vf[s].w = quad + 3 >= lo_min && quad + 3 <= last_pos ? vf[s].w : 0.f;
+                        vf[s].x = af_finite(vf[s].x, quad + 0, lo_min, last_pos, odd);
+                        vf[s].y = af_finite(vf[s].y, quad + 1, lo_min, last_pos, odd);
+                        vf[s].z = af_finite(vf[s].z, quad + 2, lo_min, last_pos, odd);
+                        vf[s].w = af_finite(vf[s].w, quad + 3, lo_min, last_pos, odd);
                     }
                 }
 #pragma unroll
                 for (int c = 0; c < NC; ++c)
 #pragma unroll
                     for (int s = 0; s < DF; ++s) o[c][s] = af_mfma16(vf[s], p[c][f], o[c][s]);
+            }
+        }
+        if (__any(odd)) {        // what the values that were left out amount to for the columns that see them, their number by kind
+#pragma unroll 1
+            for (int k = begin; k <= last_pos; k += 32 * PARTS) {
+                if (!(k < lo_max || k + 31 > first_pos)) continue;
+#pragma unroll 1
+                for (int f = 0; f < 2; ++f) {
+                    const int quad = k + 16 * f + 4 * g, key = min(max(quad, lo_min & ~3), last_pos & ~3);
+                    const float* vp = v_cache + ((size_t)bt[key >> ps_shift] * nkv + g_kv) * ps * D + (key & (ps - 1)) + (size_t)r * ps;
+#pragma unroll
+                    for (int s = 0; s < DF; ++s) {
+                        const float4 v = *reinterpret_cast<const float4*>(vp + (size_t)16 * s * ps);
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) {
+                            auto sees = [&](int j) { return j >= lo[c] && j <= pos[c] ? 1.f : 0.f; };
+                            const af_floatx4 n = af_mfma16(make_float4(af_kind(v.x), af_kind(v.y), af_kind(v.z), af_kind(v.w)),
+                                                           make_float4(sees(quad), sees(quad + 1), sees(quad + 2), sees(quad + 3)),
+                                                           af_floatx4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) o[c][s][i] += af_sum_of_kinds((int)n[i]);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
             }
         }
 #pragma unroll
