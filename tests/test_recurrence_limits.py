@@ -1,0 +1,62 @@
+"""Which steps the recurrences take in chunks on the matrix cores: the dispatch asks the kernels' own rule, and what the rule
+refuses stays with the forms that have no such limit."""
+import types
+
+import pytest
+import torch
+
+
+def _lib():
+    from tffinfer_amd.kernels import lib
+    return lib.load()
+
+
+def test_wkv_chunks_up_to_what_a_launch_holds():
+    L = _lib()
+    for tokens, fits in ((128, 1), (16 * 65535, 1), (16 * 65535 + 1, 0), ((1 << 20) - 1, 0), (1 << 20, 0)):
+        assert L.tff_wkv_chunks_supported(3, tokens, 64, 4096) == fits, tokens
+    assert L.tff_wkv_chunks_supported(65535, 128, 128, 4096) == 1 and L.tff_wkv_chunks_supported(65536, 128, 128, 4096) == 0
+    assert [L.tff_wkv_chunks_supported(1, 128, D, 4096) for D in (48, 64, 96, 128, 256)] == [0, 1, 0, 1, 0]
+    assert [L.tff_wkv_chunks_supported(1, 128, 64, row) for row in (4098, (1 << 25) - 4, 1 << 25)] == [0, 1, 0]
+
+
+def test_gated_delta_chunks_up_to_32_bit_offsets():
+    """Seventeen rows of channels in bytes stay under 2^32; the token-by-token form takes rows up to twice as long."""
+    L = _lib()
+    H, G, D = 2, 1, 64
+
+    def bytes_of(E):
+        return (2 * G * D + H * E + 2 * H) * 17 * 4
+    for E in (64, 1 << 20, 31_580_000, 31_581_000, 40_000_000):
+        assert L.tff_gdelta_chunks_supported(1, H, G, D, E, 4096) == (bytes_of(E) < 1 << 32 and E <= 16 * 65535), E
+    H = 65534
+    for E in (480, 960, 964, 1928):
+        assert L.tff_gdelta_chunks_supported(1, H, G, D, E, 4096) == (bytes_of(E) < 1 << 32), E
+    assert L.tff_gdelta_chunks_supported(65536, 2, 1, 64, 64, 4096) == 0 and L.tff_gdelta_chunks_supported(65535, 2, 1, 64, 64, 4096) == 1
+    assert L.tff_gdelta_chunks_supported(1, 3, 1, 64, 64, 4096) == 0 and L.tff_gdelta_chunks_supported(1, 4, 2, 64, 64, 4098) == 0
+
+
+@pytest.mark.parametrize("longest,chunks", [(127, False), (128, True), (16 * 65535, True), (16 * 65535 + 1, False), ((1 << 20) - 1, False)])
+def test_wkv_dispatch_keeps_to_the_rule(monkeypatch, longest, chunks):
+    """The op calls the entry for chunks exactly where the rule takes the step (the entries themselves are not run)."""
+    from tffinfer_amd.kernels import ops
+    real, called = _lib(), []
+
+    class Library:
+        def __getattr__(self, name):
+            if name in ("tff_wkv_recurrence", "tff_wkv_recurrence_chunks"):
+                return lambda *a: called.append(name) or 0
+            return getattr(real, name)
+
+    class OnGpu(torch.Tensor):
+        is_cuda = True
+    monkeypatch.setattr(ops._lib, "load", lambda: Library())
+    monkeypatch.setattr(ops, "_req", lambda t, *a, **k: t)
+    monkeypatch.setattr(ops, "_state_rows", lambda t, *a: t.shape[1])
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    H, D, T = 1, 64, 4
+    r, k, v, z = (torch.zeros(T, H * D).as_subclass(OnGpu) for _ in range(4))
+    i32 = torch.zeros(2, dtype=torch.int32)
+    batch = types.SimpleNamespace(num_reqs=1, max_new_tokens=longest, cu_tokens=i32, state_slots=i32)
+    ops.wkv_recurrence(r, k, v, z, torch.zeros(H * D), torch.zeros(H * D), torch.zeros(1, H * D * D), batch, H, D)
+    assert called == ["tff_wkv_recurrence_chunks" if chunks else "tff_wkv_recurrence"]

@@ -659,8 +659,11 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
 
 TFF_API size_t tff_gdelta_chunks_workspace_bytes(int T, int R, int H) { return ((size_t)T / 16 + R + 1) * H * GD_WORK * sizeof(float); }
 
-TFF_API int tff_gdelta_chunks_supported(int D, int E, size_t state_row) {
-    return (D == 64 || D == 128 || D == 256) && E % 4 == 0 && state_row % 4 == 0;
+// (a lane's offset within sixteen rows of pre is 32 bits of bytes)
+TFF_API int tff_gdelta_chunks_supported(int R, int H, int G, int D, int E, size_t state_row) {
+    const size_t row = 2 * (size_t)G * D + (size_t)H * E + 2 * (size_t)H;
+    return (D == 64 || D == 128 || D == 256) && E % 4 == 0 && H % 2 == 0 && state_row % 4 == 0 && H <= 65535 && R <= 65535 &&
+           (E + 15) / 16 <= 65535 && row * 17 * sizeof(float) < ((size_t)1 << 32);
 }
 
 // As tff_gdelta_recurrence, in chunks; max_tokens: the longest portion.  Every row's first 2 G D + H E + 2 H channels of pre are
@@ -672,19 +675,17 @@ TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, si
     TFF_REQUIRE(R >= 0 && H > 0 && G > 0 && H % G == 0 && E > 0 && taps >= 1 && taps <= GD_MAX_TAPS && T >= 0 && max_tokens > 0,
                 "gdelta_chunks: bad sizes heads=%d kv_heads=%d vdim=%d taps=%d", H, G, E, taps);
     const size_t C = 2 * (size_t)G * D + (size_t)H * E;
-    TFF_REQUIRE(tff_gdelta_chunks_supported(D, E, state_row) && H % 2 == 0, "gdelta_chunks: heads of %d x %d, state rows of %zu", D, E, state_row);
+    TFF_REQUIRE(tff_gdelta_chunks_supported(R, H, G, D, E, state_row), "gdelta_chunks: %d requests, %d and %d heads of %d x %d, state rows of %zu",
+                R, H, G, D, E, state_row);
     TFF_REQUIRE(((uintptr_t)pre % 16) == 0 && ((uintptr_t)state % 16) == 0 && ((uintptr_t)work % 16) == 0,
                 "gdelta_chunks: operands must be 16-byte aligned");
     TFF_REQUIRE(ldp >= C + 2 * (size_t)H && (size_t)H * E * D <= tail_off && tail_off + (size_t)(taps - 1) * C <= state_row,
                 "gdelta_chunks: rows of %zu or state rows of %zu are too short", ldp, state_row);
-    TFF_REQUIRE(H <= 65535 && R <= 65535, "gdelta_chunks: too many heads or requests");
-    TFF_REQUIRE((C + 2 * (size_t)H) * 17 < ((size_t)1 << 31), "gdelta_chunks: rows of %zu channels are too long", C);
     if (R == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     gdelta_chunk_kernel<<<dim3((max_tokens + 15) / 16, H, R), 64, 0, s>>>(pre, cu_tokens, work, H, G, D, E);
     if (int rc = tff_check_launch("gdelta_chunk")) return rc;
     const dim3 grid(H, (E + 15) / 16, R);
-    TFF_REQUIRE(grid.y <= 65535, "gdelta_chunks: heads of %d value channels", E);
 #define GD_SCAN(NT, WV) gdelta_scan_kernel<NT, WV><<<grid, 64 * WV, 0, s>>>(pre, proj, ldp, state, state_row, tail_off, taps, cu_tokens, state_slots, work, o, H, G, E)
     if (D == 64) GD_SCAN(1, 4);
     else if (D == 128) GD_SCAN(2, 4);

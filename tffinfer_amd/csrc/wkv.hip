@@ -649,6 +649,11 @@ TFF_API size_t tff_wkv_chunks_workspace_bytes(int T, int R, int H, int D) {
     return ((size_t)T / 16 + R + 1) * H * wkv_work(D) * sizeof(float);
 }
 
+// (the chunks of a portion are the launch's second dimension; a lane's offset within sixteen rows is 32 bits of bytes)
+TFF_API int tff_wkv_chunks_supported(int R, int max_tokens, int D, size_t row) {
+    return (D == 64 || D == 128) && row % 4 == 0 && row < ((size_t)1 << 25) && R <= 65535 && max_tokens <= 16 * 65535;
+}
+
 // As tff_wkv_recurrence, for heads of 64 and 128; max_tokens: the longest portion; row a multiple of 4 and r, k, z, w0, u and
 // work 16-byte aligned.
 TFF_API int tff_wkv_recurrence_chunks(const float* r, const float* k, const float* v, const float* z, size_t row, const float* w0,
@@ -656,13 +661,12 @@ TFF_API int tff_wkv_recurrence_chunks(const float* r, const float* k, const floa
                                       const int32_t* state_slots, float* work, float* o, int T, int R, int H, int D, const float* x,
                                       int W, size_t prev_off, int max_tokens, tff_stream_t stream) {
     TFF_REQUIRE(r && k && v && z && w0 && u && state && cu_tokens && state_slots && work && o, "wkv_chunks: null pointer");
-    TFF_REQUIRE(R >= 0 && T >= 0 && H > 0 && max_tokens > 0 && (D == 64 || D == 128), "wkv_chunks: %d heads of %d (64 or 128)", H, D);
-    TFF_REQUIRE(row >= (size_t)H * D && row % 4 == 0 && (size_t)H * D * D <= state_row && (!x || prev_off + (size_t)W <= state_row),
+    TFF_REQUIRE(R >= 0 && T >= 0 && H > 0 && max_tokens > 0 && tff_wkv_chunks_supported(R, max_tokens, D, row),
+                "wkv_chunks: %d requests of up to %d tokens, %d heads of %d (64 or 128), rows of %zu", R, max_tokens, H, D, row);
+    TFF_REQUIRE(row >= (size_t)H * D && (size_t)H * D * D <= state_row && (!x || prev_off + (size_t)W <= state_row),
                 "wkv_chunks: rows of %zu, state rows of %zu do not hold %d heads of %d", row, state_row, H, D);
     TFF_REQUIRE(((uintptr_t)r % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)z % 16) == 0 && ((uintptr_t)w0 % 16) == 0 &&
                 ((uintptr_t)u % 16) == 0 && ((uintptr_t)work % 16) == 0, "wkv_chunks: operands must be 16-byte aligned");
-    TFF_REQUIRE(row < ((size_t)1 << 25), "wkv_chunks: rows of %zu are too long", row);
-    TFF_REQUIRE(R <= 65535 && max_tokens <= 16 * 65535, "wkv_chunks: too many requests or tokens");
     if (R == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     const dim3 pieces(H, (max_tokens + 15) / 16, R), grid(H, D / 16, R);

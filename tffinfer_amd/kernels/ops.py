@@ -1452,20 +1452,20 @@ def wkv_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.T
     if T == 0:
         return o
     longest = int(getattr(batch, "max_new_tokens", 0) or 0)
-    if WKV_CHUNKS_MIN_TOKENS <= longest < 1 << 20 and D in (64, 128) and r.stride(0) % 4 == 0 and r.stride(0) < 1 << 25 \
+    L = _lib.load()
+    if longest >= WKV_CHUNKS_MIN_TOKENS and L.tff_wkv_chunks_supported(batch.num_reqs, longest, D, r.stride(0)) \
             and all(t.data_ptr() % 16 == 0 for t in (r, k, z, w0, u)):
-        L = _lib.load()
         work = torch.empty(L.tff_wkv_chunks_workspace_bytes(T, batch.num_reqs, H, D) // 4, dtype=torch.float32, device=r.device)
         _lib.check(L.tff_wkv_recurrence_chunks(
             r.data_ptr(), k.data_ptr(), v.data_ptr(), z.data_ptr(), r.stride(0), w0.data_ptr(), u.data_ptr(), state.data_ptr(), row,
             batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), work.data_ptr(), o.data_ptr(), T, batch.num_reqs, H, D, _ptr(x), W,
             int(prev_off), longest, _stream()))
         return o
-    _lib.check(_lib.load().tff_wkv_recurrence(r.data_ptr(), k.data_ptr(), v.data_ptr(), z.data_ptr(), r.stride(0),
-                                              w0.data_ptr(), u.data_ptr(), state.data_ptr(), row,
-                                              batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), o.data_ptr(),
-                                              batch.num_reqs, H, D, _ptr(x), W, int(prev_off),
-                                              1 if longest >= WKV_LONG_PORTION else 0, _stream()))
+    _lib.check(L.tff_wkv_recurrence(r.data_ptr(), k.data_ptr(), v.data_ptr(), z.data_ptr(), r.stride(0),
+                                    w0.data_ptr(), u.data_ptr(), state.data_ptr(), row,
+                                    batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), o.data_ptr(),
+                                    batch.num_reqs, H, D, _ptr(x), W, int(prev_off),
+                                    1 if longest >= WKV_LONG_PORTION else 0, _stream()))
     return o
 
 
@@ -2071,7 +2071,8 @@ def gated_delta(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, d
                                  state.data_ptr(), row, tail, batch.token_req.data_ptr(), batch.cu_tokens.data_ptr(),
                                  batch.state_slots.data_ptr(), pre.data_ptr(), T, H, G, D, E, stream))
     longest = int(getattr(batch, "max_new_tokens", 0) or 0)
-    if longest >= GDELTA_CHUNKS_MIN_TOKENS and H % 2 == 0 and state.data_ptr() % 16 == 0 and L.tff_gdelta_chunks_supported(D, E, row):
+    if longest >= GDELTA_CHUNKS_MIN_TOKENS and state.data_ptr() % 16 == 0 \
+            and L.tff_gdelta_chunks_supported(batch.num_reqs, H, G, D, E, row):
         work = torch.empty(L.tff_gdelta_chunks_workspace_bytes(T, batch.num_reqs, H) // 4, dtype=torch.float32, device=proj.device)
         _lib.check(L.tff_gdelta_recurrence_chunks(
             pre.data_ptr(), proj.data_ptr(), ldp, state.data_ptr(), row, tail, taps, batch.cu_tokens.data_ptr(),
