@@ -225,6 +225,27 @@ def test_delta_rule_in_chunks_of_sixteen(H, G, D, E, taps, extreme):
         assert float(state[1].abs().max()) == 0
 
 
+@pytest.mark.parametrize("H,G,D,E", [(2, 1, 64, 20), (4, 2, 128, 128), (2, 2, 256, 36)])
+@pytest.mark.parametrize("ns", [[1, 200, 2], [95, 96, 0, 4, 150, 1], [300, 1, 1, 97]])
+def test_delta_rule_of_a_portion_is_its_own_in_any_step(H, G, D, E, ns):
+    """Portions too short for the chunks beside portions long enough, with one of no tokens: outputs and states of every
+    request are the bits that it gives alone."""
+    ops = _ops()
+    taps, T = 4, sum(ns)
+    proj, conv, a_log, dt = _delta_case(T, H, G, D, E, taps, D + E + T)
+    row = H * E * D + (taps - 1) * (2 * G * D + H * E)
+    row += -row % 4
+    dev, many = [x.to(DEV) for x in (conv, a_log, dt)], torch.zeros(len(ns), row, device=DEV)
+    alone = many.normal_(generator=torch.Generator(device=DEV).manual_seed(D)).clone()
+    o = ops.gated_delta(proj.to(DEV), *dev, many, _batch(ns, [0] * len(ns), list(range(len(ns)))), H, G, D, E)
+    for i, n in enumerate(ns):
+        at = sum(ns[:i])
+        if n:
+            one = ops.gated_delta(proj[at:at + n].to(DEV), *dev, alone, _batch([n], [0], [i]), H, G, D, E)
+            assert torch.equal(one, o[at:at + n]), (i, n)
+        assert torch.equal(alone[i], many[i]), (i, n)
+
+
 @pytest.mark.parametrize("H,G,D,E", [(2, 1, 64, 20), (4, 2, 128, 128), (2, 2, 256, 36), (4, 2, 16, 8)])
 def test_delta_rule_of_many_tokens_is_that_of_few(H, G, D, E):
     """More tokens than the preparation takes one by one, in requests too short for the chunks, from states that are not zero:

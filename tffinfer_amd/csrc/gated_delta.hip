@@ -21,6 +21,7 @@
 // tff_sigmoid_gate_heads: out = o * sigmoid(gate) * scale, heads of o a stride apart.
 #include "common.h"
 #include "tffinfer_kernels.h"
+#include <limits.h>
 
 #define GD_MAX_TAPS 8
 #define GD_FEW 4        // tokens a request up to which a step counts as decoding
@@ -210,7 +211,7 @@ __device__ __forceinline__ void gd_keep_inputs(const float* __restrict__ proj, s
 
 // One token of one value channel, on the row of sixteen lanes that shares the channel; lane s holds the key
 // channels s, s + 16, ... of S, k and q.  The same additions in the same order wherever it is used, so that a
-// sequence gives the same bits however it is cut into steps of portions that are too short for chunks (below).
+// sequence gives the same bits however it is cut into portions that are too short for chunks (below), whatever else a step holds.
 template <int KPL>
 __device__ __forceinline__ float gd_token(float (&S)[KPL], const float (&kk)[KPL], const float (&qq)[KPL], float v, float beta,
                                           float g) {
@@ -235,13 +236,14 @@ template <int KPL>
 __global__ __launch_bounds__(256) void gdelta_recurrence_few_kernel(
     const float* __restrict__ pre, const float* __restrict__ proj, size_t ldp, float* __restrict__ state, size_t state_row,
     size_t tail_off, int taps, const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ state_slots,
-    float* __restrict__ o, int H, int G, int D, int E) {
+    float* __restrict__ o, int H, int G, int D, int E, int below) {
     const int h = blockIdx.y, r = blockIdx.z, j0 = blockIdx.x * 16;
     const int tid = threadIdx.x, s = tid & 15, j = j0 + (tid >> 4), jc = min(j, E - 1);
     const int C = 2 * G * D + H * E;
     const size_t ldq = (size_t)C + 2 * H;
     const int gk = h / (H / G);
     const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0;
+    if (n >= below) return;                                // (a portion for the kernels over chunks)
     float* srow = state + (size_t)state_slots[r] * state_row;
     float* sp = srow + ((size_t)h * E + jc) * D + s;
     const bool row_live = j < E;
@@ -284,7 +286,7 @@ template <int KPL>
 __global__ __launch_bounds__(256) void gdelta_recurrence_kernel(
     const float* __restrict__ pre, const float* __restrict__ proj, size_t ldp, float* __restrict__ state, size_t state_row,
     size_t tail_off, int taps, const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ state_slots,
-    float* __restrict__ o, int H, int G, int D, int E) {
+    float* __restrict__ o, int H, int G, int D, int E, int below) {
     constexpr int DP = 16 * KPL;
     constexpr int GD_CHUNK = KPL >= 16 ? 8 : 16;           // (two chunks of the widest heads fill LDS otherwise)
     constexpr int ROWW = 2 * DP + 20;                      // k, q, sixteen v, beta, decay of a token; rows of 16 bytes
@@ -297,7 +299,7 @@ __global__ __launch_bounds__(256) void gdelta_recurrence_kernel(
     const size_t ldq = (size_t)C + 2 * H;
     const int gk = h / (H / G);
     const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0;
-    if (n <= 0) return;                                    // (the whole block: a request without tokens changes nothing)
+    if (n <= 0 || n >= below) return;                      // (the whole block: a request without tokens changes nothing; chunks)
     float* srow = state + (size_t)state_slots[r] * state_row;
     float S[KPL];
     float* sp = srow + ((size_t)h * E + min(j, E - 1)) * D + s;
@@ -396,7 +398,7 @@ __global__ __launch_bounds__(256) void gdelta_recurrence_kernel(
 
 TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
                                   size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* o,
-                                  int R, int H, int G, int D, int E, int max_tokens, tff_stream_t stream) {
+                                  int R, int H, int G, int D, int E, int max_tokens, int below, tff_stream_t stream) {
     TFF_REQUIRE(pre && proj && state && cu_tokens && state_slots && o, "gdelta_recurrence: null pointer");
     TFF_REQUIRE(R >= 0 && H > 0 && G > 0 && H % G == 0 && D > 0 && D <= 256 && E > 0 && taps >= 1 && taps <= GD_MAX_TAPS,
                 "gdelta_recurrence: bad sizes heads=%d kv_heads=%d dim=%d vdim=%d taps=%d (dim up to 256, taps up to %d)", H, G, D,
@@ -407,6 +409,7 @@ TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ld
     TFF_REQUIRE(H <= 65535 && R <= 65535, "gdelta_recurrence: too many heads or requests");
     TFF_REQUIRE((C + 2 * (size_t)H) * 17 < ((size_t)1 << 31), "gdelta_recurrence: rows of %zu channels are too long", C);
     if (R == 0) return 0;
+    if (below <= 0) below = INT_MAX;
     const dim3 grid((E + 15) / 16, H, R);
     hipStream_t s = (hipStream_t)stream;
     // (a request's tokens go one after the other: up to GD_FEW of them need no staging through LDS)
@@ -414,10 +417,10 @@ TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ld
     do {                                                                                                                   \
         if (max_tokens > 0 && max_tokens <= GD_FEW)                                                                        \
             gdelta_recurrence_few_kernel<KPL><<<grid, 256, 0, s>>>(pre, proj, ldp, state, state_row, tail_off, taps,        \
-                                                                   cu_tokens, state_slots, o, H, G, D, E);                 \
+                                                                   cu_tokens, state_slots, o, H, G, D, E, below);          \
         else                                                                                                               \
             gdelta_recurrence_kernel<KPL><<<grid, 256, 0, s>>>(pre, proj, ldp, state, state_row, tail_off, taps, cu_tokens, \
-                                                               state_slots, o, H, G, D, E);                                \
+                                                               state_slots, o, H, G, D, E, below);                         \
     } while (0)
     if (D <= 16) GD_LAUNCH(1);
     else if (D <= 32) GD_LAUNCH(2);
@@ -429,7 +432,8 @@ TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ld
 }
 
 // ------------------------------------------------- long portions: chunks of sixteen tokens ---
-// For head sizes of 64, 128 and 256.  Within a chunk that starts from S0, with G_t = g_0 .. g_t and P_ts = g_(s+1) .. g_t,
+// For head sizes of 64, 128 and 256.  Each portion goes by its own length, so that a request's bits do not change with what else
+// the step holds: portions of `from` tokens and more run here, shorter ones in the same step token by token.  Within a chunk that starts from S0, with G_t = g_0 .. g_t and P_ts = g_(s+1) .. g_t,
 //
 //   (I + L) U = B (V - diag(G) K S0),   L_ts = beta_t P_ts (k_t . k_s), s < t;      S_t = G_t S0 + sum over s <= t of P_ts k_s u_s^T
 //   O = diag(G) Q S0 + A U,             A_ts = P_ts (q_t . k_s), s <= t
@@ -464,11 +468,11 @@ __device__ __forceinline__ gd_floatx4 gd_mfma16(const float4& a, const gd_floatx
 }
 
 __global__ __launch_bounds__(64) void gdelta_chunk_kernel(const float* __restrict__ pre, const int32_t* __restrict__ cu_tokens,
-                                                          float* __restrict__ work, int H, int G, int D, int E) {
+                                                          float* __restrict__ work, int H, int G, int D, int E, int from) {
     __shared__ double sl[16][17];
     const int h = blockIdx.y, r = blockIdx.z, lane = threadIdx.x, c = lane & 15, g = lane >> 4;
     const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0, first = blockIdx.x * 16;
-    if (first >= n) return;
+    if (n < from || first >= n) return;
     const int C = 2 * G * D + H * E, gk = h / (H / G);
     const size_t ldq = (size_t)C + 2 * H;
     const int tok = first + c;                            // this lane's token as a row and as a column
@@ -530,13 +534,13 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
                                                           float* __restrict__ state, size_t state_row, size_t tail_off, int taps,
                                                           const int32_t* __restrict__ cu_tokens,
                                                           const int32_t* __restrict__ state_slots, const float* __restrict__ work,
-                                                          float* __restrict__ o, int H, int G, int E) {
+                                                          float* __restrict__ o, int H, int G, int E, int from) {
     constexpr int D = 16 * WV * NT;
     __shared__ gd_floatx4 px[2][WV][64], py[2][WV][WV][64];      // parts of K S0 by turns; of Q S0 by turns and chunk
     const int h = blockIdx.x, r = blockIdx.z, j0 = blockIdx.y * 16;      // (a head's blocks on one XCD: they read the same keys and queries)
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
     const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0;
-    if (n <= 0) return;                                    // (the whole block: a request without tokens changes nothing)
+    if (n < from) return;                                  // (the whole block: a portion for the token-by-token form)
     const int C = 2 * G * D + H * E, gk = h / (H / G);
     const size_t ldq = (size_t)C + 2 * H;
     const bool live = j0 + c < E;
@@ -666,13 +670,13 @@ TFF_API int tff_gdelta_chunks_supported(int R, int H, int G, int D, int E, size_
            (E + 15) / 16 <= 65535 && row * 17 * sizeof(float) < ((size_t)1 << 32);
 }
 
-// As tff_gdelta_recurrence, in chunks; max_tokens: the longest portion.  Every row's first 2 G D + H E + 2 H channels of pre are
+// As tff_gdelta_recurrence, in chunks, for the portions of `from` tokens and more; max_tokens: the longest portion.  Every row's first 2 G D + H E + 2 H channels of pre are
 // a multiple of four long, and pre, state and work are 16-byte aligned.
 TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
                                          size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* work,
-                                         float* o, int T, int R, int H, int G, int D, int E, int max_tokens, tff_stream_t stream) {
+                                         float* o, int T, int R, int H, int G, int D, int E, int max_tokens, int from, tff_stream_t stream) {
     TFF_REQUIRE(pre && proj && state && cu_tokens && state_slots && work && o, "gdelta_chunks: null pointer");
-    TFF_REQUIRE(R >= 0 && H > 0 && G > 0 && H % G == 0 && E > 0 && taps >= 1 && taps <= GD_MAX_TAPS && T >= 0 && max_tokens > 0,
+    TFF_REQUIRE(R >= 0 && H > 0 && G > 0 && H % G == 0 && E > 0 && taps >= 1 && taps <= GD_MAX_TAPS && T >= 0 && max_tokens > 0 && from > 0,
                 "gdelta_chunks: bad sizes heads=%d kv_heads=%d vdim=%d taps=%d", H, G, E, taps);
     const size_t C = 2 * (size_t)G * D + (size_t)H * E;
     TFF_REQUIRE(tff_gdelta_chunks_supported(R, H, G, D, E, state_row), "gdelta_chunks: %d requests, %d and %d heads of %d x %d, state rows of %zu",
@@ -683,10 +687,10 @@ TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, si
                 "gdelta_chunks: rows of %zu or state rows of %zu are too short", ldp, state_row);
     if (R == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
-    gdelta_chunk_kernel<<<dim3((max_tokens + 15) / 16, H, R), 64, 0, s>>>(pre, cu_tokens, work, H, G, D, E);
+    gdelta_chunk_kernel<<<dim3((max_tokens + 15) / 16, H, R), 64, 0, s>>>(pre, cu_tokens, work, H, G, D, E, from);
     if (int rc = tff_check_launch("gdelta_chunk")) return rc;
     const dim3 grid(H, (E + 15) / 16, R);
-#define GD_SCAN(NT, WV) gdelta_scan_kernel<NT, WV><<<grid, 64 * WV, 0, s>>>(pre, proj, ldp, state, state_row, tail_off, taps, cu_tokens, state_slots, work, o, H, G, E)
+#define GD_SCAN(NT, WV) gdelta_scan_kernel<NT, WV><<<grid, 64 * WV, 0, s>>>(pre, proj, ldp, state, state_row, tail_off, taps, cu_tokens, state_slots, work, o, H, G, E, from)
     if (D == 64) GD_SCAN(1, 4);
     else if (D == 128) GD_SCAN(2, 4);
     else GD_SCAN(4, 4);

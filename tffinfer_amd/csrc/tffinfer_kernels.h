@@ -391,18 +391,19 @@ TFF_API int tff_gdelta_prep(const float* proj, size_t ldp, const float* wconv, i
 // Per request (cu_tokens, state_slots) and head h (keys and queries of head h / (H / G)), S^T [E, D] at the start of
 // the state row: S <- decay S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q.  o float32 [T, H * E].  The
 // portion's last taps - 1 rows of proj's channels are left at tail_off of the state row.  max_tokens: the most
-// tokens that a request brings in this step (0: unknown); it chooses between the form for decoding and for prompts.
+// tokens that a request brings in this step (0: unknown); it chooses between the form for decoding and for prompts, whose bits are
+// the same.  Requests of `below` tokens and more (0: none) are left alone.
 TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
                                   size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* o,
-                                  int R, int H, int G, int D, int E, int max_tokens, tff_stream_t stream);
-// The same for long portions (max_tokens: the longest), in chunks of sixteen tokens on the float32 matrix cores: head sizes of
+                                  int R, int H, int G, int D, int E, int max_tokens, int below, tff_stream_t stream);
+// The same for the portions of `from` tokens and more (max_tokens: the longest), in chunks of sixteen tokens on the float32 matrix cores: head sizes of
 // 64, 128 and 256, what tff_gdelta_chunks_supported says; work: tff_gdelta_chunks_workspace_bytes.  A token's result depends on where its portion
 // began, beyond rounding it does not.
 TFF_API size_t tff_gdelta_chunks_workspace_bytes(int T, int R, int H);
 TFF_API int tff_gdelta_chunks_supported(int R, int H, int G, int D, int E, size_t state_row);
 TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
                                          size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* work,
-                                         float* o, int T, int R, int H, int G, int D, int E, int max_tokens, tff_stream_t stream);
+                                         float* o, int T, int R, int H, int G, int D, int E, int max_tokens, int from, tff_stream_t stream);
 
 // out[t * out_row + h * E + e] = o[t, h, e] / sqrt(mean over e of o^2 + eps) * w[e] * silu(g[t * g_row + h * E + e]) * scale
 TFF_API int tff_head_norm_silu_gate(const float* o, const float* g, size_t g_row, const float* w, float eps, float scale,

@@ -2023,6 +2023,13 @@ def route_by_table(table: torch.Tensor, token_ids: torch.Tensor, num_experts: in
     return idx, wts
 
 
+def _longest_below(batch, limit: int) -> int:
+    """The longest portion of a step among those of fewer than ``limit`` tokens (0: there is none); where the host
+    does not hold the portions, the longest there can be."""
+    cu = getattr(batch, "host_cu_tokens", None)
+    return limit - 1 if cu is None else max((b - a for a, b in zip(cu, cu[1:]) if b - a < limit), default=0)
+
+
 def _rows2(t: torch.Tensor, name: str, dtype, cols: int):
     """A GPU matrix with unit inner stride (rows may be strided) of at least ``cols`` columns; its row stride."""
     if not isinstance(t, torch.Tensor) or not t.is_cuda or t.dim() != 2 or t.stride(1) != 1 or t.dtype != dtype \
@@ -2031,9 +2038,9 @@ def _rows2(t: torch.Tensor, name: str, dtype, cols: int):
     return t.stride(0) if t.shape[0] > 1 else t.shape[1]
 
 
-#: tokens of the longest portion from which the gated delta rule runs in chunks on the matrix cores: 96 tokens of 32 heads of
-#: 128 x 128 take 31 us, preparation and all, against 43 token by token; shorter portions are worked through token by token, so that a
-#: sequence gives the same bits however it is cut into them
+#: tokens from which a portion runs in chunks on the matrix cores under the gated delta rule: 96 tokens of 32 heads of
+#: 128 x 128 take 31 us, preparation and all, against 43 token by token.  Each portion goes by its own length: shorter ones are
+#: worked through token by token, so that a sequence gives the same bits however it is cut into them and whatever else a step holds
 GDELTA_CHUNKS_MIN_TOKENS = 96
 
 
@@ -2070,17 +2077,21 @@ def gated_delta(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, d
     _lib.check(L.tff_gdelta_prep(proj.data_ptr(), ldp, conv_w.data_ptr(), taps, a_log.data_ptr(), dt_bias.data_ptr(),
                                  state.data_ptr(), row, tail, batch.token_req.data_ptr(), batch.cu_tokens.data_ptr(),
                                  batch.state_slots.data_ptr(), pre.data_ptr(), T, H, G, D, E, stream))
-    longest = int(getattr(batch, "max_new_tokens", 0) or 0)
+    longest, below = int(getattr(batch, "max_new_tokens", 0) or 0), 0
     if longest >= GDELTA_CHUNKS_MIN_TOKENS and state.data_ptr() % 16 == 0 \
             and L.tff_gdelta_chunks_supported(batch.num_reqs, H, G, D, E, row):
         work = torch.empty(L.tff_gdelta_chunks_workspace_bytes(T, batch.num_reqs, H) // 4, dtype=torch.float32, device=proj.device)
         _lib.check(L.tff_gdelta_recurrence_chunks(
             pre.data_ptr(), proj.data_ptr(), ldp, state.data_ptr(), row, tail, taps, batch.cu_tokens.data_ptr(),
-            batch.state_slots.data_ptr(), work.data_ptr(), o.data_ptr(), T, batch.num_reqs, H, G, D, E, longest, stream))
-        return o
+            batch.state_slots.data_ptr(), work.data_ptr(), o.data_ptr(), T, batch.num_reqs, H, G, D, E, longest,
+            GDELTA_CHUNKS_MIN_TOKENS, stream))
+        below = GDELTA_CHUNKS_MIN_TOKENS
+        longest = _longest_below(batch, below)
+        if longest == 0:
+            return o
     _lib.check(L.tff_gdelta_recurrence(pre.data_ptr(), proj.data_ptr(), ldp, state.data_ptr(), row, tail, taps,
                                        batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), o.data_ptr(),
-                                       batch.num_reqs, H, G, D, E, longest, stream))
+                                       batch.num_reqs, H, G, D, E, longest, below, stream))
     return o
 
 
