@@ -173,6 +173,29 @@ def test_output_norm_and_depth_at_the_edges_of_a_block(group):
     assert torch.equal(deep[-1].cpu(), x) and torch.equal(deep[:-1].cpu(), hist[:-1])
 
 
+@pytest.mark.parametrize("H,D", [(2, 64), (1, 128), (2, 48)])
+@pytest.mark.parametrize("portions", [(1, 200, 2), (15, 16, 0, 127, 128, 1), (17, 3), (140, 300), (150, 20)])
+def test_recurrence_of_a_portion_is_its_own_in_any_step(H, D, portions):
+    """Portions on both sides of every limit between the forms, one of no tokens among them: outputs, states and kept rows
+    of every request are the bits that it gives alone."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(D + len(portions))
+    T, R, W = sum(portions), len(portions), 8
+    r, k, v, z = (torch.randn(T, H * D, generator=g).to(DEV) for _ in range(4))
+    w0, u, x = (torch.randn(*s, generator=g).to(DEV) for s in ((H * D,), (H * D,), (T, W)))
+    row = H * D * D + W
+    many = torch.randn(R, row, generator=g).to(DEV)
+    alone = many.clone()
+    o = ops.wkv_recurrence(r, k, v, z, w0, u, many, _batch(list(portions), [0] * R, list(range(R))), H, D, x=x, prev_off=H * D * D)
+    for i, n in enumerate(portions):
+        at = sum(portions[:i])
+        if n:
+            part = [t[at:at + n].contiguous() for t in (r, k, v, z)]
+            one = ops.wkv_recurrence(*part, w0, u, alone, _batch([n], [0], [i]), H, D, x=x[at:at + n].contiguous(), prev_off=H * D * D)
+            assert torch.equal(one, o[at:at + n]), (i, n)
+        assert torch.equal(alone[i], many[i]), (i, n)
+
+
 @pytest.mark.parametrize("H,D,portions", [(2, 64, (128,)), (3, 64, (129, 3, 250)), (1, 128, (145, 128)), (2, 128, (16, 15, 200))])
 def test_recurrence_in_chunks_of_sixteen(H, D, portions):
     """Portions beside one another, the longest of 128 tokens and more, from states that are not zero, with rows

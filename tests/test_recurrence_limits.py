@@ -57,6 +57,6 @@ def test_wkv_dispatch_keeps_to_the_rule(monkeypatch, longest, chunks):
     H, D, T = 1, 64, 4
     r, k, v, z = (torch.zeros(T, H * D).as_subclass(OnGpu) for _ in range(4))
     i32 = torch.zeros(2, dtype=torch.int32)
-    batch = types.SimpleNamespace(num_reqs=1, max_new_tokens=longest, cu_tokens=i32, state_slots=i32)
+    batch = types.SimpleNamespace(num_reqs=1, max_new_tokens=longest, host_cu_tokens=[0, longest], cu_tokens=i32, state_slots=i32)
     ops.wkv_recurrence(r, k, v, z, torch.zeros(H * D), torch.zeros(H * D), torch.zeros(1, H * D * D), batch, H, D)
     assert called == ["tff_wkv_recurrence_chunks" if chunks else "tff_wkv_recurrence"]

@@ -10,17 +10,19 @@
 // tff_token_shift_mix: out[m, t, :] = x[t] + (x'[t] - x[t]) * mu[m], x' the row of the token
 //   before t in the same request: the row above, or for the first token of a request's portion
 //   the row that the state keeps (zeros for a request's first token).
-// tff_wkv_recurrence: the recurrence over the tokens of each request's portion, one block per
-//   (head, request), a thread per value channel and slice of the key channels; the order of every
+// tff_wkv_recurrence: the recurrence over the tokens of each request's portion of `from` tokens and more but fewer than
+//   `below`, one block per (head, request), a thread per value channel and slice of the key channels; the order of every
 //   sum is fixed by the head size and the kernel's form alone, so a token's result does not depend on
 //   how the tokens were cut into steps beyond rounding (`long_portions` picks the form for prompts, whose
 //   sums run in another order than those of the form for single tokens).  The block of head 0 also
 //   leaves the portion's last row of x in the state.
 // tff_wkv_recurrence_chunks: the same in chunks of sixteen tokens on the float32 matrix cores, for heads of 64 and 128.
+// Each portion takes the form that its own length asks for, so that a request's bits do not change with what else a step holds.
 // tff_head_norm_gate: out = o / sqrt(mean over the head of o^2 + eps) * weight * silu(g).
 // tff_tanh: out = tanh(in), float32 in, the activation type out.
 #include "common.h"
 #include "tffinfer_kernels.h"
+#include <limits.h>
 
 template <typename TO>
 __global__ __launch_bounds__(256) void token_shift_mix_kernel(
@@ -77,14 +79,14 @@ __global__ __launch_bounds__(512) void wkv_recurrence_kernel(
     const float* __restrict__ z, size_t row, const float* __restrict__ w0, const float* __restrict__ u,
     float* __restrict__ state, size_t state_row, const int32_t* __restrict__ cu_tokens,
     const int32_t* __restrict__ state_slots, float* __restrict__ o, int H, int D, const float* __restrict__ x, int W,
-    size_t prev_off) {
+    size_t prev_off, int from, int below) {
     __shared__ __attribute__((aligned(16))) float buf[2][3][WKV_CHUNK_ELEMS];       // r, k, w of a chunk, [token][channel]
     __shared__ float bv[2][WKV_CHUNK_ELEMS];                                       // v of a chunk
     __shared__ float so[WKV_CHUNK_ELEMS];
     __shared__ float part[2][WKV_MAX_SLICES][WKV_MAX_D];
     const int h = blockIdx.x, req = blockIdx.y, tid = threadIdx.x, nt = blockDim.x;
     const int t0 = cu_tokens[req], t1 = cu_tokens[req + 1];
-    if (t1 <= t0) return;
+    if (t1 - t0 < from || t1 - t0 >= below) return;       // (the whole block: a portion of no tokens or of another form)
     const int slices = nt / D;
     const int Dp = slices * KPT;
     const int vi = tid % D, ks = tid / D;
@@ -188,7 +190,7 @@ __global__ __launch_bounds__(512) void wkv_recurrence_wave_kernel(
     const float* __restrict__ z, size_t row, const float* __restrict__ w0, const float* __restrict__ u,
     float* __restrict__ state, size_t state_row, const int32_t* __restrict__ cu_tokens,
     const int32_t* __restrict__ state_slots, float* __restrict__ o, int H, const float* __restrict__ x, int W,
-    size_t prev_off) {
+    size_t prev_off, int from, int below) {
     constexpr int D = 4 * KPT;
     constexpr int C = (WKV_CHUNK_ELEMS / D) < 16 ? (WKV_CHUNK_ELEMS / D) : 16;      // tokens a chunk
     constexpr int NT = 4 * D;                                                      // threads: D / 16 waves
@@ -197,7 +199,7 @@ __global__ __launch_bounds__(512) void wkv_recurrence_wave_kernel(
     __shared__ float bv[2][C * D];
     const int h = blockIdx.x, req = blockIdx.y, tid = threadIdx.x;
     const int t0 = cu_tokens[req], t1 = cu_tokens[req + 1];
-    if (t1 <= t0) return;
+    if (t1 - t0 < from || t1 - t0 >= below) return;       // (the whole block: a portion of no tokens or of another form)
     const int lane = tid & 63;
     const int ks = lane >> 4, vi = (tid >> 6) * 16 + (lane & 15);
     float* srow = state + (size_t)state_slots[req] * state_row;
@@ -286,7 +288,7 @@ __global__ __launch_bounds__(256) void wkv_recurrence_rows_kernel(
     const float* __restrict__ z, size_t row, const float* __restrict__ w0, const float* __restrict__ u,
     float* __restrict__ state, size_t state_row, const int32_t* __restrict__ cu_tokens,
     const int32_t* __restrict__ state_slots, float* __restrict__ o, int H, const float* __restrict__ x, int W,
-    size_t prev_off) {
+    size_t prev_off, int from, int below) {
     constexpr int D = 16 * KPT;
     constexpr int C = WKV_CHUNK_ELEMS / D;         // tokens a chunk: 16 or 8
     constexpr int NT = 256;
@@ -296,7 +298,7 @@ __global__ __launch_bounds__(256) void wkv_recurrence_rows_kernel(
     __shared__ float bv[2][C * 16];                                        // v of the block's sixteen channels
     const int h = blockIdx.x, req = blockIdx.y, tid = threadIdx.x;
     const int t0 = cu_tokens[req], t1 = cu_tokens[req + 1];
-    if (t1 <= t0) return;
+    if (t1 - t0 < from || t1 - t0 >= below) return;       // (the whole block: a portion of no tokens or of another form)
     const int lane = tid & 63;
     const int ks = lane & 15, vl = (tid >> 6) * 4 + (lane >> 4), vi = blockIdx.z * 16 + vl;
     float* srow = state + (size_t)state_slots[req] * state_row;
@@ -382,28 +384,30 @@ __global__ __launch_bounds__(256) void wkv_recurrence_rows_kernel(
 TFF_API int tff_wkv_recurrence(const float* r, const float* k, const float* v, const float* z, size_t row, const float* w0,
                                const float* u, float* state, size_t state_row, const int32_t* cu_tokens,
                                const int32_t* state_slots, float* o, int R, int H, int D, const float* x, int W,
-                               size_t prev_off, int long_portions, tff_stream_t stream) {
+                               size_t prev_off, int long_portions, int from, int below, tff_stream_t stream) {
     TFF_REQUIRE(r && k && v && z && w0 && u && state && cu_tokens && state_slots && o, "wkv_recurrence: null pointer");
     TFF_REQUIRE(R >= 0 && H > 0 && D > 0 && D <= WKV_MAX_D, "wkv_recurrence: %d heads of %d (up to %d)", H, D, WKV_MAX_D);
     TFF_REQUIRE(row >= (size_t)H * D && (size_t)H * D * D <= state_row && (!x || prev_off + (size_t)W <= state_row),
                 "wkv_recurrence: rows of %zu, state rows of %zu do not hold %d heads of %d", row, state_row, H, D);
+    TFF_REQUIRE(from > 0, "wkv_recurrence: portions from %d tokens on", from);
     if (R == 0) return 0;
+    if (below <= 0) below = INT_MAX;
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid(H, R);
 #define WKV_LAUNCH(KPT)                                                                                              \
     wkv_recurrence_kernel<KPT><<<grid, D * ((D + KPT - 1) / KPT), 0, s>>>(r, k, v, z, row, w0, u, state, state_row, \
-                                                                           cu_tokens, state_slots, o, H, D, x, W, prev_off)
+                                                                           cu_tokens, state_slots, o, H, D, x, W, prev_off, from, below)
 #define WKV_WAVES(KPT)                                                                                             \
     wkv_recurrence_wave_kernel<KPT><<<grid, 16 * KPT, 0, s>>>(r, k, v, z, row, w0, u, state, state_row, cu_tokens, \
-                                                              state_slots, o, H, x, W, prev_off)
+                                                              state_slots, o, H, x, W, prev_off, from, below)
     if (long_portions && (D == 64 || D == 128)) {
         const dim3 grid3(H, R, D / 16);
         if (D == 64)
             wkv_recurrence_rows_kernel<4><<<grid3, 256, 0, s>>>(r, k, v, z, row, w0, u, state, state_row, cu_tokens,
-                                                                state_slots, o, H, x, W, prev_off);
+                                                                state_slots, o, H, x, W, prev_off, from, below);
         else
             wkv_recurrence_rows_kernel<8><<<grid3, 256, 0, s>>>(r, k, v, z, row, w0, u, state, state_row, cu_tokens,
-                                                                state_slots, o, H, x, W, prev_off);
+                                                                state_slots, o, H, x, W, prev_off, from, below);
     } else if (D % 16 == 0) {
         switch (D / 4) {
             case 4: WKV_WAVES(4); break;
@@ -457,12 +461,12 @@ template <int D>
 __global__ __launch_bounds__(64) void wkv_chunk_kernel(const float* __restrict__ r, const float* __restrict__ k,
                                                        const float* __restrict__ z, size_t row, const float* __restrict__ w0,
                                                        const float* __restrict__ u, const int32_t* __restrict__ cu_tokens,
-                                                       float* __restrict__ work, int H) {
+                                                       float* __restrict__ work, int H, int from) {
     constexpr int M = D / 16, LDR = D + 4;
     __shared__ __attribute__((aligned(16))) float ks[16 * LDR], ws[16 * LDR];
     const int h = blockIdx.x, req = blockIdx.z, lane = threadIdx.x, c = lane & 15, g = lane >> 4;
     const int t0 = cu_tokens[req], n = cu_tokens[req + 1] - t0, first = blockIdx.y * 16;
-    if (first >= n) return;
+    if (n < from || first >= n) return;
     const bool live = first + c < n;                      // (tokens past the portion's end: no key, no decay)
     const size_t at = (size_t)(t0 + min(first + c, n - 1)) * row + (size_t)h * D + 4 * g;
     const float* up = u + (size_t)h * D + 4 * g;
@@ -559,13 +563,13 @@ template <int NT>
 __global__ __launch_bounds__(256) void wkv_scan_kernel(const float* __restrict__ v, size_t row, float* __restrict__ state, size_t state_row,
                                                        const int32_t* __restrict__ cu_tokens,
                                                        const int32_t* __restrict__ state_slots, const float* __restrict__ work,
-                                                       float* __restrict__ o, int H, const float* __restrict__ x, int W, size_t prev_off) {
+                                                       float* __restrict__ o, int H, const float* __restrict__ x, int W, size_t prev_off, int from) {
     constexpr int D = 64 * NT;
     __shared__ wkv_floatx4 part[2][4][4][64];              // by turns, chunk, wave
     const int h = blockIdx.x, req = blockIdx.z, j0 = blockIdx.y * 16;
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
     const int t0 = cu_tokens[req], n = cu_tokens[req + 1] - t0;
-    if (n <= 0) return;
+    if (n < from) return;
     float* srow = state + (size_t)state_slots[req] * state_row;
     float* sp = srow + (size_t)h * D * D + (size_t)(wv * 16 * NT + 4 * g) * D + j0 + c;
     wkv_floatx4 S[NT];
@@ -654,14 +658,14 @@ TFF_API int tff_wkv_chunks_supported(int R, int max_tokens, int D, size_t row) {
     return (D == 64 || D == 128) && row % 4 == 0 && row < ((size_t)1 << 25) && R <= 65535 && max_tokens <= 16 * 65535;
 }
 
-// As tff_wkv_recurrence, for heads of 64 and 128; max_tokens: the longest portion; row a multiple of 4 and r, k, z, w0, u and
+// As tff_wkv_recurrence, for heads of 64 and 128 and portions of `from` tokens and more; max_tokens: the longest portion; row a multiple of 4 and r, k, z, w0, u and
 // work 16-byte aligned.
 TFF_API int tff_wkv_recurrence_chunks(const float* r, const float* k, const float* v, const float* z, size_t row, const float* w0,
                                       const float* u, float* state, size_t state_row, const int32_t* cu_tokens,
                                       const int32_t* state_slots, float* work, float* o, int T, int R, int H, int D, const float* x,
-                                      int W, size_t prev_off, int max_tokens, tff_stream_t stream) {
+                                      int W, size_t prev_off, int max_tokens, int from, tff_stream_t stream) {
     TFF_REQUIRE(r && k && v && z && w0 && u && state && cu_tokens && state_slots && work && o, "wkv_chunks: null pointer");
-    TFF_REQUIRE(R >= 0 && T >= 0 && H > 0 && max_tokens > 0 && tff_wkv_chunks_supported(R, max_tokens, D, row),
+    TFF_REQUIRE(R >= 0 && T >= 0 && H > 0 && max_tokens > 0 && from > 0 && tff_wkv_chunks_supported(R, max_tokens, D, row),
                 "wkv_chunks: %d requests of up to %d tokens, %d heads of %d (64 or 128), rows of %zu", R, max_tokens, H, D, row);
     TFF_REQUIRE(row >= (size_t)H * D && (size_t)H * D * D <= state_row && (!x || prev_off + (size_t)W <= state_row),
                 "wkv_chunks: rows of %zu, state rows of %zu do not hold %d heads of %d", row, state_row, H, D);
@@ -670,11 +674,11 @@ TFF_API int tff_wkv_recurrence_chunks(const float* r, const float* k, const floa
     if (R == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     const dim3 pieces(H, (max_tokens + 15) / 16, R), grid(H, D / 16, R);
-    if (D == 64) wkv_chunk_kernel<64><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, H);
-    else wkv_chunk_kernel<128><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, H);
+    if (D == 64) wkv_chunk_kernel<64><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, H, from);
+    else wkv_chunk_kernel<128><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, H, from);
     if (int rc = tff_check_launch("wkv_chunk")) return rc;
-    if (D == 64) wkv_scan_kernel<1><<<grid, 256, 0, s>>>(v, row, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off);
-    else wkv_scan_kernel<2><<<grid, 256, 0, s>>>(v, row, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off);
+    if (D == 64) wkv_scan_kernel<1><<<grid, 256, 0, s>>>(v, row, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off, from);
+    else wkv_scan_kernel<2><<<grid, 256, 0, s>>>(v, row, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off, from);
     return tff_check_launch("wkv_scan");
 }
 

@@ -1411,14 +1411,21 @@ def token_shift_mix(x: torch.Tensor, state: torch.Tensor, prev_off: int, mu: tor
     return out
 
 
-#: tokens of a step's longest entry from which the recurrence runs in its form for prompts
+#: tokens from which a portion runs in the recurrence's form for prompts (heads of 64 and 128).  Here and below each portion
+#: goes by its own length, so that a request's bits do not change with what else a step holds
 WKV_LONG_PORTION = 16
 
 
-#: tokens of the longest portion from which heads of 64 and 128 run in chunks of sixteen on the matrix cores: two kernels and a
+#: tokens from which a portion of heads of 64 and 128 runs in chunks of sixteen on the matrix cores: two kernels and a
 #: workspace for one kernel.  Called from here, us for 96 tokens of 64 heads of 64 27 token by token, 22 - 29 in chunks; 128 33 / 23;
 #: 400 97 / 38
 WKV_CHUNKS_MIN_TOKENS = 128
+
+
+def _portions_between(batch, low: int, high: int) -> bool:
+    """Whether the step has a portion of ``low`` tokens and more but fewer than ``high`` (yes, where the host does not hold them)."""
+    cu = getattr(batch, "host_cu_tokens", None)
+    return cu is None or any(low <= b - a < high for a, b in zip(cu, cu[1:]))
 
 
 def wkv_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tensor, w0: torch.Tensor,
@@ -1453,19 +1460,23 @@ def wkv_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.T
         return o
     longest = int(getattr(batch, "max_new_tokens", 0) or 0)
     L = _lib.load()
+    below = 0                   # portions of so many tokens and more are done (0: none is)
     if longest >= WKV_CHUNKS_MIN_TOKENS and L.tff_wkv_chunks_supported(batch.num_reqs, longest, D, r.stride(0)) \
             and all(t.data_ptr() % 16 == 0 for t in (r, k, z, w0, u)):
+        below = WKV_CHUNKS_MIN_TOKENS
         work = torch.empty(L.tff_wkv_chunks_workspace_bytes(T, batch.num_reqs, H, D) // 4, dtype=torch.float32, device=r.device)
         _lib.check(L.tff_wkv_recurrence_chunks(
             r.data_ptr(), k.data_ptr(), v.data_ptr(), z.data_ptr(), r.stride(0), w0.data_ptr(), u.data_ptr(), state.data_ptr(), row,
             batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), work.data_ptr(), o.data_ptr(), T, batch.num_reqs, H, D, _ptr(x), W,
-            int(prev_off), longest, _stream()))
-        return o
-    _lib.check(L.tff_wkv_recurrence(r.data_ptr(), k.data_ptr(), v.data_ptr(), z.data_ptr(), r.stride(0),
-                                    w0.data_ptr(), u.data_ptr(), state.data_ptr(), row,
-                                    batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), o.data_ptr(),
-                                    batch.num_reqs, H, D, _ptr(x), W, int(prev_off),
-                                    1 if longest >= WKV_LONG_PORTION else 0, _stream()))
+            int(prev_off), longest, below, _stream()))
+    split = D in (64, 128) and longest >= WKV_LONG_PORTION
+    for from_, long_portions in ((WKV_LONG_PORTION, 1), (1, 0)) if split else ((1, 0),):
+        if not split or _portions_between(batch, from_, below or longest + 1):
+            _lib.check(L.tff_wkv_recurrence(r.data_ptr(), k.data_ptr(), v.data_ptr(), z.data_ptr(), r.stride(0),
+                                            w0.data_ptr(), u.data_ptr(), state.data_ptr(), row,
+                                            batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), o.data_ptr(),
+                                            batch.num_reqs, H, D, _ptr(x), W, int(prev_off), long_portions, from_, below, _stream()))
+        below = from_
     return o
 
 
