@@ -13,11 +13,29 @@ def _lib():
 
 def test_wkv_chunks_up_to_what_a_launch_holds():
     L = _lib()
-    for tokens, fits in ((128, 1), (16 * 65535, 1), (16 * 65535 + 1, 0), ((1 << 20) - 1, 0), (1 << 20, 0)):
-        assert L.tff_wkv_chunks_supported(3, tokens, 64, 4096) == fits, tokens
-    assert L.tff_wkv_chunks_supported(65535, 128, 128, 4096) == 1 and L.tff_wkv_chunks_supported(65536, 128, 128, 4096) == 0
-    assert [L.tff_wkv_chunks_supported(1, 128, D, 4096) for D in (48, 64, 96, 128, 256)] == [0, 1, 0, 1, 0]
-    assert [L.tff_wkv_chunks_supported(1, 128, 64, row) for row in (4098, (1 << 25) - 4, 1 << 25)] == [0, 1, 0]
+    for tokens, heads, fits in ((128, 64, 1), (16 * 65535 + 1, 64, 1), (1 << 30, 31, 1), (1 << 30, 32, 0), (1 << 30, 64, 0)):
+        assert L.tff_wkv_chunks_supported(tokens, 3, heads, 64, 4096) == fits, tokens
+    assert L.tff_wkv_chunks_supported(128, 65535, 1, 128, 4096) == 1 and L.tff_wkv_chunks_supported(128, 65536, 1, 128, 4096) == 0
+    assert [L.tff_wkv_chunks_supported(128, 1, 1, D, 4096) for D in (48, 64, 96, 128, 256)] == [0, 1, 0, 1, 0]
+    assert [L.tff_wkv_chunks_supported(128, 1, 1, 64, row) for row in (4098, (1 << 25) - 4, 1 << 25)] == [0, 1, 0]
+
+
+def test_every_chunk_of_a_step_has_a_place_of_its_own():
+    """The numbering that the chunks' kernels and their workspaces share: place t / 16 + r, T / 16 + R places, and the way back
+    from a place to its request (the last one whose first place is not behind it)."""
+    import random
+    rng = random.Random(1)
+    for _ in range(300):
+        ns = [rng.choice((0, 1, 2, 15, 16, 17, 31, 32, 33, 96, rng.randrange(300))) for _ in range(rng.randrange(1, 150))]
+        cu = [sum(ns[:i]) for i in range(len(ns) + 1)]
+        seen = {}
+        for r, n in enumerate(ns):
+            for i in range(-(-n // 16)):
+                place = (cu[r] + 16 * i) // 16 + r
+                assert place == cu[r] // 16 + r + i and place not in seen and place < cu[-1] // 16 + len(ns)
+                seen[place] = r
+        for place, r in seen.items():
+            assert sum(cu[q] // 16 + q <= place for q in range(len(ns))) - 1 == r
 
 
 def test_gated_delta_chunks_up_to_32_bit_offsets():
@@ -36,7 +54,7 @@ def test_gated_delta_chunks_up_to_32_bit_offsets():
     assert L.tff_gdelta_chunks_supported(1, 3, 1, 64, 64, 4096) == 0 and L.tff_gdelta_chunks_supported(1, 4, 2, 64, 64, 4098) == 0
 
 
-@pytest.mark.parametrize("longest,chunks", [(127, False), (128, True), (16 * 65535, True), (16 * 65535 + 1, False), ((1 << 20) - 1, False)])
+@pytest.mark.parametrize("longest,chunks", [(127, False), (128, True), (16 * 65535, True), (16 * 65535 + 1, True), ((1 << 20) - 1, True)])
 def test_wkv_dispatch_keeps_to_the_rule(monkeypatch, longest, chunks):
     """The op calls the entry for chunks exactly where the rule takes the step (the entries themselves are not run)."""
     from tffinfer_amd.kernels import ops

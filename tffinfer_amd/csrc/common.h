@@ -114,6 +114,20 @@ __device__ __forceinline__ float rows_sum(float v) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Chunks of sixteen tokens of a step's portions have places in a workspace: the chunk that starts at token t of the step, of request
+// r, lies at place t / 16 + r (T / 16 + R places hold those of R requests with T tokens; a place may be empty).  The request
+// whose chunks place p can be of, the same in every lane; a wave looks at 64 requests at a time.
+__device__ __forceinline__ int chunk_place_request(const int32_t* __restrict__ cu_tokens, int R, int p) {
+    int upto = 0;                                          // requests whose first place is not behind p
+    for (int r0 = 0; r0 < R; r0 += 64) {
+        const int r = r0 + (int)(threadIdx.x & 63);
+        const int here = __popcll(__ballot(r < R && cu_tokens[min(r, R - 1)] / 16 + r <= p));
+        upto += here;
+        if (here < 64) break;
+    }
+    return __builtin_amdgcn_readfirstlane(upto - 1);       // (request 0 begins at place 0)
+}
+
 // Copies 16 bytes a lane from global memory straight into LDS: lane i's bytes land at
 // lds_wave_base + 16 i (global_load_lds_dwordx4; the LDS base travels in M0 and is the same for
 // the whole wave).  It is written as inline assembly on purpose: the compiler's own builtin

@@ -366,14 +366,13 @@ TFF_API int tff_wkv_recurrence(const float* r, const float* k, const float* v, c
                                const float* u, float* state, size_t state_row, const int32_t* cu_tokens,
                                const int32_t* state_slots, float* o, int R, int H, int D, const float* x, int W,
                                size_t prev_off, int long_portions, int from, int below, tff_stream_t stream);
-// The same for the portions of `from` tokens and more (max_tokens: the longest), in chunks of sixteen tokens on the float32 matrix
-// cores: heads of 64 and 128.
-TFF_API int tff_wkv_chunks_supported(int R, int max_tokens, int D, size_t row);
+// The same for the portions of `from` tokens and more, in chunks of sixteen tokens on the float32 matrix cores: heads of 64 and 128.
+TFF_API int tff_wkv_chunks_supported(int T, int R, int H, int D, size_t row);
 TFF_API size_t tff_wkv_chunks_workspace_bytes(int T, int R, int H, int D);
 TFF_API int tff_wkv_recurrence_chunks(const float* r, const float* k, const float* v, const float* z, size_t row, const float* w0,
                                       const float* u, float* state, size_t state_row, const int32_t* cu_tokens,
                                       const int32_t* state_slots, float* work, float* o, int T, int R, int H, int D, const float* x,
-                                      int W, size_t prev_off, int max_tokens, int from, tff_stream_t stream);
+                                      int W, size_t prev_off, int from, tff_stream_t stream);
 
 // out = o / sqrt(mean over each head of o^2 + eps) * nw * silu(g); g rows g_row elements apart.
 TFF_API int tff_head_norm_gate(const float* o, const float* g, size_t g_row, const float* nw, float eps, void* out, int T,
@@ -398,14 +397,14 @@ TFF_API int tff_gdelta_prep(const float* proj, size_t ldp, const float* wconv, i
 TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
                                   size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* o,
                                   int R, int H, int G, int D, int E, int max_tokens, int below, tff_stream_t stream);
-// The same for the portions of `from` tokens and more (max_tokens: the longest), in chunks of sixteen tokens on the float32 matrix cores: head sizes of
+// The same for the portions of `from` tokens and more, in chunks of sixteen tokens on the float32 matrix cores: head sizes of
 // 64, 128 and 256, what tff_gdelta_chunks_supported says; work: tff_gdelta_chunks_workspace_bytes.  A token's result depends on where its portion
 // began, beyond rounding it does not.
 TFF_API size_t tff_gdelta_chunks_workspace_bytes(int T, int R, int H);
 TFF_API int tff_gdelta_chunks_supported(int R, int H, int G, int D, int E, size_t state_row);
 TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
                                          size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* work,
-                                         float* o, int T, int R, int H, int G, int D, int E, int max_tokens, int from, tff_stream_t stream);
+                                         float* o, int T, int R, int H, int G, int D, int E, int from, tff_stream_t stream);
 
 // out[t * out_row + h * E + e] = o[t, h, e] / sqrt(mean over e of o^2 + eps) * w[e] * silu(g[t * g_row + h * E + e]) * scale
 TFF_API int tff_head_norm_silu_gate(const float* o, const float* g, size_t g_row, const float* w, float eps, float scale,

@@ -457,15 +457,19 @@ __device__ __forceinline__ wkv_floatx4 wkv_mfma16(const wkv_floatx4& a, const wk
 }
 constexpr int wkv_work(int D) { return 33 * D + 256; }
 
+// A block per place of the workspace and head (heads fastest), whatever the portions' lengths: a grid of the longest portion's chunks by
+// requests was mostly blocks without work where one long portion met many decoding requests (2,048 tokens beside 47, 64 heads of
+// 64: the whole recurrence 250 us, now 167).
 template <int D>
 __global__ __launch_bounds__(64) void wkv_chunk_kernel(const float* __restrict__ r, const float* __restrict__ k,
                                                        const float* __restrict__ z, size_t row, const float* __restrict__ w0,
                                                        const float* __restrict__ u, const int32_t* __restrict__ cu_tokens,
-                                                       float* __restrict__ work, int H, int from) {
+                                                       float* __restrict__ work, int R, int H, int from) {
     constexpr int M = D / 16, LDR = D + 4;
     __shared__ __attribute__((aligned(16))) float ks[16 * LDR], ws[16 * LDR];
-    const int h = blockIdx.x, req = blockIdx.z, lane = threadIdx.x, c = lane & 15, g = lane >> 4;
-    const int t0 = cu_tokens[req], n = cu_tokens[req + 1] - t0, first = blockIdx.y * 16;
+    const int place = blockIdx.x / H, h = blockIdx.x - place * H, lane = threadIdx.x, c = lane & 15, g = lane >> 4;
+    const int req = chunk_place_request(cu_tokens, R, place);
+    const int t0 = cu_tokens[req], n = cu_tokens[req + 1] - t0, first = (place - t0 / 16 - req) * 16;
     if (n < from || first >= n) return;
     const bool live = first + c < n;                      // (tokens past the portion's end: no key, no decay)
     const size_t at = (size_t)(t0 + min(first + c, n - 1)) * row + (size_t)h * D + 4 * g;
@@ -650,32 +654,33 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(const float* __restrict__
 }
 
 TFF_API size_t tff_wkv_chunks_workspace_bytes(int T, int R, int H, int D) {
-    return ((size_t)T / 16 + R + 1) * H * wkv_work(D) * sizeof(float);
+    return ((size_t)T / 16 + R) * H * wkv_work(D) * sizeof(float);
 }
 
-// (the chunks of a portion are the launch's second dimension; a lane's offset within sixteen rows is 32 bits of bytes)
-TFF_API int tff_wkv_chunks_supported(int R, int max_tokens, int D, size_t row) {
-    return (D == 64 || D == 128) && row % 4 == 0 && row < ((size_t)1 << 25) && R <= 65535 && max_tokens <= 16 * 65535;
+// (a lane's offset within sixteen rows is 32 bits of bytes)
+TFF_API int tff_wkv_chunks_supported(int T, int R, int H, int D, size_t row) {
+    return (D == 64 || D == 128) && row % 4 == 0 && row < ((size_t)1 << 25) && R <= 65535 && ((size_t)T / 16 + R) * H < ((size_t)1 << 31);
 }
 
-// As tff_wkv_recurrence, for heads of 64 and 128 and portions of `from` tokens and more; max_tokens: the longest portion; row a multiple of 4 and r, k, z, w0, u and
+// As tff_wkv_recurrence, for heads of 64 and 128 and portions of `from` tokens and more; row a multiple of 4 and r, k, z, w0, u and
 // work 16-byte aligned.
 TFF_API int tff_wkv_recurrence_chunks(const float* r, const float* k, const float* v, const float* z, size_t row, const float* w0,
                                       const float* u, float* state, size_t state_row, const int32_t* cu_tokens,
                                       const int32_t* state_slots, float* work, float* o, int T, int R, int H, int D, const float* x,
-                                      int W, size_t prev_off, int max_tokens, int from, tff_stream_t stream) {
+                                      int W, size_t prev_off, int from, tff_stream_t stream) {
     TFF_REQUIRE(r && k && v && z && w0 && u && state && cu_tokens && state_slots && work && o, "wkv_chunks: null pointer");
-    TFF_REQUIRE(R >= 0 && T >= 0 && H > 0 && max_tokens > 0 && from > 0 && tff_wkv_chunks_supported(R, max_tokens, D, row),
-                "wkv_chunks: %d requests of up to %d tokens, %d heads of %d (64 or 128), rows of %zu", R, max_tokens, H, D, row);
+    TFF_REQUIRE(R >= 0 && T >= 0 && H > 0 && from > 0 && tff_wkv_chunks_supported(T, R, H, D, row),
+                "wkv_chunks: %d requests of %d tokens, %d heads of %d (64 or 128), rows of %zu", R, T, H, D, row);
     TFF_REQUIRE(row >= (size_t)H * D && (size_t)H * D * D <= state_row && (!x || prev_off + (size_t)W <= state_row),
                 "wkv_chunks: rows of %zu, state rows of %zu do not hold %d heads of %d", row, state_row, H, D);
     TFF_REQUIRE(((uintptr_t)r % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)z % 16) == 0 && ((uintptr_t)w0 % 16) == 0 &&
                 ((uintptr_t)u % 16) == 0 && ((uintptr_t)work % 16) == 0, "wkv_chunks: operands must be 16-byte aligned");
     if (R == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 pieces(H, (max_tokens + 15) / 16, R), grid(H, D / 16, R);
-    if (D == 64) wkv_chunk_kernel<64><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, H, from);
-    else wkv_chunk_kernel<128><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, H, from);
+    const dim3 grid(H, D / 16, R);
+    const unsigned pieces = (unsigned)((T / 16 + R) * H);
+    if (D == 64) wkv_chunk_kernel<64><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, R, H, from);
+    else wkv_chunk_kernel<128><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, R, H, from);
     if (int rc = tff_check_launch("wkv_chunk")) return rc;
     if (D == 64) wkv_scan_kernel<1><<<grid, 256, 0, s>>>(v, row, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off, from);
     else wkv_scan_kernel<2><<<grid, 256, 0, s>>>(v, row, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off, from);

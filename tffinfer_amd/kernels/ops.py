@@ -1461,14 +1461,14 @@ def wkv_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.T
     longest = int(getattr(batch, "max_new_tokens", 0) or 0)
     L = _lib.load()
     below = 0                   # portions of so many tokens and more are done (0: none is)
-    if longest >= WKV_CHUNKS_MIN_TOKENS and L.tff_wkv_chunks_supported(batch.num_reqs, longest, D, r.stride(0)) \
+    if longest >= WKV_CHUNKS_MIN_TOKENS and L.tff_wkv_chunks_supported(T, batch.num_reqs, H, D, r.stride(0)) \
             and all(t.data_ptr() % 16 == 0 for t in (r, k, z, w0, u)):
         below = WKV_CHUNKS_MIN_TOKENS
         work = torch.empty(L.tff_wkv_chunks_workspace_bytes(T, batch.num_reqs, H, D) // 4, dtype=torch.float32, device=r.device)
         _lib.check(L.tff_wkv_recurrence_chunks(
             r.data_ptr(), k.data_ptr(), v.data_ptr(), z.data_ptr(), r.stride(0), w0.data_ptr(), u.data_ptr(), state.data_ptr(), row,
             batch.cu_tokens.data_ptr(), batch.state_slots.data_ptr(), work.data_ptr(), o.data_ptr(), T, batch.num_reqs, H, D, _ptr(x), W,
-            int(prev_off), longest, below, _stream()))
+            int(prev_off), below, _stream()))
     split = D in (64, 128) and longest >= WKV_LONG_PORTION
     for from_, long_portions in ((WKV_LONG_PORTION, 1), (1, 0)) if split else ((1, 0),):
         if not split or _portions_between(batch, from_, below or longest + 1):
@@ -2094,7 +2094,7 @@ def gated_delta(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, d
         work = torch.empty(L.tff_gdelta_chunks_workspace_bytes(T, batch.num_reqs, H) // 4, dtype=torch.float32, device=proj.device)
         _lib.check(L.tff_gdelta_recurrence_chunks(
             pre.data_ptr(), proj.data_ptr(), ldp, state.data_ptr(), row, tail, taps, batch.cu_tokens.data_ptr(),
-            batch.state_slots.data_ptr(), work.data_ptr(), o.data_ptr(), T, batch.num_reqs, H, G, D, E, longest,
+            batch.state_slots.data_ptr(), work.data_ptr(), o.data_ptr(), T, batch.num_reqs, H, G, D, E,
             GDELTA_CHUNKS_MIN_TOKENS, stream))
         below = GDELTA_CHUNKS_MIN_TOKENS
         longest = _longest_below(batch, below)
