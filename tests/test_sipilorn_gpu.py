@@ -225,6 +225,43 @@ def test_delta_rule_in_chunks_of_sixteen(H, G, D, E, taps, extreme):
         assert float(state[1].abs().max()) == 0
 
 
+@pytest.mark.parametrize("H,G,D,E", [(2, 1, 64, 20), (2, 2, 128, 64), (2, 2, 256, 36)])
+@pytest.mark.parametrize("channel", ["v", "k", "q", "b", "a", "last v", "state"])
+def test_delta_rule_what_is_not_finite_reaches_later_tokens_only(H, G, D, E, channel):
+    """An infinity or NaN in one projection of token 105 of a portion in chunks, of its last token, or in the state: the values that are
+    not finite are those that are not so token by token, every other one is what it was within the bound of that form, and other
+    heads (keys and queries serve a head's group) keep their bits throughout."""
+    ops = _ops()
+    T, taps = 170, 1
+    proj, conv, a_log, dt = _delta_case(T, H, G, D, E, taps, D + E)
+    C = 2 * G * D + H * E
+    dev = [x.to(DEV) for x in (conv, a_log, dt)]
+    begin = torch.randn(1, H * E * D, generator=torch.Generator().manual_seed(1)).to(DEV)
+
+    def outputs(p, first, pieces):
+        out, state = [], first.clone()
+        for at in range(0, T, pieces):
+            n = min(pieces, T - at)
+            out.append(ops.gated_delta(p[at:at + n].contiguous().to(DEV), *dev, state, _batch([n], [at], [0]), H, G, D, E))
+        return torch.cat(out, 0).view(T, H, E), state.view(H, E, D)
+    clean, clean_state = outputs(proj, begin, T)
+    t = {"last v": T - 1, "state": 0}.get(channel, 105)
+    column = {"v": 2 * G * D + 3, "last v": 2 * G * D + 3, "k": G * D + 5, "q": 5, "b": C, "a": C + H, "state": 0}[channel]
+    for x in (float("nan"),) if channel in ("k", "q", "b", "a") else (float("inf"), float("nan")):
+        bad, first = proj.clone(), begin.clone()
+        if channel == "state":
+            first[0, 7] = x
+        else:
+            bad[t, column] = x
+        (got, state), (few, few_state) = outputs(bad, first, T), outputs(bad, first, 50)
+        touched = H // G if channel in ("k", "q") else 1
+        assert torch.equal(got[:, touched:], clean[:, touched:]) and torch.equal(state[touched:], clean_state[touched:])
+        assert torch.equal(torch.isfinite(got), torch.isfinite(few)) and not bool(torch.isfinite(got).all())
+        assert torch.equal(torch.isfinite(state), torch.isfinite(few_state))
+        if t:
+            assert _err(got[:t].flatten(1), clean[:t].flatten(1)) < 3e-5
+
+
 @pytest.mark.parametrize("H,G,D,E", [(2, 1, 64, 20), (4, 2, 128, 128), (2, 2, 256, 36)])
 @pytest.mark.parametrize("ns", [[1, 200, 2], [95, 96, 0, 4, 150, 1], [300, 1, 1, 97]])
 def test_delta_rule_of_a_portion_is_its_own_in_any_step(H, G, D, E, ns):

@@ -229,22 +229,15 @@ __device__ __forceinline__ float gd_token(float (&S)[KPL], const float (&kk)[KPL
     return row16_sum(b);
 }
 
-// For steps in which every request brings a few tokens (decoding): no LDS and no barrier.  A row of sixteen lanes
-// shares a value channel as above, but lane s takes the key channels s, s + 16, ...: a load or store of the state
+// A portion of one head and sixteen value channels from j0 on, token by token, by a block of 256: no LDS and no barrier.  A row of
+// sixteen lanes shares a value channel as above, but lane s takes the key channels s, s + 16, ...: a load or store of the state
 // is sixteen neighbouring floats a row, and k and q come straight from the prepared rows.
 template <int KPL>
-__global__ __launch_bounds__(256) void gdelta_recurrence_few_kernel(
-    const float* __restrict__ pre, const float* __restrict__ proj, size_t ldp, float* __restrict__ state, size_t state_row,
-    size_t tail_off, int taps, const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ state_slots,
-    float* __restrict__ o, int H, int G, int D, int E, int below) {
-    const int h = blockIdx.y, r = blockIdx.z, j0 = blockIdx.x * 16;
+__device__ __forceinline__ void gd_portion(const float* __restrict__ pre, int t0, int n, float* __restrict__ srow, float* __restrict__ o,
+                                           int h, int gk, int H, int G, int D, int E, int j0) {
     const int tid = threadIdx.x, s = tid & 15, j = j0 + (tid >> 4), jc = min(j, E - 1);
     const int C = 2 * G * D + H * E;
     const size_t ldq = (size_t)C + 2 * H;
-    const int gk = h / (H / G);
-    const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0;
-    if (n >= below) return;                                // (a portion for the kernels over chunks)
-    float* srow = state + (size_t)state_slots[r] * state_row;
     float* sp = srow + ((size_t)h * E + jc) * D + s;
     const bool row_live = j < E;
     float S[KPL];
@@ -270,6 +263,19 @@ __global__ __launch_bounds__(256) void gdelta_recurrence_few_kernel(
         for (int m = 0; m < KPL; ++m)
             if (s + 16 * m < D) sp[16 * m] = S[m];
     }
+}
+
+// For steps in which every request brings a few tokens (decoding).
+template <int KPL>
+__global__ __launch_bounds__(256) void gdelta_recurrence_few_kernel(
+    const float* __restrict__ pre, const float* __restrict__ proj, size_t ldp, float* __restrict__ state, size_t state_row,
+    size_t tail_off, int taps, const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ state_slots,
+    float* __restrict__ o, int H, int G, int D, int E, int below) {
+    const int h = blockIdx.y, r = blockIdx.z, gk = h / (H / G);
+    const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0;
+    if (n >= below) return;                                // (a portion for the kernels over chunks)
+    float* srow = state + (size_t)state_slots[r] * state_row;
+    gd_portion<KPL>(pre, t0, n, srow, o, h, gk, H, G, D, E, blockIdx.x * 16);
     if (blockIdx.x == 0) gd_keep_inputs(proj, ldp, srow + tail_off, taps, t0, n, h, gk, H, G, D, E);
 }
 
@@ -658,7 +664,12 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
         if (i >= chunks) break;
     }
     if (chunks % WV != 0) outputs(chunks - chunks % WV);
-    if (live) {
+    // Where a u is not finite the zeros above the diagonals do not keep it from earlier tokens (0 x inf is not 0).  It is then in every
+    // element of its channel of S for good: such a portion's sixteen channels are worked through once more token by token, from the
+    // state that still stands.
+    if (__syncthreads_or(!(fabsf(S[0][0]) < INFINITY))) {
+        gd_portion<D / 16>(pre, t0, n, srow, o, h, gk, H, G, D, E, j0);
+    } else if (live) {
 #pragma unroll
         for (int m = 0; m < NT; ++m) *reinterpret_cast<gd_floatx4*>(sp + 16 * m) = S[m];
     }
