@@ -173,6 +173,40 @@ def test_output_norm_and_depth_at_the_edges_of_a_block(group):
     assert torch.equal(deep[-1].cpu(), x) and torch.equal(deep[:-1].cpu(), hist[:-1])
 
 
+@pytest.mark.parametrize("H,D", [(2, 64), (2, 128)])
+@pytest.mark.parametrize("what", ["v", "k", "r", "z", "last v", "state"])
+def test_recurrence_what_is_not_finite_reaches_later_tokens_only(H, D, what):
+    """An infinity or NaN in a token's row of a portion in chunks, in its last token's, or in the state: what is not finite is so
+    token by token as well, every other value is what it was within the bound of that form, the other head keeps its bits."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(D)
+    T = 170
+    rows = {n: torch.randn(T, H * D, generator=g).to(DEV) for n in "rkvz"}
+    w0, u = torch.randn(H * D, generator=g).to(DEV), torch.randn(H * D, generator=g).to(DEV)
+    begin = torch.randn(1, H * D * D, generator=g).to(DEV)
+
+    def outputs(rows, first, pieces):
+        out, state = [], first.clone()
+        for at in range(0, T, pieces):
+            part = [rows[n][at:at + pieces].contiguous() for n in "rkvz"]
+            out.append(ops.wkv_recurrence(*part, w0, u, state, _batch([part[0].shape[0]], [at], [0]), H, D))
+        return torch.cat(out, 0).view(T, H, D), state.view(H, D, D)
+    clean, clean_state = outputs(rows, begin, T)
+    t = {"last v": T - 1, "state": 0}.get(what, 105)
+    for x in (float("nan"),) if what in ("k", "r", "z") else (float("inf"), float("nan")):
+        bad, first = {n: y.clone() for n, y in rows.items()}, begin.clone()
+        if what == "state":
+            first[0, 7] = x
+        else:
+            bad[what[-1]][t, 5] = x
+        (got, state), (few, few_state) = outputs(bad, first, T), outputs(bad, first, 50)
+        assert torch.equal(got[:, 1:], clean[:, 1:]) and torch.equal(state[1:], clean_state[1:])
+        assert torch.equal(torch.isfinite(got), torch.isfinite(few)) and not bool(torch.isfinite(got).all())
+        assert torch.equal(torch.isfinite(state), torch.isfinite(few_state))
+        if t:
+            assert _err(got[:t].flatten(1), clean[:t].flatten(1)) < 2e-5
+
+
 @pytest.mark.parametrize("H,D", [(2, 64), (1, 128), (2, 48)])
 @pytest.mark.parametrize("portions", [(1, 200, 2), (15, 16, 0, 127, 128, 1), (17, 3), (140, 300), (150, 20)])
 def test_recurrence_of_a_portion_is_its_own_in_any_step(H, D, portions):

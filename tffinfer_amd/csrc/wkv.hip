@@ -561,10 +561,43 @@ __global__ __launch_bounds__(64) void wkv_chunk_kernel(const float* __restrict__
     }
 }
 
+// A portion of one head and sixteen value channels from j0 on, token by token, by a block of 256: as wkv_recurrence_rows_kernel,
+// without its way through LDS.
+template <int KPT>
+__device__ __forceinline__ void wkv_portion(const float* __restrict__ r, const float* __restrict__ k, const float* __restrict__ v,
+                                            const float* __restrict__ z, size_t row, const float* __restrict__ w0,
+                                            const float* __restrict__ u, int t0, int n, float* __restrict__ S, float* __restrict__ o,
+                                            int h, int H, int j0) {
+    constexpr int D = 16 * KPT;
+    const int ks = threadIdx.x & 15, vi = j0 + (int)(threadIdx.x >> 4);
+    const size_t col = (size_t)h * D + ks * KPT;
+    float s[KPT];
+#pragma unroll
+    for (int i = 0; i < KPT; ++i) s[i] = S[(size_t)(ks * KPT + i) * D + vi];
+    for (int t = t0; t < t0 + n; ++t) {
+        const size_t a = (size_t)t * row;
+        const float vt = v[a + (size_t)h * D + vi];
+        float acc = 0.f;
+#pragma unroll
+        for (int i = 0; i < KPT; ++i) {
+            const float kv = k[a + col + i] * vt;
+            acc = fmaf(r[a + col + i], fmaf(u[col + i], kv, s[i]), acc);
+            s[i] = fmaf(expf(-expf(z[a + col + i] + w0[col + i])), s[i], kv);
+        }
+        acc = row16_sum(acc);
+        if (ks == 0) o[(size_t)t * H * D + (size_t)h * D + vi] = acc;
+    }
+#pragma unroll
+    for (int i = 0; i < KPT; ++i) S[(size_t)(ks * KPT + i) * D + vi] = s[i];
+}
+
 // Four waves of NT tiles of 16 key channels (D = 64 NT).  Four chunks between two barriers: after the barrier each wave has one
 // chunk's output to put together, so that no wave waits for another's.
 template <int NT>
-__global__ __launch_bounds__(256) void wkv_scan_kernel(const float* __restrict__ v, size_t row, float* __restrict__ state, size_t state_row,
+__global__ __launch_bounds__(256) void wkv_scan_kernel(const float* __restrict__ r, const float* __restrict__ k,
+                                                       const float* __restrict__ v, const float* __restrict__ z, size_t row,
+                                                       const float* __restrict__ w0, const float* __restrict__ u,
+                                                       float* __restrict__ state, size_t state_row,
                                                        const int32_t* __restrict__ cu_tokens,
                                                        const int32_t* __restrict__ state_slots, const float* __restrict__ work,
                                                        float* __restrict__ o, int H, const float* __restrict__ x, int W, size_t prev_off, int from) {
@@ -643,10 +676,17 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(const float* __restrict__
                 if (16 * mine + 4 * g + q < n) op[(size_t)q * H * D] = y[q];
         }
     }
+    // A value that is not finite meets the zero weights of earlier tokens of its chunk (0 x inf is not 0).  It is then in every element of
+    // its channel of S for good: such a portion's sixteen channels are worked through once more token by token, from the state
+    // that still stands.
+    if (__syncthreads_or(!(fabsf(S[0][0]) < INFINITY))) {
+        wkv_portion<D / 16>(r, k, v, z, row, w0, u, t0, n, srow + (size_t)h * D * D, o, h, H, j0);
+    } else {
 #pragma unroll
-    for (int m = 0; m < NT; ++m)
+        for (int m = 0; m < NT; ++m)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sp[(size_t)(16 * m + e) * D] = S[m][e];
+            for (int e = 0; e < 4; ++e) sp[(size_t)(16 * m + e) * D] = S[m][e];
+    }
     if (h == 0 && blockIdx.y == 0 && x) {
         const float* lastx = x + (size_t)(t0 + n - 1) * W;
         for (int e = tid; e < W; e += 256) srow[prev_off + e] = lastx[e];
@@ -682,8 +722,8 @@ TFF_API int tff_wkv_recurrence_chunks(const float* r, const float* k, const floa
     if (D == 64) wkv_chunk_kernel<64><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, R, H, from);
     else wkv_chunk_kernel<128><<<pieces, 64, 0, s>>>(r, k, z, row, w0, u, cu_tokens, work, R, H, from);
     if (int rc = tff_check_launch("wkv_chunk")) return rc;
-    if (D == 64) wkv_scan_kernel<1><<<grid, 256, 0, s>>>(v, row, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off, from);
-    else wkv_scan_kernel<2><<<grid, 256, 0, s>>>(v, row, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off, from);
+    if (D == 64) wkv_scan_kernel<1><<<grid, 256, 0, s>>>(r, k, v, z, row, w0, u, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off, from);
+    else wkv_scan_kernel<2><<<grid, 256, 0, s>>>(r, k, v, z, row, w0, u, state, state_row, cu_tokens, state_slots, work, o, H, x, W, prev_off, from);
     return tff_check_launch("wkv_scan");
 }
 
