@@ -1,5 +1,5 @@
-"""Which steps the recurrences take in chunks on the matrix cores: the dispatch asks the kernels' own rule, and what the rule
-refuses stays with the forms that have no such limit."""
+"""The host's rules between kernels: which steps the recurrences take in chunks on the matrix cores (the dispatch asks the kernels' own
+rule, and what the rule refuses stays with the forms that have no such limit), and when the draw forms the maxima of runs."""
 import types
 
 import pytest
@@ -78,3 +78,20 @@ def test_wkv_dispatch_keeps_to_the_rule(monkeypatch, longest, chunks):
     batch = types.SimpleNamespace(num_reqs=1, max_new_tokens=longest, host_cu_tokens=[0, longest], cu_tokens=i32, state_slots=i32)
     ops.wkv_recurrence(r, k, v, z, torch.zeros(H * D), torch.zeros(H * D), torch.zeros(1, H * D * D), batch, H, D)
     assert called == ["tff_wkv_recurrence_chunks" if chunks else "tff_wkv_recurrence"]
+
+
+def test_the_draw_forms_maxima_only_where_they_bound_something(monkeypatch):
+    """A top_k over half the number of a row's runs (or 256) does not ask for them, nor does a small vocabulary; one row that
+    profits is enough."""
+    from tffinfer_amd.kernels import ops
+    from tffinfer_amd.sampling.params import SamplingConfig
+    from tffinfer_amd.sampling.sampler import Sampler
+    assert [ops.sample_few_limit(V) for V in (1, 16383, 16384, 16385, 32768, 65536, 151936, 1 << 20)] == [0, 0, 64, 64, 128, 256, 256, 256]
+    sampler = Sampler(torch.device("cpu"), types.SimpleNamespace(sample=lambda *a, few=False: few))
+    monkeypatch.setattr(sampler, "_send", lambda columns: [torch.from_numpy(c) for c in columns])
+
+    def asks(V, *ks):
+        return sampler.sample_on_device(torch.zeros(len(ks), V), [SamplingConfig("random", temperature=1.0, top_k=k) for k in ks], [0] * len(ks))
+    assert asks(16384, 64) and not asks(16384, 65) and not asks(16384, 0) and not asks(16000, 20)
+    assert asks(32768, 128) and not asks(32768, 200, 256) and asks(32768, 200, 20)
+    assert asks(151936, 256) and not asks(151936, 257)

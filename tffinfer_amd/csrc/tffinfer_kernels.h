@@ -542,8 +542,8 @@ TFF_API int tff_repetition_penalty(float* logits, int rows, int V, const int32_t
 // (1: off) and min_p (0: off), by inverse CDF in index order with the given
 // uniform number per row.  temperature[r] <= 0 selects the argmax.  Probabilities
 // are weighed in units of 2^-40 of the largest one (a token below that is never
-// drawn); V up to 1,048,576.  maxima: room for rows * ceil(V / 128) floats where some row has a small top_k (such rows then
-// read little more than once, spread over the chip), or null.
+// drawn); V up to 1,048,576.  maxima: room for rows * ceil(V / 128) floats where some row has a small top_k, or null (rows with a
+// top_k of at most half as many as their runs of 128 then read little more than once, spread over the chip).
 TFF_API int tff_sample(const float* logits, int32_t* out, int rows, int V,
                        const float* temperature, const int32_t* top_k, const float* top_p,
                        const float* min_p, const float* uniform, float* probs_out, float* maxima,

@@ -2297,6 +2297,12 @@ def repetition_penalty(logits: torch.Tensor, seen: torch.Tensor, cu_seen: torch.
 SAMPLE_FEW_MIN_VOCAB = 16384
 
 
+def sample_few_limit(V: int) -> int:
+    """The largest top_k for which the maxima of a row's runs of 128 logits are worth forming: the kernel's candidates are some
+    1.4 k of them for k half the number of runs, without a bound for k of it."""
+    return min(256, -(-V // 128) // 2) if V >= SAMPLE_FEW_MIN_VOCAB else 0
+
+
 def sample(logits: torch.Tensor, temperature: torch.Tensor, uniform: torch.Tensor,
            top_k: torch.Tensor | None = None, top_p: torch.Tensor | None = None,
            min_p: torch.Tensor | None = None, return_probs: bool = False, few: bool = False):

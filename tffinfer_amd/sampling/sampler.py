@@ -101,4 +101,5 @@ class Sampler:
             np.asarray([e[0] for e in eff], dtype=np.float32), np.asarray([e[1] for e in eff], dtype=np.int32),
             np.asarray([e[2] for e in eff], dtype=np.float32), np.asarray([e[3] for e in eff], dtype=np.float32),
             np.asarray([uniform_at(c.seed, i) for c, i in zip(configs, indices)], dtype=np.float32)])
-        return self.ops.sample(logits, temperature, u, top_k, top_p, min_p, few=any(0 < e[1] <= 256 for e in eff))
+        limit = _ops.sample_few_limit(logits.shape[1])
+        return self.ops.sample(logits, temperature, u, top_k, top_p, min_p, few=any(0 < e[1] <= limit for e in eff))
