@@ -173,6 +173,20 @@ def test_output_norm_and_depth_at_the_edges_of_a_block(group):
     assert torch.equal(deep[-1].cpu(), x) and torch.equal(deep[:-1].cpu(), hist[:-1])
 
 
+@pytest.mark.parametrize("group,planes", [(1025, 3), (1025, 5), (2048, 5), (2049, 1), (2600, 3)])
+def test_output_norm_of_many_rows_is_that_of_few(group, planes):
+    """More blocks than are there at once take another form of the kernel: the same sums, the same bits."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(group)
+    n, groups = 520, 2
+    H = groups * group
+    d, x, w = torch.randn(planes, n, H, generator=g), torch.randn(n, H, generator=g), torch.randn(H, generator=g).to(DEV)
+    many, few = x.to(DEV), x[:7].to(DEV)
+    o_many = ops.group_rmsnorm_add(many, d.to(DEV), w, groups, 1e-6, torch.float32)
+    o_few = ops.group_rmsnorm_add(few, d[:, :7].contiguous().to(DEV), w, groups, 1e-6, torch.float32)
+    assert torch.equal(many[:7], few) and torch.equal(o_many[:7], o_few)
+
+
 @pytest.mark.parametrize("H,D", [(2, 64), (2, 128)])
 @pytest.mark.parametrize("what", ["v", "k", "r", "z", "last v", "state"])
 def test_recurrence_what_is_not_finite_reaches_later_tokens_only(H, D, what):

@@ -17,10 +17,11 @@
 #define GN_THREADS 256
 
 // One block per (row, group); GN_ITS x 256 elements of a group pass through memory once: 2048 at most.  Bound by latency for few
-// rows and by memory for many: the planes were added an element at a time, and weight and stream asked for after the sum over the
-// group.  With all loads under way first, us before / now, the same sums in the same order: 2 rows of 4096 in one group 8.2 / 5.7, in four
-// with four planes 5.1 / 3.8, 8 rows of 6000 14.1 / 10.4, 1,500 rows of 4096 in eight groups 25.0 / 19.9, in two with eight planes 52.6 / 50.1.
-template <typename TO, int GN_ITS>
+// rows and by memory for many: element by element the planes are added one load after the other, and weight and stream asked for after
+// the sum over the group.  EARLY: all loads under way first, the same sums in the same order; us without / with: 2 rows of 4096 in one
+// group 8.2 / 5.7, in four with four planes 5.1 / 3.8, 8 rows of 6000 14.1 / 10.4, 400 rows of 8192 24.8 / 16.5, 1,500 rows of 4096 in eight
+// groups 25.0 / 19.9, in two with eight planes 52.6 / 50.1.
+template <typename TO, int GN_ITS, bool EARLY>
 __global__ __launch_bounds__(GN_THREADS) void group_rmsnorm_add_kernel(
     float* __restrict__ resid, const float* __restrict__ delta, int planes, size_t plane,
     const int32_t* __restrict__ rows, const float* __restrict__ w, int groups, float eps,
@@ -44,14 +45,16 @@ __global__ __launch_bounds__(GN_THREADS) void group_rmsnorm_add_kernel(
 #pragma unroll
     for (int it = 0; it < GN_ITS; ++it) {
         const int j = min(tid + it * GN_THREADS, Hg - 1);
-        cache[it] = dl[j];
-        wr[it] = wg[j];
-        xr[it] = x ? x[j] : 0.f;
+        cache[it] = EARLY ? dl[j] : term(j);
+        wr[it] = EARLY ? wg[j] : 0.f;
+        xr[it] = EARLY && x ? x[j] : 0.f;
     }
+    if constexpr (EARLY) {
 #pragma unroll 4
-    for (int p = 1; p < planes; ++p)
+        for (int p = 1; p < planes; ++p)
 #pragma unroll
-        for (int it = 0; it < GN_ITS; ++it) cache[it] += dl[p * plane + min(tid + it * GN_THREADS, Hg - 1)];
+            for (int it = 0; it < GN_ITS; ++it) cache[it] += dl[p * plane + min(tid + it * GN_THREADS, Hg - 1)];
+    }
     float ss = 0.f;
 #pragma unroll
     for (int it = 0; it < GN_ITS; ++it)
@@ -73,7 +76,7 @@ __global__ __launch_bounds__(GN_THREADS) void group_rmsnorm_add_kernel(
 #pragma unroll
     for (int it = 0; it < GN_ITS; ++it) {
         const int j = tid + it * GN_THREADS;
-        if (j < Hg) emit(j, cache[it], wr[it], xr[it]);
+        if (j < Hg) emit(j, cache[it], EARLY ? wr[it] : wg[j], EARLY ? xr[it] : x ? x[j] : 0.f);
     }
     for (int j = tid + GN_ITS * GN_THREADS; j < Hg; j += GN_THREADS) emit(j, term(j), wg[j], x ? x[j] : 0.f);
 }
@@ -87,14 +90,20 @@ TFF_API int tff_group_rmsnorm_add(float* resid, const float* delta, int planes, 
     if (n == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     const int Hg = H / groups;
-#define GN_LAUNCH(T, ITS) \
-    group_rmsnorm_add_kernel<T, ITS><<<n * groups, GN_THREADS, 0, s>>>(resid, delta, planes, plane, rows, w, groups, eps, (T*)out, H)
-#define GN_BY_SIZE(T)                               \
-    do {                                            \
-        if (Hg <= GN_THREADS) GN_LAUNCH(T, 1);      \
-        else if (Hg <= 2 * GN_THREADS) GN_LAUNCH(T, 2); \
-        else if (Hg <= 4 * GN_THREADS) GN_LAUNCH(T, 4); \
-        else GN_LAUNCH(T, 8);                       \
+    // The early loads of groups over 1024 take 117 registers, four blocks to a CU instead of eight: worth it while the blocks are there
+    // at once (1,024), and where neither a tail behind 2048 elements nor many planes keep the memory busy.  us late / early: 1,000 rows of
+    // 4096 13.9 / 12.5, 1,100 rows 14.3 / 19.4, with eight planes 60.2 / 56.7 and 60.6 / 87.8; 1,000 rows of 4096 in two groups with eight
+    // planes 31.5 / 35.9, with two 16.7 / 15.1.
+    const bool early = (long)n * groups <= 1024 || (Hg <= 8 * GN_THREADS && planes <= 4);
+#define GN_LAUNCH(T, ITS, EARLY) \
+    group_rmsnorm_add_kernel<T, ITS, EARLY><<<n * groups, GN_THREADS, 0, s>>>(resid, delta, planes, plane, rows, w, groups, eps, (T*)out, H)
+#define GN_BY_SIZE(T)                                           \
+    do {                                                        \
+        if (Hg <= GN_THREADS) GN_LAUNCH(T, 1, true);            \
+        else if (Hg <= 2 * GN_THREADS) GN_LAUNCH(T, 2, true);   \
+        else if (Hg <= 4 * GN_THREADS) GN_LAUNCH(T, 4, true);   \
+        else if (early) GN_LAUNCH(T, 8, true);                  \
+        else GN_LAUNCH(T, 8, false);                            \
     } while (0)
     if (!out || out_dtype == TFF_F32) GN_BY_SIZE(float);
     else if (out_dtype == TFF_BF16) GN_BY_SIZE(bf16_t);
