@@ -95,3 +95,16 @@ def test_the_draw_forms_maxima_only_where_they_bound_something(monkeypatch):
     assert asks(16384, 64) and not asks(16384, 65) and not asks(16384, 0) and not asks(16000, 20)
     assert asks(32768, 128) and not asks(32768, 200, 256) and asks(32768, 200, 20)
     assert asks(151936, 256) and not asks(151936, 257)
+
+
+@pytest.mark.parametrize("tiles,col_blocks", [(1, 1), (3, 2), (5, 3), (63, 3), (126, 6), (220, 4), (7, 8), (40, 11), (9, 16)])
+def test_the_experts_blocks_cover_every_tile_and_load_the_xcds_alike(tiles, col_blocks):
+    """Every (column block, tile) pair has one block of a launch for up to as many tiles and more; blocks go to the eight XCDs in turn:
+    none has more than its eighth, and each walks neighbouring pairs."""
+    L = _lib()
+    for most in (tiles, tiles + 5):
+        ids = [L.tff_experts_block(b, tiles, col_blocks) for b in range(-(-most * col_blocks // 8) * 8)]
+        assert sorted(i for i in ids if i >= 0) == list(range(tiles * col_blocks))
+        for x in range(8):
+            own = [i for i in ids[x::8] if i >= 0]
+            assert len(own) <= -(-tiles * col_blocks // 8) and own == list(range(own[0], own[0] + len(own)) if own else [])

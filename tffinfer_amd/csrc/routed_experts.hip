@@ -458,27 +458,36 @@ __device__ __forceinline__ ex_bf16x8 ex_load8(const bf16_t* p, bool ok) {
 // dealt to.
 #define EXT_KSTEP 64
 
+// What a block of the experts' products works on.  A tile of 64 pairs gives a weight element 128 flops a read: the tiles of one expert
+// must meet their weight rows in a cache, or the products run at what memory gives.  Blocks go to the eight XCDs in turn by
+// their number, each XCD with an L2 of its own; of the (column block, tile) pairs in order, tiles fastest, each XCD takes an eighth,
+// so that it sees the tiles of a column block one after the other, an expert's next to each other.  Whole column blocks to an XCD left
+// XCDs without work where there are fewer than eight or no multiple of eight, more of them the wider the blocks: us for both products so /
+// now: 256 experts, eight a token, 1,024 x 512, 64 tokens 259 / 174; 96 experts, four a token, 1,536 x 512 without a gate, 150 tokens
+// 125 / 81; 32 experts, four a token, 4,096 x 1,536, 2,048 tokens 574 / 519; 16 experts, two a token, 2,048 x 2,048 71 / 70.
+// The pair's number, or -1 for a block without one.
+__host__ __device__ __forceinline__ int ex_block(unsigned block, int tiles, int col_blocks) {
+    const int all = tiles * col_blocks, share = (all + 7) >> 3, at = (int)(block >> 3), id = (int)(block & 7) * share + at;
+    return at < share && id < all ? id : -1;
+}
+TFF_API int tff_experts_block(int block, int tiles, int col_blocks) { return ex_block((unsigned)block, tiles, col_blocks); }
+
 // MODE 0: the down product; 1: gate and up; 2: up alone, y = max(Wu h, 0)^2 (a wave's 32 weight rows are 32 outputs).
 template <int MODE, int AFR>
 __global__ __launch_bounds__(256) void experts_tiles_kernel(
     const bf16_t* __restrict__ a_rows, int a_row, const bf16_t* __restrict__ W0, const bf16_t* __restrict__ W1,
     const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_rows,
     const int32_t* __restrict__ num_tiles, const float* __restrict__ wts, int T, int top, int K, int N,
-    float limit, float act_alpha, float up_offset, bf16_t* __restrict__ y, float* __restrict__ out, int max_tiles, int col_blocks,
+    float limit, float act_alpha, float up_offset, bf16_t* __restrict__ y, float* __restrict__ out, int col_blocks,
     int ldw, int weight_input) {
     // weight_input: a pair's weight multiplies what goes into its expert (both first products, before clamps
     // and activation: W (w h) = w (W h)) and the second product counts 1
     constexpr bool GATE_UP = MODE == 1;
     constexpr int ROWS = AFR * 16;       // pairs of a tile: 64, or 128 where the experts have many pairs each
     __shared__ __attribute__((aligned(16))) bf16_t lds[2 * AFR * 512];      // two sub-steps of AFR fragments
-    // A tile of 64 pairs gives a weight element 128 flops a read: the tiles of one expert must meet
-    // their weight rows in a cache, or the products run at what memory gives.  Blocks go to the
-    // eight XCDs in turn by their number, each XCD with an L2 of its own; so block L works on
-    // column block (L / 8 / max_tiles) * 8 + L % 8 and tile L / 8 % max_tiles: one XCD sees all
-    // tiles of a column block one after the other, an expert's tiles next to each other.
-    const int L = blockIdx.x, q = L >> 3;
-    const int tile = q % max_tiles, col_block = (q / max_tiles) * 8 + (L & 7);
-    if (tile >= num_tiles[0] || col_block >= col_blocks) return;
+    const int tiles = num_tiles[0], id = ex_block(blockIdx.x, tiles, col_blocks);
+    if (id < 0) return;
+    const int col_block = id / tiles, tile = id - col_block * tiles;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r = lane & 15, kg = lane >> 4;
     const int e = tile_expert[tile];
     const int c0 = col_block * (GATE_UP ? 64 : 128) + wv * (GATE_UP ? 16 : 32);     // the wave's first output
@@ -609,7 +618,7 @@ __global__ __launch_bounds__(256) void experts_lines_kernel(
     const bf16_t* __restrict__ a_rows, int a_row, const bf16_t* __restrict__ W0, const bf16_t* __restrict__ W1,
     const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_rows, const int32_t* __restrict__ num_tiles,
     const float* __restrict__ wts, int T, int top, int K, int N, float limit, float act_alpha, float up_offset,
-    bf16_t* __restrict__ y, float* __restrict__ out, int max_tiles, int col_blocks, int ldw, int weight_input) {
+    bf16_t* __restrict__ y, float* __restrict__ out, int col_blocks, int ldw, int weight_input) {
     constexpr int NW = 4, NS = 3, WGN = NW / WGM;
     constexpr int BM = WGM * WTM * 16, BN = WGN * WTN * 16;
     constexpr int LPA = BM / 8 / NW, LPW = BN / 8 / NW, CP = LPA + LPW;      // a wave's copies of a unit
@@ -618,10 +627,9 @@ __global__ __launch_bounds__(256) void experts_lines_kernel(
     static_assert(RPM >= 1 && CPM >= 1 && CP % 2 == 0 && LPA >= 1, "the MFMAs of a k-tile hide its reads and copies");
     static_assert(NS * UNIT <= 160 * 1024, "LDS");
     __shared__ __attribute__((aligned(1024))) char smem[NS * UNIT];
-    // blocks to XCDs as above: one XCD sees all tiles of a column block, an expert's tiles next to each other
-    const int L = blockIdx.x, q8 = L >> 3;
-    const int tile = q8 % max_tiles, col_block = (q8 / max_tiles) * 8 + (L & 7);
-    if (tile >= num_tiles[0] || col_block >= col_blocks) return;
+    const int tiles = num_tiles[0], id = ex_block(blockIdx.x, tiles, col_blocks);
+    if (id < 0) return;
+    const int col_block = id / tiles, tile = id - col_block * tiles;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = WGM == 2 ? wave >> 1 : 0, wn = WGM == 2 ? wave & 1 : wave;
     const int fr = lane & 15, fg = lane >> 4;
@@ -849,10 +857,10 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
     const int up_mode = Wg ? 1 : 2;
     const bf16_t *w0 = (const bf16_t*)(Wg ? Wg : Wu), *w1 = (const bf16_t*)(Wg ? Wu : nullptr);
 #define EX_ARGS_UP (const bf16_t*)h, h_row, w0, w1, tile_expert, tile_rows, num_tiles, wts, T, top, width, ff, limit, act_alpha, \
-                   up_offset, (bf16_t*)y, nullptr, max_tiles, cb, ldw_in, weight_input
+                   up_offset, (bf16_t*)y, nullptr, cb, ldw_in, weight_input
 #define EX_ARGS_DOWN (const bf16_t*)y, ff, (const bf16_t*)Wd, nullptr, tile_expert, tile_rows, num_tiles, wts, T, top, ff, width, limit, \
-                     act_alpha, up_offset, nullptr, out, max_tiles, cb, ldw_down, weight_input
-#define EX_GRID (unsigned)((cb + 7) / 8 * 8 * max_tiles)
+                     act_alpha, up_offset, nullptr, out, cb, ldw_down, weight_input
+#define EX_GRID (unsigned)(((long)cb * max_tiles + 7) / 8 * 8)
 #define EX_LINES(MODE, ...)                                                                                \
     do {                                                                                                   \
         if (tall) experts_lines_kernel<MODE, 2, 4, 8><<<EX_GRID, 256, 0, s>>>(__VA_ARGS__);                \

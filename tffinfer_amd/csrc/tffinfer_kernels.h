@@ -338,6 +338,8 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
                                  int ldw_in, int ldw_down, float limit, float act_alpha, float up_offset, int32_t* tile_expert,
                                  int32_t* tile_rows, int32_t* num_tiles, int max_tiles, void* y, float* out,
                                  int weight_input, int identity, tff_stream_t stream);
+// Which of the (column block, tile) pairs, tiles fastest, block `block` of a launch of its products works on; -1: none.
+TFF_API int tff_experts_block(int block, int tiles, int col_blocks);
 
 // ---- norms on a sublayer's output, sums over the model's depth (group_norm.hip) ----
 // y = delta row (planes added up first; row rows[r] where rows is given) cut into `groups` equal parts, each
