@@ -28,7 +28,8 @@
 
 __device__ __forceinline__ float gd_silu(float z) { return z / (1.0f + expf(-z)); }
 
-// One wave per (token, unit); units: kv_heads q heads, kv_heads k heads, heads v heads, one for beta and decay.
+// One wave per (token, unit); units: kv_heads q heads, kv_heads k heads, heads v heads, one for beta and decay.  The convolution's terms and
+// the factor of a unit vector, which a whole row of the results shares, are kept in 64 bits until they are rounded once.
 __global__ __launch_bounds__(64) void gdelta_prep_kernel(
     const float* __restrict__ proj, size_t ldp, const float* __restrict__ wconv, int taps,
     const float* __restrict__ a_log, const float* __restrict__ dt_bias, const float* __restrict__ state,
@@ -56,21 +57,21 @@ __global__ __launch_bounds__(64) void gdelta_prep_kernel(
     float ss = 0.f;
     for (int e = lane; e < n; e += 64) {
         const int c = c0 + e;
-        float acc = 0.f;
+        double acc = 0.;
         for (int k = 0; k < taps; ++k) {
             const int s = i - (taps - 1) + k;     // the input's place in the portion; before it: the state's
             const float x = s >= 0 ? proj[(size_t)(t - (taps - 1) + k) * ldp + c] : tail[(size_t)(i + k) * C + c];
-            acc = fmaf(wconv[(size_t)c * taps + k], x, acc);
+            acc = fma((double)wconv[(size_t)c * taps + k], (double)x, acc);
         }
-        const float y = gd_silu(acc);
+        const float y = gd_silu((float)acc);
         out[c] = y;
         ss = fmaf(y, y, ss);
     }
     if (u < 2 * G) {
         ss = wave_sum(ss);
-        const float f = (1.0f / sqrtf(ss + 1e-6f)) * (u < G ? 1.0f / sqrtf((float)D) : 1.0f);
+        const double f = 1.0 / sqrt(((double)ss + 1e-6) * (u < G ? (double)D : 1.0));
         __syncthreads();
-        for (int e = lane; e < n; e += 64) out[c0 + e] *= f;      // (each lane rescales what it wrote)
+        for (int e = lane; e < n; e += 64) out[c0 + e] = (float)((double)out[c0 + e] * f);      // (each lane rescales what it wrote)
     }
 }
 
@@ -455,8 +456,8 @@ TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ld
 // next product's MFMA j wants row 4 g + j.
 // One token after the other took 0.25 us a token: 2,048 tokens of 32 heads of 128 x 128 in 540 us, now 21 + 188; with the preparation,
 // 2,048 tokens of 4 heads of 64 x 64 438 / 129, four requests of 901, 700, 430 and 300 tokens 420 / 245.  Relative error against 64
-// bits over 96 to 400 tokens, with the preparation: heads of 64 1.26e-7 before, 1.11e-7 now; of 128 1.18e-7, 1.02e-7; of 256
-// 1.02e-7, 0.97e-7.
+// bits over 96 to 400 tokens, with the preparation (whose terms in 64 bits make up for more than the chunks' own roundings add), before /
+// now: heads of 64 1.22e-7 / 1.08e-7, of 128 1.16e-7 / 1.00e-7, of 256 1.03e-7 / 0.95e-7; token by token now 1.07e-7, 0.96e-7, 0.89e-7.
 //
 // work: per chunk and head 16 x 16 of (I + L)^-1 B, 16 x 16 of A, 16 G, 16 P_15,s; the chunk that starts at token t of row r
 // lies at place t / 16 + r.
