@@ -187,6 +187,29 @@ def test_output_norm_of_many_rows_is_that_of_few(group, planes):
     assert torch.equal(many[:7], few) and torch.equal(o_many[:7], o_few)
 
 
+@pytest.mark.parametrize("H,D", [(4, 64), (2, 128)])
+def test_recurrence_in_chunks_is_no_less_exact(H, D):
+    """400 tokens in chunks against the same tokens in the two forms for shorter portions, all against 64 bits, in the 2-norm: no further
+    off than those (products and sums within a chunk are formed in 64 bits), and under 1.5 units of 2^-23.  Roundings of 0.29 units each
+    add up at random: those of a sum of D terms in chains of eight and of the sixteen or so chunks that a state remembers are some
+    sqrt(16) x 0.29 = 1.2 units; measured 0.62 in chunks, 0.77 to 1.06 token by token."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(D)
+    T = 400
+    r, k, v, z = (torch.randn(T, H * D, generator=g) for _ in range(4))
+    w0, u = torch.rand(H * D, generator=g) * 3.5 - 3, torch.randn(H * D, generator=g)
+    w = torch.exp(-torch.exp(z.double() + w0.double()))
+    ref, _ = plain.wkv_recurrence(*(t.double().view(T, H, D) for t in (r, k, v, w)), u.double().view(H, D))
+    ref, errors = ref.reshape(T, H * D), []
+    for most in (T, 100, 10):
+        state, out = torch.zeros(1, H * D * D, device=DEV), []
+        for at in range(0, T, most):
+            part = [t[at:at + most].contiguous().to(DEV) for t in (r, k, v, z)]
+            out.append(ops.wkv_recurrence(*part, w0.to(DEV), u.to(DEV), state, _batch([part[0].shape[0]], [at], [0]), H, D))
+        errors.append(float((torch.cat(out).double().cpu() - ref).norm() / ref.norm()))
+    assert errors[0] < min(errors[1:]) and max(errors) < 1.5 * 2 ** -23, errors
+
+
 @pytest.mark.parametrize("H,D", [(2, 64), (2, 128)])
 @pytest.mark.parametrize("what", ["v", "k", "r", "z", "last v", "state"])
 def test_recurrence_what_is_not_finite_reaches_later_tokens_only(H, D, what):
