@@ -5,11 +5,11 @@
 // one chain of MFMAs in ascending groups of 16 k, and the parts are added in ascending order.  Both kernels keep to it,
 // so a row's result is the same bits however many other rows the step holds.
 //
-// gemm_f32_rows_kernel, up to 64 rows: a block per 16 weight rows, a wave per part of K; what bounds it is the weight's
+// gemm_f32_rows_kernel, up to 16 rows, and 17 to 64 where the model below finds it faster: a block per 16 weight rows, a wave per part of K; what bounds it is the weight's
 //   stream.  The weight goes straight into the MFMA operands (lane l of a wave holds four k of row l % 16: sixteen
 //   pieces of 64 bytes a load), no staging and one barrier.  Every block fetches all of A's rows, so the time grows
 //   by 0.2 us a row of K = 2,048.
-// gemm_f32_tiles_kernel, more rows: 2 x 2 waves of 32 or 64 x 64 elements, k-steps of 32 staged through LDS in two
+// gemm_f32_tiles_kernel, otherwise: 2 x 2 waves of 32 or 64 x 64 elements, k-steps of 32 staged through LDS in two
 //   buffers, the next step's loads in flight during the MFMAs.  A wave of 64 x 64 reads 8 KB of LDS for 64 MFMAs of
 //   32 cycles, so the matrix cores bound it.
 //

@@ -610,9 +610,9 @@ __global__ __launch_bounds__(256) void experts_tiles_kernel(
 // Unit u + 2 is copied during unit u, into the slot that unit u - 1 has left: its last operands were read, and had arrived
 // (lgkmcnt 0), before the barrier in the middle of unit u - 1.  At that barrier of unit u every wave's copies of unit u + 1 have
 // landed: all but the CP / 2 copies that it issued in the first half of unit u.
-// us for both products before / now: 32 experts, four a token, 4,096 x 1,536 gated, 2,048 tokens 883 / 578 (535 TFLOP/s; some 700 with
-// the tiles' padding), 150 tokens 273 / 262; 4,096 x 3,072 without a gate, 4,096 tokens 2,041 / 1,164; 16 experts, two a token, 2,048 x 2,048
-// without a gate, 512 tokens 130 / 86.
+// us for both products before / now: 32 experts, four a token, 4,096 x 1,536 gated, 2,048 tokens 883 / 517 (598 TFLOP/s; some 780 with
+// the tiles' padding), 150 tokens 273 / 244; 4,096 x 3,072 without a gate, 4,096 tokens 2,041 / 1,070; 16 experts, two a token, 2,048 x 2,048
+// without a gate, 512 tokens 130 / 84.
 template <int MODE, int WGM, int WTM, int WTN>
 __global__ __launch_bounds__(256) void experts_lines_kernel(
     const bf16_t* __restrict__ a_rows, int a_row, const bf16_t* __restrict__ W0, const bf16_t* __restrict__ W1,
@@ -831,8 +831,8 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
     // Tiles of 128 or of 64 pairs.  On 64-byte pieces: 128 where an expert has a few hundred pairs on average (every weight element
     // fetched serves twice the flops; the padding of an expert's last tile costs more with fewer).  On whole lines a block is
     // alone on its CU and a tile of 128 takes some 1.12 times as long as one of 64 (up to there both are their weight's stream), so
-    // what counts is how often the blocks go round the CUs.  us, 64 / 128: 32 experts, four a token, 4,096 x 1,536, 150 tokens 265 / 287,
-    // 512 tokens 328 / 301, 1,000 tokens 464 / 384; 16 experts, two a token, 2,048 x 1,024, 700 tokens 72 / 84, 1,000 tokens 117 / 85.
+    // what counts is how often the blocks go round the CUs.  us, 64 / 128: 32 experts, four a token, 4,096 x 1,536, 150 tokens 244 / 265,
+    // 512 tokens 318 / 288, 1,000 tokens 413 / 376; 16 experts, two a token, 2,048 x 1,024, 700 tokens 68 / 80, 1,000 tokens 114 / 83.
     bool tall = (long)T * top >= 192L * E;
     if (lines_up && lines_down) {
         const double n = (double)T * top / E;

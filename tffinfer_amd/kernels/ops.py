@@ -1259,8 +1259,9 @@ def _experts_by_tiles(T: int, top: int, E: int, width: int, ff: int, matrices: i
     """Whether the pairs of ``T`` tokens are dealt to their experts.  With inner sizes in units of 64 by what the two ways take,
     fitted to 1 to 31 tokens of five sizes: a pair streams its expert's matrices at 7.3 TB/s (experts that several
     tokens chose come from a cache), the tiles read every chosen expert once at 7 TB/s and have a floor of the length of
-    a block.  32 experts, four a token, 4,096 x 1,536, us by pairs / tiles: 8 tokens 172 / 195, 12 tokens 238 / 206, 31 tokens
-    549 / 235; 16 experts, two a token, 2,048 x 1,024: 16 tokens 58 / 63, 24 tokens 84 / 66."""
+    a block.  32 experts, four a token, 4,096 x 1,536, us by pairs / tiles: 6 tokens 137 / 140, 8 tokens 179 / 158, 12 tokens 241 / 221, 31
+    tokens 514 / 231; 16 experts, two a token, 2,048 x 1,024: 12 tokens 49 / 58, 16 tokens 61 / 59, 24 tokens 83 / 59.  Tiles dealt to the XCDs
+    in eighths came after the fit: the line lies up to two tokens late for some sizes, by an eighth of the time at most."""
     if width % 64 or ff % 64:
         return T >= EXPERT_TILES_MIN_TOKENS
     size = matrices * width * ff * 2e-6
