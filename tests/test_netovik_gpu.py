@@ -411,6 +411,38 @@ def test_attention_with_every_term(H, G, D, page, dtype):
             assert err < limit, f"{[k for k, v in kw.items() if v is not None and v is not False and v != 0]} cut {cuts[:3]}: {err:.3e}"
 
 
+@pytest.mark.parametrize("H,G,D,page", [(32, 8, 128, 16), (32, 32, 64, 16), (20, 5, 64, 48), (9, 3, 32, 16), (24, 24, 32, 64), (16, 1, 128, 32)])
+def test_attention_on_the_matrix_cores_at_the_tiles_edges(H, G, D, page):
+    """Portions of 64 tokens and more in bfloat16 (tiles of 64 keys, blocks of 16 queries) and single tokens (tiles of 32) whose
+    contexts, windows and kept tokens end just before, at and just behind a tile's border; slots that no token has written
+    hold NaN, which reaches nothing."""
+    ops = _ops()
+    from tffinfer_amd.parts.mixed_attention import distance_buckets
+    g = torch.Generator().manual_seed(H + G)
+    eps, B, Dmax = 1e-5, 10, 50
+    talk = torch.eye(H) + 0.3 * torch.randn(H, H, generator=g)
+    rel = torch.randn(B, H, generator=g)
+    table = rel[distance_buckets(B, Dmax)].contiguous().to(DEV)
+    for T, first, window, keep in ((65, 64, 0, 0), (193, 127, 64, 1), (258, 192, 65, 64), (320, 255, 128, 33), (129, 113, 31, 32)):
+        qk, qb, kb = _attention_case(H, G, D, T, T + H)
+        ref = _plain_attention(qk, qb, kb, H, G, D, eps, scale=min(0.7, 6.0 / D), cap=4.0, rel=rel, bias_max=Dmax, talk=talk,
+                               window=window or None, keep=keep, sink=True)
+        for cuts in ([first] + [1] * (T - first), [T - 64, 64], [first // 16 * 16, T - first // 16 * 16]):
+            cache = _Cache(G, D, page, [T], torch.bfloat16, seed=T)
+            cache.k.fill_(float("nan"))
+            cache.v.fill_(float("nan"))
+            outs, at = [], 0
+            for n in cuts:
+                if n:
+                    kv = cache.view([0], [at], [n])
+                    q = ops.qk_bias_norm_store(qk[at:at + n].contiguous().to(DEV), qb.to(DEV), kb.to(DEV), eps, H, G, D, kv)
+                    outs.append(ops.mixed_attention(q, H, G, D, kv, _batch([n], [at]), scale=min(0.7, 6.0 / D), softcap=4.0, bias=table,
+                                                    mix=talk.to(DEV), window=window, keep_first=keep, sink=True))
+                at += n
+            err = _err(torch.cat(outs, 0), ref)
+            assert err < 3e-2, (T, window, keep, cuts[:2], err)      # (bfloat16 queries, keys, weights and results, as above)
+
+
 @pytest.mark.parametrize("decode", [False, True])
 @pytest.mark.parametrize("edge", ["inside", "outside", "kept", "not_kept"])
 def test_a_loud_key_at_the_windows_and_the_kept_tokens_edges(edge, decode):

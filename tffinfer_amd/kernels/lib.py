@@ -99,6 +99,7 @@ _SIGNATURES = {
     "tff_mixed_attention_supported": [_I, _I, _I],
     "tff_mixed_attention": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _P, _F, _F, _I, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P],
     "tff_mixed_attention_workspace_bytes": [_I, _I, _I, _I],
+    "tff_mixed_attention_tile": [_I, _I, _I, _I, _I],
     "tff_mixed_attention_q16_supported": [_I, _I, _I, _I],
     "tff_mixed_attention_q16": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _P, _I, _P, _F, _F, _I, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P],
     "tff_experts_down": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _P, _I, _P],

@@ -1546,7 +1546,7 @@ def mixed_attention(q: torch.Tensor, H: int, G: int, D: int, kv, batch, scale: f
     s'_h = sum_g mix[h, g] s_g; key j is visible to query i if j <= i and (i - j < window or j < keep_first)
     (window 0: all j <= i); softmax over the visible keys, with one more term of 1 in the denominator
     if ``sink``; the values are the value pages.  q [T, H * D] in the cache's type; bias float32 [rows, H];
-    mix float32 [H, H].  A step of few tokens deals each token's keys (tiles of 64) to several blocks
+    mix float32 [H, H].  A step of few tokens deals each token's keys (tiles of 64 or 32) to several blocks
     (``splits``; by default so many that some 512 blocks run, from the longest context the step's tables
     can hold) and merges them in a second kernel."""
     dt = kv.k_cache.dtype
@@ -1581,13 +1581,13 @@ def mixed_attention(q: torch.Tensor, H: int, G: int, D: int, kv, batch, scale: f
         if cache is None:
             items = [(t, min(16, cu[r + 1] - t)) for r in range(len(cu) - 1) for t in range(cu[r], cu[r + 1], 16)]
             cache = batch._q16_work = _staging.send(q.device, [np.asarray(items, dtype=np.int32).reshape(-1, 2)])[0]
-        # tiles of 16 keys an item can have at most; where the items are fewer than the CUs, their tiles are dealt
+        # tiles of 64 keys an item can have at most; where the items are fewer than the CUs, their tiles are dealt
         # to several blocks
         reach = min(bt.shape[1] * kv.page_size, getattr(batch, "max_context", 1 << 30))
-        tiles16 = -(-min(keep_first, reach) // 16) + (-(-min(window + 15, reach) // 16) + 1 if window > 0 else -(-reach // 16))
-        parts = max(1, min(tiles16, 8, MIXED_ATTENTION_Q16_BLOCKS // cache.shape[0]))
-        per = -(-tiles16 // parts)
-        parts = -(-tiles16 // per) if parts > 1 else 1
+        tiles = -(-min(keep_first, reach) // 64) + (-(-min(window + 15, reach) // 64) + 1 if window > 0 else -(-reach // 64))
+        parts = max(1, min(tiles, 8, MIXED_ATTENTION_Q16_BLOCKS // cache.shape[0]))
+        per = -(-tiles // parts)
+        parts = -(-tiles // per) if parts > 1 else 1
         ws = None
         if parts > 1:
             ws = torch.empty(L.tff_mixed_attention_workspace_bytes(T, H, D, parts) // 4, dtype=torch.float32, device=q.device)
@@ -1597,10 +1597,11 @@ def mixed_attention(q: torch.Tensor, H: int, G: int, D: int, kv, batch, scale: f
                                              float(softcap), int(window), int(keep_first), 1 if sink else 0,
                                              out.data_ptr(), T, H, G, D, kv.page_size, parts, per, _ptr(ws), _stream()))
         return out
-    # tiles of 64 keys that a token of this step can have at most (what the block tables can hold, or the window
+    # tiles of keys that a token of this step can have at most (what the block tables can hold, or the window
     # and the kept tokens): a size the host knows without reading a position, so a captured step keeps it
     reach = bt.shape[1] * kv.page_size
-    tiles = -(-min(keep_first, reach) // 64) + (-(-min(window, reach) // 64) + 1 if window > 0 else -(-reach // 64))
+    keys = L.tff_mixed_attention_tile(H, G, D, kv.page_size, dtype_code(dt))
+    tiles = -(-min(keep_first, reach) // keys) + (-(-min(window, reach) // keys) + 1 if window > 0 else -(-reach // keys))
     if splits is None:
         splits = max(1, min(tiles, MIXED_ATTENTION_BLOCKS // max(T, 1)))
     per = -(-tiles // max(1, splits))
