@@ -393,14 +393,14 @@ TFF_API int tff_experts_down(const void* y, const void* Wd, const int32_t* idx, 
 // whatever tile and place it lands in: the result does not depend on what else the step holds, nor
 // on the order the pairs were dealt in.
 //
-// experts_sort_kernel:  tile_expert[tile], tile_rows[tile * rows + i] = pair (token * top + k) or -1,
-//                       num_tiles[0]; one block.  At most pairs / rows + E tiles.
+// experts_sort_kernel:  tile_expert[tile] = (expert, its first tile, how many tiles it has, 0), tile_rows[tile * rows + i] =
+//                       pair (token * top + k) or -1, num_tiles[0]; one block.  At most pairs / rows + E tiles.
 // experts_tiles_kernel: the two products per tile.  The down product writes
 //                       out[k][t][:] = wts[t][k] * Wd y: `top` planes that the norm after the
 //                       feed-forward adds up in the order of k.
 
 __global__ __launch_bounds__(1024) void experts_sort_kernel(const int32_t* __restrict__ idx, int pairs, int E,
-                                                            int rows, int32_t* __restrict__ tile_expert,
+                                                            int rows, int4* __restrict__ tile_expert,
                                                             int32_t* __restrict__ tile_rows,
                                                             int32_t* __restrict__ num_tiles) {
     __shared__ int count[RT_MAX_E];
@@ -423,7 +423,7 @@ __global__ __launch_bounds__(1024) void experts_sort_kernel(const int32_t* __res
     __syncthreads();
     const int tiles = first[E];
     for (int e = tid; e < E; e += blockDim.x) {
-        for (int t = first[e]; t < first[e + 1]; ++t) tile_expert[t] = e;
+        for (int t = first[e]; t < first[e + 1]; ++t) tile_expert[t] = make_int4(e, first[e], first[e + 1] - first[e], 0);
         count[e] = 0;
     }
     for (int i = tid; i < tiles * rows; i += blockDim.x) tile_rows[i] = -1;
@@ -458,17 +458,26 @@ __device__ __forceinline__ ex_bf16x8 ex_load8(const bf16_t* p, bool ok) {
 // dealt to.
 #define EXT_KSTEP 64
 
-// What a block of the experts' products works on.  A tile of 64 pairs gives a weight element 128 flops a read: the tiles of one expert
-// must meet their weight rows in a cache, or the products run at what memory gives.  Blocks go to the eight XCDs in turn by
-// their number, each XCD with an L2 of its own; of the (column block, tile) pairs in order, tiles fastest, each XCD takes an eighth,
-// so that it sees the tiles of a column block one after the other, an expert's next to each other.  Whole column blocks to an XCD left
-// XCDs without work where there are fewer than eight or no multiple of eight, more of them the wider the blocks: us for both products so /
-// now: 256 experts, eight a token, 1,024 x 512, 64 tokens 259 / 174; 96 experts, four a token, 1,536 x 512 without a gate, 150 tokens
-// 125 / 81; 32 experts, four a token, 4,096 x 1,536, 2,048 tokens 574 / 519; 16 experts, two a token, 2,048 x 2,048 71 / 70.
-// The pair's number, or -1 for a block without one.
+// What a block of the experts' products works on.  Blocks go to the eight XCDs in turn by their number, each XCD with an L2 of its own;
+// of the (tile, column block) pairs in order each XCD takes an eighth, so that none is without work.  The order is an expert after the
+// other, of an expert EX_GROUP tiles at a time, of these all column blocks, tiles fastest: the 32 blocks that an XCD runs at a time are
+// then one or two experts' whole products, whose weight rows come from memory once for the group's tiles and whose pairs' rows meet in L2
+// for the column blocks.  (A column block of all experts after the other, which stood here, shared the weight's rows as well but fetched
+// the pairs' rows once more for every column block, so
+// before / now, us for both products: 32 experts, four a token, 4,096 x 1,536 gated, 2,048 tokens 573 / 560, 4,000 tokens 852 / 817;
+// 2,048 x 1,536, 4,500 tokens 519 / 494; 64 to 150 tokens within 1 %.)
+// The pair's number in that order, or -1 for a block without one.
 __host__ __device__ __forceinline__ int ex_block(unsigned block, int tiles, int col_blocks) {
     const int all = tiles * col_blocks, share = (all + 7) >> 3, at = (int)(block >> 3), id = (int)(block & 7) * share + at;
     return at < share && id < all ? id : -1;
+}
+#define EX_GROUP 8
+// The tile and column block of pair `id`; `t` is the entry of tile id / col_blocks, which belongs to the same expert.
+__host__ __device__ __forceinline__ void ex_place(int id, int col_blocks, int4 t, int& tile, int& col_block) {
+    const int in = id - t.y * col_blocks, group = in / (EX_GROUP * col_blocks);
+    const int rest = in - group * EX_GROUP * col_blocks, left = t.z - group * EX_GROUP, n = left < EX_GROUP ? left : EX_GROUP;
+    col_block = rest / n;
+    tile = t.y + group * EX_GROUP + rest - col_block * n;
 }
 TFF_API int tff_experts_block(int block, int tiles, int col_blocks) { return ex_block((unsigned)block, tiles, col_blocks); }
 
@@ -476,7 +485,7 @@ TFF_API int tff_experts_block(int block, int tiles, int col_blocks) { return ex_
 template <int MODE, int AFR>
 __global__ __launch_bounds__(256) void experts_tiles_kernel(
     const bf16_t* __restrict__ a_rows, int a_row, const bf16_t* __restrict__ W0, const bf16_t* __restrict__ W1,
-    const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_rows,
+    const int4* __restrict__ tile_expert, const int32_t* __restrict__ tile_rows,
     const int32_t* __restrict__ num_tiles, const float* __restrict__ wts, int T, int top, int K, int N,
     float limit, float act_alpha, float up_offset, bf16_t* __restrict__ y, float* __restrict__ out, int col_blocks,
     int ldw, int weight_input) {
@@ -487,9 +496,11 @@ __global__ __launch_bounds__(256) void experts_tiles_kernel(
     __shared__ __attribute__((aligned(16))) bf16_t lds[2 * AFR * 512];      // two sub-steps of AFR fragments
     const int tiles = num_tiles[0], id = ex_block(blockIdx.x, tiles, col_blocks);
     if (id < 0) return;
-    const int col_block = id / tiles, tile = id - col_block * tiles;
+    const int4 of = tile_expert[id / col_blocks];
+    int tile, col_block;
+    ex_place(id, col_blocks, of, tile, col_block);
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r = lane & 15, kg = lane >> 4;
-    const int e = tile_expert[tile];
+    const int e = of.x;
     const int c0 = col_block * (GATE_UP ? 64 : 128) + wv * (GATE_UP ? 16 : 32);     // the wave's first output
     // the pairs' rows: 2 AFR fragments a step (AFR of 16 pairs, two sub-steps of 32 k), AFR / 2 a wave
     constexpr int AU = AFR / 2;
@@ -610,13 +621,18 @@ __global__ __launch_bounds__(256) void experts_tiles_kernel(
 // Unit u + 2 is copied during unit u, into the slot that unit u - 1 has left: its last operands were read, and had arrived
 // (lgkmcnt 0), before the barrier in the middle of unit u - 1.  At that barrier of unit u every wave's copies of unit u + 1 have
 // landed: all but the CP / 2 copies that it issued in the first half of unit u.
-// us for both products before / now: 32 experts, four a token, 4,096 x 1,536 gated, 2,048 tokens 883 / 517 (598 TFLOP/s; some 780 with
-// the tiles' padding), 150 tokens 273 / 244; 4,096 x 3,072 without a gate, 4,096 tokens 2,041 / 1,070; 16 experts, two a token, 2,048 x 2,048
-// without a gate, 512 tokens 130 / 84.
+// A block that works on one pair of tile and column block spends 10 to 15 us of its 40 to 75 on what nothing overlaps: three loads that wait for
+// each other, the first units on their way, the results' way out.  So the launch has a block a CU, and a block goes on to its next
+// pair: that one's list of rows travels during the second unit of the present pair, its first two units of operands during the
+// last two, and the results leave through the third slot while they land.
+// us for both products, a pair a block / now: 32 experts, four a token, 4,096 x 1,536 gated, 2,048 tokens 560 / 537 (576 TFLOP/s; some 720
+// with the tiles' padding), 4,000 tokens 817 / 783; 4,096 x 3,072 without a gate, 2,919 tokens 776 / 739; 2,048 x 1,536 gated, 4,500 tokens
+// 494 / 462; 16 experts, two a token, 2,048 x 1,024, 2,000 tokens 121 / 101; 150 tokens of the first within 2 % (the weight's stream).
+#define EXL_CHAIN 5      // units of K from which a block may go on to another pair: its list is there before its first copies
 template <int MODE, int WGM, int WTM, int WTN>
 __global__ __launch_bounds__(256) void experts_lines_kernel(
     const bf16_t* __restrict__ a_rows, int a_row, const bf16_t* __restrict__ W0, const bf16_t* __restrict__ W1,
-    const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_rows, const int32_t* __restrict__ num_tiles,
+    const int4* __restrict__ tile_expert, const int32_t* __restrict__ tile_rows, const int32_t* __restrict__ num_tiles,
     const float* __restrict__ wts, int T, int top, int K, int N, float limit, float act_alpha, float up_offset,
     bf16_t* __restrict__ y, float* __restrict__ out, int col_blocks, int ldw, int weight_input) {
     constexpr int NW = 4, NS = 3, WGN = NW / WGM;
@@ -625,45 +641,52 @@ __global__ __launch_bounds__(256) void experts_lines_kernel(
     constexpr unsigned A_BYTES = BM * 128u, UNIT = (BM + BN) * 128u;
     constexpr int NMF = WTM * WTN, RPM = NMF / (WTM + WTN), CPM = NMF / (CP / 2);
     static_assert(RPM >= 1 && CPM >= 1 && CP % 2 == 0 && LPA >= 1, "the MFMAs of a k-tile hide its reads and copies");
-    static_assert(NS * UNIT <= 160 * 1024, "LDS");
-    __shared__ __attribute__((aligned(1024))) char smem[NS * UNIT];
-    const int tiles = num_tiles[0], id = ex_block(blockIdx.x, tiles, col_blocks);
+    constexpr unsigned LIST = NS * UNIT;                // behind the units: each wave's lists of pairs, this tile's and the next one's
+    static_assert(LIST + NW * 2048 <= 160 * 1024 && BM * 4 <= 1024, "LDS");
+    __shared__ __attribute__((aligned(1024))) char smem[LIST + NW * 2048];
+    const int tiles = num_tiles[0];
+    unsigned block = blockIdx.x;
+    int id = ex_block(block, tiles, col_blocks);
     if (id < 0) return;
-    const int col_block = id / tiles, tile = id - col_block * tiles;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = WGM == 2 ? wave >> 1 : 0, wn = WGM == 2 ? wave & 1 : wave;
     const int fr = lane & 15, fg = lane >> 4;
-    const int e = tile_expert[tile];
-    const int32_t* pairs = tile_rows + (size_t)tile * BM;
-    const int c0 = col_block * (MODE == 1 ? BN / 2 : BN);           // the block's first output
-
-    floatx4 acc[WTN][WTM];
-#pragma unroll
-    for (int i = 0; i < WTN; ++i)
-#pragma unroll
-        for (int j = 0; j < WTM; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    int4 of = tile_expert[id / col_blocks];
+    int tile, col_block;
+    ex_place(id, col_blocks, of, tile, col_block);
 
     // what a wave copies of a unit: the pairs' rows, eight at a time, and the weight's
+    const unsigned smem_addr = (unsigned)(size_t)(lds_ptr_t)smem;
     const unsigned chunk = (unsigned)(((lane & 7) ^ (lane >> 3)) * 16);
     unsigned off[CP];
     unsigned long long base[3];
     base[0] = (unsigned long long)a_rows;
-    base[1] = (unsigned long long)(W0 + (size_t)e * N * ldw);
-    base[2] = MODE == 1 ? (unsigned long long)(W1 + (size_t)e * N * ldw) : base[1];
+    auto weight_rows = [&]() {
+        base[1] = (unsigned long long)(W0 + (size_t)of.x * N * ldw);
+        base[2] = MODE == 1 ? (unsigned long long)(W1 + (size_t)of.x * N * ldw) : base[1];
 #pragma unroll
-    for (int c = 0; c < LPA; ++c) {
-        const int p = max(pairs[(wave + NW * c) * 8 + (lane >> 3)], 0);      // (a place without a pair repeats pair 0, nobody reads it)
-        off[c] = (unsigned)(MODE != 0 ? p / top : p) * (unsigned)a_row * 2u + chunk;
-    }
+        for (int c = 0; c < LPW; ++c) {
+            const int r0 = (wave + NW * c) * 8, grp = r0 >> 4, in = (r0 & 15) + (lane >> 3);
+            const int n = col_block * (MODE == 1 ? BN / 2 : BN) + (MODE == 1 ? grp >> 1 : grp) * 16 + in;
+            off[LPA + c] = (unsigned)min(n, N - 1) * (unsigned)ldw * 2u + chunk;
+        }
+    };
+    auto pair_row = [&](int p) {     // (a place without a pair repeats pair 0, nobody reads it)
+        p = max(p, 0);
+        return (unsigned)(MODE != 0 ? p / top : p) * (unsigned)a_row * 2u + chunk;
+    };
+    // a tile's list into the wave's buffer `to`: the lanes past its end repeat it
+    auto copy_list = [&](int of_tile, unsigned to) {
+        copy16_to_lds_sbase((unsigned long long)(tile_rows + (size_t)of_tile * BM), (unsigned)(lane * 16) & (BM * 4 - 1),
+                            smem_addr + LIST + (unsigned)wave * 2048u + to);
+    };
+    unsigned list = 0;                                // the present tile's list
 #pragma unroll
-    for (int c = 0; c < LPW; ++c) {
-        const int r0 = (wave + NW * c) * 8, grp = r0 >> 4, in = (r0 & 15) + (lane >> 3);
-        const int n = c0 + (MODE == 1 ? grp >> 1 : grp) * 16 + in;
-        off[LPA + c] = (unsigned)min(n, N - 1) * (unsigned)ldw * 2u + chunk;
-    }
-    const unsigned smem_addr = (unsigned)(size_t)(lds_ptr_t)smem;
+    for (int c = 0; c < LPA; ++c) off[c] = pair_row(tile_rows[(size_t)tile * BM + (wave + NW * c) * 8 + (lane >> 3)]);
+    weight_rows();
+    copy_list(tile, list);
     const int nu = K >> 6;
-    int u_next = 0;                                   // the unit to copy next; past the end the last one once more
+    int u_next = 0;                                   // the unit to copy next
     unsigned long long k_off = 0;
     unsigned ws = 0;                                  // its slot
 #define EXL_COPY(c)                                                                                                 \
@@ -681,7 +704,7 @@ __global__ __launch_bounds__(256) void experts_lines_kernel(
     for (int u = 0; u < 2; ++u) {
 #pragma unroll
         for (int c = 0; c < CP; ++c) EXL_COPY(c)
-        EXL_ISSUED()
+        EXL_ISSUED()                                  // (past the end of K the last unit once more)
     }
     // a lane's 16 bytes of an operand: row fr of 16, chunk h * 4 + fg of the row's 8
     unsigned rd[2];
@@ -717,72 +740,111 @@ __global__ __launch_bounds__(256) void experts_lines_kernel(
                 }                                                                                                   \
                 if (q % CPM == CPM - 1 && q / CPM < CP / 2) EXL_COPY((h) * (CP / 2) + q / CPM)                      \
             }                                                                                                       \
-        if (h) EXL_ISSUED()                                                                                         \
     }
-    for (int u = 0; u < nu; ++u) {
-        EXL_TILE(0)
-        EXL_TILE(1)
+    floatx4 acc[WTN][WTM];
+    for (;;) {
+        const int c0 = col_block * (MODE == 1 ? BN / 2 : BN);           // the pair's first output
+        block += gridDim.x;
+        const int next = nu >= EXL_CHAIN ? ex_block(block, tiles, col_blocks) : -1;
+        if (next >= 0) {
+            of = tile_expert[next / col_blocks];
+            ex_place(next, col_blocks, of, tile, col_block);
+        }
+#pragma unroll
+        for (int i = 0; i < WTN; ++i)
+#pragma unroll
+            for (int j = 0; j < WTM; ++j) {
+                acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+                asm volatile("" : "+a"(acc[i][j]));
+            }
+        asm volatile("s_nop 7");
+        for (int u = 0; u < nu; ++u) {
+            EXL_TILE(0)
+            EXL_TILE(1)
+            EXL_ISSUED()
+            if (next >= 0) {
+                if (u == 1) copy_list(tile, list ^ 1024u);             // here since the barrier of unit 2
+                if (u == nu - 3) {                                      // the coming copies are the next pair's
+                    const int32_t* in_list = reinterpret_cast<const int32_t*>(smem + LIST + wave * 2048 + (list ^ 1024u));
+#pragma unroll
+                    for (int c = 0; c < LPA; ++c) off[c] = pair_row(in_list[(wave + NW * c) * 8 + (lane >> 3)]);
+                    weight_rows();
+                    u_next = 0;
+                    k_off = 0;
+                }
+            }
+        }
+        // The last MFMAs have written.  The unit that was worked on last has left its slot (its last operands had arrived before the barrier in
+        // its middle), and the next pair's first two units are in the other two or on their way: the results go through that slot, a
+        // part of it for each wave, so that its stores are whole pieces of a pair's row.
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        typedef typename std::conditional<MODE == 0, float, bf16_t>::type TO;
+        constexpr int OW = MODE == 1 ? WTN / 2 : WTN, EL = 16 / (int)sizeof(TO);
+        constexpr int RB = OW * 16 * (int)sizeof(TO), RBP = RB + 16, LPR = RB / 16, RPI = 64 / LPR;
+        constexpr int REGION = (int)(UNIT / NW) & ~1023;
+        constexpr int JS = WTM * 16 * RBP <= REGION ? WTM : WTM / 2 * 16 * RBP <= REGION ? WTM / 2 : 1;      // groups of 16 pairs at a time
+        static_assert(JS * 16 * RBP <= REGION && WTM % JS == 0 && LPR <= 64 && (LPR & (LPR - 1)) == 0 && 16 % RPI == 0, "the wave's part holds its results");
+        char* region = smem + ws + wave * REGION;
+        const int32_t* pairs = reinterpret_cast<const int32_t*>(smem + LIST + wave * 2048 + list) + wm * WTM * 16;
+        const int ln = w4_lane(), r = ln & 15, g = ln >> 4;
+        const int srow = ln / LPR, sch = ln % LPR, n = c0 + wn * OW * 16 + sch * EL;
+#pragma unroll
+        for (int j0 = 0; j0 < WTM; j0 += JS) {
+#pragma unroll
+            for (int j = j0; j < j0 + JS; ++j) {
+                __builtin_amdgcn_sched_barrier(0);
+                float w = 1.0f;
+                if (MODE == 0 ? !weight_input : weight_input != 0) {
+                    const int p = pairs[j * 16 + r];
+                    w = p >= 0 ? wts[p] : 0.f;
+                }
+#pragma unroll
+                for (int i = 0; i < OW; ++i) {
+                    char* dst = region + ((j - j0) * 16 + r) * RBP + (i * 16 + g * 4) * (int)sizeof(TO);
+                    float v[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        if constexpr (MODE == 1) {
+                            const float gv = fminf(acc[2 * i][j][c] * w, limit);
+                            const float uv = fminf(fmaxf(acc[2 * i + 1][j][c] * w, -limit), limit);
+                            v[c] = gv * (1.0f / (1.0f + expf(-act_alpha * gv))) * (uv + up_offset);
+                        } else if constexpr (MODE == 2) {
+                            const float u = fmaxf(acc[i][j][c] * w, 0.f);
+                            v[c] = u * u;
+                        } else {
+                            v[c] = w * acc[i][j][c];
+                        }
+                    }
+                    if constexpr (sizeof(TO) == 4) {
+                        *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+                    } else {
+                        union { bf16_t h[4]; uint2 u; } pk;
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) pk.h[c] = (bf16_t)v[c];
+                        *reinterpret_cast<uint2*>(dst) = pk.u;
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (other lanes' results, as another type)
+#pragma unroll 4
+            for (int t = 0; t < JS * 16 / RPI; ++t) {
+                const int row = t * RPI + srow, p = pairs[j0 * 16 + row];
+                const uint4 v = *reinterpret_cast<const uint4*>(region + row * RBP + sch * 16);
+                if (p < 0 || n >= N) continue;                // (N is a multiple of 8: a piece is whole or not there)
+                if constexpr (MODE == 0) *reinterpret_cast<uint4*>(out + ((size_t)(p % top) * T + p / top) * N + n) = v;
+                else *reinterpret_cast<uint4*>(y + (size_t)p * N + n) = v;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+        if (next < 0) break;
+        asm volatile("s_barrier" ::: "memory");       // every wave has left the slot: the next unit's copies go there
+        list ^= 1024u;
     }
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));         // the copies past the end must not outlive the block
 #undef EXL_TILE
 #undef EXL_COPY
 #undef EXL_ISSUED
-    // every copy has landed, every operand has come back and the last MFMAs have written: LDS is free for the results
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
-    __syncthreads();
-    // A wave's results go through its own part of LDS, so that its stores are whole pieces of a pair's row.
-    typedef typename std::conditional<MODE == 0, float, bf16_t>::type TO;
-    constexpr int OW = MODE == 1 ? WTN / 2 : WTN, EL = 16 / (int)sizeof(TO);
-    constexpr int RB = OW * 16 * (int)sizeof(TO), RBP = RB + 16, LPR = RB / 16, RPI = 64 / LPR;
-    constexpr int REGION = (int)(NS * UNIT / NW) & ~1023;
-    static_assert(WTM * 16 * RBP <= REGION && LPR <= 64 && (LPR & (LPR - 1)) == 0, "the wave's part holds its results");
-    char* region = smem + wave * REGION;
-    const int ln = w4_lane(), r = ln & 15, g = ln >> 4;
-#pragma unroll
-    for (int j = 0; j < WTM; ++j) {
-        __builtin_amdgcn_sched_barrier(0);
-        float w = 1.0f;
-        if (MODE == 0 ? !weight_input : weight_input != 0) {
-            const int p = pairs[(wm * WTM + j) * 16 + r];
-            w = p >= 0 ? wts[p] : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < OW; ++i) {
-            char* dst = region + (j * 16 + r) * RBP + (i * 16 + g * 4) * (int)sizeof(TO);
-            float v[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                if constexpr (MODE == 1) {
-                    const float gv = fminf(acc[2 * i][j][c] * w, limit);
-                    const float uv = fminf(fmaxf(acc[2 * i + 1][j][c] * w, -limit), limit);
-                    v[c] = gv * (1.0f / (1.0f + expf(-act_alpha * gv))) * (uv + up_offset);
-                } else if constexpr (MODE == 2) {
-                    const float u = fmaxf(acc[i][j][c] * w, 0.f);
-                    v[c] = u * u;
-                } else {
-                    v[c] = w * acc[i][j][c];
-                }
-            }
-            if constexpr (sizeof(TO) == 4) {
-                *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-            } else {
-                union { bf16_t h[4]; uint2 u; } pk;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) pk.h[c] = (bf16_t)v[c];
-                *reinterpret_cast<uint2*>(dst) = pk.u;
-            }
-        }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    const int srow = ln / LPR, sch = ln % LPR, n = c0 + wn * OW * 16 + sch * EL;
-#pragma unroll 4
-    for (int t = 0; t < WTM * 16 / RPI; ++t) {
-        const int row = t * RPI + srow, p = pairs[wm * WTM * 16 + row];
-        const uint4 v = *reinterpret_cast<const uint4*>(region + row * RBP + sch * 16);
-        if (p < 0 || n >= N) continue;                // (N is a multiple of 8: a piece is whole or not there)
-        if constexpr (MODE == 0) *reinterpret_cast<uint4*>(out + ((size_t)(p % top) * T + p / top) * N + n) = v;
-        else *reinterpret_cast<uint4*>(y + (size_t)p * N + n) = v;
-    }
 }
 
 // The planes of the pairs whose expert has no matrices: out[k][t][:] = wts[t][k] * h[t][:].
@@ -805,7 +867,7 @@ TFF_API int tff_experts_tiles_supported(int width, int ff, int h_row) {
     return width % 8 == 0 && ff % 8 == 0 && h_row % 8 == 0;
 }
 
-// h [T, width] bfloat16; workspace: tile_expert [max_tiles], tile_rows [max_tiles * 128], num_tiles [1] (int32),
+// h [T, width] bfloat16; workspace: tile_expert [max_tiles * 4] (16-byte aligned), tile_rows [max_tiles * 128], num_tiles [1] (int32),
 // y [T * top, ff] bfloat16; out float32 [top, T, width].  max_tiles >= T * top / 64 + E.
 TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const void* Wu, const void* Wd,
                                  const int32_t* idx, const float* wts, int T, int top, int E, int width, int ff,
@@ -820,7 +882,8 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
                 ldw_down >= ff, "experts_by_tiles: width %d, ff %d, rows of %d and the weights' rows of %d and %d must be "
                 "multiples of 8", width, ff, h_row, ldw_in, ldw_down);
     TFF_REQUIRE(((uintptr_t)h % 16) == 0 && ((uintptr_t)Wg % 16) == 0 && ((uintptr_t)Wu % 16) == 0 &&
-                ((uintptr_t)Wd % 16) == 0 && ((uintptr_t)y % 16) == 0, "experts_by_tiles: operands must be 16-byte aligned");
+                ((uintptr_t)Wd % 16) == 0 && ((uintptr_t)y % 16) == 0 && ((uintptr_t)tile_expert % 16) == 0 && ((uintptr_t)tile_rows % 16) == 0,
+                "experts_by_tiles: operands must be 16-byte aligned");
     TFF_REQUIRE((long)T * top < (1L << 31) && max_tiles <= (1 << 20) && max_tiles >= (long)T * top / 64 + E,
                 "experts_by_tiles: %d tiles do not hold %d x %d pairs of %d experts", max_tiles, T, top, E);
     // Inner sizes in units of 64 run on whole cache lines, the others on 64-byte pieces.  (A lane's offset into the rows is 32 bits.)
@@ -851,20 +914,22 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
         experts_identity_kernel<<<T * top, 256, 0, s>>>((const bf16_t*)h, h_row, idx, wts, T, top, E, width, out);
         if (int rc0 = tff_check_launch("experts_identity")) return rc0;
     }
-    experts_sort_kernel<<<1, 1024, 0, s>>>(idx, T * top, E, rows, tile_expert, tile_rows, num_tiles);
+    experts_sort_kernel<<<1, 1024, 0, s>>>(idx, T * top, E, rows, (int4*)tile_expert, tile_rows, num_tiles);
     int rc = tff_check_launch("experts_sort");
     if (rc) return rc;
     const int up_mode = Wg ? 1 : 2;
     const bf16_t *w0 = (const bf16_t*)(Wg ? Wg : Wu), *w1 = (const bf16_t*)(Wg ? Wu : nullptr);
-#define EX_ARGS_UP (const bf16_t*)h, h_row, w0, w1, tile_expert, tile_rows, num_tiles, wts, T, top, width, ff, limit, act_alpha, \
+#define EX_ARGS_UP (const bf16_t*)h, h_row, w0, w1, (const int4*)tile_expert, tile_rows, num_tiles, wts, T, top, width, ff, limit, act_alpha, \
                    up_offset, (bf16_t*)y, nullptr, cb, ldw_in, weight_input
-#define EX_ARGS_DOWN (const bf16_t*)y, ff, (const bf16_t*)Wd, nullptr, tile_expert, tile_rows, num_tiles, wts, T, top, ff, width, limit, \
+#define EX_ARGS_DOWN (const bf16_t*)y, ff, (const bf16_t*)Wd, nullptr, (const int4*)tile_expert, tile_rows, num_tiles, wts, T, top, ff, width, limit, \
                      act_alpha, up_offset, nullptr, out, cb, ldw_down, weight_input
 #define EX_GRID (unsigned)(((long)cb * max_tiles + 7) / 8 * 8)
+// (one block a CU, which goes on from pair to pair; each pair a block of its own where K has too few units for that)
+#define EXL_GRID(MODE) (((MODE) == 0 ? ff : width) / 64 < EXL_CHAIN ? EX_GRID : EX_GRID < 256u ? EX_GRID : 256u)
 #define EX_LINES(MODE, ...)                                                                                \
     do {                                                                                                   \
-        if (tall) experts_lines_kernel<MODE, 2, 4, 8><<<EX_GRID, 256, 0, s>>>(__VA_ARGS__);                \
-        else experts_lines_kernel<MODE, 1, 4, 4><<<EX_GRID, 256, 0, s>>>(__VA_ARGS__);                     \
+        if (tall) experts_lines_kernel<MODE, 2, 4, 8><<<EXL_GRID(MODE), 256, 0, s>>>(__VA_ARGS__);         \
+        else experts_lines_kernel<MODE, 1, 4, 4><<<EXL_GRID(MODE), 256, 0, s>>>(__VA_ARGS__);              \
     } while (0)
 #define EX_TILES(MODE, ...)                                                                                \
     do {                                                                                                   \
@@ -886,6 +951,7 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
 #undef EX_ARGS_UP
 #undef EX_ARGS_DOWN
 #undef EX_GRID
+#undef EXL_GRID
 #undef EX_LINES
 #undef EX_TILES
     return tff_check_launch("experts_down_tiles");
