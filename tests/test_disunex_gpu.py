@@ -221,6 +221,39 @@ def test_products_per_head_with_gate_and_rotated_tail(dtype, T, H, K, N, tail, d
     assert _err(gated, ref * torch.sigmoid(gate[:, :H * N].double().view(T, H, N))) < t_
 
 
+@pytest.mark.parametrize("T", [63, 64, 65, 200])        # (from 64 tokens on through LDS, where K is one to four units of 64)
+@pytest.mark.parametrize("H,K,N,tail,dims,pairing,pad", [(2, 64, 8, 16, 16, 0, 32), (3, 128, 192, 64, 64, 1, 256), (2, 192, 72, 24, 16, 1, 104),
+                                                         (3, 256, 136, 0, 0, 1, 136), (20, 256, 264, 32, 32, 0, 296), (2, 320, 64, 8, 8, 1, 72)])
+def test_products_per_head_in_whole_pieces(T, H, K, N, tail, dims, pairing, pad):
+    """Sizes in units of eight: runs of outputs and blocks of tokens that end inside, both pairings, every number of units of K.
+    The products are summed in float32 and rounded once to bfloat16: 2^-8 of the largest value."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(H * K + T)
+    row = 8 + H * (K + tail)
+    x = torch.randn(T, row, generator=g).bfloat16().to(DEV)
+    wt = (torch.randn(H, N, K, generator=g) * 0.3).bfloat16().to(DEV)
+    positions = torch.randint(0, 50, (T,), generator=g).to(torch.int32).to(DEV)
+    table = torch.randn(64, dims // 2, 2, generator=g).to(DEV) if dims else None
+    gate = torch.randn(T, H * N + 8, generator=g).bfloat16().to(DEV)
+    xh = x[:, 8:].double().view(T, H, K + tail)
+    ref = torch.stack([xh[:, h, :K] @ wt[h].double().T for h in range(H)], 1)
+    rt = xh[..., K:].clone()
+    if dims:
+        cs = table.double()[positions.long()][:, None]
+        a, b = (rt[..., 0:dims:2], rt[..., 1:dims:2]) if pairing else (rt[..., :dims // 2], rt[..., dims // 2:dims])
+        u, v = a * cs[..., 0] - b * cs[..., 1], b * cs[..., 0] + a * cs[..., 1]
+        rt[..., :dims] = torch.stack((u, v), -1).flatten(-2) if pairing else torch.cat((u, v), -1)
+    how = dict(out_head=pad, tail=tail, cos_sin=table, pairing=pairing)
+    want = torch.cat((ref, rt, torch.zeros(T, H, pad - N - tail, dtype=torch.float64, device=DEV)), -1)
+    run = lambda n, gt=None: ops.head_linear(x[:n, 8:], K + tail, wt, gate=None if gt is None else gt[:n],        # noqa: E731
+                                             positions=positions[:n] if dims else None, **how).view(n, H, pad)
+    out = run(T)
+    assert float((out.double() - want).abs().max()) < 2.0 ** -8 * float(want.abs().max())
+    want[..., :N] *= torch.sigmoid(gate[:, :H * N].double().view(T, H, N))
+    assert float((run(T, gate).double() - want).abs().max()) < 2.0 ** -8 * float(want.abs().max())
+    assert torch.equal(run(3), out[:3])              # (the kernel for few tokens: the same order of k)
+
+
 def _sink_ref(q, keys, vals, positions, window, scale, sinks):
     """q [T, nq, d] against one key head: keys [S, d], vals [S, dv]."""
     T, nq, _ = q.shape

@@ -16,12 +16,8 @@
 //                       an optional sigmoid gate on the result and an optional tail of the
 //                       input row that is rotated by the token's position (either pairing) and copied behind
 //                       the product (the query's rotated part), zeros up to pad_to.
-//                       bfloat16 on the matrix cores where rows are 16-byte aligned: a wave
-//                       holds 32 tokens x 64 outputs in accumulators and reads its operands
-//                       straight from memory in MFMA fragment order (eight consecutive k a
-//                       lane), W as the first operand so that a lane ends up with four
-//                       consecutive outputs of one token.
-#include "common.h"
+//                       bfloat16 on the matrix cores where rows are 16-byte aligned.
+#include "mfma_tiles.h"
 #include "tffinfer_kernels.h"
 
 // Element e of the rotated part (rot elements at x, the first rot_dims of them rotated) after the rotation
@@ -138,6 +134,7 @@ TFF_API int tff_latent_kv_store(const void* x, int x_stride, int T, int rank, in
 // elements at a time; thread n walks k along its row W[h][n][:], adding into TT accumulators,
 // k ascending for every token whatever the batch.
 #define HL_TT 8
+#define HL_LINES_FROM 64      // tokens: a block's worth
 #define HL_KC 128
 
 struct HeadLinearTail {
@@ -216,84 +213,269 @@ __global__ __launch_bounds__(256) void head_linear_kernel(
     if (blockIdx.z == 0 && tl.pad_to > N) head_tail<T>(x, x_row, x_head, out, out_row, out_head, t0, nt, h, K, N, tl);
 }
 
-// bfloat16 on the matrix cores.  Block: 128 tokens x 64 outputs of one head, four waves of 32
-// tokens each.  C[n][t] += W[n][k] x[t][k]: W's rows are the first operand's rows, so lane
-// (t = lane & 15, kg = lane >> 4) holds outputs n = kg * 4 .. + 3 of token t for each of the
-// 4 x 2 tiles.  k ascends in steps of 32 for every token whatever the batch.
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 hl_bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float hl_floatx4;
-
-__device__ __forceinline__ hl_bf16x8 hl_load8(const bf16_t* p, bool ok) {
-    union { uint4 u; hl_bf16x8 v; } x;
-    x.u = ok ? *reinterpret_cast<const uint4*>(p) : make_uint4(0, 0, 0, 0);
-    return x.v;
+// The same by whole pieces of eight elements, where sizes and addresses allow it.
+__device__ __forceinline__ void head_tail_vec(const bf16_t* __restrict__ x, int x_row, int x_head, bf16_t* __restrict__ out,
+                                              int out_row, int out_head, int t0, int nt, int h, int K, int N, const HeadLinearTail tl) {
+    union Eight { uint4 u; bf16_t b[8]; };
+    const int pieces = (tl.pad_to - N) >> 3;
+    for (int i = threadIdx.x; i < nt * pieces; i += blockDim.x) {
+        const int tt = i / pieces, e = (i - tt * pieces) * 8, t = t0 + tt;
+        const bf16_t* xr = x + (size_t)t * x_row + (size_t)h * x_head + K;
+        Eight v;
+        v.u = make_uint4(0, 0, 0, 0);
+        if (e < tl.tail) v.u = *reinterpret_cast<const uint4*>(xr + e);
+        if (e < tl.rot_dims) {
+            const int pos = min(max(tl.positions[t], 0), tl.max_pos - 1), half = tl.rot_dims >> 1;
+            const float* cs = tl.cos_sin + (size_t)pos * tl.rot_dims;
+            float c[16];
+            if (tl.pairing == 1) {
+                reinterpret_cast<float4*>(c)[0] = *reinterpret_cast<const float4*>(cs + e);
+                reinterpret_cast<float4*>(c)[1] = *reinterpret_cast<const float4*>(cs + e + 4);
+                Eight y;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const float a = (float)v.b[k], o = (float)v.b[k ^ 1], co = c[k & 6], si = c[(k & 6) + 1];
+                    y.b[k] = (bf16_t)(!(k & 1) ? fmaf(a, co, -(o * si)) : fmaf(a, co, o * si));
+                }
+                v = y;
+            } else {
+                const bool first = e < half;
+                const int i0 = first ? e : e - half;
+                Eight w, y;
+                w.u = *reinterpret_cast<const uint4*>(xr + (first ? e + half : e - half));
+#pragma unroll
+                for (int k = 0; k < 4; ++k) reinterpret_cast<float4*>(c)[k] = *reinterpret_cast<const float4*>(cs + 2 * i0 + 4 * k);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const float a = (float)v.b[k], o = (float)w.b[k], co = c[2 * k], si = c[2 * k + 1];
+                    y.b[k] = (bf16_t)(first ? fmaf(a, co, -(o * si)) : fmaf(a, co, o * si));
+                }
+                v = y;
+            }
+        }
+        *reinterpret_cast<uint4*>(out + (size_t)t * out_row + (size_t)h * out_head + N + e) = v.u;
+    }
 }
 
-__global__ __launch_bounds__(256) void head_linear_mfma_kernel(
+// bfloat16 on the matrix cores.  What bounds it is the rows going in and out, some 60 MB for 2,048 tokens of 32 heads of 128 + 64
+// into 256 elements.  Block: 64 tokens of one head, two waves of 32 tokens each for every second run of 64 outputs; a wave asks
+// for four k-steps of both operands at a time (24 loads), straight into the operands, and its results leave through LDS as whole pieces
+// of 16 bytes.  C[n][t] += W[n][k] x[t][k]: W's rows are the first operand's rows, so lane (t = lane & 15, kg = lane >> 4) holds
+// outputs n = kg * 4 .. + 3 of token t for each of the 4 x 2 tiles.  k ascends in steps of 32 for every token whatever the batch.
+// With fewer loads in flight and its results stored one by one 8,192 tokens of 16 heads of 64 + 32 into 128 took 42 us, now 18.
+// VEC: output rows, heads, N and the tail's sizes are multiples of eight elements at 16-byte aligned addresses, and the gate's rows
+// of four at 8-byte aligned ones; else the results go out one by one.  `runs`: runs of 64 outputs of a block.
+template <bool VEC>
+__global__ __launch_bounds__(256, 3) void head_linear_mfma_kernel(
     const bf16_t* __restrict__ x, int x_row, int x_head, const bf16_t* __restrict__ W, bf16_t* __restrict__ out,
     int out_row, int out_head, int Tn, int K, int N, const bf16_t* __restrict__ gate, int gate_row,
-    HeadLinearTail tl) {
+    HeadLinearTail tl, int runs) {
+    constexpr int RB = 64 * 2 + 16, KS = 4;       // bytes of a staged row of 64 outputs; k-steps asked for at a time
+    __shared__ __attribute__((aligned(16))) char staged[VEC ? 4 * 32 * RB : 16];
+    union Eight { uint4 u; bf16x8 v; };
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, kg = lane >> 4;
-    const int h = blockIdx.y, n0 = blockIdx.z * 64;
-    const int tb = blockIdx.x * 128, t0 = tb + wv * 32;
-    hl_floatx4 acc[4][2];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[j][i] = hl_floatx4{0.f, 0.f, 0.f, 0.f};
+    const int h = blockIdx.x, tb = blockIdx.y * 64, t0 = tb + (wv & 1) * 32;
+    const int n_end = min(N, (int)(blockIdx.z + 1) * runs * 64);
     const bf16_t* xp[2];
-    bool xok[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int t = t0 + i * 16 + r;
-        xok[i] = t < Tn;
-        xp[i] = x + (size_t)min(t, Tn - 1) * x_row + (size_t)h * x_head + kg * 8;
-    }
-    const bf16_t* wp[4];
-    bool wok[4];
+    for (int i = 0; i < 2; ++i) xp[i] = x + (size_t)min(t0 + i * 16 + r, Tn - 1) * x_row + (size_t)h * x_head;
+    if (t0 < Tn)        // (a wave's condition: the MFMAs below run for whole waves; rows and outputs past the end repeat the last one)
+        for (int n0 = (blockIdx.z * runs + (wv >> 1)) * 64; n0 < n_end; n0 += 128) {
+            const bf16_t* wp[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int n = n0 + j * 16 + r;
-        wok[j] = n < N;
-        wp[j] = W + ((size_t)h * N + min(n, N - 1)) * K + kg * 8;
-    }
-    if (t0 < Tn) {      // (a wave's condition: the MFMAs below run for whole waves)
-        for (int k0 = 0; k0 < K; k0 += 32) {
-            const bool kok = k0 + kg * 8 < K;      // K is a multiple of 8: a lane's eight elements exist together
-            hl_bf16x8 a[4], b[2];
+            for (int j = 0; j < 4; ++j) wp[j] = W + ((size_t)h * N + min(n0 + j * 16 + r, N - 1)) * K;
+            union Four { uint2 u; bf16_t b[4]; } gz[4][2];
+            if (VEC && gate) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) a[j] = hl_load8(wp[j] + k0, wok[j] && kok);
+                for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) b[i] = hl_load8(xp[i] + k0, xok[i] && kok);
+                    for (int i = 0; i < 2; ++i)
+                        gz[j][i].u = *reinterpret_cast<const uint2*>(gate + (size_t)min(t0 + i * 16 + r, Tn - 1) * gate_row + (size_t)h * N +
+                                                                     min(n0 + j * 16 + kg * 4, N - 4));
+            }
+            floatx4 acc[4][2];
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j], b[i], acc[j][i], 0, 0, 0);
-        }
+                for (int i = 0; i < 2; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+            int k0 = 0;
+            for (; k0 + KS * 32 <= K; k0 += KS * 32) {
+                Eight a[KS][4], b[KS][2];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int t = t0 + i * 16 + r;
+                for (int q = 0; q < KS; ++q) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float v4[4] = {acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]};
+                    for (int j = 0; j < 4; ++j) a[q][j].u = *reinterpret_cast<const uint4*>(wp[j] + k0 + q * 32 + kg * 8);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int n = n0 + j * 16 + kg * 4 + e;
-                    if (t < Tn && n < N) {
-                        float v = v4[e];
-                        if (gate) {
-                            const float gz = (float)gate[(size_t)t * gate_row + (size_t)h * N + n];
-                            v *= 1.0f / (1.0f + expf(-gz));
+                    for (int i = 0; i < 2; ++i) b[q][i].u = *reinterpret_cast<const uint4*>(xp[i] + k0 + q * 32 + kg * 8);
+                }
+#pragma unroll
+                for (int q = 0; q < KS; ++q)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+                            acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q][j].v, b[q][i].v, acc[j][i], 0, 0, 0);
+            }
+            for (; k0 < K; k0 += 32) {       // (K is a multiple of 8: a lane's eight elements exist together)
+                const bool kok = k0 + kg * 8 < K;
+                const int k = min(k0 + kg * 8, K - 8);
+                Eight a[4], b[2];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) a[j].u = *reinterpret_cast<const uint4*>(wp[j] + k);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) b[i].u = *reinterpret_cast<const uint4*>(xp[i] + k);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) a[j].u = kok ? a[j].u : make_uint4(0, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) b[i].u = kok ? b[i].u : make_uint4(0, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j].v, b[i].v, acc[j][i], 0, 0, 0);
+            }
+            char* region = staged + (VEC ? wv * 32 * RB : 0);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int t = t0 + i * 16 + r;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float v4[4] = {acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]};
+                    if constexpr (VEC) {
+                        Four p;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            p.b[e] = (bf16_t)(gate ? v4[e] * (1.0f / (1.0f + expf(-(float)gz[j][i].b[e]))) : v4[e]);
+                        *reinterpret_cast<uint2*>(region + (i * 16 + r) * RB + (j * 16 + kg * 4) * 2) = p.u;
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int n = n0 + j * 16 + kg * 4 + e;
+                            if (t < Tn && n < N) {
+                                float v = v4[e];
+                                if (gate) v *= 1.0f / (1.0f + expf(-(float)gate[(size_t)t * gate_row + (size_t)h * N + n]));
+                                out[(size_t)t * out_row + (size_t)h * out_head + n] = (bf16_t)v;
+                            }
                         }
-                        out[(size_t)t * out_row + (size_t)h * out_head + n] = (bf16_t)v;
                     }
                 }
             }
+            if constexpr (VEC) {             // (the wave's own part: its LDS operations come in order)
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                const int n = n0 + (lane & 7) * 8;
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const int row = p * 8 + (lane >> 3), t = t0 + row;
+                    const uint4 v = *reinterpret_cast<const uint4*>(region + row * RB + (lane & 7) * 16);
+                    if (t < Tn && n < N) *reinterpret_cast<uint4*>(out + (size_t)t * out_row + (size_t)h * out_head + n) = v;
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            }
         }
+    if (blockIdx.z == 0 && tl.pad_to > N) {
+        if constexpr (VEC) head_tail_vec(x, x_row, x_head, out, out_row, out_head, tb, min(64, Tn - tb), h, K, N, tl);
+        else head_tail<bf16_t>(x, x_row, x_head, out, out_row, out_head, tb, min(64, Tn - tb), h, K, N, tl);
     }
-    if (blockIdx.z == 0 && tl.pad_to > N)
-        head_tail<bf16_t>(x, x_row, x_head, out, out_row, out_head, tb, min(128, Tn - tb), h, K, N, tl);
+}
+
+// The same for steps of many tokens and inner sizes of one to four units of 64: through LDS as whole cache lines.  In the kernel
+// above sixteen lanes of a load lie in sixteen rows, which costs the address unit a cycle a lane: 95 cycles a load, whatever the
+// caches give.  Block: 64 tokens of one head and `runs` runs of 64 outputs, four waves of 32 tokens x 32 outputs.  The tokens' rows are
+// copied once (eight rows x 128 bytes a copy, lane i takes chunk (i % 8) ^ (i / 8) of row i / 8, so that an operand's sixteen
+// rows come back from different banks), a run's rows of W while the run before goes out.  The same order of k: the same bits.
+// What bounds it is the rows going in and out, 60 MB for 2,048 tokens of 32 heads.  us, the stores one by one / the kernel above / this one:
+// heads of 128 with a rotated tail of 64 into 256 elements, 2,048 tokens 56 / 29 / 19, 8,192 tokens 172 / 102 / 61; of 256 into 128
+// with a gate 52 / 36 / 23 and 259 / 136 / 89.
+__global__ __launch_bounds__(256) void head_linear_lines_kernel(
+    const bf16_t* __restrict__ x, int x_row, int x_head, const bf16_t* __restrict__ W, bf16_t* __restrict__ out,
+    int out_row, int out_head, int Tn, int K, int N, const bf16_t* __restrict__ gate, int gate_row,
+    HeadLinearTail tl, int runs) {
+    constexpr int RB = 32 * 2 + 16;               // bytes of a wave's staged row
+    __shared__ __attribute__((aligned(16))) char staged[4 * 32 * RB];
+    extern __shared__ __attribute__((aligned(1024))) char tiles[];       // the tokens' units, then the run's: 8 KB each
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, kg = lane >> 4;
+    const int h = blockIdx.x, tb = blockIdx.y * 64, units = K >> 6;
+    const int wm = wv & 1, wn = wv >> 1;
+    const int n_first = blockIdx.z * runs * 64, n_end = min(N, n_first + runs * 64);
+    const unsigned x_lds = (unsigned)(size_t)(lds_ptr_t)tiles, w_lds = x_lds + (unsigned)units * 8192u;
+    const unsigned chunk = (unsigned)(((lane & 7) ^ (lane >> 3)) * 16);
+    // a wave's copies of a unit: rows 16 wv .. + 15 of both operands
+    unsigned xo[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) xo[c] = (unsigned)min(wv * 16 + c * 8 + (lane >> 3), Tn - 1 - tb) * (unsigned)x_row * 2u + chunk;
+    const unsigned long long xb = (unsigned long long)(x + (size_t)tb * x_row + (size_t)h * x_head);
+    for (int u = 0; u < units; ++u)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) copy16_to_lds_sbase(xb + (unsigned)u * 128u, xo[c], x_lds + (unsigned)u * 8192u + (unsigned)(wv * 2 + c) * 1024u);
+    auto copy_run = [&](int n0) {
+        const unsigned long long wb = (unsigned long long)(W + ((size_t)h * N + n0) * K);
+        for (int u = 0; u < units; ++u)
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                copy16_to_lds_sbase(wb + (unsigned)u * 128u, (unsigned)min(wv * 16 + c * 8 + (lane >> 3), N - 1 - n0) * (unsigned)K * 2u + chunk,
+                                    w_lds + (unsigned)u * 8192u + (unsigned)(wv * 2 + c) * 1024u);
+    };
+    copy_run(n_first);
+    unsigned rd[2];               // a lane's 16 bytes of an operand: row r of 16, chunk half * 4 + kg of the row's 8
+#pragma unroll
+    for (int q = 0; q < 2; ++q) rd[q] = (unsigned)(r >> 3) * 1024u + (unsigned)(((r & 7) * 8 + ((q * 4 + kg) ^ (r & 7))) * 16);
+    const char* xt = tiles + wm * 4096;
+    const char* wt = tiles + units * 8192 + wn * 4096;
+    char* region = staged + wv * 32 * RB;
+    for (int n0 = n_first; n0 < n_end; n0 += 64) {
+        union Four { uint2 u; bf16_t b[4]; } gz[2][2];
+        if (gate) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    gz[j][i].u = *reinterpret_cast<const uint2*>(gate + (size_t)min(tb + wm * 32 + i * 16 + r, Tn - 1) * gate_row + (size_t)h * N +
+                                                                 min(n0 + wn * 32 + j * 16 + kg * 4, N - 4));
+        }
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        __syncthreads();
+        floatx4 acc[2][2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int u = 0; u < units; ++u)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                bf16x8 a[2], b[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) a[j] = *reinterpret_cast<const bf16x8*>(wt + u * 8192 + j * 2048 + rd[q]);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) b[i] = *reinterpret_cast<const bf16x8*>(xt + u * 8192 + i * 2048 + rd[q]);
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j], b[i], acc[j][i], 0, 0, 0);
+            }
+        __syncthreads();                             // the run's rows have been read
+        if (n0 + 64 < n_end) copy_run(n0 + 64);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                Four p;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float v = acc[j][i][e];
+                    p.b[e] = (bf16_t)(gate ? v * (1.0f / (1.0f + expf(-(float)gz[j][i].b[e]))) : v);
+                }
+                *reinterpret_cast<uint2*>(region + (i * 16 + r) * RB + (j * 16 + kg * 4) * 2) = p.u;
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (the wave's own part)
+        const int n = n0 + wn * 32 + (lane & 3) * 8;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const int row = p * 16 + (lane >> 2), t = tb + wm * 32 + row;
+            const uint4 v = *reinterpret_cast<const uint4*>(region + row * RB + (lane & 3) * 16);
+            if (t < Tn && n < N) *reinterpret_cast<uint4*>(out + (size_t)t * out_row + (size_t)h * out_head + n) = v;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    if (blockIdx.z == 0 && tl.pad_to > N) head_tail_vec(x, x_row, x_head, out, out_row, out_head, tb, min(64, Tn - tb), h, K, N, tl);
 }
 
 TFF_API int tff_head_linear(const void* x, int x_row, int x_head, const void* Wt, void* out, int out_row, int out_head,
@@ -321,10 +503,26 @@ TFF_API int tff_head_linear(const void* x, int x_row, int x_head, const void* Wt
     else if (dtype == TFF_BF16) {
         const bool aligned = K % 8 == 0 && x_row % 8 == 0 && x_head % 8 == 0 && ((uintptr_t)x % 16) == 0 &&
                              ((uintptr_t)Wt % 16) == 0;
-        if (aligned)
-            head_linear_mfma_kernel<<<dim3((T + 127) / 128, H, (N + 63) / 64), 256, 0, s>>>(
-                (const bf16_t*)x, x_row, x_head, (const bf16_t*)Wt, (bf16_t*)out, out_row, out_head, T, K, N,
-                (const bf16_t*)gate, gate_row, tl);
+        if (aligned) {
+            // whole pieces: of the results and the tail eight elements, of the gate four (its row of a head starts at h * N)
+            const int extra = pad_to > N ? pad_to - N : 0;
+            const bool vec = N % 8 == 0 && out_row % 8 == 0 && out_head % 8 == 0 && ((uintptr_t)out % 16) == 0 && extra % 8 == 0 && tail % 8 == 0 &&
+                             rot_dims % (pairing == 0 ? 16 : 8) == 0 && ((uintptr_t)cos_sin % 16) == 0 &&
+                             (!gate || (gate_row % 4 == 0 && ((uintptr_t)gate % 8) == 0));
+            // A block has all of a head's outputs where that fills the chip (the tokens' rows are read once), else each pair of waves one
+            // run of 64 outputs: a step of few tokens is two latencies to memory, not a stream.
+            const int all = (N + 63) / 64, runs = (long)((T + 63) / 64) * H >= 512 ? all : 2;
+            const dim3 mg(H, (T + 63) / 64, (all + runs - 1) / runs);
+#define TFF_HL(VEC)                                                                                                              \
+    head_linear_mfma_kernel<VEC><<<mg, 256, 0, s>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)Wt, (bf16_t*)out, out_row,     \
+                                                    out_head, T, K, N, (const bf16_t*)gate, gate_row, tl, runs)
+            if (vec && K % 64 == 0 && K <= 256 && T >= HL_LINES_FROM)
+                head_linear_lines_kernel<<<mg, 256, (unsigned)K * 256u, s>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)Wt, (bf16_t*)out, out_row,
+                                                                           out_head, T, K, N, (const bf16_t*)gate, gate_row, tl, runs);
+            else if (vec) TFF_HL(true);
+            else TFF_HL(false);
+#undef TFF_HL
+        }
         else
             head_linear_kernel<bf16_t><<<grid, 256, 0, s>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)Wt, (bf16_t*)out,
                                                             out_row, out_head, T, K, N, (const bf16_t*)gate, gate_row, tl);
