@@ -221,7 +221,7 @@ def test_products_per_head_with_gate_and_rotated_tail(dtype, T, H, K, N, tail, d
     assert _err(gated, ref * torch.sigmoid(gate[:, :H * N].double().view(T, H, N))) < t_
 
 
-@pytest.mark.parametrize("T", [63, 64, 65, 200])        # (from 64 tokens on through LDS, where K is one to four units of 64)
+@pytest.mark.parametrize("T", [1, 17, 64, 65, 200])     # (through LDS where K is one to four units of 64, a block 64 tokens)
 @pytest.mark.parametrize("H,K,N,tail,dims,pairing,pad", [(2, 64, 8, 16, 16, 0, 32), (3, 128, 192, 64, 64, 1, 256), (2, 192, 72, 24, 16, 1, 104),
                                                          (3, 256, 136, 0, 0, 1, 136), (20, 256, 264, 32, 32, 0, 296), (2, 320, 64, 8, 8, 1, 72)])
 def test_products_per_head_in_whole_pieces(T, H, K, N, tail, dims, pairing, pad):
@@ -251,7 +251,8 @@ def test_products_per_head_in_whole_pieces(T, H, K, N, tail, dims, pairing, pad)
     assert float((out.double() - want).abs().max()) < 2.0 ** -8 * float(want.abs().max())
     want[..., :N] *= torch.sigmoid(gate[:, :H * N].double().view(T, H, N))
     assert float((run(T, gate).double() - want).abs().max()) < 2.0 ** -8 * float(want.abs().max())
-    assert torch.equal(run(3), out[:3])              # (the kernel for few tokens: the same order of k)
+    n = min(T, 3)
+    assert torch.equal(run(n), out[:n])              # (another number of tokens: the same order of k)
 
 
 def _sink_ref(q, keys, vals, positions, window, scale, sinks):

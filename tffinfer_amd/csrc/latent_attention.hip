@@ -134,7 +134,6 @@ TFF_API int tff_latent_kv_store(const void* x, int x_stride, int T, int rank, in
 // elements at a time; thread n walks k along its row W[h][n][:], adding into TT accumulators,
 // k ascending for every token whatever the batch.
 #define HL_TT 8
-#define HL_LINES_FROM 64      // tokens: a block's worth
 #define HL_KC 128
 
 struct HeadLinearTail {
@@ -257,16 +256,15 @@ __device__ __forceinline__ void head_tail_vec(const bf16_t* __restrict__ x, int 
     }
 }
 
-// bfloat16 on the matrix cores.  What bounds it is the rows going in and out, some 60 MB for 2,048 tokens of 32 heads of 128 + 64
-// into 256 elements.  Block: 64 tokens of one head, two waves of 32 tokens each for every second run of 64 outputs; a wave asks
-// for four k-steps of both operands at a time (24 loads), straight into the operands, and its results leave through LDS as whole pieces
-// of 16 bytes.  C[n][t] += W[n][k] x[t][k]: W's rows are the first operand's rows, so lane (t = lane & 15, kg = lane >> 4) holds
-// outputs n = kg * 4 .. + 3 of token t for each of the 4 x 2 tiles.  k ascends in steps of 32 for every token whatever the batch.
-// With fewer loads in flight and its results stored one by one 8,192 tokens of 16 heads of 64 + 32 into 128 took 42 us, now 18.
+// bfloat16 on the matrix cores, any inner size.  Block: 64 tokens of one head, two waves of 32 tokens each for every second run of 64
+// outputs; a wave asks for four k-steps of both operands at a time (24 loads), straight into the operands, and its results leave
+// through LDS as whole pieces of 16 bytes.  C[n][t] += W[n][k] x[t][k]: W's rows are the first operand's rows, so lane (t = lane & 15,
+// kg = lane >> 4) holds outputs n = kg * 4 .. + 3 of token t for each of the 4 x 2 tiles.  k ascends in steps of 32 for every token
+// whatever the batch.
 // VEC: output rows, heads, N and the tail's sizes are multiples of eight elements at 16-byte aligned addresses, and the gate's rows
 // of four at 8-byte aligned ones; else the results go out one by one.  `runs`: runs of 64 outputs of a block.
 template <bool VEC>
-__global__ __launch_bounds__(256, 3) void head_linear_mfma_kernel(
+__global__ __launch_bounds__(256, 2) void head_linear_mfma_kernel(
     const bf16_t* __restrict__ x, int x_row, int x_head, const bf16_t* __restrict__ W, bf16_t* __restrict__ out,
     int out_row, int out_head, int Tn, int K, int N, const bf16_t* __restrict__ gate, int gate_row,
     HeadLinearTail tl, int runs) {
@@ -277,9 +275,13 @@ __global__ __launch_bounds__(256, 3) void head_linear_mfma_kernel(
     const int h = blockIdx.x, tb = blockIdx.y * 64, t0 = tb + (wv & 1) * 32;
     const int n_end = min(N, (int)(blockIdx.z + 1) * runs * 64);
     const bf16_t* xp[2];
+    bool xok[2];        // (a lane whose row does not exist does not ask: the address unit takes a cycle for each lane that does)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) xp[i] = x + (size_t)min(t0 + i * 16 + r, Tn - 1) * x_row + (size_t)h * x_head;
-    if (t0 < Tn)        // (a wave's condition: the MFMAs below run for whole waves; rows and outputs past the end repeat the last one)
+    for (int i = 0; i < 2; ++i) {
+        xok[i] = t0 + i * 16 + r < Tn;
+        xp[i] = x + (size_t)min(t0 + i * 16 + r, Tn - 1) * x_row + (size_t)h * x_head;
+    }
+    if (t0 < Tn)        // (a wave's condition: the MFMAs below run for whole waves; outputs past the end repeat the last one)
         for (int n0 = (blockIdx.z * runs + (wv >> 1)) * 64; n0 < n_end; n0 += 128) {
             const bf16_t* wp[4];
 #pragma unroll
@@ -290,8 +292,9 @@ __global__ __launch_bounds__(256, 3) void head_linear_mfma_kernel(
                 for (int j = 0; j < 4; ++j)
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
-                        gz[j][i].u = *reinterpret_cast<const uint2*>(gate + (size_t)min(t0 + i * 16 + r, Tn - 1) * gate_row + (size_t)h * N +
-                                                                     min(n0 + j * 16 + kg * 4, N - 4));
+                        gz[j][i].u = xok[i] ? *reinterpret_cast<const uint2*>(gate + (size_t)(t0 + i * 16 + r) * gate_row + (size_t)h * N +
+                                                                              min(n0 + j * 16 + kg * 4, N - 4))
+                                            : make_uint2(0, 0);
             }
             floatx4 acc[4][2];
 #pragma unroll
@@ -306,7 +309,8 @@ __global__ __launch_bounds__(256, 3) void head_linear_mfma_kernel(
 #pragma unroll
                     for (int j = 0; j < 4; ++j) a[q][j].u = *reinterpret_cast<const uint4*>(wp[j] + k0 + q * 32 + kg * 8);
 #pragma unroll
-                    for (int i = 0; i < 2; ++i) b[q][i].u = *reinterpret_cast<const uint4*>(xp[i] + k0 + q * 32 + kg * 8);
+                    for (int i = 0; i < 2; ++i)
+                        b[q][i].u = xok[i] ? *reinterpret_cast<const uint4*>(xp[i] + k0 + q * 32 + kg * 8) : make_uint4(0, 0, 0, 0);
                 }
 #pragma unroll
                 for (int q = 0; q < KS; ++q)
@@ -377,14 +381,14 @@ __global__ __launch_bounds__(256, 3) void head_linear_mfma_kernel(
     }
 }
 
-// The same for steps of many tokens and inner sizes of one to four units of 64: through LDS as whole cache lines.  In the kernel
+// The same for inner sizes of one to four units of 64: through LDS as whole cache lines.  In the kernel
 // above sixteen lanes of a load lie in sixteen rows, which costs the address unit a cycle a lane: 95 cycles a load, whatever the
 // caches give.  Block: 64 tokens of one head and `runs` runs of 64 outputs, four waves of 32 tokens x 32 outputs.  The tokens' rows are
 // copied once (eight rows x 128 bytes a copy, lane i takes chunk (i % 8) ^ (i / 8) of row i / 8, so that an operand's sixteen
 // rows come back from different banks), a run's rows of W while the run before goes out.  The same order of k: the same bits.
-// What bounds it is the rows going in and out, 60 MB for 2,048 tokens of 32 heads.  us, the stores one by one / the kernel above / this one:
-// heads of 128 with a rotated tail of 64 into 256 elements, 2,048 tokens 56 / 29 / 19, 8,192 tokens 172 / 102 / 61; of 256 into 128
-// with a gate 52 / 36 / 23 and 259 / 136 / 89.
+// What bounds it is the rows going in and out, 60 MB for 2,048 tokens of 32 heads; with few tokens two latencies to memory.
+// us, the kernel above as it was with results one by one / now: heads of 128 with a rotated tail of 64 into 256 elements, 1, 100, 2,048 and
+// 8,192 tokens 4.5 / 3.5, 18.7 / 4.2, 56 / 19, 171 / 63; of 256 into 128 with a gate 7.2 / 4.4, 16.4 / 5.0, 52 / 23, 257 / 87.
 __global__ __launch_bounds__(256) void head_linear_lines_kernel(
     const bf16_t* __restrict__ x, int x_row, int x_head, const bf16_t* __restrict__ W, bf16_t* __restrict__ out,
     int out_row, int out_head, int Tn, int K, int N, const bf16_t* __restrict__ gate, int gate_row,
@@ -509,14 +513,14 @@ TFF_API int tff_head_linear(const void* x, int x_row, int x_head, const void* Wt
             const bool vec = N % 8 == 0 && out_row % 8 == 0 && out_head % 8 == 0 && ((uintptr_t)out % 16) == 0 && extra % 8 == 0 && tail % 8 == 0 &&
                              rot_dims % (pairing == 0 ? 16 : 8) == 0 && ((uintptr_t)cos_sin % 16) == 0 &&
                              (!gate || (gate_row % 4 == 0 && ((uintptr_t)gate % 8) == 0));
-            // A block has all of a head's outputs where that fills the chip (the tokens' rows are read once), else each pair of waves one
-            // run of 64 outputs: a step of few tokens is two latencies to memory, not a stream.
-            const int all = (N + 63) / 64, runs = (long)((T + 63) / 64) * H >= 512 ? all : 2;
+            // A block has all of a head's outputs where that fills the chip (the tokens' rows are read once), else one run of 64: a step
+            // of few tokens is two latencies to memory and what the address units of the CUs in use take for its loads.
+            const int all = (N + 63) / 64, runs = (long)((T + 63) / 64) * H >= 512 ? all : 1;
             const dim3 mg(H, (T + 63) / 64, (all + runs - 1) / runs);
 #define TFF_HL(VEC)                                                                                                              \
     head_linear_mfma_kernel<VEC><<<mg, 256, 0, s>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)Wt, (bf16_t*)out, out_row,     \
                                                     out_head, T, K, N, (const bf16_t*)gate, gate_row, tl, runs)
-            if (vec && K % 64 == 0 && K <= 256 && T >= HL_LINES_FROM)
+            if (vec && K % 64 == 0 && K <= 256)
                 head_linear_lines_kernel<<<mg, 256, (unsigned)K * 256u, s>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)Wt, (bf16_t*)out, out_row,
                                                                            out_head, T, K, N, (const bf16_t*)gate, gate_row, tl, runs);
             else if (vec) TFF_HL(true);
