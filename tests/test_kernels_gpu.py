@@ -1596,3 +1596,36 @@ def test_measured_ceilings_are_plausible():
 
     # operands that change cost power, never gain speed (a tenth of slack for the clock's wander)
     assert 300 < c["mfma_bf16_TFLOPs_varied_operands"] <= c["mfma_bf16_TFLOPs_4_waves_per_simd"] * 1.1
+
+
+@pytest.mark.parametrize("M", [1, 3, 16, 17, 33, 64, 65, 130, 300, 1500])
+@pytest.mark.parametrize("P,N,K", [(4, 128, 64), (3, 384, 192), (2, 1024, 320), (4, 2176, 128)])
+def test_products_of_several_planes(M, P, N, K):
+    """Every kernel the plan picks for several products in one launch, tiles that end with a plane; against the products one by one in
+    64 bits: float32 sums of products of bfloat16, K terms of size one: 2^-20 K of the largest value is far above their rounding."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(P, M, K, generator=g).bfloat16().to(DEV)
+    w = torch.randn(P * N, K, generator=g).bfloat16().to(DEV)
+    out = ops.linear_planes(x, ops.pack_weight(w))
+    ref = torch.stack([x[p].double() @ w[p * N:(p + 1) * N].double().T for p in range(P)])
+    assert tuple(out.shape) == (P, M, N)
+    assert float((out.double() - ref).abs().max()) < 2.0 ** -20 * K * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("act", ["tanh", "gelu", "gelu_tanh", "relu2"])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 4096), (5, 72, 128), (16, 200, 520), (40, 64, 2048), (300, 64, 4096), (300, 640, 192)])
+def test_products_with_an_activation(act, M, N, K):
+    """In the streaming kernel, in the sum over a split K's parts, and as a kernel of its own.  A rounding to bfloat16
+    moves a value by up to 2^-8 of itself; the square doubles that of the product, and its own comes on top: 3 * 2^-8 (the other
+    activations' slopes are at most 1.13); in float32 the sums of K terms."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    z = x.double() @ w.double().T
+    ref = {"tanh": torch.tanh, "gelu": torch.nn.functional.gelu, "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh"),
+           "relu2": lambda t: t.clamp(min=0) ** 2}[act](z)
+    for dtype, tol in ((torch.bfloat16, 3 * 2.0 ** -8), (torch.float32, 2.0 ** -18)):
+        out = ops.linear_unary(x, ops.pack_weight(w), act, dtype)
+        assert out.dtype == dtype and float((out.double() - ref).abs().max()) < tol * float(ref.abs().max())

@@ -23,6 +23,20 @@ static inline GluAct glu_act(float limit, float alpha, float up_offset) {
 
 __device__ __forceinline__ float to_f32(float v) { return v; }
 __device__ __forceinline__ float to_f32(bf16_t v) { return (float)v; }
+// form 0: gelu with erf; 1: its tanh approximation; 2: the square of relu
+__device__ __forceinline__ float ffn_activation(float z, int form) {
+    if (form == 2) {
+        const float r = fmaxf(z, 0.f);
+        return r * r;
+    }
+    if (form == 1) return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+    return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
+}
+// What a product's epilogue may do with a result: 0 nothing, 1 tanh, 2 .. 4 ffn_activation's forms 0 .. 2.
+__device__ __forceinline__ float unary_activation(float v, int kind) {
+    return kind == 0 ? v : kind == 1 ? tanhf(v) : ffn_activation(v, kind - 2);
+}
+
 template <typename T> __device__ __forceinline__ T from_f32(float v);
 template <> __device__ __forceinline__ float from_f32<float>(float v) { return v; }
 template <> __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) { return (bf16_t)v; }

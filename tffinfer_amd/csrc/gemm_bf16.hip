@@ -41,9 +41,15 @@ __device__ __forceinline__ void store4(TC* dst, const floatx4& v, int n, int N, 
 
 // What a product takes besides its operands: a bias (float32, in the order of W's rows, ceil16(N) numbers) or null,
 // and how a gated product joins gate and up.
+// unary: what becomes of a result that is not gated (unary_activation), where the streaming kernel or the sum over a split K's
+// parts stores it.  plane_cols > 0: several products in one launch.  W's rows are theirs one after the other, plane_cols each; the
+// columns of plane p take their rows from A + p * a_step, and C holds the planes [p][M][plane_cols].
 struct GemmExtra {
     const float* bias;
     GluAct act;
+    int unary;
+    int plane_cols;
+    size_t a_step;
 };
 
 // GLU: the 16-row groups of W alternate between a gate and an up projection
@@ -285,7 +291,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bf16_async_kernel(
 template <bool GLU, typename TC>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __restrict__ part, int S,
                                                                   int M, int N, TC* __restrict__ C,
-                                                                  int n_out, GluAct act) {
+                                                                  int n_out, GluAct act, int unary) {
     const int per_row = (n_out + 3) / 4;
     const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (long)M * per_row) return;
@@ -315,6 +321,10 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
                     if (j + e < N) a[e] += p[e];
             }
         }
+        if (unary) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] = unary_activation(a[e], unary);
+        }
     }
     store4<TC>(C + (size_t)m * n_out + j, a, j, n_out, (n_out % 4) == 0);
 }
@@ -343,9 +353,9 @@ static int launch_async_g(const bf16_t* A, const bf16_t* Wp, void* C, int M, int
         const long threads = (long)M * ((No + 3) / 4);
         const int blocks = (int)((threads + 255) / 256);
         if (c_dtype == TFF_F32)
-            gemm_splitk_reduce_kernel<GLU, float><<<blocks, 256, 0, s>>>(part, splits, M, N, (float*)C, No, ex.act);
+            gemm_splitk_reduce_kernel<GLU, float><<<blocks, 256, 0, s>>>(part, splits, M, N, (float*)C, No, ex.act, ex.unary);
         else
-            gemm_splitk_reduce_kernel<GLU, bf16_t><<<blocks, 256, 0, s>>>(part, splits, M, N, (bf16_t*)C, No, ex.act);
+            gemm_splitk_reduce_kernel<GLU, bf16_t><<<blocks, 256, 0, s>>>(part, splits, M, N, (bf16_t*)C, No, ex.act, ex.unary);
         return tff_check_launch("gemm_splitk_reduce");
     }
     return 0;
@@ -494,6 +504,13 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     const int tn = j / grp_rows, tm = grp * 8 + j % grp_rows;
     const int m0 = tm * BM, n0 = tn * BN;
     const int NB = (N + 15) / 16;
+    int ldc = N;
+    if (ex.plane_cols) {      // (a tile's columns are one plane's; C as its column 0 of row 0 would lie)
+        const size_t plane = (size_t)(n0 / ex.plane_cols);
+        A += plane * ex.a_step;
+        C += plane * (size_t)(M - 1) * ex.plane_cols;
+        ldc = ex.plane_cols;
+    }
     const int nu = KB / 2;                            // units of 64 k
     const int u_per = (nu + (int)gridDim.z - 1) / (int)gridDim.z;
     const int u0 = (int)blockIdx.z * u_per;
@@ -678,8 +695,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     } else {
         // (partial sums of a split K: plane blockIdx.z of the launcher's float32 workspace, which it passes as C)
         TC* out = C + (size_t)blockIdx.z * M * N;
-        w4_store_rows<WTN, REGION, TC, WTM>(region, [&](int i, int jj) { return scaled(acc[i][jj]); }, out, (size_t)N, mw,
-                                       n0 + wn * WTN * 16, M, N, lane_out, N % E == 0);
+        w4_store_rows<WTN, REGION, TC, WTM>(region, [&](int i, int jj) { return scaled(acc[i][jj]); }, out, (size_t)ldc, mw,
+                                       n0 + wn * WTN * 16, M, N, lane_out, ldc % E == 0);
     }
 }
 
@@ -713,9 +730,9 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
         const long threads = (long)M * ((No + 3) / 4);
         const int blocks = (int)((threads + 255) / 256);
         if (c_dtype == TFF_F32)
-            gemm_splitk_reduce_kernel<GLU, float><<<blocks, 256, 0, s>>>(part, splits, M, N, (float*)C, No, ex.act);
+            gemm_splitk_reduce_kernel<GLU, float><<<blocks, 256, 0, s>>>(part, splits, M, N, (float*)C, No, ex.act, ex.unary);
         else
-            gemm_splitk_reduce_kernel<GLU, bf16_t><<<blocks, 256, 0, s>>>(part, splits, M, N, (bf16_t*)C, No, ex.act);
+            gemm_splitk_reduce_kernel<GLU, bf16_t><<<blocks, 256, 0, s>>>(part, splits, M, N, (bf16_t*)C, No, ex.act, ex.unary);
         return tff_check_launch("gemm_splitk_reduce");
     }
     return 0;
@@ -780,6 +797,15 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
     const int fr = lane & 15, fg = lane >> 4;
     const int NB = (N + 15) / 16;
     const int nb0 = (blockIdx.x * NSETS + set) * R;
+    int ldc = N;
+    if constexpr (EPI == 0 && !GLU) {
+        if (ex.plane_cols) {      // (a wave's columns are one plane's; C as its column 0 of row 0 would lie)
+            const size_t plane = (size_t)(min(nb0, NB - 1) * 16 / ex.plane_cols);
+            A += plane * ex.a_step;
+            C += plane * (size_t)(M - 1) * ex.plane_cols;
+            ldc = ex.plane_cols;
+        }
+    }
 
     floatx4 acc[R][MT];
 #pragma unroll
@@ -973,7 +999,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
                 }
             }
         } else {
-            const bool vec = (N % 4) == 0;
+            const bool vec = (ldc % 4) == 0;
 #pragma unroll
             for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -1020,7 +1046,13 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
                             *reinterpret_cast<uint2*>(fz.x_out + (size_t)m * N + n) = pk.u;
                         }
                     } else if (m < M && n < N) {
-                        store4<TC>(C + (size_t)m * N + n, v, n, N, vec);
+                        if constexpr (EPI == 0) {
+                            if (ex.unary) {
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) v[e] = unary_activation(v[e], ex.unary);
+                            }
+                        }
+                        store4<TC>(C + (size_t)m * ldc + n, v, n, N, vec);
                     }
                 }
         }
@@ -1100,7 +1132,8 @@ static int plan_rows32(int N, int K) {
     return best;
 }
 
-static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep) {
+// plane > 0: the columns of several products, so many each; a tile takes columns of one of them, and K is not split.
+static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0) {
     const double CUS = (double)device_cus();
     // Up to 16 rows: the streaming kernel, a block per 16 columns, unless those blocks go badly
     // round the 256 CUs (320 of them take as long as 512 would: N = 5120), the caller takes
@@ -1108,6 +1141,7 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep) {
     // stream) to pay for the norm's own kernel, which the streaming kernel would have taken into
     // its epilogue: then the tiles below, whose blocks split K as finely as it takes.
     if (M <= 16 && glu && few_rows_gated_on_tiles(M, N, K)) return {32, plan_rows32(N, K), 1};
+    if (M <= 16 && plane) return {0, 0, 1};
     if (M <= 16) {
         const int nb = (N + 15) / 16;
         const double fill = (double)nb / (ceil(nb / CUS) * CUS);
@@ -1144,7 +1178,8 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep) {
             if (c.bm == 256 && M <= 64) continue;
             if (c.slots == 1 && c.bm <= 64 && M > c.bm) continue;         // (four waves side by side: one row tile)
             if (c.slots == 2 && (M <= 64 || M > 512)) continue;            // (64 x 128 with several row tiles)
-            for (int S = 1; S <= ((glu && M > 64) ? 2 : 8); S *= 2) {
+            if (plane % c.bn) continue;
+            for (int S = 1; S <= (plane ? 1 : (glu && M > 64) ? 2 : 8); S *= 2) {
                 if (S > 1 && nk / S < 4) break;
                 const double blocks = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * S;
                 const double rounds = ceil(blocks / (CUS * c.slots));
@@ -1285,11 +1320,13 @@ int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int 
     TFF_REQUIRE(((uintptr_t)A % 16) == 0 && ((uintptr_t)Wp % 16) == 0 && ((uintptr_t)C % 16) == 0,
                 "gemm: operands must be 16-byte aligned");
     TFF_REQUIRE(c_dtype == TFF_F32 || c_dtype == TFF_BF16, "gemm: unknown output type %d", c_dtype);
-    GemmPlan plan = plan_for(M, N, K, glu_out > 0, keep_partials != 0);
+    GemmPlan plan = plan_for(M, N, K, glu_out > 0, keep_partials != 0, ex.plane_cols);
     const int planned_splits = plan.splits;
     if (!workspace || workspace_bytes < (size_t)plan.splits * M * N * sizeof(float)) plan.splits = 1;
     const int S = plan.splits;
     const bool red = !keep_partials;
+    TFF_REQUIRE(!ex.unary || (glu_out == 0 && !keep_partials && (plan.tile == 0 || plan.splits > 1)),
+                "gemm: an activation is applied by the streaming kernel or by the sum over the parts of K");
     TFF_REQUIRE(!keep_partials || (glu_out == 0 && c_dtype == TFF_F32),
                 "gemm: partial sums are kept for a plain float32 result only");
     if (glu_out > 0) {
@@ -1450,6 +1487,37 @@ TFF_API int tff_gemm(const void* A, const void* W, void* C, int M, int N, int K,
                              (float*)workspace, workspace ? workspace_bytes : 0, keep_partials, s);
     }
     return tff_fail("gemm: unknown operand type %d", ab_dtype);
+}
+
+// C = act(A . W^T), act one of unary_activation's kinds, where the product's plan lets its last kernel apply it: the streaming
+// kernel, or the sum over the parts of a split K (tff_gemm_takes_unary).  Else 0 there, and the activation is a kernel of its own.
+TFF_API int tff_gemm_takes_unary(int M, int N, int K) {
+    const GemmPlan p = plan_for(M, N, K, false, false);
+    return p.tile == 0 || p.splits > 1;
+}
+TFF_API int tff_gemm_unary(const void* A, const void* W, void* C, int M, int N, int K, int lda, int c_dtype, int kind, void* workspace,
+                           size_t workspace_bytes, tff_stream_t stream) {
+    TFF_REQUIRE(A && W && C, "gemm_unary: null pointer");
+    TFF_REQUIRE(M >= 0 && N > 0 && K > 0 && lda >= K && kind >= 1 && kind <= 4, "gemm_unary: bad sizes M=%d N=%d K=%d lda=%d or kind %d", M, N, K, lda, kind);
+    TFF_REQUIRE(((uintptr_t)workspace % 16) == 0, "gemm_unary: the workspace must be 16-byte aligned");
+    if (M == 0) return 0;
+    return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, GemmExtra{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f), kind, 0, 0},
+                         c_dtype, 0, (float*)workspace, workspace ? workspace_bytes : 0, 0, (hipStream_t)stream);
+}
+
+// Several products of the same sizes in one launch: C[p] = A[p] . W[p]^T, p < planes, A[p] = A + p * a_step, C [planes, M, N] float32; W
+// their weights one after the other in fragment order.  Four products of 4,096 x 4,096 of 1,500 rows go three times round the CUs
+// instead of four times one that fills three quarters of them, and of one row they are one stream of 134 MB.
+// us, one by one / now: 4 x 4,096 x 4,096, 1,500 rows 234 / 181, one row 31 / 25.
+TFF_API int tff_gemm_planes_supported(int N, int K) { return N % 128 == 0 && K % 64 == 0; }
+TFF_API int tff_gemm_planes(const void* A, size_t a_step, const void* W, float* C, int planes, int M, int N, int K, int lda, tff_stream_t stream) {
+    TFF_REQUIRE(A && W && C, "gemm_planes: null pointer");
+    TFF_REQUIRE(M >= 0 && planes > 0 && N > 0 && K > 0 && lda >= K && (long)planes * N < (1L << 30), "gemm_planes: bad sizes %d x M=%d N=%d K=%d lda=%d",
+                planes, M, N, K, lda);
+    TFF_REQUIRE(tff_gemm_planes_supported(N, K) && a_step % 8 == 0, "gemm_planes: N=%d in units of 128, K=%d of 64, rows' planes (%zu apart) of 8", N, K, a_step);
+    if (M == 0) return 0;
+    return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, planes * N, K, lda, GemmExtra{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f), 0, N, a_step},
+                         TFF_F32, 0, nullptr, 0, 0, (hipStream_t)stream);
 }
 
 // ------------------------------------------------------------- packing ---

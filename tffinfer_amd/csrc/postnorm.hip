@@ -172,16 +172,6 @@ TFF_API int tff_scale_add_rmsnorm(float* resid, const float* delta, int delta_pl
     return tff_check_launch("scale_add_rmsnorm");
 }
 
-// form 0: gelu with erf; 1: its tanh approximation; 2: the square of relu
-__device__ __forceinline__ float ffn_activation(float z, int form) {
-    if (form == 2) {
-        const float r = fmaxf(z, 0.f);
-        return r * r;
-    }
-    if (form == 1) return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-    return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
-}
-
 template <typename T>
 __global__ void gelu_kernel(const T* __restrict__ x, T* __restrict__ out, int64_t n, int tanh_form) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

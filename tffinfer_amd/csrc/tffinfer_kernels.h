@@ -59,6 +59,15 @@ TFF_API size_t tff_gemm_workspace_bytes(int M, int N, int K, int ab_dtype, int g
 TFF_API int tff_gemm_plan(int M, int N, int K, int glu, int keep_partials, int* tile_rows, int* tile_cols,
                           int* splits);
 
+// C = act(A . W^T) in one go (kind 1: tanh, 2: gelu, 3: its tanh form, 4: the square of relu), where tff_gemm_takes_unary says so.
+TFF_API int tff_gemm_takes_unary(int M, int N, int K);
+TFF_API int tff_gemm_unary(const void* A, const void* W, void* C, int M, int N, int K, int lda, int c_dtype, int kind, void* workspace,
+                           size_t workspace_bytes, tff_stream_t stream);
+// C[p] = A[p] . W[p]^T, p < planes, in one launch: A[p] = A + p * a_step, C [planes, M, N] float32, W the weights one after the other in
+// fragment order; N in units of 128, K of 64.
+TFF_API int tff_gemm_planes_supported(int N, int K);
+TFF_API int tff_gemm_planes(const void* A, size_t a_step, const void* W, float* C, int planes, int M, int N, int K, int lda, tff_stream_t stream);
+
 // resid[M, N] += A . W^T; x_out[M, N] = bfloat16 of tanh(alpha * resid) * norm_w + bias over the new resid: a norm
 // without statistics in the epilogue of the product before it.  Up to 16 rows, bfloat16, N a multiple of 8.
 TFF_API int tff_gemm_residual_dyt(const void* A, const void* Wp, int M, int N, int K, int lda, float* resid, float alpha,

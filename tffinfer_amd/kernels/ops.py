@@ -443,6 +443,58 @@ def linear(x: torch.Tensor, weight, out_dtype: torch.dtype | None = None,
     return out
 
 
+_takes_unary_cache: dict[tuple, bool] = {}
+
+#: what :func:`linear_unary` may apply, and the number the kernels know it by
+UNARY = {"tanh": 1, "gelu": 2, "gelu_tanh": 3, "relu2": 4}
+
+
+def linear_unary(x: torch.Tensor, weight, act: str, out_dtype: torch.dtype) -> torch.Tensor:
+    """``act(x . weight^T)`` in ``out_dtype``: ``act`` tanh, gelu, gelu_tanh or relu2.  In the product's last kernel where that is the
+    streaming kernel (a few rows) or the sum over a split K's parts, else a kernel of its own over the product."""
+    packed = isinstance(weight, PackedWeight)
+    if packed and isinstance(x, torch.Tensor) and x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and x.stride(1) == 1 \
+            and x.shape[1] == weight.shape[1] and not weight.glu_out and x.shape[0] > 0:
+        M, K = x.shape
+        N = weight.shape[0]
+        lda = x.stride(0) if M > 1 else K
+        L = _lib.load()
+        key = (M, N, K)
+        if key not in _takes_unary_cache:
+            _takes_unary_cache[key] = bool(L.tff_gemm_takes_unary(M, N, K))
+        if _takes_unary_cache[key] and lda >= K and lda % 8 == 0 and x.data_ptr() % 16 == 0:
+            ws_bytes = L.tff_gemm_workspace_bytes(M, N, K, dtype_code(x.dtype), 0, 0)
+            ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device) if ws_bytes else None
+            out = torch.empty(M, N, dtype=out_dtype, device=x.device)
+            _lib.check(L.tff_gemm_unary(x.data_ptr(), weight.data_ptr(), out.data_ptr(), M, N, K, lda, dtype_code(out_dtype), UNARY[act],
+                                        _ptr(ws), ws_bytes, _stream()))
+            return out
+    if act == "tanh":
+        return tanh(linear(x, weight, out_dtype=torch.float32), out_dtype)
+    u = linear(x, weight, out_dtype=out_dtype)
+    return relu_squared(u) if act == "relu2" else gelu(u, act == "gelu_tanh")
+
+
+def planes_supported(N: int, K: int) -> bool:
+    """Whether :func:`linear_planes` takes bfloat16 products of [N, K]."""
+    return N % 128 == 0 and K % 64 == 0
+
+
+def linear_planes(x: torch.Tensor, weight: PackedWeight) -> torch.Tensor:
+    """``x[p] . weight[p]^T`` for contiguous bfloat16 x [P, M, K] and a packed weight of the P matrices [N, K] one after the other, in one
+    launch: float32 [P, M, N].  N in units of 128, K of 64 (:func:`planes_supported`)."""
+    _req(x, "linear_planes x", torch.bfloat16, 3)
+    P, M, K = x.shape
+    if not isinstance(weight, PackedWeight) or weight.glu_out or weight.shape[1] != K or weight.shape[0] % P \
+            or not planes_supported(weight.shape[0] // P, K):
+        raise _lib.KernelError(f"linear_planes: {P} planes of {K} and a weight of {tuple(weight.shape)} (a plane's rows in units of 128, "
+                               "the inner size of 64)")
+    N = weight.shape[0] // P
+    out = torch.empty(P, M, N, dtype=torch.float32, device=x.device)
+    _lib.check(_lib.load().tff_gemm_planes(x.data_ptr(), M * K, weight.data_ptr(), out.data_ptr(), P, M, N, K, K, _stream()))
+    return out
+
+
 def _linear_row_scaled(x: ScaledRows, weight: "PackedWeight", out_dtype: torch.dtype) -> torch.Tensor:
     M, K = x.shape
     N = weight.shape[0]
@@ -2382,6 +2434,8 @@ OP_TABLE = {
     "add_rmsnorm": add_rmsnorm,
     "rmsnorm": rmsnorm,
     "linear": linear,
+    "linear_unary": linear_unary,
+    "linear_planes": linear_planes,
     "as_tensor": as_tensor,
     "pack_weight": pack_weight,
     "qk_norm_rope_kv": qk_norm_rope_kv,

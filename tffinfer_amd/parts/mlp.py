@@ -127,8 +127,8 @@ class GeluMLP(FeedForward):
         self.w_down = to_device(weights["down"], dtype, device)
 
     def forward(self, ctx, x):
-        u = ctx.ops.linear(x, self.w_up)
-        a = ctx.ops.relu_squared(u) if self.activation == "relu2" else ctx.ops.gelu(u, self.tanh_form)
+        act = "relu2" if self.activation == "relu2" else "gelu_tanh" if self.tanh_form else "gelu"
+        a = ctx.ops.linear_unary(x, self.w_up, act, x.dtype)
         return ctx.ops.linear(a, self.w_down, out_dtype=torch.float32, partials=True)
 
 

@@ -45,7 +45,7 @@ class WKVMixer(Mixer):
             raise ConfigError(f"wkv: {num_heads} heads of {head_dim} on rows of {hidden_size} "
                               "(a head has up to 128 channels)")
         self.mu = self.w0 = self.u = self.norm = None
-        self.w_r = self.w_k = self.w_v = self.w_g = self.w_w1 = self.w_w2 = self.w_o = None
+        self.w_four = self.w_each = self.w_w1 = self.w_w2 = self.w_o = None
 
     @property
     def inner(self) -> int:
@@ -75,7 +75,13 @@ class WKVMixer(Mixer):
     def load_weights(self, weights, dtype, device):
         f32 = lambda t: t.to(torch.float32).contiguous().to(device)      # noqa: E731
         self.mu = f32(torch.stack([weights[f"mu.{s}"].to(torch.float32) for s in self.MIXES], 0))
-        self.w_r, self.w_k, self.w_v, self.w_g = (to_device(weights[s], dtype, device) for s in ("r", "k", "v", "g"))
+        four = [weights[s] for s in ("r", "k", "v", "g")]
+        self.w_four, self.w_each = None, None
+        if dtype == torch.bfloat16 and torch.device(device).type == "cuda" and self.inner % 128 == 0 and self.hidden_size % 64 == 0:
+            # one weight, a product of four planes
+            self.w_four = to_device(torch.cat([w.to(dtype) for w in four], 0), dtype, device)
+        else:
+            self.w_each = [to_device(w, dtype, device) for w in four]
         if weights["w1"].shape[0] != weights["w2"].shape[1]:
             raise ConfigError(f"wkv: the decay's matrices {tuple(weights['w1'].shape)} and "
                               f"{tuple(weights['w2'].shape)} do not fit each other")
@@ -91,11 +97,11 @@ class WKVMixer(Mixer):
         H, D = self.num_heads, self.head_dim
         f32 = torch.float32
         m = ops.token_shift_mix(x, ctx.state, self.prev_offset, self.mu, b, ctx.act_dtype)
-        r = ops.linear(m[0], self.w_r, out_dtype=f32)
-        k = ops.linear(m[1], self.w_k, out_dtype=f32)
-        v = ops.linear(m[2], self.w_v, out_dtype=f32)
-        g = ops.linear(m[3], self.w_g, out_dtype=f32)
-        z = ops.linear(ops.tanh(ops.linear(m[4], self.w_w1, out_dtype=f32), ctx.act_dtype), self.w_w2, out_dtype=f32)
+        if self.w_four is not None:
+            r, k, v, g = ops.linear_planes(m[:4], self.w_four)
+        else:
+            r, k, v, g = (ops.linear(m[i], w, out_dtype=f32) for i, w in enumerate(self.w_each))
+        z = ops.linear(ops.linear_unary(m[4], self.w_w1, "tanh", ctx.act_dtype), self.w_w2, out_dtype=f32)
         o = ops.wkv_recurrence(r, k, v, z, self.w0, self.u, ctx.state, b, H, D, x=x, prev_off=self.prev_offset)
         y = ops.head_norm_gate(o, g, self.norm, self.norm_eps, H, D, ctx.act_dtype)
         return ops.linear(y, self.w_o, out_dtype=f32, partials=True)
