@@ -425,14 +425,17 @@ __device__ __forceinline__ void v_page_write_block(
     }
 }
 
-// bfloat16, head sizes 16 .. 256 that are powers of two, the whole head rotated (or none of it):
+// bfloat16, head sizes 16 .. 256 that are powers of two, the whole head rotated, or none of it, or its first elements:
 // a lane has 8 consecutive elements of a head (one 16-byte access), LPH = d / 8 lanes a head,
 // 64 / LPH heads a wave.  The sum of squares goes over the head's lanes by shuffles; with pairs
 // (i, i + d/2) a lane's partner is LPH / 2 lanes away, with pairs (2i, 2i+1) it is the lane itself.
-template <int LPH>
+// PART: only the first `rot` elements of a head rotate (in units of 16 with pairs (i, i + rot / 2), of 8 with (2i, 2i+1)): the partner
+// is rot / 16 lanes away, the lanes behind keep theirs.  A wave a head and token with two bytes a lane, which took those shapes,
+// needed 49 us for 2,900 tokens of 40 heads of 128 whose first half rotates; now 19 (pairs (2i, 2i+1): 49 and 16).
+template <int LPH, bool PART>
 __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
     bf16_t* __restrict__ qkv, int nq, int nkv, const float* __restrict__ qw,
-    const float* __restrict__ kw, float eps, const float* __restrict__ cos_sin, int pairing,
+    const float* __restrict__ kw, float eps, const float* __restrict__ cos_sin, int rot, int pairing,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ slot_mapping,
     bf16_t* __restrict__ k_cache, int page_size, int qk_rows, int T, bf16_t* __restrict__ v_cache) {
     constexpr int D = LPH * 8, HPW = 64 / LPH;
@@ -465,10 +468,12 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
     union { uint4 u; bf16_t e[8]; } in, outv;
     in.u = *reinterpret_cast<const uint4*>(x);
     float4 q0 = make_float4(0.f, 0.f, 0.f, 0.f), q1 = q0, q2 = q0, q3 = q0;
-    if (cos_sin) {
-        const float* cs = cos_sin + (size_t)pos * D;   // [pos][pair][cos, sin]
+    const bool turns = cos_sin && (!PART || l * 8 < rot);
+    const int hl = PART ? rot >> 4 : LPH / 2;
+    if (turns) {
+        const float* cs = cos_sin + (size_t)pos * (PART ? rot : D);   // [pos][pair][cos, sin]
         if (pairing == 0) {
-            const float4* c4 = reinterpret_cast<const float4*>(cs + (l % (LPH / 2)) * 16);
+            const float4* c4 = reinterpret_cast<const float4*>(cs + (PART ? (l < hl ? l : l - hl) : l % (LPH / 2)) * 16);
             q0 = c4[0]; q1 = c4[1]; q2 = c4[2]; q3 = c4[3];
         } else {
             const float4* c4 = reinterpret_cast<const float4*>(cs + l * 8);
@@ -491,17 +496,18 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
     }
     if (cos_sin) {
         if (pairing == 0) {
-            constexpr int HL = LPH / 2;
             const float c[8] = {q0.x, q0.z, q1.x, q1.z, q2.x, q2.z, q3.x, q3.z};
             const float sn[8] = {q0.y, q0.w, q1.y, q1.w, q2.y, q2.w, q3.y, q3.w};
-            const bool first = l < HL;
+            const bool first = l < hl;
+            const int partner = !turns ? lane : first ? lane + hl : lane - hl;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float pv = __shfl_xor(v[e], HL, 64);
+                const float pv = PART ? __shfl(v[e], partner, 64) : __shfl_xor(v[e], LPH / 2, 64);
                 // first half: a = v, b = pv -> a c - b s;  second half: a = pv, b = v -> a s + b c
-                v[e] = first ? v[e] * c[e] - pv * sn[e] : pv * sn[e] + v[e] * c[e];
+                const float y = first ? v[e] * c[e] - pv * sn[e] : pv * sn[e] + v[e] * c[e];
+                if (!PART || turns) v[e] = y;
             }
-        } else {
+        } else if (turns) {
             const float c[4] = {q0.x, q0.z, q1.x, q1.z};
             const float sn[4] = {q0.y, q0.w, q1.y, q1.w};
 #pragma unroll
@@ -527,13 +533,17 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
 
 template <int LPH>
 static void launch_qk_vec(bf16_t* qkv, int T, int nq, int nkv, const float* qw, const float* kw, float eps,
-                          const float* cos_sin, int pairing, const int32_t* positions,
+                          const float* cos_sin, int rot, int pairing, const int32_t* positions,
                           const int32_t* slot_mapping, bf16_t* k_cache, bf16_t* v_cache, int page_size, hipStream_t s) {
     constexpr int HPB = 4 * (64 / LPH);
     const int qk_rows = (nq + nkv + HPB - 1) / HPB;
     const int v_rows = (int)(((long)((T + 7) / 8) * nkv + T - 1) / T);   // the values' blocks fill whole rows of the grid
-    qk_norm_rope_vec_kernel<LPH><<<dim3(T, qk_rows + v_rows), 256, 0, s>>>(
-        qkv, nq, nkv, qw, kw, eps, cos_sin, pairing, positions, slot_mapping, k_cache, page_size, qk_rows, T, v_cache);
+    if (cos_sin && rot < LPH * 8)
+        qk_norm_rope_vec_kernel<LPH, true><<<dim3(T, qk_rows + v_rows), 256, 0, s>>>(
+            qkv, nq, nkv, qw, kw, eps, cos_sin, rot, pairing, positions, slot_mapping, k_cache, page_size, qk_rows, T, v_cache);
+    else
+        qk_norm_rope_vec_kernel<LPH, false><<<dim3(T, qk_rows + v_rows), 256, 0, s>>>(
+            qkv, nq, nkv, qw, kw, eps, cos_sin, rot, pairing, positions, slot_mapping, k_cache, page_size, qk_rows, T, v_cache);
 }
 
 TFF_API int tff_qk_norm_rope_kv(void* qkv, int T, int nq, int nkv, int d, const float* q_weight,
@@ -565,12 +575,12 @@ TFF_API int tff_qk_norm_rope_kv(void* qkv, int T, int nq, int nkv, int d, const 
     TFF_REQUIRE(dtype == TFF_F32 || dtype == TFF_BF16, "qk_norm_rope_kv: unknown dtype %d", dtype);
     const bool pow2 = d >= 16 && d <= 256 && (d & (d - 1)) == 0;
     // for prompt portions: 16-byte accesses, the q and k heads and the values in blocks of their own of one launch
-    if (T >= 128 && dtype == TFF_BF16 && pow2 && (!cos_sin || rot_dim == d) && ((uintptr_t)qkv % 16) == 0 &&
+    if (T >= 128 && dtype == TFF_BF16 && pow2 && (!cos_sin || rot_dim == d || rot_dim % (pairing == 0 ? 16 : 8) == 0) && ((uintptr_t)qkv % 16) == 0 &&
         ((uintptr_t)k_cache % 16) == 0 && ((uintptr_t)v_cache % 16) == 0 &&
         (!q_weight || (((uintptr_t)q_weight % 16) == 0 && ((uintptr_t)k_weight % 16) == 0)) &&
         (!cos_sin || ((uintptr_t)cos_sin % 16) == 0)) {
 #define TFF_QK_VEC(L)                                                                               \
-    launch_qk_vec<L>((bf16_t*)qkv, T, nq, nkv, q_weight, k_weight, eps, cos_sin, pairing, positions, \
+    launch_qk_vec<L>((bf16_t*)qkv, T, nq, nkv, q_weight, k_weight, eps, cos_sin, rot_dim, pairing, positions, \
                      slot_mapping, (bf16_t*)k_cache, (bf16_t*)v_cache, page_size, s)
         switch (d) {
             case 16: TFF_QK_VEC(2); break;
