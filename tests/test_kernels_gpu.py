@@ -1629,3 +1629,13 @@ def test_products_with_an_activation(act, M, N, K):
     for dtype, tol in ((torch.bfloat16, 3 * 2.0 ** -8), (torch.float32, 2.0 ** -18)):
         out = ops.linear_unary(x, ops.pack_weight(w), act, dtype)
         assert out.dtype == dtype and float((out.double() - ref).abs().max()) < tol * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("sizes", [[4], [16, 20], [4096, 5, 1 << 20], [3 * i + 1 for i in range(50)]])
+def test_rows_set_to_zero(sizes):
+    """Buffers of any number of words, more than one launch of them, at addresses that are no multiple of 16; what lies beside stays."""
+    ops = _ops()
+    bufs = [torch.full((n + 8,), 7.0, device=DEV) for n in sizes]
+    ops.zero_rows([b[i % 5:i % 5 + n] for i, (b, n) in enumerate(zip(bufs, sizes))])
+    for i, (b, n) in enumerate(zip(bufs, sizes)):
+        assert int((b == 0).sum()) == n and float(b[i % 5:i % 5 + n].abs().max()) == 0

@@ -3,6 +3,7 @@ level of its op or part, then whole models through the step function (whole prom
 token by token, portions down to two tokens, mixed batches on a pool whose pages and slots are
 used again), and greedy generation through the engine's own entry point and scheduler."""
 import math
+import types
 
 import pytest
 import torch
@@ -204,6 +205,31 @@ def test_clamps_in_the_gated_product(M, I, K, limit):
     plain_act = ops.linear(x.to(DEV), ops.pack_gate_up(g.to(DEV), u.to(DEV)))
     full = (x.double() @ g.double().T, x.double() @ u.double().T)
     assert _err(plain_act.float(), plain.silu(full[0]) * full[1]) < 6e-3
+
+
+@pytest.mark.parametrize("T,pairing", [(128, 0), (203, 0), (129, 1)])
+@pytest.mark.parametrize("H,G,D,ps,turn,bias,norm", [(4, 2, 128, 16, True, True, False), (9, 3, 64, 16, True, False, True), (2, 1, 24, 8, True, True, True),
+                                                     (10, 2, 256, 32, False, False, False), (16, 4, 40, 4, True, False, False)])
+def test_grouped_projections_of_many_tokens(T, pairing, H, G, D, ps, turn, bias, norm):
+    """From 128 tokens on in whole pieces, the values eight tokens at a time: the same bits as for the same tokens in steps of fewer, with
+    slots that begin and end inside runs of eight, and tokens that write no key."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(D + T)
+    r = lambda *s: torch.randn(*s, generator=g).to(DEV)       # noqa: E731
+    proj, table = r(T, (H + 2 * G) * D + 4), r(64, D // 2, 2) if turn else None
+    pages = T // ps + 6
+    slots = torch.cat([torch.arange(90) + 3, torch.arange(T - 90) + 96]).to(torch.int32)      # (two requests; the second begins a run)
+    slots[40] = -1
+    positions = torch.randint(0, 64, (T,), generator=g).to(torch.int32).to(DEV)
+    how = dict(bias=r((H + 2 * G) * D) if bias else None, q_norm=r(H * D) if norm else None, k_norm=r(G * D) if norm else None, eps=1e-5)
+    got = []
+    for step in (T, 60):
+        kc = torch.zeros(pages, G, ps, D, dtype=torch.bfloat16, device=DEV)
+        vc = torch.zeros(pages, G, D, ps, dtype=torch.bfloat16, device=DEV)
+        q = [ops.grouped_qkv_store(proj[i:i + step], H, G, D, D, table, pairing, (0.1, 5), positions[i:i + step],
+                                   types.SimpleNamespace(k_cache=kc, v_cache=vc, slot_mapping=slots[i:i + step].to(DEV)), **how) for i in range(0, T, step)]
+        got.append((torch.cat(q), kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and float(got[0][2].abs().sum()) > 0
 
 
 @pytest.mark.parametrize("E,top,groups,keep,ff,shared,scale", [

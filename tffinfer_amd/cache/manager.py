@@ -173,8 +173,13 @@ class CacheManager:
         for g in self.groups:
             g.tables[req] = []
             g.pool_tables[req] = [[] for _ in g.spec.pools]
-        for t in self.state_tensors.values():
-            t[slot].zero_()
+        rows = [t[slot] for t in self.state_tensors.values()]
+        if rows and rows[0].is_cuda:
+            from ..kernels import ops
+            ops.zero_rows(rows)             # (one launch for all layers' rows)
+        else:
+            for row in rows:
+                row.zero_()
         return slot
 
     def pages_needed(self, req, n_new: int) -> list[int]:

@@ -135,6 +135,113 @@ __global__ __launch_bounds__(NT) void grouped_qkv_store_kernel(
     }
 }
 
+// The same for steps of many tokens in bfloat16 whose heads are of one size in units of eight and turn as a whole, in either pairing, or
+// not at all: a thread has four neighbouring elements of either half of a head, 16 bytes a load, and the values go to their transposed pages eight
+// tokens at a time, 16 bytes a store, in blocks of their own (the grid's rows from qk_rows on).  One value of a token is two bytes
+// of a line that its neighbours' blocks write too, on other XCDs.  The same sums in the same order: the same bits.
+// us, an element a thread and load / now: 4,500 tokens of 32 + 8 + 8 heads of 128 65 / 45, with norms over all of q and k 74 / 60;
+// 1,500 tokens 24 / 17 and 30 / 23.
+template <int NT>
+__global__ __launch_bounds__(NT) void grouped_qkv_store_vec_kernel(
+    const float* __restrict__ proj, size_t row, const float* __restrict__ cos_sin, int pairing, int max_pos, float temp_coef, int temp_every,
+    const GroupedPre pre, const int32_t* __restrict__ positions, const int32_t* __restrict__ slots, bf16_t* __restrict__ q_out,
+    bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache, int page_size, int T, int H, int G, int D, int q_blocks, int per_q,
+    int qk_rows, int per_kv) {
+    __shared__ float red[NT / 64];
+    __shared__ __attribute__((aligned(16))) bf16_t tile[8][256 + 8];
+    __shared__ int vslots[8];
+    const int tid = threadIdx.x, y = blockIdx.y;
+    if (y >= qk_rows) {                     // values: eight tokens and one kv head
+        const long item = (long)(y - qk_rows) * T + blockIdx.x;
+        if (item >= (long)((T + 7) / 8) * G) return;
+        const int t0 = (int)(item / G) * 8, g = (int)(item % G), ppr = D >> 2;
+        if (tid < 8) vslots[tid] = t0 + tid < T ? slots[t0 + tid] : -1;
+        const size_t cv = (size_t)H * D + (size_t)G * D + (size_t)g * D;
+        for (int i = tid; i < 8 * ppr; i += NT) {
+            const int tk = i / ppr, e = (i - tk * ppr) * 4;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (t0 + tk < T) v = *reinterpret_cast<const float4*>(proj + (size_t)(t0 + tk) * row + cv + e);
+            if (pre.bias) {
+                const float4 b = *reinterpret_cast<const float4*>(pre.bias + cv + e);
+                v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
+            }
+            tile[tk][e] = (bf16_t)v.x; tile[tk][e + 1] = (bf16_t)v.y; tile[tk][e + 2] = (bf16_t)v.z; tile[tk][e + 3] = (bf16_t)v.w;
+        }
+        __syncthreads();
+        const int s0 = vslots[0];
+        bool run = s0 >= 0 && (s0 & 7) == 0 && page_size % 8 == 0;
+#pragma unroll
+        for (int i = 1; i < 8; ++i) run = run && vslots[i] == s0 + i;
+        for (int e = tid; e < D; e += NT) {
+            if (run) {
+                union { uint4 u; bf16_t h[8]; } pk;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) pk.h[i] = tile[i][e];
+                *reinterpret_cast<uint4*>(v_cache + (((size_t)(s0 / page_size) * G + g) * D + e) * page_size + s0 % page_size) = pk.u;
+            } else {
+                for (int i = 0; i < 8; ++i)
+                    if (vslots[i] >= 0) v_cache[(((size_t)(vslots[i] / page_size) * G + g) * D + e) * page_size + vslots[i] % page_size] = tile[i][e];
+            }
+        }
+        return;
+    }
+    const int t = blockIdx.x, half = D >> 1, pieces = D >> 3;
+    const bool is_q = y < q_blocks;
+    const int slot = is_q ? 0 : slots[t];
+    const int pos = max(positions[t], 0), tpos = min(pos, max(max_pos - 1, 0));
+    if (slot < 0) return;      // (the whole block: a token that writes no key)
+    const size_t c0 = is_q ? 0 : (size_t)H * D;
+    const float* x = proj + (size_t)t * row + c0;
+    const float* bias = pre.bias ? pre.bias + c0 : nullptr;
+    const float* nw = is_q ? pre.q_norm : pre.k_norm;
+    const int heads = is_q ? H : G, first = is_q ? y * per_q : (y - q_blocks) * per_kv, count = min(heads, first + (is_q ? per_q : per_kv)) - first;
+    const float temp = is_q && temp_coef != 0.f ? 1.0f + temp_coef * logf((float)((pos + 1) / temp_every + 1)) : 1.0f;
+    const float rr = nw ? grouped_rms<NT>(x, bias, heads * D, pre.eps, 1, red) : 1.0f;
+    const float* cs = cos_sin ? cos_sin + (size_t)tpos * D : nullptr;
+    bf16_t* const to = is_q ? q_out + (size_t)t * H * D : k_cache + (((size_t)(slot / page_size) * G) * page_size + slot % page_size) * D;
+    const size_t step = is_q ? (size_t)D : (size_t)page_size * D;
+    for (int idx = tid; idx < count * pieces; idx += NT) {
+        const int h = first + idx / pieces, p = (idx % pieces) * 4, e = h * D + p;
+        float u[4], w[4], c[8];
+        auto take = [&](float* v, int at) {
+            *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(x + at);
+            if (bias) {
+                const float4 b = *reinterpret_cast<const float4*>(bias + at);
+                v[0] += b.x; v[1] += b.y; v[2] += b.z; v[3] += b.w;
+            }
+            if (nw) {
+                const float4 n = *reinterpret_cast<const float4*>(nw + at);
+                v[0] = v[0] * rr * n.x; v[1] = v[1] * rr * n.y; v[2] = v[2] * rr * n.z; v[3] = v[3] * rr * n.w;
+            }
+        };
+        if (cs) {
+            // (cosine and sine of the piece's four pairs, or of its two pairs in the first half and of the two in the second)
+            *reinterpret_cast<float4*>(c) = *reinterpret_cast<const float4*>(pairing == 0 ? cs + 2 * p : cs + p);
+            *reinterpret_cast<float4*>(c + 4) = *reinterpret_cast<const float4*>(pairing == 0 ? cs + 2 * p + 4 : cs + half + p);
+        }
+        take(u, e);
+        take(w, e + half);
+        union { uint2 v; bf16_t b[4]; } a, b;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float yu = u[k], yw = w[k];
+            if (cs && pairing == 0) {
+                yu = fmaf(u[k], c[2 * k], -(w[k] * c[2 * k + 1]));
+                yw = fmaf(w[k], c[2 * k], u[k] * c[2 * k + 1]);
+            } else if (cs) {
+                const int j = k & 2;
+                yu = !(k & 1) ? fmaf(u[k], c[j], -(u[k ^ 1] * c[j + 1])) : fmaf(u[k], c[j], u[k ^ 1] * c[j + 1]);
+                yw = !(k & 1) ? fmaf(w[k], c[4 + j], -(w[k ^ 1] * c[4 + j + 1])) : fmaf(w[k], c[4 + j], w[k ^ 1] * c[4 + j + 1]);
+            }
+            a.b[k] = (bf16_t)(is_q ? yu * temp : yu);
+            b.b[k] = (bf16_t)(is_q ? yw * temp : yw);
+        }
+        bf16_t* const o = to + (size_t)h * step + p;
+        *reinterpret_cast<uint2*>(o) = a.v;
+        *reinterpret_cast<uint2*>(o + half) = b.v;
+    }
+}
+
 TFF_API int tff_grouped_qkv_store(const float* proj, size_t row, const float* cos_sin, int rot_dims, int pairing, int max_pos,
                                   float temp_coef, int temp_every, const float* bias, const float* q_norm, const float* k_norm,
                                   float norm_eps, const int32_t* positions, const int32_t* slots, void* q_out, void* k_cache,
@@ -158,6 +265,21 @@ TFF_API int tff_grouped_qkv_store(const float* proj, size_t row, const float* co
     TFF_REQUIRE(q_blocks + kv_blocks <= 65535, "grouped_qkv_store: too many heads");
     const dim3 grid(T, q_blocks + kv_blocks);
     const bool wide = q_norm || k_norm || T < 128;
+    auto ok16 = [](const void* p) { return ((uintptr_t)p % 16) == 0; };
+    if (T >= 128 && store && dtype == TFF_BF16 && vec && D == E && D == P && D % 8 == 0 && D <= 256 && ok16(q_norm) && ok16(k_norm) && ok16(cos_sin) &&
+        ok16(q_out) && ok16(k_cache) && ok16(v_cache) && (rot_dims == 0 || rot_dims == D)) {
+        const int qk_rows = q_blocks + kv_blocks, v_rows = (int)(((long)((T + 7) / 8) * G + T - 1) / T);      // (the values' blocks fill whole rows of the grid)
+        const dim3 vgrid(T, qk_rows + v_rows);
+#define GQ_VEC(NT)                                                                                                                  \
+    grouped_qkv_store_vec_kernel<NT><<<vgrid, NT, 0, s>>>(proj, row, rot_dims ? cos_sin : nullptr, pairing, max_pos, temp_coef, temp_every, \
+                                                          GroupedPre{bias, q_norm, k_norm, norm_eps}, positions, slots, (bf16_t*)q_out, \
+                                                          (bf16_t*)k_cache, (bf16_t*)v_cache, page_size, T, H, G, D, q_blocks, per_q,    \
+                                                          qk_rows, per_kv)
+        if (wide) GQ_VEC(GQ_WIDE);
+        else GQ_VEC(GQ_THREADS);
+#undef GQ_VEC
+        return tff_check_launch("grouped_qkv_store");
+    }
 #define GQ_LAUNCH(TC, NT)                                                                                                      \
     grouped_qkv_store_kernel<TC, NT><<<grid, NT, 0, s>>>(proj, row, cos_sin, rot_dims, pairing, max_pos, temp_coef, temp_every, \
                                                          GroupedPre{bias, q_norm, k_norm, norm_eps}, positions, slots, (TC*)q_out, \

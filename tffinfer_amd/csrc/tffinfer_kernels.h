@@ -388,6 +388,8 @@ TFF_API int tff_wkv_recurrence_chunks(const float* r, const float* k, const floa
 // out = o / sqrt(mean over each head of o^2 + eps) * nw * silu(g); g rows g_row elements apart.
 TFF_API int tff_head_norm_gate(const float* o, const float* g, size_t g_row, const float* nw, float eps, void* out, int T,
                                int H, int D, int out_dtype, tff_stream_t stream);
+// n buffers of bytes[i] bytes (multiples of four, at addresses of such) set to zero, up to 24 in a launch; both tables on the host.
+TFF_API int tff_zero_rows(void* const* p, const size_t* bytes, int n, tff_stream_t stream);
 TFF_API int tff_tanh(const float* in, void* out, size_t count, int out_dtype, tff_stream_t stream);
 
 // ---- the gated delta rule (gated_delta.hip) ----

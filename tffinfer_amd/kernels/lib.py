@@ -88,6 +88,7 @@ _SIGNATURES = {
     "tff_wkv_chunks_workspace_bytes": [_I, _I, _I, _I],
     "tff_wkv_recurrence_chunks": [_P, _P, _P, _P, _Z, _P, _P, _P, _Z, _P, _P, _P, _P, _I, _I, _I, _I, _P, _I, _Z, _I, _P],
     "tff_head_norm_gate": [_P, _P, _Z, _P, _F, _P, _I, _I, _I, _I, _P],
+    "tff_zero_rows": [_P, _P, _I, _P],
     "tff_tanh": [_P, _P, _Z, _I, _P],
     "tff_gdelta_prep": [_P, _Z, _P, _I, _P, _P, _P, _Z, _Z, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "tff_gdelta_recurrence": [_P, _P, _Z, _P, _Z, _Z, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],

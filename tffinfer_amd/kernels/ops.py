@@ -1549,6 +1549,22 @@ def head_norm_gate(o: torch.Tensor, g: torch.Tensor, weight: torch.Tensor, eps: 
     return out
 
 
+def zero_rows(rows: list) -> None:
+    """Contiguous tensors on one device set to zero, many in a launch."""
+    if not rows:
+        return
+    with torch.cuda.device(rows[0].device):
+        for t in rows:
+            if not t.is_cuda or not t.is_contiguous() or t.device != rows[0].device or t.numel() * t.element_size() % 4 or t.data_ptr() % 4:
+                for r in rows:
+                    r.zero_()
+                return
+        n = len(rows)
+        ptrs = (ctypes.c_void_p * n)(*[t.data_ptr() for t in rows])
+        sizes = (ctypes.c_size_t * n)(*[t.numel() * t.element_size() for t in rows])
+        _lib.check(_lib.load().tff_zero_rows(ctypes.addressof(ptrs), ctypes.addressof(sizes), n, _stream()))
+
+
 def tanh(x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     _req(x, "tanh input", torch.float32)
     out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
