@@ -11,6 +11,7 @@ from __future__ import annotations
 
 from dataclasses import dataclass, field
 
+import numpy as np
 import torch
 
 from ..kernels.key_runs import deal_key_runs
@@ -98,27 +99,31 @@ def _pad4(n: int) -> int:
 
 
 class PinnedTables:
-    """A pinned host buffer for the step's tables that is used again step after step: to pin
-    memory anew for every step costs more than the copy it speeds up.  The copy out of it is
-    asynchronous, so the next step waits for that copy (an event) before it writes."""
+    """Pinned host buffers for the step's tables that are used again step after step: to pin
+    memory anew for every step costs more than the copy it speeds up.  The copy out of one is
+    asynchronous, and it runs when the device reaches the step; the buffers go round, so that the
+    host waits for a copy (an event) only ``RING`` steps later and can prepare the next steps meanwhile."""
+    RING = 4
 
     def __init__(self, ints: int = 1 << 16):
-        self._buf = torch.empty(int(ints), dtype=torch.int32, pin_memory=True)
-        self._copied = torch.cuda.Event()
-        self._busy = False
+        self._bufs = list(torch.empty(self.RING, int(ints), dtype=torch.int32, pin_memory=True).unbind(0))
+        self._copied: list = [None] * self.RING
+        self._at = 0
 
     def take(self, ints: int) -> torch.Tensor:
-        if self._busy:
-            self._copied.synchronize()
-            self._busy = False
-        if ints > self._buf.numel():
-            self._buf = torch.empty(max(int(ints), 2 * self._buf.numel()), dtype=torch.int32, pin_memory=True)
-        return self._buf[:ints]
+        i = self._at
+        if self._copied[i] is not None:
+            self._copied[i].synchronize()
+            self._copied[i] = None
+        if ints > self._bufs[i].numel():
+            self._bufs[i] = torch.empty(max(int(ints), 2 * self._bufs[i].numel()), dtype=torch.int32, pin_memory=True)
+        return self._bufs[i][:ints]
 
     def copied(self) -> None:
         """To be called right after the copy to the device was queued."""
-        self._copied.record()
-        self._busy = True
+        self._copied[self._at] = torch.cuda.Event()
+        self._copied[self._at].record()
+        self._at = (self._at + 1) % self.RING
 
 
 def build_step_batch(entries, cache, device, pinned: PinnedTables | None = None) -> StepBatch:
@@ -128,13 +133,11 @@ def build_step_batch(entries, cache, device, pinned: PinnedTables | None = None)
     memory, and a copy that waits)."""
     b = StepBatch()
     R = len(entries)
-    tok, pos, treq, cu, start, ctxl, slots, rows = [], [], [], [0], [], [], [], []
-    for r, e in enumerate(entries):
+    tok, cu, start, ctxl, slots, rows = [], [0], [], [], [], []
+    for e in entries:
         P = cache.num_tokens(e.req)
         n = len(e.tokens)
         tok.extend(e.tokens)
-        pos.extend(range(P, P + n))
-        treq.extend([r] * n)
         base = cu[-1]
         rows.extend(base + w for w in e.want)
         cu.append(base + n)
@@ -144,7 +147,10 @@ def build_step_batch(entries, cache, device, pinned: PinnedTables | None = None)
         b.max_new_tokens = max(b.max_new_tokens, n)
         b.max_context = max(b.max_context, P + n)
     T = cu[-1]
-    sections = [tok, pos, treq, cu, start, ctxl, slots, rows, [-1] * T]
+    counts = np.diff(np.array(cu, dtype=np.int32))
+    treq = np.repeat(np.arange(R, dtype=np.int32), counts)
+    pos = np.arange(T, dtype=np.int32) + np.repeat(np.array(start, dtype=np.int32) - np.array(cu[:-1], dtype=np.int32), counts)
+    sections = [tok, pos, treq, cu, start, ctxl, slots, rows, np.full(T, -1, dtype=np.int32)]
     group_meta = []
     for gi, g in enumerate(cache.groups):
         tables = [cache.block_table(gi, e.req) for e in entries]
@@ -153,9 +159,7 @@ def build_step_batch(entries, cache, device, pinned: PinnedTables | None = None)
         for t in tables:
             flat.extend(p if p >= 0 else 0 for p in t)
             flat.extend([0] * (width - len(t)))
-        sm = []
-        for e, P in zip(entries, start):
-            sm.extend(cache.slot_mapping(gi, e.req, P, len(e.tokens)))
+        sm = np.concatenate([cache.slot_array(gi, e.req, P, len(e.tokens)) for e, P in zip(entries, start)] or [np.empty(0, dtype=np.int32)])
         group_meta.append((len(sections), width))
         sections.append(flat)
         sections.append(sm)

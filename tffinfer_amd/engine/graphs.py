@@ -32,7 +32,7 @@ import weakref
 import numpy as np
 import torch
 
-from .batch import GroupTables, StepBatch
+from .batch import GroupTables, PinnedTables, StepBatch
 from ..kernels.key_runs import deal_key_runs, max_key_runs
 
 
@@ -206,8 +206,10 @@ class DecodeGraph:
         widths = [-(-runner.max_model_len // cache.page_size) for _ in cache.groups]
         _, total = table_layout(B, widths, [max_key_runs(B, g.spec.num_kv_heads) for g in cache.groups],
                                 [w for _, _, w in pool_table_widths(cache, runner.max_model_len)])
-        self.host = torch.zeros(total, dtype=torch.int32, pin_memory=True)
-        self.tables = DecodeTables(cache, B, runner.max_model_len, self.host.numpy())
+        self.tables = DecodeTables(cache, B, runner.max_model_len)
+        # The tables leave through pinned buffers that go round: a copy runs when the device reaches its step, and the host, which
+        # writes into `tables` only, waits for a buffer's copy no sooner than some steps later.
+        self._pinned = PinnedTables(total)
         self.widths = self.tables.widths
         self.offs = o = self.tables.offs
         self.dev = torch.zeros(total, dtype=torch.int32, device=runner.device)
@@ -241,8 +243,7 @@ class DecodeGraph:
         # results is left out), and, per cache group, whether a run gets a block of eight waves or a
         # single one.  Each variant is captured when it is first wanted, on tables of padding rows.
         self._variants: dict[tuple, list[_Piece]] = {}
-        self._padding = self.host.clone()           # the tables as they are with no live row
-        self._copied = torch.cuda.Event()
+        self._padding = torch.from_numpy(self.tables.hv.copy())      # the tables as they are with no live row
 
     @property
     def runner(self):
@@ -254,7 +255,6 @@ class DecodeGraph:
         return next(iter(self._variants.values())) if self._variants else []
 
     def fill(self, entries) -> None:
-        self._copied.synchronize()      # the last copy out of the host buffer is done
         self.tables.fill(entries)
 
     def possible_variants(self) -> list:
@@ -364,8 +364,10 @@ class DecodeGraph:
         if variant not in self._variants:
             self.capture(variant)
         pieces = self._variants[variant]
-        self.dev.copy_(self.host, non_blocking=True)
-        self._copied.record()
+        host = self._pinned.take(self.tables.total)
+        host.numpy()[:] = self.tables.hv
+        self.dev.copy_(host, non_blocking=True)
+        self._pinned.copied()
         R = len(entries)
         if token_source is not None:
             self.dev[self.offs[0]:self.offs[0] + R].copy_(token_source)
