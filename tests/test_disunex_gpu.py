@@ -255,6 +255,31 @@ def test_products_per_head_in_whole_pieces(T, H, K, N, tail, dims, pairing, pad)
     assert torch.equal(run(n), out[:n])              # (another number of tokens: the same order of k)
 
 
+@pytest.mark.parametrize("T", [1, 5, 64, 67, 150])
+@pytest.mark.parametrize("H,K,N,rank,rot,dims,ps,Dp,dtype", [(4, 64, 40, 40, 8, 8, 16, 48, torch.bfloat16), (3, 128, 192, 192, 64, 64, 8, 256, torch.bfloat16),
+                                                             (2, 72, 24, 24, 16, 0, 16, 48, torch.bfloat16), (2, 64, 24, 24, 16, 16, 16, 48, torch.float32)])
+def test_keys_stored_beside_the_products(T, H, K, N, rank, rot, dims, ps, Dp, dtype):
+    """In one launch (inner sizes of whole units, bfloat16) or in one before: cache and products are the same bits as apart."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(K + T)
+    proj = torch.randn(T, H * K + rank + rot + 8, generator=g).to(dtype).to(DEV)
+    wt = (torch.randn(H, N, K, generator=g) * 0.2).to(dtype).to(DEV)
+    norm = (1 + 0.2 * torch.randn(rank, generator=g)).to(DEV)
+    table = torch.randn(64, dims // 2, 2, generator=g).to(DEV) if dims else None
+    positions = torch.randint(0, 64, (T,), generator=g).to(torch.int32).to(DEV)
+    pages = T // ps + 3
+    slots = torch.randperm(pages * ps, generator=g)[:T].to(torch.int32)
+    slots[T // 2] = -1 if T > 1 else slots[0]
+    slots = slots.to(DEV)
+    got = []
+    for later in (False, True):
+        kc = torch.full((pages, 1, ps, Dp), 3.0, dtype=dtype, device=DEV)
+        vc = torch.full((pages, 1, Dp, ps), 3.0, dtype=dtype, device=DEV)
+        store = ops.latent_kv_store(proj[:, H * K:H * K + rank + rot], rank, rot, norm, 1e-5, table, positions, slots, kc, vc, later=later)
+        got.append((ops.head_linear(proj[:, :H * K], K, wt, store=store), kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and float((got[0][1] != 3.0).sum()) > 0
+
+
 def _sink_ref(q, keys, vals, positions, window, scale, sinks):
     """q [T, nq, d] against one key head: keys [S, d], vals [S, dv]."""
     T, nq, _ = q.shape

@@ -44,6 +44,35 @@ __device__ __forceinline__ float latent_rotated(const T* __restrict__ x, int e, 
     return first ? fmaf(v, c, -(o * s)) : fmaf(v, c, o * s);
 }
 
+// A token's key side: x's latent part normed and its rotated part into the token's slot; by all threads of the block.
+template <typename T, typename TC>
+__device__ __forceinline__ void latent_store_token(const T* __restrict__ xr, int t, int rank, int rot, int rot_dims, int pairing,
+                                                   const float* __restrict__ norm_w, float eps, const float* __restrict__ cos_sin, int max_pos,
+                                                   const int32_t* __restrict__ positions, int slot, TC* __restrict__ k_cache,
+                                                   TC* __restrict__ v_cache, int page_size, int Dp, float* red) {
+    const int tid = threadIdx.x;
+    float ss = 0.f;
+    for (int e = tid; e < rank; e += blockDim.x) {
+        const float v = to_f32(xr[e]);
+        ss = fmaf(v, v, ss);
+    }
+    ss = block_sum(ss, red);
+    const float rr = 1.0f / sqrtf(ss / (float)rank + eps);
+    const int page = slot / page_size, off = slot - page * page_size;
+    TC* kr = k_cache + ((size_t)page * page_size + off) * Dp;
+    TC* vr = v_cache + (size_t)page * Dp * page_size + off;
+    for (int e = tid; e < rank; e += blockDim.x) {
+        const TC c = from_f32<TC>(to_f32(xr[e]) * rr * norm_w[e]);
+        kr[e] = c;
+        vr[(size_t)e * page_size] = c;
+    }
+    int pos = positions[t];
+    pos = min(max(pos, 0), max_pos - 1);
+    const float* cs = cos_sin ? cos_sin + (size_t)pos * rot_dims : nullptr;   // [pair][cos, sin]
+    for (int e = tid; e < Dp - rank; e += blockDim.x)
+        kr[rank + e] = from_f32<TC>(e < rot ? latent_rotated<T>(xr + rank, e, rot_dims, pairing, cs) : 0.f);
+}
+
 // One block a token.  xq (may be null): the query's latent vector, q_rank elements, whose RMS norm times
 // q_norm_w goes to q_out.  x (may be null: a layer that reads another layer's cache): the key side.
 template <typename T, typename TC>
@@ -70,27 +99,8 @@ __global__ __launch_bounds__(256) void latent_kv_store_kernel(
     if (!x) return;
     const int slot = slots[t];
     if (slot < 0) return;      // (the whole block: a token that writes no key)
-    const T* xr = x + (size_t)t * x_stride;
-    float ss = 0.f;
-    for (int e = tid; e < rank; e += blockDim.x) {
-        const float v = to_f32(xr[e]);
-        ss = fmaf(v, v, ss);
-    }
-    ss = block_sum(ss, red);
-    const float rr = 1.0f / sqrtf(ss / (float)rank + eps);
-    const int page = slot / page_size, off = slot - page * page_size;
-    TC* kr = k_cache + ((size_t)page * page_size + off) * Dp;
-    TC* vr = v_cache + (size_t)page * Dp * page_size + off;
-    for (int e = tid; e < rank; e += blockDim.x) {
-        const TC c = from_f32<TC>(to_f32(xr[e]) * rr * norm_w[e]);
-        kr[e] = c;
-        vr[(size_t)e * page_size] = c;
-    }
-    int pos = positions[t];
-    pos = min(max(pos, 0), max_pos - 1);
-    const float* cs = cos_sin ? cos_sin + (size_t)pos * rot_dims : nullptr;   // [pair][cos, sin]
-    for (int e = tid; e < Dp - rank; e += blockDim.x)
-        kr[rank + e] = from_f32<TC>(e < rot ? latent_rotated<T>(xr + rank, e, rot_dims, pairing, cs) : 0.f);
+    latent_store_token<T, TC>(x + (size_t)t * x_stride, t, rank, rot, rot_dims, pairing, norm_w, eps, cos_sin, max_pos, positions, slot, k_cache,
+                              v_cache, page_size, Dp, red);
 }
 
 TFF_API int tff_latent_kv_store(const void* x, int x_stride, int T, int rank, int rot, int rot_dims, int pairing,
@@ -389,12 +399,31 @@ __global__ __launch_bounds__(256, 2) void head_linear_mfma_kernel(
 // What bounds it is the rows going in and out, 60 MB for 2,048 tokens of 32 heads; with few tokens two latencies to memory.
 // us, the kernel above as it was with results one by one / now: heads of 128 with a rotated tail of 64 into 256 elements, 1, 100, 2,048 and
 // 8,192 tokens 4.5 / 3.5, 18.7 / 4.2, 56 / 19, 171 / 63; of 256 into 128 with a gate 7.2 / 4.4, 16.4 / 5.0, 52 / 23, 257 / 87.
+// STORE: the launch writes the tokens' keys too (TffLatentStore, bfloat16): the blocks behind the heads', four tokens each.  The products
+// and the keys come from the same projection and wait for nothing of each other; a launch costs a decode step some 5 us.
+#define HL_STORE_TOKENS 4
+template <bool STORE>
 __global__ __launch_bounds__(256) void head_linear_lines_kernel(
     const bf16_t* __restrict__ x, int x_row, int x_head, const bf16_t* __restrict__ W, bf16_t* __restrict__ out,
     int out_row, int out_head, int Tn, int K, int N, const bf16_t* __restrict__ gate, int gate_row,
-    HeadLinearTail tl, int runs) {
+    HeadLinearTail tl, int runs, int H, const TffLatentStore st) {
     constexpr int RB = 32 * 2 + 16;               // bytes of a wave's staged row
     __shared__ __attribute__((aligned(16))) char staged[4 * 32 * RB];
+    if constexpr (STORE) {
+        if ((int)blockIdx.x >= H) {
+            if (blockIdx.z) return;
+            for (int i = 0; i < HL_STORE_TOKENS; ++i) {
+                const int t = blockIdx.y * 64 + ((int)blockIdx.x - H) * HL_STORE_TOKENS + i;
+                if (t >= Tn) return;
+                const int slot = st.slots[t];
+                if (slot >= 0)                    // (the whole block)
+                    latent_store_token<bf16_t, bf16_t>((const bf16_t*)st.x + (size_t)t * st.x_stride, t, st.rank, st.rot, st.rot_dims, st.pairing,
+                                                       st.norm_w, st.eps, st.rot_dims ? st.cos_sin : nullptr, st.max_pos, st.positions, slot,
+                                                       (bf16_t*)st.k_cache, (bf16_t*)st.v_cache, st.page_size, st.Dp, reinterpret_cast<float*>(staged));
+            }
+            return;
+        }
+    }
     extern __shared__ __attribute__((aligned(1024))) char tiles[];       // the tokens' units, then the run's: 8 KB each
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, kg = lane >> 4;
     const int h = blockIdx.x, tb = blockIdx.y * 64, units = K >> 6;
@@ -485,7 +514,7 @@ __global__ __launch_bounds__(256) void head_linear_lines_kernel(
 TFF_API int tff_head_linear(const void* x, int x_row, int x_head, const void* Wt, void* out, int out_row, int out_head,
                             int T, int H, int K, int N, const void* gate, int gate_row, int tail, int rot_dims,
                             int pairing, int pad_to, const float* cos_sin, int max_pos, const int32_t* positions, int dtype,
-                            tff_stream_t stream) {
+                            const TffLatentStore* store, tff_stream_t stream) {
     TFF_REQUIRE(x && Wt && out, "head_linear: null pointer");
     TFF_REQUIRE(T >= 0 && H > 0 && K > 0 && N > 0 && H <= 65535, "head_linear: bad sizes T=%d H=%d K=%d N=%d", T, H, K, N);
     TFF_REQUIRE(x_head >= K + tail && x_row >= (H - 1) * x_head + K + tail,
@@ -498,9 +527,23 @@ TFF_API int tff_head_linear(const void* x, int x_row, int x_head, const void* Wt
                 "head_linear: %d rotated dimensions of a tail of %d need an even count, a table and positions", rot_dims, tail);
     TFF_REQUIRE(!gate || gate_row >= H * N, "head_linear: gate rows of %d hold fewer than %d", gate_row, H * N);
     if (T == 0) return 0;
+    auto keys_apart = [&]() {
+        return tff_latent_kv_store(store->x, store->x_stride, T, store->rank, store->rot, store->rot_dims, store->pairing, store->norm_w, store->eps,
+                                   store->cos_sin, store->max_pos, store->positions, store->slots, store->k_cache, store->v_cache, store->page_size,
+                                   store->num_pages, store->Dp, nullptr, 0, 0, nullptr, nullptr, 0, store->dtype, store->cache_dtype, stream);
+    };
+    if (store) {        // (checked here as there)
+        TFF_REQUIRE(store->x && store->norm_w && store->positions && store->slots && store->k_cache && store->v_cache, "head_linear: a null pointer among the keys'");
+        TFF_REQUIRE(store->rank > 0 && store->rot >= 0 && store->Dp >= store->rank + store->rot && store->x_stride >= store->rank + store->rot &&
+                    store->rot_dims >= 0 && store->rot_dims <= store->rot && store->rot_dims % 2 == 0 &&
+                    (store->rot_dims == 0 || (store->cos_sin && store->max_pos > 0)) && (store->pairing == 0 || store->pairing == 1) &&
+                    store->page_size > 0 && store->num_pages > 0, "head_linear: bad sizes of the keys");
+    }
     hipStream_t s = (hipStream_t)stream;
     const HeadLinearTail tl{tail, rot_dims, pairing, pad_to, max_pos, cos_sin, positions};
     const dim3 grid((T + HL_TT - 1) / HL_TT, H, (N + 255) / 256);
+    if (store && dtype != TFF_BF16)
+        if (int rc = keys_apart()) return rc;
     if (dtype == TFF_F32)
         head_linear_kernel<float><<<grid, 256, 0, s>>>((const float*)x, x_row, x_head, (const float*)Wt, (float*)out, out_row,
                                                        out_head, T, K, N, (const float*)gate, gate_row, tl);
@@ -520,16 +563,34 @@ TFF_API int tff_head_linear(const void* x, int x_row, int x_head, const void* Wt
 #define TFF_HL(VEC)                                                                                                              \
     head_linear_mfma_kernel<VEC><<<mg, 256, 0, s>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)Wt, (bf16_t*)out, out_row,     \
                                                     out_head, T, K, N, (const bf16_t*)gate, gate_row, tl, runs)
-            if (vec && K % 64 == 0 && K <= 256)
-                head_linear_lines_kernel<<<mg, 256, (unsigned)K * 256u, s>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)Wt, (bf16_t*)out, out_row,
-                                                                           out_head, T, K, N, (const bf16_t*)gate, gate_row, tl, runs);
-            else if (vec) TFF_HL(true);
+#define TFF_HL_LINES(STORE, GRID, KEYS)                                                                                            \
+    head_linear_lines_kernel<STORE><<<GRID, 256, (unsigned)K * 256u, s>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)Wt, (bf16_t*)out, \
+                                                                          out_row, out_head, T, K, N, (const bf16_t*)gate, gate_row, tl, runs, H, KEYS)
+            if (vec && K % 64 == 0 && K <= 256) {
+                if (store && store->dtype == TFF_BF16 && store->cache_dtype == TFF_BF16) {
+                    const int per_tile = (T < 64 ? T : 64), columns = (per_tile + HL_STORE_TOKENS - 1) / HL_STORE_TOKENS;
+                    TFF_HL_LINES(true, dim3(mg.x + columns, mg.y, mg.z), *store);
+                    return tff_check_launch("head_linear");
+                }
+                if (store)
+                    if (int rc = keys_apart()) return rc;
+                TFF_HL_LINES(false, mg, TffLatentStore{});
+                return tff_check_launch("head_linear");
+            }
+#undef TFF_HL_LINES
+            if (store)
+                if (int rc = keys_apart()) return rc;
+            store = nullptr;
+            if (vec) TFF_HL(true);
             else TFF_HL(false);
 #undef TFF_HL
         }
-        else
+        else {
+            if (store)
+                if (int rc = keys_apart()) return rc;
             head_linear_kernel<bf16_t><<<grid, 256, 0, s>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)Wt, (bf16_t*)out,
                                                             out_row, out_head, T, K, N, (const bf16_t*)gate, gate_row, tl);
+        }
     }
     else
         return tff_fail("head_linear: unknown dtype %d", dtype);

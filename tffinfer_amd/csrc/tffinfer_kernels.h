@@ -272,15 +272,27 @@ TFF_API int tff_latent_kv_store(const void* x, int x_stride, int T, int rank, in
                                 int page_size, int num_pages, int Dp, const void* xq, int xq_stride, int q_rank,
                                 const float* q_norm_w, void* q_out, int q_out_stride, int dtype, int cache_dtype,
                                 tff_stream_t stream);
+// What tff_latent_kv_store writes, for tff_head_linear to write it in the same launch.
+typedef struct TffLatentStore {
+    const void* x;
+    int x_stride, rank, rot, rot_dims, pairing;
+    const float* norm_w;
+    float eps;
+    const float* cos_sin;
+    int max_pos;
+    const int32_t *positions, *slots;
+    void *k_cache, *v_cache;
+    int page_size, num_pages, Dp, dtype, cache_dtype;
+} TffLatentStore;
 // Products per head: out[t, h * out_head + n] = sum_k x[t, h * x_head + k] * Wt[h, n, k], Wt [H, N, K].
 // gate (may be null): the result is multiplied by sigmoid(gate[t, h * N + n]).  tail > 0: the
 // `tail` elements of the input head behind the K multiplied ones are copied behind the N results,
 // the first rot_dims of them rotated in pairs (2i, 2i+1) by the token's position; pad_to > N + tail:
-// zeros up to there.
+// zeros up to there.  store (may be null): written too, in the same launch where the product is one of whole pieces.
 TFF_API int tff_head_linear(const void* x, int x_row, int x_head, const void* Wt, void* out, int out_row, int out_head,
                             int T, int H, int K, int N, const void* gate, int gate_row, int tail, int rot_dims,
                             int pairing, int pad_to, const float* cos_sin, int max_pos, const int32_t* positions, int dtype,
-                            tff_stream_t stream);
+                            const TffLatentStore* store, tff_stream_t stream);
 
 // ---- a norm after the residual sum, and the gelu (postnorm.hip) ----
 // v = alpha * resid + delta (delta may be null, or delta_planes partial sums delta_plane apart);

@@ -6,7 +6,7 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
 from .build import ensure_built
 
-ABI_VERSION = 45
+ABI_VERSION = 46
 
 
 class KernelLibraryError(RuntimeError):
@@ -27,6 +27,13 @@ class Recurrence(ctypes.Structure):
                 + [(n, _P) for n in ("cu_tokens", "state_slots", "out")] + [("out_row", _Z)]
                 + [(n, _I) for n in ("kind", "R", "H", "D", "E", "rank", "w_per_head", "sigmoid_gate", "out_dtype")]
                 + [(n, _F) for n in ("inv_tau", "cap", "den_eps", "eps", "q_scale", "out_scale")])
+
+
+class LatentStore(ctypes.Structure):
+    """``TffLatentStore`` of csrc/tffinfer_kernels.h, field by field."""
+    _fields_ = ([("x", _P)] + [(n, _I) for n in ("x_stride", "rank", "rot", "rot_dims", "pairing")] + [("norm_w", _P), ("eps", _F), ("cos_sin", _P),
+                ("max_pos", _I)] + [(n, _P) for n in ("positions", "slots", "k_cache", "v_cache")]
+                + [(n, _I) for n in ("page_size", "num_pages", "Dp", "dtype", "cache_dtype")])
 
 
 #: ``Recurrence.kind``: a decay per key channel; exponential gates per head with a running maximum
@@ -68,7 +75,7 @@ _SIGNATURES = {
     "tff_attention_split_reduce": [_P, _P, _P, _I, _I, _I, _I, _P, _I, _P, _P],
     "tff_latent_kv_store": [_P, _I, _I, _I, _I, _I, _I, _P, _F, _P, _I, _P, _P, _P, _P, _I, _I, _I, _P, _I, _I, _P, _P, _I,
                             _I, _I, _P],
-    "tff_head_linear": [_P, _I, _I, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _I, _I, _P, _I, _P, _I, _P],
+    "tff_head_linear": [_P, _I, _I, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _I, _I, _P, _I, _P, _I, _P, _P],
     "tff_add_dyt": [_P, _P, _I, _Z, _P, _I, _Z, _F, _P, _P, _P, _P, _I, _I, _I, _P],
     "tff_diff_qkv_store": [_P, _Z, _P, _P, _P, _P, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P],
     "tff_diff_combine": [_P, _Z, _I, _P, _Z, _F, _F, _F, _P, _Z, _I, _I, _I, _I, _P],

@@ -1105,14 +1105,15 @@ def padded_head_size(d: int, dtype: torch.dtype) -> int:
 def latent_kv_store(x: torch.Tensor | None, rank: int, rot: int, norm_w: torch.Tensor | None, eps: float,
                     cos_sin: torch.Tensor | None, positions: torch.Tensor, slot_mapping: torch.Tensor,
                     k_cache: torch.Tensor, v_cache: torch.Tensor, pairing: int = 1,
-                    q_latent: torch.Tensor | None = None, q_norm_w: torch.Tensor | None = None) -> torch.Tensor | None:
+                    q_latent: torch.Tensor | None = None, q_norm_w: torch.Tensor | None = None, later: bool = False):
     """Rows x [T, >= rank + rot] (rows may be strided; float32 rows may go to a bfloat16 cache): the RMS norm of
     the first ``rank`` elements times ``norm_w`` and the next ``rot`` elements, rotated by ``cos_sin``
     [max_pos, dims / 2, 2] in pairs (2i, 2i+1) (``pairing`` 1) or (i, i + dims/2) (``pairing`` 0), go to the
     tokens' slots of a cache of one key head of the padded size (keys [pages, 1, page_size, Dp], values
     transposed).  ``q_latent`` [T, q_rank] (rows may be strided, x's type): the queries' latent vectors, whose
     RMS norm times ``q_norm_w`` is returned in the cache's type, from the same launch.  ``x`` None: only
-    that (a layer that reads a cache another layer fills)."""
+    that (a layer that reads a cache another layer fills).  ``later``: nothing is launched; what is returned is for
+    ``head_linear``'s ``store``, which writes the cache in its launch (no ``q_latent`` then)."""
     _req(k_cache, "k cache", ndim=4)
     _req(v_cache, "v cache", k_cache.dtype, 4)
     Dp = k_cache.shape[3]
@@ -1156,6 +1157,13 @@ def latent_kv_store(x: torch.Tensor | None, rank: int, rot: int, norm_w: torch.T
     def row(t):
         return t.stride(0) if T > 1 else t.shape[1]
 
+    if later:
+        if x is None or q_latent is not None:
+            raise _lib.KernelError("latent_kv_store: what is written later are rows for the cache alone")
+        keep = (x, norm_w, cos_sin, positions, slot_mapping, k_cache, v_cache)
+        return keep, _lib.LatentStore(x.data_ptr(), row(x), int(rank), int(rot), dims, int(pairing), norm_w.data_ptr(), float(eps), _ptr(cos_sin), max_pos,
+                                      positions.data_ptr(), slot_mapping.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), k_cache.shape[2],
+                                      k_cache.shape[0], Dp, dtype_code(src.dtype), dtype_code(k_cache.dtype))
     _lib.check(_lib.load().tff_latent_kv_store(
         _ptr(x), row(x) if x is not None else 0, T, int(rank), int(rot), dims, int(pairing), _ptr(norm_w), float(eps),
         _ptr(cos_sin) if x is not None else None, max_pos, _ptr(positions), _ptr(slot_mapping), k_cache.data_ptr(),
@@ -1166,14 +1174,15 @@ def latent_kv_store(x: torch.Tensor | None, rank: int, rot: int, norm_w: torch.T
 
 def head_linear(x: torch.Tensor, x_head: int, weight_t: torch.Tensor, out_head: int | None = None,
                 gate: torch.Tensor | None = None, tail: int = 0, cos_sin: torch.Tensor | None = None,
-                positions: torch.Tensor | None = None, pairing: int = 1) -> torch.Tensor:
+                positions: torch.Tensor | None = None, pairing: int = 1, store=None) -> torch.Tensor:
     """Products per head: x [T, >= H * x_head] (head h starts at h * x_head; rows may be strided),
     ``weight_t`` [H, N, K]: out[t, h, :N] = weight_t[h] x[t, h, :K].  Returns [T, H * out_head]
     (``out_head`` >= N + tail, by default N + tail), zeros behind what is written.
     ``gate`` [T, >= H * N] (rows may be strided): the products are multiplied by its sigmoid.
     ``tail``: so many elements of the input head behind the K are copied behind the products, the
     first ``2 * cos_sin.shape[1]`` of them rotated by the tokens' positions, in pairs (2i, 2i+1)
-    (``pairing`` 1) or (i, i + dims/2) (``pairing`` 0)."""
+    (``pairing`` 1) or (i, i + dims/2) (``pairing`` 0).  ``store``: what ``latent_kv_store(..., later=True)`` returned for
+    as many tokens, written in the same launch where that is possible, else in one before it."""
     if not isinstance(x, torch.Tensor) or not x.is_cuda or x.dim() != 2 or x.stride(1) != 1:
         raise _lib.KernelError("head_linear x: expected a GPU matrix with unit inner stride")
     _req(weight_t, "head_linear weight", x.dtype, 3)
@@ -1198,11 +1207,14 @@ def head_linear(x: torch.Tensor, x_head: int, weight_t: torch.Tensor, out_head: 
         max_pos, dims = cos_sin.shape[0], 2 * cos_sin.shape[1]
         if cos_sin.shape[2] != 2 or dims > tail or positions.numel() != T:
             raise _lib.KernelError(f"head_linear: rotation table {tuple(cos_sin.shape)} or positions do not fit")
+    if store is not None and store[0][0].shape[0] != T:
+        raise _lib.KernelError(f"head_linear: {T} tokens beside the keys of {store[0][0].shape[0]}")
     out = torch.empty(T, H * out_head, dtype=x.dtype, device=x.device)
     _lib.check(_lib.load().tff_head_linear(
         x.data_ptr(), x.stride(0) if T > 1 else x.shape[1], int(x_head), weight_t.data_ptr(), out.data_ptr(),
         H * out_head, out_head, T, H, K, N, _ptr(gate), gate_row, int(tail), dims, int(pairing), out_head if out_head > N else 0,
-        _ptr(cos_sin) if dims else None, max_pos, _ptr(positions) if dims else None, dtype_code(x.dtype), _stream()))
+        _ptr(cos_sin) if dims else None, max_pos, _ptr(positions) if dims else None, dtype_code(x.dtype),
+        None if store is None else ctypes.addressof(store[1]), _stream()))
     return out
 
 

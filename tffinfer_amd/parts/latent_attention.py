@@ -142,6 +142,7 @@ class LatentAttention(Mixer):
         if self.position is not None and self.position.rotary_dim:
             table = self.position.cached_table(ctx.max_positions, x.device)
             pairing = 1 if self.position.pairing == "interleaved" else 0
+        store = None
         if self.q_rank:
             qr = self.q_rank
             proj = ops.linear(x, self.w_in, out_dtype=torch.float32)
@@ -153,12 +154,12 @@ class LatentAttention(Mixer):
             gate = ops.linear(x, self.w_g) if self.has_gate else None
         else:
             proj = ops.linear(x, self.w_in)
-            ops.latent_kv_store(proj[:, nq:nq + rank + rot], rank, rot, self.latent_norm, self.latent_norm_eps, table,
-                                b.positions, kv.slot_mapping, kv.k_cache, kv.v_cache, pairing=pairing)
+            store = ops.latent_kv_store(proj[:, nq:nq + rank + rot], rank, rot, self.latent_norm, self.latent_norm_eps, table,
+                                        b.positions, kv.slot_mapping, kv.k_cache, kv.v_cache, pairing=pairing, later=True)
             q_in = proj[:, :nq]
             gate = proj[:, nq + rank + rot:] if self.has_gate else None
         q = ops.head_linear(q_in, self.head_dim + rot, self.w_uk_t, out_head=Dp, tail=rot, cos_sin=table,
-                            positions=b.positions, pairing=pairing)
+                            positions=b.positions, pairing=pairing, store=store)
         o = ops.paged_attention(q, H, 1, Dp, kv, b, self.window, self.scale, sinks=self.sink)
         o = ops.head_linear(o, Dp, self.w_uv_t, gate=gate)
         return ops.linear(o, self.w_o, out_dtype=torch.float32, partials=True)
