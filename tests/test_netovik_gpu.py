@@ -515,6 +515,23 @@ def test_batches_of_unequal_requests_share_the_attention():
         assert _err(ops.mixed_attention(q, H, G, D, kv, _batch(news, firsts), **dict(args, splits=splits)), want) < 2e-6
 
 
+@pytest.mark.parametrize("n,H,groups,planes,levels", [(1, 256, 1, 1, 2), (3, 1000, 2, 2, 5), (1, 4096, 2, 1, 8), (700, 2048, 2, 4, 3), (600, 4096, 2, 6, 4),
+                                                      (2, 6000, 1, 1, 1)])
+def test_output_norm_with_the_sum_over_depth(n, H, groups, planes, levels):
+    """Every form of the kernel, a group longer than it holds among them: the same bits as the two launches."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(n + H)
+    r = lambda *s: torch.randn(*s, generator=g).to(DEV)       # noqa: E731
+    x, d, w, hist, coef = r(n, H), r(planes, n, H), r(H), r(levels + 1, n, H), r(levels)
+    d = d if planes > 1 else d[0]
+    for out_dtype in (torch.bfloat16, None):
+        x1, x2, h1, h2 = x.clone(), x.clone(), hist.clone(), hist.clone()
+        ops.group_rmsnorm_add(x1, d, w, groups, 1e-5)
+        o1 = ops.depth_average(h1, levels, coef, x1, out_dtype)
+        o2 = ops.group_rmsnorm_add(x2, d, w, groups, 1e-5, out_dtype, depth=(h2, levels, coef))
+        assert torch.equal(x1, x2) and torch.equal(h1, h2) and ((o1 is None and o2 is None) or torch.equal(o1, o2))
+
+
 @pytest.mark.parametrize("E,top", [(8, 3), (2, 2), (5, 1), (70, 4)])
 def test_softmax_router_and_plain_gated_experts(E, top):
     ops = _ops()

@@ -21,11 +21,19 @@
 // the sum over the group.  EARLY: all loads under way first, the same sums in the same order; us without / with: 2 rows of 4096 in one
 // group 8.2 / 5.7, in four with four planes 5.1 / 3.8, 8 rows of 6000 14.1 / 10.4, 400 rows of 8192 24.8 / 16.5, 1,500 rows of 4096 in eight
 // groups 25.0 / 19.9, in two with eight planes 52.6 / 50.1.
-template <typename TO, int GN_ITS, bool EARLY>
+// DEPTH: the new row is a level of the sum over depth, which takes its place in the stream and goes to `out` (tff_depth_average in the same
+// launch): the levels before do not wait for the norm, and the stream is not written and read in between.
+struct GroupDepth {
+    float* hist;
+    const float* coef;
+    size_t level;
+    int n;
+};
+template <typename TO, int GN_ITS, bool EARLY, bool DEPTH>
 __global__ __launch_bounds__(GN_THREADS) void group_rmsnorm_add_kernel(
     float* __restrict__ resid, const float* __restrict__ delta, int planes, size_t plane,
     const int32_t* __restrict__ rows, const float* __restrict__ w, int groups, float eps,
-    TO* __restrict__ out, int H) {
+    TO* __restrict__ out, int H, const GroupDepth dp) {
     __shared__ float red[17];
     const int r = blockIdx.x / groups, g = blockIdx.x % groups, tid = threadIdx.x;
     const int src = rows ? rows[r] : r;
@@ -55,6 +63,23 @@ __global__ __launch_bounds__(GN_THREADS) void group_rmsnorm_add_kernel(
 #pragma unroll
             for (int it = 0; it < GN_ITS; ++it) cache[it] += dl[p * plane + min(tid + it * GN_THREADS, Hg - 1)];
     }
+    float* const hist = DEPTH ? dp.hist + (size_t)r * H + base : nullptr;
+    auto below = [&](int j) {                          // the levels before, in their order
+        float acc = 0.f;
+        for (int l = 0; l + 1 < dp.n; ++l) acc = fmaf(dp.coef[l], hist[l * dp.level + j], acc);
+        return acc;
+    };
+    float acc[DEPTH ? GN_ITS : 1];
+    if constexpr (DEPTH) {
+#pragma unroll
+        for (int it = 0; it < GN_ITS; ++it) acc[it] = 0.f;
+#pragma unroll 2
+        for (int l = 0; l + 1 < dp.n; ++l) {
+            const float c = dp.coef[l];
+#pragma unroll
+            for (int it = 0; it < GN_ITS; ++it) acc[it] = fmaf(c, hist[l * dp.level + min(tid + it * GN_THREADS, Hg - 1)], acc[it]);
+        }
+    }
     float ss = 0.f;
 #pragma unroll
     for (int it = 0; it < GN_ITS; ++it)
@@ -65,10 +90,14 @@ __global__ __launch_bounds__(GN_THREADS) void group_rmsnorm_add_kernel(
     }
     ss = block_sum(ss, red);
     const float rr = 1.0f / sqrtf(ss / (float)Hg + eps);
-    auto emit = [&](int j, float d, float weight, float before) {
+    auto emit = [&](int j, float d, float weight, float before, float levels) {
         float y = d * rr * weight;
         if (x) {
             y += before;
+            if constexpr (DEPTH) {
+                hist[(dp.n - 1) * dp.level + j] = y;
+                y = fmaf(dp.coef[dp.n - 1], y, levels);
+            }
             x[j] = y;
         }
         if (o) o[j] = from_f32<TO>(y);
@@ -76,14 +105,14 @@ __global__ __launch_bounds__(GN_THREADS) void group_rmsnorm_add_kernel(
 #pragma unroll
     for (int it = 0; it < GN_ITS; ++it) {
         const int j = tid + it * GN_THREADS;
-        if (j < Hg) emit(j, cache[it], EARLY ? wr[it] : wg[j], EARLY ? xr[it] : x ? x[j] : 0.f);
+        if (j < Hg) emit(j, cache[it], EARLY ? wr[it] : wg[j], EARLY ? xr[it] : x ? x[j] : 0.f, DEPTH ? acc[it] : 0.f);
     }
-    for (int j = tid + GN_ITS * GN_THREADS; j < Hg; j += GN_THREADS) emit(j, term(j), wg[j], x ? x[j] : 0.f);
+    for (int j = tid + GN_ITS * GN_THREADS; j < Hg; j += GN_THREADS) emit(j, term(j), wg[j], x ? x[j] : 0.f, DEPTH ? below(j) : 0.f);
 }
 
-TFF_API int tff_group_rmsnorm_add(float* resid, const float* delta, int planes, size_t plane, const int32_t* rows,
-                                  const float* w, int groups, float eps, void* out, int n, int H, int out_dtype,
-                                  tff_stream_t stream) {
+template <bool DEPTH>
+static int group_norm_launch(float* resid, const float* delta, int planes, size_t plane, const int32_t* rows, const float* w, int groups,
+                             float eps, void* out, int n, int H, int out_dtype, const GroupDepth dp, tff_stream_t stream) {
     TFF_REQUIRE(delta && w && (resid || out), "group_rmsnorm_add: null pointer");
     TFF_REQUIRE(n >= 0 && H > 0 && groups > 0 && H % groups == 0, "group_rmsnorm_add: rows of %d in %d groups", H, groups);
     TFF_REQUIRE(planes >= 1 && !(rows && (resid || planes > 1)), "group_rmsnorm_add: bad combination of operands");
@@ -96,7 +125,7 @@ TFF_API int tff_group_rmsnorm_add(float* resid, const float* delta, int planes, 
     // planes 31.5 / 35.9, with two 16.7 / 15.1.
     const bool early = (long)n * groups <= 1024 || (Hg <= 8 * GN_THREADS && planes <= 4);
 #define GN_LAUNCH(T, ITS, EARLY) \
-    group_rmsnorm_add_kernel<T, ITS, EARLY><<<n * groups, GN_THREADS, 0, s>>>(resid, delta, planes, plane, rows, w, groups, eps, (T*)out, H)
+    group_rmsnorm_add_kernel<T, ITS, EARLY, DEPTH><<<n * groups, GN_THREADS, 0, s>>>(resid, delta, planes, plane, rows, w, groups, eps, (T*)out, H, dp)
 #define GN_BY_SIZE(T)                                           \
     do {                                                        \
         if (Hg <= GN_THREADS) GN_LAUNCH(T, 1, true);            \
@@ -112,6 +141,18 @@ TFF_API int tff_group_rmsnorm_add(float* resid, const float* delta, int planes, 
 #undef GN_BY_SIZE
 #undef GN_LAUNCH
     return tff_check_launch("group_rmsnorm_add");
+}
+TFF_API int tff_group_rmsnorm_add(float* resid, const float* delta, int planes, size_t plane, const int32_t* rows,
+                                  const float* w, int groups, float eps, void* out, int n, int H, int out_dtype,
+                                  tff_stream_t stream) {
+    return group_norm_launch<false>(resid, delta, planes, plane, rows, w, groups, eps, out, n, H, out_dtype, GroupDepth{}, stream);
+}
+TFF_API int tff_group_rmsnorm_add_depth(float* resid, const float* delta, int planes, size_t plane, const float* w, int groups, float eps,
+                                        float* hist, size_t level, int levels, const float* coef, void* out, int n, int H, int out_dtype,
+                                        tff_stream_t stream) {
+    TFF_REQUIRE(resid && hist && coef && levels >= 1 && level >= (size_t)n * H, "group_rmsnorm_add_depth: %d levels, %zu apart, of %d rows of %d", levels,
+                level, n, H);
+    return group_norm_launch<true>(resid, delta, planes, plane, nullptr, w, groups, eps, out, n, H, out_dtype, GroupDepth{hist, coef, level, levels}, stream);
 }
 
 template <typename TO>

@@ -369,6 +369,10 @@ TFF_API int tff_experts_block(int block, int tiles, int col_blocks);
 TFF_API int tff_group_rmsnorm_add(float* resid, const float* delta, int planes, size_t plane, const int32_t* rows,
                                   const float* w, int groups, float eps, void* out, int n, int H, int out_dtype,
                                   tff_stream_t stream);
+// tff_group_rmsnorm_add with `resid`, then tff_depth_average over `levels` levels, `level` elements apart, in one launch.
+TFF_API int tff_group_rmsnorm_add_depth(float* resid, const float* delta, int planes, size_t plane, const float* w, int groups, float eps,
+                                        float* hist, size_t level, int levels, const float* coef, void* out, int n, int H, int out_dtype,
+                                        tff_stream_t stream);
 // hist [>= n levels, `level` elements apart]: hist[n - 1] <- x; x <- sum_{j < n} coef[j] * hist[j]; out (optional) = x.
 TFF_API int tff_depth_average(float* hist, size_t level, int n, const float* coef, float* x, void* out, size_t count,
                               int out_dtype, tff_stream_t stream);

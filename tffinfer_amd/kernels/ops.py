@@ -1389,12 +1389,13 @@ def routed_experts(h: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_
 
 
 def group_rmsnorm_add(resid: torch.Tensor | None, delta, weight: torch.Tensor, groups: int, eps: float,
-                      out_dtype: torch.dtype | None = None, rows: torch.Tensor | None = None):
+                      out_dtype: torch.dtype | None = None, rows: torch.Tensor | None = None, depth: tuple | None = None):
     """A norm on a sublayer's output: every row of ``delta`` is cut into ``groups`` equal parts, each
     divided by its own root mean square, the whole times ``weight``.  With ``resid`` the result is
     added into the float32 residual stream in place and the new rows are returned in ``out_dtype``
     (None: nothing is returned); without, the normed rows themselves are returned (of the rows
-    ``rows`` only, where given).  ``delta`` may be what ``linear`` returns with ``partials=True``."""
+    ``rows`` only, where given).  ``delta`` may be what ``linear`` returns with ``partials=True``.  ``depth`` = (hist, n,
+    coef), with ``resid``: ``depth_average(hist, n, coef, resid, out_dtype)`` of the sum in the same launch."""
     if isinstance(delta, PendingProduct):
         delta = delta.run()
     if isinstance(delta, ScaledRows):
@@ -1420,6 +1421,18 @@ def group_rmsnorm_add(resid: torch.Tensor | None, delta, weight: torch.Tensor, g
     if resid is None and out_dtype is None:
         out_dtype = torch.float32
     out = torch.empty(n, H, dtype=out_dtype, device=delta.device) if out_dtype is not None else None
+    if depth is not None:
+        hist, levels, coef = depth
+        if resid is None:
+            raise _lib.KernelError("group_rmsnorm_add: a sum over depth is one of the stream")
+        _req(hist, "group_rmsnorm_add hist", torch.float32, 3)
+        _req(coef, "group_rmsnorm_add coef", torch.float32, 1)
+        if tuple(hist.shape[1:]) != (n, H) or not 1 <= levels <= hist.shape[0] or coef.numel() < levels:
+            raise _lib.KernelError(f"group_rmsnorm_add: {levels} levels of {tuple(hist.shape)} for rows {(n, H)}, {coef.numel()} coefficients")
+        _lib.check(_lib.load().tff_group_rmsnorm_add_depth(
+            resid.data_ptr(), delta.data_ptr(), planes, plane, weight.data_ptr(), int(groups), float(eps), hist.data_ptr(), hist.stride(0),
+            int(levels), coef.data_ptr(), _ptr(out), n, H, dtype_code(out_dtype) if out_dtype is not None else 0, _stream()))
+        return out
     _lib.check(_lib.load().tff_group_rmsnorm_add(
         _ptr(resid), delta.data_ptr(), planes, plane, _ptr(rows), weight.data_ptr(), int(groups), float(eps), _ptr(out),
         n, H, dtype_code(out_dtype) if out_dtype is not None else 0, _stream()))

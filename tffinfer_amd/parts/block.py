@@ -178,7 +178,10 @@ class OutputNormBlock(Block):
             h = self._rows(ctx, resid)
         a = self.mixer.forward(ctx, resid if getattr(self.mixer, "reads_stream", False) else h)
         h = self.norm1.forward_add(ctx, resid, a)
-        if self.has_ffn:
+        if self.has_ffn and hist is not None and getattr(self.norm2, "adds_depth", False):
+            h = self.norm2.forward_add(ctx, resid, self.feed_forward.forward(ctx, h), depth=(hist, self.depth + 2, self.dwa))
+            hist = None
+        elif self.has_ffn:
             h = self.norm2.forward_add(ctx, resid, self.feed_forward.forward(ctx, h))
         if hist is not None:
             h = ops.depth_average(hist, self.depth + 2, self.dwa, resid, act)

@@ -84,11 +84,15 @@ class GroupRMSNorm(Norm):
         self.weight = (weights["weight"].to(torch.float32).contiguous().to(device)
                        if "weight" in weights else None)
 
-    def forward_add(self, ctx, resid, delta):
+    #: ``forward_add`` takes the sum over depth that follows
+    adds_depth = True
+
+    def forward_add(self, ctx, resid, delta, depth=None):
         """``resid <- resid + norm(delta)`` in place; returns the new rows in the activation type
-        (the stream itself where that is float32)."""
+        (the stream itself where that is float32).  ``depth`` = (history, levels, coefficients): the sum over
+        depth (``ops.depth_average``) in the same launch."""
         out = ctx.ops.group_rmsnorm_add(resid, delta, self.weight, self.groups, self.eps,
-                                        None if ctx.act_dtype == torch.float32 else ctx.act_dtype)
+                                        None if ctx.act_dtype == torch.float32 else ctx.act_dtype, depth=depth)
         return resid if out is None else out
 
     def forward(self, ctx, resid, delta, rows=None, for_linear=False):
