@@ -404,9 +404,71 @@ __global__ __launch_bounds__(64 * WAVES) void mixed_attention_merge_kernel(const
     }
 }
 
+// The same for the up to MA_MERGE splits of a prompt's tokens: D / 4 lanes a (token, head), 16 bytes a lane and load, several heads a
+// wave and four waves a block.  A wave and block of its own for each head of 1,500 tokens are 48,000 blocks, which are placed no
+// faster than some 50 us, whatever they read.  The values are added in the same order.  us, a block a head / now: 1,500 tokens of
+// 32 heads of 128 57 / 13.
+template <typename TC, int LPH>
+__global__ __launch_bounds__(256) void mixed_attention_merge_vec_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                                        int nsplit, int sink, TC* __restrict__ out, int pairs, int H) {
+    constexpr int D = LPH * 4;
+    const int lane = threadIdx.x & 63, e = (lane % LPH) * 4;
+    const int id = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / LPH) + lane / LPH;
+    if (id >= pairs) return;
+    const int t = id / H, h = id - t * H, HD = H * D;
+    const float* pm = part_ml + (size_t)t * nsplit * 2 * H + h;
+    const float* po = part_o + (size_t)t * nsplit * HD + (size_t)h * D + e;
+    float m[MA_MERGE], l[MA_MERGE];
+    float4 o[MA_MERGE];
+#pragma unroll
+    for (int s = 0; s < MA_MERGE; ++s) {
+        m[s] = -INFINITY;
+        l[s] = 0.f;
+        o[s] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (s < nsplit) {
+            m[s] = pm[(size_t)s * 2 * H];
+            l[s] = pm[(size_t)s * 2 * H + H];
+            o[s] = *reinterpret_cast<const float4*>(po + (size_t)s * HD);
+        }
+    }
+    float M = sink ? 0.f : -INFINITY;
+#pragma unroll
+    for (int s = 0; s < MA_MERGE; ++s) M = fmaxf(M, m[s]);
+    float L = sink ? expf(-M) : 0.f;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int s = 0; s < MA_MERGE; ++s)
+        if (m[s] > -INFINITY) {                          // (a split without visible keys has left no values)
+            const float f = expf(m[s] - M);
+            L = fmaf(l[s], f, L);
+            a.x = fmaf(o[s].x, f, a.x); a.y = fmaf(o[s].y, f, a.y); a.z = fmaf(o[s].z, f, a.z); a.w = fmaf(o[s].w, f, a.w);
+        }
+    const float4 y = L > 0.f ? make_float4(a.x / L, a.y / L, a.z / L, a.w / L) : make_float4(0.f, 0.f, 0.f, 0.f);
+    TC* to = out + (size_t)t * HD + (size_t)h * D + e;
+    if constexpr (sizeof(TC) == 4) {
+        *reinterpret_cast<float4*>(to) = y;
+    } else {
+        union { bf16_t b[4]; uint2 u; } pk;
+        pk.b[0] = (bf16_t)y.x; pk.b[1] = (bf16_t)y.y; pk.b[2] = (bf16_t)y.z; pk.b[3] = (bf16_t)y.w;
+        *reinterpret_cast<uint2*>(to) = pk.u;
+    }
+}
+
 // (a wave does for the splits of a prompt's blocks, eight at most; a step of few tokens has many splits and few blocks)
 template <typename TC>
 static int ma_merge(const float* part_o, const float* part_ml, int splits, int sink, void* out, int T, int H, int D, hipStream_t s) {
+    if (splits <= MA_MERGE && D >= 16 && D <= 256 && (D & (D - 1)) == 0 && ((uintptr_t)part_o % 16) == 0 && ((uintptr_t)out % 16) == 0) {
+        const int pairs = T * H, per = 1024 / D;             // heads a block
+        const unsigned blocks = (unsigned)((pairs + per - 1) / per);
+#define MA_MERGE_VEC(L) mixed_attention_merge_vec_kernel<TC, L><<<blocks, 256, 0, s>>>(part_o, part_ml, splits, sink, (TC*)out, pairs, H)
+        if (D == 16) MA_MERGE_VEC(4);
+        else if (D == 32) MA_MERGE_VEC(8);
+        else if (D == 64) MA_MERGE_VEC(16);
+        else if (D == 128) MA_MERGE_VEC(32);
+        else MA_MERGE_VEC(64);
+#undef MA_MERGE_VEC
+        return tff_check_launch("mixed_attention_merge");
+    }
     if (splits <= MA_MERGE)
         mixed_attention_merge_kernel<TC, 1><<<T * H, 64, 0, s>>>(part_o, part_ml, splits, sink, (TC*)out, H, D);
     else
