@@ -308,6 +308,30 @@ def test_delta_rule_of_a_portion_is_its_own_in_any_step(H, G, D, E, ns):
         assert torch.equal(alone[i], many[i]), (i, n)
 
 
+@pytest.mark.parametrize("H,G,D,E,ns", [(20, 10, 64, 136, [130, 97, 250, 1]), (20, 20, 128, 136, [96, 161, 0, 130]), (60, 30, 64, 20, [100] * 5),
+                                        (34, 17, 128, 32, [99] * 8)])
+def test_delta_rule_in_blocks_of_two_groups_of_channels(H, G, D, E, ns):
+    """More blocks than are resident at once: two groups of value channels a block, the last of which may not exist or end inside.  The
+    bits of each request alone, which takes one group a block; one value that is not finite stays with its request and channel."""
+    ops = _ops()
+    taps, T = 4, sum(ns)
+    assert H * -(-E // 16) * len(ns) > 512 >= H * -(-E // 16)
+    proj, conv, a_log, dt = _delta_case(T, H, G, D, E, taps, D + E + T)
+    proj[ns[0] // 2, 2 * G * D + E + 3] = math.inf              # (the first request, second head)
+    row = H * E * D + (taps - 1) * (2 * G * D + H * E)
+    row += -row % 4
+    dev, many = [x.to(DEV) for x in (conv, a_log, dt)], torch.zeros(len(ns), row, device=DEV)
+    alone = many.normal_(generator=torch.Generator(device=DEV).manual_seed(D)).clone()
+    o = ops.gated_delta(proj.to(DEV), *dev, many, _batch(ns, [0] * len(ns), list(range(len(ns)))), H, G, D, E)
+    for i, n in enumerate(ns):
+        at = sum(ns[:i])
+        if n:
+            one = ops.gated_delta(proj[at:at + n].to(DEV), *dev, alone, _batch([n], [0], [i]), H, G, D, E)
+            assert torch.equal(one.view(torch.int32), o[at:at + n].view(torch.int32)), (i, n)
+            assert bool(torch.isfinite(one).all()) == (i > 0)
+        assert torch.equal(alone[i].view(torch.int32), many[i].view(torch.int32)), (i, n)
+
+
 @pytest.mark.parametrize("H,G,D,E", [(2, 1, 64, 20), (4, 2, 128, 128), (2, 2, 256, 36), (4, 2, 16, 8)])
 def test_delta_rule_of_many_tokens_is_that_of_few(H, G, D, E):
     """More tokens than the preparation takes one by one, in requests too short for the chunks, from states that are not zero:

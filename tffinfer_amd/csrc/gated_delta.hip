@@ -539,32 +539,42 @@ __global__ __launch_bounds__(64) void gdelta_chunk_kernel(const float* __restric
     }
 }
 
-// WV waves of NT tiles of 16 key channels each (D = 16 WV NT).
-template <int NT, int WV>
+// WV waves of NT tiles of 16 key channels each (D = 16 WV NT), NC groups of sixteen value channels.  Two groups a block where one group a
+// block would not be resident at once (two blocks a CU): the groups share a chunk's keys, queries and factors, so that the portions
+// run side by side instead of in two rounds, and each fills the waits of the other's chain.  A chunk then takes long enough for
+// operands that are asked for one chunk ahead (AHEAD + 1 sets of registers).  Four requests of 901, 848, 677 and 664
+// tokens, 32 heads of 128 x 128: 230 us with a group a block, now 196.
+template <int NT, int WV, int NC>
 __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __restrict__ pre, const float* __restrict__ proj, size_t ldp,
                                                           float* __restrict__ state, size_t state_row, size_t tail_off, int taps,
                                                           const int32_t* __restrict__ cu_tokens,
                                                           const int32_t* __restrict__ state_slots, const float* __restrict__ work,
                                                           float* __restrict__ o, int H, int G, int E, int from) {
-    constexpr int D = 16 * WV * NT;
-    __shared__ gd_floatx4 px[2][WV][64], py[2][WV][WV][64];      // parts of K S0 by turns; of Q S0 by turns and chunk
-    const int h = blockIdx.x, r = blockIdx.z, j0 = blockIdx.y * 16;      // (a head's blocks on one XCD: they read the same keys and queries)
+    constexpr int D = 16 * WV * NT, AHEAD = NC == 1 ? 2 : 1;
+    __shared__ gd_floatx4 px[2][NC][WV][64], py[2][NC][WV][WV][64];      // parts of K S0 by turns; of Q S0 by turns and chunk
+    const int h = blockIdx.x, r = blockIdx.z, j0 = blockIdx.y * 16 * NC;      // (a head's blocks on one XCD: they read the same keys and queries)
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
     const int t0 = cu_tokens[r], n = cu_tokens[r + 1] - t0;
     if (n < from) return;                                  // (the whole block: a portion for the token-by-token form)
     const int C = 2 * G * D + H * E, gk = h / (H / G);
     const size_t ldq = (size_t)C + 2 * H;
-    const bool live = j0 + c < E;
-    const int j = min(j0 + c, E - 1);
     float* srow = state + (size_t)state_slots[r] * state_row;
-    float* sp = srow + ((size_t)h * E + j) * D + wv * 16 * NT + 4 * g;
-    gd_floatx4 S[NT];
+    bool live[NC];
+    int j[NC];
+    float* sp[NC];
+    gd_floatx4 S[NC][NT];
 #pragma unroll
-    for (int m = 0; m < NT; ++m) S[m] = *reinterpret_cast<const gd_floatx4*>(sp + 16 * m);
+    for (int w = 0; w < NC; ++w) {
+        live[w] = j0 + 16 * w + c < E;
+        j[w] = min(j0 + 16 * w + c, E - 1);
+        sp[w] = srow + ((size_t)h * E + j[w]) * D + wv * 16 * NT + 4 * g;
+#pragma unroll
+        for (int m = 0; m < NT; ++m) S[w][m] = *reinterpret_cast<const gd_floatx4*>(sp[w] + 16 * m);
+    }
     struct Ops {
         float4 k[NT], q[NT], inv, att, gt, pe;
-        float kt[NT][4], v[4];
-    } x0, x1, x2;
+        float kt[NT][4], v[NC][4];
+    } x[AHEAD + 1];
     // Addresses are a uniform base and a lane's 32-bit offset that is the same for all chunks but the last, whose tokens past the
     // portion's end repeat its last one (their u is zero): with one wave to a SIMD address arithmetic is time.
     const unsigned wstep = (unsigned)H * GD_WORK * 4u, ld = (unsigned)ldq * 4u;
@@ -572,7 +582,9 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
     const char* base = (const char*)(pre + (size_t)t0 * ldq);
     const char* wbase = (const char*)(work + ((size_t)(t0 / 16 + r) * H + h) * GD_WORK);
     const unsigned kcol = (unsigned)((G + gk) * D + wv * 16 * NT) * 4u, qcol = (unsigned)(gk * D + wv * 16 * NT) * 4u;
-    const unsigned vcol = (unsigned)(2 * G * D + h * E + j) * 4u;
+    unsigned vcol[NC];
+#pragma unroll
+    for (int w = 0; w < NC; ++w) vcol[w] = (unsigned)(2 * G * D + h * E + j[w]) * 4u;
     const unsigned in_w = (unsigned)(c * 16 + 4 * g) * 4u, in_g = (unsigned)(4 * g) * 4u;
     auto fetch = [&](int i, Ops& x) {
         const int most = i + 1 < chunks ? 15 : last;
@@ -587,7 +599,8 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const unsigned tr = (unsigned)min(4 * g + q, most) * ld;
-            x.v[q] = *reinterpret_cast<const float*>(b + (tr + vcol));
+#pragma unroll
+            for (int u = 0; u < NC; ++u) x.v[u][q] = *reinterpret_cast<const float*>(b + (tr + vcol[u]));
 #pragma unroll
             for (int m = 0; m < NT; ++m) x.kt[m][q] = *reinterpret_cast<const float*>(b + (tr + kcol + 64u * m + 4u * c));
         }
@@ -596,9 +609,9 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
         x.gt = *reinterpret_cast<const float4*>(w + (in_g + 2048u));
         x.pe = *reinterpret_cast<const float4*>(w + (in_g + 2112u));
     };
-    // a chunk's operands are asked for two chunks ahead: a chunk takes less time than a load from far memory
+    // a chunk's operands are asked for ahead: one group's chunk takes less time than a load from far memory
     int i = 0;
-    float* ocol = o + (size_t)t0 * H * E + (size_t)h * E + j;
+    float* ocol = o + (size_t)t0 * H * E + (size_t)h * E;
     auto meet = [&](const gd_floatx4 (&p)[WV][64]) {       // the waves' parts, added as a tree
         gd_floatx4 v[WV];
 #pragma unroll
@@ -610,69 +623,103 @@ __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __res
         return v[0];
     };
     // The outputs hang off the chain from chunk to chunk: each wave puts one of WV chunks' together once all of them are through.
-    gd_floatx4 own_u = {0.f, 0.f, 0.f, 0.f}, own_gt = own_u;
+    gd_floatx4 own_u[NC], own_gt = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NC; ++w) own_u[w] = own_gt;
     float4 own_att = make_float4(0.f, 0.f, 0.f, 0.f);
     auto outputs = [&](int first) {
         const int mine = first + wv;
         if (mine >= chunks) return;
-        const gd_floatx4 y = gd_mfma16(own_att, own_u) + own_gt * meet(py[first / WV & 1][wv]);
-        float* op = ocol + (size_t)(16 * mine + 4 * g) * H * E;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (live && 16 * mine + 4 * g + q < n) op[(size_t)q * H * E] = y[q];
+        for (int w = 0; w < NC; ++w) {
+            const gd_floatx4 y = gd_mfma16(own_att, own_u[w]) + own_gt * meet(py[first / WV & 1][w][wv]);
+            float* op = ocol + (size_t)(16 * mine + 4 * g) * H * E + j[w];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (live[w] && 16 * mine + 4 * g + q < n) op[(size_t)q * H * E] = y[q];
+        }
     };
     auto chunk = [&](const Ops& now, Ops& ahead) {
-        fetch(min(i + 2, chunks - 1), ahead);      // (past the end the last one again: with a condition the wait for a chunk would be one for all)
+        fetch(min(i + AHEAD, chunks - 1), ahead);      // (past the end the last one again: with a condition the wait for a chunk would be one for all)
         const int buf = i & 1;
-        gd_floatx4 x = gd_mfma16(now.k[0], S[0]), y = gd_mfma16(now.q[0], S[0]);
+        gd_floatx4 xw[NC];
 #pragma unroll
-        for (int m = 1; m < NT; ++m) {
-            x = x + gd_mfma16(now.k[m], S[m]);
-            y = y + gd_mfma16(now.q[m], S[m]);
+        for (int w = 0; w < NC; ++w) {
+            gd_floatx4 x = gd_mfma16(now.k[0], S[w][0]), y = gd_mfma16(now.q[0], S[w][0]);
+#pragma unroll
+            for (int m = 1; m < NT; ++m) {
+                x = x + gd_mfma16(now.k[m], S[w][m]);
+                y = y + gd_mfma16(now.q[m], S[w][m]);
+            }
+            px[buf][w][wv][lane] = x;
+            py[i / WV & 1][w][i % WV][wv][lane] = y;
         }
-        px[buf][wv][lane] = x;
-        py[i / WV & 1][i % WV][wv][lane] = y;
         __syncthreads();          // (the other buffers were last read before this barrier)
-        x = meet(px[buf]);
+#pragma unroll
+        for (int w = 0; w < NC; ++w) xw[w] = meet(px[buf][w]);
         const gd_floatx4 gt = {now.gt.x, now.gt.y, now.gt.z, now.gt.w};
-        gd_floatx4 v = {now.v[0], now.v[1], now.v[2], now.v[3]};
-        v = v - gt * x;
-        const gd_floatx4 u = gd_mfma16(now.inv, v);
         const float gend = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(now.gt.w), 48));      // G_15: the whole chunk's decay
+        gd_floatx4 u[NC];
+#pragma unroll
+        for (int w = 0; w < NC; ++w) {
+            gd_floatx4 v = {now.v[w][0], now.v[w][1], now.v[w][2], now.v[w][3]};
+            v = v - gt * xw[w];
+            u[w] = gd_mfma16(now.inv, v);
+        }
 #pragma unroll
         for (int m = 0; m < NT; ++m) {
             const float4 kt = make_float4(now.kt[m][0] * now.pe.x, now.kt[m][1] * now.pe.y, now.kt[m][2] * now.pe.z, now.kt[m][3] * now.pe.w);
-            const gd_floatx4 add = gd_mfma16(kt, u);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) S[m][e] = fmaf(S[m][e], gend, add[e]);
+            for (int w = 0; w < NC; ++w) {
+                const gd_floatx4 add = gd_mfma16(kt, u[w]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) S[w][m][e] = fmaf(S[w][m][e], gend, add[e]);
+            }
         }
         if (wv == i % WV) {
-            own_u = u;
+#pragma unroll
+            for (int w = 0; w < NC; ++w) own_u[w] = u[w];
             own_gt = gt;
             own_att = now.att;
         }
         if (i % WV == WV - 1) outputs(i - (WV - 1));
         ++i;
     };
-    fetch(0, x0);
-    fetch(min(1, chunks - 1), x1);
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a) fetch(min(a, chunks - 1), x[a]);
     for (;;) {
-        chunk(x0, x2);
-        if (i >= chunks) break;
-        chunk(x1, x0);
-        if (i >= chunks) break;
-        chunk(x2, x1);
+        if constexpr (AHEAD == 2) {
+            chunk(x[0], x[2]);
+            if (i >= chunks) break;
+            chunk(x[1], x[0]);
+            if (i >= chunks) break;
+            chunk(x[2], x[1]);
+        } else {
+            chunk(x[0], x[1]);
+            if (i >= chunks) break;
+            chunk(x[1], x[0]);
+        }
         if (i >= chunks) break;
     }
     if (chunks % WV != 0) outputs(chunks - chunks % WV);
     // Where a u is not finite the zeros above the diagonals do not keep it from earlier tokens (0 x inf is not 0).  It is then in every
     // element of its channel of S for good: such a portion's sixteen channels are worked through once more token by token, from the
     // state that still stands.
-    if (__syncthreads_or(!(fabsf(S[0][0]) < INFINITY))) {
-        gd_portion<D / 16>(pre, t0, n, srow, o, h, gk, H, G, D, E, j0);
-    } else if (live) {
 #pragma unroll
-        for (int m = 0; m < NT; ++m) *reinterpret_cast<gd_floatx4*>(sp + 16 * m) = S[m];
+    for (int w = 0; w < NC; ++w) {
+        // (the block's vote in LDS that is there: two blocks of two groups take a CU's to the last byte)
+        int* vote = reinterpret_cast<int*>(&px[0][0][0][0]);
+        __syncthreads();
+        if (tid == 0) *vote = 0;
+        __syncthreads();
+        if (!(fabsf(S[w][0][0]) < INFINITY)) *vote = 1;
+        __syncthreads();
+        if (*vote) {
+            gd_portion<D / 16>(pre, t0, n, srow, o, h, gk, H, G, D, E, j0 + 16 * w);
+        } else if (live[w]) {
+#pragma unroll
+            for (int m = 0; m < NT; ++m) *reinterpret_cast<gd_floatx4*>(sp[w] + 16 * m) = S[w][m];
+        }
     }
     if (blockIdx.y == 0) gd_keep_inputs(proj, ldp, srow + tail_off, taps, t0, n, h, gk, H, G, D, E);
 }
@@ -705,11 +752,16 @@ TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, si
     hipStream_t s = (hipStream_t)stream;
     gdelta_chunk_kernel<<<dim3(T / 16 + R, H), 64, 0, s>>>(pre, cu_tokens, work, R, H, G, D, E, from);
     if (int rc = tff_check_launch("gdelta_chunk")) return rc;
-    const dim3 grid(H, (E + 15) / 16, R);
-#define GD_SCAN(NT, WV) gdelta_scan_kernel<NT, WV><<<grid, 64 * WV, 0, s>>>(pre, proj, ldp, state, state_row, tail_off, taps, cu_tokens, state_slots, work, o, H, G, E, from)
-    if (D == 64) GD_SCAN(1, 4);
-    else if (D == 128) GD_SCAN(2, 4);
-    else GD_SCAN(4, 4);
+    // (two blocks of four waves a CU are resident at once.  Heads of 256 keep one group: their state alone is eight tiles.)
+    const bool two = D <= 128 && E > 16 && (long)H * ((E + 15) / 16) * R > 512;
+#define GD_SCAN(NT, WV, NC)                                                                                                       \
+    gdelta_scan_kernel<NT, WV, NC><<<dim3(H, (E + 16 * NC - 1) / (16 * NC), R), 64 * WV, 0, s>>>(                                    \
+        pre, proj, ldp, state, state_row, tail_off, taps, cu_tokens, state_slots, work, o, H, G, E, from)
+    if (D == 64 && two) GD_SCAN(1, 4, 2);
+    else if (D == 64) GD_SCAN(1, 4, 1);
+    else if (D == 128 && two) GD_SCAN(2, 4, 2);
+    else if (D == 128) GD_SCAN(2, 4, 1);
+    else GD_SCAN(4, 4, 1);
 #undef GD_SCAN
     return tff_check_launch("gdelta_scan");
 }
