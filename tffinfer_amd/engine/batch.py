@@ -116,7 +116,12 @@ class PinnedTables:
             self._copied[i].synchronize()
             self._copied[i] = None
         if ints > self._bufs[i].numel():
-            self._bufs[i] = torch.empty(max(int(ints), 2 * self._bufs[i].numel()), dtype=torch.int32, pin_memory=True)
+            # (all of them at once: pinning memory is slow, and the next long prompts would each stop for it)
+            for k, ev in enumerate(self._copied):
+                if ev is not None:
+                    ev.synchronize()
+                    self._copied[k] = None
+            self._bufs = list(torch.empty(self.RING, max(int(ints), 2 * self._bufs[i].numel()), dtype=torch.int32, pin_memory=True).unbind(0))
         return self._bufs[i][:ints]
 
     def copied(self) -> None:
