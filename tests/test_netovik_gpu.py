@@ -305,6 +305,43 @@ def test_recurrence_in_chunks_of_sixteen(H, D, portions):
         assert torch.equal(state[slot].cpu().double(), start[slot])
 
 
+def test_mixes_of_many_tokens_in_pieces():
+    """Four tokens a block (1,030 rows of 4,096): requests that begin inside a block, one of a single token, a last block that is not full.
+    The same bits as row by row (a request alone, one token a block)."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(4)
+    W, lengths, starts, slots = 4096, [501, 1, 526, 2], [0, 7, 2, 9], [2, 0, 3, 1]
+    x, mu, state = (torch.randn(*s, generator=g).to(DEV) for s in ((sum(lengths), W), (5, W), (5, 16 + W)))
+    for dtype in (torch.bfloat16, torch.float32):
+        out, at = ops.token_shift_mix(x, state, 16, mu, _batch(lengths, starts, slots), dtype), 0
+        for n, s, slot in zip(lengths, starts, slots):
+            rows = x[at:at + n]
+            one = ops.token_shift_mix(rows.contiguous(), state, 16, mu, _batch([n], [s], [slot]), dtype)
+            assert torch.equal(out[:, at:at + n], one)
+            before = torch.cat((state[slot, 16:][None], rows[:-1])).double()
+            ref = rows.double() + (before - rows.double()) * mu[:, None].double()
+            assert _err(one.float(), ref) < (1e-6 if dtype == torch.float32 else 2.0 ** -8)
+            at += n
+
+
+@pytest.mark.parametrize("T", [1, 37])
+@pytest.mark.parametrize("H,D", [(3, 16), (5, 32), (3, 64), (7, 128), (2, 256)])
+def test_norm_over_each_head_in_pieces(H, D, T):
+    """Heads of a power of two on aligned rows, several a wave, a last wave that is not full; the shared weight and scale of the
+    delta rule's form too.  bfloat16: one rounding, 2^-8 of the largest value."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(H + D)
+    o, gz = 5 * torch.randn(T, H * D, generator=g), 2 * torch.randn(T, H * D + 4, generator=g)
+    w = 1 + 0.3 * torch.randn(H * D, generator=g)
+    unit = plain.unit_rms(o.double().view(T, H, D), 1e-4).reshape(T, H * D) * plain.silu(gz[:, 4:].double())
+    for dtype, tol in ((torch.float32, 2e-6), (torch.bfloat16, 2.0 ** -8)):
+        got = ops.head_norm_gate(o.to(DEV), gz.to(DEV)[:, 4:], w.to(DEV), 1e-4, H, D, dtype)
+        assert _err(got.float(), unit * w.double()) < tol
+        wide = torch.zeros(T, H * D + 8, device=DEV, dtype=dtype)
+        ops.head_norm_silu_gate(o.to(DEV), gz.to(DEV)[:, 4:], w[:D].to(DEV), 1e-4, H, D, wide[:, 8:], 0.7)
+        assert _err(wide[:, 8:].float(), 0.7 * unit * w[:D].double().repeat(H)) < tol and float(wide[:, :8].abs().max()) == 0
+
+
 @pytest.mark.parametrize("H,D", [(3, 8), (2, 40), (1, 128)])
 def test_norm_over_each_head_and_gate(H, D):
     ops = _ops()

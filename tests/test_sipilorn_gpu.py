@@ -439,6 +439,61 @@ def test_norm_over_each_head_and_gates(H, E):
     assert _err(got, 1.3 * ref) < 2e-6 and float(wide[:, H * E:].abs().max()) == 0
 
 
+@pytest.mark.parametrize("T,H,E,P", [(1, 3, 8, 8), (37, 5, 40, 48), (130, 32, 128, 128)])
+def test_gates_of_heads_in_pieces(T, H, E, P):
+    """bfloat16 in pieces of eight: one rounding, 2^-8 of the largest value; what lies beside the heads stays."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(E)
+    a, gz = torch.randn(T, H * P, generator=g).bfloat16().to(DEV), torch.randn(T, H * E + 8, generator=g).bfloat16().to(DEV)
+    wide = torch.zeros(T, H * E + 8, dtype=torch.bfloat16, device=DEV)
+    ops.sigmoid_gate_heads(a, P, gz[:, 8:], H, E, wide[:, :H * E], 1.3)
+    ref = 1.3 * a.double().view(T, H, P)[:, :, :E].reshape(T, H * E) * torch.sigmoid(gz[:, 8:].double())
+    assert float((wide[:, :H * E].double() - ref).abs().max()) < 2.0 ** -8 * float(ref.abs().max()) and float(wide[:, H * E:].abs().max()) == 0
+
+
+@pytest.mark.parametrize("n,W", [(3, 2048), (3, 4100), (140, 1028), (140, 4096)])
+@pytest.mark.parametrize("planes", [(1, 1), (3, 1), (1, 4), (2, 6)])
+def test_two_norms_of_one_sum_in_pieces(n, W, planes):
+    """Aligned rows and rows that begin one number later: the same bits."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(W + n)
+    x, w1, w2, bias = (torch.randn(*s, generator=g).to(DEV) for s in ((n, W), (W,), (W,), (W,)))
+    terms = [torch.randn(p, n, W, generator=g).to(DEV) for p in planes]
+
+    def late(t):
+        return torch.cat((t.new_zeros(1), t.flatten()))[1:].view(t.shape)
+    got = []
+    for move in (lambda t: t.clone(), late):
+        resid = move(x)
+        delta = ops.PendingTerms([move(t) if t.shape[0] > 1 else move(t[0]) for t in terms])
+        got.append(ops.add_rmsnorm_pair(resid, delta, move(bias), move(w1), move(w2), 1e-5, torch.bfloat16) + (resid,))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("D,rot,pairing", [(128, 64, 0), (128, 64, 1), (64, 16, 0), (32, 8, 1), (256, 112, 0)])
+def test_projections_whose_heads_turn_in_part(D, rot, pairing):
+    """From 128 tokens on in pieces of eight elements; against the same tokens in steps of fewer: the sum of squares in another order, one
+    rounding to bfloat16 falls the other way now and then (2^-7 of the largest value), values the same bits."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(D + rot)
+    T, nq, nkv, ps = 137, 5, 2, 16
+    qkv = torch.randn(T, (nq + 2 * nkv) * D, generator=g).bfloat16().to(DEV)
+    qw, kw = ((1 + 0.2 * torch.randn(D, generator=g)).to(DEV) for _ in range(2))
+    table, pos = torch.randn(200, rot // 2, 2, generator=g).to(DEV), _i32(list(range(3, T + 3)))
+    slots = _i32([i + 5 if i != 50 else -1 for i in range(T)])
+    got = []
+    for step in (T, 70):
+        kc = torch.zeros(T // ps + 2, nkv, ps, D, dtype=torch.bfloat16, device=DEV)
+        vc = torch.zeros(T // ps + 2, nkv, D, ps, dtype=torch.bfloat16, device=DEV)
+        x = qkv.clone()
+        for i in range(0, T, step):
+            ops.qk_norm_rope_kv(x[i:i + step], nq, nkv, D, qw, kw, 1e-6, table, pairing, pos[i:i + step], slots[i:i + step], kc, vc)
+        got.append((x[:, :nq * D], kc, vc))
+    for a, b in zip(*got):
+        assert float((a.double() - b.double()).abs().max()) < 2.0 ** -7 * float(b.double().abs().max())
+    assert torch.equal(got[0][2], got[1][2]) and float(got[0][1].abs().sum()) > 0
+
+
 def _ctx(cache, entries, act_dtype, max_positions=1024, cache_id=0):
     from tffinfer_amd.engine.batch import KVView, build_step_batch
     from tffinfer_amd.engine.runner import LayerContext
