@@ -108,3 +108,18 @@ def test_the_experts_blocks_cover_every_tile_and_load_the_xcds_alike(tiles, col_
         for x in range(8):
             own = [i for i in ids[x::8] if i >= 0]
             assert len(own) <= -(-tiles * col_blocks // 8) and own == list(range(own[0], own[0] + len(own)) if own else [])
+
+
+@pytest.mark.parametrize("col_blocks", [1, 3, 16])
+@pytest.mark.parametrize("counts", [[1], [3, 1, 8], [9, 16, 25], [2, 0, 17, 1]])
+def test_an_experts_pairs_lie_together_and_cover_its_tiles(counts, col_blocks):
+    """Pairs in order: an expert after the other, groups of up to eight of its tiles, all column blocks of a group, tiles fastest; the
+    entry of tile id / col_blocks, which the kernels look up, is one of the same expert."""
+    L = _lib()
+    first = 0
+    for n in counts:
+        seen = [divmod(L.tff_experts_place(i, col_blocks, first, n), col_blocks) for i in range(first * col_blocks, (first + n) * col_blocks)]
+        want = [(first + t, c) for g in range(0, n, 8) for c in range(col_blocks) for t in range(g, min(n, g + 8))]
+        assert seen == want
+        assert all(first <= i // col_blocks < first + n for i in range(first * col_blocks, (first + n) * col_blocks))
+        first += n

@@ -463,9 +463,8 @@ __device__ __forceinline__ ex_bf16x8 ex_load8(const bf16_t* p, bool ok) {
 // other, of an expert EX_GROUP tiles at a time, of these all column blocks, tiles fastest: the 32 blocks that an XCD runs at a time are
 // then one or two experts' whole products, whose weight rows come from memory once for the group's tiles and whose pairs' rows meet in L2
 // for the column blocks.  (A column block of all experts after the other, which stood here, shared the weight's rows as well but fetched
-// the pairs' rows once more for every column block, so
-// before / now, us for both products: 32 experts, four a token, 4,096 x 1,536 gated, 2,048 tokens 573 / 560, 4,000 tokens 852 / 817;
-// 2,048 x 1,536, 4,500 tokens 519 / 494; 64 to 150 tokens within 1 %.)
+// the pairs' rows once more for every column block.  us for both products, so / now: 32 experts, four a token, 4,096 x 1,536 gated,
+// 2,048 tokens 573 / 560, 4,000 tokens 852 / 817; 2,048 x 1,536, 4,500 tokens 519 / 494; 64 to 150 tokens within 1 %.)
 // The pair's number in that order, or -1 for a block without one.
 __host__ __device__ __forceinline__ int ex_block(unsigned block, int tiles, int col_blocks) {
     const int all = tiles * col_blocks, share = (all + 7) >> 3, at = (int)(block >> 3), id = (int)(block & 7) * share + at;
@@ -478,6 +477,14 @@ __host__ __device__ __forceinline__ void ex_place(int id, int col_blocks, int4 t
     const int rest = in - group * EX_GROUP * col_blocks, left = t.z - group * EX_GROUP, n = left < EX_GROUP ? left : EX_GROUP;
     col_block = rest / n;
     tile = t.y + group * EX_GROUP + rest - col_block * n;
+}
+// For tests: tile * col_blocks + column block of pair `id` of an expert whose `n` tiles begin at `first`.
+TFF_API int tff_experts_place(int id, int col_blocks, int first, int n) {
+    int4 t;
+    t.x = 0; t.y = first; t.z = n; t.w = 0;
+    int tile, col_block;
+    ex_place(id, col_blocks, t, tile, col_block);
+    return tile * col_blocks + col_block;
 }
 TFF_API int tff_experts_block(int block, int tiles, int col_blocks) { return ex_block((unsigned)block, tiles, col_blocks); }
 

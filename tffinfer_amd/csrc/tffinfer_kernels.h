@@ -359,8 +359,10 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
                                  int ldw_in, int ldw_down, float limit, float act_alpha, float up_offset, int32_t* tile_expert,
                                  int32_t* tile_rows, int32_t* num_tiles, int max_tiles, void* y, float* out,
                                  int weight_input, int identity, tff_stream_t stream);
-// Which of the (column block, tile) pairs, tiles fastest, block `block` of a launch of its products works on; -1: none.
+// Which of the (tile, column block) pairs, in the order of the launch, block `block` of one of its products works on; -1: none.
 TFF_API int tff_experts_block(int block, int tiles, int col_blocks);
+// Tile * col_blocks + column block of pair `id` of an expert whose `n` tiles begin at `first`.
+TFF_API int tff_experts_place(int id, int col_blocks, int first, int n);
 
 // ---- norms on a sublayer's output, sums over the model's depth (group_norm.hip) ----
 // y = delta row (planes added up first; row rows[r] where rows is given) cut into `groups` equal parts, each

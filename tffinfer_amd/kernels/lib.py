@@ -85,6 +85,7 @@ _SIGNATURES = {
     "tff_experts_gate_up": [_P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P, _P, _I, _P],
     "tff_experts_tiles_supported": [_I, _I, _I],
     "tff_experts_block": [_I, _I, _I],
+    "tff_experts_place": [_I, _I, _I, _I],
     "tff_experts_by_tiles": [_P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P, _P, _P, _I, _P, _P, _I, _I, _P],
     "tff_group_rmsnorm_add": [_P, _P, _I, _Z, _P, _P, _I, _F, _P, _I, _I, _I, _P],
     "tff_group_rmsnorm_add_depth": [_P, _P, _I, _Z, _P, _I, _F, _P, _Z, _I, _P, _P, _I, _I, _I, _P],
