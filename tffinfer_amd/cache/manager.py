@@ -296,6 +296,30 @@ class CacheManager:
         """Flat slot (page * page_size + offset) of tokens start .. start+n-1."""
         return self.slot_array(group, req, start, n).tolist()
 
+    #: tokens from which a request's slots are looked up a page at a time: ten calls of numpy, six microseconds however few they are
+    ARRAY_SLOTS = 128
+
+    def slots_of(self, group: int, spans):
+        """The flat slots of the tokens start .. start + n - 1 of every (request, start, n) in ``spans``, one
+        span after the other: a list, or an int32 array where a span is long."""
+        ps = self.page_size
+        tables = self.groups[group].tables
+        parts, some = [], []
+        for req, start, n in spans:
+            if n >= self.ARRAY_SLOTS:
+                parts += [some, self.slot_array(group, req, start, n)]
+                some = []
+                continue
+            table = tables[req]
+            for j in range(start, start + n):
+                page = table[j // ps]
+                if page < 0:
+                    raise RuntimeError(f"request {req!r}: token {j} lies in a page already given back")
+                some.append(page * ps + j % ps)
+        if not parts:
+            return some
+        return np.concatenate([np.asarray(p, dtype=np.int32) for p in parts + [some]])
+
     def slot_array(self, group: int, req, start: int, n: int) -> np.ndarray:
         """:meth:`slot_mapping` as int32, a page at a time: 4.5 ms for 16,384 tokens one by one, now 0.07."""
         ps = self.page_size

@@ -131,6 +131,11 @@ class PinnedTables:
         self._at = (self._at + 1) % self.RING
 
 
+#: tokens of a step from which its per-token tables are formed by numpy, whose calls cost a microsecond or two each
+#: whatever they do: a list is a tenth of a microsecond a token
+ARRAY_TOKENS = 256
+
+
 def build_step_batch(entries, cache, device, pinned: PinnedTables | None = None) -> StepBatch:
     """Packs all tables of a step into one host buffer and sends it with one
     copy.  ``cache`` is the CacheManager; pages for the new tokens must have
@@ -139,32 +144,45 @@ def build_step_batch(entries, cache, device, pinned: PinnedTables | None = None)
     b = StepBatch()
     R = len(entries)
     tok, cu, start, ctxl, slots, rows = [], [0], [], [], [], []
+    T = 0
     for e in entries:
         P = cache.num_tokens(e.req)
         n = len(e.tokens)
         tok.extend(e.tokens)
-        base = cu[-1]
-        rows.extend(base + w for w in e.want)
-        cu.append(base + n)
+        rows.extend([T + w for w in e.want])
+        T += n
+        cu.append(T)
         start.append(P)
         ctxl.append(P + n)
         slots.append(cache.slot(e.req))
-        b.max_new_tokens = max(b.max_new_tokens, n)
-        b.max_context = max(b.max_context, P + n)
-    T = cu[-1]
-    counts = np.diff(np.array(cu, dtype=np.int32))
-    treq = np.repeat(np.arange(R, dtype=np.int32), counts)
-    pos = np.arange(T, dtype=np.int32) + np.repeat(np.array(start, dtype=np.int32) - np.array(cu[:-1], dtype=np.int32), counts)
-    sections = [tok, pos, treq, cu, start, ctxl, slots, rows, np.full(T, -1, dtype=np.int32)]
+        if n > b.max_new_tokens:
+            b.max_new_tokens = n
+        if P + n > b.max_context:
+            b.max_context = P + n
+    if T < ARRAY_TOKENS:
+        treq, pos, none = [], [], [-1] * T
+        for r, P in enumerate(start):
+            n = cu[r + 1] - cu[r]
+            treq.extend([r] * n)
+            pos.extend(range(P, P + n))
+    else:
+        counts = np.diff(np.array(cu, dtype=np.int32))
+        treq = np.repeat(np.arange(R, dtype=np.int32), counts)
+        pos = np.arange(T, dtype=np.int32) + np.repeat(np.array(start, dtype=np.int32) - np.array(cu[:-1], dtype=np.int32), counts)
+        none = np.full(T, -1, dtype=np.int32)
+    sections = [tok, pos, treq, cu, start, ctxl, slots, rows, none]
     group_meta = []
+    spans = [(e.req, P, end - P) for e, P, end in zip(entries, start, ctxl)]
     for gi, g in enumerate(cache.groups):
         tables = [cache.block_table(gi, e.req) for e in entries]
         width = max(1, max((len(t) for t in tables), default=1))
         flat = []
         for t in tables:
-            flat.extend(p if p >= 0 else 0 for p in t)
+            flat.extend(t)
             flat.extend([0] * (width - len(t)))
-        sm = np.concatenate([cache.slot_array(gi, e.req, P, len(e.tokens)) for e, P in zip(entries, start)] or [np.empty(0, dtype=np.int32)])
+        if g.spec.window > 0:       # (pages given back: nothing reads them)
+            flat = np.maximum(np.array(flat, dtype=np.int32), 0) if len(flat) > 100 else [p if p > 0 else 0 for p in flat]
+        sm = cache.slots_of(gi, spans)
         group_meta.append((len(sections), width))
         sections.append(flat)
         sections.append(sm)
