@@ -185,6 +185,28 @@ def test_a_shorter_request_takes_over_a_row():
     assert not np.any(row[1:])                         # nothing of the former tenant is left
 
 
+def test_a_step_that_failed_leaves_no_page_behind_in_a_row():
+    """A step's tables are filled, the step fails and its new page goes back; another request takes that page before
+    the first one reserves again."""
+    cache = CacheManager([(0, True, FULL, None)], 8, 8, 2)
+    t = DecodeTables(cache, 1, 64)
+    for rid in ("a", "b"):
+        cache.add_request(rid)
+        cache.reserve(rid, 8)
+        cache.commit(rid, 8)
+    e = [StepEntry("a", [1], [0])]
+    cache.reserve("a", 1)
+    t.fill(e)
+    check_rows(t, cache, e)
+    first = list(cache.block_table(0, "a"))
+    cache.rollback("a")                                # the step failed
+    cache.reserve("b", 1)
+    cache.reserve("a", 1)
+    assert cache.block_table(0, "a") != first and len(cache.block_table(0, "a")) == len(first)
+    t.fill(e)
+    check_rows(t, cache, e)
+
+
 def test_lives_are_unique():
     cache = CacheManager([(0, True, FULL, None)], 8, 4, 2)
     seen = set()

@@ -58,7 +58,8 @@ class RequestCacheState:
     slot: int
     num_tokens: int = 0
     #: unique to this stay of the request in the cache: a request that is released and added
-    #: again under the same id (preemption, an id used twice) gets another one
+    #: again under the same id (preemption, an id used twice) gets another one, and so does one whose
+    #: table has lost pages at its end
     life: int = 0
 
 
@@ -149,9 +150,9 @@ class CacheManager:
         return self.max_seqs
 
     def life(self, req) -> int:
-        """A number that no other stay of any request in this cache has had.  Whoever keeps
-        a copy of a request's block table keys it on this, never on the request's id alone:
-        the id comes back with other pages after a preemption."""
+        """A number that no other stay of any request in this cache has had, another one once pages were
+        taken back from the table's end (``rollback``).  Whoever keeps a copy of a request's block table keys it on
+        this, never on the request's id alone: the id comes back with other pages after a preemption."""
         return self.requests[req].life
 
     def has_request(self, req) -> bool:
@@ -255,6 +256,10 @@ class CacheManager:
                 g.pool.free(t[whole:])
                 n += len(t[whole:])
                 del t[whole:]
+        if n:
+            # (the next pages in their places may be others: a copy of the table is no longer one that only grew)
+            self._lives += 1
+            st.life = self._lives
         return n
 
     def commit(self, req, n_new: int) -> None:
