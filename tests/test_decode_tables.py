@@ -52,8 +52,9 @@ class TableRunner:
     """Stands where the step function stands: decode-only plans go through the
     tables of their bucket (as ModelRunner._step_graph does) and are checked."""
 
-    def __init__(self, cache, max_seqs, max_len):
+    def __init__(self, cache, max_seqs, max_len, ring=1):
         self.cache = cache
+        self.ring = ring                # tables of a bucket that take turns
         self.buckets = graph_buckets(max_seqs)
         self.tables = {}
         self.max_len = max_len
@@ -65,9 +66,11 @@ class TableRunner:
         if all(p.count == 1 for p in plan):
             entries = [StepEntry(p.request.id, [p.request.tokens[p.start]], [0]) for p in plan]
             bucket = next(b for b in self.buckets if b >= len(entries))
-            t = self.tables.get(bucket)
-            if t is None:
-                t = self.tables[bucket] = DecodeTables(self.cache, bucket, self.max_len)
+            turns = self.tables.get(bucket)
+            if turns is None:
+                turns = self.tables[bucket] = [DecodeTables(self.cache, bucket, self.max_len) for _ in range(self.ring)]
+            t = turns[0]
+            turns.append(turns.pop(0))
             t.fill(entries)
             check_rows(t, self.cache, entries)
             self.graph_steps += 1
@@ -78,12 +81,12 @@ class TableRunner:
         return sampled
 
 
-def drive(seed, specs, num_pages, ps, max_seqs, n_requests):
+def drive(seed, specs, num_pages, ps, max_seqs, n_requests, ring):
     rng = random.Random(seed)
     max_len = 160
     cache = CacheManager([(i, True, s, None) for i, s in enumerate(specs)], ps, num_pages, max_seqs)
     sched = Scheduler(cache, SchedulerOptions(max_seqs, 48, 16), max_len)
-    runner = TableRunner(cache, max_seqs, max_len)
+    runner = TableRunner(cache, max_seqs, max_len, ring)
     pending = [Request(i, [rng.randrange(1, 50) for _ in range(rng.randrange(1, 40))],
                        max_new_tokens=rng.randrange(4, 60), ignore_eos=True) for i in range(n_requests)]
     steps = 0
@@ -101,11 +104,12 @@ def drive(seed, specs, num_pages, ps, max_seqs, n_requests):
     return sched.stats.preemptions, runner.graph_steps
 
 
+@pytest.mark.parametrize("ring", [1, 4])
 @pytest.mark.parametrize("specs", [(FULL,), (FULL, WIN)], ids=["full", "full+window"])
-def test_rows_equal_the_block_tables_through_preemptions(specs):
+def test_rows_equal_the_block_tables_through_preemptions(specs, ring):
     preemptions = graph_steps = 0
     for seed in range(60):
-        p, g = drive(seed, specs, num_pages=14, ps=8, max_seqs=3, n_requests=7)
+        p, g = drive(seed, specs, num_pages=14, ps=8, max_seqs=3, n_requests=7, ring=ring)
         preemptions += p
         graph_steps += g
     assert preemptions > 50 and graph_steps > 1000     # the schedules do preempt and do decode

@@ -106,28 +106,37 @@ class PinnedTables:
     RING = 4
 
     def __init__(self, ints: int = 1 << 16):
-        self._bufs = list(torch.empty(self.RING, int(ints), dtype=torch.int32, pin_memory=True).unbind(0))
-        self._copied: list = [None] * self.RING
+        self.bufs = self._pin(int(ints))
+        self._copied = [torch.cuda.Event() for _ in range(self.RING)]
+        self._under_way = [False] * self.RING
         self._at = 0
 
-    def take(self, ints: int) -> torch.Tensor:
+    def _pin(self, ints: int) -> list:
+        return list(torch.zeros(self.RING, ints, dtype=torch.int32, pin_memory=True).unbind(0))
+
+    def turn(self) -> int:
+        """Which of ``bufs`` the next step writes; the copy out of it is done."""
         i = self._at
-        if self._copied[i] is not None:
+        if self._under_way[i]:
             self._copied[i].synchronize()
-            self._copied[i] = None
-        if ints > self._bufs[i].numel():
+            self._under_way[i] = False
+        return i
+
+    def take(self, ints: int) -> torch.Tensor:
+        i = self.turn()
+        if ints > self.bufs[i].numel():
             # (all of them at once: pinning memory is slow, and the next long prompts would each stop for it)
             for k, ev in enumerate(self._copied):
-                if ev is not None:
+                if self._under_way[k]:
                     ev.synchronize()
-                    self._copied[k] = None
-            self._bufs = list(torch.empty(self.RING, max(int(ints), 2 * self._bufs[i].numel()), dtype=torch.int32, pin_memory=True).unbind(0))
-        return self._bufs[i][:ints]
+                    self._under_way[k] = False
+            self.bufs = self._pin(max(int(ints), 2 * self.bufs[i].numel()))
+        return self.bufs[i][:ints]
 
     def copied(self) -> None:
         """To be called right after the copy to the device was queued."""
-        self._copied[self._at] = torch.cuda.Event()
         self._copied[self._at].record()
+        self._under_way[self._at] = True
         self._at = (self._at + 1) % self.RING
 
 

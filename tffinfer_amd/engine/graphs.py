@@ -206,10 +206,12 @@ class DecodeGraph:
         widths = [-(-runner.max_model_len // cache.page_size) for _ in cache.groups]
         _, total = table_layout(B, widths, [max_key_runs(B, g.spec.num_kv_heads) for g in cache.groups],
                                 [w for _, _, w in pool_table_widths(cache, runner.max_model_len)])
-        self.tables = DecodeTables(cache, B, runner.max_model_len)
-        # The tables leave through pinned buffers that go round: a copy runs when the device reaches its step, and the host, which
-        # writes into `tables` only, waits for a buffer's copy no sooner than some steps later.
+        # The tables leave through pinned buffers that go round, so that the host waits for a step's copy no sooner than some
+        # steps later.  Each buffer is a set of tables of its own, which a step brings up to date: it writes what has changed
+        # since the buffer's last turn (64 rows of 40,960 tokens are 655 KB, which no step copies on the host).
         self._pinned = PinnedTables(total)
+        self._turns = [DecodeTables(cache, B, runner.max_model_len, buf.numpy()) for buf in self._pinned.bufs]
+        self.tables, self._host = self._turns[0], self._pinned.bufs[0]       # those of the last step
         self.widths = self.tables.widths
         self.offs = o = self.tables.offs
         self.dev = torch.zeros(total, dtype=torch.int32, device=runner.device)
@@ -255,6 +257,8 @@ class DecodeGraph:
         return next(iter(self._variants.values())) if self._variants else []
 
     def fill(self, entries) -> None:
+        i = self._pinned.turn()
+        self.tables, self._host = self._turns[i], self._pinned.bufs[i]
         self.tables.fill(entries)
 
     def possible_variants(self) -> list:
@@ -364,9 +368,7 @@ class DecodeGraph:
         if variant not in self._variants:
             self.capture(variant)
         pieces = self._variants[variant]
-        host = self._pinned.take(self.tables.total)
-        host.numpy()[:] = self.tables.hv
-        self.dev.copy_(host, non_blocking=True)
+        self.dev.copy_(self._host, non_blocking=True)
         self._pinned.copied()
         R = len(entries)
         if token_source is not None:
