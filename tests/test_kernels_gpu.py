@@ -76,6 +76,24 @@ def test_add_rmsnorm(H, out_dtype):
            1e-6 if out_dtype == torch.float32 else 8e-3, "norm without delta")
 
 
+@pytest.mark.parametrize("H", [8, 100, 1024, 1028, 4096, 5120, 15996, 16000, 16004])
+def test_rmsnorm_row_has_the_same_bits_in_any_step(H):
+    """The norm of float32 rows alone: against 64 bits, and the same bits of a row among however many others, also where
+    the weight's address does not allow 16-byte pieces (the general kernel's order of sums)."""
+    from tffinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(H)
+    x, w, eps = torch.randn(300, H, generator=g), 1 + 0.1 * torch.randn(H, generator=g), 1e-6
+    ref = x.double() * torch.rsqrt(x.double().square().mean(1, keepdim=True) + eps) * w.double()
+    xd, wd = x.to(DEV), w.to(DEV)
+    shifted = torch.empty(H + 1, device=DEV)
+    shifted[1:] = wd
+    whole = ops.rmsnorm(xd, wd, eps)
+    _close(whole, ref, 1e-6)
+    for n in (1, 127, 128, 129, 300):
+        assert torch.equal(ops.rmsnorm(xd[:n], wd, eps), whole[:n]), n
+        assert torch.equal(ops.rmsnorm(xd[:n], shifted[1:], eps), whole[:n]), n
+
+
 def test_rmsnorm_eps_position():
     """eps is added to the mean inside the root: a row of tiny values tells it
     from eps added to the sum or outside the root."""
