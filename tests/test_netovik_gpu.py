@@ -2,6 +2,7 @@
 the level of its op, then whole models through the step function (whole prompts, decoding
 token by token, portions down to two tokens, mixed batches on a pool whose pages and slots are
 used again), and greedy generation through the engine's own entry point and scheduler."""
+import math
 import types
 
 import pytest
@@ -478,6 +479,59 @@ def test_attention_on_the_matrix_cores_at_the_tiles_edges(H, G, D, page):
                 at += n
             err = _err(torch.cat(outs, 0), ref)
             assert err < 3e-2, (T, window, keep, cuts[:2], err)      # (bfloat16 queries, keys, weights and results, as above)
+
+
+def _queries_keys_values(H, G, D, T, seed):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(T, n, D, generator=g).to(torch.bfloat16) for n in (H, G, G)]
+
+
+def _filled_cache(k, v, page, seed=0):
+    """A cache of one request that holds keys and values [T, G, D]."""
+    T, G, D = k.shape
+    cache = _Cache(G, D, page, [T], k.dtype, seed=seed)
+    at = torch.tensor([cache.tables[0][j // page] for j in range(T)]), torch.arange(T) % page
+    cache.k[at[0].to(DEV), :, at[1].to(DEV)] = k.to(DEV)
+    cache.v[at[0].to(DEV), :, :, at[1].to(DEV)] = v.to(DEV)
+    return cache
+
+
+def _softmax_of_values(scores, v, rep, sink):
+    """scores [H, T] of one query in 64 bits, v [T, G, D]: the weighted values, without the keys of weight zero."""
+    m = torch.clamp(scores.max(1, keepdim=True).values, min=0.0 if sink else -math.inf)
+    p = torch.exp(scores - torch.where(m > -math.inf, m, 0.0))
+    total = p.sum(1, keepdim=True) + (torch.exp(-m) if sink else 0.0)
+    p = torch.where(total > 0, p / total, 0.0)
+    out = torch.zeros(scores.shape[0], v.shape[2], dtype=torch.float64)
+    for h in range(scores.shape[0]):
+        keep = p[h] > 0
+        out[h] = (p[h, keep, None] * v[keep, h // rep].double()).sum(0)
+    return out
+
+
+@pytest.mark.parametrize("splits", [1, 3, None])
+@pytest.mark.parametrize("H,G,D,page", [(8, 4, 32, 16), (32, 8, 128, 16), (12, 12, 64, 8), (16, 16, 128, 16), (32, 32, 64, 16)])
+def test_infinite_values_of_single_tokens(H, G, D, page, splits):
+    """A key whose values are infinite in some elements gives these elements their infinity and leaves the others alone, also where its
+    weight is one exactly; a NaN stays a NaN; keys that the token does not see reach nothing."""
+    ops = _ops()
+    rep, inf = H // G, math.inf
+    for T, at in ((1, 0), (20, 7), (100, 99), (161, 31)):
+        q, k, v = _queries_keys_values(H, G, D, T + 1, T + H)
+        v[at, :, 3], v[at, :, 10], v[at, 0, 17], v[T, :, 20] = inf, -inf, math.nan, inf
+        if at > 5:
+            v[at - 3, :, 5], v[at - 3, :, 10] = -inf, -inf
+        cache = _filled_cache(k, v, page)
+        kv = cache.view([0], [T - 1], [1])
+        out = ops.mixed_attention(q[T - 1:T].reshape(1, H * D).to(DEV), H, G, D, kv, _batch([1], [T - 1]), scale=0.5 / D ** 0.5, splits=splits)
+        scores = torch.einsum("hd,thd->ht", q[T - 1].double(), k[:T].double().repeat_interleave(rep, 1)) * (0.5 / D ** 0.5)
+        ref = _softmax_of_values(scores, v[:T], rep, False)
+        got = out.double().cpu().view(H, D)
+        for what in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(what(got), what(ref)), (T, what.__name__)
+        fine = torch.isfinite(ref)
+        assert fine.sum() > 0.8 * H * D
+        assert float((got - ref)[fine].abs().max()) < 3e-2 * float(ref[fine].abs().max())
 
 
 @pytest.mark.parametrize("decode", [False, True])

@@ -530,6 +530,13 @@ __device__ __forceinline__ ma_bf16x8 ma_visible(ma_bf16x8 v, int j, int lo, int 
     return v;
 }
 
+// Eight values with those that are not finite as zero.
+__device__ __forceinline__ ma_bf16x8 ma_finite(ma_bf16x8 v) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = fabsf((float)v[i]) < INFINITY ? v[i] : (bf16_t)0.f;
+    return v;
+}
+
 #define Q16_THREADS 512
 #define Q16_WAVES 8
 #define Q16_TK 64        // keys a tile
@@ -875,6 +882,7 @@ __global__ __launch_bounds__(Q16_THREADS) void mixed_attention_few_kernel(
     __shared__ __attribute__((aligned(16))) float s_s[32 * SROW];
     __shared__ __attribute__((aligned(16))) bf16_t p_s[3][32 * FEW_TK];
     __shared__ float m_s[32], l_s[32], c_s[32];
+    __shared__ int again;
     const int t = blockIdx.x, split = blockIdx.y, nsplit = gridDim.y;
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, g4 = lane >> 4;
     const int pos = positions[t], rep = H / G, HD = H * D;
@@ -884,10 +892,6 @@ __global__ __launch_bounds__(Q16_THREADS) void mixed_attention_few_kernel(
     const MaTiles<FEW_TK> tiles(pos, window, keep_first);
     const int i_lo = nsplit == 1 ? 0 : split * tiles_per_split;
     const int i_hi = split == nsplit - 1 ? tiles.n : min(tiles.n, i_lo + tiles_per_split);      // (the last split takes what is left)
-    if (tid < 32) {
-        m_s[tid] = own_sink ? 0.f : -INFINITY;
-        l_s[tid] = own_sink ? 1.f : 0.f;
-    }
     for (int i = tid; i < (32 - H) * SROW; i += Q16_THREADS) s_s[H * SROW + i] = 0.f;      // rows of no head
     const size_t page_elems = (size_t)G * D * page_size;
     float mixf[8];
@@ -899,150 +903,170 @@ __global__ __launch_bounds__(Q16_THREADS) void mixed_attention_few_kernel(
         }
     }
     ma_floatx4 oacc[GPW][EB];
-#pragma unroll
-    for (int gg = 0; gg < GPW; ++gg)
-#pragma unroll
-        for (int eb = 0; eb < EB; ++eb) oacc[gg][eb] = ma_floatx4{0.f, 0.f, 0.f, 0.f};
     const ma_bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-    __syncthreads();
-    for (int ti = i_lo; ti < i_hi; ++ti) {
-        const bool first = ti < tiles.n_a;
-        const int jt = first ? ti * FEW_TK : tiles.jt_b + (ti - tiles.n_a) * FEW_TK;
-        const int r_lo = first ? 0 : tiles.lo, r_hi = first ? tiles.a_hi : tiles.hi;
-        // the lane's places: keys jt + col and jt + 16 + col for the scores, jt + g4 * 8 and the seven after it for the values
-        // (no page is looked up for keys the token does not see)
-        const int j8 = jt + g4 * 8;
-        const bool live = j8 < r_hi && j8 + 8 > r_lo;
-        const size_t vbase = live ? (size_t)table[j8 / page_size] * page_elems + j8 % page_size + (size_t)col * page_size : 0;
-        size_t kbase[2];
-        bool kon[2];
-#pragma unroll
-        for (int k2 = 0; k2 < 2; ++k2) {
-            const int j = jt + k2 * 16 + col;
-            kon[k2] = j >= r_lo && j < r_hi;
-            kbase[k2] = kon[k2] ? (size_t)table[j / page_size] * page_elems + (size_t)(j % page_size) * D + g4 * 8 : 0;
+    if (tid == 0) again = 0;
+    // finite_only: the weights' second and third terms meet values that are not finite as zero (below)
+    for (bool finite_only = false;; finite_only = true) {
+        if (tid < 32) {
+            m_s[tid] = own_sink ? 0.f : -INFINITY;
+            l_s[tid] = own_sink ? 1.f : 0.f;
         }
-        ma_bf16x8 vb[GPW == 1 ? EB : 1];
-#pragma unroll 1
-        for (int gg = 0; gg < GPW; ++gg) {
-            const int kvh = wv + gg * Q16_WAVES;
-            if (kvh < G) {
-                ma_bf16x8 kf[2][KC], qf[KC];
-                const int h = kvh * rep + col;
 #pragma unroll
-                for (int k2 = 0; k2 < 2; ++k2)
+        for (int gg = 0; gg < GPW; ++gg)
 #pragma unroll
-                    for (int kc = 0; kc < KC; ++kc)
-                        kf[k2][kc] = kon[k2] ? *reinterpret_cast<const ma_bf16x8*>(k_cache + kbase[k2] + (size_t)kvh * page_size * D + kc * 32) : zero;
-#pragma unroll
-                for (int kc = 0; kc < KC; ++kc)
-                    qf[kc] = col < rep ? *reinterpret_cast<const ma_bf16x8*>(q + (size_t)t * HD + (size_t)h * D + kc * 32 + g4 * 8) : zero;
-                float bf[2][4];
-#pragma unroll
-                for (int k2 = 0; k2 < 2; ++k2)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        bf[k2][i] = bias && col < rep ? bias[(size_t)min(max(pos - (jt + k2 * 16 + g4 * 4 + i), 0), bias_rows - 1) * H + h] : 0.f;
-                if (GPW == 1) {
-#pragma unroll
-                    for (int e = 0; e < (GPW == 1 ? EB : 1); ++e)
-                        vb[e] = live ? *reinterpret_cast<const ma_bf16x8*>(v_cache + vbase + ((size_t)kvh * D + e * 16) * page_size) : zero;
-                }
-#pragma unroll
-                for (int k2 = 0; k2 < 2; ++k2) {
-                    ma_floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int kc = 0; kc < KC; ++kc) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[k2][kc], qf[kc], acc, 0, 0, 0);
-                    if (col < rep) {                          // (keys g4 * 4 + i, head col)
-                        float sc[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            sc[i] = acc[i] * scale;
-                            if (cap > 0.f) sc[i] = cap * ma_tanh(sc[i] * inv_cap);
-                            sc[i] += bf[k2][i];
-                        }
-                        *reinterpret_cast<float4*>(s_s + h * SROW + k2 * 16 + g4 * 4) = make_float4(sc[0], sc[1], sc[2], sc[3]);
-                    }
-                }
-            }
-        }
+            for (int eb = 0; eb < EB; ++eb) oacc[gg][eb] = ma_floatx4{0.f, 0.f, 0.f, 0.f};
         __syncthreads();
-        if (wv < 2 && wv * 16 < H) {                          // sixteen mixed heads a wave: lane (quarter g4, col) has wv * 16 + g4 * 4 + i of keys col, 16 + col
-            ma_floatx4 sm[2];
-            bool vis[2];
+        for (int ti = i_lo; ti < i_hi; ++ti) {
+            const bool first = ti < tiles.n_a;
+            const int jt = first ? ti * FEW_TK : tiles.jt_b + (ti - tiles.n_a) * FEW_TK;
+            const int r_lo = first ? 0 : tiles.lo, r_hi = first ? tiles.a_hi : tiles.hi;
+            // the lane's places: keys jt + col and jt + 16 + col for the scores, jt + g4 * 8 and the seven after it for the values
+            // (no page is looked up for keys the token does not see)
+            const int j8 = jt + g4 * 8;
+            const bool live = j8 < r_hi && j8 + 8 > r_lo;
+            const size_t vbase = live ? (size_t)table[j8 / page_size] * page_elems + j8 % page_size + (size_t)col * page_size : 0;
+            size_t kbase[2];
+            bool kon[2];
 #pragma unroll
             for (int k2 = 0; k2 < 2; ++k2) {
                 const int j = jt + k2 * 16 + col;
-                vis[k2] = j >= r_lo && j < r_hi;
-                sm[k2] = ma_floatx4{0.f, 0.f, 0.f, 0.f};
-                if (mix) {
+                kon[k2] = j >= r_lo && j < r_hi;
+                kbase[k2] = kon[k2] ? (size_t)table[j / page_size] * page_elems + (size_t)(j % page_size) * D + g4 * 8 : 0;
+            }
+            ma_bf16x8 vb[GPW == 1 ? EB : 1];
+#pragma unroll 1
+            for (int gg = 0; gg < GPW; ++gg) {
+                const int kvh = wv + gg * Q16_WAVES;
+                if (kvh < G) {
+                    ma_bf16x8 kf[2][KC], qf[KC];
+                    const int h = kvh * rep + col;
 #pragma unroll
-                    for (int ks = 0; ks < 8; ++ks)
-                        sm[k2] = __builtin_amdgcn_mfma_f32_16x16x4f32(mixf[ks], s_s[(ks * 4 + g4) * SROW + k2 * 16 + col], sm[k2], 0, 0, 0);
-                } else {
+                    for (int k2 = 0; k2 < 2; ++k2)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) sm[k2][i] = s_s[(wv * 16 + g4 * 4 + i) * SROW + k2 * 16 + col];
+                        for (int kc = 0; kc < KC; ++kc)
+                            kf[k2][kc] = kon[k2] ? *reinterpret_cast<const ma_bf16x8*>(k_cache + kbase[k2] + (size_t)kvh * page_size * D + kc * 32) : zero;
+#pragma unroll
+                    for (int kc = 0; kc < KC; ++kc)
+                        qf[kc] = col < rep ? *reinterpret_cast<const ma_bf16x8*>(q + (size_t)t * HD + (size_t)h * D + kc * 32 + g4 * 8) : zero;
+                    float bf[2][4];
+#pragma unroll
+                    for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            bf[k2][i] = bias && col < rep ? bias[(size_t)min(max(pos - (jt + k2 * 16 + g4 * 4 + i), 0), bias_rows - 1) * H + h] : 0.f;
+                    if (GPW == 1) {
+#pragma unroll
+                        for (int e = 0; e < (GPW == 1 ? EB : 1); ++e)
+                            vb[e] = live ? *reinterpret_cast<const ma_bf16x8*>(v_cache + vbase + ((size_t)kvh * D + e * 16) * page_size) : zero;
+                    }
+#pragma unroll
+                    for (int k2 = 0; k2 < 2; ++k2) {
+                        ma_floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int kc = 0; kc < KC; ++kc) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[k2][kc], qf[kc], acc, 0, 0, 0);
+                        if (col < rep) {                          // (keys g4 * 4 + i, head col)
+                            float sc[4];
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                sc[i] = acc[i] * scale;
+                                if (cap > 0.f) sc[i] = cap * ma_tanh(sc[i] * inv_cap);
+                                sc[i] += bf[k2][i];
+                            }
+                            *reinterpret_cast<float4*>(s_s + h * SROW + k2 * 16 + g4 * 4) = make_float4(sc[0], sc[1], sc[2], sc[3]);
+                        }
+                    }
                 }
             }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int h = wv * 16 + g4 * 4 + i;
-                const float m_old = m_s[h];
-                float mx = m_old;
-#pragma unroll
-                for (int k2 = 0; k2 < 2; ++k2)
-                    if (vis[k2]) mx = fmaxf(mx, sm[k2][i]);
-                mx = row16_max(mx);
-                const float corr = mx > -INFINITY ? expf(m_old - mx) : 1.f;
-                float sum = 0.f;
+            __syncthreads();
+            if (wv < 2 && wv * 16 < H) {                          // sixteen mixed heads a wave: lane (quarter g4, col) has wv * 16 + g4 * 4 + i of keys col, 16 + col
+                ma_floatx4 sm[2];
+                bool vis[2];
 #pragma unroll
                 for (int k2 = 0; k2 < 2; ++k2) {
-                    const float p = vis[k2] ? ma_exp(sm[k2][i] - mx) : 0.f;
-                    sum += p;
-                    const bf16_t p1 = (bf16_t)p;
-                    const float r1 = p - (float)p1;
-                    const bf16_t p2 = (bf16_t)r1;
-                    const int at = h * FEW_TK + k2 * 16 + col;
-                    p_s[0][at] = p1;
-                    p_s[1][at] = p2;
-                    p_s[2][at] = (bf16_t)(r1 - (float)p2);
+                    const int j = jt + k2 * 16 + col;
+                    vis[k2] = j >= r_lo && j < r_hi;
+                    sm[k2] = ma_floatx4{0.f, 0.f, 0.f, 0.f};
+                    if (mix) {
+#pragma unroll
+                        for (int ks = 0; ks < 8; ++ks)
+                            sm[k2] = __builtin_amdgcn_mfma_f32_16x16x4f32(mixf[ks], s_s[(ks * 4 + g4) * SROW + k2 * 16 + col], sm[k2], 0, 0, 0);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) sm[k2][i] = s_s[(wv * 16 + g4 * 4 + i) * SROW + k2 * 16 + col];
+                    }
                 }
-                sum = row16_sum(sum);
-                if (col == 0) {
-                    m_s[h] = mx;
-                    l_s[h] = l_s[h] * corr + sum;
-                    c_s[h] = corr;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int h = wv * 16 + g4 * 4 + i;
+                    const float m_old = m_s[h];
+                    float mx = m_old;
+#pragma unroll
+                    for (int k2 = 0; k2 < 2; ++k2)
+                        if (vis[k2]) mx = fmaxf(mx, sm[k2][i]);
+                    mx = row16_max(mx);
+                    const float corr = mx > -INFINITY ? expf(m_old - mx) : 1.f;
+                    float sum = 0.f;
+#pragma unroll
+                    for (int k2 = 0; k2 < 2; ++k2) {
+                        const float p = vis[k2] ? ma_exp(sm[k2][i] - mx) : 0.f;
+                        sum += p;
+                        const bf16_t p1 = (bf16_t)p;
+                        const float r1 = p - (float)p1;
+                        const bf16_t p2 = (bf16_t)r1;
+                        const int at = h * FEW_TK + k2 * 16 + col;
+                        p_s[0][at] = p1;
+                        p_s[1][at] = p2;
+                        p_s[2][at] = (bf16_t)(r1 - (float)p2);
+                    }
+                    sum = row16_sum(sum);
+                    if (col == 0) {
+                        m_s[h] = mx;
+                        l_s[h] = l_s[h] * corr + sum;
+                        c_s[h] = corr;
+                    }
                 }
             }
+            __syncthreads();
+#pragma unroll
+            for (int gg = 0; gg < GPW; ++gg) {
+                const int kvh = wv + gg * Q16_WAVES;
+                if (kvh < G) {
+                    ma_bf16x8 pa[3];
+#pragma unroll
+                    for (int s = 0; s < 3; ++s)
+                        pa[s] = col < rep ? *reinterpret_cast<const ma_bf16x8*>(&p_s[s][(kvh * rep + col) * FEW_TK + g4 * 8]) : zero;
+                    float cr[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) cr[i] = g4 * 4 + i < rep ? c_s[kvh * rep + g4 * 4 + i] : 1.f;
+#pragma unroll
+                    for (int e = 0; e < EB; ++e) {
+                        ma_bf16x8 v = GPW == 1 ? vb[GPW == 1 ? e : 0]
+                                               : (live ? *reinterpret_cast<const ma_bf16x8*>(v_cache + vbase + ((size_t)kvh * D + e * 16) * page_size) : zero);
+                        v = ma_visible(v, j8, r_lo, r_hi);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) oacc[gg][e][i] *= cr[i];
+                        const ma_bf16x8 vf = finite_only ? ma_finite(v) : v;
+#pragma unroll
+                        for (int s = 2; s >= 0; --s) oacc[gg][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[s], s ? vf : v, oacc[gg][e], 0, 0, 0);
+                    }
+                }
+            }
+            // (the next tile's scores go to s_s, which nobody reads any more; its first barrier stands between these reads of
+            // p_s and c_s and their next writes)
         }
+        // A term of zero or of the other sign makes NaN of an infinite value, whose product with the whole weight is infinite.  Values
+        // are seldom infinite, so that is looked for in the results, and the block's keys are then worked through once more.
+        float sum = 0.f;
+#pragma unroll
+        for (int gg = 0; gg < GPW; ++gg)
+#pragma unroll
+            for (int eb = 0; eb < EB; ++eb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sum = fmaf(0.f, oacc[gg][eb][i], sum);
+        if (sum != 0.f) again = 1;
         __syncthreads();
-#pragma unroll
-        for (int gg = 0; gg < GPW; ++gg) {
-            const int kvh = wv + gg * Q16_WAVES;
-            if (kvh < G) {
-                ma_bf16x8 pa[3];
-#pragma unroll
-                for (int s = 0; s < 3; ++s)
-                    pa[s] = col < rep ? *reinterpret_cast<const ma_bf16x8*>(&p_s[s][(kvh * rep + col) * FEW_TK + g4 * 8]) : zero;
-                float cr[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) cr[i] = g4 * 4 + i < rep ? c_s[kvh * rep + g4 * 4 + i] : 1.f;
-#pragma unroll
-                for (int e = 0; e < EB; ++e) {
-                    ma_bf16x8 v = GPW == 1 ? vb[GPW == 1 ? e : 0]
-                                           : (live ? *reinterpret_cast<const ma_bf16x8*>(v_cache + vbase + ((size_t)kvh * D + e * 16) * page_size) : zero);
-                    v = ma_visible(v, j8, r_lo, r_hi);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) oacc[gg][e][i] *= cr[i];
-#pragma unroll
-                    for (int s = 2; s >= 0; --s) oacc[gg][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[s], v, oacc[gg][e], 0, 0, 0);
-                }
-            }
-        }
-        // (the next tile's scores go to s_s, which nobody reads any more; its first barrier stands between these reads of
-        // p_s and c_s and their next writes)
+        if (!again || finite_only) break;
     }
-    __syncthreads();
 #pragma unroll
     for (int gg = 0; gg < GPW; ++gg) {
         const int kvh = wv + gg * Q16_WAVES;
