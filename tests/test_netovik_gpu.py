@@ -534,6 +534,30 @@ def test_infinite_values_of_single_tokens(H, G, D, page, splits):
         assert float((got - ref)[fine].abs().max()) < 3e-2 * float(ref[fine].abs().max())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("low", [-math.inf, torch.finfo(torch.float32).min])
+def test_biases_that_shut_keys_out_of_single_tokens(low, dtype):
+    """A bias of minus infinity, or of the lowest number there is, for distances from 40 on: whole tiles of visible keys without a weight
+    of their own, before keys that have one, in one block and in splits of their own; or no weight at all."""
+    ops = _ops()
+    H, G, D, page = 8, 4, 32, 16
+    bias = torch.zeros(60, H)
+    bias[40:] = low
+    bias[:, 5] = low                             # (head 5: for all distances)
+    for T in (30, 100, 300):
+        q, k, v = (t.to(dtype) for t in _queries_keys_values(H, G, D, T, T))
+        cache = _filled_cache(k, v, page)
+        kv = cache.view([0], [T - 1], [1])
+        scores = torch.einsum("hd,thd->ht", q[T - 1].float(), k.float().repeat_interleave(H // G, 1)) * 0.1
+        scores = (scores + bias[(T - 1 - torch.arange(T)).clamp(max=59)].T).double()      # (sums as float32 has them)
+        for sink in (False, True):
+            ref = _softmax_of_values(scores, v, H // G, sink)
+            for splits in (1, 3, None):
+                out = ops.mixed_attention(q[T - 1:T].reshape(1, H * D).to(DEV), H, G, D, kv, _batch([1], [T - 1]), scale=0.1, bias=bias.to(DEV),
+                                          sink=sink, splits=splits).double().cpu().view(H, D)
+                assert float((out - ref).abs().max()) < (3e-2 if dtype == torch.bfloat16 else 2e-5) * float(ref.abs().max()), (T, sink, splits)
+
+
 @pytest.mark.parametrize("decode", [False, True])
 @pytest.mark.parametrize("edge", ["inside", "outside", "kept", "not_kept"])
 def test_a_loud_key_at_the_windows_and_the_kept_tokens_edges(edge, decode):

@@ -1005,10 +1005,11 @@ __global__ __launch_bounds__(Q16_THREADS) void mixed_attention_few_kernel(
                         if (vis[k2]) mx = fmaxf(mx, sm[k2][i]);
                     mx = row16_max(mx);
                     const float corr = mx > -INFINITY ? expf(m_old - mx) : 1.f;
+                    const float from = mx > -INFINITY ? mx : 0.f;      // (no key has a weight yet: weights of zero)
                     float sum = 0.f;
 #pragma unroll
                     for (int k2 = 0; k2 < 2; ++k2) {
-                        const float p = vis[k2] ? ma_exp(sm[k2][i] - mx) : 0.f;
+                        const float p = vis[k2] ? ma_exp(sm[k2][i] - from) : 0.f;
                         sum += p;
                         const bf16_t p1 = (bf16_t)p;
                         const float r1 = p - (float)p1;
