@@ -558,6 +558,47 @@ def test_biases_that_shut_keys_out_of_single_tokens(low, dtype):
                 assert float((out - ref).abs().max()) < (3e-2 if dtype == torch.bfloat16 else 2e-5) * float(ref.abs().max()), (T, sink, splits)
 
 
+@pytest.mark.parametrize("low", [-math.inf, torch.finfo(torch.float32).min, -1e37])
+def test_biases_that_shut_keys_out_of_prompts(low):
+    """The same for prompts of 64 tokens and more: tiles in which all that a query sees has the lowest score there is, before the tiles
+    that count; head 5 sees nothing else, and the keys count alike (minus infinity: nothing)."""
+    ops = _ops()
+    H, G, D, page, T = 8, 4, 32, 16, 300
+    bias = torch.zeros(60, H)
+    bias[40:] = low
+    bias[:, 5] = low
+    q, k, v = _queries_keys_values(H, G, D, T, T)
+    cache = _filled_cache(k, v, page)
+    kv = cache.view([0], [0], [T])
+    raw = torch.einsum("ihd,thd->iht", q.float(), k.float().repeat_interleave(H // G, 1)) * 0.1
+    for sink in (False, True):
+        out = ops.mixed_attention(q.reshape(T, H * D).to(DEV), H, G, D, kv, _batch([T], [0]), scale=0.1, bias=bias.to(DEV), sink=sink)
+        got = out.double().cpu().view(T, H, D)
+        for i in (0, 15, 16, 39, 40, 63, 64, 103, 104, 128, 200, 299):
+            scores = (raw[i, :, :i + 1] + bias[(i - torch.arange(i + 1)).clamp(max=59)].T).double()
+            ref = _softmax_of_values(scores, v[:i + 1], H // G, sink)
+            assert float((got[i] - ref).abs().max()) < 3e-2 * float(ref.abs().max()), (i, sink)
+
+
+@pytest.mark.parametrize("loudest", [0.0, 30.7, 100.3, 255.1, 700.1])
+def test_a_prompt_whose_maximum_stays_gives_all_keys_alike(loudest):
+    """Keys that all score the same, over 128 tiles without a window: a weight of one each, so the sums are whole numbers and exact,
+    and values of +1 in the first half and of -1 in the second leave (first - second) / keys.  A factor that is not quite one where the
+    maximum stays would take from the first tiles at every later one."""
+    ops = _ops()
+    H, G, D, page, T = 8, 8, 32, 16, 8192
+    q, k = torch.zeros(T, H, D, dtype=torch.bfloat16), torch.ones(T, G, D, dtype=torch.bfloat16)
+    v = torch.ones(T, G, D, dtype=torch.bfloat16)
+    v[T // 2:] = -1
+    cache = _filled_cache(k, v, page)
+    kv = cache.view([0], [0], [T])
+    bias = torch.full((1, H), loudest, device=DEV)
+    out = ops.mixed_attention(q.reshape(T, H * D).to(DEV), H, G, D, kv, _batch([T], [0]), scale=1.0, bias=bias).float().cpu().view(T, H * D)
+    sums = v[:, 0, 0].double().cumsum(0) / torch.arange(1, T + 1)
+    # (the quotient's rounding and that to bfloat16; where the sum is zero nothing at all)
+    assert bool(((out.double() - sums[:, None]).abs() <= sums.abs()[:, None] * 2 ** -8).all())
+
+
 @pytest.mark.parametrize("decode", [False, True])
 @pytest.mark.parametrize("edge", ["inside", "outside", "kept", "not_kept"])
 def test_a_loud_key_at_the_windows_and_the_kept_tokens_edges(edge, decode):

@@ -748,18 +748,20 @@ __global__ __launch_bounds__(Q16_THREADS) void mixed_attention_q16_kernel(
                     for (int i = 0; i < 4; ++i) {
                         Q16_IN_TURN;
                         const float mx = row16_max(ma_max(ma_max(ma_max(sm[0][hb][i], sm[1][hb][i]), ma_max(sm[2][hb][i], sm[3][hb][i])), m_old[i]));
-                        const float m2 = mx > -INFINITY ? mx * LOG2E : 0.f;      // (nothing visible yet: weights of zero)
+                        // (nothing visible yet: weights of zero.  Differences are what is scaled: a maximum of its own scaled would be
+                        // rounded, so that results kept from tile to tile drift, and the lowest number there is would overflow)
+                        const float from = mx > -INFINITY ? mx : 0.f;
                         union { bf16_t h[4]; uint2 u; } p;
                         float sum = 0.f;
 #pragma unroll
                         for (int kb = 0; kb < 4; ++kb) {
                             // (the sum takes the weights as the product will see them)
-                            p.h[kb] = (bf16_t)__builtin_amdgcn_exp2f(fmaf(sm[kb][hb][i], LOG2E, -m2));
+                            p.h[kb] = (bf16_t)__builtin_amdgcn_exp2f((sm[kb][hb][i] - from) * LOG2E);
                             sum += (float)p.h[kb];
                         }
                         *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(s_s + qq * HP * Q16_TK) + (h0 + i) * Q16_TK
                                                   + Q16_PIECE(col >> 1, qq) * 8 + (col & 1) * 4) = p.u;
-                        const float corr = __builtin_amdgcn_exp2f(fmaf(m_old[i], LOG2E, -m2));
+                        const float corr = __builtin_amdgcn_exp2f((m_old[i] - from) * LOG2E);
                         m_new[i] = mx;
                         l[i] = fmaf(l[i], corr, row16_sum(sum));
                         if (col == 0) c_s[(h0 + i) * 16 + qq] = corr;
