@@ -80,6 +80,25 @@ def test_wkv_dispatch_keeps_to_the_rule(monkeypatch, longest, chunks):
     assert called == ["tff_wkv_recurrence_chunks" if chunks else "tff_wkv_recurrence"]
 
 
+@pytest.mark.parametrize("lengths,heads,dim,groups", [
+    ([901], 32, 128, 1), ([901] + [1] * 63, 32, 128, 1), ([1] * 30 + [95, 500], 32, 128, 1), ([901, 400, 400], 32, 128, 1), ([2000] + [200] * 5, 32, 128, 1),
+    ([901, 848, 677, 664], 32, 128, 2), ([500] * 6, 32, 128, 2), ([901, 848, 677, 664], 16, 128, 1), ([200] * 16, 16, 128, 2), ([200] * 16, 8, 128, 2),
+    ([901, 848, 677, 664], 32, 64, 1), ([500] * 6, 32, 64, 2), ([901] * 8, 64, 128, 2), ([901], 200, 128, 2), ([901] * 6, 32, 256, 1)])
+def test_the_delta_rules_scan_takes_two_groups_where_portions_would_wait(lengths, heads, dim, groups):
+    """Not by the number of requests: those that decode, and portions that are through before a longer one, keep no block waiting."""
+    from tffinfer_amd.kernels import ops
+    cu = [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    batch = types.SimpleNamespace(num_reqs=len(lengths), host_cu_tokens=cu)
+    assert ops.gdelta_scan_groups(batch, heads, dim, dim, 512) == groups
+    assert ops.gdelta_scan_groups(batch, heads, dim, 16, 512) == 1
+
+
+def test_portions_start_in_turn_where_blocks_run():
+    from tffinfer_amd.kernels.ops import _through
+    assert _through([], 8, 16) == 0 and _through([5], 8, 16) == 5 and _through([5, 9], 8, 16) == 9
+    assert _through([5, 9, 3], 8, 16) == 9 and _through([5, 9, 7], 8, 16) == 12 and _through([4, 4], 32, 16) == 16
+
+
 def test_the_draw_forms_maxima_only_where_they_bound_something(monkeypatch):
     """A top_k over half the number of a row's runs (or 256) does not ask for them, nor does a small vocabulary; one row that
     profits is enough."""

@@ -539,11 +539,11 @@ __global__ __launch_bounds__(64) void gdelta_chunk_kernel(const float* __restric
     }
 }
 
-// WV waves of NT tiles of 16 key channels each (D = 16 WV NT), NC groups of sixteen value channels.  Two groups a block where one group a
-// block would not be resident at once (two blocks a CU): the groups share a chunk's keys, queries and factors, so that the portions
-// run side by side instead of in two rounds, and each fills the waits of the other's chain.  A chunk then takes long enough for
-// operands that are asked for one chunk ahead (AHEAD + 1 sets of registers).  Four requests of 901, 848, 677 and 664
-// tokens, 32 heads of 128 x 128: 230 us with a group a block, now 196.
+// WV waves of NT tiles of 16 key channels each (D = 16 WV NT), NC groups of sixteen value channels.  Two groups a block where portions would
+// wait for others' blocks (two blocks a CU are resident): the groups share a chunk's keys, queries and factors, so that the portions
+// run side by side instead of in two rounds, and each fills the waits of the other's chain.  A chunk then takes 1.45 times as long, and
+// its operands are asked for one chunk ahead (AHEAD + 1 sets of registers).  Four requests of 901, 848, 677 and 664
+// tokens, 32 heads of 128 x 128, the recurrence with its preparation: 278 us with a group a block, with two 245; a single portion of 901 116 and 159.
 template <int NT, int WV, int NC>
 __global__ __launch_bounds__(64 * WV) void gdelta_scan_kernel(const float* __restrict__ pre, const float* __restrict__ proj, size_t ldp,
                                                           float* __restrict__ state, size_t state_row, size_t tail_off, int taps,
@@ -733,12 +733,14 @@ TFF_API int tff_gdelta_chunks_supported(int R, int H, int G, int D, int E, size_
            (E + 15) / 16 <= 65535 && row * 17 * sizeof(float) < ((size_t)1 << 32);
 }
 
-// As tff_gdelta_recurrence, in chunks, for the portions of `from` tokens and more.  Every row's first 2 G D + H E + 2 H channels of pre are
+// As tff_gdelta_recurrence, in chunks, for the portions of `from` tokens and more.  groups: of sixteen value channels a block of the scan, 1,
+// or 2 with heads of up to 128 (those of 256 keep one group: their state alone is eight tiles).  Every row's first 2 G D + H E + 2 H channels of pre are
 // a multiple of four long, and pre, state and work are 16-byte aligned.
 TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
                                          size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* work,
-                                         float* o, int T, int R, int H, int G, int D, int E, int from, tff_stream_t stream) {
+                                         float* o, int T, int R, int H, int G, int D, int E, int from, int groups, tff_stream_t stream) {
     TFF_REQUIRE(pre && proj && state && cu_tokens && state_slots && work && o, "gdelta_chunks: null pointer");
+    TFF_REQUIRE(groups == 1 || (groups == 2 && D <= 128), "gdelta_chunks: %d groups of value channels a block, heads of %d", groups, D);
     TFF_REQUIRE(R >= 0 && H > 0 && G > 0 && H % G == 0 && E > 0 && taps >= 1 && taps <= GD_MAX_TAPS && T >= 0 && from > 0,
                 "gdelta_chunks: bad sizes heads=%d kv_heads=%d vdim=%d taps=%d", H, G, E, taps);
     const size_t C = 2 * (size_t)G * D + (size_t)H * E;
@@ -752,14 +754,12 @@ TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, si
     hipStream_t s = (hipStream_t)stream;
     gdelta_chunk_kernel<<<dim3(T / 16 + R, H), 64, 0, s>>>(pre, cu_tokens, work, R, H, G, D, E, from);
     if (int rc = tff_check_launch("gdelta_chunk")) return rc;
-    // (two blocks of four waves a CU are resident at once.  Heads of 256 keep one group: their state alone is eight tiles.)
-    const bool two = D <= 128 && E > 16 && (long)H * ((E + 15) / 16) * R > 512;
 #define GD_SCAN(NT, WV, NC)                                                                                                       \
     gdelta_scan_kernel<NT, WV, NC><<<dim3(H, (E + 16 * NC - 1) / (16 * NC), R), 64 * WV, 0, s>>>(                                    \
         pre, proj, ldp, state, state_row, tail_off, taps, cu_tokens, state_slots, work, o, H, G, E, from)
-    if (D == 64 && two) GD_SCAN(1, 4, 2);
+    if (D == 64 && groups == 2) GD_SCAN(1, 4, 2);
     else if (D == 64) GD_SCAN(1, 4, 1);
-    else if (D == 128 && two) GD_SCAN(2, 4, 2);
+    else if (D == 128 && groups == 2) GD_SCAN(2, 4, 2);
     else if (D == 128) GD_SCAN(2, 4, 1);
     else GD_SCAN(4, 4, 1);
 #undef GD_SCAN

@@ -430,12 +430,13 @@ TFF_API int tff_gdelta_recurrence(const float* pre, const float* proj, size_t ld
                                   int R, int H, int G, int D, int E, int max_tokens, int below, tff_stream_t stream);
 // The same for the portions of `from` tokens and more, in chunks of sixteen tokens on the float32 matrix cores: head sizes of
 // 64, 128 and 256, what tff_gdelta_chunks_supported says; work: tff_gdelta_chunks_workspace_bytes.  A token's result depends on where its portion
-// began, beyond rounding it does not.
+// began, beyond rounding it does not.  groups: of sixteen value channels that a block of the scan takes, 1, or 2 with heads of up to 128: the
+// same bits, fewer and longer blocks.
 TFF_API size_t tff_gdelta_chunks_workspace_bytes(int T, int R, int H);
 TFF_API int tff_gdelta_chunks_supported(int R, int H, int G, int D, int E, size_t state_row);
 TFF_API int tff_gdelta_recurrence_chunks(const float* pre, const float* proj, size_t ldp, float* state, size_t state_row,
                                          size_t tail_off, int taps, const int32_t* cu_tokens, const int32_t* state_slots, float* work,
-                                         float* o, int T, int R, int H, int G, int D, int E, int from, tff_stream_t stream);
+                                         float* o, int T, int R, int H, int G, int D, int E, int from, int groups, tff_stream_t stream);
 
 // out[t * out_row + h * E + e] = o[t, h, e] / sqrt(mean over e of o^2 + eps) * w[e] * silu(g[t * g_row + h * E + e]) * scale
 TFF_API int tff_head_norm_silu_gate(const float* o, const float* g, size_t g_row, const float* w, float eps, float scale,

@@ -13,6 +13,7 @@ with a device dispatch; here the table has one entry per op and no dispatch.
 from __future__ import annotations
 
 import ctypes
+import heapq
 import math
 
 import numpy as np
@@ -2150,6 +2151,32 @@ def _rows2(t: torch.Tensor, name: str, dtype, cols: int):
 GDELTA_CHUNKS_MIN_TOKENS = 96
 
 
+def _through(lengths: list, blocks: int, places: int) -> float:
+    """When portions of so many tokens, ``blocks`` blocks each, are through that start in turn wherever ``places`` blocks run at a time."""
+    lanes = places // blocks
+    if lanes == 0:
+        return sum(lengths) * blocks / places
+    if len(lengths) <= lanes:
+        return max(lengths, default=0)
+    free = [0] * lanes
+    for n in lengths:
+        heapq.heapreplace(free, free[0] + n)
+    return max(free)
+
+
+def gdelta_scan_groups(batch, H: int, D: int, E: int, places: int) -> int:
+    """Groups of sixteen value channels a block of the delta rule's scan: two where that brings the step's portions through sooner than one,
+    of which ``places`` blocks run at a time.  A chunk of two groups takes 1.45 times as long as one's, so only portions that would wait
+    for their turn gain; requests that decode have no blocks that stay.  us with one / two groups, 32 heads of 128 x 128: portions of 901,
+    848, 677 and 664 tokens 278 / 245, six of 500 274 / 253, one of 901 beside eight that decode 125 / 169, 901 and two of 400 157 / 192,
+    2,000 and five of 200 281 / 365."""
+    if D > 128 or E <= 16:
+        return 1
+    cu = getattr(batch, "host_cu_tokens", None)
+    ns = [GDELTA_CHUNKS_MIN_TOKENS] * batch.num_reqs if cu is None else [b - a for a, b in zip(cu, cu[1:]) if b - a >= GDELTA_CHUNKS_MIN_TOKENS]
+    return 2 if _through(ns, H * -(-E // 16), places) > 1.45 * _through(ns, H * -(-E // 32), places) else 1
+
+
 def gated_delta(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
                 state: torch.Tensor, batch, H: int, G: int, D: int, E: int) -> torch.Tensor:
     """The gated delta rule over the step's tokens.  ``proj`` float32 [T, >= C + 2 H]: the projections q [G, D],
@@ -2190,7 +2217,7 @@ def gated_delta(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, d
         _lib.check(L.tff_gdelta_recurrence_chunks(
             pre.data_ptr(), proj.data_ptr(), ldp, state.data_ptr(), row, tail, taps, batch.cu_tokens.data_ptr(),
             batch.state_slots.data_ptr(), work.data_ptr(), o.data_ptr(), T, batch.num_reqs, H, G, D, E,
-            GDELTA_CHUNKS_MIN_TOKENS, stream))
+            GDELTA_CHUNKS_MIN_TOKENS, gdelta_scan_groups(batch, H, D, E, 2 * _num_cus(proj.device)), stream))
         below = GDELTA_CHUNKS_MIN_TOKENS
         longest = _longest_below(batch, below)
         if longest == 0:
