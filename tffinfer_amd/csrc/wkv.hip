@@ -45,7 +45,8 @@ __global__ __launch_bounds__(256) void token_shift_mix_kernel(
 
 // The same, four columns a thread and TT tokens a block: a plane's row of mu is fetched for TT tokens, a token's row serves the next
 // one as its predecessor, and every row of the block is asked for before the first is used.  us, a column a
-// thread and a token a block / now: 2,900 tokens of 4,096 into five planes 48 / 28 (5.9 TB/s), 1,500 tokens 27 / 16, one token 2.7 / 2.9.
+// thread and a token a block / this: 2,900 tokens of 4,096 into five planes 47 / 28 (5.9 TB/s), 1,000 tokens 20 / 15.5, 128 tokens
+// 4.1 / 3.7; 16 tokens and one 2.7 / 2.9, which stay with the kernel above.
 template <typename TO, int TT>
 __global__ __launch_bounds__(256) void token_shift_mix_vec_kernel(
     const float* __restrict__ x, const float* __restrict__ state, size_t state_row, size_t prev_off,
@@ -89,7 +90,8 @@ TFF_API int tff_token_shift_mix(const float* x, const float* state, size_t state
     TFF_REQUIRE(T >= 0 && W > 0 && M > 0 && prev_off + (size_t)W <= state_row, "token_shift_mix: bad sizes");
     if (T == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
-    if (W % 4 == 0 && state_row % 4 == 0 && prev_off % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)state % 16) == 0 && ((uintptr_t)mu % 16) == 0 &&
+    // (up to 2^18 elements, 64 rows of 4,096, more blocks with fewer bytes each are through a little sooner)
+    if ((long)T * W >= (1L << 18) && W % 4 == 0 && state_row % 4 == 0 && prev_off % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)state % 16) == 0 && ((uintptr_t)mu % 16) == 0 &&
         ((uintptr_t)out % 16) == 0 && (out_dtype == TFF_F32 || out_dtype == TFF_BF16)) {
         // four tokens a block where that still leaves a few blocks a CU
         const int cols = (W + 1023) / 1024;
