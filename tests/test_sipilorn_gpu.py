@@ -440,7 +440,7 @@ def test_norm_over_each_head_and_gates(H, E):
     assert _err(got, 1.3 * ref) < 2e-6 and float(wide[:, H * E:].abs().max()) == 0
 
 
-@pytest.mark.parametrize("T,H,E,P", [(1, 3, 8, 8), (37, 5, 40, 48), (130, 32, 128, 128)])
+@pytest.mark.parametrize("T,H,E,P", [(1, 3, 8, 8), (37, 5, 40, 48), (130, 32, 128, 128), (1311, 5, 40, 48), (10923, 3, 8, 8)])
 def test_gates_of_heads_in_pieces(T, H, E, P):
     """bfloat16 in pieces of eight: one rounding, 2^-8 of the largest value; what lies beside the heads stays."""
     ops = _ops()

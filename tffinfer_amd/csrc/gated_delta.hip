@@ -819,8 +819,8 @@ __global__ __launch_bounds__(256) void sigmoid_gate_heads_kernel(const T* __rest
     out[t * out_row + c] = from_f32<T>(to_f32(o[t * o_row + (size_t)h * o_head + e]) * (scale / (1.0f + expf(-gz))));
 }
 
-// bfloat16, eight elements of a head a thread: 16-byte accesses.  us, an element a thread / now: 2,900 tokens of
-// 32 heads of 128 32 / 16, one token 2.2 / 2.4.
+// bfloat16, eight elements of a head a thread: 16-byte accesses.  us, an element a thread / this: 2,900 tokens of
+// 32 heads of 128 30 / 15, 128 tokens 3.3 / 2.8; 48 tokens 2.5 / 2.6 and one 2.3 / 2.5, which stay with the kernel above.
 __global__ __launch_bounds__(256) void sigmoid_gate_heads_vec_kernel(const bf16_t* __restrict__ o, size_t o_row, int o_head,
                                                                      const bf16_t* __restrict__ g, size_t g_row, float scale,
                                                                      bf16_t* __restrict__ out, size_t out_row, int HE, int E, size_t eighths) {
@@ -844,7 +844,8 @@ TFF_API int tff_sigmoid_gate_heads(const void* o, size_t o_row, int o_head, cons
     if (T == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     const size_t count = (size_t)T * H * E;
-    if (dtype == TFF_BF16 && E % 8 == 0 && o_row % 8 == 0 && o_head % 8 == 0 && g_row % 8 == 0 && out_row % 8 == 0 && ((uintptr_t)o % 16) == 0 &&
+    // (up to 2^18 elements, 64 rows of 4,096, more blocks with fewer bytes each are through a little sooner)
+    if (dtype == TFF_BF16 && count >= ((size_t)1 << 18) && E % 8 == 0 && o_row % 8 == 0 && o_head % 8 == 0 && g_row % 8 == 0 && out_row % 8 == 0 && ((uintptr_t)o % 16) == 0 &&
         ((uintptr_t)g % 16) == 0 && ((uintptr_t)out % 16) == 0) {
         sigmoid_gate_heads_vec_kernel<<<(unsigned)((count / 8 + 255) / 256), 256, 0, s>>>((const bf16_t*)o, o_row, o_head, (const bf16_t*)g, g_row,
                                                                                           scale, (bf16_t*)out, out_row, H * E, E, count / 8);
