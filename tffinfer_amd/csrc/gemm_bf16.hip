@@ -288,7 +288,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bf16_async_kernel(
 // Adds up the partial sums part[s][M][N] of a product whose blocks split K, s = 0, 1, ... in
 // turn, and writes C; with GLU, columns come as gate and up groups of 16 in turn and
 // C[m][j] = silu(gate) * up.  One thread makes four neighbouring outputs.
-template <bool GLU, typename TC>
+template <bool GLU, typename TC, bool UNARY>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __restrict__ part, int S,
                                                                   int M, int N, TC* __restrict__ C,
                                                                   int n_out, GluAct act, int unary) {
@@ -321,12 +321,29 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
                     if (j + e < N) a[e] += p[e];
             }
         }
-        if (unary) {
+        if constexpr (UNARY) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) a[e] = unary_activation(a[e], unary);
         }
     }
     store4<TC>(C + (size_t)m * n_out + j, a, j, n_out, (n_out % 4) == 0);
+}
+
+template <bool GLU>
+static int launch_reduce(const float* part, int S, int M, int N, void* C, int n_out, const GemmExtra& ex, int c_dtype, hipStream_t s) {
+    const int blocks = (int)(((long)M * ((n_out + 3) / 4) + 255) / 256);
+#define TFF_REDUCE(TC, UNARY) gemm_splitk_reduce_kernel<GLU, TC, UNARY><<<blocks, 256, 0, s>>>(part, S, M, N, (TC*)C, n_out, ex.act, ex.unary)
+    if constexpr (!GLU) {
+        if (ex.unary) {
+            if (c_dtype == TFF_F32) TFF_REDUCE(float, true);
+            else TFF_REDUCE(bf16_t, true);
+            return tff_check_launch("gemm_splitk_reduce");
+        }
+    }
+    if (c_dtype == TFF_F32) TFF_REDUCE(float, false);
+    else TFF_REDUCE(bf16_t, false);
+#undef TFF_REDUCE
+    return tff_check_launch("gemm_splitk_reduce");
 }
 
 // splits > 1: the blocks of a tile split K among them; part holds splits * M * N floats
@@ -349,14 +366,7 @@ static int launch_async_g(const bf16_t* A, const bf16_t* Wp, void* C, int M, int
             <<<grid, 64 * WGM * WGN, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, part, ex);
     if (int rc = tff_check_launch("gemm_bf16_async")) return rc;
     if (splits > 1 && reduce) {
-        const int No = GLU ? n_out : N;
-        const long threads = (long)M * ((No + 3) / 4);
-        const int blocks = (int)((threads + 255) / 256);
-        if (c_dtype == TFF_F32)
-            gemm_splitk_reduce_kernel<GLU, float><<<blocks, 256, 0, s>>>(part, splits, M, N, (float*)C, No, ex.act, ex.unary);
-        else
-            gemm_splitk_reduce_kernel<GLU, bf16_t><<<blocks, 256, 0, s>>>(part, splits, M, N, (bf16_t*)C, No, ex.act, ex.unary);
-        return tff_check_launch("gemm_splitk_reduce");
+        return launch_reduce<GLU>(part, splits, M, N, C, GLU ? n_out : N, ex, c_dtype, s);
     }
     return 0;
 }
@@ -736,14 +746,7 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
         gemm_bf16_w4_kernel<WTN, NWS, GLU, bf16_t, WGM, SCALE, WTM><<<grid, 256, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, sc, ex);
     if (int rc = tff_check_launch("gemm_bf16_w4")) return rc;
     if (splits > 1 && reduce) {
-        const int No = GLU ? n_out : N;
-        const long threads = (long)M * ((No + 3) / 4);
-        const int blocks = (int)((threads + 255) / 256);
-        if (c_dtype == TFF_F32)
-            gemm_splitk_reduce_kernel<GLU, float><<<blocks, 256, 0, s>>>(part, splits, M, N, (float*)C, No, ex.act, ex.unary);
-        else
-            gemm_splitk_reduce_kernel<GLU, bf16_t><<<blocks, 256, 0, s>>>(part, splits, M, N, (bf16_t*)C, No, ex.act, ex.unary);
-        return tff_check_launch("gemm_splitk_reduce");
+        return launch_reduce<GLU>(part, splits, M, N, C, GLU ? n_out : N, ex, c_dtype, s);
     }
     return 0;
 }
@@ -792,13 +795,16 @@ struct SkinnyFuse {
     float alpha;
 };
 
-template <int MT, int R, int UNROLL, int KSPLIT, int NSETS, bool GLU, typename TC, bool RING = false, int EPI = 0>
+// MORE: several products in one launch, or an activation of the result (GemmExtra).  Kernels of their own: the tests for them and the registers
+// of the activations cost every plain product 0.2 us (a decode step's of 2,048 to 4,096 columns 9.4 / 9.6, of 8 rows 10.9 / 11.1).
+template <int MT, int R, int UNROLL, int KSPLIT, int NSETS, bool GLU, typename TC, bool RING = false, int EPI = 0, bool MORE = false>
 __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, TC* __restrict__ C, int M, int N,
     int K, int lda, int KB, int n_out, SkinnyFuse fz, const GemmExtra ex) {
     const float* __restrict__ const bias = ex.bias;
     static_assert(EPI == 0 || MT == 1, "the fused norm is for up to 16 rows");
     static_assert(EPI < 2 || !GLU, "the product before a norm has a plain float32 result");
+    static_assert(!MORE || (EPI == 0 && !GLU), "planes and activations are for plain products");
     constexpr int SK_WAVES = KSPLIT * NSETS;
     static_assert(!GLU || (R == 1 && NSETS % 2 == 0), "a gate and its up group are one row group each");
     __shared__ floatx4 part[SK_WAVES][R * MT][64];
@@ -808,7 +814,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
     const int NB = (N + 15) / 16;
     const int nb0 = (blockIdx.x * NSETS + set) * R;
     int ldc = N;
-    if constexpr (EPI == 0 && !GLU) {
+    if constexpr (MORE) {
         if (ex.plane_cols) {      // (a wave's columns are one plane's; C as its column 0 of row 0 would lie)
             const size_t plane = (size_t)(min(nb0, NB - 1) * 16 / ex.plane_cols);
             A += plane * ex.a_step;
@@ -1056,7 +1062,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
                             *reinterpret_cast<uint2*>(fz.x_out + (size_t)m * N + n) = pk.u;
                         }
                     } else if (m < M && n < N) {
-                        if constexpr (EPI == 0) {
+                        if constexpr (MORE) {
                             if (ex.unary) {
 #pragma unroll
                                 for (int e = 0; e < 4; ++e) v[e] = unary_activation(v[e], ex.unary);
@@ -1076,6 +1082,19 @@ static int launch_skinny(const bf16_t* A, const bf16_t* Wp, void* C, int M, int 
     const int per_block = NSETS * R;
     const dim3 grid((NB + per_block - 1) / per_block);
     const SkinnyFuse fz = fuse ? *fuse : SkinnyFuse{nullptr, 0, 0, 0.f, 0.f, nullptr, nullptr, nullptr, nullptr, 0, nullptr, 0.f};
+    if (ex.plane_cols || ex.unary) {
+        if constexpr (EPI == 0 && !GLU) {
+            if (c_dtype == TFF_F32)
+                gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, false, float, RING, 0, true>
+                    <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, KB, n_out, fz, ex);
+            else
+                gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, false, bf16_t, RING, 0, true>
+                    <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, fz, ex);
+            return tff_check_launch("gemm_bf16_skinny");
+        } else {
+            return tff_fail("gemm: planes or an activation of a gated or fused product");
+        }
+    }
     if (c_dtype == TFF_F32)
         gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, GLU, float, RING, EPI>
             <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, KB, n_out, fz, ex);
