@@ -121,14 +121,8 @@ def test_experts(dtype, E, top, width, ff, limit, T):
         assert torch.equal(alone[0], tiles[7])
 
 
-@pytest.mark.parametrize("T", [33, 300, 1700])
-@pytest.mark.parametrize("E,top,width,ff,gate,on_input,pad", [
-    (3, 1, 64, 64, True, False, 0), (5, 2, 192, 320, True, True, 64), (4, 2, 1216, 64, False, False, 8), (9, 4, 320, 448, False, True, 0),
-    (12, 3, 576, 200, True, False, 64), (6, 2, 72, 704, False, False, 0)])
-def test_experts_on_whole_lines(E, top, width, ff, gate, on_input, pad, T):
-    """Inner sizes in units of 64 (one of them, both, one unit and many; the last two cases mix the two kernels), output columns
-    that end inside a tile, an expert without pairs and one with most of them, padded rows.  Products of bfloat16 summed in
-    float32, the inner row rounded once: 2^-8 of the largest value covers both roundings."""
+def _experts_case(E, top, width, ff, gate, on_input, pad, T):
+    """Outputs against 64 bits, and the bits of the first token and the first forty by themselves; the pairs of each expert."""
     ops = _ops()
     g = torch.Generator().manual_seed(E + ff + T)
     h = torch.randn(T, width, generator=g).bfloat16().to(DEV)
@@ -154,6 +148,29 @@ def test_experts_on_whole_lines(E, top, width, ff, gate, on_input, pad, T):
     assert float((out.double() - ref).abs().max()) < 2.0 ** -8 * float(ref.abs().max())
     for n in (1, 40):                                # (another split into tiles, other tiles: the same bits)
         assert torch.equal(run(h[:n].contiguous(), idx[:n].contiguous(), wts[:n].contiguous()), out[:n])
+    return torch.bincount(idx.flatten().long(), minlength=E).tolist()
+
+
+@pytest.mark.parametrize("T", [33, 300, 1700])
+@pytest.mark.parametrize("E,top,width,ff,gate,on_input,pad", [
+    (3, 1, 64, 64, True, False, 0), (5, 2, 192, 320, True, True, 64), (4, 2, 1216, 64, False, False, 8), (9, 4, 320, 448, False, True, 0),
+    (12, 3, 576, 200, True, False, 64), (6, 2, 72, 704, False, False, 0)])
+def test_experts_on_whole_lines(E, top, width, ff, gate, on_input, pad, T):
+    """Inner sizes in units of 64 (one of them, both, one unit and many; the last two cases mix the two kernels), output columns
+    that end inside a tile, an expert without pairs and one with most of them, padded rows.  Products of bfloat16 summed in
+    float32, the inner row rounded once: 2^-8 of the largest value covers both roundings."""
+    _experts_case(E, top, width, ff, gate, on_input, pad, T)
+
+
+@pytest.mark.parametrize("E,top,width,ff,gate,on_input,T", [
+    (5, 2, 320, 2048, False, True, 4000), (5, 2, 320, 2048, False, False, 6000), (5, 2, 320, 1792, True, False, 2200), (6, 3, 384, 1152, True, True, 2500),
+    (5, 2, 2048, 320, False, True, 4000), (5, 2, 2048, 320, True, False, 6000), (4, 1, 2048, 448, False, False, 8000)])
+def test_experts_blocks_that_go_on_from_tile_to_tile(E, top, width, ff, gate, on_input, T):
+    """A block a CU, more (tile, column block) pairs than CUs: up products with and without a gate and down products of five units of K (the
+    fewest with which a block goes on), six and seven, in tiles of 64 and of 128 pairs, one expert after the other in a block."""
+    counts = _experts_case(E, top, width, ff, gate, on_input, 8, T)
+    tiles = sum(-(-n // 128) for n in counts)
+    assert max(tiles * -(-ff // (128 if gate else 256)), tiles * -(-width // 256)) > 256 and min(width, ff) // 64 >= 5
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
