@@ -117,3 +117,24 @@ def test_slots_of_spans_as_of_their_tokens():
     assert len(cache.slots_of(1, [("a", live, 420 - live)])) == 420 - live
     with pytest.raises(RuntimeError, match=f"token {live - 1} lies in a page already given back"):
         cache.slot_array(1, "a", live - 1, 3)
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 40])
+def test_the_check_of_a_portions_tokens(n):
+    """Plain whole numbers pass at once where there are more than sixteen; what is outside the vocabulary, or no whole number, is named
+    wherever it stands, and a truth value counts as the number it is, as in short portions."""
+    from types import SimpleNamespace
+    from tffinfer_amd.engine.runner import ModelRunner, StepError
+    cache = CacheManager([(0, True, FULL, None)], 8, 16, 1)
+    cache.add_request("r")
+    runner = SimpleNamespace(cache=cache, vocab_size=100, max_model_len=64)
+    good = [(7 * i) % 100 for i in range(n)]
+    check = lambda toks: ModelRunner._validate(runner, [StepEntry("r", toks, [len(toks) - 1])])      # noqa: E731
+    check(good)
+    check(tuple(good))
+    for at in {0, n // 2, n - 1}:
+        for fine in (0, 99, True, False):
+            check(good[:at] + [fine] + good[at + 1:])
+        for bad in (-1, 100, 1 << 40, -(1 << 40), 3.0, "3", None, np.int64(3), np.int32(200), float("nan")):
+            with pytest.raises(StepError, match="outside the vocabulary"):
+                check(good[:at] + [bad] + good[at + 1:])
