@@ -80,6 +80,23 @@ def test_wkv_dispatch_keeps_to_the_rule(monkeypatch, longest, chunks):
     assert called == ["tff_wkv_recurrence_chunks" if chunks else "tff_wkv_recurrence"]
 
 
+@pytest.mark.parametrize("fits", [True, False])
+def test_a_wkv_layer_asks_the_kernels_rule_for_its_four_products(monkeypatch, fits):
+    """One packed weight where the rule takes it, else four: whatever the rule comes to be."""
+    from tffinfer_amd.kernels import ops
+    from tffinfer_amd.parts import wkv
+    assert [ops.planes_supported(N, K) for N, K in ((128, 64), (4096, 4096), (64, 64), (192, 64), (128, 32), (128, 96))] == [True, True] + [False] * 4
+    asked = []
+    monkeypatch.setattr(ops, "planes_supported", lambda N, K: asked.append((N, K)) or fits)
+    monkeypatch.setattr(wkv, "to_device", lambda t, dtype, device: t)
+    monkeypatch.setattr(torch.Tensor, "to", lambda t, *a, **k: t)              # (nothing goes to a device here)
+    mixer = wkv.WKVMixer(64, 2, 32, decay_rank=4)
+    shapes = {name: spec.shape for name, spec in mixer.weight_specs().items()}
+    mixer.load_weights({name: torch.zeros(shape) for name, shape in shapes.items()}, torch.bfloat16, "cuda:0")
+    assert asked == [(64, 64)] and (mixer.w_four is not None) == fits and (mixer.w_each is None) == fits
+    assert not fits or tuple(mixer.w_four.shape) == (256, 64)
+
+
 @pytest.mark.parametrize("lengths,heads,dim,groups", [
     ([901], 32, 128, 1), ([901] + [1] * 63, 32, 128, 1), ([1] * 30 + [95, 500], 32, 128, 1), ([901, 400, 400], 32, 128, 1), ([2000] + [200] * 5, 32, 128, 1),
     ([901, 848, 677, 664], 32, 128, 2), ([500] * 6, 32, 128, 2), ([901, 848, 677, 664], 16, 128, 1), ([200] * 16, 16, 128, 2), ([200] * 16, 8, 128, 2),

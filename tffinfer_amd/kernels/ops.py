@@ -478,7 +478,7 @@ def linear_unary(x: torch.Tensor, weight, act: str, out_dtype: torch.dtype) -> t
 
 def planes_supported(N: int, K: int) -> bool:
     """Whether :func:`linear_planes` takes bfloat16 products of [N, K]."""
-    return N % 128 == 0 and K % 64 == 0
+    return bool(_lib.load().tff_gemm_planes_supported(N, K))
 
 
 def linear_planes(x: torch.Tensor, weight: PackedWeight) -> torch.Tensor:

@@ -77,7 +77,8 @@ class WKVMixer(Mixer):
         self.mu = f32(torch.stack([weights[f"mu.{s}"].to(torch.float32) for s in self.MIXES], 0))
         four = [weights[s] for s in ("r", "k", "v", "g")]
         self.w_four, self.w_each = None, None
-        if dtype == torch.bfloat16 and torch.device(device).type == "cuda" and self.inner % 128 == 0 and self.hidden_size % 64 == 0:
+        from ..kernels import ops
+        if dtype == torch.bfloat16 and torch.device(device).type == "cuda" and ops.planes_supported(self.inner, self.hidden_size):
             # one weight, a product of four planes
             self.w_four = to_device(torch.cat([w.to(dtype) for w in four], 0), dtype, device)
         else:
