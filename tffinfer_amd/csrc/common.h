@@ -102,6 +102,7 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 // that tff_last_error() hands out.
 int tff_fail(const char* fmt, ...);
 int tff_check_launch(const char* what);
+int tff_device_cus();      // compute units of the current device
 
 #define TFF_REQUIRE(cond, ...)                     \
     do {                                           \

@@ -22,6 +22,18 @@ int tff_check_launch(const char* what) {
     if (e != hipSuccess) return tff_fail("%s: launch failed: %s", what, hipGetErrorString(e));
     return 0;
 }
+// Compute units of the current device (256 on an MI355X), for plans that count how often blocks go round them; 256 if it cannot be asked.
+int tff_device_cus() {
+    static int cached[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (cached[dev] == 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        cached[dev] = n;
+    }
+    return cached[dev];
+}
 TFF_API const char* tff_last_error() { return g_error; }
 TFF_API int tff_abi_version() { return 47; }
 

@@ -1112,25 +1112,11 @@ static int launch_skinny(const bf16_t* A, const bf16_t* Wp, void* C, int M, int 
 // up to 64 and 32 rows, of 64 and 32 rows (256 or 128 columns), and from 65 to 512 rows also
 // 64 x 128 with several row tiles; otherwise the sixteen-wave kernel's tiles.
 struct GemmPlan { int tile; int bn; int splits; };   // tile = rows of a block tile
-// Compute units of the current device (256 on an MI355X, which the rates below were fitted on; a
-// device with another count gets plans for its own number of blocks a round).  256 if it cannot
-// be asked.
-static int device_cus() {
-    static int cached[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cached[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cached[dev] = n;
-    }
-    return cached[dev];
-}
 // Up to 16 rows, not gated: more row groups of 16 columns than CUs, but at most 1.6 times as many
 // (a second round of blocks that would be less than 0.6 full): the streaming kernel then gives a block
 // two row groups (skinny_for).
 static bool two_row_groups(int N) {
-    const int nb = (N + 15) / 16, cus = device_cus();
+    const int nb = (N + 15) / 16, cus = tff_device_cus();
     return nb > cus && nb * 10 <= cus * 16;
 }
 // Up to 16 rows, gated: the streaming kernel's blocks each fetch all of A's rows, so its time grows
@@ -1146,7 +1132,7 @@ static bool few_rows_gated_on_tiles(int M, int N, int K) {
 }
 // One row tile of 32 rows, K in one part: the width (128 or 256 columns) that plan_for's model prices lowest.
 static int plan_rows32(int N, int K) {
-    const double CUS = (double)device_cus();
+    const double CUS = (double)tff_device_cus();
     const int widths[2] = {128, 256};
     const double rates[2] = {1.3e6, 1.4e6};
     int best = 256;
@@ -1163,7 +1149,7 @@ static int plan_rows32(int N, int K) {
 
 // plane > 0: the columns of several products, so many each; a tile takes columns of one of them, and K is not split.
 static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0) {
-    const double CUS = (double)device_cus();
+    const double CUS = (double)tff_device_cus();
     // Up to 16 rows: the streaming kernel, a block per 16 columns, unless those blocks go badly
     // round the 256 CUs (320 of them take as long as 512 would: N = 5120), the caller takes
     // partial sums anyway and the weight is large enough for the gain (three eighths of its

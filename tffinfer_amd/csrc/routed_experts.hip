@@ -903,6 +903,7 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
     // alone on its CU and a tile of 128 takes some 1.12 times as long as one of 64 (up to there both are their weight's stream), so
     // what counts is how often the blocks go round the CUs.  us, 64 / 128: 32 experts, four a token, 4,096 x 1,536, 150 tokens 244 / 265,
     // 512 tokens 318 / 288, 1,000 tokens 413 / 376; 16 experts, two a token, 2,048 x 1,024, 700 tokens 68 / 80, 1,000 tokens 114 / 83.
+    const int cus = tff_device_cus();
     bool tall = (long)T * top >= 192L * E;
     if (lines_up && lines_down) {
         const double n = (double)T * top / E;
@@ -910,7 +911,7 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
         double cost[2];
         for (int i = 0; i < 2; ++i) {
             const double tiles = E * fmax(1.0, n / (64 << i) + 0.5);      // (half of an expert's last tile is padding on average)
-            cost[i] = ceil(tiles * cb_up / 256) * width + ceil(tiles * cb_down / 256) * ff;
+            cost[i] = ceil(tiles * cb_up / cus) * width + ceil(tiles * cb_down / cus) * ff;
         }
         tall = cost[1] * 1.12 < cost[0];
     }
@@ -932,7 +933,7 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
                      act_alpha, up_offset, nullptr, out, cb, ldw_down, weight_input
 #define EX_GRID (unsigned)(((long)cb * max_tiles + 7) / 8 * 8)
 // (one block a CU, which goes on from pair to pair; each pair a block of its own where K has too few units for that)
-#define EXL_GRID(MODE) (((MODE) == 0 ? ff : width) / 64 < EXL_CHAIN ? EX_GRID : EX_GRID < 256u ? EX_GRID : 256u)
+#define EXL_GRID(MODE) (((MODE) == 0 ? ff : width) / 64 < EXL_CHAIN ? EX_GRID : EX_GRID < most ? EX_GRID : most)
 #define EX_LINES(MODE, ...)                                                                                \
     do {                                                                                                   \
         if (tall) experts_lines_kernel<MODE, 2, 4, 8><<<EXL_GRID(MODE), 256, 0, s>>>(__VA_ARGS__);         \
@@ -943,6 +944,7 @@ TFF_API int tff_experts_by_tiles(const void* h, int h_row, const void* Wg, const
         if (tall) experts_tiles_kernel<MODE, 8><<<EX_GRID, 256, 0, s>>>(__VA_ARGS__);                      \
         else experts_tiles_kernel<MODE, 4><<<EX_GRID, 256, 0, s>>>(__VA_ARGS__);                           \
     } while (0)
+    const unsigned most = (unsigned)(cus < 8 ? 8 : cus / 8 * 8);      // (a multiple of the XCDs, which the blocks' numbering deals them to)
     {
         const int out_cols = (lines_up ? 256 : 128) / (Wg ? 2 : 1), cb = (ff + out_cols - 1) / out_cols;
         if (lines_up && up_mode == 1) EX_LINES(1, EX_ARGS_UP);
