@@ -16,6 +16,7 @@
 #include "common.h"
 #include "mfma_tiles.h"
 #include "tffinfer_kernels.h"
+#include <type_traits>
 
 
 __device__ __forceinline__ uint4 ld16(const bf16_t* p) { return *reinterpret_cast<const uint4*>(p); }
@@ -41,12 +42,16 @@ __device__ __forceinline__ void store4(TC* dst, const floatx4& v, int n, int N, 
 
 // What a product takes besides its operands: a bias (float32, in the order of W's rows, ceil16(N) numbers) or null,
 // and how a gated product joins gate and up.
+struct GemmEpilogue {
+    const float* bias;
+    GluAct act;
+};
+// And what some kernels of their own take beside that (in the arguments of all, it changed the schedule of most: gate and up of 2,048 columns
+// and 3 rows 11.8 / 12.3 us).
 // unary: what becomes of a result that is not gated (unary_activation), where the streaming kernel or the sum over a split K's
 // parts stores it.  plane_cols > 0: several products in one launch.  W's rows are theirs one after the other, plane_cols each; the
 // columns of plane p take their rows from A + p * a_step, and C holds the planes [p][M][plane_cols].
-struct GemmExtra {
-    const float* bias;
-    GluAct act;
+struct GemmExtra : GemmEpilogue {
     int unary;
     int plane_cols;
     size_t a_step;
@@ -92,7 +97,7 @@ typedef const __attribute__((address_space(1))) void* glb_ptr_t;
 template <int WGM, int WGN, int WTM, int WTN, int STAGES, bool GLU, typename TC, int KPS = 2, bool EARLY = false>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bf16_async_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, TC* __restrict__ C, int M, int N,
-    int K, int lda, int KB, int n_out, float* __restrict__ part, const GemmExtra ex) {
+    int K, int lda, int KB, int n_out, float* __restrict__ part, const GemmEpilogue ex) {
     const float* __restrict__ const bias = ex.bias;
     // WGM x WGN waves, each WTM x WTN MFMA tiles of 16 x 16
     constexpr int NW = WGM * WGN;
@@ -473,7 +478,8 @@ struct W4Scale {
 template <int WTN, int NWS, bool GLU, typename TC, int WGM = 2, bool SCALE = false, int WTM = 8, bool PLANES = false>
 __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, TC* __restrict__ C, int M, int N,
-    int K, int lda, int KB, int n_out, W4Scale sc, const GemmExtra ex) {
+    int K, int lda, int KB, int n_out, W4Scale sc,
+    const typename std::conditional<PLANES, GemmExtra, GemmEpilogue>::type ex) {
     const float* __restrict__ const bias = ex.bias;
     static_assert(!SCALE || WGM == 1, "rows that lack their norm's factor: up to 16, one row tile");
     // WGM: waves along the rows, 2 (a block tile of 256 rows, two waves side by side) or 1 (128 rows, four side by side)
@@ -704,7 +710,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
                                            n_out % E == 0);
     } else {
         // (partial sums of a split K: plane blockIdx.z of the launcher's float32 workspace, which it passes as C)
-        const int ldc = PLANES ? ex.plane_cols : N;
+        int ldc = N;
+        if constexpr (PLANES) ldc = ex.plane_cols;
         TC* out = PLANES ? C : C + (size_t)blockIdx.z * M * N;
         w4_store_rows<WTN, REGION, TC, WTM>(region, [&](int i, int jj) { return scaled(acc[i][jj]); }, out, (size_t)ldc, mw,
                                        n0 + wn * WTN * 16, M, N, lane_out, ldc % E == 0);
@@ -800,7 +807,8 @@ struct SkinnyFuse {
 template <int MT, int R, int UNROLL, int KSPLIT, int NSETS, bool GLU, typename TC, bool RING = false, int EPI = 0, bool MORE = false>
 __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, TC* __restrict__ C, int M, int N,
-    int K, int lda, int KB, int n_out, SkinnyFuse fz, const GemmExtra ex) {
+    int K, int lda, int KB, int n_out, SkinnyFuse fz,
+    const typename std::conditional<MORE, GemmExtra, GemmEpilogue>::type ex) {
     const float* __restrict__ const bias = ex.bias;
     static_assert(EPI == 0 || MT == 1, "the fused norm is for up to 16 rows");
     static_assert(EPI < 2 || !GLU, "the product before a norm has a plain float32 result");
@@ -1431,7 +1439,7 @@ TFF_API int tff_gemm_residual_prenorm(const void* A, const void* Wp, int M, int 
     TFF_REQUIRE(((uintptr_t)resid % 16) == 0 && ((uintptr_t)norm_w % 16) == 0 && ((uintptr_t)x_out % 8) == 0,
                 "gemm_residual_prenorm: operands must be 16-byte aligned");
     SkinnyFuse fz{nullptr, 0, 0, 0.f, 0.f, resid, norm_w, (bf16_t*)x_out, ss_out, ss_stride, nullptr, 0.f};
-    return skinny_for<2>((const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmExtra{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, TFF_F32, 0, (hipStream_t)stream, &fz);
+    return skinny_for<2>((const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmExtra{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, 0, 0}, TFF_F32, 0, (hipStream_t)stream, &fz);
 }
 
 // resid[M, N] += A . W^T (bfloat16 A and packed W, float32 sums); x_out[M, N] = bfloat16 of
@@ -1445,7 +1453,7 @@ TFF_API int tff_gemm_residual_dyt(const void* A, const void* Wp, int M, int N, i
     TFF_REQUIRE(((uintptr_t)resid % 16) == 0 && ((uintptr_t)norm_w % 16) == 0 && ((uintptr_t)bias % 16) == 0 &&
                 ((uintptr_t)x_out % 8) == 0, "gemm_residual_dyt: operands must be 16-byte aligned");
     SkinnyFuse fz{nullptr, 0, 0, 0.f, 0.f, resid, norm_w, (bf16_t*)x_out, nullptr, 0, bias, alpha};
-    return skinny_for<3>((const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmExtra{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, TFF_F32, 0, (hipStream_t)stream, &fz);
+    return skinny_for<3>((const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmExtra{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, 0, 0}, TFF_F32, 0, (hipStream_t)stream, &fz);
 }
 
 // C = rstd[m] * (A . W^T) with rstd[m] = rsqrt(sum_g ss[m][g] / dim + eps), g < ss_count: the product
@@ -1453,7 +1461,7 @@ TFF_API int tff_gemm_residual_dyt(const void* A, const void* Wp, int M, int N, i
 TFF_API int tff_gemm_row_scaled(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int c_dtype,
                                 int glu_out, const float* ss, int ss_stride, int ss_count, int dim, float eps,
                                 float glu_limit, float glu_alpha, float glu_up_offset, tff_stream_t stream) {
-    const GemmExtra ex{nullptr, glu_act(glu_limit, glu_alpha, glu_up_offset)};
+    const GemmExtra ex{{nullptr, glu_act(glu_limit, glu_alpha, glu_up_offset)}, 0, 0, 0};
     if (int rc = check_fused_operands("gemm_row_scaled", A, Wp, M, N, K, lda)) return rc;
     TFF_REQUIRE(C && ss && ((uintptr_t)C % 16) == 0 && ((uintptr_t)ss % 16) == 0, "gemm_row_scaled: null or unaligned pointer");
     TFF_REQUIRE(c_dtype == TFF_F32 || c_dtype == TFF_BF16, "gemm_row_scaled: unknown output type %d", c_dtype);
@@ -1498,7 +1506,7 @@ TFF_API int tff_gemm(const void* A, const void* W, void* C, int M, int N, int K,
         TFF_REQUIRE(((uintptr_t)workspace % 16) == 0, "gemm: the workspace must be 16-byte aligned");
         TFF_REQUIRE(((uintptr_t)bias % 16) == 0, "gemm: the bias must be 16-byte aligned");
         return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda,
-                             GemmExtra{bias, glu_act(glu_limit, glu_alpha, glu_up_offset)}, c_dtype, glu_out,
+                             GemmExtra{{bias, glu_act(glu_limit, glu_alpha, glu_up_offset)}, 0, 0, 0}, c_dtype, glu_out,
                              (float*)workspace, workspace ? workspace_bytes : 0, keep_partials, s);
     }
     return tff_fail("gemm: unknown operand type %d", ab_dtype);
@@ -1516,7 +1524,7 @@ TFF_API int tff_gemm_unary(const void* A, const void* W, void* C, int M, int N, 
     TFF_REQUIRE(M >= 0 && N > 0 && K > 0 && lda >= K && kind >= 1 && kind <= 4, "gemm_unary: bad sizes M=%d N=%d K=%d lda=%d or kind %d", M, N, K, lda, kind);
     TFF_REQUIRE(((uintptr_t)workspace % 16) == 0, "gemm_unary: the workspace must be 16-byte aligned");
     if (M == 0) return 0;
-    return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, GemmExtra{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f), kind, 0, 0},
+    return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, GemmExtra{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, kind, 0, 0},
                          c_dtype, 0, (float*)workspace, workspace ? workspace_bytes : 0, 0, (hipStream_t)stream);
 }
 
@@ -1531,7 +1539,7 @@ TFF_API int tff_gemm_planes(const void* A, size_t a_step, const void* W, float* 
                 planes, M, N, K, lda);
     TFF_REQUIRE(tff_gemm_planes_supported(N, K) && a_step % 8 == 0, "gemm_planes: N=%d in units of 128, K=%d of 64, rows' planes (%zu apart) of 8", N, K, a_step);
     if (M == 0) return 0;
-    return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, planes * N, K, lda, GemmExtra{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f), 0, N, a_step},
+    return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, planes * N, K, lda, GemmExtra{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, N, a_step},
                          TFF_F32, 0, nullptr, 0, 0, (hipStream_t)stream);
 }
 
