@@ -80,6 +80,42 @@ def test_wkv_dispatch_keeps_to_the_rule(monkeypatch, longest, chunks):
     assert called == ["tff_wkv_recurrence_chunks" if chunks else "tff_wkv_recurrence"]
 
 
+@pytest.mark.parametrize("lengths,starts,window,sixteen", [
+    ([64], [0], 0, False), ([88], [0], 0, False), ([89], [0], 0, False), ([100], [0], 0, False), ([111], [0], 0, False), ([112], [0], 0, True), ([300], [0], 0, True), ([112], [0], 37, False),
+    ([113], [0], 37, True), ([64], [1000], 0, True), ([64], [1000], 100, False), ([20] * 5, [0] * 5, 0, False), ([60] + [1] * 10, [0] + [900] * 10, 0, True),
+    ([63], [5000], 0, False), ([15] * 40, [5000] * 40, 0, False)])
+def test_short_prompts_of_mixed_heads_take_a_block_a_token(monkeypatch, lengths, starts, window, sixteen):
+    """Sixteen queries a block from 64 tokens on, with an entry of 16 and more, where the tokens see enough keys; a batch that does not
+    hold its contexts is taken to see all that a window lets it."""
+    from tffinfer_amd.kernels import ops
+    real, called = _lib(), []
+
+    class Library:
+        def __getattr__(self, name):
+            if name in ("tff_mixed_attention", "tff_mixed_attention_q16"):
+                return lambda *a: called.append(name) or 0
+            return getattr(real, name)
+    monkeypatch.setattr(ops._lib, "load", lambda: Library())
+    monkeypatch.setattr(ops, "_req", lambda t, *a, **k: t)
+    monkeypatch.setattr(ops, "_check_cache", lambda *a: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    H, G, D, page, T = 20, 5, 64, 16, sum(lengths)
+    contexts = [s + n for s, n in zip(starts, lengths)]
+    i32 = torch.zeros(max(T, len(lengths)), dtype=torch.int32)
+    kv = types.SimpleNamespace(k_cache=torch.zeros(1, dtype=torch.bfloat16), v_cache=torch.zeros(1, dtype=torch.bfloat16), page_size=page,
+                               block_tables=torch.zeros(len(lengths), -(-max(contexts) // page), dtype=torch.int32))
+    batch = types.SimpleNamespace(token_req=i32, positions=i32, max_new_tokens=max(lengths), host_cu_tokens=[sum(lengths[:i]) for i in range(len(lengths) + 1)])
+    q = torch.zeros(T, H * D, dtype=torch.bfloat16)
+    ops.mixed_attention(q, H, G, D, kv, types.SimpleNamespace(max_context=max(contexts), **vars(batch)), 1.0, window=window)
+    ops.mixed_attention(q, H, G, D, kv, batch, 1.0, window=window)
+    blind = T >= 64 and max(lengths) >= 16 and (window == 0 or T > 112)
+    assert called == ["tff_mixed_attention_q16" if x else "tff_mixed_attention" for x in (sixteen, blind)]
+    if T in (88, 89) and max(contexts) < 100:                 # (more than one kv head a wave: up to 88 tokens)
+        del called[:]
+        ops.mixed_attention(q[:, :20 * 32].contiguous(), 20, 20, 32, kv, types.SimpleNamespace(max_context=T, **vars(batch)), 1.0)
+        assert called == ["tff_mixed_attention_q16" if T == 89 else "tff_mixed_attention"]
+
+
 @pytest.mark.parametrize("fits", [True, False])
 def test_a_wkv_layer_asks_the_kernels_rule_for_its_four_products(monkeypatch, fits):
     """One packed weight where the rule takes it, else four: whatever the rule comes to be."""

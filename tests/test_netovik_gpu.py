@@ -481,6 +481,33 @@ def test_attention_on_the_matrix_cores_at_the_tiles_edges(H, G, D, page):
             assert err < 3e-2, (T, window, keep, cuts[:2], err)      # (bfloat16 queries, keys, weights and results, as above)
 
 
+@pytest.mark.parametrize("H,G,D,page", [(32, 8, 128, 16), (20, 5, 64, 16), (32, 32, 64, 16), (16, 1, 32, 32)])
+@pytest.mark.parametrize("lengths", [[64], [111], [20, 37, 1, 28], [20, 37, 1, 50]])
+def test_short_prompts_a_block_a_token(H, G, D, page, lengths):
+    """Steps of 64 tokens and more whose requests hold little: a block a token, several of a request among them.  (Bound as above.)"""
+    ops = _ops()
+    from tffinfer_amd.parts.mixed_attention import distance_buckets
+    g = torch.Generator().manual_seed(H + len(lengths))
+    eps, B, Dmax, T = 1e-5, 10, 50, sum(lengths)
+    talk, rel = torch.eye(H) + 0.3 * torch.randn(H, H, generator=g), torch.randn(B, H, generator=g)
+    table = rel[distance_buckets(B, Dmax)].contiguous().to(DEV)
+    qk, qb, kb = _attention_case(H, G, D, T, T + H)
+    cache = _Cache(G, D, page, lengths, torch.bfloat16, seed=T)
+    cache.k.fill_(float("nan"))
+    cache.v.fill_(float("nan"))
+    kv = cache.view(list(range(len(lengths))), [0] * len(lengths), lengths)
+    q = ops.qk_bias_norm_store(qk.to(DEV), qb.to(DEV), kb.to(DEV), eps, H, G, D, kv)
+    batch = _batch(lengths, [0] * len(lengths))
+    batch.max_context = max(lengths)
+    args = dict(scale=min(0.7, 6.0 / D), softcap=4.0, bias=table, mix=talk.to(DEV), window=33, keep_first=5, sink=True)
+    out = ops.mixed_attention(q, H, G, D, kv, batch, **args)
+    at = 0
+    for n in lengths:
+        ref = _plain_attention(qk[at:at + n], qb, kb, H, G, D, eps, scale=min(0.7, 6.0 / D), cap=4.0, rel=rel, bias_max=Dmax, talk=talk, window=33, keep=5, sink=True)
+        assert _err(out[at:at + n], ref) < 3e-2
+        at += n
+
+
 def _queries_keys_values(H, G, D, T, seed):
     g = torch.Generator().manual_seed(seed)
     return [torch.randn(T, n, D, generator=g).to(torch.bfloat16) for n in (H, G, G)]

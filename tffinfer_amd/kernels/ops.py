@@ -1628,6 +1628,12 @@ def qk_bias_norm_store(qk: torch.Tensor, q_bias, k_bias, eps: float, H: int, G: 
 MIXED_ATTENTION_BLOCKS = 512
 #: tokens of a step from which bfloat16 attention runs sixteen queries a block on the matrix cores
 MIXED_ATTENTION_Q16_TOKENS = 64
+#: up to so many tokens times the keys that one of them can see, and up to 112 tokens (88 where a wave has more than one kv head), such a
+#: step takes a block a token all the same: blocks of sixteen queries are few then, and none is through its first 64 keys before some
+#: 20 us.  us, a block a token / sixteen queries a block: prompts of 64 and 100 tokens, 32 heads of 128 on 8 kv heads 12.9 / 32.2 and
+#: 19.5 / 32.7, 20 of 64 on 5 9.9 / 27.1 and 12.1 / 27.5, 16 of 128 on 16 17.6 / 23.9 and 23.6 / 24.0; of 128 tokens, the last 27.5 / 24.3;
+#: 64 behind 1,000 others 137 / 64; 200 under a window of 37 47 / 25
+MIXED_ATTENTION_Q16_KEYS = 12500
 #: blocks that kernel's items are spread over where they are fewer (a block a CU)
 MIXED_ATTENTION_Q16_BLOCKS = 256
 
@@ -1667,8 +1673,10 @@ def mixed_attention(q: torch.Tensor, H: int, G: int, D: int, kv, batch, scale: f
         raise _lib.KernelError("mixed_attention: the step's tables are shorter than q")
     out = torch.empty(T, H * D, dtype=dt, device=q.device)
     cu = getattr(batch, "host_cu_tokens", None)
+    longest = getattr(batch, "max_context", 1 << 30)
     if (splits is None and dt == torch.bfloat16 and cu is not None and T >= MIXED_ATTENTION_Q16_TOKENS
             and getattr(batch, "max_new_tokens", 0) >= 16
+            and (T > (112 if G <= 8 else 88) or T * (min(longest, window + keep_first) if window > 0 else longest) > MIXED_ATTENTION_Q16_KEYS)
             and L.tff_mixed_attention_q16_supported(H, D, kv.page_size, 1 if mix is not None else 0)):
         # a prompt's portions: sixteen queries a block, the products on the matrix cores
         cache = getattr(batch, "_q16_work", None)
@@ -1677,7 +1685,7 @@ def mixed_attention(q: torch.Tensor, H: int, G: int, D: int, kv, batch, scale: f
             cache = batch._q16_work = _staging.send(q.device, [np.asarray(items, dtype=np.int32).reshape(-1, 2)])[0]
         # tiles of 64 keys an item can have at most; where the items are fewer than the CUs, their tiles are dealt
         # to several blocks
-        reach = min(bt.shape[1] * kv.page_size, getattr(batch, "max_context", 1 << 30))
+        reach = min(bt.shape[1] * kv.page_size, longest)
         tiles = -(-min(keep_first, reach) // 64) + (-(-min(window + 15, reach) // 64) + 1 if window > 0 else -(-reach // 64))
         parts = max(1, min(tiles, 8, MIXED_ATTENTION_Q16_BLOCKS // cache.shape[0]))
         per = -(-tiles // parts)
