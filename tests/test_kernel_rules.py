@@ -116,6 +116,14 @@ def test_short_prompts_of_mixed_heads_take_a_block_a_token(monkeypatch, lengths,
         assert called == ["tff_mixed_attention_q16" if T == 89 else "tff_mixed_attention"]
 
 
+@pytest.mark.parametrize("n,H,groups,levels,one", [
+    (1, 4096, 2, 10, 1), (1, 4096, 2, 11, 0), (1, 4096, 1, 2, 0), (1, 2049, 1, 1, 0), (1, 2048, 1, 1, 1), (31, 4096, 2, 12, 0), (32, 4096, 2, 12, 1), (32, 4096, 2, 13, 0),
+    (127, 4096, 2, 20, 0), (128, 4096, 2, 20, 1), (128, 4096, 2, 21, 0), (256, 4096, 2, 40, 1), (4000, 8192, 2, 2, 0), (4000, 8192, 4, 40, 1)])
+def test_the_sum_over_depth_goes_with_a_norm_that_it_does_not_hold_up(n, H, groups, levels, one):
+    """Not behind groups that a block reads more than once, nor over many levels of few rows."""
+    assert _lib().tff_group_depth_in_norm(n, H, groups, levels) == one
+
+
 @pytest.mark.parametrize("fits", [True, False])
 def test_a_wkv_layer_asks_the_kernels_rule_for_its_four_products(monkeypatch, fits):
     """One packed weight where the rule takes it, else four: whatever the rule comes to be."""

@@ -699,9 +699,11 @@ def test_batches_of_unequal_requests_share_the_attention():
 
 
 @pytest.mark.parametrize("n,H,groups,planes,levels", [(1, 256, 1, 1, 2), (3, 1000, 2, 2, 5), (1, 4096, 2, 1, 8), (700, 2048, 2, 4, 3), (600, 4096, 2, 6, 4),
-                                                      (2, 6000, 1, 1, 1)])
+                                                      (2, 6000, 1, 1, 1), (5, 2049, 1, 2, 9), (1, 4096, 2, 1, 10), (1, 4096, 2, 1, 11), (64, 1024, 2, 1, 20),
+                                                      (128, 2048, 2, 2, 20), (128, 2048, 2, 2, 21), (256, 2048, 2, 1, 33)])
 def test_output_norm_with_the_sum_over_depth(n, H, groups, planes, levels):
-    """Every form of the kernel, a group longer than it holds among them: the same bits as the two launches."""
+    """Every form of the kernel, and what is better left to two launches (groups longer than it holds, many levels of few rows): the same bits
+    as the two launches."""
     ops = _ops()
     g = torch.Generator().manual_seed(n + H)
     r = lambda *s: torch.randn(*s, generator=g).to(DEV)       # noqa: E731

@@ -22,7 +22,8 @@
 // group 8.2 / 5.7, in four with four planes 5.1 / 3.8, 8 rows of 6000 14.1 / 10.4, 400 rows of 8192 24.8 / 16.5, 1,500 rows of 4096 in eight
 // groups 25.0 / 19.9, in two with eight planes 52.6 / 50.1.
 // DEPTH: the new row is a level of the sum over depth, which takes its place in the stream and goes to `out` (tff_depth_average in the same
-// launch): the levels before do not wait for the norm, and the stream is not written and read in between.
+// launch): the levels before do not wait for the norm, and the stream is not written and read in between.  For groups that pass through memory
+// once (tff_group_depth_in_norm).
 struct GroupDepth {
     float* hist;
     const float* coef;
@@ -64,11 +65,6 @@ __global__ __launch_bounds__(GN_THREADS) void group_rmsnorm_add_kernel(
             for (int it = 0; it < GN_ITS; ++it) cache[it] += dl[p * plane + min(tid + it * GN_THREADS, Hg - 1)];
     }
     float* const hist = DEPTH ? dp.hist + (size_t)r * H + base : nullptr;
-    auto below = [&](int j) {                          // the levels before, in their order
-        float acc = 0.f;
-        for (int l = 0; l + 1 < dp.n; ++l) acc = fmaf(dp.coef[l], hist[l * dp.level + j], acc);
-        return acc;
-    };
     float acc[DEPTH ? GN_ITS : 1];
     if constexpr (DEPTH) {
 #pragma unroll
@@ -107,7 +103,8 @@ __global__ __launch_bounds__(GN_THREADS) void group_rmsnorm_add_kernel(
         const int j = tid + it * GN_THREADS;
         if (j < Hg) emit(j, cache[it], EARLY ? wr[it] : wg[j], EARLY ? xr[it] : x ? x[j] : 0.f, DEPTH ? acc[it] : 0.f);
     }
-    for (int j = tid + GN_ITS * GN_THREADS; j < Hg; j += GN_THREADS) emit(j, term(j), wg[j], x ? x[j] : 0.f, DEPTH ? below(j) : 0.f);
+    if constexpr (!DEPTH)
+        for (int j = tid + GN_ITS * GN_THREADS; j < Hg; j += GN_THREADS) emit(j, term(j), wg[j], x ? x[j] : 0.f, 0.f);
 }
 
 template <bool DEPTH>
@@ -147,14 +144,6 @@ TFF_API int tff_group_rmsnorm_add(float* resid, const float* delta, int planes, 
                                   tff_stream_t stream) {
     return group_norm_launch<false>(resid, delta, planes, plane, rows, w, groups, eps, out, n, H, out_dtype, GroupDepth{}, stream);
 }
-TFF_API int tff_group_rmsnorm_add_depth(float* resid, const float* delta, int planes, size_t plane, const float* w, int groups, float eps,
-                                        float* hist, size_t level, int levels, const float* coef, void* out, int n, int H, int out_dtype,
-                                        tff_stream_t stream) {
-    TFF_REQUIRE(resid && hist && coef && levels >= 1 && level >= (size_t)n * H, "group_rmsnorm_add_depth: %d levels, %zu apart, of %d rows of %d", levels,
-                level, n, H);
-    return group_norm_launch<true>(resid, delta, planes, plane, nullptr, w, groups, eps, out, n, H, out_dtype, GroupDepth{hist, coef, level, levels}, stream);
-}
-
 template <typename TO>
 __global__ __launch_bounds__(256) void depth_average_kernel(float* __restrict__ hist, size_t level, int n,
                                                             const float* __restrict__ coef, float* __restrict__ x,
@@ -224,6 +213,27 @@ TFF_API int tff_depth_average(float* hist, size_t level, int n, const float* coe
     else
         return tff_fail("depth_average: unknown dtype %d", out_dtype);
     return tff_check_launch("depth_average");
+}
+
+// Whether the sum over depth goes with the norm.  Not for groups that a block reads more than once, whose elements past the first 2,048 would
+// take a load a level one after the other; nor, for few blocks, over many levels: a block asks for two levels at a time, the sum by
+// itself for eight.  us, two launches / one, rows of 4,096 in two groups: one row, 4, 7, 12 and 33 levels 5.6 / 4.9, 5.9 / 5.3, 5.8 / 6.0 and 6.2 / 9.0;
+// 48 rows, 12 and 20 levels 6.7 / 6.3 and 6.9 / 7.4; 128 rows, 20 and 33 12.6 / 11.4 and 16.3 / 15.2; 1,500 rows, 33 186 / 172; in one group, one row,
+// 7 and 33 levels 8.9 / 12.6 and 9.2 / 36.
+TFF_API int tff_group_depth_in_norm(int n, int H, int groups, int levels) {
+    const long blocks = (long)n * groups;
+    return H / groups <= 8 * GN_THREADS && (levels <= (blocks < 64 ? 10 : blocks < 256 ? 12 : 20) || blocks >= 512);
+}
+TFF_API int tff_group_rmsnorm_add_depth(float* resid, const float* delta, int planes, size_t plane, const float* w, int groups, float eps,
+                                        float* hist, size_t level, int levels, const float* coef, void* out, int n, int H, int out_dtype,
+                                        tff_stream_t stream) {
+    TFF_REQUIRE(resid && hist && coef && levels >= 1 && level >= (size_t)n * H, "group_rmsnorm_add_depth: %d levels, %zu apart, of %d rows of %d", levels,
+                level, n, H);
+    TFF_REQUIRE(n >= 0 && H > 0 && groups > 0 && H % groups == 0, "group_rmsnorm_add_depth: rows of %d in %d groups", H, groups);
+    if (tff_group_depth_in_norm(n, H, groups, levels))
+        return group_norm_launch<true>(resid, delta, planes, plane, nullptr, w, groups, eps, out, n, H, out_dtype, GroupDepth{hist, coef, level, levels}, stream);
+    if (int rc = group_norm_launch<false>(resid, delta, planes, plane, nullptr, w, groups, eps, nullptr, n, H, TFF_F32, GroupDepth{}, stream)) return rc;
+    return tff_depth_average(hist, level, levels, coef, resid, out, (size_t)n * H, out_dtype, stream);
 }
 
 __global__ __launch_bounds__(256) void scale_rows_kernel(float* __restrict__ x, float alpha, size_t count) {

@@ -371,7 +371,9 @@ TFF_API int tff_experts_place(int id, int col_blocks, int first, int n);
 TFF_API int tff_group_rmsnorm_add(float* resid, const float* delta, int planes, size_t plane, const int32_t* rows,
                                   const float* w, int groups, float eps, void* out, int n, int H, int out_dtype,
                                   tff_stream_t stream);
-// tff_group_rmsnorm_add with `resid`, then tff_depth_average over `levels` levels, `level` elements apart, in one launch.
+// tff_group_rmsnorm_add with `resid`, then tff_depth_average over `levels` levels, `level` elements apart, in one launch where that is the
+// sooner done (tff_group_depth_in_norm): the same bits.
+TFF_API int tff_group_depth_in_norm(int n, int H, int groups, int levels);
 TFF_API int tff_group_rmsnorm_add_depth(float* resid, const float* delta, int planes, size_t plane, const float* w, int groups, float eps,
                                         float* hist, size_t level, int levels, const float* coef, void* out, int n, int H, int out_dtype,
                                         tff_stream_t stream);

@@ -88,6 +88,7 @@ _SIGNATURES = {
     "tff_experts_place": [_I, _I, _I, _I],
     "tff_experts_by_tiles": [_P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _P, _P, _P, _I, _P, _P, _I, _I, _P],
     "tff_group_rmsnorm_add": [_P, _P, _I, _Z, _P, _P, _I, _F, _P, _I, _I, _I, _P],
+    "tff_group_depth_in_norm": [_I, _I, _I, _I],
     "tff_group_rmsnorm_add_depth": [_P, _P, _I, _Z, _P, _I, _F, _P, _Z, _I, _P, _P, _I, _I, _I, _P],
     "tff_depth_average": [_P, _Z, _I, _P, _P, _P, _Z, _I, _P],
     "tff_scale_rows": [_P, _F, _Z, _P],

@@ -1396,7 +1396,7 @@ def group_rmsnorm_add(resid: torch.Tensor | None, delta, weight: torch.Tensor, g
     added into the float32 residual stream in place and the new rows are returned in ``out_dtype``
     (None: nothing is returned); without, the normed rows themselves are returned (of the rows
     ``rows`` only, where given).  ``delta`` may be what ``linear`` returns with ``partials=True``.  ``depth`` = (hist, n,
-    coef), with ``resid``: ``depth_average(hist, n, coef, resid, out_dtype)`` of the sum in the same launch."""
+    coef), with ``resid``: ``depth_average(hist, n, coef, resid, out_dtype)`` of the sum, in the same launch where that is the sooner done."""
     if isinstance(delta, PendingProduct):
         delta = delta.run()
     if isinstance(delta, ScaledRows):
