@@ -147,7 +147,11 @@ TFF_API int tff_add_rmsnorm_pair(float* resid, const float* d0, int planes0, siz
     hipStream_t s = (hipStream_t)stream;
     const size_t lds = (size_t)W * sizeof(float);
     auto ok16 = [](const void* p) { return ((uintptr_t)p % 16) == 0; };
-    const bool vec = W % 4 == 0 && plane0 % 4 == 0 && plane1 % 4 == 0 && ok16(resid) && ok16(d0) && ok16(d1) && ok16(bias) && ok16(w1) && ok16(w2) &&
+    // Rows of a few hundred elements leave most threads of the 16-byte form idle, and of its blocks 1,024 run at a time: a second, mostly empty
+    // round costs narrow rows what the form saves.  us, an element a thread / 16 bytes, with four planes: 1,200 rows of 256 4.1 / 5.9, of 1,024
+    // 7.2 / 8.1, of 1,536 12.3 / 12.0; 1,000 rows of 512 4.8 / 4.6, of 1,024 6.8 / 5.7; 2,900 of 512 10.1 / 11.9, of 1,024 18.9 / 17.7.
+    const bool pays = W >= 512 && (n <= 1024 || W >= 1536 || (W >= 1024 && (planes0 + planes1 <= 2 || n >= 2048)));
+    const bool vec = pays && W % 4 == 0 && plane0 % 4 == 0 && plane1 % 4 == 0 && ok16(resid) && ok16(d0) && ok16(d1) && ok16(bias) && ok16(w1) && ok16(w2) &&
                      ok16(out1) && ok16(out2);
 #define PN_LAUNCH(TO, NT)                                                                                              \
     (vec ? add_rmsnorm_pair_vec_kernel<TO, NT> : add_rmsnorm_pair_kernel<TO, NT>)<<<n, NT, lds, s>>>(resid, d0, planes0, plane0, d1, planes1, plane1, bias, w1, w2, eps, \
