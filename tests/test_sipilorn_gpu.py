@@ -473,14 +473,15 @@ def test_two_norms_of_one_sum_in_pieces(n, W, planes):
 
 @pytest.mark.parametrize("D,rot,pairing", [(128, 64, 0), (128, 64, 1), (64, 16, 0), (32, 8, 1), (256, 112, 0)])
 def test_projections_whose_heads_turn_in_part(D, rot, pairing):
-    """From 128 tokens on in pieces of eight elements; against the same tokens in steps of fewer: the sum of squares in another order, one
+    """From 128 tokens and 2^17 elements on in pieces of eight elements; against the same tokens in steps of fewer: the sum of squares in another order, one
     rounding to bfloat16 falls the other way now and then (2^-7 of the largest value), values the same bits."""
     ops = _ops()
     g = torch.Generator().manual_seed(D + rot)
-    T, nq, nkv, ps = 137, 5, 2, 16
+    nq, nkv, ps = 5, 2, 16
+    T = max(137, (1 << 17) // ((nq + nkv) * D) + 6)
     qkv = torch.randn(T, (nq + 2 * nkv) * D, generator=g).bfloat16().to(DEV)
     qw, kw = ((1 + 0.2 * torch.randn(D, generator=g)).to(DEV) for _ in range(2))
-    table, pos = torch.randn(200, rot // 2, 2, generator=g).to(DEV), _i32(list(range(3, T + 3)))
+    table, pos = torch.randn(T + 3, rot // 2, 2, generator=g).to(DEV), _i32(list(range(3, T + 3)))
     slots = _i32([i + 5 if i != 50 else -1 for i in range(T)])
     got = []
     for step in (T, 70):
