@@ -209,7 +209,8 @@ def test_clamps_in_the_gated_product(M, I, K, limit):
 
 @pytest.mark.parametrize("T,pairing", [(128, 0), (203, 0), (129, 1)])
 @pytest.mark.parametrize("H,G,D,ps,turn,bias,norm", [(4, 2, 128, 16, True, True, False), (9, 3, 64, 16, True, False, True), (2, 1, 24, 8, True, True, True),
-                                                     (10, 2, 256, 32, False, False, False), (16, 4, 40, 4, True, False, False)])
+                                                     (10, 2, 256, 32, False, False, False), (16, 4, 40, 4, True, False, False),
+                                                     (6, 2, 72, 16, True, True, True), (3, 1, 136, 8, True, True, False), (300, 100, 72, 8, True, False, False)])
 def test_grouped_projections_of_many_tokens(T, pairing, H, G, D, ps, turn, bias, norm):
     """From 128 tokens on in whole pieces, the values eight tokens at a time: the same bits as for the same tokens in steps of fewer, with
     slots that begin and end inside runs of eight, and tokens that write no key."""

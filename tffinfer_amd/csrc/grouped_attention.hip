@@ -266,7 +266,11 @@ TFF_API int tff_grouped_qkv_store(const float* proj, size_t row, const float* co
     const dim3 grid(T, q_blocks + kv_blocks);
     const bool wide = q_norm || k_norm || T < 128;
     auto ok16 = [](const void* p) { return ((uintptr_t)p % 16) == 0; };
-    if (T >= 128 && store && dtype == TFF_BF16 && vec && D == E && D == P && D % 8 == 0 && D <= 256 && ok16(q_norm) && ok16(k_norm) && ok16(cos_sin) &&
+    // Heads of 128 and more; of 64 and more with norms, or once their rows are some megabytes: smaller ones are a few pieces a head, and
+    // the lanes that share a head's index arithmetic are fewer.  us, an element a thread / pieces: 16 + 4 + 4 heads of 64, 1,000 tokens 6.7 / 7.2,
+    // 3,000 15.1 / 14.8, with norms 1,000 9.8 / 9.4; 20 + 20 + 20 of 40, 3,000 41 / 45, with norms 34 / 44.
+    const bool pays = D >= 128 || (D >= 64 && (wide || (long)T * (H + 2 * G) * D >= (1L << 22)));
+    if (pays && T >= 128 && store && dtype == TFF_BF16 && vec && D == E && D == P && D % 8 == 0 && D <= 256 && ok16(q_norm) && ok16(k_norm) && ok16(cos_sin) &&
         ok16(q_out) && ok16(k_cache) && ok16(v_cache) && (rot_dims == 0 || rot_dims == D)) {
         const int qk_rows = q_blocks + kv_blocks, v_rows = (int)(((long)((T + 7) / 8) * G + T - 1) / T);      // (the values' blocks fill whole rows of the grid)
         const dim3 vgrid(T, qk_rows + v_rows);
