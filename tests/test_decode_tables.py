@@ -69,6 +69,8 @@ class TableRunner:
             turns = self.tables.get(bucket)
             if turns is None:
                 turns = self.tables[bucket] = [DecodeTables(self.cache, bucket, self.max_len) for _ in range(self.ring)]
+                for i, t in enumerate(turns if self.ring > 1 else ()):
+                    t.like = turns[i - 1]
             t = turns[0]
             turns.append(turns.pop(0))
             t.fill(entries)
@@ -209,6 +211,40 @@ def test_a_step_that_failed_leaves_no_page_behind_in_a_row():
     assert cache.block_table(0, "a") != first and len(cache.block_table(0, "a")) == len(first)
     t.fill(e)
     check_rows(t, cache, e)
+
+
+def test_tables_that_take_turns_copy_a_rows_pages():
+    """Four tables in turn: a long row is looked up page by page once, the other three copy it; a request that has come back under the
+    same id is looked up again."""
+    class Pages(list):
+        reads = 0
+
+        def __getitem__(self, i):
+            got = super().__getitem__(i)
+            Pages.reads += len(got) if isinstance(i, slice) else 1
+            return got
+
+        def __iter__(self):
+            Pages.reads += len(self)
+            return super().__iter__()
+    cache = CacheManager([(0, True, FULL, None)], 8, 200, 2)
+    turns = [DecodeTables(cache, 1, 1000) for _ in range(4)]
+    for i, t in enumerate(turns):
+        t.like = turns[i - 1]
+    for life in range(2):
+        cache.add_request("a")
+        cache.reserve("a", 800)
+        cache.commit("a", 800)
+        cache.groups[0].tables["a"] = Pages(cache.groups[0].tables["a"])
+        for step in range(9):
+            cache.reserve("a", 1)
+            e = [StepEntry("a", [step], [0])]
+            Pages.reads = 0
+            turns[step % 4].fill(e)
+            assert Pages.reads > 100 if step == 0 else Pages.reads < 10, (life, step, Pages.reads)
+            check_rows(turns[step % 4], cache, e)
+            cache.commit("a", 1)
+        cache.release("a")
 
 
 def test_lives_are_unique():

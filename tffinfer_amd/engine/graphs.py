@@ -97,6 +97,9 @@ class DecodeTables:
         hv[o[3]:o[3] + B + 1] = np.arange(B + 1)    # cu_tokens
         hv[o[7]:o[7] + B] = np.arange(B)            # logit rows: every row
         hv[o[8]:o[8] + B] = -1                      # no-slot mapping
+        #: other tables of this layout, which the step before filled where several take turns: a row that is to be written anew and
+        #: holds the same stay there is copied from them as far as they go (a page from a list costs twenty times as much)
+        self.like: DecodeTables | None = None
         self._row_state = [None] * B                # (request, life, table lengths) last written per row
         self.host_start_pos, self.host_state_slots = [], []    # of the live rows of the last fill
         self.variant = (False, ())                  # (some row has several runs, per group: dealt for blocks) at the last fill
@@ -132,7 +135,7 @@ class DecodeTables:
 
     def fill(self, entries) -> None:
         """Writes the step's tables for ``entries`` (one token each, pages reserved)."""
-        cache, o, hv = self.cache, self.offs, self.hv
+        cache, o, hv, like = self.cache, self.offs, self.hv, self.like
         ps = cache.page_size
         R = len(entries)
         if R > self.B:
@@ -149,6 +152,9 @@ class DecodeTables:
             hv[o[5] + r] = P + 1
             hv[o[6] + r] = cache.slot(e.req)
             prev = self._row_state[r]
+            theirs = like._row_state[r] if like is not None else None
+            if theirs is not None and (theirs[0] != e.req or theirs[1] != life):
+                theirs = None
             lens = []
             for gi, w in enumerate(self.widths):
                 table = cache.block_table(gi, e.req)
@@ -163,7 +169,9 @@ class DecodeTables:
                     if n > old:
                         hv[base + old:base + n] = [p if p >= 0 else 0 for p in table[old:]]
                 else:
-                    hv[base:base + n] = [p if p >= 0 else 0 for p in table]
+                    have = 0 if theirs is None else min(theirs[2][gi], n)
+                    hv[base:base + have] = like.hv[base:base + have] if have else 0
+                    hv[base + have:base + n] = [p if p >= 0 else 0 for p in table[have:]]
                     if old > n:
                         hv[base + n:base + old] = 0
                 lens.append(n)
@@ -211,6 +219,8 @@ class DecodeGraph:
         # since the buffer's last turn (64 rows of 40,960 tokens are 655 KB, which no step copies on the host).
         self._pinned = PinnedTables(total)
         self._turns = [DecodeTables(cache, B, runner.max_model_len, buf.numpy()) for buf in self._pinned.bufs]
+        for i, t in enumerate(self._turns):
+            t.like = self._turns[i - 1]
         self.tables, self._host = self._turns[0], self._pinned.bufs[0]       # those of the last step
         self.widths = self.tables.widths
         self.offs = o = self.tables.offs
