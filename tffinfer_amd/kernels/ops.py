@@ -1630,8 +1630,8 @@ MIXED_ATTENTION_BLOCKS = 512
 MIXED_ATTENTION_Q16_TOKENS = 64
 #: up to so many tokens times the keys that one of them can see, and up to 112 tokens (88 where a wave has more than one kv head), such a
 #: step takes a block a token all the same: blocks of sixteen queries are few then, and none is through its first 64 keys before some
-#: 20 us.  us, a block a token / sixteen queries a block: prompts of 64 and 100 tokens, 32 heads of 128 on 8 kv heads 12.9 / 32.2 and
-#: 19.5 / 32.7, 20 of 64 on 5 9.9 / 27.1 and 12.1 / 27.5, 16 of 128 on 16 17.6 / 23.9 and 23.6 / 24.0; of 128 tokens, the last 27.5 / 24.3;
+#: 20 us.  us, a block a token / sixteen queries a block: prompts of 64 and 100 tokens, 32 heads of 128 on 8 kv heads 13.3 / 33.7 and
+#: 20.2 / 34.4, 20 of 64 on 5 10.1 / 29.2 and 12.3 / 29.5, 16 of 128 on 16 17.9 / 24.3 and 24.7 / 24.8;
 #: 64 behind 1,000 others 137 / 64; 200 under a window of 37 47 / 25
 MIXED_ATTENTION_Q16_KEYS = 12500
 #: blocks that kernel's items are spread over where they are fewer (a block a CU)
