@@ -480,6 +480,20 @@ def test_cases_of_few_rows_cover_every_tile():
     assert {((r, c), glu) for r in (32, 64) for c in (128, 256) for glu in (False, True)} <= tiles, tiles
 
 
+@pytest.mark.parametrize("units", [1, 2, 3, 4, 5, 6, 9])
+@pytest.mark.parametrize("M,N", [(2304, 2100), (2000, 6144), (300, 4096), (60, 2048), (20, 1030)])
+def test_linear_of_few_units_of_k(M, N, units):
+    """The four-wave kernel's rings of copies (three units of A, four or five k-tiles of W) with fewer, as many and more units of K
+    than they hold: the copies past the end repeat the last unit and nothing reads them."""
+    ops = _ops()
+    K = 64 * units
+    g = torch.Generator().manual_seed(N + units)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(N, K, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
+    y = ops.linear(x, ops.pack_weight(w), out_dtype=torch.float32)
+    _close(y, ops.linear(x.float(), w.float()), 3e-5, "product")
+
+
 @pytest.mark.parametrize("M,N,K", [(2600, 6144, 264), (4500, 520, 200), (1100, 300, 96), (9000, 130, 64),
                                    (2304, 2100, 72)])
 def test_linear_with_many_row_tiles(M, N, K):

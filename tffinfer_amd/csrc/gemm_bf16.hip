@@ -389,9 +389,21 @@ static int launch_async_g(const bf16_t* A, const bf16_t* Wp, void* C, int M, int
 // packed (NWS k-tiles in LDS).  Within a copy's 1 KB lane i lands at byte 16 i; it fetches row
 // i / 8, 16-byte chunk (i % 8) ^ (i / 8), so that the sixteen rows an MFMA operand is made of are
 // read back from different banks.
-// In k-tile t (32 k) a wave issues, if t is even, its copies of A unit t / 2 + 2, and its copies of W
-// tile t + NWS - 1; at the start of t it needs W tile t + 1 and the A unit of t + 1, issued in tile
-// t - NWS + 2 at the latest.  Copies complete in the order issued, so the wait is by count.
+// In k-tile t (32 k) a wave copies half of A unit u + 3 (t = 2 u + 1 the first, t = 2 u + 2 the second half) and W tile
+// t + NWS: into the slots of the unit and tile whose fragments were last read in tile t - 1 or before.  Every wave waits
+// for its own reads before the barrier at the start of t, which makes those slots free; the last quarter of a tile's
+// MFMAs has no reads, so the reads have come back by then.  At the start of t it needs W tile t + 1 and the A unit of
+// t + 1, issued in tiles t - NWS + 1 and t - 3 at the latest.  Copies complete in the order issued, so the wait is by count.
+//
+// What bounds the loop of one wave a SIMD is the issue of what stands between the MFMAs: a wave issues an instruction
+// every four cycles and an MFMA takes sixteen, so three others fit behind each and the fourth leaves the matrix core
+// idle.  With a 64-bit address a copy that each walks k, its LDS address and the ring's bookkeeping a tile took 1,340
+// cycles (no copies at all: 1,093, whatever the clock; a tile of the same reads and MFMAs whose copies do not walk: 1,180).
+// So all copies of an operand share one address, the lane's part of it in a register that never changes; a copy is an
+// s_add into M0 before an MFMA and the load after it; and what moves the rings and addresses on is dealt over the gaps
+// behind a tile's last copies: 1,110 cycles.  The clock falls with the idle cycles (1.80 -> 1.72 GHz: the power limit), so
+// the time falls by less: us before / now, 2,048 rows of the 8B shape: QKV 77.0 / 72.9, O 57.8 / 53.0, gate+up 299 / 284,
+// down 159 / 145; 16,384 rows, gate+up 2,343 / 2,221; 600 rows of 2,048: O 16.0 / 15.2, gate+up 32.5 / 29.3.
 // K a multiple of 64; a split of K takes whole units.
 // A wave's 128 rows x OW column groups of results go out through LDS, so that a store instruction
 // writes whole rows instead of 16 rows x 8 or 16 bytes: a lane leaves its four columns of a row in
@@ -489,14 +501,18 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     static_assert(WTM == 8 || (WGM == 1 && (WTM == 4 || WTM == 2)), "fewer rows a wave only with the waves side by side");
     constexpr int BM = WGM * WTM * 16, BN = WGN * WTN * 16;
     constexpr int WF = BN / 16;                       // W fragments a k-tile, 1 KB each
+    static_assert(WF % NW == 0, "every wave copies as many fragments of W");
     constexpr int ACP = BM / 8;                       // A copies a unit, 1 KB each
-    constexpr int LPA = ACP / NW, LPW = (WF + NW - 1) / NW;
+    constexpr int LPA = ACP / NW, LPW = WF / NW;
     constexpr int NMF = WTM * WTN;                    // MFMAs a k-tile
-    constexpr int RPM = NMF / (WTM + WTN);            // a read after every RPM MFMAs
-    constexpr int CPM = NMF / (LPA + LPW);            // a copy after every CPM MFMAs
-    constexpr int D = NWS - 1;                        // W is copied D tiles ahead
-    static_assert(D == 3 || D == 4, "the waits below are written for three or four tiles ahead");
-    static_assert(RPM >= 1 && CPM >= 1, "not enough MFMAs to hide the reads and copies");
+    constexpr int RPM = NMF * 3 / 4 / (WTM + WTN) > 0 ? NMF * 3 / 4 / (WTM + WTN) : 1;   // a read after every RPM MFMAs
+    constexpr int LPA_O = (LPA + 1) / 2, LPA_E = LPA / 2;   // copies of A in an odd and an even k-tile
+    constexpr int CPM = (NMF - 4) / (LPA_O + LPW) > 0 ? (NMF - 4) / (LPA_O + LPW) : 1;   // a copy with every CPM-th MFMA
+    static_assert(NWS == 4 || NWS == 5, "the waits below are written for four or five tiles ahead");
+    static_assert(RPM * (WTM + WTN) <= NMF, "a tile's MFMAs hold the reads of the next");
+    constexpr int UP0 = NMF >= 8 ? NMF - 4 : NMF - 1, UP1 = NMF >= 8 ? NMF - 3 : NMF - 1;   // the gaps that move rings and addresses on
+    constexpr int UP2 = NMF >= 8 ? NMF - 2 : NMF - 1, UP3 = NMF - 1;
+    static_assert(RPM >= 1 && CPM * (LPA_O + LPW) <= UP1, "not enough MFMAs to hide the reads and copies");
     constexpr unsigned A_UNIT = ACP * 1024u, W_TILE = WF * 1024u, W_BASE = NA * A_UNIT;
     static_assert(W_BASE + NWS * W_TILE <= 160 * 1024, "LDS");
     __shared__ __attribute__((aligned(1024))) char smem[W_BASE + NWS * W_TILE];
@@ -565,69 +581,41 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
             for (int j = vec_end; j < sc.count; ++j) row_ss += sp[j];
     }
 
-    // this wave's copies: of an A unit the copies wave + 4 c, of a W tile the fragments wave + 4 c
-    unsigned long long abase[LPA], wbase[LPW];
-    unsigned aoff[LPA];
-    unsigned wlds[LPW];
-    const unsigned woff = lane * 16;
+    // this wave's copies: of an A unit the copies wave + 4 c, of a W tile the fragments wave + 4 c; a lane's bytes from the operand's address on
+    const unsigned long long a0 = (unsigned long long)(A + (size_t)m0 * lda + (size_t)kt0 * 32);
+    const unsigned long long w0 = (unsigned long long)(Wp + ((size_t)(n0 / 16) * KB + kt0) * 512);
+    unsigned aoff[LPA], woff[LPW];
 #pragma unroll
-    for (int c = 0; c < LPA; ++c) {
-        const int cp = wave + NW * c;
-        const int row0 = min(m0 + cp * 8, M - 1);
-        const int row = min(m0 + cp * 8 + (lane >> 3), M - 1);
-        abase[c] = (unsigned long long)(A + (size_t)row0 * lda + (size_t)kt0 * 32);
-        aoff[c] = (unsigned)(row - row0) * (unsigned)lda * 2u + (unsigned)(((lane & 7) ^ (lane >> 3)) * 16);
-    }
+    for (int c = 0; c < LPA; ++c)
+        aoff[c] = (unsigned)(min(m0 + (wave + NW * c) * 8 + (lane >> 3), M - 1) - m0) * (unsigned)lda * 2u + (unsigned)(((lane & 7) ^ (lane >> 3)) * 16);
 #pragma unroll
-    for (int c = 0; c < LPW; ++c) {
-        const int f = min(wave + NW * c, WF - 1);     // the last waves copy the last fragment once more
-        const int nb = min(n0 / 16 + f, NB - 1);
-        wbase[c] = (unsigned long long)(Wp + ((size_t)nb * KB + kt0) * 512);
-        wlds[c] = W_BASE + (unsigned)f * 1024u;
-    }
-    const unsigned smem_addr = (unsigned)(size_t)(lds_ptr_t)smem;
-    // copies past the end repeat the last unit or tile, so that the counts in flight stay the same
-    int a_next = u0, w_next = kt0;                    // the next unit and tile to copy
-    unsigned a_ws = 0, w_ws = 0;                      // where they go: byte offsets of the slots
-#define W4_COPY_A(c)                                                                                \
-    {                                                                                               \
-        copy16_to_lds_sbase(abase[c], aoff[c], smem_addr + a_ws + (unsigned)(wave + NW * (c)) * 1024u); \
-        abase[c] += a_next + 1 < u1 ? 128ull : 0ull;                                                \
-    }
-#define W4_A_ISSUED()                                                                               \
-    {                                                                                               \
-        a_next += a_next + 1 < u1 ? 1 : 0;                                                          \
-        a_ws = a_ws + A_UNIT == NA * A_UNIT ? 0u : a_ws + A_UNIT;                                   \
-    }
-#define W4_COPY_W(c)                                                                                \
-    {                                                                                               \
-        copy16_to_lds_sbase(wbase[c], woff, smem_addr + w_ws + wlds[c]);                            \
-        wbase[c] += w_next + 1 < kt1 ? 1024ull : 0ull;                                              \
-    }
-#define W4_W_ISSUED()                                                                               \
-    {                                                                                               \
-        w_next += w_next + 1 < kt1 ? 1 : 0;                                                         \
-        w_ws = w_ws + W_TILE == NWS * W_TILE ? 0u : w_ws + W_TILE;                                  \
-    }
+    for (int c = 0; c < LPW; ++c)
+        woff[c] = (unsigned)(min(n0 / 16 + wave + NW * c, NB - 1) - n0 / 16) * (unsigned)KB * 1024u + (unsigned)lane * 16u;
+    const unsigned lds_wave = (unsigned)(size_t)(lds_ptr_t)smem + (unsigned)wave * 1024u;
     if (u0 < u1) {   // (a part of a split K that holds no unit only stores its zeros)
-        // the tiles before the first, in the order of the loop: t = -4 .. -1
+        // copies past the end repeat the last unit or tile, so that the counts in flight stay the same
+        const unsigned a_end = (unsigned)(u1 - u0 - 1) * 128u, w_end = (unsigned)(kt1 - kt0 - 1) * 1024u;
+        // the tiles before the first, in the order of the loop: t = -5 .. -1
 #pragma unroll
-        for (int t = -4; t < 0; ++t) {
-            if ((t & 1) == 0) {
+        for (int t = -5; t < 0; ++t) {
+            const int u = (t + 5) / 2;                    // unit 0 in tiles -5 and -4, 1 in -3 and -2, the first half of 2 in -1
 #pragma unroll
-                for (int c = 0; c < LPA; ++c) W4_COPY_A(c)
-                W4_A_ISSUED()
-            }
-            if (t + D >= 0) {
+            for (int c = (t & 1) ? 0 : LPA_O; c < ((t & 1) ? LPA_O : LPA); ++c)
+                copy16_to_lds_sbase(a0 + min((unsigned)u * 128u, a_end), aoff[c], lds_wave + (unsigned)u * A_UNIT + (unsigned)c * 4096u);
+            if (t + NWS >= 0) {
 #pragma unroll
-                for (int c = 0; c < LPW; ++c) W4_COPY_W(c)
-                W4_W_ISSUED()
+                for (int c = 0; c < LPW; ++c)
+                    copy16_to_lds_sbase(w0 + min((unsigned)(t + NWS) * 1024u, w_end), woff[c],
+                                        lds_wave + W_BASE + (unsigned)(t + NWS) * W_TILE + (unsigned)c * 4096u);
             }
         }
-        // what may still be in flight at the start of tile t: the copies of tiles t - D + 2 .. t - 1
-        constexpr int EVEN = LPA + LPW, ODD = LPW;
-        constexpr int FLY_E = D == 4 ? EVEN + ODD : ODD;  // t even: t - 1 is odd
-        constexpr int FLY_O = D == 4 ? EVEN + ODD : EVEN;
+        unsigned a_ko = min(2u * 128u, a_end), w_ko = min((unsigned)NWS * 1024u, w_end);   // the unit and tile copied next, in bytes of k
+        unsigned long long a_at = a0 + a_ko, w_at = w0 + w_ko;
+        unsigned a_to = lds_wave + 2u * A_UNIT, w_to = lds_wave;   // where they go
+        // what may still be in flight at the start of tile t: the copies of the last two tiles, of three where W is that far ahead
+        constexpr int ODD = LPA_O + LPW, EVEN = LPA_E + LPW;
+        constexpr int FLY_E = NWS == 5 ? 2 * ODD + EVEN : ODD + EVEN;   // t even: t - 1 is odd
+        constexpr int FLY_O = ODD + EVEN;
         // a lane's 16 bytes of an A operand: row fr of 16, chunk h * 4 + fg of the row's 8
         unsigned a_rd[2];
 #pragma unroll
@@ -635,8 +623,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
             a_rd[h] = (unsigned)(wm * WTM * 2 + (fr >> 3)) * 1024u + (unsigned)(((fr & 7) * 8 + ((h * 4 + fg) ^ (fr & 7))) * 16);
         const unsigned w_rd = W_BASE + (unsigned)(wn * WTN) * 1024u + lane * 16;
         unsigned a_rs = 0, w_rs = W_TILE;                 // slots of the tile whose fragments are read next (kt0 + 1)
-        // before the first tile: A unit u0 and W tile kt0, issued in tile -4 and tile -D
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(D == 4 ? LPA + 3 * LPW : LPA + 2 * LPW));
+        // before the first tile: A unit u0 and W tile kt0, issued in tile -4 at the latest
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * ODD + EVEN));
         __syncthreads();
         bf16x8 fw[2][WTN], fa[2][WTM];
 #pragma unroll
@@ -645,33 +633,36 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
         for (int jj = 0; jj < WTM; ++jj) fa[0][jj] = *reinterpret_cast<const bf16x8*>(smem + a_rd[0] + jj * 2048);
 
         // a k-tile's MFMAs with the LDS reads of the next tile and the copies of later ones between them
+        const char* a_src = smem + a_rd[1];
+        const char* w_src = smem + w_rd + w_rs;
 #define W4_TILE(h)                                                                                  \
         {                                                                                           \
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm((h) ? FLY_O : FLY_E));                             \
+            constexpr int NA_C = (h) ? LPA_O : LPA_E, A_C0 = (h) ? 0 : LPA_O, NC = NA_C + LPW;      \
+            __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm((h) ? FLY_O : FLY_E));                       \
             asm volatile("s_barrier" ::: "memory");                                                 \
-            const char* na = smem + a_rs + a_rd[(h) ^ 1];                                           \
-            const char* nw = smem + w_rs + w_rd;                                                    \
             _Pragma("unroll") for (int i = 0; i < WTN; ++i)                                         \
                 _Pragma("unroll") for (int jj = 0; jj < WTM; ++jj) {                                \
                     const int q = i * WTM + jj;                                                     \
-                    mfma_acc(acc[i][jj], fw[h][i], fa[h][jj]);                                      \
+                    const int cp = q % CPM == CPM - 1 && q / CPM < NC ? q / CPM : -1;               \
+                    if (cp >= 0 && cp < NA_C)                                                       \
+                        mfma_acc_copy(acc[i][jj], fw[h][i], fa[h][jj], a_to, (unsigned)(A_C0 + cp) * 4096u, aoff[cp >= 0 && cp < NA_C ? A_C0 + cp : 0], a_at); \
+                    else if (cp >= 0)                                                               \
+                        mfma_acc_copy(acc[i][jj], fw[h][i], fa[h][jj], w_to, W_BASE + (unsigned)(cp - NA_C) * 4096u, woff[cp >= NA_C ? cp - NA_C : 0], w_at); \
+                    else mfma_acc(acc[i][jj], fw[h][i], fa[h][jj]);                                 \
                     if (q % RPM == RPM - 1 && q / RPM < WTN + WTM) {                                \
                         const int rd = q / RPM;                                                     \
-                        if (rd < WTM) fa[(h) ^ 1][rd < WTM ? rd : 0] = *reinterpret_cast<const bf16x8*>(na + rd * 2048); \
-                        else fw[(h) ^ 1][rd >= WTM ? rd - WTM : 0] = *reinterpret_cast<const bf16x8*>(nw + (rd - WTM) * 1024); \
+                        if (rd < WTM) fa[(h) ^ 1][rd < WTM ? rd : 0] = *reinterpret_cast<const bf16x8*>(a_src + rd * 2048); \
+                        else fw[(h) ^ 1][rd >= WTM ? rd - WTM : 0] = *reinterpret_cast<const bf16x8*>(w_src + (rd - WTM) * 1024); \
                     }                                                                               \
-                    if (q % CPM == CPM - 1) {                                                       \
-                        const int cp = q / CPM;                                                     \
-                        if ((h) == 0) {                                                             \
-                            if (cp < LPA) W4_COPY_A(cp < LPA ? cp : 0)                              \
-                            else if (cp < LPA + LPW) W4_COPY_W(cp >= LPA && cp < LPA + LPW ? cp - LPA : 0) \
-                        } else if (cp < LPW) W4_COPY_W(cp < LPW ? cp : 0)                           \
-                    }                                                                               \
+                    if (q == UP0) w_ko = step_to(w_ko, 1024u, w_end);                           \
+                    if (q == UP1) { w_at = w0 + w_ko; w_to = lds_wave + w_rs; }                 \
+                    if (q == UP2) w_rs = ring_next<W_TILE, NWS * W_TILE>(w_rs);                 \
+                    if ((h) == 0 && q == UP1) a_ko = step_to(a_ko, 128u, a_end);                \
+                    if ((h) == 0 && q == UP2) { a_at = a0 + a_ko; a_to = lds_wave + a_rs; }     \
+                    if ((h) == 0 && q == UP3) a_rs = ring_next<A_UNIT, NA * A_UNIT>(a_rs);      \
                 }                                                                                   \
-            if ((h) == 0) W4_A_ISSUED()                                                             \
-            W4_W_ISSUED()                                                                           \
-            if ((h) == 0) a_rs = a_rs + A_UNIT == NA * A_UNIT ? 0u : a_rs + A_UNIT;                 \
-            w_rs = w_rs + W_TILE == NWS * W_TILE ? 0u : w_rs + W_TILE;                              \
+            a_src = smem + a_rs + a_rd[h];                                                          \
+            w_src = smem + w_rs + w_rd;                                                             \
         }
         // tile 2 u reads its successor from its own unit, tile 2 u + 1 from the next: a_rs moves on after an even tile
         for (int kt = kt0; kt < kt1; kt += 2) {
@@ -680,10 +671,6 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
         }
     }
 #undef W4_TILE
-#undef W4_COPY_A
-#undef W4_COPY_W
-#undef W4_A_ISSUED
-#undef W4_W_ISSUED
     // every copy has landed and every read of LDS has come back, in every wave: LDS is free for the results
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");   // (and the last MFMAs have written their accumulators)
@@ -733,7 +720,8 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
     const long TM = (M + BM - 1) / BM, TN = (N + BN - 1) / BN;
     const long tiles = 8 * ((TM / 8) * TN + ((TM % 8) * TN + 7) / 8);   // eight equal shares, see the kernel
     TFF_REQUIRE(tiles < (1L << 31), "gemm: too many tiles for M=%d N=%d", M, N);
-    TFF_REQUIRE((size_t)15 * lda * 2 + 128 < (1ull << 32), "gemm: row stride %d too large", lda);
+    TFF_REQUIRE((size_t)(BM - 1) * lda * 2 + 128 < (1ull << 32) && (size_t)(BN / 16) * KB * 1024 < (1ull << 32),
+                "gemm: rows of %d elements at a stride of %d are too long", K, lda);
     const dim3 grid((unsigned)tiles, 1, splits);
     // the blocks of a split K leave plain float32 sums, plane by plane; a gate is applied when they are added up
     if (ex.plane_cols) {
