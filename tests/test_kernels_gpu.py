@@ -1153,6 +1153,34 @@ def test_attention_mfma_blocks_of_256_columns(nq, nkv, d, ps, window, bins):
             _close(out.reshape(T, nq, d)[mine], ref, ATTN_TOL, f"blocks of 256 columns, request {r}")
 
 
+@pytest.mark.parametrize("wide,sink", [(1.0, None), (200.0, None), (1.0, 45.0), (200.0, 0.5)])
+@pytest.mark.parametrize("nq,nkv,d,ps,window,groups,entries", [
+    (8, 2, 128, 16, 0, 1, [(0, 700), (333, 200), (5, 1), (1000, 130)]),      # whole and part blocks of columns, odd and even numbers of slices
+    (8, 2, 128, 16, 0, 2, [(0, 700), (333, 200), (5, 1), (1000, 130)]),
+    (5, 1, 128, 32, 77, 1, [(0, 333), (200, 64), (31, 33)]),                 # windows that begin within a slice: first slices without a key
+    (5, 1, 128, 8, 77, 2, [(0, 333), (200, 64), (31, 33)]),
+    (40, 2, 128, 64, 0, 2, [(0, 2), (0, 31), (40, 32)]),                     # one slice, or two: a group with none
+    (2, 1, 128, 8, 0, 1, [(16400, 40)]),                                     # more pages than LDS holds
+    (2, 1, 128, 8, 0, 2, [(16400, 40)]),
+    (3, 1, 256, 16, 0, 1, [(0, 300), (90, 61)]),
+    (6, 1, 256, 64, 40, 1, [(0, 257), (300, 31)])])
+def test_attention_of_prompts_on_blocks_of_four_waves(nq, nkv, d, ps, window, groups, entries, wide, sink):
+    """Portions on four waves of several column tiles.  ``wide``: queries so long that the scores exceed those of a column's first slice
+    by far more than float32 holds as a power of two: the block repeats its item against the largest score.  ``sink``: a sink among
+    the scores, or so far above them that a sum against the largest score would not hold it."""
+    ops = _ops()
+    batch, kv, ks, vs, positions, token_req = _fake_step(entries, ps, nkv, d, torch.bfloat16, seed=nq * 7 + d + ps)
+    T = batch.num_tokens
+    q = (wide * torch.randn(T, nq * d, generator=torch.Generator().manual_seed(5))).to(torch.bfloat16).to(DEV)
+    scale = 1 / math.sqrt(d)
+    sinks = None if sink is None else torch.linspace(sink / 2, sink * 2, nq, device=DEV)
+    out = torch.full((T, nq * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.attention_prompt(q, out, nq, nkv, d, kv, batch, window, scale, sinks, "all", groups)
+    gen = ops.attention_generic(q, nq, nkv, d, kv.k_cache, kv.v_cache, kv.block_tables, batch.token_req, batch.positions, window, scale,
+                                sinks=sinks)
+    _close(out, gen.double(), ATTN_TOL, "blocks of four waves against the general kernel")
+
+
 def test_attention_mfma_picks_its_blocks_by_the_work():
     """A prompt of 2,048 tokens goes to the blocks of 128 columns, one of 32,768 tokens to those
     of 256; head sizes beyond 128 never do.  A prompt of 6,000 tokens through either gives

@@ -165,6 +165,15 @@ TFF_API int tff_attention_mfma(const void* q, int q_stride, void* out, float* pa
                                int nq, int nkv, int d, int page_size, int num_pages, int window,
                                float scale, const float* sinks, float softcap, const int32_t* pool_tables, int pt_stride,
                                int pool, tff_stream_t stream);
+// The same for long portions, without a cap on the scores and pooled blocks of keys, on blocks of four waves of several column
+// tiles (attention_prompt.hip): head size 128 with work items of 256 columns (key_groups 1) or of 128 columns whose slices
+// two groups of two waves share (2), head size 256 with items of 128 columns (1): tff_attention_prompt_cols, 0: not built.
+TFF_API int tff_attention_prompt_cols(int d, int key_groups);
+TFF_API int tff_attention_prompt(const void* q, int q_stride, void* out, const void* k_cache, const void* v_cache,
+                                 const int32_t* block_tables, int bt_stride, const int32_t* cu_tokens, const int32_t* start_pos,
+                                 const int32_t* work, int num_work, const int32_t* block_items, int num_blocks, int key_groups,
+                                 int nq, int nkv, int d, int page_size, int num_pages, int window, float scale, const float* sinks,
+                                 tff_stream_t stream);
 // Decoding steps (every entry brings one token), bfloat16, from the fused projection's output:
 // row r of qkv ([R, (nq + 2 nkv) d], q heads first, then k, then v) is token r.  The kernel
 // does what tff_qk_norm_rope_kv and tff_attention_mfma do one after the other, in one pass:

@@ -6,7 +6,7 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
 from .build import ensure_built
 
-ABI_VERSION = 47
+ABI_VERSION = 48
 
 
 class KernelLibraryError(RuntimeError):
@@ -64,6 +64,8 @@ _SIGNATURES = {
     "tff_attention_mfma_supported": [_I, _I],
     "tff_attention_mfma": [_P, _I, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I,
                            _I, _I, _I, _I, _I, _I, _F, _P, _F, _P, _I, _I, _P],
+    "tff_attention_prompt_cols": [_I, _I],
+    "tff_attention_prompt": [_P, _I, _P, _P, _P, _P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _P, _P],
     "tff_attention_decode_fused": [_P, _I, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _F, _P, _I, _I,
                                    _I, _I, _I, _I, _I, _I, _I, _I, _F, _P],
     "tff_attention_decode_runs": [_P, _I, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _F, _P, _I, _I,

@@ -918,6 +918,10 @@ def attention_mfma(q: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, window
                 cache["single_rows"] = _staging.send(q.device, [np.asarray([(r, cu[r]) for r in single], dtype=np.int32)])[0]
             sp = splits if splits is not None else pick_splits(work.shape[0] * nkv, reach)
             launch(work, work.shape[0], None, 0, 1, 16, sp, cache["single_rows"])
+    if cols == 128 and d in PROMPT_HEAD_SIZES and not pool and softcap == 0.0 and block_cols is None:
+        groups = 1 if d > 128 else key_groups or _prompt_key_groups(batch, G, nkv, int(window), q.device, which)
+        attention_prompt(q, out, nq, nkv, d, kv, batch, int(window), scale, sinks, which, groups, block_bins)
+        return out
     if cols == 128:
         bcols = 128 if pool else block_cols or _pick_block_cols(batch, G, nkv, int(window), q.device, which, d)
         if bcols == 256:
@@ -937,6 +941,54 @@ def attention_mfma(q: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, window
         work = _attention_work(batch, G, cols, q.device, which)
         launch(work, work.shape[0], None, 0, 1, cols, 1)
     return out
+
+
+#: head sizes of :func:`attention_prompt`
+PROMPT_HEAD_SIZES = (128, 256)
+
+
+def _prompt_key_groups(batch, G: int, nkv: int, window: int, device, which: str) -> int:
+    """One group of four waves on items of 256 columns, or two of two waves that share the slices of items of 128, for heads of 128: by
+    what the block with the most to do takes.  A step (a slice of an item, of two slices with two groups) is some 0.82 and 0.90 us,
+    what an item has before its first and after its last step 7 and 10 us (measured with 32 query and 8 key heads, one / two
+    groups, us: 901 tokens 33 / 25, 1,500 47 / 38, 2,048 61 / 52, 3,000 88 / 100, 4,096 141 / 165, 16,384 1,793 / 2,024; 3,001 and
+    1,700 tokens of 16 and 4 heads in a window of 1,024 45 / 61)."""
+    cache = getattr(batch, "_attn_work", None)
+    if cache is None:
+        cache = batch._attn_work = {}
+    key = ("prompt_groups", G, nkv, window, which)
+    if key not in cache:
+        cu, P = batch.host_cu_tokens, batch.host_start_pos
+        slices = []
+        for r in _entries(batch, which):
+            ncols = (cu[r + 1] - cu[r]) * G
+            for c0 in range(0, ncols, 256):
+                first, last = P[r] + c0 // G, P[r] + (min(c0 + 256, ncols) - 1) // G
+                slices.append(last // 32 - (max(0, first - window + 1) // 32 if window > 0 else 0) + 1)
+        num_cus = _num_cus(device) if torch.device(device).type == "cuda" else 256
+        bins, most, total = max(1, num_cus // max(1, nkv)), max(slices), sum(slices)
+        one = 0.82 * max(most, total / bins) + 7.0 * -(-len(slices) // bins)
+        two = 0.90 * max(most / 2, total / bins) + 10.0 * -(-2 * len(slices) // bins)
+        cache[key] = 1 if one <= two else 2
+    return cache[key]
+
+
+def attention_prompt(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, window: int, scale: float,
+                     sinks: torch.Tensor | None, which: str, key_groups: int, bins: int | None = None) -> None:
+    """The portions of a step on blocks of four waves of several column tiles (attention_prompt.hip), one block a CU.  ``attention_mfma``
+    has checked the operands."""
+    L = _lib.load()
+    cols = L.tff_attention_prompt_cols(d, key_groups)
+    if not cols:
+        raise _lib.KernelError(f"attention: no blocks of long portions for a head size of {d} with {key_groups} key groups")
+    work, block_items, num_blocks, _ = _attention_block_work(batch, nq // nkv, nkv, int(window), q.device, cols=cols,
+                                                             bins=bins or max(1, _num_cus(q.device) // max(1, nkv)), which=which,
+                                                             key_groups=key_groups, head_dim=d)
+    _lib.check(L.tff_attention_prompt(
+        q.data_ptr(), q.stride(0), out.data_ptr(), kv.k_cache.data_ptr(), kv.v_cache.data_ptr(), kv.block_tables.data_ptr(),
+        kv.block_tables.stride(0), batch.cu_tokens.data_ptr(), batch.start_pos.data_ptr(), work.data_ptr(), work.shape[0],
+        block_items.data_ptr(), num_blocks, key_groups, nq, nkv, d, kv.k_cache.shape[2], kv.k_cache.shape[0], int(window), float(scale),
+        _ptr(sinks), _stream()))
 
 
 def decode_fused_supported(qkv: torch.Tensor, d: int, page_size: int, cos_sin, pairing: int, batch) -> bool:
