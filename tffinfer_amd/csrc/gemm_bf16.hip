@@ -404,6 +404,8 @@ static int launch_async_g(const bf16_t* A, const bf16_t* Wp, void* C, int M, int
 // behind a tile's last copies: 1,110 cycles.  The clock falls with the idle cycles (1.80 -> 1.72 GHz: the power limit), so
 // the time falls by less: us before / now, 2,048 rows of the 8B shape: QKV 77.0 / 72.9, O 57.8 / 53.0, gate+up 299 / 284,
 // down 159 / 145; 16,384 rows, gate+up 2,343 / 2,221; 600 rows of 2,048: O 16.0 / 15.2, gate+up 32.5 / 29.3.
+// Before its first tile a block sets its accumulators while the first copies are on their way (set twice before and behind
+// them, 512 instructions, a product of 600 rows of 6,144 took 27.9 us, now 26.7; 16,384 rows, gate+up 2,221 / 2,213).
 // K a multiple of 64; a split of K takes whole units.
 // A wave's 128 rows x OW column groups of results go out through LDS, so that a store instruction
 // writes whole rows instead of 16 rows x 8 or 16 bytes: a lane leaves its four columns of a row in
@@ -549,18 +551,14 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     const int u1 = min(nu, u0 + u_per);
     const int kt0 = 2 * u0, kt1 = 2 * u1;
 
-    floatx4 acc[WTN][WTM];
+    floatx4 start[WTN];      // what the accumulators start from
 #pragma unroll
-    for (int i = 0; i < WTN; ++i)
-#pragma unroll
-        for (int jj = 0; jj < WTM; ++jj) acc[i][jj] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < WTN; ++i) start[i] = floatx4{0.f, 0.f, 0.f, 0.f};
     if (bias && blockIdx.z == 0) {
 #pragma unroll
-        for (int i = 0; i < WTN; ++i) {
-            const floatx4 b = bias4(bias, n0 + (wn * WTN + i) * 16 + fg * 4, NB);
+        for (int i = 0; i < WTN; ++i) start[i] = bias4(bias, n0 + (wn * WTN + i) * 16 + fg * 4, NB);
 #pragma unroll
-            for (int jj = 0; jj < WTM; ++jj) acc[i][jj] = b;
-        }
+        for (int i = 0; i < WTN; ++i) asm volatile("" : "+v"(start[i]));      // (here, before the copies, which the compiler does not see)
     }
     // (a lane's results are four columns of row fr of each row group: of row fr itself in the first,
     // the only one that counts with up to 16 rows; the four lanes of a row share out its sums)
@@ -592,6 +590,16 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     for (int c = 0; c < LPW; ++c)
         woff[c] = (unsigned)(min(n0 / 16 + wave + NW * c, NB - 1) - n0 / 16) * (unsigned)KB * 1024u + (unsigned)lane * 16u;
     const unsigned lds_wave = (unsigned)(size_t)(lds_ptr_t)smem + (unsigned)wave * 1024u;
+    floatx4 acc[WTN][WTM];
+    auto start_acc = [&]() {
+#pragma unroll
+        for (int i = 0; i < WTN; ++i)
+#pragma unroll
+            for (int jj = 0; jj < WTM; ++jj) {
+                acc[i][jj] = start[i];
+                asm volatile("" : "+a"(acc[i][jj]));
+            }
+    };
     if (u0 < u1) {   // (a part of a split K that holds no unit only stores its zeros)
         // copies past the end repeat the last unit or tile, so that the counts in flight stay the same
         const unsigned a_end = (unsigned)(u1 - u0 - 1) * 128u, w_end = (unsigned)(kt1 - kt0 - 1) * 1024u;
@@ -623,6 +631,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
             a_rd[h] = (unsigned)(wm * WTM * 2 + (fr >> 3)) * 1024u + (unsigned)(((fr & 7) * 8 + ((h * 4 + fg) ^ (fr & 7))) * 16);
         const unsigned w_rd = W_BASE + (unsigned)(wn * WTN) * 1024u + lane * 16;
         unsigned a_rs = 0, w_rs = W_TILE;                 // slots of the tile whose fragments are read next (kt0 + 1)
+        start_acc();      // (while the first copies are on their way)
         // before the first tile: A unit u0 and W tile kt0, issued in tile -4 at the latest
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * ODD + EVEN));
         __syncthreads();
@@ -669,6 +678,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
             W4_TILE(0)
             W4_TILE(1)
         }
+    } else {
+        start_acc();
     }
 #undef W4_TILE
     // every copy has landed and every read of LDS has come back, in every wave: LDS is free for the results
