@@ -20,6 +20,12 @@
 
 
 __device__ __forceinline__ uint4 ld16(const bf16_t* p) { return *reinterpret_cast<const uint4*>(p); }
+// The same of a weight that one block reads once.
+__device__ __forceinline__ uint4 ld16_once(const bf16_t* p) {
+    typedef __attribute__((__vector_size__(16))) unsigned once_t;
+    const once_t v = __builtin_nontemporal_load(reinterpret_cast<const once_t*>(p));
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
 __device__ __forceinline__ bf16x8 as_frag(const uint4& v) { return *reinterpret_cast<const bf16x8*>(&v); }
 
 template <typename TC>
@@ -489,7 +495,8 @@ struct W4Scale {
 };
 // PLANES: several products in one launch (GemmExtra).  A kernel of its own: a test of plane_cols in every product cost those of a short
 // prompt up to 1.5 % (gate+up of 560 rows 34.5 / 35.0 us).
-template <int WTN, int NWS, bool GLU, typename TC, int WGM = 2, bool SCALE = false, int WTM = 8, bool PLANES = false>
+// ONCE: the block reads its columns of W alone (see launch_w4; SCALE: always so).
+template <int WTN, int NWS, bool GLU, typename TC, int WGM = 2, bool SCALE = false, int WTM = 8, bool PLANES = false, bool ONCE = SCALE>
 __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, TC* __restrict__ C, int M, int N,
     int K, int lda, int KB, int n_out, W4Scale sc,
@@ -613,7 +620,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
             if (t + NWS >= 0) {
 #pragma unroll
                 for (int c = 0; c < LPW; ++c)
-                    copy16_to_lds_sbase(w0 + min((unsigned)(t + NWS) * 1024u, w_end), woff[c],
+                    copy16_to_lds_sbase<ONCE>(w0 + min((unsigned)(t + NWS) * 1024u, w_end), woff[c],
                                         lds_wave + W_BASE + (unsigned)(t + NWS) * W_TILE + (unsigned)c * 4096u);
             }
         }
@@ -656,7 +663,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
                     if (cp >= 0 && cp < NA_C)                                                       \
                         mfma_acc_copy(acc[i][jj], fw[h][i], fa[h][jj], a_to, (unsigned)(A_C0 + cp) * 4096u, aoff[cp >= 0 && cp < NA_C ? A_C0 + cp : 0], a_at); \
                     else if (cp >= 0)                                                               \
-                        mfma_acc_copy(acc[i][jj], fw[h][i], fa[h][jj], w_to, W_BASE + (unsigned)(cp - NA_C) * 4096u, woff[cp >= NA_C ? cp - NA_C : 0], w_at); \
+                        mfma_acc_copy<ONCE>(acc[i][jj], fw[h][i], fa[h][jj], w_to, W_BASE + (unsigned)(cp - NA_C) * 4096u, woff[cp >= NA_C ? cp - NA_C : 0], w_at); \
                     else mfma_acc(acc[i][jj], fw[h][i], fa[h][jj]);                                 \
                     if (q % RPM == RPM - 1 && q / RPM < WTN + WTM) {                                \
                         const int rd = q / RPM;                                                     \
@@ -744,12 +751,26 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
             return tff_fail("gemm: planes of a gated or scaled product");
         }
     }
-    if (splits > 1)
-        gemm_bf16_w4_kernel<WTN, NWS, false, float, WGM, false, WTM><<<grid, 256, 0, s>>>(A, Wp, part, M, N, K, lda, KB, 0, sc, ex);
-    else if (c_dtype == TFF_F32)
-        gemm_bf16_w4_kernel<WTN, NWS, GLU, float, WGM, SCALE, WTM><<<grid, 256, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, KB, n_out, sc, ex);
-    else
-        gemm_bf16_w4_kernel<WTN, NWS, GLU, bf16_t, WGM, SCALE, WTM><<<grid, 256, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, sc, ex);
+    auto launch = [&](auto ONCE) {
+        constexpr bool once = decltype(ONCE)::value;
+        if (splits > 1)
+            gemm_bf16_w4_kernel<WTN, NWS, false, float, WGM, false, WTM><<<grid, 256, 0, s>>>(A, Wp, part, M, N, K, lda, KB, 0, sc, ex);
+        else if (c_dtype == TFF_F32)
+            gemm_bf16_w4_kernel<WTN, NWS, GLU, float, WGM, SCALE, WTM, false, once><<<grid, 256, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, KB, n_out, sc, ex);
+        else
+            gemm_bf16_w4_kernel<WTN, NWS, GLU, bf16_t, WGM, SCALE, WTM, false, once><<<grid, 256, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, sc, ex);
+    };
+    // A weight that one block reads, K in one part: 40 and 100 rows of 24,576 x 4,096 38.0 / 35.6 and 43.9 / 40.7 us, 17 rows of 151,936
+    // 218 / 192 (plain loads / once).  The short streams of a split K lose by it: 100 rows of 4,096 x 4,096 16.3 / 19.4, 128 of
+    // 7,168 x 5,120 24.8 / 27.8.  (256 rows are two waves' of A, and a product that long is not bound by its weight's stream.)
+    if constexpr (SCALE) {
+        launch(std::true_type{});
+    } else if constexpr (WGM == 1) {
+        if (TM == 1 && splits == 1) launch(std::true_type{});
+        else launch(std::false_type{});
+    } else {
+        launch(std::false_type{});
+    }
     if (int rc = tff_check_launch("gemm_bf16_w4")) return rc;
     if (splits > 1 && reduce) {
         return launch_reduce<GLU>(part, splits, M, N, C, GLU ? n_out : N, ex, c_dtype, s);
@@ -773,6 +794,11 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
 // that, not W, is most of a wave's traffic.  With GLU, sets 2p and 2p+1 hold a
 // gate group and the up group that follows it in W; the epilogue writes
 // silu(gate) * up.
+// The weight's loads say that nobody asks for the line again (nt): the caches then keep the rows of A and do not write lines about
+// that nothing will hit.  us, four decode steps of 8 requests on 8 layers of the 8B shape 4,300 / 4,057, a prompt of 96 tokens and 15
+// decode steps of the 0.6B shape 18,700 / 17,800; the head of 151,936 columns, 3 rows, 200 / 177 (7.0 TB/s).
+// The four-wave kernel has the same where it reads a weight once (launch_w4).
+// Weights that others read too (several row tiles), or in pieces of 64 bytes (float32 rows, 8,030 -> 8,200), lose by it.
 //
 // An RMS norm between two such products costs a kernel of a few microseconds for a few rows.
 // Its per-row factor commutes with the product that follows it, so the two products take the
@@ -931,7 +957,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
             for (int u = 0; u < UNROLL; ++u) {
                 const int st = min(s0 + u, last);
 #pragma unroll
-                for (int r = 0; r < R; ++r) rw[u][r] = ld16(wfrag[r] + (size_t)st * 512);
+                for (int r = 0; r < R; ++r) rw[u][r] = ld16_once(wfrag[r] + (size_t)st * 512);
 #pragma unroll
                 for (int t = 0; t < MT; ++t) ra[u][t] = ld16(arow[t] + st * 32 + fg * 8);
             }
@@ -948,7 +974,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
                     }
                     const int st = min(s0 + UNROLL + u, last);
 #pragma unroll
-                    for (int r = 0; r < R; ++r) rw[u][r] = ld16(wfrag[r] + (size_t)st * 512);
+                    for (int r = 0; r < R; ++r) rw[u][r] = ld16_once(wfrag[r] + (size_t)st * 512);
 #pragma unroll
                     for (int t = 0; t < MT; ++t) ra[u][t] = ld16(arow[t] + st * 32 + fg * 8);
                 }
@@ -961,7 +987,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) rw[u][r] = ld16(wfrag[r] + (size_t)(s0 + u) * 512);
+            for (int r = 0; r < R; ++r) rw[u][r] = ld16_once(wfrag[r] + (size_t)(s0 + u) * 512);
 #pragma unroll
             for (int t = 0; t < MT; ++t) ra[u][t] = ld16(arow[t] + (s0 + u) * 32 + fg * 8);
         }
@@ -980,7 +1006,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
         const bool kok = k < K;
         uint4 rw[R], ra[MT];
 #pragma unroll
-        for (int r = 0; r < R; ++r) rw[r] = ld16(wfrag[r] + (size_t)s0 * 512);
+        for (int r = 0; r < R; ++r) rw[r] = ld16_once(wfrag[r] + (size_t)s0 * 512);
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             const uint4 v = ld16(arow[t] + (kok ? k : 0));
