@@ -368,6 +368,26 @@ def test_four_wave_cases_cover_every_tile_width():
     assert {(128, False), (192, False), (256, False), (192, True), (256, True)} <= widths, widths
 
 
+MANY_TILE_ROWS = [
+    # M, N, K: more tile rows than one band, so that the last band or the last bands together are ragged
+    (1030, 60, 64),        # 128 x 128: nine tile rows of one column, fewer tiles than the eighths asked for
+    (1300, 300, 64),       # 128 x 128: a band of eight and one of three
+    (2200, 520, 128),      # 128 x 128: two bands and two tile rows, bands of five columns
+    (2310, 2100, 64),      # 256 x 128: ten tile rows, bands of four together
+    (4300, 8300, 64),      # 256 x 256: two bands together, twice, and a last row alone
+]
+
+
+@pytest.mark.parametrize("M,N,K", MANY_TILE_ROWS)
+def test_linear_of_more_tile_rows_than_a_band(M, N, K):
+    """Every tile is worked on, whatever is left over when the tile rows go to the XCDs in bands."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(N, K, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
+    _close(ops.linear(x, ops.pack_weight(w), out_dtype=torch.float32), ops.linear(x.float(), w.float()), 3e-5, "product")
+
+
 ONE_BY_FOUR_CASES = [
     # M, N, K, gated: few rows and K in units of 64, so tiles of 128 rows on four waves side by side
     (100, 6150, 4096, False),      # 128 x 128, K split; rows of the result that are no multiple of 16 bytes

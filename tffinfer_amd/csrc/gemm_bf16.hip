@@ -486,6 +486,47 @@ __device__ __forceinline__ void w4_store_rows(char* region, F val, TO* out, size
     }
 }
 
+// Which tile a block works on.  Blocks go to the eight XCDs in turn by their number, and an XCD's 32 CUs share an L2 that holds a
+// stretch of k of the tile rows and columns they work on at a time: so those should be few, and every XCD should get as many
+// tiles.  The tile rows are cut into bands of w4_band of them (up to 1,024 rows of A), a band's tiles numbered column after column; as many bands as
+// hold 256 tiles at least go together, and an XCD takes an eighth of their tiles, one after the other: 4 x 8 tiles of 256 rows at a time.
+// (Eight tile rows of every column to an XCD, whatever their number, were 32 x 1 tiles of a result 1,024 wide: every XCD
+// read all of A.  us before / now: 7,376 rows of 1,024 x 3,072 on tiles of 256 x 128 55 / 40,
+// 4,700 of 2,048 x 2,048 37.4 / 35.9, 16,384 of 4,096 x 12,288 1,070 / 1,041, of 24,576 x 4,096 2,198 / 2,177.)
+template <int BM>
+constexpr int w4_band() { return BM >= 256 ? 4 : 8; }
+template <int BM>
+__host__ __device__ inline int w4_rows_together(int TN) {
+    const int band = w4_band<BM>() * TN;
+    return w4_band<BM>() * ((256 + band - 1) / band);
+}
+template <int BM>
+__host__ __device__ inline long w4_blocks(long TM, long TN) {
+    const long rows = w4_rows_together<BM>((int)TN), full = TM / rows, rest = TM - full * rows;
+    return 8 * (full * ((rows * TN + 7) / 8) + (rest * TN + 7) / 8);
+}
+template <int BM>
+__device__ __forceinline__ bool w4_place(unsigned block, int TM, int TN, int& tm, int& tn) {
+    constexpr int BAND = w4_band<BM>();
+    const int xcd = block & 7, seq = block >> 3;
+    if (TM <= BAND) {      // (one band: the same with one division, which few rows' products notice)
+        const int mine = (TM * TN + 7) >> 3, j = xcd * mine + seq;
+        if (seq >= mine || j >= TM * TN) return false;
+        tn = j / TM;
+        tm = j - tn * TM;
+        return true;
+    }
+    const int together = w4_rows_together<BM>(TN), share = (together * TN + 7) >> 3;
+    const int at = min(seq / share, TM / together);
+    const int first = at * together, rows = min(together, TM - first);
+    const int mine = (rows * TN + 7) >> 3, i = seq - at * share, j = xcd * mine + i;
+    if (i >= mine || j >= rows * TN) return false;
+    const int band = j / (BAND * TN), in = j - band * BAND * TN, high = min(BAND, rows - band * BAND);
+    tn = in / high;
+    tm = first + band * BAND + (in - tn * high);
+    return true;
+}
+
 // SCALE: A's rows (up to 16 of them) still lack the factor of the RMS norm they went through; the
 // factor, rsqrt(sum of the row's sums of squares / dim + eps), is applied to the accumulators.
 struct W4Scale {
@@ -530,21 +571,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     const int wm = WGM == 2 ? wave >> 1 : 0, wn = WGM == 2 ? wave & 1 : wave;
     const int fr = lane & 15, fg = lane >> 4;
     const int TM = (M + BM - 1) / BM, TN = (N + BN - 1) / BN;
-    const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-    const int full = (TM >> 3) * TN;
-    int grp, grp_rows, j;
-    if (seq < full) {
-        grp = seq / TN;
-        grp_rows = 8;
-        j = xcd * TN + (seq - grp * TN);
-    } else {
-        grp = TM >> 3;
-        grp_rows = TM & 7;
-        const int per = (grp_rows * TN + 7) >> 3;
-        j = xcd * per + (seq - full);
-        if (seq - full >= per || j >= grp_rows * TN) return;
-    }
-    const int tn = j / grp_rows, tm = grp * 8 + j % grp_rows;
+    int tm, tn;
+    if (!w4_place<BM>(blockIdx.x, TM, TN, tm, tn)) return;
     const int m0 = tm * BM, n0 = tn * BN;
     const int NB = (N + 15) / 16;
     if constexpr (PLANES) {   // (a tile's columns are one plane's; C as its column 0 of row 0 would lie)
@@ -736,7 +764,7 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
     if (splits <= 1 || !part) { splits = 1; part = nullptr; }
     TFF_REQUIRE(splits <= KB / 2, "gemm: %d parts of %d units of K", splits, KB / 2);
     const long TM = (M + BM - 1) / BM, TN = (N + BN - 1) / BN;
-    const long tiles = 8 * ((TM / 8) * TN + ((TM % 8) * TN + 7) / 8);   // eight equal shares, see the kernel
+    const long tiles = w4_blocks<BM>(TM, TN);   // eight equal shares
     TFF_REQUIRE(tiles < (1L << 31), "gemm: too many tiles for M=%d N=%d", M, N);
     TFF_REQUIRE((size_t)(BM - 1) * lda * 2 + 128 < (1ull << 32) && (size_t)(BN / 16) * KB * 1024 < (1ull << 32),
                 "gemm: rows of %d elements at a stride of %d are too long", K, lda);
