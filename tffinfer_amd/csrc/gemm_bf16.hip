@@ -1233,21 +1233,24 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
         // the model picks it rather too seldom).  A block goes through its part of K in
         // units of 64; a unit takes what its MFMAs take at the tile's rate or what its columns of W take
         // to arrive, whichever is longer: a block's share of the HBM stream, at most what one CU pulls.
-        // Blocks go round the CUs; each round ends with the pipeline filled and the tile stored.  The
-        // constants were fitted to measurements of the four products of the 8B, 14B and 32B shapes at
-        // 17 .. 4,096 rows on an MI355X (weights in turn, so that none comes from a cache; every tile
-        // with 1 .. 8 parts, 204 cases): the pick is 0.3 % from the best candidate on average, 6 % at worst.
+        // Blocks go round the CUs; each round ends with the pipeline filled and the tile stored.  Beyond 64 rows the
+        // constants stand for 840 products of the 0.6B to 14B shapes and of the other designs, 65 .. 9,000 rows, every tile with
+        // 1 .. 8 parts timed in a graph on an MI355X (weights in turn, so that none comes from a cache, and none of a launch's
+        // host work in the figure): the pick is 1.5 % from the best candidate on average; the constants before, fitted to a slower loop
+        // and to launches from the host, were 5.3 % from it there, 11 % at 128 .. 512 rows, where they split K for a kernel
+        // more (us: 229 rows of 4,096 x 2,048 16.2 / 11.2, 501 of 2,048 x 2,048 16.7 / 10.3, 901 of it 19.5 / 14.8, 333 of 2,048 x 6,144 23.7 / 18.5).
         // Up to 64 rows the four waves side by side take 64 or 32 rows: a product of so few rows is its
         // weight's stream, and a block that does not work through 128 rows for 32 asks for its next
         // columns sooner (3 to 10 % less time than the tiles of 128 rows and the sixteen-wave kernel's
         // 64 x 128 on the four products of the three shapes at 17 to 64 rows; their rates fitted to
         // those 88 cases stand for that, the pick 0.5 % from the best on average, 5 % at worst).
-        struct Cand { int bm, bn, slots; double rate; };
-        static const Cand cands[11] = {{256, 256, 1, 6.01e6}, {256, 192, 1, 5.45e6}, {256, 128, 1, 5.04e6},
-                                       {128, 384, 1, 3.24e6}, {128, 256, 1, 4.61e6}, {128, 128, 1, 3.45e6},
-                                       {64, 256, 1, 2.4e6}, {64, 128, 1, 2.0e6}, {32, 256, 1, 1.4e6}, {32, 128, 1, 1.3e6},
-                                       {64, 128, 2, 2.18e6}};
-        const double HBM = 7.72e6, CU_MAX = 6.0e4;       // bytes a microsecond: all CUs together, one alone
+        struct Cand { int bm, bn, slots; double rate, rate_few; };      // flops a microsecond of a CU, beyond 64 rows and up to them
+        static const Cand cands[11] = {{256, 256, 1, 6.45e6, 0}, {256, 192, 1, 6.10e6, 0}, {256, 128, 1, 5.42e6, 0},
+                                       {128, 384, 1, 6.49e6, 3.24e6}, {128, 256, 1, 5.38e6, 4.61e6}, {128, 128, 1, 3.56e6, 3.45e6},
+                                       {64, 256, 1, 0, 2.4e6}, {64, 128, 1, 0, 2.0e6}, {32, 256, 1, 0, 1.4e6}, {32, 128, 1, 0, 1.3e6},
+                                       {64, 128, 2, 2.48e6, 0}};
+        const bool few = M <= 64;
+        const double HBM = few ? 7.72e6 : 8.18e6, CU_MAX = few ? 6.0e4 : 6.54e4;   // bytes a microsecond: all CUs together, one alone
         GemmPlan best = {128, 128, 1};
         double best_t = 1e30;
         for (const Cand& c : cands) {
@@ -1261,11 +1264,13 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
                 const double rounds = ceil(blocks / (CUS * c.slots));
                 const double share = fmin((double)c.slots, ceil(blocks / CUS));   // blocks that share a CU's MFMAs
                 const double bw = fmin(CU_MAX, HBM / fmin(blocks, CUS * c.slots));
-                const double unit = fmax(2.0 * c.bm * c.bn * 64.0 * share / c.rate, c.bn * 128.0 / bw);
-                double t = rounds * ((double)nk / S * unit + 3.0) + 3.0;
+                const double unit = fmax(2.0 * c.bm * c.bn * 64.0 * share / (few ? c.rate_few : c.rate), c.bn * 128.0 / bw);
+                const double ends = few ? 3.0 : 1.29 + 2.55 * (c.bm * c.bn / 65536.0);   // a block's first fetch, and storing its tile
+                double t = rounds * ((double)nk / S * unit + ends) + 3.0;
                 // the partial sums: written, read and added by a second kernel, or (kept) read by the
                 // consumer in place of one plane
-                if (S > 1) t += keep ? (S - 1.0) * M * N * 4.0 / 4e6 : (double)S * M * N * 4.0 / 2.54e6 + 2.7;
+                if (S > 1 && few) t += keep ? (S - 1.0) * M * N * 4.0 / 4e6 : (double)S * M * N * 4.0 / 2.54e6 + 2.7;
+                else if (S > 1) t += keep ? (S - 1.0) * M * N * 4.0 / 1.97e6 : (double)S * M * N * 4.0 / 2.15e6 + 6.78;
                 if (t < best_t) { best_t = t; best = {c.bm, c.bn, S}; }
             }
         }
