@@ -1,8 +1,7 @@
 // bfloat16 attention of prompt portions over the paged cache: the blocks that attention_mfma.hip gives long portions,
 // for large heads without a cap on the scores and without pooled blocks of keys, on four waves of several column tiles.
-// (Reference: src/kernel/cuda/paged_flash_attention.cu:855-1055.)  Columns, operand orders, the softmax on raw scores
-// with its reference that moves by more than 8 in the exponent only, and the merge of key groups are those of that
-// file; what differs is what bounds it.
+// (Reference: src/kernel/cuda/paged_flash_attention.cu:855-1055.)  Columns, operand orders, the softmax on raw scores and
+// the merge of key groups are those of that file; what differs is what bounds it.
 //
 // With a column tile (16 columns) a wave every MFMA wants an operand of 1 KB from LDS, and LDS gives a CU 128 bytes a
 // cycle: eight waves' slices of 32 keys take 1,024 cycles there, 512 on the matrix cores.  So a wave works on NQT
@@ -13,9 +12,10 @@
 // The fragments of K(s+1) are read from LDS behind the first half of the MFMAs, those of V(s) behind the second.
 //
 // What is left to bound it is the issue of that one wave, so the softmax has neither a maximum nor a rescaling: the
-// reference of a column's exponentials is the largest score of its first slice, and float32 holds what the others exceed it by: sums and outputs are of the size 2^(largest - reference), without any loss
-// of precision up to 2^100.  Where a sum turns out beyond 2^100, or below 2^-100, or is no number, the block goes over the
-// item's keys once more for the largest score of every column and then repeats the item against that.
+// reference of a column's exponentials is the largest score of its first slice, and float32 holds what the others exceed
+// it by: sums and outputs are of the size 2^(largest - reference), without any loss of precision up to 2^100.  Where a sum
+// turns out beyond 2^100, or below 2^-100, or is no number, the block goes over the item's keys once more for the largest
+// score of every column and then repeats the item against that.
 //
 // us, the blocks of eight waves / these, 32 query and 8 key heads of 128: 512 tokens 19.3 / 17.5, 901 27.8 / 23.9, 2,048 60.0 / 50.5,
 // 4,096 207 / 141, 16,384 2,610 / 1,793 (0.84 / 1.23 PFLOP/s); 3,001 and 1,700 tokens of 16 and 4 heads in a window of 1,024
