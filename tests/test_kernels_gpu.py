@@ -47,6 +47,21 @@ def test_embed(dtype):
     assert torch.equal(out.cpu(), table.float()[ids.long()])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,skip", [(4, 0), (1024, 0), (1028, 0), (4100, 0), (1030, 0), (1024, 1), (7, 3)])
+def test_embed_of_row_major_tables(dtype, H, skip):
+    """Four elements a thread where rows and pointers allow it, else one (``skip``: elements that the table is off
+    its alignment by): whole and short last rounds of a block, an id out of range is a row of NaN."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(H)
+    flat = torch.randn(skip + 9 * H, generator=g).to(dtype).to(DEV)
+    table = flat[skip:].view(9, H)
+    ids = torch.tensor([8, 0, 3, 9, -1, 3], dtype=torch.int32)
+    out = ops.embed(table, ids.to(DEV)).cpu()
+    ok = (ids >= 0) & (ids < 9)
+    assert torch.equal(out[ok], table.cpu().float()[ids[ok].long()]) and bool(out[~ok].isnan().all())
+
+
 @pytest.mark.parametrize("H", [40, 96, 1000, 4096, 5120])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_add_rmsnorm(H, out_dtype):

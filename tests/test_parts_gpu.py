@@ -177,6 +177,26 @@ def test_prenorm_block(dtype, tol, T):
     assert _err(resid + out_pending, ref) < tol
 
 
+@pytest.mark.parametrize("H", [24, 20])
+def test_embedding_of_a_table_without_a_head(H):
+    """Such a table stays row-major until someone asks for it as a product's weight; the rows are the same either way."""
+    from tffinfer_amd.engine.runner import LayerContext
+    from tffinfer_amd.kernels import ops
+    from tffinfer_amd.parts import Embedding, OutputHead
+    table = torch.randn(50, H).to(torch.bfloat16)
+    ids = torch.tensor([3, 49, 0], dtype=torch.int32, device=DEV)
+    ctx = LayerContext(ops, torch.bfloat16, None, 0)
+    emb = Embedding(50, H)
+    emb.load_weights({"weight": table}, torch.bfloat16, DEV)
+    assert torch.equal(emb.forward(ctx, ids).cpu(), table.float()[[3, 49, 0]])
+    assert isinstance(emb.weight, ops.PackedWeight) and emb.weight is emb.weight
+    assert torch.equal(emb.forward(ctx, ids).cpu(), table.float()[[3, 49, 0]])
+    late = Embedding(50, H)      # (a head made after its table was loaded)
+    late.load_weights({"weight": table}, torch.bfloat16, DEV)
+    y = late.forward(ctx, ids).to(torch.bfloat16)
+    assert _err(OutputHead(50, H, tied_to=late).forward(ctx, y), table.double()[[3, 49, 0]] @ table.double().T) < 1e-5
+
+
 def test_embedding_and_tied_head():
     from tffinfer_amd.engine.runner import LayerContext
     from tffinfer_amd.kernels import ops

@@ -53,18 +53,44 @@ __global__ void embed_kernel(const T* __restrict__ table, const int32_t* __restr
     for (int j = threadIdx.x; j < H; j += blockDim.x) o[j] = bad ? __builtin_nanf("") : to_f32(row[j]);
 }
 
+// The same four elements a thread: loads of 8 or 16 bytes, stores of 16, so that a row is a few requests in flight at once
+// (element by element 16,384 rows of 4,096 in bfloat16 take 131 us, so 78: 402 MB).
+template <typename T>
+__global__ __launch_bounds__(256) void embed_vec_kernel(const T* __restrict__ table, const int32_t* __restrict__ ids,
+                                                        float* __restrict__ out, int H, int V) {
+    const int t = blockIdx.x;
+    int id = ids[t];
+    const bool bad = id < 0 || id >= V;
+    if (bad) id = 0;
+    const T* row = table + (size_t)id * H;
+    float* o = out + (size_t)t * H;
+#pragma unroll 4
+    for (int j = threadIdx.x * 4; j < H; j += 1024) {
+        struct alignas(4 * sizeof(T)) { T h[4]; } v = *reinterpret_cast<const decltype(v)*>(row + j);
+        float4 y = make_float4(to_f32(v.h[0]), to_f32(v.h[1]), to_f32(v.h[2]), to_f32(v.h[3]));
+        if (bad) y.x = y.y = y.z = y.w = __builtin_nanf("");
+        *reinterpret_cast<float4*>(o + j) = y;
+    }
+}
+
 TFF_API int tff_embed(const void* table, const int32_t* ids, float* out, int T, int H, int V,
                       int dtype, tff_stream_t stream) {
     TFF_REQUIRE(table && ids && out, "embed: null pointer");
     TFF_REQUIRE(T >= 0 && H > 0 && V > 0, "embed: bad sizes T=%d H=%d V=%d", T, H, V);
     if (T == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
-    if (dtype == TFF_F32)
-        embed_kernel<float><<<T, 256, 0, s>>>((const float*)table, ids, out, H, V);
-    else if (dtype == TFF_BF16)
-        embed_kernel<bf16_t><<<T, 256, 0, s>>>((const bf16_t*)table, ids, out, H, V);
-    else
+    const bool vec = H % 4 == 0 && (uintptr_t)table % (dtype == TFF_F32 ? 16 : 8) == 0 && (uintptr_t)out % 16 == 0;
+#define TFF_EMBED(T_)                                                                        \
+    if (vec) embed_vec_kernel<T_><<<T, 256, 0, s>>>((const T_*)table, ids, out, H, V);       \
+    else embed_kernel<T_><<<T, 256, 0, s>>>((const T_*)table, ids, out, H, V);
+    if (dtype == TFF_F32) {
+        TFF_EMBED(float)
+    } else if (dtype == TFF_BF16) {
+        TFF_EMBED(bf16_t)
+    } else {
         return tff_fail("embed: unknown dtype %d", dtype);
+    }
+#undef TFF_EMBED
     return tff_check_launch("embed");
 }
 
