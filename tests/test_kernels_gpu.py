@@ -1216,6 +1216,87 @@ def test_attention_of_prompts_on_blocks_of_four_waves(nq, nkv, d, ps, window, gr
     _close(out, gen.double(), ATTN_TOL, "blocks of four waves against the general kernel")
 
 
+def _prompt_of_scores(P, n, ps, d, exponents, values, seed=0):
+    """A portion of n tokens behind P cached ones, one head: every query sees key j at a score of exponents[j] ln 2 (with the scale ln 2 that
+    is returned) and the values values[j]."""
+    batch, kv, ks, vs, positions, token_req = _fake_step([(P, n)], ps, 1, d, torch.bfloat16, seed=seed)
+    keys = torch.zeros(P + n, d)
+    keys[:, 0] = torch.tensor(exponents)
+    assert torch.equal(keys, keys.bfloat16().float())
+    q = torch.zeros(n, 1, d, dtype=torch.bfloat16)
+    q[:, 0, 0] = 1
+    ks[0][:, 0], vs[0][:, 0] = keys.bfloat16(), values.bfloat16()
+    j = torch.arange(P + n)
+    pages = kv.block_tables[0].cpu().long()[j // ps]
+    kc, vc = kv.k_cache.cpu(), kv.v_cache.cpu()
+    kc[pages, 0, j % ps], vc[pages, 0, :, j % ps] = ks[0][:, 0], vs[0][:, 0]
+    kv.k_cache, kv.v_cache = kc.to(DEV), vc.to(DEV)
+    return q, batch, kv, ks[0], vs[0], positions, math.log(2)
+
+
+def _four_waves(q, d, kv, batch, window, scale, groups, sinks=None):
+    ops = _ops()
+    nq = q.shape[1]
+    out = torch.full((q.shape[0], nq * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.attention_prompt(q.reshape(-1, nq * d).to(DEV), out, nq, kv.k_cache.shape[1], d, kv, batch, window, scale, sinks, "all", groups)
+    return out.reshape(-1, nq, d)
+
+
+@pytest.mark.parametrize("first,later,value", [(-40, 86.5, -8.0), (-130, -3, 64.0), (-126, 0, 64.0), (60, 60, 8.0), (-60, -60, 8.0), (-300, -290, 8.0)])
+def test_attention_of_prompts_whose_key_groups_lie_far_apart(first, later, value):
+    """Two groups take every other slice of 32 keys, each against the largest score of its own first one.  The second group's keys lie at
+    ``first``, but one, of value ``value``, at ``later``: what its sums exceed float32 by, or the merge scales to nothing, must not
+    be lost when the sum of both looks harmless."""
+    P, n, d = 128, 70, 128
+    exps = [0.0 if j // 32 % 2 == 0 else float(first) for j in range(P + n)]
+    exps[100] = float(later)
+    values = torch.randn(P + n, d, generator=torch.Generator().manual_seed(3))
+    values[100] = value
+    q, batch, kv, k, v, positions, scale = _prompt_of_scores(P, n, 16, d, exps, values)
+    ref = _attn_ref(q, k, v, positions, 0, scale)
+    _close(_four_waves(q, d, kv, batch, 0, scale, 2), ref, ATTN_TOL, f"second group at 2^{first}, one key at 2^{later}")
+
+
+@pytest.mark.parametrize("d,groups", [(128, 1), (128, 2), (256, 1)])
+@pytest.mark.parametrize("top,value", [(49, 1.0), (49.5, 1.0), (51, 1.0), (99, 1.0), (101, 1.0), (126, 1.0), (128, 1.0), (48, 2.0 ** 90), (90, 2.0 ** 60)])
+def test_attention_of_prompts_whose_scores_leave_their_reference(d, groups, top, value):
+    """Scores that creep up from slice to slice and then jump, to just inside and just outside of what the sums against a first slice's
+    reference may reach, and values that carry the outputs further than the sums."""
+    P, n = 200, 90
+    exps = [round(j / 32) / 2 for j in range(P + n)]
+    exps[217] = float(top)
+    exps[266] = float(top) - 1
+    values = value * torch.randn(P + n, d, generator=torch.Generator().manual_seed(4))
+    q, batch, kv, k, v, positions, scale = _prompt_of_scores(P, n, 16, d, exps, values)
+    _close(_four_waves(q, d, kv, batch, 0, scale, groups), _attn_ref(q, k, v, positions, 0, scale), ATTN_TOL, f"scores up to 2^{top}")
+
+
+@pytest.mark.parametrize("d,groups", [(128, 1), (128, 2), (256, 1)])
+@pytest.mark.parametrize("loud", [48, 49.5, 51, 100, 140])
+def test_attention_of_prompts_past_a_loud_key(d, groups, loud):
+    """A key that the first columns' windows hold and the next have just passed: its score is a reference that the sums of the latter lie
+    far below."""
+    P, n, window = 300, 70, 73
+    exps = [0.0] * (P + n)
+    exps[P - window + 3] = exps[P - window + 34] = float(loud)
+    values = torch.randn(P + n, d, generator=torch.Generator().manual_seed(5))
+    q, batch, kv, k, v, positions, scale = _prompt_of_scores(P, n, 8, d, exps, values)
+    _close(_four_waves(q, d, kv, batch, window, scale, groups), _attn_ref(q, k, v, positions, window, scale), ATTN_TOL, f"a loud key of 2^{loud}")
+
+
+@pytest.mark.parametrize("groups", [1, 2])
+@pytest.mark.parametrize("first,last", [(60, 0), (0, 60), (120, 120)])
+def test_attention_of_prompts_repeats_over_more_pages_than_lds_holds(groups, first, last):
+    """Loud keys in the first and in the last of two segments of pages: the repeat goes through both."""
+    P, n, d = 16380, 20, 128
+    exps = [0.0] * (P + n)
+    exps[40] = exps[70] = float(first)
+    exps[16390] = float(last)
+    values = torch.randn(P + n, d, generator=torch.Generator().manual_seed(6))
+    q, batch, kv, k, v, positions, scale = _prompt_of_scores(P, n, 8, d, exps, values)
+    _close(_four_waves(q, d, kv, batch, 0, scale, groups), _attn_ref(q, k, v, positions, 0, scale), ATTN_TOL, f"loud keys of 2^{first} and 2^{last}")
+
+
 def test_attention_mfma_picks_its_blocks_by_the_work():
     """A prompt of 2,048 tokens goes to the blocks of 128 columns, one of 32,768 tokens to those
     of 256; head sizes beyond 128 never do.  A prompt of 6,000 tokens through either gives

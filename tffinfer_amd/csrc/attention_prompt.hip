@@ -13,9 +13,11 @@
 //
 // What is left to bound it is the issue of that one wave, so the softmax has neither a maximum nor a rescaling: the
 // reference of a column's exponentials is the largest score of its first slice, and float32 holds what the others exceed
-// it by: sums and outputs are of the size 2^(largest - reference), without any loss of precision up to 2^100.  Where a sum
-// turns out beyond 2^100, or below 2^-100, or is no number, the block goes over the item's keys once more for the largest
-// score of every column and then repeats the item against that.
+// it by: sums and outputs are of the size 2^(largest - reference), without any loss of precision up to 2^50 and values up
+// to 2^77.  Where a column's sum turns out below 2^-50, or a group's part of it beyond 2^50, or an output is no finite
+// number, the block goes over the item's keys once more for the largest score of every column and then repeats the item
+// against that.  The bound is for two groups, whose references differ: what a group brings to their merge is scaled by
+// 2^-126 at least or is zero, so that of sums up to 2^50 no more than 2^-76 is lost of one that must be 2^-50.
 //
 // us, the blocks of eight waves / these, 32 query and 8 key heads of 128: 512 tokens 19.3 / 17.5, 901 27.8 / 23.9, 2,048 60.0 / 50.5,
 // 4,096 207 / 141, 16,384 2,610 / 1,793 (0.84 / 1.23 PFLOP/s); 3,001 and 1,700 tokens of 16 and 4 heads in a window of 1,024
@@ -73,7 +75,7 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
     constexpr unsigned K_SLOT = KGRP * KFR * 1024u, V_SLOT = KGRP * VFR * 1024u, V_BASE = NR * K_SLOT;
     constexpr int NPV = DT * NQT, NQK = KFR * NQT, NP = NQT * 4;      // MFMAs of the two halves, pairs of scores a lane
     static_assert(NPV == 32 && NQK == 32 && 4 + 3 * NP <= 62, "a step's schedule");
-    constexpr float NO_KEY = 1e30f, SUM_MIN = 0x1p-100f, SUM_MAX = 0x1p100f;
+    constexpr float NO_KEY = 1e30f, SUM_MIN = 0x1p-50f, SUM_MAX = 0x1p50f;
     static_assert(KGRP == 1 || V_BASE + NR * V_SLOT >= NW * NQT * (DT * 1024u + 512u), "the merge borrows the slices' place");
     __shared__ __attribute__((aligned(1024))) char smem[V_BASE + NR * V_SLOT];
     __shared__ int32_t pages[ATTN_PROMPT_PAGES];      // starts of pages in units of 16 bytes
@@ -293,7 +295,7 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
 #pragma unroll
                             for (int e = 0; e < 8; ++e) m = e <= last ? fmaxf(m, sc[0][t][e >> 2][e & 3]) : m;
                             m = rows_max(m);
-                            neg_ref[t] = m == -INFINITY ? 0.f : -m * sl2;
+                            neg_ref[t] = m == -INFINITY ? NO_KEY : -m * sl2;
                         }
                     }
                     const uint4 zero = make_uint4(0, 0, 0, 0);
@@ -397,7 +399,9 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
             // the slices' place.
             static_assert(KGRP <= 2 && NQT % KGRP == 0, "two groups at most");
             float* mo = reinterpret_cast<float*>(smem) + wcol * NQT * (DT * 256 + 128) + lane * 4;
-            bool again = false;      // a column whose sum leaves float32's comfortable range: the whole block once more
+            bool again = false;      // a column whose sums leave float32's comfortable range: the whole block once more
+#pragma unroll
+            for (int t = 0; t < NQT; ++t) again |= !(l_run[t] <= SUM_MAX);      // (a lane's part of its group's; zero without a key)
             auto give = [&](auto FROM) {
 #pragma unroll
                 for (int t = decltype(FROM)::value; t < decltype(FROM)::value + NQT / KGRP; ++t) {
@@ -428,7 +432,10 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
                         }
                     }
                     l_run[t] = rows_sum(l_run[t]);
-                    again |= !(l_run[t] >= SUM_MIN && l_run[t] <= SUM_MAX);
+                    float all = 0.f;      // infinite or no number where one of the outputs is
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) all += (o[t][dt][0] + o[t][dt][1]) + (o[t][dt][2] + o[t][dt][3]);
+                    again |= !(l_run[t] >= SUM_MIN) || !(fabsf(all) < INFINITY);
                 }
             };
             if constexpr (KGRP > 1) {
