@@ -1297,6 +1297,26 @@ def test_attention_of_prompts_repeats_over_more_pages_than_lds_holds(groups, fir
     _close(_four_waves(q, d, kv, batch, 0, scale, groups), _attn_ref(q, k, v, positions, 0, scale), ATTN_TOL, f"loud keys of 2^{first} and 2^{last}")
 
 
+@pytest.mark.parametrize("nq,nkv,d,groups", [(4, 1, 128, 1), (4, 1, 128, 2), (6, 2, 256, 1)])
+@pytest.mark.parametrize("ps", [8, 16, 64])
+def test_attention_of_prompts_does_not_look_at_pages_given_back(nq, nkv, d, groups, ps):
+    """The first slice of a windowed portion begins up to 31 keys before the first key that a token sees.  Pages that hold no other keys
+    are given back, and the table names some page of another request there: the same bits whatever that page holds."""
+    P, n, window = 3000, 70, 100
+    batch, kv, ks, vs, positions, token_req = _fake_step([(P, n)], ps, nkv, d, torch.bfloat16, seed=d + ps)
+    other = (set(range(kv.k_cache.shape[0])) - set(kv.block_tables[0].tolist())).pop()
+    kv.block_tables[0, :(P - window + 1) // ps] = other
+    q = torch.randn(n, nq, d, generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
+    outs = []
+    for loud in (0.0, 1.0, 50.0):
+        g = torch.Generator().manual_seed(6)
+        kv.k_cache[other] = (loud * torch.randn(nkv, ps, d, generator=g)).bfloat16().to(DEV)
+        kv.v_cache[other] = (loud * torch.randn(nkv, d, ps, generator=g)).bfloat16().to(DEV)
+        outs.append(_four_waves(q, d, kv, batch, window, 1 / math.sqrt(d), groups))
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    _close(outs[0], _attn_ref(q, ks[0], vs[0], positions, window, 1 / math.sqrt(d)), ATTN_TOL, "beside pages given back")
+
+
 def test_attention_mfma_picks_its_blocks_by_the_work():
     """A prompt of 2,048 tokens goes to the blocks of 128 columns, one of 32,768 tokens to those
     of 256; head sizes beyond 128 never do.  A prompt of 6,000 tokens through either gives

@@ -289,11 +289,12 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
                         settle(sc[0]);
 #pragma unroll
                         for (int t = 0; t < NQT; ++t) {
-                            // (keys that the window has passed count here: what matters is the scores' size)
-                            const int last = kgi < seg1 ? c_pos[t] - (kb0 + kgi * 32 + kg * 8) : -1;
+                            // Keys that a column's window has passed count here: what matters is the scores' size.  Those that every column's
+                            // has passed do not: their pages may be given back, and then the table has another request's in their place.
+                            const unsigned from = kgi < seg1 ? (unsigned)(kb0 + kgi * 32 + kg * 8 - kmin) : 0x40000000u, span = (unsigned)(c_pos[t] - kmin);
                             float m = -INFINITY;
 #pragma unroll
-                            for (int e = 0; e < 8; ++e) m = e <= last ? fmaxf(m, sc[0][t][e >> 2][e & 3]) : m;
+                            for (int e = 0; e < 8; ++e) m = from + (unsigned)e <= span ? fmaxf(m, sc[0][t][e >> 2][e & 3]) : m;
                             m = rows_max(m);
                             neg_ref[t] = m == -INFINITY ? NO_KEY : -m * sl2;
                         }
