@@ -1317,6 +1317,29 @@ def test_attention_of_prompts_does_not_look_at_pages_given_back(nq, nkv, d, grou
     _close(outs[0], _attn_ref(q, ks[0], vs[0], positions, window, 1 / math.sqrt(d)), ATTN_TOL, "beside pages given back")
 
 
+@pytest.mark.parametrize("nq,nkv,d,groups,block_tokens", [(4, 1, 128, 1, 16), (4, 1, 128, 2, 16), (4, 2, 128, 1, 32), (8, 2, 256, 1, 8)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), -float("inf")])
+def test_attention_of_prompts_keeps_values_that_are_not_finite_to_those_that_see_them(nq, nkv, d, groups, block_tokens, bad):
+    """A value that is not finite reaches the tokens that see its key and, of the others, those of the same 64 (32) columns of a wave only:
+    not the rest of the block's columns, whatever is left in the places behind the last key, in pages given back, or before the window."""
+    P, n, window, ps, at = 1000, 128, 300, 16, 1105
+    batch, kv, ks, vs, positions, token_req = _fake_step([(P, n)], ps, nkv, d, torch.bfloat16, seed=d)
+    q = torch.randn(n, nq, d, generator=torch.Generator().manual_seed(7)).to(torch.bfloat16)
+    ref = _attn_ref(q, ks[0], vs[0], positions, window, 1 / math.sqrt(d))
+    other = (set(range(kv.k_cache.shape[0])) - set(kv.block_tables[0].tolist())).pop()
+    kv.block_tables[0, :(P - window + 1) // ps] = other
+    kv.v_cache[other] = bad
+    kv.v_cache[kv.block_tables[0, (P - window) // ps].long(), :, :, :(P - window + 1) % ps] = bad      # (the last keys before the window)
+    kv.v_cache[kv.block_tables[0, (P + n - 1) // ps].long(), :, :, (P + n - 1) % ps + 1:] = bad        # (places that no token has yet)
+    out = _four_waves(q, d, kv, batch, window, 1 / math.sqrt(d), groups)
+    _close(out, ref, ATTN_TOL, "what is not finite is no token's")
+    kv.v_cache[kv.block_tables[0, at // ps].long(), :, :, at % ps] = bad
+    out = _four_waves(q, d, kv, batch, window, 1 / math.sqrt(d), groups)
+    first = (at - P) // block_tokens * block_tokens
+    _close(out[:first], ref[:first], ATTN_TOL, "the columns before")
+    assert not bool(out[at - P:].isfinite().any())
+
+
 def test_attention_mfma_picks_its_blocks_by_the_work():
     """A prompt of 2,048 tokens goes to the blocks of 128 columns, one of 32,768 tokens to those
     of 256; head sizes beyond 128 never do.  A prompt of 6,000 tokens through either gives

@@ -18,6 +18,8 @@
 // number, the block goes over the item's keys once more for the largest score of every column and then repeats the item
 // against that.  The bound is for two groups, whose references differ: what a group brings to their merge is scaled by
 // 2^-126 at least or is zero, so that of sums up to 2^50 no more than 2^-76 is lost of one that must be 2^-50.
+// Values that are not finite reach columns that do not see them (0 . inf is no number), and with them the test, which sends the
+// item into its second pass: there a wave takes values that none of its columns sees as zeros.
 //
 // us, the blocks of eight waves / these, 32 query and 8 key heads of 128: 512 tokens 19.3 / 17.5, 901 27.8 / 23.9, 2,048 60.0 / 50.5,
 // 4,096 207 / 141, 16,384 2,610 / 1,793 (0.84 / 1.23 PFLOP/s); 3,001 and 1,700 tokens of 16 and 4 heads in a window of 1,024
@@ -158,7 +160,7 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
                 const unsigned from = (unsigned)(kb + kg * 8 - c_lo[t]), span = (unsigned)(c_pos[t] - c_lo[t]);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) x[t][e >> 2][e & 3] = from + (unsigned)e <= span ? x[t][e >> 2][e & 3] : -INFINITY;
-                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("" : "+v"(x[t][0]), "+v"(x[t][1]));      // (here, in the branch)
             }
         };
         // (the scores' MFMAs have written: named one by one, or the compiler, which does not know them for MFMAs, reads them before)
@@ -172,6 +174,26 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
 #pragma unroll
             for (int e = 1; e < 4; ++e) m = fmaxf(m, fmaxf(x[0][e], x[1][e]));
             return m;
+        };
+
+        // a slice's values of keys that none of the wave's columns sees become zeros
+        auto hide = [&](int kb) {
+            const int w_from = __builtin_amdgcn_readfirstlane(c_lo[0]), w_to = __builtin_amdgcn_readlane(c_pos[NQT - 1], 15);
+            const unsigned from = (unsigned)(kb + kg * 8 - w_from), span = (unsigned)(w_to - w_from);
+            unsigned seen[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                seen[i] = (from + 2u * i <= span ? 0xffffu : 0u) | (from + 2u * i + 1u <= span ? 0xffff0000u : 0u);
+#pragma unroll
+            for (int dt = 0; dt < VFR; ++dt) {
+                union { bf16x8 f; unsigned u[4]; } x;
+                x.f = vf[dt];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x.u[i] &= seen[i];
+                vf[dt] = x.f;
+                asm volatile("" : "+v"(vf[dt]));
+            }
+            asm volatile("s_nop 1");      // (what a vector instruction has written an MFMA may read two instructions later: the compiler does not know these for MFMAs)
         };
 
         // the columns' references for the second pass: the largest score of all of the group's slices
@@ -312,17 +334,19 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
                 const int full0 = max(0, (w_lo - kb0 + 31) / 32 - seg0 - kgi + KGRP - 1) / KGRP;
                 const int full1 = min((w_min - 31 - kb0 >= 0 ? (w_min - 31 - kb0) / 32 + 1 : 0), seg1) - seg0 - kgi;
                 const unsigned full = (unsigned)max(0, (full1 > 0 ? (full1 + KGRP - 1) / KGRP : 0) - full0);
+                // the first key of the group's slice of step s; past the segment's last slice one that no column sees
+                auto group_slice = [&](int s) { return seg0 + s * KGRP + kgi < seg1 ? kb0 + (seg0 + s * KGRP + kgi) * 32 : 0x40000000; };
                 auto step = [&](auto H, int s) {
                     constexpr int h = decltype(H)::value;
                     __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm((NR - 2) * CPI));
                     asm volatile("s_barrier\n\ts_nop 7" ::: "memory");        // (the scores' last MFMAs have written before a vector instruction reads them)
-                    const int kb = kb0 + (seg0 + s * KGRP + kgi) * 32;
                     const char* ksrc = smem + k_rd + kgi * KFR * 1024 + lane * 16;
                     const char* vsrc = smem + V_BASE + v_rd + kgi * VFR * 1024 + lane * 16;
                     float tmp0 = 0.f, tmp1 = 0.f;
                     uint32_t pk = 0, pv = 0;
                     int jk = 0, jv = 0;
                     unsigned long long ka = 0, va = 0;
+                    if (pass > 0) hide(group_slice(s - 1));
                     static_for<NPV + NQK>([&](auto slot) {
                         constexpr int n = decltype(slot)::value;
                         if constexpr (n < NPV) {
@@ -342,7 +366,7 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
                             vf[dt] = *reinterpret_cast<const bf16x8*>(vsrc + dt * 1024);
                         }
                         // the softmax of slice s
-                        if constexpr (n == 3) if ((unsigned)(s - full0) >= full) mask(sc[h], seg0 + s * KGRP + kgi < seg1 ? kb : 0x40000000);
+                        if constexpr (n == 3) if ((unsigned)(s - full0) >= full) mask(sc[h], group_slice(s));
                         if constexpr (n >= 4 && n < 4 + 3 * NP) {
                             constexpr int p = (n - 4) / 3, t = p / 4, e = (p % 4) * 2;
                             if constexpr ((n - 4) % 3 == 0) {
@@ -374,6 +398,9 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     });
+                    // (worked out here: the compiler would move the softmax out of the MFMAs, behind the next step's branch: 16,384 tokens 1,885 / 1,940)
+#pragma unroll
+                    for (int t = 0; t < NQT; ++t) asm volatile("" : "+v"(pf[h][t]), "+v"(l_run[t]));
                     k_wr = k_to + k_rd;
                     v_wr = v_to + v_rd;
                     k_rd = ring_next<K_SLOT, NR * K_SLOT>(k_rd);
@@ -386,6 +413,7 @@ __global__ __launch_bounds__(256, 1) void attn_prompt_kernel(
                     step(std::integral_constant<int, 1>{}, s + 1);
                 }
                 // the values of the segment's last slice
+                if (pass > 0) hide(group_slice((nsup + 1) / 2 * 2 - 1));
 #pragma unroll
                 for (int n = 0; n < NPV; ++n) mfma_acc(o[n % NQT][n / NQT], vf[n / NQT], pf[1][n % NQT]);
             }
