@@ -1850,6 +1850,27 @@ def test_products_with_an_activation(act, M, N, K):
         assert out.dtype == dtype and float((out.double() - ref).abs().max()) < tol * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("act", ["gelu", "gelu_tanh", "relu2"])
+@pytest.mark.parametrize("M,N,K", [
+    (20, 200, 64), (60, 1030, 128), (200, 1030, 192), (333, 512, 192), (700, 100, 64),              # row tiles of 32, 64 and 128, ragged rows of results
+    (1055, 4096, 4096), (1018, 18432, 8192),                                                        # tiles of 256 rows
+    (82, 18432, 4096), (234, 18432, 4096), (102, 9216, 2048), (351, 12288, 4096)])                  # wide layers over few rows
+def test_activations_see_float32_sums(act, M, N, K):
+    """The product reaches the activation in float32, whatever the plan: the result is the one rounding to bfloat16 (8 bits: 2^-8 of a value
+    at most) away from the exact one, and the sums' error (K terms, far below 2^-16 of the largest value).  A product that is rounded before
+    its square is off by up to 3 * 2^-8, before a gelu by 2 * 2^-8."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    z = x.double() @ w.double().T
+    ref = {"gelu": torch.nn.functional.gelu, "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh"),
+           "relu2": lambda t: t.clamp(min=0) ** 2}[act](z)
+    out = ops.linear_unary(x, ops.pack_weight(w), act, torch.bfloat16)
+    bound = 1.001 * 2.0 ** -8 * ref.abs() + 2.0 ** -16 * ref.abs().max()
+    assert bool(((out.double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("sizes", [[4], [16, 20], [4096, 5, 1 << 20], [3 * i + 1 for i in range(50)]])
 def test_rows_set_to_zero(sizes):
     """Buffers of any number of words, more than one launch of them, at addresses that are no multiple of 16; what lies beside stays."""

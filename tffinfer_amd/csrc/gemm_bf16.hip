@@ -1321,6 +1321,17 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
     return best;
 }
 
+// A product in one part before an activation (tff_gemm_unary) leaves float32 sums, which the sum's kernel reads, as long as their
+// traffic, twice that of sums in bfloat16, is little beside the product's own work, which grows with K: wherever splitting K in two is
+// not far behind either.  us, bfloat16 and a kernel over it / float32, gelu: 50 rows of 18,432 x 4,096 36.6 / 37.3, 122 46.4 / 48.7, 234 61.6 / 63.8,
+// 102 of 9,216 x 2,048 16.0 / 16.1; past the line 1,500 rows of 9,216 x 2,048 would be 62 / 69, and the activation is a kernel over
+// the product's own type.  In the tiles' epilogue the exact gelu takes longer than in a kernel of its own, one wave a SIMD with
+// nothing beside it: 200 rows of 18,432 68, 2,048 rows 300 for 262.
+static bool unary_in_float32(const GemmPlan& p, int M, int N, int K) {
+    if (p.tile == 0 || p.splits > 1 || K % 64) return false;
+    return (long)M * N <= (K < 6144 ? 1150L : 3300L) * K;
+}
+
 TFF_API size_t tff_gemm_workspace_bytes(int M, int N, int K, int ab_dtype, int glu, int keep_partials) {
     if (ab_dtype != TFF_BF16 || M <= 0 || N <= 0 || K <= 0) return 0;
     const GemmPlan p = plan_for(M, N, K, glu != 0, keep_partials != 0);
@@ -1406,8 +1417,16 @@ int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int 
     if (!workspace || workspace_bytes < (size_t)plan.splits * M * N * sizeof(float)) plan.splits = 1;
     const int S = plan.splits;
     const bool red = !keep_partials;
+    if (ex.unary && glu_out == 0 && !keep_partials && planned_splits == 1 && unary_in_float32(plan, M, N, K) && workspace &&
+        workspace_bytes >= (size_t)M * N * sizeof(float)) {
+        // K in one part, whose float32 results the sum's kernel takes as the only plane
+        GemmExtra plain = ex;
+        plain.unary = 0;
+        if (int rc = tff_gemm_bf16(A, Wp, workspace, M, N, K, lda, plain, TFF_F32, 0, nullptr, 0, 0, s)) return rc;
+        return launch_reduce<false>(workspace, 1, M, N, C, N, ex, c_dtype, s);
+    }
     TFF_REQUIRE(!ex.unary || (glu_out == 0 && !keep_partials && (plan.tile == 0 || plan.splits > 1)),
-                "gemm: an activation is applied by the streaming kernel or by the sum over the parts of K");
+                "gemm: an activation is applied by the streaming kernel or to the sum over the parts of K");
     TFF_REQUIRE(!keep_partials || (glu_out == 0 && c_dtype == TFF_F32),
                 "gemm: partial sums are kept for a plain float32 result only");
     if (glu_out > 0) {
@@ -1570,11 +1589,17 @@ TFF_API int tff_gemm(const void* A, const void* W, void* C, int M, int N, int K,
     return tff_fail("gemm: unknown operand type %d", ab_dtype);
 }
 
-// C = act(A . W^T), act one of unary_activation's kinds, where the product's plan lets its last kernel apply it: the streaming
-// kernel, or the sum over the parts of a split K (tff_gemm_takes_unary).  Else 0 there, and the activation is a kernel of its own.
+// C = act(A . W^T), act one of unary_activation's kinds, where the product's plan lets a kernel apply it to float32 sums: the streaming
+// kernel, or the sum over the parts of a split K, which may be one (unary_in_float32).  Else 0 there, and the activation is a kernel of its own.
 TFF_API int tff_gemm_takes_unary(int M, int N, int K) {
     const GemmPlan p = plan_for(M, N, K, false, false);
-    return p.tile == 0 || p.splits > 1;
+    return p.tile == 0 || p.splits > 1 || unary_in_float32(p, M, N, K);
+}
+// Room for its float32 sums.
+TFF_API size_t tff_gemm_unary_workspace_bytes(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const GemmPlan p = plan_for(M, N, K, false, false);
+    return p.splits > 1 || unary_in_float32(p, M, N, K) ? (size_t)p.splits * M * N * sizeof(float) : 0;
 }
 TFF_API int tff_gemm_unary(const void* A, const void* W, void* C, int M, int N, int K, int lda, int c_dtype, int kind, void* workspace,
                            size_t workspace_bytes, tff_stream_t stream) {

@@ -6,7 +6,7 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
 from .build import ensure_built
 
-ABI_VERSION = 48
+ABI_VERSION = 49
 
 
 class KernelLibraryError(RuntimeError):
@@ -46,6 +46,7 @@ _SIGNATURES = {
     "tff_gemm": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _F, _F, _F, _P, _Z, _I, _P],
     "tff_gemm_workspace_bytes": [_I, _I, _I, _I, _I, _I],
     "tff_gemm_takes_unary": [_I, _I, _I],
+    "tff_gemm_unary_workspace_bytes": [_I, _I, _I],
     "tff_gemm_unary": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _Z, _P],
     "tff_gemm_planes_supported": [_I, _I],
     "tff_gemm_planes": [_P, _Z, _P, _P, _I, _I, _I, _I, _I, _P],

@@ -451,8 +451,9 @@ UNARY = {"tanh": 1, "gelu": 2, "gelu_tanh": 3, "relu2": 4}
 
 
 def linear_unary(x: torch.Tensor, weight, act: str, out_dtype: torch.dtype) -> torch.Tensor:
-    """``act(x . weight^T)`` in ``out_dtype``: ``act`` tanh, gelu, gelu_tanh or relu2.  In the product's last kernel where that is the
-    streaming kernel (a few rows) or the sum over a split K's parts, else a kernel of its own over the product."""
+    """``act(x . weight^T)`` in ``out_dtype``: ``act`` tanh, gelu, gelu_tanh or relu2.  To float32 sums in the product's last
+    kernel where that is the streaming kernel (a few rows) or the sum over the parts of K (some hundred rows: one part and more), else a
+    kernel of its own over the product."""
     packed = isinstance(weight, PackedWeight)
     if packed and isinstance(x, torch.Tensor) and x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and x.stride(1) == 1 \
             and x.shape[1] == weight.shape[1] and not weight.glu_out and x.shape[0] > 0:
@@ -464,7 +465,7 @@ def linear_unary(x: torch.Tensor, weight, act: str, out_dtype: torch.dtype) -> t
         if key not in _takes_unary_cache:
             _takes_unary_cache[key] = bool(L.tff_gemm_takes_unary(M, N, K))
         if _takes_unary_cache[key] and lda >= K and lda % 8 == 0 and x.data_ptr() % 16 == 0:
-            ws_bytes = L.tff_gemm_workspace_bytes(M, N, K, dtype_code(x.dtype), 0, 0)
+            ws_bytes = L.tff_gemm_unary_workspace_bytes(M, N, K)
             ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device) if ws_bytes else None
             out = torch.empty(M, N, dtype=out_dtype, device=x.device)
             _lib.check(L.tff_gemm_unary(x.data_ptr(), weight.data_ptr(), out.data_ptr(), M, N, K, lda, dtype_code(out_dtype), UNARY[act],
