@@ -1,9 +1,15 @@
 """The host's rules between kernels: which steps the recurrences take in chunks on the matrix cores (the dispatch asks the kernels' own
-rule, and what the rule refuses stays with the forms that have no such limit), and when the draw forms the maxima of runs."""
+rule, and what the rule refuses stays with the forms that have no such limit), when the draw forms the maxima of runs, and what the
+sources' inline assembly keeps to."""
+import glob
+import os
+import re
 import types
 
 import pytest
 import torch
+
+from tffinfer_amd.kernels import build
 
 
 def _lib():
@@ -203,3 +209,19 @@ def test_an_experts_pairs_lie_together_and_cover_its_tiles(counts, col_blocks):
         assert seen == want
         assert all(first <= i // col_blocks < first + n for i in range(first * col_blocks, (first + n) * col_blocks))
         first += n
+
+
+def test_loads_into_lds_leave_a_wait_state_behind_m0():
+    """A load into LDS takes its LDS address from M0 and may follow the scalar instruction that writes it one wait state later at the earliest.
+    The compiler does not look into inline assembly, so every piece of it that writes M0 has an instruction between the two."""
+    pieces = 0
+    for path in sorted(glob.glob(os.path.join(build.CSRC_DIR, "*.h")) + glob.glob(os.path.join(build.CSRC_DIR, "*.hip"))):
+        with open(path) as f:
+            for text in re.findall(r'asm volatile\(((?:\s*"[^"]*")+)', f.read()):
+                lines = "".join(re.findall(r'"([^"]*)"', text)).replace("\\t", "").split("\\n")
+                for first, second in zip(lines, lines[1:]):
+                    if re.match(r"s_\w+ m0,", first):
+                        pieces += 1
+                        assert "_lds_" not in second, (os.path.basename(path), lines)
+                assert "_lds_" not in lines[0], (os.path.basename(path), lines)      # (M0 is written beside its load)
+    assert pieces >= 7, pieces
