@@ -197,6 +197,30 @@ def test_embedding_of_a_table_without_a_head(H):
     assert _err(OutputHead(50, H, tied_to=late).forward(ctx, y), table.double()[[3, 49, 0]] @ table.double().T) < 1e-5
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_embedding_keeps_its_rows(dtype):
+    """A table on the GPU that the caller writes again after loading does not change the model's bfloat16 rows, whatever type it came in, and rows
+    stay where a captured lookup finds them when the table is asked for as a product's weight."""
+    from tffinfer_amd.engine.runner import LayerContext
+    from tffinfer_amd.kernels import ops
+    from tffinfer_amd.parts import Embedding, OutputHead
+    table = torch.randn(50, 24).to(dtype).to(DEV)
+    rows = table.to(torch.bfloat16).float()[[3, 49, 0]]
+    ids = torch.tensor([3, 49, 0], dtype=torch.int32, device=DEV)
+    ctx = LayerContext(ops, torch.bfloat16, None, 0)
+    emb = Embedding(50, 24)
+    emb.load_weights({"weight": table}, torch.bfloat16, DEV)
+    table.zero_()
+    assert torch.equal(emb.forward(ctx, ids), rows)
+    place = emb._table.data_ptr()
+    head = OutputHead(50, 24, tied_to=emb)
+    assert isinstance(head.weight, ops.PackedWeight) and head.weight is emb.weight
+    assert emb._table.data_ptr() == place and torch.equal(emb.forward(ctx, ids), rows)
+    emb.weight = torch.ones(50, 24, dtype=torch.bfloat16, device=DEV)      # (a table set by hand replaces both)
+    assert bool((emb.forward(ctx, ids) == 1).all()) and isinstance(emb.weight, ops.PackedWeight)
+    assert float((head.forward(ctx, torch.ones(1, 24, dtype=torch.bfloat16, device=DEV)) - 24).abs().max()) == 0
+
+
 def test_embedding_and_tied_head():
     from tffinfer_amd.engine.runner import LayerContext
     from tffinfer_amd.kernels import ops

@@ -50,7 +50,8 @@ class Embedding(Part):
         self.scale = float(scale)
         self.norm = norm
         self.serves_head = False        # a tied head multiplies by the table
-        self._table = None
+        self._table = None              # what rows are looked up in
+        self._product = None            # the same as products read it, of a table that stays row-major
 
     def children(self):
         return {"norm": self.norm} if self.norm is not None else {}
@@ -60,18 +61,25 @@ class Embedding(Part):
 
     def load_weights(self, weights, dtype, device):
         table = weights["weight"]
-        self._table = to_device(table, dtype, device) if self.serves_head else table.to(dtype).contiguous().to(device)
+        if self.serves_head:
+            self.weight = to_device(table, dtype, device)
+            return
+        out = table.to(dtype).contiguous().to(device)
+        if out.is_cuda and out.dtype == torch.bfloat16 and out.data_ptr() == table.data_ptr():
+            out = out.clone()           # (as of a table put into the products' order: what becomes of the caller's tensor is not the model's)
+        self.weight = out
 
     @property
     def weight(self):
-        """The table as products read it (``to_device``); one that was only looked up is put into that order first."""
-        if isinstance(self._table, torch.Tensor):
-            self._table = to_device(self._table, self._table.dtype, self._table.device)
-        return self._table
+        """The table as products read it (``to_device``).  Of one that was only looked up a copy in that order is made and kept; the
+        rows stay where they are, where a captured step may look them up."""
+        if isinstance(self._table, torch.Tensor) and self._product is None:
+            self._product = to_device(self._table, self._table.dtype, self._table.device)
+        return self._table if self._product is None else self._product
 
     @weight.setter
     def weight(self, table):
-        self._table = table
+        self._table, self._product = table, None
 
     def state_spec(self) -> StateSpec | None:
         """State per request that the embedding carries from step to step."""
@@ -115,7 +123,7 @@ class OutputHead(Part):
         self.tied_to = tied_to
         if tied_to is not None:
             tied_to.serves_head = True
-            tied_to.weight              # (a table that is loaded already is put into the products' order here)
+            tied_to.weight              # (of a table that is loaded already the copy for products is made here)
         self.softcap = float(softcap) if softcap else 0.0
         self.scale = float(scale) if scale is not None else 1.0
         self._weight = None
