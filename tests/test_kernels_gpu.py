@@ -529,6 +529,49 @@ def test_linear_of_few_units_of_k(M, N, units):
     _close(y, ops.linear(x.float(), w.float()), 3e-5, "product")
 
 
+@pytest.mark.parametrize("M,N,K,lda", [
+    (20, 100, 128, 70 << 20), (60, 2048, 512, 35 << 20), (70, 64, 4096, 35 << 20),                              # tiles of 32 and 64 rows
+    (100, 18432, 4096, 17 << 20), (300, 34816, 320, 17 << 20),                                                  # of 128
+    (234, 18432, 4096, 9 << 20), (130, 40000, 64, 9 << 20), (260, 65536, 64, 9 << 20),                          # of 256
+    (17, 32, (1 << 24) + 64, 0), (65, 32, (1 << 24) + 64, 0)])                                                  # weights beyond 32-bit offsets
+def test_linear_of_rows_far_apart(M, N, K, lda):
+    """Rows, strides and weights that the four-wave tiles' 32-bit offsets do not reach: the same product as of the rows one behind the other
+    (K of 16 million: against 64 bits, where a float32 sum of K / 256 terms and more in a row may lose 2^-8 of itself)."""
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).bfloat16()
+    pw, gated = ops.pack_weight(w), ops.pack_gate_up(w[:N // 2].contiguous(), w[N // 2:].contiguous())
+    if lda:
+        far = torch.empty((M - 1) * lda + K, dtype=torch.bfloat16, device=DEV).as_strided((M, K), (lda, 1))
+        far.copy_(x)
+        ref, ref_gated, tol = ops.linear(x, pw, out_dtype=torch.float32), ops.linear(x, gated, out_dtype=torch.float32), 3e-5
+    else:
+        far, at = x, 1 << 22
+        ref = sum(x[:, i:i + at].double() @ w[:, i:i + at].double().T for i in range(0, K, at))
+        ref_gated, tol = torch.nn.functional.silu(ref[:, :N // 2]) * ref[:, N // 2:], 2.0 ** -8
+    _close(ops.linear(far, pw, out_dtype=torch.float32), ref, tol, "rows far apart")
+    _close(ops.as_tensor(ops.linear(far, pw, out_dtype=torch.float32, partials=True)), ref, tol, "rows far apart, parts kept")
+    _close(ops.linear(far, gated, out_dtype=torch.float32), ref_gated, tol, "rows far apart, gated")
+    if lda:
+        _close(ops.linear_unary(far, pw, "gelu", torch.float32), torch.nn.functional.gelu(ref), tol, "rows far apart, an activation")
+
+
+def test_planes_of_rows_far_apart():
+    """Several products in one call whose rows the tiles' offsets do not reach go one after the other."""
+    ops = _ops()
+    from tffinfer_amd.kernels import lib
+    M, P, N, K, lda = 20, 3, 128, 192, 70 << 20
+    g = torch.Generator(device=DEV).manual_seed(5)
+    x = torch.randn(P, M, K, generator=g, device=DEV).bfloat16()
+    pw = ops.pack_weight((torch.randn(P * N, K, generator=g, device=DEV) * 0.1).bfloat16())
+    far = torch.empty((M - 1) * lda + P * K, dtype=torch.bfloat16, device=DEV)
+    far.as_strided((P, M, K), (K, lda, 1)).copy_(x)
+    out = torch.empty(P, M, N, device=DEV)
+    lib.check(lib.load().tff_gemm_planes(far.data_ptr(), K, pw.data_ptr(), out.data_ptr(), P, M, N, K, lda, torch.cuda.current_stream().cuda_stream))
+    _close(out, ops.linear_planes(x, pw), 3e-5, "planes of rows far apart")
+
+
 @pytest.mark.parametrize("M,N,K", [(2600, 6144, 264), (4500, 520, 200), (1100, 300, 96), (9000, 130, 64),
                                    (2304, 2100, 72)])
 def test_linear_with_many_row_tiles(M, N, K):

@@ -751,6 +751,11 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     }
 }
 
+// Whether a tile's offsets fit (see launch_far).
+static bool w4_reaches(int rows, int cols, int K, int lda) {
+    return (size_t)(rows - 1) * lda * 2 + 128 < (1ull << 32) && (size_t)(cols / 16) * (K / 32) * 1024 < (1ull << 32);
+}
+
 // splits > 1: the blocks of a tile split K among them in units of 64; part holds splits * M * N floats
 template <int WTN, int NWS, bool GLU = false, int WGM = 2, bool SCALE = false, int WTM = 8>
 static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmExtra ex, int c_dtype,
@@ -766,8 +771,7 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
     const long TM = (M + BM - 1) / BM, TN = (N + BN - 1) / BN;
     const long tiles = w4_blocks<BM>(TM, TN);   // eight equal shares
     TFF_REQUIRE(tiles < (1L << 31), "gemm: too many tiles for M=%d N=%d", M, N);
-    TFF_REQUIRE((size_t)(BM - 1) * lda * 2 + 128 < (1ull << 32) && (size_t)(BN / 16) * KB * 1024 < (1ull << 32),
-                "gemm: rows of %d elements at a stride of %d are too long", K, lda);
+    TFF_REQUIRE(w4_reaches(BM, BN, K, lda), "gemm: rows of %d elements at a stride of %d are too long", K, lda);
     const dim3 grid((unsigned)tiles, 1, splits);
     // the blocks of a split K leave plain float32 sums, plane by plane; a gate is applied when they are added up
     if (ex.plane_cols) {
@@ -1396,6 +1400,19 @@ static int skinny_for(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, 
     return launch_skinny<1, 1, 8, 4, 1, false, false, EPI>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, fuse);
 }
 
+// The four-wave tiles address a block's rows and its columns of W by 32-bit offsets.  Rows or a stride too long for a plan's tile (256 rows
+// 8.4 million elements apart, K of 11 million on 192 columns) go to the sixteen-wave kernel, which has 64 bits a copy, K in as many parts.
+template <bool GLU>
+static int launch_far(const GemmPlan& plan, const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmExtra ex, int c_dtype,
+                      int n_out, hipStream_t s, float* part, bool reduce) {
+    TFF_REQUIRE((size_t)15 * lda * 2 + 128 < (1ull << 32), "gemm: row stride %d too large", lda);
+    if (plan.tile <= 64) return launch_async_g<2, 2, 2, 4, 3, GLU>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
+    if (plan.tile == 128 && plan.bn == 128)
+        return launch_async_g<2, 2, 4, 4, 3, GLU>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
+    if (plan.tile == 128) return launch_async_g<2, 4, 4, 4, 3, GLU>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
+    return launch_async_g<4, 4, 4, 4, 5, GLU, 1, true>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
+}
+
 // glu_out > 0: W holds gate and up groups in turn (N = 2 * ceil16(glu_out) rows) and C is
 // [M, glu_out] = silu(gate) * up.  workspace: room for partial sums (tff_gemm_workspace_bytes);
 // with less the blocks do not split K.
@@ -1417,6 +1434,16 @@ int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int 
     if (!workspace || workspace_bytes < (size_t)plan.splits * M * N * sizeof(float)) plan.splits = 1;
     const int S = plan.splits;
     const bool red = !keep_partials;
+    const bool far = plan.tile > 0 && K % 64 == 0 && !w4_reaches(plan.tile, plan.bn, K, lda);
+    if (far && ex.plane_cols) {      // (one product after the other)
+        GemmExtra one = ex;
+        one.plane_cols = 0;
+        const size_t w_plane = (size_t)(ex.plane_cols / 16) * (K / 32) * 512;
+        for (int p = 0; p < N / ex.plane_cols; ++p)
+            if (int rc = tff_gemm_bf16(A + p * ex.a_step, Wp + p * w_plane, (float*)C + (size_t)p * M * ex.plane_cols, M, ex.plane_cols, K, lda, one,
+                                       c_dtype, 0, nullptr, 0, 0, s)) return rc;
+        return 0;
+    }
     if (ex.unary && glu_out == 0 && !keep_partials && planned_splits == 1 && unary_in_float32(plan, M, N, K) && workspace &&
         workspace_bytes >= (size_t)M * N * sizeof(float)) {
         // K in one part, whose float32 results the sum's kernel takes as the only plane
@@ -1433,6 +1460,7 @@ int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int 
         TFF_REQUIRE(N % 32 == 0 && glu_out <= N / 2 && glu_out > N / 2 - 16,
                     "gemm: a gated weight of %d rows does not fit %d output columns", N, glu_out);
         if (plan.tile == 0) return skinny_for<0>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, nullptr);
+        if (far) return launch_far<true>(plan, A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, workspace, true);
         if (plan.tile <= 64 && K % 64 == 0) {                // the four waves side by side on 64 or 32 rows
             if (plan.tile == 32 && plan.bn == 128) return launch_w4<2, 5, true, 1, false, 2>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
             if (plan.tile == 32) return launch_w4<4, 5, true, 1, false, 2>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
@@ -1465,6 +1493,7 @@ int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int 
             if (M <= 32) return launch_skinny<2, 2, 4, 8>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s);
             return launch_skinny<4, 2, 4, 8>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s);
         }
+        if (far) return launch_far<false>(plan, A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, workspace, red);
         if (K % 64 == 0) {                                   // the four waves side by side on 64 or 32 rows
             if (plan.tile == 32 && plan.bn == 128) return launch_w4<2, 5, false, 1, false, 2>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
             if (plan.tile == 32) return launch_w4<4, 5, false, 1, false, 2>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
@@ -1473,6 +1502,7 @@ int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int 
         }
         return launch_async_g<2, 2, 2, 4, 3>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
     }
+    if (far) return launch_far<false>(plan, A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, workspace, red);
     if (K % 64 == 0) {
         if (plan.tile == 128) {
             if (plan.bn == 128) return launch_w4<2, 5, false, 1>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
@@ -1549,7 +1579,7 @@ TFF_API int tff_gemm_row_scaled(const void* A, const void* Wp, void* C, int M, i
         TFF_REQUIRE(N % 32 == 0 && glu_out <= N / 2 && glu_out > N / 2 - 16,
                     "gemm_row_scaled: a gated weight of %d rows does not fit %d output columns", N, glu_out);
     // (the four-wave kernel's tiles of 32 rows take the rows' factors into their epilogue too)
-    if (glu_out > 0 && few_rows_gated_on_tiles(M, N, K)) {
+    if (glu_out > 0 && few_rows_gated_on_tiles(M, N, K) && w4_reaches(32, plan_rows32(N, K), K, lda)) {
         const W4Scale sc{ss, ss_stride, ss_count, 1.0f / (float)dim, eps};
         const bf16_t* a = (const bf16_t*)A;
         const bf16_t* w = (const bf16_t*)Wp;
