@@ -70,6 +70,21 @@ def test_key_groups_and_blocks_follow_the_amount_of_work():
     assert (blocks, groups) == (64, 1)
 
 
+def test_portions_take_the_blocks_that_end_first():
+    """Short portions the blocks of eight waves, which begin and end sooner; longer ones those of four waves, with two key groups while
+    there is no more than an item a block, with one where items of 256 columns spare a round; whatever the order of the portions."""
+    from tffinfer_amd.kernels.ops import _prompt_blocks
+    def pick(entries, G=4, nkv=8, window=0, d=128):
+        return _prompt_blocks(_batch(entries), G, nkv, window, "cpu", "all", d, num_cus=256)
+    assert [pick([(0, n)]) for n in (17, 96, 150, 333, 901, 2048, 6000, 32768)] == [0, 0, 0, 0, 2, 2, 1, 1]
+    assert [pick([(0, n)], 32, 1, 0, 256) for n in (17, 96, 333, 6000)] == [0, 0, 1, 1]
+    assert pick([(0, 901)], 5) == 2 and pick([(0, 333)], 1, 2) == 0
+    mixed = [(0, 700), (2000, 300), (50, 20), (8000, 90)]
+    assert pick(mixed, 4, 8, 1024) == pick(mixed[::-1], 4, 8, 1024) == 2 and pick(mixed) == 2
+    assert pick([(9000, 500)]) == 2 and pick([(0, 40)] * 8) == 0
+    assert pick([(0, 5), (100000, 40)] * 300) in (1, 2)      # more items than are dealt to find the longest block
+
+
 def test_staged_tables_keep_shape_and_type_on_the_host():
     """The staging module's host form (what the work lists' tests above go through): every
     column comes back as a tensor of its own shape and element type, a copy of the array."""

@@ -1203,6 +1203,20 @@ def test_attention_mfma_long_portions(nq, nkv, d, ps, window, bins, groups):
             _close(out.reshape(T, nq, d)[mine], ref, ATTN_TOL, f"block attention, request {r}")
 
 
+@pytest.mark.parametrize("nq,nkv,d,window,entries", [
+    (8, 2, 128, 0, [(0, 17)]), (5, 1, 128, 0, [(0, 150), (33, 40)]), (8, 2, 128, 40, [(0, 333), (500, 64), (7, 1)]),
+    (32, 1, 256, 0, [(0, 3)]), (6, 1, 256, 30, [(0, 96), (200, 33)])])
+def test_short_portions_take_blocks_of_eight_waves(nq, nkv, d, window, entries):
+    """The step as it comes, on the blocks that the rule names, against the general kernel."""
+    ops = _ops()
+    batch, kv, ks, vs, positions, token_req = _fake_step(entries, 16, nkv, d, torch.bfloat16, seed=nq + d)
+    q = torch.randn(batch.num_tokens, nq * d, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to(DEV)
+    out = ops.attention_mfma(q, nq, nkv, d, kv, batch, window)
+    assert ops._prompt_blocks(batch, nq // nkv, nkv, window, DEV, "multi" if any(n == 1 for _, n in entries) and batch.max_context >= 256 else "all", d) == 0
+    gen = ops.attention_generic(q, nq, nkv, d, kv.k_cache, kv.v_cache, kv.block_tables, batch.token_req, batch.positions, window, 1 / math.sqrt(d))
+    _close(out, gen.double(), ATTN_TOL, "short portions against the general kernel")
+
+
 @pytest.mark.parametrize("bins", [None, 3, 1])
 @pytest.mark.parametrize("nq,nkv,d,ps,window", [
     (32, 8, 128, 16, 0), (8, 2, 32, 8, 300), (6, 3, 48, 8, 0), (5, 1, 128, 32, 0), (40, 2, 96, 8, 77),

@@ -1331,13 +1331,10 @@ static int launch_attn(const bf16_t* q, int q_stride, bf16_t* out, float* part_o
                 attn_mfma_block_kernel<DT, 1, 8, 1><<<dim3(num_blocks, nkv), 512, 0, s>>>(
                     q, q_stride, out, k_cache, v_cache, block_tables, bt_stride, cu_tokens, start_pos, work,
                     block_items, nq, nkv, page_size, page_shift, window, scale, sinks, softcap, pool_tables, pt_stride, pool);
-        } else if constexpr (DT < 16) {
+        } else
             attn_mfma_block_kernel<DT, 1, 8, 1><<<dim3(num_blocks, nkv), 512, 0, s>>>(
                 q, q_stride, out, k_cache, v_cache, block_tables, bt_stride, cu_tokens, start_pos, work,
                 block_items, nq, nkv, page_size, page_shift, window, scale, sinks, softcap, pool_tables, pt_stride, pool);
-        } else {
-            return tff_fail("attention_mfma: long portions of heads of 256 are attention_prompt's");
-        }
         return tff_check_launch("attention_mfma_block");
     }
     const dim3 grid(num_work, nkv, max(splits, 1));
@@ -1443,9 +1440,6 @@ TFF_API int tff_attention_mfma(const void* q, int q_stride, void* out, float* pa
     TFF_REQUIRE(work || tiles_per_entry >= 1, "attention_mfma: neither a work table nor a tile count");
     TFF_REQUIRE(bt_stride > 0 && num_pages > 0 && window >= 0 && T_total >= 0, "attention_mfma: bad geometry");
     if (num_work <= 0) return 0;
-    if (d == 256 && cols_per_wave == 128 && pool == 0)
-        return tff_attention_prompt(q, q_stride, out, k_cache, v_cache, block_tables, bt_stride, cu_tokens, start_pos, work, num_work,
-                                    block_items, num_blocks, 1, nq, nkv, d, page_size, num_pages, window, scale, sinks, stream);
     hipStream_t s = (hipStream_t)stream;
 #define TFF_ATTN_CASE(DTV)                                                                          \
     case DTV * 16:                                                                                  \

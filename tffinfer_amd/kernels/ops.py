@@ -694,6 +694,37 @@ def _num_cus(device) -> int:
     return _cu_count[idx]
 
 
+def _block_items(batch, G: int, window: int, cols: int, which: str, pool: int = 0) -> list[tuple[int, int, int]]:
+    """(32-key slices, entry, first column) of the items of ``cols`` columns of the step's entries."""
+    cu, P = batch.host_cu_tokens, batch.host_start_pos
+    items = []
+    for r in _entries(batch, which):
+        ncols = (cu[r + 1] - cu[r]) * G
+        for c0 in range(0, ncols, cols):
+            first = P[r] + c0 // G
+            last = P[r] + (min(c0 + cols, ncols) - 1) // G
+            lo = max(0, first - window + 1) if window > 0 else 0
+            blocks = max(0, last - window + 1) // pool if pool else 0      # keys of blocks before the window
+            items.append((last // 32 - lo // 32 + 1 + -(-blocks // 32), r, c0))
+    return items
+
+
+def _deal_items(items: list, nbins: int) -> list[list]:
+    """The items of every block: one each, the longest first, or with more items than blocks the longest first, each to the block with
+    the least to do so far."""
+    if len(items) <= nbins:
+        return [[it] for it in sorted(items, reverse=True)]
+    import heapq
+    loads = [(0, b) for b in range(nbins)]
+    heapq.heapify(loads)
+    per_bin = [[] for _ in range(nbins)]
+    for it in sorted(items, reverse=True):
+        load, b = heapq.heappop(loads)
+        per_bin[b].append(it)
+        heapq.heappush(loads, (load + it[0], b))
+    return per_bin
+
+
 def _attention_block_work(batch, G: int, nkv: int, window: int, device, cols: int = 128,
                           bins: int | None = None, which: str = "all", key_groups: int | None = None,
                           head_dim: int = 128, num_cus: int | None = None, pool: int = 0):
@@ -710,16 +741,7 @@ def _attention_block_work(batch, G: int, nkv: int, window: int, device, cols: in
         cache = batch._attn_work = {}
     key = ("blocks", G, nkv, cols, window, bins, which, key_groups, head_dim, num_cus) + ((pool,) if pool else ())
     if key not in cache:
-        cu, P = batch.host_cu_tokens, batch.host_start_pos
-        items = []                       # (slices, entry, first column)
-        for r in _entries(batch, which):
-            ncols = (cu[r + 1] - cu[r]) * G
-            for c0 in range(0, ncols, cols):
-                first = P[r] + c0 // G
-                last = P[r] + (min(c0 + cols, ncols) - 1) // G
-                lo = max(0, first - window + 1) if window > 0 else 0
-                blocks = max(0, last - window + 1) // pool if pool else 0      # keys of blocks before the window
-                items.append((last // 32 - lo // 32 + 1 + -(-blocks // 32), r, c0))
+        items = _block_items(batch, G, window, cols, which, pool)
         if num_cus is None:
             num_cus = _num_cus(device) if torch.device(device).type == "cuda" else 256
         per_cu = max(1, num_cus // max(1, nkv))
@@ -731,23 +753,10 @@ def _attention_block_work(batch, G: int, nkv: int, window: int, device, cols: in
         if head_dim > 128:
             groups = 1                   # LDS holds one group's stages there
         nbins = bins if bins is not None else (per_cu if groups == 2 or head_dim > 128 else 2 * per_cu)
-        if len(items) <= nbins:
-            order = sorted(items, reverse=True)        # the longest start first
-            starts = list(range(len(order) + 1))
-        else:
-            # longest first, each to the block with the least to do so far
-            import heapq
-            loads = [(0, b) for b in range(nbins)]
-            heapq.heapify(loads)
-            per_bin = [[] for _ in range(nbins)]
-            for it in sorted(items, reverse=True):
-                load, b = heapq.heappop(loads)
-                per_bin[b].append(it)
-                heapq.heappush(loads, (load + it[0], b))
-            order, starts = [], [0]
-            for lst in per_bin:
-                order.extend(lst)
-                starts.append(len(order))
+        order, starts = [], [0]
+        for lst in _deal_items(items, nbins):
+            order.extend(lst)
+            starts.append(len(order))
         flat = [x for it in order for x in it[1:]]
         items_d, starts_d = _staging.send(device, [np.asarray(flat, dtype=np.int32).reshape(-1, 2),
                                                    np.asarray(starts, dtype=np.int32)])
@@ -920,9 +929,10 @@ def attention_mfma(q: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, window
             sp = splits if splits is not None else pick_splits(work.shape[0] * nkv, reach)
             launch(work, work.shape[0], None, 0, 1, 16, sp, cache["single_rows"])
     if cols == 128 and d in PROMPT_HEAD_SIZES and not pool and softcap == 0.0 and block_cols is None:
-        groups = 1 if d > 128 else key_groups or _prompt_key_groups(batch, G, nkv, int(window), q.device, which)
-        attention_prompt(q, out, nq, nkv, d, kv, batch, int(window), scale, sinks, which, groups, block_bins)
-        return out
+        groups = (1 if d > 128 else key_groups) if key_groups else _prompt_blocks(batch, G, nkv, int(window), q.device, which, d)
+        if groups:
+            attention_prompt(q, out, nq, nkv, d, kv, batch, int(window), scale, sinks, which, groups, block_bins)
+            return out
     if cols == 128:
         bcols = 128 if pool else block_cols or _pick_block_cols(batch, G, nkv, int(window), q.device, which, d)
         if bcols == 256:
@@ -948,29 +958,41 @@ def attention_mfma(q: torch.Tensor, nq: int, nkv: int, d: int, kv, batch, window
 PROMPT_HEAD_SIZES = (128, 256)
 
 
-def _prompt_key_groups(batch, G: int, nkv: int, window: int, device, which: str) -> int:
-    """One group of four waves on items of 256 columns, or two of two waves that share the slices of items of 128, for heads of 128: by
-    what the block with the most to do takes.  A step (a slice of an item, of two slices with two groups) is some 0.82 and 0.90 us,
-    what an item has before its first and after its last step 7 and 10 us (measured with 32 query and 8 key heads, one / two
-    groups, us: 901 tokens 33 / 25, 1,500 47 / 38, 2,048 61 / 52, 3,000 88 / 100, 4,096 141 / 165, 16,384 1,793 / 2,024; 3,001 and
-    1,700 tokens of 16 and 4 heads in a window of 1,024 45 / 61)."""
+#: what a block takes in us by head size and form: before it begins, for a step, for an item.  Form 0 is the blocks of eight waves, 1 and 2 those of four
+#: waves with one key group and two; columns of an item, and slices of 32 keys of a step
+_PROMPT_FORMS = {128: {0: (0.9, 1.24, 9.0, 128, 2), 1: (-1.6, 0.80, 13.9, 256, 1), 2: (1.8, 0.83, 11.0, 128, 2)},
+                 256: {0: (0.2, 1.27, 10.4, 128, 1), 1: (1.1, 0.74, 12.2, 128, 1)}}
+
+
+def _prompt_blocks(batch, G: int, nkv: int, window: int, device, which: str, d: int, num_cus: int | None = None) -> int:
+    """Which blocks the step's portions take at head sizes of :data:`PROMPT_HEAD_SIZES`: 0 those of eight waves, 1 and 2 those of four with so
+    many key groups (one on items of 256 columns; two that share the slices of items of 128), by what the block with the most to do takes.
+
+    Four waves take less for a step and more before an item's first and behind its last.  The numbers are fitted to 4,678 steps of 1 to 16
+    portions, twelve and six pairs of head counts, windows of 512 to 4,096 or none, every form timed: the pick is 0.2 % from the best form on
+    average (of 1,386 further steps too), and behind the blocks of eight waves by 2 % in one of a hundred.  us, eight waves / four, one group / two, 32 query and 8 key heads:
+    17 tokens 9.8 / 10.6 / 12.1, 150 12.9 / 15.6 / 14.5, 333 16.7 / 20.4 / 17.5, 901 29.5 / 36.1 / 26.4, 2,048 64 / 66 / 56, 6,000 417 / 281 / 299;
+    portions of 700, 300, 20 and 90 tokens in a window of 1,024 34.7 / 43.6 / 30.9.  A head size of 256, 32 heads on one: 17 tokens 11.9 / 13.7,
+    333 25.3 / 22.6."""
     cache = getattr(batch, "_attn_work", None)
     if cache is None:
         cache = batch._attn_work = {}
-    key = ("prompt_groups", G, nkv, window, which)
+    key = ("prompt_blocks", G, nkv, window, which, d, num_cus)
     if key not in cache:
-        cu, P = batch.host_cu_tokens, batch.host_start_pos
-        slices = []
-        for r in _entries(batch, which):
-            ncols = (cu[r + 1] - cu[r]) * G
-            for c0 in range(0, ncols, 256):
-                first, last = P[r] + c0 // G, P[r] + (min(c0 + 256, ncols) - 1) // G
-                slices.append(last // 32 - (max(0, first - window + 1) // 32 if window > 0 else 0) + 1)
-        num_cus = _num_cus(device) if torch.device(device).type == "cuda" else 256
-        bins, most, total = max(1, num_cus // max(1, nkv)), max(slices), sum(slices)
-        one = 0.82 * max(most, total / bins) + 7.0 * -(-len(slices) // bins)
-        two = 0.90 * max(most / 2, total / bins) + 10.0 * -(-2 * len(slices) // bins)
-        cache[key] = 1 if one <= two else 2
+        if num_cus is None:
+            num_cus = _num_cus(device) if torch.device(device).type == "cuda" else 256
+        bins = max(1, num_cus // max(1, nkv))
+        items = {cols: _block_items(batch, G, window, cols, which) for cols in {f[3] for f in _PROMPT_FORMS[d].values()}}
+        times = {}
+        for form, (start, step, item, cols, slices) in _PROMPT_FORMS[d].items():
+            its = items[cols]
+            if form == 0 and d <= 128 and sum(it[0] for it in its) >= 96 * 2 * bins:
+                continue                 # (long portions, where eight waves are never ahead)
+            if len(its) > min(256, 4 * bins):
+                times[form] = start + (step * sum(it[0] for it in its) / slices + item * len(its)) / bins      # (as good as even)
+            else:
+                times[form] = start + max(step * sum(-(-it[0] // slices) for it in lst) + item * len(lst) for lst in _deal_items(its, bins))
+        cache[key] = min(times, key=times.get)
     return cache[key]
 
 
