@@ -557,6 +557,35 @@ def test_linear_of_rows_far_apart(M, N, K, lda):
         _close(ops.linear_unary(far, pw, "gelu", torch.float32), torch.nn.functional.gelu(ref), tol, "rows far apart, an activation")
 
 
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 40, 100])
+@pytest.mark.parametrize("N,K", [(96, 200), (1030, 1024), (5120, 512), (5120, 4096), (34000, 256), (8256, 4096)])
+def test_weights_loaded_as_read_once(M, N, K):
+    """The same bits whether a weight's loads say that nobody asks for them again or not, in every kernel of few rows: plain, gated, with a
+    norm taken in on either side, with an activation, of several planes."""
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).bfloat16()
+    back = ops.pack_weight((torch.randn(K, N // 8 * 8, generator=g, device=DEV) * N ** -0.5).bfloat16())
+    norm = 1 + 0.1 * torch.randn(K, generator=g, device=DEV)
+    resid = torch.randn(M, K, generator=g, device=DEV)
+    plain, gated = ops.pack_weight(w), ops.pack_gate_up(w[:N // 2].contiguous(), w[N // 2:N // 2 * 2].contiguous())
+    assert not plain.once and not gated.once
+    results = []
+    for once in (False, True):
+        plain.once = gated.once = back.once = once
+        r = resid.clone()
+        out = [ops.linear(x, plain), ops.linear(x, plain, out_dtype=torch.float32), ops.linear(x, gated), ops.linear_unary(x, plain, "relu2", torch.bfloat16)]
+        y = ops.linear(out[0][:, :N // 8 * 8].contiguous(), back, out_dtype=torch.float32, partials=True)
+        rows = ops.add_rmsnorm(r, y, norm, 1e-5, torch.bfloat16, for_linear=True)
+        out += [ops.linear(rows, gated), ops.linear(rows, plain), r]
+        if N % 256 == 0 and K % 64 == 0:
+            out.append(ops.linear_planes(torch.stack([x, x]), plain))
+        results.append(out)
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
 def test_planes_of_rows_far_apart():
     """Several products in one call whose rows the tiles' offsets do not reach go one after the other."""
     ops = _ops()
@@ -568,7 +597,7 @@ def test_planes_of_rows_far_apart():
     far = torch.empty((M - 1) * lda + P * K, dtype=torch.bfloat16, device=DEV)
     far.as_strided((P, M, K), (K, lda, 1)).copy_(x)
     out = torch.empty(P, M, N, device=DEV)
-    lib.check(lib.load().tff_gemm_planes(far.data_ptr(), K, pw.data_ptr(), out.data_ptr(), P, M, N, K, lda, torch.cuda.current_stream().cuda_stream))
+    lib.check(lib.load().tff_gemm_planes(far.data_ptr(), K, pw.data_ptr(), out.data_ptr(), P, M, N, K, lda, 0, torch.cuda.current_stream().cuda_stream))
     _close(out, ops.linear_planes(x, pw), 3e-5, "planes of rows far apart")
 
 

@@ -250,3 +250,25 @@ def test_rotary_table_closed_form():
     for pos, i in ((0, 0), (1, 0), (7, 3), (99, 15)):
         ang = pos * 1e6 ** (-2 * i / 32)
         assert abs(float(t[pos, i, 0]) - math.cos(ang)) < 1e-6 and abs(float(t[pos, i, 1]) - math.sin(ang)) < 1e-6
+
+
+def test_models_beyond_the_caches_say_so_to_their_products(monkeypatch):
+    """Every packed weight of a model whose matrices the caches do not hold is loaded as read once, none of one that fits; experts' matrices
+    count, a table whose rows are looked up does not."""
+    from helpers import TINY_CONFIGS
+    from disunex_models import DISUNEX_CONFIGS
+    from tffinfer_amd.kernels import ops
+    from tffinfer_amd.models import build_model_skeleton, config_from_dict
+    for cfg in [dict(c) for c, _ in TINY_CONFIGS.values()] + [dict(c) for c, _ in DISUNEX_CONFIGS.values()]:
+        model = build_model_skeleton(config_from_dict(cfg))
+
+        def weights():
+            model.init_random(3, torch.bfloat16, DEV)
+            return [w for _, p in model._weighted_parts() for v in vars(p).values() for w in (v if isinstance(v, list) else [v])
+                    if isinstance(w, ops.PackedWeight)]
+        monkeypatch.setattr(ops, "CACHE_BYTES", 256 << 20)
+        packed = weights()
+        assert len(packed) > 2 and not any(w.once for w in packed)
+        size = sum(w.data.numel() * 2 for w in {id(w): w for w in packed}.values())
+        monkeypatch.setattr(ops, "CACHE_BYTES", size - 1)
+        assert all(w.once for w in weights())

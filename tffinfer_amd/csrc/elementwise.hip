@@ -35,7 +35,7 @@ int tff_device_cus() {
     return cached[dev];
 }
 TFF_API const char* tff_last_error() { return g_error; }
-TFF_API int tff_abi_version() { return 49; }
+TFF_API int tff_abi_version() { return 50; }
 
 // ----------------------------------------------------------------- embed ---
 // x[t, :] = E[token[t], :]   (reference: src/kernel/cpu/embedding.cpp:34-49,

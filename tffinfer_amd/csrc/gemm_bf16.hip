@@ -20,8 +20,10 @@
 
 
 __device__ __forceinline__ uint4 ld16(const bf16_t* p) { return *reinterpret_cast<const uint4*>(p); }
-// The same of a weight that one block reads once.
-__device__ __forceinline__ uint4 ld16_once(const bf16_t* p) {
+// The same of a weight that one block reads; ONCE: and that nobody asks for again before it has left the caches.
+template <bool ONCE>
+__device__ __forceinline__ uint4 ld16_weight(const bf16_t* p) {
+    if constexpr (!ONCE) return ld16(p);
     typedef __attribute__((__vector_size__(16))) unsigned once_t;
     const once_t v = __builtin_nontemporal_load(reinterpret_cast<const once_t*>(p));
     return make_uint4(v[0], v[1], v[2], v[3]);
@@ -61,6 +63,10 @@ struct GemmExtra : GemmEpilogue {
     int unary;
     int plane_cols;
     size_t a_step;
+};
+// And what only the launches ask.  once: no cache holds the weight from one call to the next (see the streaming kernel's note).
+struct GemmCall : GemmExtra {
+    int once;
 };
 
 // GLU: the 16-row groups of W alternate between a gate and an up projection
@@ -360,7 +366,7 @@ static int launch_reduce(const float* part, int S, int M, int N, void* C, int n_
 // splits > 1: the blocks of a tile split K among them; part holds splits * M * N floats
 template <int WGM, int WGN, int WTM, int WTN, int STAGES, bool GLU = false, int KPS = 2, bool EARLY = false>
 static int launch_async_g(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda,
-                          const GemmExtra ex, int c_dtype, int n_out, hipStream_t s, int splits = 1, float* part = nullptr,
+                          const GemmCall ex, int c_dtype, int n_out, hipStream_t s, int splits = 1, float* part = nullptr,
                           bool reduce = true) {
     const int KB = (K + 31) / 32;
     constexpr int BM = WGM * WTM * 16, BN = WGN * WTN * 16;
@@ -536,8 +542,8 @@ struct W4Scale {
 };
 // PLANES: several products in one launch (GemmExtra).  A kernel of its own: a test of plane_cols in every product cost those of a short
 // prompt up to 1.5 % (gate+up of 560 rows 34.5 / 35.0 us).
-// ONCE: the block reads its columns of W alone (see launch_w4; SCALE: always so).
-template <int WTN, int NWS, bool GLU, typename TC, int WGM = 2, bool SCALE = false, int WTM = 8, bool PLANES = false, bool ONCE = SCALE>
+// ONCE: the block reads its columns of W alone, and no later call finds them in a cache (see launch_w4).
+template <int WTN, int NWS, bool GLU, typename TC, int WGM = 2, bool SCALE = false, int WTM = 8, bool PLANES = false, bool ONCE = false>
 __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, TC* __restrict__ C, int M, int N,
     int K, int lda, int KB, int n_out, W4Scale sc,
@@ -758,7 +764,7 @@ static bool w4_reaches(int rows, int cols, int K, int lda) {
 
 // splits > 1: the blocks of a tile split K among them in units of 64; part holds splits * M * N floats
 template <int WTN, int NWS, bool GLU = false, int WGM = 2, bool SCALE = false, int WTM = 8>
-static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmExtra ex, int c_dtype,
+static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmCall ex, int c_dtype,
                      int n_out, hipStream_t s, int splits = 1, float* part = nullptr, bool reduce = true,
                      W4Scale sc = W4Scale{nullptr, 0, 0, 0.f, 0.f}) {
     TFF_REQUIRE(!SCALE || (M <= 16 && sc.ss && (splits <= 1 || !part)),
@@ -795,10 +801,8 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
     // A weight that one block reads, K in one part: 40 and 100 rows of 24,576 x 4,096 38.0 / 35.6 and 43.9 / 40.7 us, 17 rows of 151,936
     // 218 / 192 (plain loads / once).  The short streams of a split K lose by it: 100 rows of 4,096 x 4,096 16.3 / 19.4, 128 of
     // 7,168 x 5,120 24.8 / 27.8.  (256 rows are two waves' of A, and a product that long is not bound by its weight's stream.)
-    if constexpr (SCALE) {
-        launch(std::true_type{});
-    } else if constexpr (WGM == 1) {
-        if (TM == 1 && splits == 1) launch(std::true_type{});
+    if constexpr (WGM == 1) {
+        if (ex.once && TM == 1 && splits == 1) launch(std::true_type{});
         else launch(std::false_type{});
     } else {
         launch(std::false_type{});
@@ -826,9 +830,11 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
 // that, not W, is most of a wave's traffic.  With GLU, sets 2p and 2p+1 hold a
 // gate group and the up group that follows it in W; the epilogue writes
 // silu(gate) * up.
-// The weight's loads say that nobody asks for the line again (nt): the caches then keep the rows of A and do not write lines about
+// Where the caller says that no cache holds the weight from one call to the next (once: a model's weights are more than the 256 MB behind the
+// L2), its loads say that nobody asks for the line again (nt): the caches then keep the rows of A and do not write lines about
 // that nothing will hit.  us, four decode steps of 8 requests on 8 layers of the 8B shape 4,300 / 4,057, a prompt of 96 tokens and 15
 // decode steps of the 0.6B shape 18,700 / 17,800; the head of 151,936 columns, 3 rows, 200 / 177 (7.0 TB/s).
+// Weights that do fit lose by it: four of 5,120 x 5,120 (210 MB) in turn, 8 rows, 10.6 / 15.8 us, 24 of 4,096 x 1,024, one row, 3.4 / 3.7.
 // The four-wave kernel has the same where it reads a weight once (launch_w4).
 // Weights that others read too (several row tiles), or in pieces of 64 bytes (float32 rows, 8,030 -> 8,200), lose by it.
 //
@@ -861,7 +867,7 @@ struct SkinnyFuse {
 
 // MORE: several products in one launch, or an activation of the result (GemmExtra).  Kernels of their own: the tests for them and the registers
 // of the activations cost every plain product 0.2 us (a decode step's of 2,048 to 4,096 columns 9.4 / 9.6, of 8 rows 10.9 / 11.1).
-template <int MT, int R, int UNROLL, int KSPLIT, int NSETS, bool GLU, typename TC, bool RING = false, int EPI = 0, bool MORE = false>
+template <int MT, int R, int UNROLL, int KSPLIT, int NSETS, bool GLU, typename TC, bool RING = false, int EPI = 0, bool MORE = false, bool ONCE = false>
 __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, TC* __restrict__ C, int M, int N,
     int K, int lda, int KB, int n_out, SkinnyFuse fz,
@@ -989,7 +995,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
             for (int u = 0; u < UNROLL; ++u) {
                 const int st = min(s0 + u, last);
 #pragma unroll
-                for (int r = 0; r < R; ++r) rw[u][r] = ld16_once(wfrag[r] + (size_t)st * 512);
+                for (int r = 0; r < R; ++r) rw[u][r] = ld16_weight<ONCE>(wfrag[r] + (size_t)st * 512);
 #pragma unroll
                 for (int t = 0; t < MT; ++t) ra[u][t] = ld16(arow[t] + st * 32 + fg * 8);
             }
@@ -1006,7 +1012,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
                     }
                     const int st = min(s0 + UNROLL + u, last);
 #pragma unroll
-                    for (int r = 0; r < R; ++r) rw[u][r] = ld16_once(wfrag[r] + (size_t)st * 512);
+                    for (int r = 0; r < R; ++r) rw[u][r] = ld16_weight<ONCE>(wfrag[r] + (size_t)st * 512);
 #pragma unroll
                     for (int t = 0; t < MT; ++t) ra[u][t] = ld16(arow[t] + st * 32 + fg * 8);
                 }
@@ -1019,7 +1025,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) rw[u][r] = ld16_once(wfrag[r] + (size_t)(s0 + u) * 512);
+            for (int r = 0; r < R; ++r) rw[u][r] = ld16_weight<ONCE>(wfrag[r] + (size_t)(s0 + u) * 512);
 #pragma unroll
             for (int t = 0; t < MT; ++t) ra[u][t] = ld16(arow[t] + (s0 + u) * 32 + fg * 8);
         }
@@ -1038,7 +1044,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
         const bool kok = k < K;
         uint4 rw[R], ra[MT];
 #pragma unroll
-        for (int r = 0; r < R; ++r) rw[r] = ld16_once(wfrag[r] + (size_t)s0 * 512);
+        for (int r = 0; r < R; ++r) rw[r] = ld16_weight<ONCE>(wfrag[r] + (size_t)s0 * 512);
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             const uint4 v = ld16(arow[t] + (kok ? k : 0));
@@ -1142,33 +1148,37 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
 
 template <int MT, int R, int UNROLL, int KSPLIT, int NSETS = 1, bool GLU = false, bool RING = false, int EPI = 0>
 static int launch_skinny(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda,
-                         const GemmExtra ex, int c_dtype, int n_out, hipStream_t s, const SkinnyFuse* fuse = nullptr) {
+                         const GemmCall ex, int c_dtype, int n_out, hipStream_t s, const SkinnyFuse* fuse = nullptr) {
     const int NB = (N + 15) / 16, KB = (K + 31) / 32;
     const int per_block = NSETS * R;
     const dim3 grid((NB + per_block - 1) / per_block);
     const SkinnyFuse fz = fuse ? *fuse : SkinnyFuse{nullptr, 0, 0, 0.f, 0.f, nullptr, nullptr, nullptr, nullptr, 0, nullptr, 0.f};
-    if (ex.plane_cols || ex.unary) {
-        if constexpr (EPI == 0 && !GLU) {
-            if (c_dtype == TFF_F32)
-                gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, false, float, RING, 0, true>
-                    <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, KB, n_out, fz, ex);
-            else
-                gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, false, bf16_t, RING, 0, true>
-                    <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, fz, ex);
-            return tff_check_launch("gemm_bf16_skinny");
-        } else {
-            return tff_fail("gemm: planes or an activation of a gated or fused product");
+    auto launch = [&](auto ONCE) {
+        constexpr bool once = decltype(ONCE)::value;
+        if (ex.plane_cols || ex.unary) {
+            if constexpr (EPI == 0 && !GLU) {
+                if (c_dtype == TFF_F32)
+                    gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, false, float, RING, 0, true, once>
+                        <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, KB, n_out, fz, ex);
+                else
+                    gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, false, bf16_t, RING, 0, true, once>
+                        <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, fz, ex);
+                return tff_check_launch("gemm_bf16_skinny");
+            } else {
+                return tff_fail("gemm: planes or an activation of a gated or fused product");
+            }
         }
-    }
-    if (c_dtype == TFF_F32)
-        gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, GLU, float, RING, EPI>
-            <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, KB, n_out, fz, ex);
-    else if constexpr (EPI < 2)
-        gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, GLU, bf16_t, RING, EPI>
-            <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, fz, ex);
-    else
-        return tff_fail("gemm: the product before a norm has a float32 result");
-    return tff_check_launch("gemm_bf16_skinny");
+        if (c_dtype == TFF_F32)
+            gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, GLU, float, RING, EPI, false, once>
+                <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, KB, n_out, fz, ex);
+        else if constexpr (EPI < 2)
+            gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, GLU, bf16_t, RING, EPI, false, once>
+                <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, fz, ex);
+        else
+            return tff_fail("gemm: the product before a norm has a float32 result");
+        return tff_check_launch("gemm_bf16_skinny");
+    };
+    return ex.once ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 // The tiled product's plan for M > 16: which tile, and into how many parts the blocks of a
@@ -1356,7 +1366,7 @@ TFF_API int tff_gemm_plan(int M, int N, int K, int glu, int keep_partials, int* 
 // a group's whole K through a ring (384 such waves, at N = 6,144, are too few: 3 % slower).  Plain: more waves per block where there are few blocks
 // (small N) or long rows (large K), fewer and deeper ones in between.
 template <int EPI>
-static int skinny_for(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmExtra ex, int c_dtype,
+static int skinny_for(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmCall ex, int c_dtype,
                       int glu_out, hipStream_t s, const SkinnyFuse* fuse) {
     if (glu_out > 0) {
         if constexpr (EPI < 2) {
@@ -1403,7 +1413,7 @@ static int skinny_for(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, 
 // The four-wave tiles address a block's rows and its columns of W by 32-bit offsets.  Rows or a stride too long for a plan's tile (256 rows
 // 8.4 million elements apart, K of 11 million on 192 columns) go to the sixteen-wave kernel, which has 64 bits a copy, K in as many parts.
 template <bool GLU>
-static int launch_far(const GemmPlan& plan, const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmExtra ex, int c_dtype,
+static int launch_far(const GemmPlan& plan, const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmCall ex, int c_dtype,
                       int n_out, hipStream_t s, float* part, bool reduce) {
     TFF_REQUIRE((size_t)15 * lda * 2 + 128 < (1ull << 32), "gemm: row stride %d too large", lda);
     if (plan.tile <= 64) return launch_async_g<2, 2, 2, 4, 3, GLU>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
@@ -1421,7 +1431,7 @@ static int launch_far(const GemmPlan& plan, const bf16_t* A, const bf16_t* Wp, v
 // keep_partials: where the plan splits K, the partial sums stay in the workspace
 // ([splits, M, N] float32) for the caller to add up, and C is not written.
 int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda,
-                  const GemmExtra ex, int c_dtype, int glu_out, float* workspace, size_t workspace_bytes,
+                  const GemmCall ex, int c_dtype, int glu_out, float* workspace, size_t workspace_bytes,
                   int keep_partials, hipStream_t s) {
     TFF_REQUIRE(K % 8 == 0 && lda % 8 == 0,
                 "gemm: the bfloat16 product needs the inner size (K=%d, row stride %d) to be a multiple of 8",
@@ -1436,7 +1446,7 @@ int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int 
     const bool red = !keep_partials;
     const bool far = plan.tile > 0 && K % 64 == 0 && !w4_reaches(plan.tile, plan.bn, K, lda);
     if (far && ex.plane_cols) {      // (one product after the other)
-        GemmExtra one = ex;
+        GemmCall one = ex;
         one.plane_cols = 0;
         const size_t w_plane = (size_t)(ex.plane_cols / 16) * (K / 32) * 512;
         for (int p = 0; p < N / ex.plane_cols; ++p)
@@ -1447,7 +1457,7 @@ int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int 
     if (ex.unary && glu_out == 0 && !keep_partials && planned_splits == 1 && unary_in_float32(plan, M, N, K) && workspace &&
         workspace_bytes >= (size_t)M * N * sizeof(float)) {
         // K in one part, whose float32 results the sum's kernel takes as the only plane
-        GemmExtra plain = ex;
+        GemmCall plain = ex;
         plain.unary = 0;
         if (int rc = tff_gemm_bf16(A, Wp, workspace, M, N, K, lda, plain, TFF_F32, 0, nullptr, 0, 0, s)) return rc;
         return launch_reduce<false>(workspace, 1, M, N, C, N, ex, c_dtype, s);
@@ -1538,7 +1548,7 @@ static int check_fused_operands(const char* what, const void* A, const void* Wp,
 // sum of squares of the new resid over columns 16 g .. 16 g + 15 of row m.  N a multiple of 8.
 TFF_API int tff_gemm_residual_prenorm(const void* A, const void* Wp, int M, int N, int K, int lda, float* resid,
                                       const float* norm_w, void* x_out, float* ss_out, int ss_stride,
-                                      tff_stream_t stream) {
+                                      int w_once, tff_stream_t stream) {
     if (int rc = check_fused_operands("gemm_residual_prenorm", A, Wp, M, N, K, lda)) return rc;
     TFF_REQUIRE(resid && norm_w && x_out && ss_out, "gemm_residual_prenorm: null pointer");
     TFF_REQUIRE(N % 8 == 0 && ss_stride >= (N + 15) / 16, "gemm_residual_prenorm: N=%d must be a multiple of 8 and "
@@ -1546,29 +1556,29 @@ TFF_API int tff_gemm_residual_prenorm(const void* A, const void* Wp, int M, int 
     TFF_REQUIRE(((uintptr_t)resid % 16) == 0 && ((uintptr_t)norm_w % 16) == 0 && ((uintptr_t)x_out % 8) == 0,
                 "gemm_residual_prenorm: operands must be 16-byte aligned");
     SkinnyFuse fz{nullptr, 0, 0, 0.f, 0.f, resid, norm_w, (bf16_t*)x_out, ss_out, ss_stride, nullptr, 0.f};
-    return skinny_for<2>((const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmExtra{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, 0, 0}, TFF_F32, 0, (hipStream_t)stream, &fz);
+    return skinny_for<2>((const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmCall{{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, 0, 0}, w_once}, TFF_F32, 0, (hipStream_t)stream, &fz);
 }
 
 // resid[M, N] += A . W^T (bfloat16 A and packed W, float32 sums); x_out[M, N] = bfloat16 of
 // tanh(alpha * resid) * norm_w + bias over the new resid: the norm without statistics in the epilogue of the
 // product before it.  Up to 16 rows; N a multiple of 8.
 TFF_API int tff_gemm_residual_dyt(const void* A, const void* Wp, int M, int N, int K, int lda, float* resid, float alpha,
-                                  const float* norm_w, const float* bias, void* x_out, tff_stream_t stream) {
+                                  const float* norm_w, const float* bias, void* x_out, int w_once, tff_stream_t stream) {
     if (int rc = check_fused_operands("gemm_residual_dyt", A, Wp, M, N, K, lda)) return rc;
     TFF_REQUIRE(resid && norm_w && bias && x_out, "gemm_residual_dyt: null pointer");
     TFF_REQUIRE(N % 8 == 0, "gemm_residual_dyt: N=%d must be a multiple of 8", N);
     TFF_REQUIRE(((uintptr_t)resid % 16) == 0 && ((uintptr_t)norm_w % 16) == 0 && ((uintptr_t)bias % 16) == 0 &&
                 ((uintptr_t)x_out % 8) == 0, "gemm_residual_dyt: operands must be 16-byte aligned");
     SkinnyFuse fz{nullptr, 0, 0, 0.f, 0.f, resid, norm_w, (bf16_t*)x_out, nullptr, 0, bias, alpha};
-    return skinny_for<3>((const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmExtra{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, 0, 0}, TFF_F32, 0, (hipStream_t)stream, &fz);
+    return skinny_for<3>((const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmCall{{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, 0, 0}, w_once}, TFF_F32, 0, (hipStream_t)stream, &fz);
 }
 
 // C = rstd[m] * (A . W^T) with rstd[m] = rsqrt(sum_g ss[m][g] / dim + eps), g < ss_count: the product
 // after tff_gemm_residual_prenorm (A = its x_out, ss = its ss_out, dim = its N).  glu_out as in tff_gemm.
 TFF_API int tff_gemm_row_scaled(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int c_dtype,
                                 int glu_out, const float* ss, int ss_stride, int ss_count, int dim, float eps,
-                                float glu_limit, float glu_alpha, float glu_up_offset, tff_stream_t stream) {
-    const GemmExtra ex{{nullptr, glu_act(glu_limit, glu_alpha, glu_up_offset)}, 0, 0, 0};
+                                float glu_limit, float glu_alpha, float glu_up_offset, int w_once, tff_stream_t stream) {
+    const GemmCall ex{{{nullptr, glu_act(glu_limit, glu_alpha, glu_up_offset)}, 0, 0, 0}, w_once};
     if (int rc = check_fused_operands("gemm_row_scaled", A, Wp, M, N, K, lda)) return rc;
     TFF_REQUIRE(C && ss && ((uintptr_t)C % 16) == 0 && ((uintptr_t)ss % 16) == 0, "gemm_row_scaled: null or unaligned pointer");
     TFF_REQUIRE(c_dtype == TFF_F32 || c_dtype == TFF_BF16, "gemm_row_scaled: unknown output type %d", c_dtype);
@@ -1598,7 +1608,7 @@ int tff_gemm_f32(const float* A, const float* W, void* C, int M, int N, int K, i
 TFF_API int tff_gemm(const void* A, const void* W, void* C, int M, int N, int K, int lda,
                      int ab_dtype, int c_dtype, int w_packed, int glu_out, const float* bias, float glu_limit,
                      float glu_alpha, float glu_up_offset, void* workspace, size_t workspace_bytes, int keep_partials,
-                     tff_stream_t stream) {
+                     int w_once, tff_stream_t stream) {
     TFF_REQUIRE(A && W && C, "gemm: null pointer");
     TFF_REQUIRE(M >= 0 && N > 0 && K > 0 && lda >= K, "gemm: bad sizes M=%d N=%d K=%d lda=%d", M, N, K, lda);
     if (M == 0) return 0;
@@ -1613,7 +1623,7 @@ TFF_API int tff_gemm(const void* A, const void* W, void* C, int M, int N, int K,
         TFF_REQUIRE(((uintptr_t)workspace % 16) == 0, "gemm: the workspace must be 16-byte aligned");
         TFF_REQUIRE(((uintptr_t)bias % 16) == 0, "gemm: the bias must be 16-byte aligned");
         return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda,
-                             GemmExtra{{bias, glu_act(glu_limit, glu_alpha, glu_up_offset)}, 0, 0, 0}, c_dtype, glu_out,
+                             GemmCall{{{bias, glu_act(glu_limit, glu_alpha, glu_up_offset)}, 0, 0, 0}, w_once}, c_dtype, glu_out,
                              (float*)workspace, workspace ? workspace_bytes : 0, keep_partials, s);
     }
     return tff_fail("gemm: unknown operand type %d", ab_dtype);
@@ -1632,12 +1642,12 @@ TFF_API size_t tff_gemm_unary_workspace_bytes(int M, int N, int K) {
     return p.splits > 1 || unary_in_float32(p, M, N, K) ? (size_t)p.splits * M * N * sizeof(float) : 0;
 }
 TFF_API int tff_gemm_unary(const void* A, const void* W, void* C, int M, int N, int K, int lda, int c_dtype, int kind, void* workspace,
-                           size_t workspace_bytes, tff_stream_t stream) {
+                           size_t workspace_bytes, int w_once, tff_stream_t stream) {
     TFF_REQUIRE(A && W && C, "gemm_unary: null pointer");
     TFF_REQUIRE(M >= 0 && N > 0 && K > 0 && lda >= K && kind >= 1 && kind <= 4, "gemm_unary: bad sizes M=%d N=%d K=%d lda=%d or kind %d", M, N, K, lda, kind);
     TFF_REQUIRE(((uintptr_t)workspace % 16) == 0, "gemm_unary: the workspace must be 16-byte aligned");
     if (M == 0) return 0;
-    return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, GemmExtra{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, kind, 0, 0},
+    return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, GemmCall{{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, kind, 0, 0}, w_once},
                          c_dtype, 0, (float*)workspace, workspace ? workspace_bytes : 0, 0, (hipStream_t)stream);
 }
 
@@ -1646,13 +1656,13 @@ TFF_API int tff_gemm_unary(const void* A, const void* W, void* C, int M, int N, 
 // instead of four times one that fills three quarters of them, and of one row they are one stream of 134 MB.
 // us, one by one / now: 4 x 4,096 x 4,096, 1,500 rows 234 / 181, one row 31 / 25.
 TFF_API int tff_gemm_planes_supported(int N, int K) { return N % 128 == 0 && K % 64 == 0; }
-TFF_API int tff_gemm_planes(const void* A, size_t a_step, const void* W, float* C, int planes, int M, int N, int K, int lda, tff_stream_t stream) {
+TFF_API int tff_gemm_planes(const void* A, size_t a_step, const void* W, float* C, int planes, int M, int N, int K, int lda, int w_once, tff_stream_t stream) {
     TFF_REQUIRE(A && W && C, "gemm_planes: null pointer");
     TFF_REQUIRE(M >= 0 && planes > 0 && N > 0 && K > 0 && lda >= K && (long)planes * N < (1L << 30), "gemm_planes: bad sizes %d x M=%d N=%d K=%d lda=%d",
                 planes, M, N, K, lda);
     TFF_REQUIRE(tff_gemm_planes_supported(N, K) && a_step % 8 == 0, "gemm_planes: N=%d in units of 128, K=%d of 64, rows' planes (%zu apart) of 8", N, K, a_step);
     if (M == 0) return 0;
-    return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, planes * N, K, lda, GemmExtra{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, N, a_step},
+    return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, planes * N, K, lda, GemmCall{{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, N, a_step}, w_once},
                          TFF_F32, 0, nullptr, 0, 0, (hipStream_t)stream);
 }
 

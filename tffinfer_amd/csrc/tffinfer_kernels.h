@@ -49,10 +49,12 @@ TFF_API int tff_rmsnorm(const void* x, const float* weight, float eps, void* out
 // cheaper hand-over) and the workspace has that size, the partial
 // sums [bytes / (M * N * 4), M, N] are left there for the caller to add up
 // (tff_add_rmsnorm takes them as they are) and C is not written.
+// w_once, here and below: no cache holds the weight from one call to the next (it belongs to more of them than the caches hold), so that
+// its loads may say so.
 TFF_API int tff_gemm(const void* A, const void* W, void* C, int M, int N, int K, int lda,
                      int ab_dtype, int c_dtype, int w_packed, int glu_out, const float* bias, float glu_limit,
                      float glu_alpha, float glu_up_offset, void* workspace, size_t workspace_bytes, int keep_partials,
-                     tff_stream_t stream);
+                     int w_once, tff_stream_t stream);
 TFF_API size_t tff_gemm_workspace_bytes(int M, int N, int K, int ab_dtype, int glu, int keep_partials);
 // The bfloat16 product's plan for these sizes: rows and columns of a block tile (0: the
 // streaming kernel for up to 16 rows) and the number of parts K is split into.
@@ -63,16 +65,16 @@ TFF_API int tff_gemm_plan(int M, int N, int K, int glu, int keep_partials, int* 
 TFF_API int tff_gemm_takes_unary(int M, int N, int K);
 TFF_API size_t tff_gemm_unary_workspace_bytes(int M, int N, int K);
 TFF_API int tff_gemm_unary(const void* A, const void* W, void* C, int M, int N, int K, int lda, int c_dtype, int kind, void* workspace,
-                           size_t workspace_bytes, tff_stream_t stream);
+                           size_t workspace_bytes, int w_once, tff_stream_t stream);
 // C[p] = A[p] . W[p]^T, p < planes, in one launch: A[p] = A + p * a_step, C [planes, M, N] float32, W the weights one after the other in
 // fragment order; N in units of 128, K of 64.
 TFF_API int tff_gemm_planes_supported(int N, int K);
-TFF_API int tff_gemm_planes(const void* A, size_t a_step, const void* W, float* C, int planes, int M, int N, int K, int lda, tff_stream_t stream);
+TFF_API int tff_gemm_planes(const void* A, size_t a_step, const void* W, float* C, int planes, int M, int N, int K, int lda, int w_once, tff_stream_t stream);
 
 // resid[M, N] += A . W^T; x_out[M, N] = bfloat16 of tanh(alpha * resid) * norm_w + bias over the new resid: a norm
 // without statistics in the epilogue of the product before it.  Up to 16 rows, bfloat16, N a multiple of 8.
 TFF_API int tff_gemm_residual_dyt(const void* A, const void* Wp, int M, int N, int K, int lda, float* resid, float alpha,
-                                  const float* norm_w, const float* bias, void* x_out, tff_stream_t stream);
+                                  const float* norm_w, const float* bias, void* x_out, int w_once, tff_stream_t stream);
 
 // An RMS norm between two bfloat16 products of up to 16 rows, taken into them (its per-row
 // factor commutes with the product after it):
@@ -83,10 +85,10 @@ TFF_API int tff_gemm_residual_dyt(const void* A, const void* Wp, int M, int N, i
 //     + eps), the sums added in a fixed order; glu_out as in tff_gemm.
 TFF_API int tff_gemm_residual_prenorm(const void* A, const void* Wp, int M, int N, int K, int lda, float* resid,
                                       const float* norm_w, void* x_out, float* ss_out, int ss_stride,
-                                      tff_stream_t stream);
+                                      int w_once, tff_stream_t stream);
 TFF_API int tff_gemm_row_scaled(const void* A, const void* Wp, void* C, int M, int N, int K, int lda, int c_dtype,
                                 int glu_out, const float* ss, int ss_stride, int ss_count, int dim, float eps,
-                                float glu_limit, float glu_alpha, float glu_up_offset, tff_stream_t stream);
+                                float glu_limit, float glu_alpha, float glu_up_offset, int w_once, tff_stream_t stream);
 
 // bfloat16 row-major [N, K] (K a multiple of 8) -> fragment order: tiles of
 // 16 rows x 32 k, each stored as the 1 KB operand of a 16x16x32 MFMA, element

@@ -6,7 +6,7 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
 from .build import ensure_built
 
-ABI_VERSION = 49
+ABI_VERSION = 50
 
 
 class KernelLibraryError(RuntimeError):
@@ -43,17 +43,17 @@ _SIGNATURES = {
     "tff_embed": [_P, _P, _P, _I, _I, _I, _I, _P],
     "tff_add_rmsnorm": [_P, _P, _I, _Z, _P, _F, _P, _P, _I, _I, _I, _P],
     "tff_rmsnorm": [_P, _P, _F, _P, _I, _I, _I, _P],
-    "tff_gemm": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _F, _F, _F, _P, _Z, _I, _P],
+    "tff_gemm": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _F, _F, _F, _P, _Z, _I, _I, _P],
     "tff_gemm_workspace_bytes": [_I, _I, _I, _I, _I, _I],
     "tff_gemm_takes_unary": [_I, _I, _I],
     "tff_gemm_unary_workspace_bytes": [_I, _I, _I],
-    "tff_gemm_unary": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _Z, _P],
+    "tff_gemm_unary": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _Z, _I, _P],
     "tff_gemm_planes_supported": [_I, _I],
-    "tff_gemm_planes": [_P, _Z, _P, _P, _I, _I, _I, _I, _I, _P],
+    "tff_gemm_planes": [_P, _Z, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "tff_gemm_plan": [_I, _I, _I, _I, _I, _P, _P, _P],
-    "tff_gemm_residual_prenorm": [_P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P],
-    "tff_gemm_residual_dyt": [_P, _P, _I, _I, _I, _I, _P, _F, _P, _P, _P, _P],
-    "tff_gemm_row_scaled": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _F, _F, _F, _F, _P],
+    "tff_gemm_residual_prenorm": [_P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _I, _I, _P],
+    "tff_gemm_residual_dyt": [_P, _P, _I, _I, _I, _I, _P, _F, _P, _P, _P, _I, _P],
+    "tff_gemm_row_scaled": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _F, _F, _F, _F, _I, _P],
     "tff_pack_weight": [_P, _P, _I, _I, _P],
     "tff_embed_packed": [_P, _P, _P, _I, _I, _I, _P],
     "tff_qk_norm_rope_kv": [_P, _I, _I, _I, _I, _P, _P, _F, _P, _I, _I, _I, _P, _P, _P, _P,

@@ -74,11 +74,15 @@ def _ptr(t):
 SILU = (math.inf, 1.0, 0.0)
 
 
+#: what the caches hold of a model's weights from one step to the next (the 256 MB behind the XCDs' L2)
+CACHE_BYTES = 256 << 20
+
+
 class PackedWeight:
     """A bfloat16 matrix [N, K] in the fragment order of the matrix-core
     products: tiles of 16 rows by 32 k stored as the 1 KB operand a wave loads,
     rows and k padded with zeros to multiples of 16 and 32."""
-    __slots__ = ("data", "N", "K", "glu_out", "k_in", "glu_act")
+    __slots__ = ("data", "N", "K", "glu_out", "k_in", "glu_act", "once")
 
     def __init__(self, data: torch.Tensor, N: int, K: int, glu_out: int = 0, k_in: int | None = None):
         self.data, self.N, self.K = data, int(N), int(K)
@@ -90,6 +94,9 @@ class PackedWeight:
         self.glu_out = int(glu_out)
         #: (limit, alpha, up_offset) of the gated product's activation, see :func:`swiglu`
         self.glu_act = SILU
+        #: whether no cache holds the weight from one call to the next: it is larger than they are, or belongs to a model
+        #: that is (the model says so when it is loaded); products of few rows then load it as such
+        self.once = data.numel() * data.element_size() > CACHE_BYTES
 
     @property
     def shape(self):
@@ -295,7 +302,7 @@ def _fused_prenorm(p: PendingProduct, resid: torch.Tensor, weight: torch.Tensor,
     ss = torch.empty(16, stride, dtype=torch.float32, device=x.device)
     L = _lib.load()
     _lib.check(L.tff_gemm_residual_prenorm(x.data_ptr(), p.weight.data_ptr(), M, N, K, lda, resid.data_ptr(),
-                                           weight.data_ptr(), xs.data_ptr(), ss.data_ptr(), stride, _stream()))
+                                           weight.data_ptr(), xs.data_ptr(), ss.data_ptr(), stride, int(p.weight.once), _stream()))
     return ScaledRows(xs, ss, groups, eps, resid, weight)
 
 
@@ -440,7 +447,7 @@ def linear(x: torch.Tensor, weight, out_dtype: torch.dtype | None = None,
             raise _lib.KernelError(f"linear out: shape {tuple(out.shape)} is not {(M, n_out)}")
     _lib.check(L.tff_gemm(x.data_ptr(), weight.data_ptr(), out.data_ptr(), M, N, K, lda,
                           dtype_code(x.dtype), dtype_code(out_dtype), 1 if packed else 0, glu_out, _ptr(bias),
-                          *(weight.glu_act if packed else SILU), _ptr(ws), ws_bytes, 1 if keep else 0, _stream()))
+                          *(weight.glu_act if packed else SILU), _ptr(ws), ws_bytes, 1 if keep else 0, int(packed and weight.once), _stream()))
     return out
 
 
@@ -469,7 +476,7 @@ def linear_unary(x: torch.Tensor, weight, act: str, out_dtype: torch.dtype) -> t
             ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device) if ws_bytes else None
             out = torch.empty(M, N, dtype=out_dtype, device=x.device)
             _lib.check(L.tff_gemm_unary(x.data_ptr(), weight.data_ptr(), out.data_ptr(), M, N, K, lda, dtype_code(out_dtype), UNARY[act],
-                                        _ptr(ws), ws_bytes, _stream()))
+                                        _ptr(ws), ws_bytes, int(weight.once), _stream()))
             return out
     if act == "tanh":
         return tanh(linear(x, weight, out_dtype=torch.float32), out_dtype)
@@ -493,7 +500,7 @@ def linear_planes(x: torch.Tensor, weight: PackedWeight) -> torch.Tensor:
                                "the inner size of 64)")
     N = weight.shape[0] // P
     out = torch.empty(P, M, N, dtype=torch.float32, device=x.device)
-    _lib.check(_lib.load().tff_gemm_planes(x.data_ptr(), M * K, weight.data_ptr(), out.data_ptr(), P, M, N, K, K, _stream()))
+    _lib.check(_lib.load().tff_gemm_planes(x.data_ptr(), M * K, weight.data_ptr(), out.data_ptr(), P, M, N, K, K, int(weight.once), _stream()))
     return out
 
 
@@ -505,7 +512,7 @@ def _linear_row_scaled(x: ScaledRows, weight: "PackedWeight", out_dtype: torch.d
     L = _lib.load()
     _lib.check(L.tff_gemm_row_scaled(x.x.data_ptr(), weight.data_ptr(), out.data_ptr(), M, N, K, K,
                                      dtype_code(out_dtype), glu_out, x.ss.data_ptr(), x.ss.stride(0), x.count, K,
-                                     x.eps, *weight.glu_act, _stream()))
+                                     x.eps, *weight.glu_act, int(weight.once), _stream()))
     return out
 
 
@@ -2362,7 +2369,7 @@ def add_dyt(resid: torch.Tensor, delta, alpha: float, weight: torch.Tensor, bias
         out = torch.empty(M, H, dtype=torch.bfloat16, device=resid.device)
         _lib.check(_lib.load().tff_gemm_residual_dyt(p.x.data_ptr(), p.weight.data_ptr(), M, H, K,
                                                      p.x.stride(0) if M > 1 else K, resid.data_ptr(), float(alpha),
-                                                     weight.data_ptr(), bias.data_ptr(), out.data_ptr(), _stream()))
+                                                     weight.data_ptr(), bias.data_ptr(), out.data_ptr(), int(p.weight.once), _stream()))
         return out
     terms = delta.terms if isinstance(delta, PendingTerms) else ([] if delta is None else [delta])
     d = [_planes_of(t, resid.shape, "add_dyt term") for t in terms] + [(None, 0, 0)] * 2

@@ -156,6 +156,7 @@ class DecoderModel:
                 part.load_weights({local: normalize_stored(found[self.names.tensor(prefix, local)])
                                    for local in specs if self.names.tensor(prefix, local) in found},
                                   dtype, self.device)
+        self._note_weights_size()
 
     def init_random(self, seed: int, dtype: torch.dtype, device, on_device: bool = False) -> None:
         """Seeded random weights without a file.  ``on_device`` draws on the GPU
@@ -172,6 +173,24 @@ class DecoderModel:
                     t = random_tensor(spec, seed, self.names.tensor(prefix, local), device=gen_dev)
                     ws[local] = t if spec.init in FLOAT32_INITS else t.to(torch.bfloat16)
                 part.load_weights(ws, dtype, self.device)
+        self._note_weights_size()
+
+    def _note_weights_size(self) -> None:
+        """Tells the products whether a step finds its weights in the caches (``PackedWeight.once``): not those of a model whose matrices are
+        larger.  A model that fits keeps plain loads: 24 weights of 4,096 x 1,024 (201 MB) in turn, one row, 3.4 us a product, and 3.7 with
+        loads that leave nothing behind; beyond it is the other way round (24,576 x 4,096 of 600 MB 38.0 / 34.1)."""
+        from ..kernels import ops
+        packed, total = {}, 0
+        for _, part in self._weighted_parts():
+            for value in vars(part).values():
+                for w in value if isinstance(value, (list, tuple)) else (value,):
+                    if isinstance(w, ops.PackedWeight):
+                        packed[id(w)] = w
+                    elif isinstance(w, torch.Tensor) and w.dim() >= 2 and not isinstance(part, (Embedding, BigramTable)):
+                        total += w.numel() * w.element_size()       # (a table's rows are looked up, here and there one)
+        total += sum(w.data.numel() * w.data.element_size() for w in packed.values())
+        for w in packed.values():
+            w.once = total > ops.CACHE_BYTES
 
     def graph_safe(self) -> bool:
         """True if every part launches only kernels that read the step's sizes
