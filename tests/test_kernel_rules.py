@@ -225,3 +225,20 @@ def test_loads_into_lds_leave_a_wait_state_behind_m0():
                         assert "_lds_" not in second, (os.path.basename(path), lines)
                 assert "_lds_" not in lines[0], (os.path.basename(path), lines)      # (M0 is written beside its load)
     assert pieces >= 7, pieces
+
+
+def test_products_whose_weights_stream_wants_more_blocks_split_k():
+    """Some hundred rows of a weight that comes from memory: fewer columns of tiles than keep it coming split K.  Kept sums, up to 64
+    rows, long products and K in no units of 64 have plans of their own."""
+    import ctypes
+    L = _lib()
+
+    def plan(M, N, K, glu=0, keep=0):
+        r, c, s = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+        assert L.tff_gemm_plan(M, N, K, glu, keep, ctypes.byref(r), ctypes.byref(c), ctypes.byref(s)) == 0
+        return r.value, c.value, s.value
+
+    assert plan(110, 6144, 2560) == (128, 128, 4) and plan(78, 6144, 2560, glu=1) == (64, 128, 2)
+    assert plan(202, 6144, 4096) == plan(330, 4096, 4096) == (128, 128, 2)
+    assert plan(110, 6144, 2560, keep=1)[2] > 1 and plan(60, 6144, 2560) == (64, 128, 4)
+    assert plan(16384, 24576, 4096, glu=1) == (256, 256, 1) and plan(2048, 6144, 4096) == (256, 192, 1)

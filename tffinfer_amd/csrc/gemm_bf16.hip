@@ -1242,29 +1242,31 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
     const int nk = (K + 63) / 64;
     if (K % 64 == 0) {
         // The four-wave kernel's tiles (256 rows on 2 x 2 waves, 128 rows on 1 x 4) and, up to 512 rows,
-        // its 64 x 128, two blocks to a CU (the last candidate; its rate is that of the sixteen-wave
-        // kernel's 64 x 128, which it replaced and is 8 to 17 % faster than at 128 to 512 rows, so
-        // the model picks it rather too seldom).  A block goes through its part of K in
+        // its 64 x 128, two blocks to a CU.  A block goes through its part of K in
         // units of 64; a unit takes what its MFMAs take at the tile's rate or what its columns of W take
         // to arrive, whichever is longer: a block's share of the HBM stream, at most what one CU pulls.
-        // Blocks go round the CUs; each round ends with the pipeline filled and the tile stored.  Beyond 64 rows the
-        // constants stand for 840 products of the 0.6B to 14B shapes and of the other designs, 65 .. 9,000 rows, every tile with
-        // 1 .. 8 parts timed in a graph on an MI355X (weights in turn, so that none comes from a cache, and none of a launch's
-        // host work in the figure): the pick is 1.5 % from the best candidate on average; the constants before, fitted to a slower loop
-        // and to launches from the host, were 5.3 % from it there, 11 % at 128 .. 512 rows, where they split K for a kernel
-        // more (us: 229 rows of 4,096 x 2,048 16.2 / 11.2, 501 of 2,048 x 2,048 16.7 / 10.3, 901 of it 19.5 / 14.8, 333 of 2,048 x 6,144 23.7 / 18.5).
-        // Up to 64 rows the four waves side by side take 64 or 32 rows: a product of so few rows is its
-        // weight's stream, and a block that does not work through 128 rows for 32 asks for its next
-        // columns sooner (3 to 10 % less time than the tiles of 128 rows and the sixteen-wave kernel's
-        // 64 x 128 on the four products of the three shapes at 17 to 64 rows; their rates fitted to
-        // those 88 cases stand for that, the pick 0.5 % from the best on average, 5 % at worst).
-        struct Cand { int bm, bn, slots; double rate, rate_few; };      // flops a microsecond of a CU, beyond 64 rows and up to them
-        static const Cand cands[11] = {{256, 256, 1, 6.45e6, 0}, {256, 192, 1, 6.10e6, 0}, {256, 128, 1, 5.42e6, 0},
-                                       {128, 384, 1, 6.49e6, 3.24e6}, {128, 256, 1, 5.38e6, 4.61e6}, {128, 128, 1, 3.56e6, 3.45e6},
-                                       {64, 256, 1, 0, 2.4e6}, {64, 128, 1, 0, 2.0e6}, {32, 256, 1, 0, 1.4e6}, {32, 128, 1, 0, 1.3e6},
-                                       {64, 128, 2, 2.48e6, 0}};
-        const bool few = M <= 64;
-        const double HBM = few ? 7.72e6 : 8.18e6, CU_MAX = few ? 6.0e4 : 6.54e4;   // bytes a microsecond: all CUs together, one alone
+        // Blocks go round the CUs; each round ends with the pipeline filled and the tile stored.  The constants are
+        // fitted to products of the 0.6B to 14B shapes and of the other designs, every tile with
+        // 1 .. 8 parts timed in a graph on an MI355X (weights in turn, none of a launch's host work in the figure), in three pieces:
+        // * Results of one kernel or of the sum over the parts, more than 64 rows: 8,500 products of 65 .. 9,000 rows.  The pick is 1.2 % from the best
+        //   candidate on average (gated 0.5 %), and in 97 of 100 not 3 % slower than what the constants for a slower loop picked.  One
+        //   fit with the kept sums left K in one part where a weight's stream wants more blocks (us, that / these: 110 rows of 6,144 x 2,560
+        //   20.9 / 16.6, gated 78 rows 20.2 / 15.6, 202 of 6,144 x 4,096 29.9 / 26.0, 330 of 4,096 x 4,096 29.2 / 25.8).
+        // * Sums kept for a norm, more than 64 rows: 840 products; 1.1 % from the best with the norm behind it.
+        // * Up to 64 rows the four waves side by side take 64 or 32 rows: a product of so few rows is its
+        //   weight's stream, and a block that does not work through 128 rows for 32 asks for its next
+        //   columns sooner (3 to 10 % less time than the tiles of 128 rows and the sixteen-wave kernel's
+        //   64 x 128 on the four products of the three shapes at 17 to 64 rows; their rates fitted to
+        //   those 88 cases stand for that, the pick 0.5 % from the best on average, 5 % at worst).
+        // A rate is in flops a microsecond of a CU: of results, of kept sums, up to 64 rows.  ends: us that a block's first fetch and storing its tile take.
+        struct Cand { int bm, bn, slots; double rate, rate_kept, rate_few, ends; };
+        static const Cand cands[11] = {{256, 256, 1, 7.69e6, 6.45e6, 0, 1.42}, {256, 192, 1, 7.02e6, 6.10e6, 0, 1.05}, {256, 128, 1, 6.13e6, 5.42e6, 0, 0.75},
+                                       {128, 384, 1, 6.00e6, 6.49e6, 3.24e6, 1.05}, {128, 256, 1, 5.97e6, 5.38e6, 4.61e6, 0.75}, {128, 128, 1, 4.41e6, 3.56e6, 3.45e6, 0.56},
+                                       {64, 256, 1, 0, 0, 2.4e6, 0}, {64, 128, 1, 0, 0, 2.0e6, 0}, {32, 256, 1, 0, 0, 1.4e6, 0}, {32, 128, 1, 0, 0, 1.3e6, 0},
+                                       {64, 128, 2, 2.72e6, 2.48e6, 0, 0.50}};
+        const bool few = M <= 64, kept = keep && !few;
+        // bytes a microsecond of all CUs together and of one alone
+        const double HBM = few ? 7.72e6 : kept ? 8.18e6 : 14.65e6, CU_MAX = few ? 6.0e4 : kept ? 6.54e4 : 5.57e4;
         GemmPlan best = {128, 128, 1};
         double best_t = 1e30;
         for (const Cand& c : cands) {
@@ -1275,16 +1277,23 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
             for (int S = 1; S <= (plane ? 1 : (glu && M > 64) ? 2 : 8); S *= 2) {
                 if (S > 1 && nk / S < 4) break;
                 const double blocks = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * S;
-                const double rounds = ceil(blocks / (CUS * c.slots));
-                const double share = fmin((double)c.slots, ceil(blocks / CUS));   // blocks that share a CU's MFMAs
-                const double bw = fmin(CU_MAX, HBM / fmin(blocks, CUS * c.slots));
-                const double unit = fmax(2.0 * c.bm * c.bn * 64.0 * share / (few ? c.rate_few : c.rate), c.bn * 128.0 / bw);
-                const double ends = few ? 3.0 : 1.29 + 2.55 * (c.bm * c.bn / 65536.0);   // a block's first fetch, and storing its tile
-                double t = rounds * ((double)nk / S * unit + ends) + 3.0;
+                const double rounds = ceil(blocks / (CUS * c.slots)), at_once = fmin(blocks, CUS * c.slots);
+                double rate = c.rate, ends = c.ends, start = 2.47, streams = ceil((double)N / c.bn) * S;   // (row tiles fetch a column tile's weight once between them)
+                double share = c.slots == 2 && blocks > CUS ? 1.79 : 1.0;       // blocks that share a CU's MFMAs, and each other's waits
+                if (few || kept) {
+                    rate = few ? c.rate_few : c.rate_kept;
+                    ends = few ? 3.0 : 1.29 + 2.55 * (c.bm * c.bn / 65536.0);
+                    start = 3.0;
+                    streams = at_once;
+                    share = fmin((double)c.slots, ceil(blocks / CUS));
+                }
+                const double bw = fmin(CU_MAX, HBM / fmin(at_once, streams));
+                const double unit = fmax(2.0 * c.bm * c.bn * 64.0 * share / rate, c.bn * 128.0 / bw);
+                double t = rounds * ((double)nk / S * unit + ends) + start;
                 // the partial sums: written, read and added by a second kernel, or (kept) read by the
                 // consumer in place of one plane
-                if (S > 1 && few) t += keep ? (S - 1.0) * M * N * 4.0 / 4e6 : (double)S * M * N * 4.0 / 2.54e6 + 2.7;
-                else if (S > 1) t += keep ? (S - 1.0) * M * N * 4.0 / 1.97e6 : (double)S * M * N * 4.0 / 2.15e6 + 6.78;
+                if (S > 1 && keep) t += (S - 1.0) * M * N * 4.0 / (few ? 4e6 : 1.97e6);
+                else if (S > 1) t += (double)S * M * N * 4.0 / (few ? 2.54e6 : 2.12e6) + (few ? 2.7 : 3.84);
                 if (t < best_t) { best_t = t; best = {c.bm, c.bn, S}; }
             }
         }
