@@ -85,6 +85,23 @@ def test_portions_take_the_blocks_that_end_first():
     assert pick([(0, 5), (100000, 40)] * 300) in (1, 2)      # more items than are dealt to find the longest block
 
 
+@pytest.mark.parametrize("pool", [0, 16])
+@pytest.mark.parametrize("window", [77, 0])
+@pytest.mark.parametrize("entries", [[(0, 40), (3, 1), (900, 70)], [(0, 3001), (7, 1), (50, 1), (2000, 700), (0, 33)]])
+def test_items_of_few_and_of_many_columns(entries, window, pool):
+    """An item's slices are those of the keys its columns see, and of the blocks of keys before the window, whether the items are counted one
+    by one or by arrays; the longest come first."""
+    from tffinfer_amd.kernels.ops import _block_items
+    for G, cols, which in ((4, 128, "all"), (5, 256, "multi")):
+        want = []
+        for r, (P, n) in enumerate(entries):
+            for c0 in range(0, n * G, cols) if which == "all" or n > 1 else ():
+                last = P + (min(c0 + cols, n * G) - 1) // G
+                blocks = max(0, last - window + 1) // pool if pool and window else 0
+                want.append((_slices(P, n, G, c0, cols, window) + -(-blocks // 32), r, c0))
+        assert _block_items(_batch(entries), G, window, cols, which, pool if window else 0) == sorted(want, reverse=True)
+
+
 def test_staged_tables_keep_shape_and_type_on_the_host():
     """The staging module's host form (what the work lists' tests above go through): every
     column comes back as a tensor of its own shape and element type, a copy of the array."""

@@ -404,7 +404,7 @@ static int launch_async_g(const bf16_t* A, const bf16_t* Wp, void* C, int M, int
 // In k-tile t (32 k) a wave copies half of A unit u + 3 (t = 2 u + 1 the first, t = 2 u + 2 the second half) and W tile
 // t + NWS: into the slots of the unit and tile whose fragments were last read in tile t - 1 or before.  Every wave waits
 // for its own reads before the barrier at the start of t, which makes those slots free; the last quarter of a tile's
-// MFMAs has no reads, so the reads have come back by then.  At the start of t it needs W tile t + 1 and the A unit of
+// MFMAs has no reads (of tiles of eight MFMAs and more), so that wait seldom lasts.  At the start of t it needs W tile t + 1 and the A unit of
 // t + 1, issued in tiles t - NWS + 1 and t - 3 at the latest.  Copies complete in the order issued, so the wait is by count.
 //
 // What bounds the loop of one wave a SIMD is the issue of what stands between the MFMAs: a wave issues an instruction

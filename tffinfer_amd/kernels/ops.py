@@ -702,34 +702,63 @@ def _num_cus(device) -> int:
 
 
 def _block_items(batch, G: int, window: int, cols: int, which: str, pool: int = 0) -> list[tuple[int, int, int]]:
-    """(32-key slices, entry, first column) of the items of ``cols`` columns of the step's entries."""
+    """(32-key slices, entry, first column) of the items of ``cols`` columns of the step's entries, the longest first."""
     cu, P = batch.host_cu_tokens, batch.host_start_pos
-    items = []
-    for r in _entries(batch, which):
-        ncols = (cu[r + 1] - cu[r]) * G
-        for c0 in range(0, ncols, cols):
-            first = P[r] + c0 // G
-            last = P[r] + (min(c0 + cols, ncols) - 1) // G
-            lo = max(0, first - window + 1) if window > 0 else 0
-            blocks = max(0, last - window + 1) // pool if pool else 0      # keys of blocks before the window
-            items.append((last // 32 - lo // 32 + 1 + -(-blocks // 32), r, c0))
-    return items
+    rows = _entries(batch, which)
+    widths = [(cu[r + 1] - cu[r]) * G for r in rows]
+    counts = [-(-n // cols) for n in widths]
+    if sum(counts) < 64:                 # (arrays cost more than a few items)
+        items = []
+        for r, ncols in zip(rows, widths):
+            begin = P[r]
+            for c0 in range(0, ncols, cols):
+                last = begin + (min(c0 + cols, ncols) - 1) // G
+                lo = max(0, begin + c0 // G - window + 1) if window > 0 else 0
+                blocks = max(0, last - window + 1) // pool if pool else 0      # keys of blocks before the window
+                items.append((last // 32 - lo // 32 + 1 + -(-blocks // 32), r, c0))
+        return sorted(items, reverse=True)
+    counts = np.asarray(counts)
+    at = np.repeat(np.arange(len(rows)), counts)
+    r, start, ncols = np.asarray(rows)[at], np.asarray([P[r] for r in rows])[at], np.asarray(widths)[at]
+    c0 = (np.arange(at.size) - np.repeat(np.cumsum(counts) - counts, counts)) * cols
+    last = start + (np.minimum(c0 + cols, ncols) - 1) // G
+    slices = last // 32 + 1
+    if window > 0:
+        slices -= np.maximum(0, start + c0 // G - window + 1) // 32
+    if pool:
+        slices += -(-(np.maximum(0, last - window + 1) // pool) // 32)
+    order = np.lexsort((c0, r, slices))[::-1]
+    return list(zip(slices[order].tolist(), r[order].tolist(), c0[order].tolist()))
 
 
 def _deal_items(items: list, nbins: int) -> list[list]:
-    """The items of every block: one each, the longest first, or with more items than blocks the longest first, each to the block with
-    the least to do so far."""
+    """The items (the longest first) of every block: one each, or with more items than blocks each to the block with the least to do
+    so far."""
     if len(items) <= nbins:
-        return [[it] for it in sorted(items, reverse=True)]
-    import heapq
-    loads = [(0, b) for b in range(nbins)]
+        return [[it] for it in items]
+    per_bin = [[it] for it in items[:nbins]]
+    loads = [(it[0], b) for b, it in enumerate(items[:nbins])]
     heapq.heapify(loads)
-    per_bin = [[] for _ in range(nbins)]
-    for it in sorted(items, reverse=True):
-        load, b = heapq.heappop(loads)
+    for it in items[nbins:]:
+        load, b = loads[0]
         per_bin[b].append(it)
-        heapq.heappush(loads, (load + it[0], b))
+        heapq.heapreplace(loads, (load + it[0], b))
     return per_bin
+
+
+def _dealt(batch, G: int, window: int, cols: int, which: str, nbins: int, pool: int = 0) -> list[list]:
+    """The step's items dealt to ``nbins`` blocks, worked out once a step."""
+    key = ("dealt", G, window, cols, which, nbins, pool)
+    if key not in batch._attn_work:
+        batch._attn_work[key] = _deal_items(_items_once(batch, G, window, cols, which, pool), nbins)
+    return batch._attn_work[key]
+
+
+def _items_once(batch, G: int, window: int, cols: int, which: str, pool: int = 0) -> list[tuple[int, int, int]]:
+    key = ("items", G, window, cols, which, pool)
+    if key not in batch._attn_work:
+        batch._attn_work[key] = _block_items(batch, G, window, cols, which, pool)
+    return batch._attn_work[key]
 
 
 def _attention_block_work(batch, G: int, nkv: int, window: int, device, cols: int = 128,
@@ -748,7 +777,7 @@ def _attention_block_work(batch, G: int, nkv: int, window: int, device, cols: in
         cache = batch._attn_work = {}
     key = ("blocks", G, nkv, cols, window, bins, which, key_groups, head_dim, num_cus) + ((pool,) if pool else ())
     if key not in cache:
-        items = _block_items(batch, G, window, cols, which, pool)
+        items = _items_once(batch, G, window, cols, which, pool)
         if num_cus is None:
             num_cus = _num_cus(device) if torch.device(device).type == "cuda" else 256
         per_cu = max(1, num_cus // max(1, nkv))
@@ -761,7 +790,7 @@ def _attention_block_work(batch, G: int, nkv: int, window: int, device, cols: in
             groups = 1                   # LDS holds one group's stages there
         nbins = bins if bins is not None else (per_cu if groups == 2 or head_dim > 128 else 2 * per_cu)
         order, starts = [], [0]
-        for lst in _deal_items(items, nbins):
+        for lst in _dealt(batch, G, window, cols, which, nbins, pool):
             order.extend(lst)
             starts.append(len(order))
         flat = [x for it in order for x in it[1:]]
@@ -772,7 +801,8 @@ def _attention_block_work(batch, G: int, nkv: int, window: int, device, cols: in
 
 
 def _pick_block_cols(batch, G: int, nkv: int, window: int, device, which: str, head_dim: int) -> int:
-    """128 or 256 columns to a block of the prompt attention.  Blocks of 256 columns (two
+    """128 or 256 columns to a block of eight waves of the prompt attention (heads of 128 without a cap come here with short portions only, see
+    :func:`_prompt_blocks`).  Blocks of 256 columns (two
     column tiles a wave) read half as much from LDS and fetch half as many keys per flop.
     Measured alone they are ahead from some 3,500 tokens on (a tenth at 32,768 tokens, a
     quarter on the slower boxes of the pool); inside a whole prefill, between products that
@@ -989,17 +1019,24 @@ def _prompt_blocks(batch, G: int, nkv: int, window: int, device, which: str, d: 
         if num_cus is None:
             num_cus = _num_cus(device) if torch.device(device).type == "cuda" else 256
         bins = max(1, num_cus // max(1, nkv))
-        items = {cols: _block_items(batch, G, window, cols, which) for cols in {f[3] for f in _PROMPT_FORMS[d].values()}}
-        times = {}
+        bounds, loads = [], {}
         for form, (start, step, item, cols, slices) in _PROMPT_FORMS[d].items():
-            its = items[cols]
-            if form == 0 and d <= 128 and sum(it[0] for it in its) >= 96 * 2 * bins:
+            its = _items_once(batch, G, window, cols, which)
+            total = sum([it[0] for it in its])
+            if form == 0 and d <= 128 and total >= 96 * 2 * bins:
                 continue                 # (long portions, where eight waves are never ahead)
-            if len(its) > min(256, 4 * bins):
-                times[form] = start + (step * sum(it[0] for it in its) / slices + item * len(its)) / bins      # (as good as even)
-            else:
-                times[form] = start + max(step * sum(-(-it[0] // slices) for it in lst) + item * len(lst) for lst in _deal_items(its, bins))
-        cache[key] = min(times, key=times.get)
+            bounds.append((start + max(step * -(-its[0][0] // slices) + item, (step * total / slices + item * len(its)) / bins), form))
+        best, best_t = 0, math.inf
+        for t, form in sorted(bounds):   # (no less than that, whatever the dealing)
+            start, step, item, cols, slices = _PROMPT_FORMS[d][form]
+            its = _items_once(batch, G, window, cols, which)
+            if t < best_t and bins < len(its) <= min(256, 4 * bins):       # (more items are dealt as good as evenly)
+                if cols not in loads:
+                    loads[cols] = {(sum([it[0] for it in lst]), len(lst)) for lst in _dealt(batch, G, window, cols, which, bins)}
+                t = start + max([step / slices * load + item * n for load, n in loads[cols]])
+            if t < best_t:
+                best, best_t = form, t
+        cache[key] = best
     return cache[key]
 
 
