@@ -1232,6 +1232,21 @@ def test_attention_mfma_long_portions(nq, nkv, d, ps, window, bins, groups):
             _close(out.reshape(T, nq, d)[mine], ref, ATTN_TOL, f"block attention, request {r}")
 
 
+@pytest.mark.parametrize("groups,softcap", [(1, 0.0), (2, 0.0), (1, 5.0), (2, 5.0)])
+@pytest.mark.parametrize("nq,nkv,d,ps,window", [(32, 8, 128, 16, 0), (5, 1, 128, 32, 77), (3, 1, 256, 64, 0), (6, 1, 256, 16, 40)])
+def test_long_portions_on_blocks_of_eight_waves(nq, nkv, d, ps, window, groups, softcap):
+    """Heads of 128 and 256 on the blocks that short portions and capped scores take, whose key groups are named (256: one, and no cap)."""
+    if d == 256 and (groups == 2 or softcap):
+        pytest.skip("heads of 256 have one key group and no cap there")
+    ops = _ops()
+    batch, kv, ks, vs, positions, token_req = _fake_step([(0, 700), (333, 200), (5, 1), (1000, 130)], ps, nkv, d, torch.bfloat16, seed=nq + ps)
+    q = torch.randn(batch.num_tokens, nq * d, generator=torch.Generator().manual_seed(9)).to(torch.bfloat16).to(DEV)
+    out = ops.attention_mfma(q, nq, nkv, d, kv, batch, window, key_groups=groups, block_cols=128, softcap=softcap)
+    gen = ops.attention_generic(q, nq, nkv, d, kv.k_cache, kv.v_cache, kv.block_tables, batch.token_req, batch.positions, window, 1 / math.sqrt(d),
+                                softcap=softcap)
+    _close(out, gen.double(), ATTN_TOL, "blocks of eight waves against the general kernel")
+
+
 @pytest.mark.parametrize("nq,nkv,d,window,entries", [
     (8, 2, 128, 0, [(0, 17)]), (5, 1, 128, 0, [(0, 150), (33, 40)]), (8, 2, 128, 40, [(0, 333), (500, 64), (7, 1)]),
     (32, 1, 256, 0, [(0, 3)]), (6, 1, 256, 30, [(0, 96), (200, 33)])])
@@ -1427,9 +1442,9 @@ def test_attention_of_prompts_keeps_values_that_are_not_finite_to_those_that_see
 
 
 def test_attention_mfma_picks_its_blocks_by_the_work():
-    """A prompt of 2,048 tokens goes to the blocks of 128 columns, one of 32,768 tokens to those
-    of 256; head sizes beyond 128 never do.  A prompt of 6,000 tokens through either gives
-    what the general kernel gives."""
+    """Of the blocks of eight waves a prompt of 2,048 tokens would take those of 128 columns, one of 32,768 tokens those
+    of 256; head sizes beyond 128 never do.  A prompt of 6,000 tokens through the blocks that it goes to (four waves) and through blocks of
+    eight waves and 256 columns gives what the general kernel gives."""
     from types import SimpleNamespace
     ops = _ops()
     nq, nkv, d, ps = 32, 8, 128, 16
