@@ -242,3 +242,12 @@ def test_products_whose_weights_stream_wants_more_blocks_split_k():
     assert plan(202, 6144, 4096) == plan(330, 4096, 4096) == (128, 128, 2)
     assert plan(110, 6144, 2560, keep=1)[2] > 1 and plan(60, 6144, 2560) == (64, 128, 4)
     assert plan(16384, 24576, 4096, glu=1) == (256, 256, 1) and plan(2048, 6144, 4096) == (256, 192, 1)
+
+
+def test_an_activation_counts_the_kernel_that_adds_up_the_parts():
+    """With an activation behind it a product in one part has the kernel that adds up the parts as well, so that two parts may be the
+    sooner; the room that is asked for is that plan's."""
+    L = _lib()
+    for M, N, K, parts in ((200, 18432, 4096, 2), (128, 12288, 4096, 2), (90, 9216, 2048, 2), (1055, 4096, 4096, 2), (333, 512, 192, 1), (16, 18432, 4096, 0), (2048, 18432, 4096, 0)):
+        assert L.tff_gemm_unary_workspace_bytes(M, N, K) == parts * M * N * 4, (M, N, K)
+        assert L.tff_gemm_takes_unary(M, N, K) == (parts > 0 or M <= 16)

@@ -1223,7 +1223,9 @@ static int plan_rows32(int N, int K) {
 }
 
 // plane > 0: the columns of several products, so many each; a tile takes columns of one of them, and K is not split.
-static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0) {
+// unary: an activation follows, in the kernel that adds up the parts, which one part then has as well (200 rows of 18,432 x 4,096, a squared relu: in
+// one part, as without it, 63 us, in two 54).
+static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0, bool unary = false) {
     const double CUS = (double)tff_device_cus();
     // Up to 16 rows: the streaming kernel, a block per 16 columns, unless those blocks go badly
     // round the 256 CUs (320 of them take as long as 512 would: N = 5120), the caller takes
@@ -1293,7 +1295,7 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
                 // the partial sums: written, read and added by a second kernel, or (kept) read by the
                 // consumer in place of one plane
                 if (S > 1 && keep) t += (S - 1.0) * M * N * 4.0 / (few ? 4e6 : 1.97e6);
-                else if (S > 1) t += (double)S * M * N * 4.0 / (few ? 2.54e6 : 2.12e6) + (few ? 2.7 : 3.84);
+                else if (S > 1 || unary) t += (double)S * M * N * 4.0 / (few ? 2.54e6 : 2.12e6) + (few ? 2.7 : 3.84);
                 if (t < best_t) { best_t = t; best = {c.bm, c.bn, S}; }
             }
         }
@@ -1432,49 +1434,10 @@ static int launch_far(const GemmPlan& plan, const bf16_t* A, const bf16_t* Wp, v
     return launch_async_g<4, 4, 4, 4, 5, GLU, 1, true>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
 }
 
-// glu_out > 0: W holds gate and up groups in turn (N = 2 * ceil16(glu_out) rows) and C is
-// [M, glu_out] = silu(gate) * up.  workspace: room for partial sums (tff_gemm_workspace_bytes);
-// with less the blocks do not split K.
-// bias (may be null): ceil16(N) float32 numbers in the order of W's rows, added to the product (before the gate's
-// activation): the accumulators start from them (of a split K, the first part's).
-// keep_partials: where the plan splits K, the partial sums stay in the workspace
-// ([splits, M, N] float32) for the caller to add up, and C is not written.
-int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda,
-                  const GemmCall ex, int c_dtype, int glu_out, float* workspace, size_t workspace_bytes,
-                  int keep_partials, hipStream_t s) {
-    TFF_REQUIRE(K % 8 == 0 && lda % 8 == 0,
-                "gemm: the bfloat16 product needs the inner size (K=%d, row stride %d) to be a multiple of 8",
-                K, lda);
-    TFF_REQUIRE(((uintptr_t)A % 16) == 0 && ((uintptr_t)Wp % 16) == 0 && ((uintptr_t)C % 16) == 0,
-                "gemm: operands must be 16-byte aligned");
-    TFF_REQUIRE(c_dtype == TFF_F32 || c_dtype == TFF_BF16, "gemm: unknown output type %d", c_dtype);
-    GemmPlan plan = plan_for(M, N, K, glu_out > 0, keep_partials != 0, ex.plane_cols);
-    const int planned_splits = plan.splits;
-    if (!workspace || workspace_bytes < (size_t)plan.splits * M * N * sizeof(float)) plan.splits = 1;
+// A product by its plan (planned_splits: the parts it would have with room for their sums).
+static int run_plan(const GemmPlan& plan, int planned_splits, bool far, const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda,
+                    const GemmCall ex, int c_dtype, int glu_out, float* workspace, bool red, hipStream_t s) {
     const int S = plan.splits;
-    const bool red = !keep_partials;
-    const bool far = plan.tile > 0 && K % 64 == 0 && !w4_reaches(plan.tile, plan.bn, K, lda);
-    if (far && ex.plane_cols) {      // (one product after the other)
-        GemmCall one = ex;
-        one.plane_cols = 0;
-        const size_t w_plane = (size_t)(ex.plane_cols / 16) * (K / 32) * 512;
-        for (int p = 0; p < N / ex.plane_cols; ++p)
-            if (int rc = tff_gemm_bf16(A + p * ex.a_step, Wp + p * w_plane, (float*)C + (size_t)p * M * ex.plane_cols, M, ex.plane_cols, K, lda, one,
-                                       c_dtype, 0, nullptr, 0, 0, s)) return rc;
-        return 0;
-    }
-    if (ex.unary && glu_out == 0 && !keep_partials && planned_splits == 1 && unary_in_float32(plan, M, N, K) && workspace &&
-        workspace_bytes >= (size_t)M * N * sizeof(float)) {
-        // K in one part, whose float32 results the sum's kernel takes as the only plane
-        GemmCall plain = ex;
-        plain.unary = 0;
-        if (int rc = tff_gemm_bf16(A, Wp, workspace, M, N, K, lda, plain, TFF_F32, 0, nullptr, 0, 0, s)) return rc;
-        return launch_reduce<false>(workspace, 1, M, N, C, N, ex, c_dtype, s);
-    }
-    TFF_REQUIRE(!ex.unary || (glu_out == 0 && !keep_partials && (plan.tile == 0 || plan.splits > 1)),
-                "gemm: an activation is applied by the streaming kernel or to the sum over the parts of K");
-    TFF_REQUIRE(!keep_partials || (glu_out == 0 && c_dtype == TFF_F32),
-                "gemm: partial sums are kept for a plain float32 result only");
     if (glu_out > 0) {
         TFF_REQUIRE(N % 32 == 0 && glu_out <= N / 2 && glu_out > N / 2 - 16,
                     "gemm: a gated weight of %d rows does not fit %d output columns", N, glu_out);
@@ -1539,6 +1502,50 @@ int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int 
     if (plan.bn == 192)
         return launch_async_g<4, 4, 4, 3, 5, false, 1, true>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
     return launch_async_g<4, 4, 4, 4, 5, false, 1, true>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
+}
+
+// glu_out > 0: W holds gate and up groups in turn (N = 2 * ceil16(glu_out) rows) and C is
+// [M, glu_out] = silu(gate) * up.  workspace: room for partial sums (tff_gemm_workspace_bytes);
+// with less the blocks do not split K.
+// bias (may be null): ceil16(N) float32 numbers in the order of W's rows, added to the product (before the gate's
+// activation): the accumulators start from them (of a split K, the first part's).
+// keep_partials: where the plan splits K, the partial sums stay in the workspace
+// ([splits, M, N] float32) for the caller to add up, and C is not written.
+int tff_gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda,
+                  const GemmCall ex, int c_dtype, int glu_out, float* workspace, size_t workspace_bytes,
+                  int keep_partials, hipStream_t s) {
+    TFF_REQUIRE(K % 8 == 0 && lda % 8 == 0,
+                "gemm: the bfloat16 product needs the inner size (K=%d, row stride %d) to be a multiple of 8",
+                K, lda);
+    TFF_REQUIRE(((uintptr_t)A % 16) == 0 && ((uintptr_t)Wp % 16) == 0 && ((uintptr_t)C % 16) == 0,
+                "gemm: operands must be 16-byte aligned");
+    TFF_REQUIRE(c_dtype == TFF_F32 || c_dtype == TFF_BF16, "gemm: unknown output type %d", c_dtype);
+    GemmPlan plan = plan_for(M, N, K, glu_out > 0, keep_partials != 0, ex.plane_cols, ex.unary != 0);
+    const int planned_splits = plan.splits;
+    if (!workspace || workspace_bytes < (size_t)plan.splits * M * N * sizeof(float)) plan.splits = 1;
+    const bool far = plan.tile > 0 && K % 64 == 0 && !w4_reaches(plan.tile, plan.bn, K, lda);
+    if (far && ex.plane_cols) {      // (one product after the other)
+        GemmCall one = ex;
+        one.plane_cols = 0;
+        const size_t w_plane = (size_t)(ex.plane_cols / 16) * (K / 32) * 512;
+        for (int p = 0; p < N / ex.plane_cols; ++p)
+            if (int rc = tff_gemm_bf16(A + p * ex.a_step, Wp + p * w_plane, (float*)C + (size_t)p * M * ex.plane_cols, M, ex.plane_cols, K, lda, one,
+                                       c_dtype, 0, nullptr, 0, 0, s)) return rc;
+        return 0;
+    }
+    if (ex.unary && glu_out == 0 && !keep_partials && planned_splits == 1 && unary_in_float32(plan, M, N, K) && workspace &&
+        workspace_bytes >= (size_t)M * N * sizeof(float)) {
+        // K in one part, whose float32 results the sum's kernel takes as the only plane
+        GemmCall plain = ex;
+        plain.unary = 0;
+        if (int rc = run_plan(plan, 1, far, A, Wp, workspace, M, N, K, lda, plain, TFF_F32, 0, nullptr, true, s)) return rc;
+        return launch_reduce<false>(workspace, 1, M, N, C, N, ex, c_dtype, s);
+    }
+    TFF_REQUIRE(!ex.unary || (glu_out == 0 && !keep_partials && (plan.tile == 0 || plan.splits > 1)),
+                "gemm: an activation is applied by the streaming kernel or to the sum over the parts of K");
+    TFF_REQUIRE(!keep_partials || (glu_out == 0 && c_dtype == TFF_F32),
+                "gemm: partial sums are kept for a plain float32 result only");
+    return run_plan(plan, planned_splits, far, A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, workspace, !keep_partials, s);
 }
 
 // ---- the norm between two products of up to 16 rows, taken into them ----
@@ -1641,13 +1648,13 @@ TFF_API int tff_gemm(const void* A, const void* W, void* C, int M, int N, int K,
 // C = act(A . W^T), act one of unary_activation's kinds, where the product's plan lets a kernel apply it to float32 sums: the streaming
 // kernel, or the sum over the parts of a split K, which may be one (unary_in_float32).  Else 0 there, and the activation is a kernel of its own.
 TFF_API int tff_gemm_takes_unary(int M, int N, int K) {
-    const GemmPlan p = plan_for(M, N, K, false, false);
+    const GemmPlan p = plan_for(M, N, K, false, false, 0, true);
     return p.tile == 0 || p.splits > 1 || unary_in_float32(p, M, N, K);
 }
 // Room for its float32 sums.
 TFF_API size_t tff_gemm_unary_workspace_bytes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const GemmPlan p = plan_for(M, N, K, false, false);
+    const GemmPlan p = plan_for(M, N, K, false, false, 0, true);
     return p.splits > 1 || unary_in_float32(p, M, N, K) ? (size_t)p.splits * M * N * sizeof(float) : 0;
 }
 TFF_API int tff_gemm_unary(const void* A, const void* W, void* C, int M, int N, int K, int lda, int c_dtype, int kind, void* workspace,
