@@ -557,7 +557,7 @@ def test_linear_of_rows_far_apart(M, N, K, lda):
         _close(ops.linear_unary(far, pw, "gelu", torch.float32), torch.nn.functional.gelu(ref), tol, "rows far apart, an activation")
 
 
-@pytest.mark.parametrize("M", [1, 8, 16, 17, 40, 100])
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 40, 100, 200])
 @pytest.mark.parametrize("N,K", [(96, 200), (1030, 1024), (5120, 512), (5120, 4096), (34000, 256), (8256, 4096)])
 def test_weights_loaded_as_read_once(M, N, K):
     """The same bits whether a weight's loads say that nobody asks for them again or not, in every kernel of few rows: plain, gated, with a

@@ -799,14 +799,10 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
             gemm_bf16_w4_kernel<WTN, NWS, GLU, bf16_t, WGM, SCALE, WTM, false, once><<<grid, 256, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, sc, ex);
     };
     // A weight that one block reads, K in one part: 40 and 100 rows of 24,576 x 4,096 38.0 / 35.6 and 43.9 / 40.7 us, 17 rows of 151,936
-    // 218 / 192 (plain loads / once).  The short streams of a split K lose by it: 100 rows of 4,096 x 4,096 16.3 / 19.4, 128 of
-    // 7,168 x 5,120 24.8 / 27.8.  (256 rows are two waves' of A, and a product that long is not bound by its weight's stream.)
-    if constexpr (WGM == 1) {
-        if (ex.once && TM == 1 && splits == 1) launch(std::true_type{});
-        else launch(std::false_type{});
-    } else {
-        launch(std::false_type{});
-    }
+    // 218 / 192 (plain loads / once), on one tile of 256 rows 200 of 24,576 x 4,096, gated, 61.3 / 58.5, of 34,816 x 5,120 105.7 / 102.9.  The short
+    // streams of a split K lose by it: 100 rows of 4,096 x 4,096 16.3 / 19.4, 128 of 7,168 x 5,120 24.8 / 27.8.
+    if (ex.once && TM == 1 && splits == 1) launch(std::true_type{});
+    else launch(std::false_type{});
     if (int rc = tff_check_launch("gemm_bf16_w4")) return rc;
     if (splits > 1 && reduce) {
         return launch_reduce<GLU>(part, splits, M, N, C, GLU ? n_out : N, ex, c_dtype, s);
