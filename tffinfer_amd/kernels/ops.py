@@ -96,7 +96,7 @@ class PackedWeight:
         self.glu_act = SILU
         #: whether no cache holds the weight from one call to the next: it is larger than they are, or belongs to a model
         #: that is (the model says so when it is loaded); products of few rows then load it as such
-        self.once = data.numel() * data.element_size() > CACHE_BYTES
+        self.once = int(data.numel() * data.element_size() > CACHE_BYTES)
 
     @property
     def shape(self):
@@ -302,7 +302,7 @@ def _fused_prenorm(p: PendingProduct, resid: torch.Tensor, weight: torch.Tensor,
     ss = torch.empty(16, stride, dtype=torch.float32, device=x.device)
     L = _lib.load()
     _lib.check(L.tff_gemm_residual_prenorm(x.data_ptr(), p.weight.data_ptr(), M, N, K, lda, resid.data_ptr(),
-                                           weight.data_ptr(), xs.data_ptr(), ss.data_ptr(), stride, int(p.weight.once), _stream()))
+                                           weight.data_ptr(), xs.data_ptr(), ss.data_ptr(), stride, p.weight.once, _stream()))
     return ScaledRows(xs, ss, groups, eps, resid, weight)
 
 
@@ -447,7 +447,7 @@ def linear(x: torch.Tensor, weight, out_dtype: torch.dtype | None = None,
             raise _lib.KernelError(f"linear out: shape {tuple(out.shape)} is not {(M, n_out)}")
     _lib.check(L.tff_gemm(x.data_ptr(), weight.data_ptr(), out.data_ptr(), M, N, K, lda,
                           dtype_code(x.dtype), dtype_code(out_dtype), 1 if packed else 0, glu_out, _ptr(bias),
-                          *(weight.glu_act if packed else SILU), _ptr(ws), ws_bytes, 1 if keep else 0, int(packed and weight.once), _stream()))
+                          *(weight.glu_act if packed else SILU), _ptr(ws), ws_bytes, 1 if keep else 0, weight.once if packed else 0, _stream()))
     return out
 
 
@@ -476,7 +476,7 @@ def linear_unary(x: torch.Tensor, weight, act: str, out_dtype: torch.dtype) -> t
             ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device) if ws_bytes else None
             out = torch.empty(M, N, dtype=out_dtype, device=x.device)
             _lib.check(L.tff_gemm_unary(x.data_ptr(), weight.data_ptr(), out.data_ptr(), M, N, K, lda, dtype_code(out_dtype), UNARY[act],
-                                        _ptr(ws), ws_bytes, int(weight.once), _stream()))
+                                        _ptr(ws), ws_bytes, weight.once, _stream()))
             return out
     if act == "tanh":
         return tanh(linear(x, weight, out_dtype=torch.float32), out_dtype)
@@ -500,7 +500,7 @@ def linear_planes(x: torch.Tensor, weight: PackedWeight) -> torch.Tensor:
                                "the inner size of 64)")
     N = weight.shape[0] // P
     out = torch.empty(P, M, N, dtype=torch.float32, device=x.device)
-    _lib.check(_lib.load().tff_gemm_planes(x.data_ptr(), M * K, weight.data_ptr(), out.data_ptr(), P, M, N, K, K, int(weight.once), _stream()))
+    _lib.check(_lib.load().tff_gemm_planes(x.data_ptr(), M * K, weight.data_ptr(), out.data_ptr(), P, M, N, K, K, weight.once, _stream()))
     return out
 
 
@@ -512,7 +512,7 @@ def _linear_row_scaled(x: ScaledRows, weight: "PackedWeight", out_dtype: torch.d
     L = _lib.load()
     _lib.check(L.tff_gemm_row_scaled(x.x.data_ptr(), weight.data_ptr(), out.data_ptr(), M, N, K, K,
                                      dtype_code(out_dtype), glu_out, x.ss.data_ptr(), x.ss.stride(0), x.count, K,
-                                     x.eps, *weight.glu_act, int(weight.once), _stream()))
+                                     x.eps, *weight.glu_act, weight.once, _stream()))
     return out
 
 
@@ -710,12 +710,14 @@ def _block_items(batch, G: int, window: int, cols: int, which: str, pool: int = 
     if sum(counts) < 64:                 # (arrays cost more than a few items)
         items = []
         for r, ncols in zip(rows, widths):
-            begin = P[r]
+            begin, top = P[r], ncols - 1
             for c0 in range(0, ncols, cols):
-                last = begin + (min(c0 + cols, ncols) - 1) // G
-                lo = max(0, begin + c0 // G - window + 1) if window > 0 else 0
-                blocks = max(0, last - window + 1) // pool if pool else 0      # keys of blocks before the window
-                items.append((last // 32 - lo // 32 + 1 + -(-blocks // 32), r, c0))
+                last = begin + (top if c0 + cols > top else c0 + cols - 1) // G
+                lo = begin + c0 // G - window + 1 if window > 0 else 0
+                n = last // 32 + 1 - (lo // 32 if lo > 0 else 0)
+                if pool and last >= window:
+                    n -= -((last - window + 1) // pool) // 32                  # (and keys of blocks before the window)
+                items.append((n, r, c0))
         return sorted(items, reverse=True)
     counts = np.asarray(counts)
     at = np.repeat(np.arange(len(rows)), counts)
@@ -731,22 +733,21 @@ def _block_items(batch, G: int, window: int, cols: int, which: str, pool: int = 
     return list(zip(slices[order].tolist(), r[order].tolist(), c0[order].tolist()))
 
 
-def _deal_items(items: list, nbins: int) -> list[list]:
-    """The items (the longest first) of every block: one each, or with more items than blocks each to the block with the least to do
-    so far."""
-    if len(items) <= nbins:
-        return [[it] for it in items]
+def _deal_items(items: list, nbins: int) -> tuple[list[list], list[tuple[int, int]]]:
+    """The items (the longest first) of every block, and (slices, block): one each, or with more items than blocks each to the block with
+    the least to do so far."""
     per_bin = [[it] for it in items[:nbins]]
     loads = [(it[0], b) for b, it in enumerate(items[:nbins])]
-    heapq.heapify(loads)
-    for it in items[nbins:]:
-        load, b = loads[0]
-        per_bin[b].append(it)
-        heapq.heapreplace(loads, (load + it[0], b))
-    return per_bin
+    if len(items) > nbins:
+        heapq.heapify(loads)
+        for it in items[nbins:]:
+            load, b = loads[0]
+            per_bin[b].append(it)
+            heapq.heapreplace(loads, (load + it[0], b))
+    return per_bin, loads
 
 
-def _dealt(batch, G: int, window: int, cols: int, which: str, nbins: int, pool: int = 0) -> list[list]:
+def _dealt(batch, G: int, window: int, cols: int, which: str, nbins: int, pool: int = 0):
     """The step's items dealt to ``nbins`` blocks, worked out once a step."""
     key = ("dealt", G, window, cols, which, nbins, pool)
     if key not in batch._attn_work:
@@ -790,7 +791,7 @@ def _attention_block_work(batch, G: int, nkv: int, window: int, device, cols: in
             groups = 1                   # LDS holds one group's stages there
         nbins = bins if bins is not None else (per_cu if groups == 2 or head_dim > 128 else 2 * per_cu)
         order, starts = [], [0]
-        for lst in _dealt(batch, G, window, cols, which, nbins, pool):
+        for lst in _dealt(batch, G, window, cols, which, nbins, pool)[0]:
             order.extend(lst)
             starts.append(len(order))
         flat = [x for it in order for x in it[1:]]
@@ -1001,6 +1002,25 @@ _PROMPT_FORMS = {128: {0: (0.9, 1.24, 9.0, 128, 2), 1: (-1.6, 0.80, 13.9, 256, 1
                  256: {0: (0.2, 1.27, 10.4, 128, 1), 1: (1.1, 0.74, 12.2, 128, 1)}}
 
 
+def _item_spans(rows: list, G: int, window: int, cols: int) -> tuple[int, float, int]:
+    """About the most 32-key slices of an item, their sum and the number of items of ``cols`` columns, for entries of so many tokens behind so many."""
+    most, total, count, d = 1, 0.0, 0, cols / G
+    for begin, n in rows:
+        k = -(-n * G // cols)
+        lo = max(0, begin + (k - 1) * cols // G - window + 1) if window > 0 else 0
+        most = max(most, (begin + n - 1) // 32 - lo // 32 + 1)
+        keys = k * begin + d * (k - 1) * k / 2 + n - 1               # (the items' last keys)
+        if window > 0:                                               # (less the first ones of items that begin behind key 0)
+            first = begin - window + 1
+            late = k - max(0, math.ceil(-first / d))
+            if late > 0:
+                keys -= late * first + d * (2 * k - 1 - late) * late / 2
+                most = max(most, (window + int(d)) // 32)
+        total += keys / 32 + 0.75 * k
+        count += k
+    return most, total, count
+
+
 def _prompt_blocks(batch, G: int, nkv: int, window: int, device, which: str, d: int, num_cus: int | None = None) -> int:
     """Which blocks the step's portions take at head sizes of :data:`PROMPT_HEAD_SIZES`: 0 those of eight waves, 1 and 2 those of four with so
     many key groups (one on items of 256 columns; two that share the slices of items of 128), by what the block with the most to do takes.
@@ -1019,21 +1039,21 @@ def _prompt_blocks(batch, G: int, nkv: int, window: int, device, which: str, d: 
         if num_cus is None:
             num_cus = _num_cus(device) if torch.device(device).type == "cuda" else 256
         bins = max(1, num_cus // max(1, nkv))
-        bounds, loads = [], {}
+        rows = [(batch.host_start_pos[r], batch.host_cu_tokens[r + 1] - batch.host_cu_tokens[r]) for r in _entries(batch, which)]
+        spans = {cols: _item_spans(rows, G, window, cols) for cols in {f[3] for f in _PROMPT_FORMS[d].values()}}
+        bounds = []
         for form, (start, step, item, cols, slices) in _PROMPT_FORMS[d].items():
-            its = _items_once(batch, G, window, cols, which)
-            total = sum([it[0] for it in its])
+            most, total, count = spans[cols]
             if form == 0 and d <= 128 and total >= 96 * 2 * bins:
                 continue                 # (long portions, where eight waves are never ahead)
-            bounds.append((start + max(step * -(-its[0][0] // slices) + item, (step * total / slices + item * len(its)) / bins), form))
+            bounds.append((start + max(step * -(-most // slices) + item, (step * total / slices + item * count) / bins), form))
         best, best_t = 0, math.inf
-        for t, form in sorted(bounds):   # (no less than that, whatever the dealing)
+        for t, form in sorted(bounds):   # (about the least it takes, however the items are dealt)
             start, step, item, cols, slices = _PROMPT_FORMS[d][form]
-            its = _items_once(batch, G, window, cols, which)
-            if t < best_t and bins < len(its) <= min(256, 4 * bins):       # (more items are dealt as good as evenly)
-                if cols not in loads:
-                    loads[cols] = {(sum([it[0] for it in lst]), len(lst)) for lst in _dealt(batch, G, window, cols, which, bins)}
-                t = start + max([step / slices * load + item * n for load, n in loads[cols]])
+            if t < best_t and bins < spans[cols][2] <= min(256, 4 * bins):       # (more items are dealt as good as evenly)
+                lists, loads = _dealt(batch, G, window, cols, which, bins)
+                per_slice = step / slices
+                t = start + max([per_slice * load + item * len(lists[b]) for load, b in loads])
             if t < best_t:
                 best, best_t = form, t
         cache[key] = best
@@ -2406,7 +2426,7 @@ def add_dyt(resid: torch.Tensor, delta, alpha: float, weight: torch.Tensor, bias
         out = torch.empty(M, H, dtype=torch.bfloat16, device=resid.device)
         _lib.check(_lib.load().tff_gemm_residual_dyt(p.x.data_ptr(), p.weight.data_ptr(), M, H, K,
                                                      p.x.stride(0) if M > 1 else K, resid.data_ptr(), float(alpha),
-                                                     weight.data_ptr(), bias.data_ptr(), out.data_ptr(), int(p.weight.once), _stream()))
+                                                     weight.data_ptr(), bias.data_ptr(), out.data_ptr(), p.weight.once, _stream()))
         return out
     terms = delta.terms if isinstance(delta, PendingTerms) else ([] if delta is None else [delta])
     d = [_planes_of(t, resid.shape, "add_dyt term") for t in terms] + [(None, 0, 0)] * 2

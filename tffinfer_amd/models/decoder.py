@@ -182,15 +182,17 @@ class DecoderModel:
         from ..kernels import ops
         packed, total = {}, 0
         for _, part in self._weighted_parts():
+            looked_up = isinstance(part, (Embedding, BigramTable))       # (a table's rows, here and there one)
             for value in vars(part).values():
-                for w in value if isinstance(value, (list, tuple)) else (value,):
-                    if isinstance(w, ops.PackedWeight):
+                kind = type(value)
+                for w in value if kind is list else (value,) if kind is ops.PackedWeight or kind is torch.Tensor else ():
+                    if type(w) is ops.PackedWeight:
                         packed[id(w)] = w
-                    elif isinstance(w, torch.Tensor) and w.dim() >= 2 and not isinstance(part, (Embedding, BigramTable)):
-                        total += w.numel() * w.element_size()       # (a table's rows are looked up, here and there one)
+                    elif type(w) is torch.Tensor and w.dim() >= 2 and not looked_up:
+                        total += w.numel() * w.element_size()
         total += sum(w.data.numel() * w.data.element_size() for w in packed.values())
         for w in packed.values():
-            w.once = total > ops.CACHE_BYTES
+            w.once = int(total > ops.CACHE_BYTES)
 
     def graph_safe(self) -> bool:
         """True if every part launches only kernels that read the step's sizes
