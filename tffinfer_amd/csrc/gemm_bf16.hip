@@ -1377,14 +1377,8 @@ static int skinny_for(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, 
                       int glu_out, hipStream_t s, const SkinnyFuse* fuse) {
     if (glu_out > 0) {
         if constexpr (EPI < 2) {
-            // Weights read once are loaded as such from 512 blocks on, two for every CU; fewer are a second round that is half empty, and take
-            // longer so (us, one and eight rows, plain / once: 9,216 x 1,536 10.4 / 10.4 and 9.8 / 11.2, 12,288 x 2,048 13.2 / 14.3 and
-            // 12.5 / 14.3, 15,360 x 2,560 17.5 / 19.0 and 17.0 / 18.6; 16,384 x 2,048 16.2 / 15.9 and 15.8 / 16.0, 20,480 x 2,560 23.3 / 21.6).
-            if (N >= 8 * 1024) {
-                GemmCall ring = ex;
-                ring.once = ex.once && N >= 16 * 1024;
-                return launch_skinny<1, 1, 8, 1, 2, true, true, EPI>(A, Wp, C, M, N, K, lda, ring, c_dtype, glu_out, s, fuse);
-            }
+            if (N >= 8 * 1024)
+                return launch_skinny<1, 1, 8, 1, 2, true, true, EPI>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, fuse);
             // A wave takes a quarter of K in groups of k-steps whose loads are issued together, and
             // the steps that are left when a group is not full go one at a time: groups of eight
             // where a quarter of K is fewer than 32 steps, of 32 (with the norm's factor taken in,
