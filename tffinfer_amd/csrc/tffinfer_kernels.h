@@ -63,6 +63,7 @@ TFF_API int tff_gemm_plan(int M, int N, int K, int glu, int keep_partials, int* 
 
 // C = act(A . W^T) in one go (kind 1: tanh, 2: gelu, 3: its tanh form, 4: the square of relu), where tff_gemm_takes_unary says so.
 TFF_API int tff_gemm_takes_unary(int M, int N, int K);
+// Room for its float32 sums (0: none is needed).
 TFF_API size_t tff_gemm_unary_workspace_bytes(int M, int N, int K);
 TFF_API int tff_gemm_unary(const void* A, const void* W, void* C, int M, int N, int K, int lda, int c_dtype, int kind, void* workspace,
                            size_t workspace_bytes, int w_once, tff_stream_t stream);
