@@ -13,86 +13,8 @@
 // staged in LDS in the same order is read back without bank conflicts.
 // Activations A [M, K] stay row-major.  The W tile is the MFMA's first operand,
 // so a lane ends up with 4 consecutive output columns of one row.
-#include "common.h"
-#include "mfma_tiles.h"
+#include "gemm_bf16.h"
 #include "tffinfer_kernels.h"
-#include <type_traits>
-
-
-__device__ __forceinline__ uint4 ld16(const bf16_t* p) { return *reinterpret_cast<const uint4*>(p); }
-// The same of a weight that one block reads; ONCE: and that nobody asks for again before it has left the caches.
-template <bool ONCE>
-__device__ __forceinline__ uint4 ld16_weight(const bf16_t* p) {
-    if constexpr (!ONCE) return ld16(p);
-    typedef __attribute__((__vector_size__(16))) unsigned once_t;
-    const once_t v = __builtin_nontemporal_load(reinterpret_cast<const once_t*>(p));
-    return make_uint4(v[0], v[1], v[2], v[3]);
-}
-__device__ __forceinline__ bf16x8 as_frag(const uint4& v) { return *reinterpret_cast<const bf16x8*>(&v); }
-
-template <typename TC>
-__device__ __forceinline__ void store4(TC* dst, const floatx4& v, int n, int N, bool vec) {
-    if (vec) {  // n % 4 == 0 and N % 4 == 0: the four columns exist
-        if constexpr (sizeof(TC) == 4) {
-            *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-            union { bf16_t h[4]; uint2 u; } pk;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) pk.h[e] = (bf16_t)v[e];
-            *reinterpret_cast<uint2*>(dst) = pk.u;
-        }
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (n + e < N) dst[e] = from_f32<TC>(v[e]);
-    }
-}
-
-// What a product takes besides its operands: a bias (float32, in the order of W's rows, ceil16(N) numbers) or null,
-// and how a gated product joins gate and up.
-struct GemmEpilogue {
-    const float* bias;
-    GluAct act;
-};
-// And what some kernels of their own take beside that (in the arguments of all, it changed the schedule of most: gate and up of 2,048 columns
-// and 3 rows 11.8 / 12.3 us).
-// unary: what becomes of a result that is not gated (unary_activation), where the streaming kernel or the sum over a split K's
-// parts stores it.  plane_cols > 0: several products in one launch.  W's rows are theirs one after the other, plane_cols each; the
-// columns of plane p take their rows from A + p * a_step, and C holds the planes [p][M][plane_cols].
-struct GemmExtra : GemmEpilogue {
-    int unary;
-    int plane_cols;
-    size_t a_step;
-};
-// And what only the launches ask.  once: no cache holds the weight from one call to the next (see the streaming kernel's note).
-struct GemmCall : GemmExtra {
-    int once;
-};
-
-// GLU: the 16-row groups of W alternate between a gate and an up projection
-// (group 2p gate, group 2p+1 up); the epilogue writes act(gate, up), N / 2 columns: silu(gate) * up, or in the form
-// with constants g sigmoid(alpha g) (u + up_offset), g = min(gate, limit), u = clamp(up, -limit, limit).
-__device__ __forceinline__ floatx4 glu4(const floatx4& g, const floatx4& u, const GluAct& act) {
-    floatx4 o;
-    if (act.plain) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = g[e] / (1.0f + __expf(-g[e])) * u[e];
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float a = fminf(g[e], act.limit), b = fminf(fmaxf(u[e], -act.limit), act.limit);
-            o[e] = a / (1.0f + __expf(-act.alpha * a)) * (b + act.up_offset);
-        }
-    }
-    return o;
-}
-
-// Four neighbouring numbers of a bias in the order of W's rows (16 NB of them), for a lane's four columns from n
-// on; columns past the end, whose results are never stored, take the last ones.
-__device__ __forceinline__ floatx4 bias4(const float* __restrict__ bias, int n, int NB) {
-    const float4 b = *reinterpret_cast<const float4*>(bias + min(n, NB * 16 - 4));
-    return floatx4{b.x, b.y, b.z, b.w};
-}
 
 // ------------------------------------------------------- tiled, async copy ---
 // Block tile (WGM*WTM*16) x (WGN*WTN*16) x (32 KPS) on WGM x WGN waves, each wave
@@ -810,218 +732,42 @@ static int launch_w4(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, i
     return 0;
 }
 
-// ------------------------------------------------------------- skinny M ---
-// For a few rows of A (decoding: M = number of live requests) the product is
-// a stream of W from HBM; what counts is bytes in flight, not LDS tiling.
-// A block owns a slab of 16*R rows of W for the whole of K; its waves split K
-// among them in contiguous runs, each wave reading its W fragments straight
-// from global memory into MFMA operands and the few rows of A from cache;
-// partial sums meet in LDS and are added in a fixed order, so no partial
-// result goes through global memory and the result does not depend on the
-// launch.  UNROLL k-steps of loads are issued before the first is used: a wave
-// keeps UNROLL * (R + MT) KB in flight, which is what hides the latency of HBM.
-// The block's waves form NSETS sets of KSPLIT waves: a set works on R row groups
-// of W, its waves split K.  Sets walk K at the same pace, so the rows of A one
-// set has fetched are in cache for the others: with many rows of A (MT > 1)
-// that, not W, is most of a wave's traffic.  With GLU, sets 2p and 2p+1 hold a
-// gate group and the up group that follows it in W; the epilogue writes
-// silu(gate) * up.
-// Where the caller says that no cache holds the weight from one call to the next (once: a model's weights are more than the 256 MB behind the
-// L2), its loads say that nobody asks for the line again (nt): the caches then keep the rows of A and do not write lines about
-// that nothing will hit.  us, four decode steps of 8 requests on 8 layers of the 8B shape 4,300 / 4,057, a prompt of 96 tokens and 15
-// decode steps of the 0.6B shape 18,700 / 17,800; the head of 151,936 columns, 3 rows, 200 / 177 (7.0 TB/s).
-// Weights that do fit lose by it: four of 5,120 x 5,120 (210 MB) in turn, 8 rows, 10.6 / 15.8 us, 24 of 4,096 x 1,024, one row, 3.4 / 3.7.
-// The four-wave kernel has the same where it reads a weight once (launch_w4).
-// Weights that others read too (several row tiles), or in pieces of 64 bytes (float32 rows, 8,030 -> 8,200), lose by it.
-//
-// An RMS norm between two such products costs a kernel of a few microseconds for a few rows.
-// Its per-row factor commutes with the product that follows it, so the two products take the
-// norm between them (EPI):
-//   2, the product before the norm (float32 result): its epilogue adds its result to the
-//      residual stream in place, writes the sum times the norm's weight as the bfloat16 input
-//      of the next product, *without* the factor rsqrt(mean of squares + eps), and leaves the
-//      sum of squares of its 16 columns of every row in ss_out[row][row group];
-//   1, the product after the norm: adds up the sums of squares of a row, in a fixed order, and
-//      multiplies its float32 accumulators by the row's factor before anything else is done
-//      to them.
-// The sum of squares is over the float32 residual stream, as in the norm's own kernel.
-//   3, the product before a norm that has no statistics (tanh(alpha v) w + b element by element): its
-//      epilogue adds its result to the residual stream in place and writes the norm of the sum as the
-//      bfloat16 input of the next product, whole: there is no factor to leave to anyone.
-struct SkinnyFuse {
-    const float* ss_in;     // EPI 1: [16][ss_stride] sums of squares, ss_count of them a row
-    int ss_stride, ss_count;
-    float inv_dim, eps;     // 1 / row length of the normalised tensor
-    float* resid;           // EPI 2: [M, N] float32, updated in place
-    const float* norm_w;    // [N]
-    bf16_t* x_out;          // [M, N]
-    float* ss_out;          // [16][ss_out_stride]
-    int ss_out_stride;
-    const float* bias;      // EPI 3: [N], and the scalar inside the tanh
-    float alpha;
-};
-
-// MORE: several products in one launch, or an activation of the result (GemmExtra).  Kernels of their own: the tests for them and the registers
-// of the activations cost every plain product 0.2 us (a decode step's of 2,048 to 4,096 columns 9.4 / 9.6, of 8 rows 10.9 / 11.1).
-template <int MT, int R, int UNROLL, int KSPLIT, int NSETS, bool GLU, typename TC, bool RING = false, int EPI = 0, bool MORE = false, bool ONCE = false>
-__global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
-    const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, TC* __restrict__ C, int M, int N,
-    int K, int lda, int KB, int n_out, SkinnyFuse fz,
-    const typename std::conditional<MORE, GemmExtra, GemmEpilogue>::type ex) {
-    const float* __restrict__ const bias = ex.bias;
-    static_assert(EPI == 0 || MT == 1, "the fused norm is for up to 16 rows");
-    static_assert(EPI < 2 || !GLU, "the product before a norm has a plain float32 result");
-    static_assert(!MORE || (EPI == 0 && !GLU), "planes and activations are for plain products");
-    constexpr int SK_WAVES = KSPLIT * NSETS;
-    static_assert(!GLU || (R == 1 && NSETS % 2 == 0), "a gate and its up group are one row group each");
-    __shared__ floatx4 part[SK_WAVES][R * MT][64];
-    const int lane = threadIdx.x & 63, wave_id = threadIdx.x >> 6;
-    const int set = wave_id / KSPLIT, wave = wave_id % KSPLIT;
+// ------------------------------------------------- few rows, no workspace ---
+// 17 to 64 rows whose plan splits K, where the caller brings no room for the parts' sums: a block owns 32 rows of W for the whole of K, its
+// eight waves split K in contiguous runs, UNROLL k-steps of loads each before the first is used, and their sums meet in LDS in a fixed order.
+template <int MT, int UNROLL, typename TC>
+__global__ __launch_bounds__(512) void gemm_bf16_row_tiles_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, TC* __restrict__ C, int M, int N, int K,
+                                                                  int lda, int KB, const GemmEpilogue ex) {
+    constexpr int R = 2, KSPLIT = 8;
+    __shared__ floatx4 part[KSPLIT][R * MT][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int fr = lane & 15, fg = lane >> 4;
     const int NB = (N + 15) / 16;
-    const int nb0 = (blockIdx.x * NSETS + set) * R;
-    int ldc = N;
-    if constexpr (MORE) {
-        if (ex.plane_cols) {      // (a wave's columns are one plane's; C as its column 0 of row 0 would lie)
-            const size_t plane = (size_t)(min(nb0, NB - 1) * 16 / ex.plane_cols);
-            A += plane * ex.a_step;
-            C += plane * (size_t)(M - 1) * ex.plane_cols;
-            ldc = ex.plane_cols;
-        }
-    }
-
+    const int nb0 = blockIdx.x * R;
     floatx4 acc[R][MT];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
+    for (int r = 0; r < R; ++r) {
+        const floatx4 b = ex.bias && wave == 0 ? bias4(ex.bias, (nb0 + r) * 16 + fg * 4, NB) : floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < MT; ++t) acc[r][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-    if (bias && wave == 0) {        // (the first of the waves that split K)
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const floatx4 b = bias4(bias, (nb0 + r) * 16 + fg * 4, NB);
-#pragma unroll
-            for (int t = 0; t < MT; ++t) acc[r][t] = b;
-        }
+        for (int t = 0; t < MT; ++t) acc[r][t] = b;
     }
-
-    // k-steps of 32 are dealt out to the waves in contiguous runs
     const int per = (KB + KSPLIT - 1) / KSPLIT;
-    const int s_begin = wave * per;
-    const int s_end = min(KB, s_begin + per);
-
-    // Row groups past the end of W and rows past the end of A repeat the last: their results
-    // are never stored, and no load of the main loop carries a predicate.
+    int s0 = wave * per;
+    const int s_end = min(KB, s0 + per);
+    // Row groups past the end of W and rows past the end of A repeat the last: their results are never stored.
     const bf16_t* wfrag[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) wfrag[r] = Wp + (size_t)min(nb0 + r, NB - 1) * KB * 512 + lane * 8;
     const bf16_t* arow[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) arow[t] = A + (size_t)min(t * 16 + fr, M - 1) * lda;
-
-    // What the epilogue needs from memory is asked for first, so that it has arrived long
-    // before the stream of W ends.
-    float row_scale = 1.f;
-    float4 resid_in[R], normw_in[R], bias_in[EPI == 3 ? R : 1];
-#pragma unroll
-    for (int r = 0; r < R; ++r) resid_in[r] = normw_in[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int r = 0; r < (EPI == 3 ? R : 1); ++r) bias_in[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-    // EPI 1: lane (fr, fg) of a set's first wave adds every fourth group of four sums of row fr,
-    // then the four lanes of a row meet: the same order in every block.  The loads are issued
-    // here, ahead of the stream of W, and added up (TFF_ROW_SCALE) when that stream has ended.
-    constexpr int SSV = 16;   // 16-byte loads a lane keeps: rows of up to 64 * SSV sums
-    float4 ssv[EPI == 1 ? SSV : 1];
-    // (the waves that write results: the first of a set, of the gate's set with GLU; rows that exist)
-    const bool scales = EPI == 1 && wave == 0 && (!GLU || (set & 1) == 0) && fr < M;
-    if constexpr (EPI == 1) {
-        if (scales) {
-            const float* sp = fz.ss_in + (size_t)fr * fz.ss_stride;
-            const int vec_end = fz.ss_count & ~3;
-#pragma unroll
-            for (int u = 0; u < SSV; ++u) {
-                const int j = fg * 4 + 16 * u;
-                ssv[u] = j < vec_end ? *reinterpret_cast<const float4*>(sp + j) : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-        }
-    }
-#define TFF_ROW_SCALE()                                                                            \
-    if constexpr (EPI == 1) {                                                                      \
-        if (scales) {                                                                              \
-            const float* sp = fz.ss_in + (size_t)fr * fz.ss_stride;                                \
-            const int vec_end = fz.ss_count & ~3;                                                  \
-            float ssum = 0.f;                                                                      \
-            _Pragma("unroll") for (int u = 0; u < SSV; ++u)                                        \
-                if (fg * 4 + 16 * u < vec_end) ssum += (ssv[u].x + ssv[u].y) + (ssv[u].z + ssv[u].w); \
-            for (int j = fg * 4 + 16 * SSV; j < vec_end; j += 16) {   /* very long rows */           \
-                const float4 v = *reinterpret_cast<const float4*>(sp + j);                         \
-                ssum += (v.x + v.y) + (v.z + v.w);                                                 \
-            }                                                                                      \
-            if (fg == 0)                                                                           \
-                for (int j = vec_end; j < fz.ss_count; ++j) ssum += sp[j];                         \
-            ssum += __shfl_xor(ssum, 16, 64);                                                      \
-            ssum += __shfl_xor(ssum, 32, 64);                                                      \
-            row_scale = rsqrtf(ssum * fz.inv_dim + fz.eps);                                        \
-        }                                                                                          \
-    }
-    if constexpr (EPI >= 2) {
-        if (wave == 0) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int n = (nb0 + r) * 16 + fg * 4;
-                if (fr < M && n < N) {
-                    resid_in[r] = *reinterpret_cast<const float4*>(fz.resid + (size_t)fr * N + n);
-                    normw_in[r] = *reinterpret_cast<const float4*>(fz.norm_w + n);
-                    if constexpr (EPI == 3) bias_in[r] = *reinterpret_cast<const float4*>(fz.bias + n);
-                }
-            }
-        }
-    }
-
     const int full_end = min(s_end, K / 32);   // steps below K / 32 have all their 32 k in A
-    int s0 = s_begin;
-    if constexpr (RING) {
-        // A ring of UNROLL k-steps in registers: a slot is loaded again as soon as it has been
-        // used, so the wave has UNROLL * (R + MT) KB in flight from its first step to its last.
-        // Loads come back in order, so the wait before a slot's use leaves the younger ones in
-        // flight.  Steps past the end load the last step again and are not used.
-        if (s0 < full_end) {
-            uint4 rw[UNROLL][R], ra[UNROLL][MT];
-            const int last = full_end - 1;
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u) {
-                const int st = min(s0 + u, last);
-#pragma unroll
-                for (int r = 0; r < R; ++r) rw[u][r] = ld16_weight<ONCE>(wfrag[r] + (size_t)st * 512);
-#pragma unroll
-                for (int t = 0; t < MT; ++t) ra[u][t] = ld16(arow[t] + st * 32 + fg * 8);
-            }
-            for (; s0 < full_end; s0 += UNROLL) {
-#pragma unroll
-                for (int u = 0; u < UNROLL; ++u) {
-                    if (s0 + u < full_end) {
-#pragma unroll
-                        for (int r = 0; r < R; ++r)
-#pragma unroll
-                            for (int t = 0; t < MT; ++t)
-                                acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                    as_frag(rw[u][r]), as_frag(ra[u][t]), acc[r][t], 0, 0, 0);
-                    }
-                    const int st = min(s0 + UNROLL + u, last);
-#pragma unroll
-                    for (int r = 0; r < R; ++r) rw[u][r] = ld16_weight<ONCE>(wfrag[r] + (size_t)st * 512);
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) ra[u][t] = ld16(arow[t] + st * 32 + fg * 8);
-                }
-            }
-            s0 = full_end;
-        }
-    }
-    for (; !RING && s0 + UNROLL <= full_end; s0 += UNROLL) {
+    for (; s0 + UNROLL <= full_end; s0 += UNROLL) {
         uint4 rw[UNROLL][R], ra[UNROLL][MT];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) rw[u][r] = ld16_weight<ONCE>(wfrag[r] + (size_t)(s0 + u) * 512);
+            for (int r = 0; r < R; ++r) rw[u][r] = ld16(wfrag[r] + (size_t)(s0 + u) * 512);
 #pragma unroll
             for (int t = 0; t < MT; ++t) ra[u][t] = ld16(arow[t] + (s0 + u) * 32 + fg * 8);
         }
@@ -1031,8 +777,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
             for (int r = 0; r < R; ++r)
 #pragma unroll
                 for (int t = 0; t < MT; ++t)
-                    acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(rw[u][r]), as_frag(ra[u][t]),
-                                                                        acc[r][t], 0, 0, 0);
+                    acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(rw[u][r]), as_frag(ra[u][t]), acc[r][t], 0, 0, 0);
     }
     // what is left, a step at a time; in the last step of K some k may not exist in A
     for (; s0 < s_end; ++s0) {
@@ -1040,7 +785,7 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
         const bool kok = k < K;
         uint4 rw[R], ra[MT];
 #pragma unroll
-        for (int r = 0; r < R; ++r) rw[r] = ld16_weight<ONCE>(wfrag[r] + (size_t)s0 * 512);
+        for (int r = 0; r < R; ++r) rw[r] = ld16(wfrag[r] + (size_t)s0 * 512);
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             const uint4 v = ld16(arow[t] + (kok ? k : 0));
@@ -1049,132 +794,35 @@ __global__ __launch_bounds__(64 * KSPLIT * NSETS) void gemm_bf16_skinny_kernel(
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
-            for (int t = 0; t < MT; ++t)
-                acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(rw[r]), as_frag(ra[t]), acc[r][t], 0, 0, 0);
+            for (int t = 0; t < MT; ++t) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(rw[r]), as_frag(ra[t]), acc[r][t], 0, 0, 0);
     }
-    TFF_ROW_SCALE()
-#undef TFF_ROW_SCALE
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int t = 0; t < MT; ++t) part[wave_id][r * MT + t][lane] = acc[r][t];
+        for (int t = 0; t < MT; ++t) part[wave][r * MT + t][lane] = acc[r][t];
     __syncthreads();
-    if (wave == 0) {   // the first wave of every set adds up the set's partial sums, in a fixed order
-        if constexpr (GLU) {
-            if ((set & 1) == 0) {
-                const bool vec = (n_out % 4) == 0;
+    if (wave != 0) return;      // the first wave adds up
 #pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    floatx4 g = part[set * KSPLIT][t][lane], u = part[(set + 1) * KSPLIT][t][lane];
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-                    for (int w = 1; w < KSPLIT; ++w) {
-                        const floatx4 pg = part[set * KSPLIT + w][t][lane], pu = part[(set + 1) * KSPLIT + w][t][lane];
+        for (int t = 0; t < MT; ++t) {
+            floatx4 v = part[0][r * MT + t][lane];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) { g[e] += pg[e]; u[e] += pu[e]; }
-                    }
-                    if constexpr (EPI == 1) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) { g[e] *= row_scale; u[e] *= row_scale; }
-                    }
-                    const int n = (nb0 >> 1) * 16 + fg * 4;
-                    const int m = t * 16 + fr;
-                    if (m < M && n < n_out) store4<TC>(C + (size_t)m * n_out + n, glu4(g, u, ex.act), n, n_out, vec);
-                }
+            for (int w = 1; w < KSPLIT; ++w) {
+                const floatx4 p = part[w][r * MT + t][lane];
+                v[0] += p[0]; v[1] += p[1]; v[2] += p[2]; v[3] += p[3];
             }
-        } else {
-            const bool vec = (ldc % 4) == 0;
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    floatx4 v = part[set * KSPLIT][r * MT + t][lane];
-#pragma unroll
-                    for (int w = 1; w < KSPLIT; ++w) {
-                        const floatx4 p = part[set * KSPLIT + w][r * MT + t][lane];
-                        v[0] += p[0]; v[1] += p[1]; v[2] += p[2]; v[3] += p[3];
-                    }
-                    const int n = (nb0 + r) * 16 + fg * 4;
-                    const int m = t * 16 + fr;
-                    if constexpr (EPI == 1) {
-                        v[0] *= row_scale; v[1] *= row_scale; v[2] *= row_scale; v[3] *= row_scale;
-                    }
-                    if constexpr (EPI == 2) {
-                        // N is a multiple of 4 here: four columns are in or out together
-                        float ss = 0.f;
-                        if (m < M && n < N) {
-                            const float4 sum = make_float4(resid_in[r].x + v[0], resid_in[r].y + v[1],
-                                                           resid_in[r].z + v[2], resid_in[r].w + v[3]);
-                            *reinterpret_cast<float4*>(fz.resid + (size_t)m * N + n) = sum;
-                            union { bf16_t h[4]; uint2 u; } pk;
-                            pk.h[0] = (bf16_t)(sum.x * normw_in[r].x);
-                            pk.h[1] = (bf16_t)(sum.y * normw_in[r].y);
-                            pk.h[2] = (bf16_t)(sum.z * normw_in[r].z);
-                            pk.h[3] = (bf16_t)(sum.w * normw_in[r].w);
-                            *reinterpret_cast<uint2*>(fz.x_out + (size_t)m * N + n) = pk.u;
-                            ss = fmaf(sum.x, sum.x, fmaf(sum.y, sum.y, fmaf(sum.z, sum.z, sum.w * sum.w)));
-                        }
-                        ss += __shfl_xor(ss, 16, 64);
-                        ss += __shfl_xor(ss, 32, 64);
-                        if (fg == 0 && nb0 + r < NB) fz.ss_out[(size_t)fr * fz.ss_out_stride + nb0 + r] = ss;
-                    } else if constexpr (EPI == 3) {
-                        if (m < M && n < N) {
-                            const float4 sum = make_float4(resid_in[r].x + v[0], resid_in[r].y + v[1],
-                                                           resid_in[r].z + v[2], resid_in[r].w + v[3]);
-                            *reinterpret_cast<float4*>(fz.resid + (size_t)m * N + n) = sum;
-                            union { bf16_t h[4]; uint2 u; } pk;
-                            pk.h[0] = (bf16_t)fmaf(tanhf(fz.alpha * sum.x), normw_in[r].x, bias_in[r].x);
-                            pk.h[1] = (bf16_t)fmaf(tanhf(fz.alpha * sum.y), normw_in[r].y, bias_in[r].y);
-                            pk.h[2] = (bf16_t)fmaf(tanhf(fz.alpha * sum.z), normw_in[r].z, bias_in[r].z);
-                            pk.h[3] = (bf16_t)fmaf(tanhf(fz.alpha * sum.w), normw_in[r].w, bias_in[r].w);
-                            *reinterpret_cast<uint2*>(fz.x_out + (size_t)m * N + n) = pk.u;
-                        }
-                    } else if (m < M && n < N) {
-                        if constexpr (MORE) {
-                            if (ex.unary) {
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) v[e] = unary_activation(v[e], ex.unary);
-                            }
-                        }
-                        store4<TC>(C + (size_t)m * ldc + n, v, n, N, vec);
-                    }
-                }
+            const int n = (nb0 + r) * 16 + fg * 4, m = t * 16 + fr;
+            if (m < M && n < N) store4<TC>(C + (size_t)m * N + n, v, n, N, (N % 4) == 0);
         }
-    }
 }
 
-template <int MT, int R, int UNROLL, int KSPLIT, int NSETS = 1, bool GLU = false, bool RING = false, int EPI = 0>
-static int launch_skinny(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda,
-                         const GemmCall ex, int c_dtype, int n_out, hipStream_t s, const SkinnyFuse* fuse = nullptr) {
-    const int NB = (N + 15) / 16, KB = (K + 31) / 32;
-    const int per_block = NSETS * R;
-    const dim3 grid((NB + per_block - 1) / per_block);
-    const SkinnyFuse fz = fuse ? *fuse : SkinnyFuse{nullptr, 0, 0, 0.f, 0.f, nullptr, nullptr, nullptr, nullptr, 0, nullptr, 0.f};
-    auto launch = [&](auto ONCE) {
-        constexpr bool once = decltype(ONCE)::value;
-        if (ex.plane_cols || ex.unary) {
-            if constexpr (EPI == 0 && !GLU) {
-                if (c_dtype == TFF_F32)
-                    gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, false, float, RING, 0, true, once>
-                        <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, KB, n_out, fz, ex);
-                else
-                    gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, false, bf16_t, RING, 0, true, once>
-                        <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, fz, ex);
-                return tff_check_launch("gemm_bf16_skinny");
-            } else {
-                return tff_fail("gemm: planes or an activation of a gated or fused product");
-            }
-        }
-        if (c_dtype == TFF_F32)
-            gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, GLU, float, RING, EPI, false, once>
-                <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, KB, n_out, fz, ex);
-        else if constexpr (EPI < 2)
-            gemm_bf16_skinny_kernel<MT, R, UNROLL, KSPLIT, NSETS, GLU, bf16_t, RING, EPI, false, once>
-                <<<grid, 64 * KSPLIT * NSETS, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, KB, n_out, fz, ex);
-        else
-            return tff_fail("gemm: the product before a norm has a float32 result");
-        return tff_check_launch("gemm_bf16_skinny");
-    };
-    return ex.once ? launch(std::true_type{}) : launch(std::false_type{});
+template <int MT>
+static int launch_row_tiles(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmEpilogue& ex, int c_dtype, hipStream_t s) {
+    const dim3 grid(((N + 15) / 16 + 1) / 2);
+    if (c_dtype == TFF_F32) gemm_bf16_row_tiles_kernel<MT, 4, float><<<grid, 512, 0, s>>>(A, Wp, (float*)C, M, N, K, lda, (K + 31) / 32, ex);
+    else gemm_bf16_row_tiles_kernel<MT, 4, bf16_t><<<grid, 512, 0, s>>>(A, Wp, (bf16_t*)C, M, N, K, lda, (K + 31) / 32, ex);
+    return tff_check_launch("gemm_bf16_row_tiles");
 }
 
 // The tiled product's plan for M > 16: which tile, and into how many parts the blocks of a
@@ -1183,23 +831,18 @@ static int launch_skinny(const bf16_t* A, const bf16_t* Wp, void* C, int M, int 
 // up to 64 and 32 rows, of 64 and 32 rows (256 or 128 columns), and from 65 to 512 rows also
 // 64 x 128 with several row tiles; otherwise the sixteen-wave kernel's tiles.
 struct GemmPlan { int tile; int bn; int splits; };   // tile = rows of a block tile
-// Up to 16 rows, not gated: more row groups of 16 columns than CUs, but at most 1.6 times as many
-// (a second round of blocks that would be less than 0.6 full): the streaming kernel then gives a block
-// two row groups (skinny_for).
+// Up to 16 rows, not gated: more row groups of 16 columns than CUs, but at most 1.6 times as many (see plan_for).
 static bool two_row_groups(int N) {
     const int nb = (N + 15) / 16, cus = tff_device_cus();
     return nb > cus && nb * 10 <= cus * 16;
 }
-// Up to 16 rows, gated: the streaming kernel's blocks each fetch all of A's rows, so its time grows
-// with the rows, and with a very large weight (the 32B shape's gate+up, 262M elements, 3,200 blocks)
-// that traffic shows even with one row.  The four-wave kernel's tiles of 32 rows, K in one part, take
-// the same time whatever the rows, so each weight crosses over at its number of rows (us at 1 / 4 /
-// 8 / 12 / 16 rows, streaming against tiles): the 32B shape 94 / 96 / 100 / 107 / 120 against 91 to
-// 92; the 14B shape (1.8e8 elements) 67 / 69 / 71 / 77 / 89 against 68 to 70; the 8B shape (1.0e8)
-// 36 / 37 / 37 / 40 / 44 against 39; the 4B shape (5e7) 21 / 21 / 22 / 24 / 28 against 25.
+// Up to 16 rows, gated: the streaming kernel's time grows with the rows, that of the four-wave kernel's tiles of 32 rows, K in one part, does not.
+// us at 2 / 8 / 12 / 16 rows after a norm, streaming against tiles: the 32B shape's gate and up (2.6e8 elements) 84.8 / 85.8 / 92.7 / 97.3 against 87; the
+// 14B shape's (1.8e8, 272 tiles of 128 columns: a second round for 16 of them) 60.8 / 62.1 / 67.6 / 70.9 against 73 to 75; the 8B shape's (1.0e8, 192
+// tiles) 35.2 / 35.8 / 41.6 / 41.6 against 39 to 41; the 4B shape's (5e7) 18.9 / 19.5 / 21.9 / 22.6 against 23.8.
 static bool few_rows_gated_on_tiles(int M, int N, int K) {
     const double w = (double)N * K;
-    return K % 64 == 0 && (w >= 2.4e8 || (w >= 1.6e8 && M >= 5) || (w >= 0.9e8 && M >= 12) || (w >= 0.45e8 && M >= 14));
+    return K % 64 == 0 && (w >= 2.4e8 || (w >= 0.9e8 && w < 1.6e8 && M >= 12));
 }
 // One row tile of 32 rows, K in one part: the width (128 or 256 columns) that plan_for's model prices lowest.
 static int plan_rows32(int N, int K) {
@@ -1369,54 +1012,6 @@ TFF_API int tff_gemm_plan(int M, int N, int K, int glu, int keep_partials, int* 
     return 0;
 }
 
-// Up to 16 rows: which streaming kernel.  Gated: with 512 row groups and more a wave takes
-// a group's whole K through a ring (384 such waves, at N = 6,144, are too few: 3 % slower).  Plain: more waves per block where there are few blocks
-// (small N) or long rows (large K), fewer and deeper ones in between.
-template <int EPI>
-static int skinny_for(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmCall ex, int c_dtype,
-                      int glu_out, hipStream_t s, const SkinnyFuse* fuse) {
-    if (glu_out > 0) {
-        if constexpr (EPI < 2) {
-            if (N >= 8 * 1024)
-                return launch_skinny<1, 1, 8, 1, 2, true, true, EPI>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, fuse);
-            // A wave takes a quarter of K in groups of k-steps whose loads are issued together, and
-            // the steps that are left when a group is not full go one at a time: groups of eight
-            // where a quarter of K is fewer than 32 steps, of 32 (with the norm's factor taken in,
-            // which needs registers of its own, 24) otherwise.
-            if (K < 4096)
-                return launch_skinny<1, 1, 8, 4, 2, true, false, EPI>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, fuse);
-            return launch_skinny<1, 1, (EPI == 1 ? 24 : 32), 4, 2, true, false, EPI>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, fuse);
-        } else {
-            return tff_fail("gemm: a gated product does not come before a norm");
-        }
-    }
-    // A block per 16 columns goes badly round the CUs when there are a little more row groups than
-    // CUs (320 of them, N = 5120, take as long as 512 would).  Then a block takes two row groups:
-    // half as many blocks, all at once, and between them they still pull what HBM gives (some 130
-    // CUs do).  Measured at N = 5120 against tiles that split K with a norm kernel to add their
-    // parts: O of the 14B shape 11.9 / 14.1 / 16.7 us at 1 / 8 / 16 rows against 13.7 / 15.1 / 19.0,
-    // of the 32B shape 20.4 / 21.6 / 24.0 against 27.2 / 27.4 / 27.5; down of the 14B shape 33.4 /
-    // 39.8 against 42.9 / 42.8 at 1 / 8 rows (at 16 rows the tiles are ahead, see plan_for).  Not for
-    // the product after a norm: the row factors' registers do not fit beside two row groups.
-    if constexpr (EPI != 1) {
-        if (two_row_groups(N)) return launch_skinny<1, 2, 4, 16, 1, false, false, EPI>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, fuse);
-    }
-    // A very wide product (an output head) has thousands of blocks, each of which fetches all of A's
-    // rows: with many rows and a long K that traffic shows (152k columns, K = 4,096: 196 / 217 / 281 us
-    // at 1 / 8 / 16 rows).  Two groups of 16 columns a block halve it: 243 us at 16 rows, K = 5,120 at
-    // 8 / 16 rows 264 / 303 us against 278 / 366; with fewer rows one group a block stays ahead.
-    if constexpr (EPI == 0) {
-        if (N >= 32 * 1024 && (long)M * K >= 40000)
-            return launch_skinny<1, 2, 4, 8, 1, false, false, 0>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, fuse);
-    }
-    // (K up to 1,024: sixteen waves would have two k-steps each, less than a group of four)
-    if (N >= 32 * 1024 || K <= 1024)
-        return launch_skinny<1, 1, 4, 8, 1, false, false, EPI>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, fuse);
-    if (K >= 8192 || N <= 4096)
-        return launch_skinny<1, 1, 4, 16, 1, false, false, EPI>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, fuse);
-    return launch_skinny<1, 1, 8, 4, 1, false, false, EPI>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, fuse);
-}
-
 // The four-wave tiles address a block's rows and its columns of W by 32-bit offsets.  Rows or a stride too long for a plan's tile (256 rows
 // 8.4 million elements apart, K of 11 million on 192 columns) go to the sixteen-wave kernel, which has 64 bits a copy, K in as many parts.
 template <bool GLU>
@@ -1437,7 +1032,7 @@ static int run_plan(const GemmPlan& plan, int planned_splits, bool far, const bf
     if (glu_out > 0) {
         TFF_REQUIRE(N % 32 == 0 && glu_out <= N / 2 && glu_out > N / 2 - 16,
                     "gemm: a gated weight of %d rows does not fit %d output columns", N, glu_out);
-        if (plan.tile == 0) return skinny_for<0>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, nullptr);
+        if (plan.tile == 0) return tff_gemm_few_rows(0, A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, FewRowsFuse{});
         if (far) return launch_far<true>(plan, A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, workspace, true);
         if (plan.tile <= 64 && K % 64 == 0) {                // the four waves side by side on 64 or 32 rows
             if (plan.tile == 32 && plan.bn == 128) return launch_w4<2, 5, true, 1, false, 2>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
@@ -1463,13 +1058,13 @@ static int run_plan(const GemmPlan& plan, int planned_splits, bool far, const bf
             return launch_async_g<2, 4, 4, 4, 3, true>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
         return launch_async_g<4, 4, 4, 4, 5, true, 1, true>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
     }
-    if (plan.tile == 0) return skinny_for<0>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, nullptr);
+    if (plan.tile == 0) return tff_gemm_few_rows(0, A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, FewRowsFuse{});
     if (plan.tile == 64 || plan.tile == 32) {
         // few columns and no room for partial sums: the streaming kernel, whose blocks split K
         // among their waves
         if (S == 1 && planned_splits > 1 && M <= 64) {
-            if (M <= 32) return launch_skinny<2, 2, 4, 8>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s);
-            return launch_skinny<4, 2, 4, 8>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s);
+            if (M <= 32) return launch_row_tiles<2>(A, Wp, C, M, N, K, lda, ex, c_dtype, s);
+            return launch_row_tiles<4>(A, Wp, C, M, N, K, lda, ex, c_dtype, s);
         }
         if (far) return launch_far<false>(plan, A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, workspace, red);
         if (K % 64 == 0) {                                   // the four waves side by side on 64 or 32 rows
@@ -1567,8 +1162,8 @@ TFF_API int tff_gemm_residual_prenorm(const void* A, const void* Wp, int M, int 
                 "ss_out needs %d floats a row, has %d", N, (N + 15) / 16, ss_stride);
     TFF_REQUIRE(((uintptr_t)resid % 16) == 0 && ((uintptr_t)norm_w % 16) == 0 && ((uintptr_t)x_out % 8) == 0,
                 "gemm_residual_prenorm: operands must be 16-byte aligned");
-    SkinnyFuse fz{nullptr, 0, 0, 0.f, 0.f, resid, norm_w, (bf16_t*)x_out, ss_out, ss_stride, nullptr, 0.f};
-    return skinny_for<2>((const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmCall{{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, 0, 0}, w_once}, TFF_F32, 0, (hipStream_t)stream, &fz);
+    FewRowsFuse fz{nullptr, 0, 0, 0.f, 0.f, resid, norm_w, (bf16_t*)x_out, ss_out, ss_stride, nullptr, 0.f};
+    return tff_gemm_few_rows(2, (const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmCall{{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, 0, 0}, w_once}, TFF_F32, 0, (hipStream_t)stream, fz);
 }
 
 // resid[M, N] += A . W^T (bfloat16 A and packed W, float32 sums); x_out[M, N] = bfloat16 of
@@ -1581,8 +1176,8 @@ TFF_API int tff_gemm_residual_dyt(const void* A, const void* Wp, int M, int N, i
     TFF_REQUIRE(N % 8 == 0, "gemm_residual_dyt: N=%d must be a multiple of 8", N);
     TFF_REQUIRE(((uintptr_t)resid % 16) == 0 && ((uintptr_t)norm_w % 16) == 0 && ((uintptr_t)bias % 16) == 0 &&
                 ((uintptr_t)x_out % 8) == 0, "gemm_residual_dyt: operands must be 16-byte aligned");
-    SkinnyFuse fz{nullptr, 0, 0, 0.f, 0.f, resid, norm_w, (bf16_t*)x_out, nullptr, 0, bias, alpha};
-    return skinny_for<3>((const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmCall{{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, 0, 0}, w_once}, TFF_F32, 0, (hipStream_t)stream, &fz);
+    FewRowsFuse fz{nullptr, 0, 0, 0.f, 0.f, resid, norm_w, (bf16_t*)x_out, nullptr, 0, bias, alpha};
+    return tff_gemm_few_rows(3, (const bf16_t*)A, (const bf16_t*)Wp, resid, M, N, K, lda, GemmCall{{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, 0, 0}, w_once}, TFF_F32, 0, (hipStream_t)stream, fz);
 }
 
 // C = rstd[m] * (A . W^T) with rstd[m] = rsqrt(sum_g ss[m][g] / dim + eps), g < ss_count: the product
@@ -1610,8 +1205,8 @@ TFF_API int tff_gemm_row_scaled(const void* A, const void* Wp, void* C, int M, i
             return launch_w4<2, 5, true, 1, true, 2>(a, w, C, M, N, K, lda, ex, c_dtype, glu_out, s, 1, nullptr, true, sc);
         return launch_w4<4, 5, true, 1, true, 2>(a, w, C, M, N, K, lda, ex, c_dtype, glu_out, s, 1, nullptr, true, sc);
     }
-    SkinnyFuse fz{ss, ss_stride, ss_count, 1.0f / (float)dim, eps, nullptr, nullptr, nullptr, nullptr, 0, nullptr, 0.f};
-    return skinny_for<1>((const bf16_t*)A, (const bf16_t*)Wp, C, M, N, K, lda, ex, c_dtype, glu_out, (hipStream_t)stream, &fz);
+    FewRowsFuse fz{ss, ss_stride, ss_count, 1.0f / (float)dim, eps, nullptr, nullptr, nullptr, nullptr, 0, nullptr, 0.f};
+    return tff_gemm_few_rows(1, (const bf16_t*)A, (const bf16_t*)Wp, C, M, N, K, lda, ex, c_dtype, glu_out, (hipStream_t)stream, fz);
 }
 
 int tff_gemm_f32(const float* A, const float* W, void* C, int M, int N, int K, int lda,
