@@ -125,3 +125,18 @@ def test_tables_too_small_are_refused():
 def test_no_rows():
     runs, start, blocks, merge = deal_key_runs([], 0, 8)
     assert start.tolist() == [0] and np.all(runs[:, 0] == -1) and not blocks and not merge
+
+
+def test_short_rows_stay_a_run_each_where_a_block_of_waves_takes_one():
+    from tffinfer_amd.kernels.key_runs import CUS, SHORT_STEPS
+    longest = SHORT_STEPS * KEY_STEP - 1
+    for R, nkv, window in ((1, 8, 0), (32, 8, 0), (3, 4, 700), (256, 1, 0)):
+        pos = [longest] + [(37 * i) % longest for i in range(1, R)]
+        dealt = deal_key_runs(pos, window, nkv, short=True)
+        assert dealt.run_start[-1] == R and not dealt.merge
+        check_runs(dealt.runs, dealt.run_start, pos, window)
+    # a step more, or more pairs than CUs: as without
+    for pos, nkv in (([longest + 1, 5], 8), ([longest] * (CUS // 8 + 1), 8)):
+        a, b = deal_key_runs(pos, 0, nkv, short=True), deal_key_runs(pos, 0, nkv)
+        assert np.array_equal(a.run_start, b.run_start) and np.array_equal(a.runs[:a.run_start[-1]], b.runs[:b.run_start[-1]])
+        assert a.merge == b.merge and a.blocks == b.blocks

@@ -90,6 +90,8 @@ struct AttnFuse {
     const int32_t* pool_tables;
     int pt_stride;
     int pool;
+    // With key_runs: every entry is one run, run r entry r's, and the page numbers are asked for together with the run instead of after it.
+    int run_is_entry;
 };
 
 // The last block that position pos sees (-1: none).
@@ -217,14 +219,18 @@ __global__ __launch_bounds__(64 * BW, 1) void attn_wave_kernel(
     // waves with work crowded on the other half (a fifth slower at 64 entries of one run each).
     bool by_runs = false;
     if constexpr (SPLIT || (FUSED && BW > 1)) by_runs = fz.key_runs != nullptr;
-    int r, col0, g = blockIdx.y, run_index = 0;
+    int r, col0, g = blockIdx.y, run_index = 0, early_page = 0;
     int4 run = make_int4(0, 0, 0, 0);
     if (by_runs) {
         const int eight = blockIdx.x / (8 * nkv), within = blockIdx.x - eight * (8 * nkv);
         run_index = eight * 8 + (within & 7);
         g = within >> 3;
+        if (fz.run_is_entry) {
+            if (run_index >= T_total) return;
+            early_page = block_tables[(size_t)run_index * bt_stride + min(lane, bt_stride - 1)];
+        }
         run = reinterpret_cast<const int4*>(fz.key_runs)[run_index];
-        r = run.x;
+        r = fz.run_is_entry ? run_index : run.x;
         if (r < 0) return;
         col0 = blockIdx.z * 16;
     } else if (work) {
@@ -276,12 +282,22 @@ __global__ __launch_bounds__(64 * BW, 1) void attn_wave_kernel(
     // runs neither overlap nor leave a gap)
     const bool run_is_partial = by_runs && (s_begin > 0 || s_end < nsteps);
     if constexpr (BW > 1) {
-        // the block's keys (all of the entry's, or its run) among its waves, never under 96 keys a
-        // wave, as below
+        // the block's keys (all of the entry's, or its run) among its waves.  Where they are a few steps each, the first wave, which starts first, has
+        // the last step alone: the new token's key is there, to norm and rotate beside its keys (one request, us, 400 / 500 / 640 keys with
+        // equal shares 8.2 / 10.4 / 11.1, so 8.2 / 9.0 / 10.5; down to a step of 32 a wave, since a wave with more goes through them one round trip to memory
+        // after the other)
         const int lo = s_begin, hi = s_end;
-        const int per = max((hi - lo + BW - 1) / BW, min(3, hi - lo));
-        s_begin = min(hi, lo + wv * per);
-        s_end = min(hi, s_begin + per);
+        if (hi - lo > 3 * BW) {
+            const int per = (hi - lo + BW - 1) / BW;
+            s_begin = min(hi, lo + wv * per);
+            s_end = min(hi, s_begin + per);
+        } else if (wv == 0) {
+            s_begin = max(lo, hi - 1);
+        } else {
+            const int last = max(lo, hi - 1), per = (last - lo + BW - 2) / (BW - 1);
+            s_begin = min(last, lo + (wv - 1) * per);
+            s_end = min(last, s_begin + per);
+        }
     }
     if (SPLIT && !by_runs) {
         // The launch is sized for the longest context the engine allows; with shorter ones a run
@@ -322,14 +338,17 @@ __global__ __launch_bounds__(64 * BW, 1) void attn_wave_kernel(
     // is a wait for nothing else): one round trip instead of one per table.  What is not needed
     // for the addresses of the keys (norm weights, angles, the raw q, k and v) is put to use
     // after the first keys and values are on their way.
-    int new_page = 0, first_page = 0, first_count = 0;
+    int first_page = 0, first_count = 0;
     if (!POOL && s_begin < s_end) {
         pi0 = page_index(kb0 + s_begin * 32, page_size, page_shift);
         first_count = page_index(min(kmax, kb0 + min(s_end, s_begin + seg_steps) * 32 - 1), page_size, page_shift) - pi0 + 1;
-        if (lane < first_count) first_page = bt[pi0 + lane];
-    }
-    if constexpr (FUSED) {
-        if (owns_new) new_page = bt[page_index(P, page_size, page_shift)];
+        if (FUSED && by_runs && fz.run_is_entry && pi0 + first_count <= 64) {     // (the entry's first pages are here already)
+            first_count += pi0;
+            pi0 = 0;
+            first_page = early_page;
+        } else if (lane < first_count) {
+            first_page = bt[pi0 + lane];
+        }
     }
     constexpr int FZN = FUSED ? (D + 63) / 64 : 1;
     float fz_q[FZN], fz_k[FZN], fz_cs[FZN];
@@ -540,23 +559,6 @@ __global__ __launch_bounds__(64 * BW, 1) void attn_wave_kernel(
                 if (has_norm || has_rope) norm_rope_fragments<DT>(qf, has_norm, fz_lds, fz.eps, has_rope, fz_lds + 2 * D, fz.pairing, kg);
                 if (owns_new) {
                     norm_rope_fragments<DT>(knew, has_norm, fz_lds + D, fz.eps, has_rope, fz_lds + 2 * D, fz.pairing, kg);
-                    if (col0 == 0) {
-                        const int page = new_page;
-                        const int slot = page_slot(P, page_size, page_shift);
-                        if (qc == 0) {
-                            bf16_t* kd = fz.k_write + (((size_t)page * nkv + g) * page_size + slot) * D;
-#pragma unroll
-                            for (int ks = 0; ks < KS; ++ks) {
-                                const int e = ks * 32 + kg * 8;
-                                if (e < D) *reinterpret_cast<uint4*>(kd + e) = *reinterpret_cast<const uint4*>(&knew[ks]);
-                            }
-                        }
-                        if (kg == 0) {
-                            bf16_t* vd = fz.v_write + ((size_t)page * nkv + g) * D * page_size + slot;
-#pragma unroll
-                            for (int dt = 0; dt < DT; ++dt) vd[(size_t)(dt * 16 + qc) * page_size] = vnew[dt];
-                        }
-                    }
                 }
             }
         }
@@ -578,6 +580,26 @@ __global__ __launch_bounds__(64 * BW, 1) void attn_wave_kernel(
             }
     }
     }   // blocks' keys, tokens' keys
+    if constexpr (FUSED) {
+        // The token's key and value into their page: behind the last loads, since a load's wait is also one for the stores before it (500 keys, one
+        // request, eight waves with two steps each: 11.0 us with the stores between the steps).
+        if (owns_new && col0 == 0) {
+            const int page = TFF_WAVE_PAGE(P), slot = page_slot(P, page_size, page_shift);
+            if (qc == 0) {
+                bf16_t* kd = fz.k_write + (((size_t)page * nkv + g) * page_size + slot) * D;
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    const int e = ks * 32 + kg * 8;
+                    if (e < D) *reinterpret_cast<uint4*>(kd + e) = *reinterpret_cast<const uint4*>(&knew[ks]);
+                }
+            }
+            if (kg == 0) {
+                bf16_t* vd = fz.v_write + ((size_t)page * nkv + g) * D * page_size + slot;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) vd[(size_t)(dt * 16 + qc) * page_size] = vnew[dt];
+            }
+        }
+    }
 #undef TFF_WAVE_PAGE
 #undef TFF_WAVE_PATCH
 #undef TFF_WAVE_LOAD
@@ -1585,6 +1607,7 @@ TFF_API int tff_attention_decode_runs(const void* qkv, int qkv_stride, void* out
     if (R == 0 || num_runs == 0) return 0;
     AttnFuse fz{q_weight, k_weight, cos_sin, slot_mapping ? (bf16_t*)k_cache : nullptr,
                 slot_mapping ? (bf16_t*)v_cache : nullptr, slot_mapping, eps, pairing, key_runs};
+    fz.run_is_entry = merge ? 0 : 1;
     hipStream_t s = (hipStream_t)stream;
     int rc = -1;
 #define TFF_ATTN_CASE(DTV)                                                                          \

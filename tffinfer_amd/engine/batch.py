@@ -197,7 +197,7 @@ def build_step_batch(entries, cache, device, pinned: PinnedTables | None = None)
         sections.append(sm)
         # a step of one token per request: the requests' keys dealt into runs for the attention
         if b.max_new_tokens == 1:
-            dealt = deal_key_runs(start, g.spec.window, g.spec.num_kv_heads)
+            dealt = deal_key_runs(start, g.spec.window, g.spec.num_kv_heads, short=g.spec.short_runs)
             sections.append(dealt.runs.reshape(-1))
             sections.append(dealt.run_start)
             group_meta[-1] += (dealt.blocks, dealt.merge)

@@ -199,7 +199,9 @@ class DecodeTables:
         for gi, g in enumerate(self.cache.groups):
             dealt = deal_key_runs(positions, g.spec.window, g.spec.num_kv_heads,
                                   runs_out=hv[o[11 + 4 * gi]:o[11 + 4 * gi] + 4 * self.run_caps[gi]],
-                                  start_out=hv[o[12 + 4 * gi]:o[12 + 4 * gi] + B + 1], live=live)
+                                  start_out=hv[o[12 + 4 * gi]:o[12 + 4 * gi] + B + 1], live=live,
+                                  # (a variant merges in all groups or in none, and short rows are a block's only where none are merged)
+                                  short=g.spec.short_runs and len(self.cache.groups) == 1)
             merge = merge or dealt.merge        # some row's keys are several runs, in some group
             blocks.append(dealt.blocks)
         #: what the last fill's dealing found: the variant of the captured step that fits these tables

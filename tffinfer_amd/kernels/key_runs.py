@@ -23,7 +23,8 @@ of a block a CU, or of two), and requests of about one length (the longest no
 more than some two times the average, see BLOCK_RATE_SHARE), a block of eight
 waves per request and kv head, which merges its waves' results in LDS, is
 faster than single waves whose results a second kernel merges: every request
-is one run then, and ``blocks`` says so.  A CU holds one such block, and a
+is one run then, and ``blocks`` says so.  So it is for a few short requests (SHORT_STEPS), and whenever rows that are
+a run each have a CU for every pair; the launch sees to that.  A CU holds one such block, and a
 block is as slow as its request is long, so uneven lengths go to single waves.
 
 Pure host code (numpy).  The reference has one sequence per forward and no such
@@ -55,6 +56,10 @@ BLOCK_PAIRS = ((160, 256), (448, 512))
 #: longest request has no more than pairs / 111 times the average's keys (per round of blocks)
 BLOCK_RATE_SHARE = 111
 CUS = 256
+#: with no more pairs of row and kv head than CUs, rows of up to so many steps stay a run each: a pair's eight waves, up to three or
+#: four steps each, and no second kernel (us a layer, 8 kv heads, in runs / in one: one row of 250 keys 12.0 / 8.4, of 500 12.2 / 9.0,
+#: of 760 12.1 / 11.3, of 1,000 12.3 / 14.7; eight rows of 500 13.9 / 10.8, sixteen of 760 19.7 / 15.1)
+SHORT_STEPS = 24
 
 
 class KeyRuns(NamedTuple):
@@ -79,13 +84,14 @@ def max_key_runs(rows: int, waves_per_run: int) -> int:
 
 def deal_key_runs(positions, window: int, waves_per_run: int, runs_out: np.ndarray | None = None,
                   start_out: np.ndarray | None = None, blocks: bool | None = None,
-                  target: int | None = None, min_steps: int | None = None, live: int | None = None) -> KeyRuns:
+                  target: int | None = None, min_steps: int | None = None, live: int | None = None, short: bool = False) -> KeyRuns:
     """``positions`` [R]: the position of each request's one new token (as many tokens are cached
     before it); ``window`` > 0: a token sees only the last ``window`` keys, itself included;
     ``waves_per_run``: waves (or blocks) that the kernel starts per run: the kv heads.  ``blocks``:
     whether a run gets a block of eight waves (None: by the number of rows and their lengths).
     ``live``: the first so many rows are requests, the others padding (a captured step's), which
-    does not count where the requests' number and lengths decide.  ``target`` and ``min_steps``
+    does not count where the requests' number and lengths decide.  ``short``: a row that is one run gets a block of waves whatever
+    ``blocks`` says, as long as there are no more pairs than CUs (short rows then stay one run).  ``target`` and ``min_steps``
     override the number of waves (or blocks) aimed at and the shortest run (for tests).
 
     The runs of row r are ``run_start[r] .. run_start[r + 1] - 1``, in the order of their keys,
@@ -122,6 +128,9 @@ def deal_key_runs(positions, window: int, waves_per_run: int, runs_out: np.ndarr
         if target is not None:
             chunk = max(1 if min_steps is None else int(min_steps), -(-wave_steps // int(target)))
             n = -(-steps // chunk)
+    elif short and R * wps <= CUS and int(steps.max()) <= SHORT_STEPS:
+        n = np.ones(R, dtype=np.int64)
+        chunk = int(steps.max())
     else:
         typical = int(np.median(mine))
         floor = max(MIN_STEPS, min(LONG_STEPS, -(-wave_steps // BUSY_WAVES))) if min_steps is None else int(min_steps)

@@ -20,7 +20,7 @@ import numpy as np
 import torch
 
 from . import lib as _lib
-from .key_runs import deal_key_runs
+from .key_runs import CUS, deal_key_runs
 from . import staging as _staging
 
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -1150,6 +1150,8 @@ def attention_decode_fused(qkv: torch.Tensor, nq: int, nkv: int, d: int, q_weigh
             raise _lib.KernelError(f"attention_decode_fused: runs of shape {tuple(key_runs.shape)} and "
                                    f"{run_start.numel()} run starts for {R} rows")
         P = key_runs.shape[0]
+        # (rows of one run each and no more blocks than CUs: a single wave would go through its run alone beside idle ones)
+        eight = (runs_for_blocks or (not runs_merge and R * nkv <= CUS)) and d <= 128 and tiles == 1
         out = torch.empty(R, nq * d, dtype=qkv.dtype, device=qkv.device)
         part_o = torch.empty(P, nq, d, dtype=torch.float32, device=qkv.device)
         part_ml = torch.empty(P, nq, 2, dtype=torch.float32, device=qkv.device)
@@ -1157,7 +1159,7 @@ def attention_decode_fused(qkv: torch.Tensor, nq: int, nkv: int, d: int, q_weigh
             qkv.data_ptr(), qkv.stride(0), out.data_ptr(), part_o.data_ptr(), part_ml.data_ptr(), k_cache.data_ptr(),
             v_cache.data_ptr(), bt.data_ptr(), bt.stride(0), batch.cu_tokens.data_ptr(), batch.start_pos.data_ptr(),
             _ptr(slot_mapping), _ptr(q_weight), _ptr(k_weight), float(eps), _ptr(cos_sin), max_pos, int(pairing),
-            key_runs.data_ptr(), run_start.data_ptr(), P, 8 if (runs_for_blocks and d <= 128 and tiles == 1) else 1,
+            key_runs.data_ptr(), run_start.data_ptr(), P, 8 if eight else 1,
             1 if runs_merge else 0, R, nq, nkv, d, k_cache.shape[2], k_cache.shape[0],
             int(window), float(scale), _stream()))
         return out

@@ -50,7 +50,9 @@ class GQAttention(Mixer):
         self.w_qkv = self.w_o = self.q_norm = self.k_norm = None
 
     def cache_spec(self):
-        return KVCacheSpec(self.num_kv_heads, self.head_dim, self.window)
+        p, d = self.position, self.head_dim
+        whole = p is None or (p.rotary_dim == d and (p.pairing == "interleaved" or d % 64 == 0))     # the fused decode attention takes it
+        return KVCacheSpec(self.num_kv_heads, d, self.window, short_runs=whole and d <= 128 and self.num_heads <= 16 * self.num_kv_heads)
 
     def flops_per_query_key_pair(self):
         return 4 * self.num_heads * self.head_dim      # q.k and p.v, a multiply and an add each

@@ -48,12 +48,15 @@ class KVCacheSpec:
     ``keep_first`` tokens of the request, which every later token goes on reading.
     ``pools``: block sizes in tokens, ascending; for each the cache also keeps, for good, one
     key and one value per whole block of so many tokens (what the mixer makes of the block's
-    keys and values), and holds a block's tokens until it is whole."""
+    keys and values), and holds a block's tokens until it is whole.
+    ``short_runs``: the mixer's decode attention gives a row that is one run of keys a block of waves
+    (how the keys are dealt, not what is kept: specs that differ in it alone are the same cache)."""
     num_kv_heads: int
     head_dim: int
     window: int = 0
     keep_first: int = 0
     pools: tuple = ()
+    short_runs: bool = field(default=False, compare=False)
 
     @property
     def reach(self) -> int:
