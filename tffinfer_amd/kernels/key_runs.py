@@ -136,10 +136,13 @@ def deal_key_runs(positions, window: int, waves_per_run: int, runs_out: np.ndarr
         floor = max(MIN_STEPS, min(LONG_STEPS, -(-wave_steps // BUSY_WAVES))) if min_steps is None else int(min_steps)
         share = -(-wave_steps // max(1, TARGET_WAVES if target is None else int(target)))
         if target is None and share * 5 > typical * 3:
-            # so many requests that the waves' fair share is most of a request: requests of about
-            # one length stay a run each (nothing to merge then); a request much longer than the
-            # others is cut to their measure
+            # so many requests that the waves' fair share is most of a request: requests of about one length stay a run each (nothing
+            # to merge then).  Beside requests much longer than that, which are cut and merged anyway, all are cut to the fair share, so
+            # that no wave is left alone at the end (us, 48 rows of 9 to 256 steps, median 69, share 43: cut to half as much again as the
+            # median 122.6, to the share 103.1; 45 such steps of 21 to 62 rows 0.976 on average, 0.88 to 1.03)
             chunk = max(share, -(-3 * typical // 2))
+            if int(steps.max()) > chunk:
+                chunk = share
             n = -(-steps // chunk)
         elif share >= floor:
             chunk = share
