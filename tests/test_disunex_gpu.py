@@ -162,6 +162,14 @@ def test_experts_on_whole_lines(E, top, width, ff, gate, on_input, pad, T):
     _experts_case(E, top, width, ff, gate, on_input, pad, T)
 
 
+@pytest.mark.parametrize("T", [150, 4000])
+@pytest.mark.parametrize("E,top,width,ff,gate,on_input", [(5, 2, 128, 2048, True, False), (5, 2, 256, 2048, False, True), (4, 2, 2048, 128, False, False),
+                                                          (4, 2, 2048, 256, True, False)])
+def test_experts_of_fewer_units_than_are_on_their_way(E, top, width, ff, gate, on_input, T):
+    """Two and four units of K, up and down: the copies run past K's end from the first units on, and no block goes on to another pair."""
+    _experts_case(E, top, width, ff, gate, on_input, 8, T)
+
+
 @pytest.mark.parametrize("E,top,width,ff,gate,on_input,T", [
     (5, 2, 320, 2048, False, True, 4000), (5, 2, 320, 2048, False, False, 6000), (5, 2, 320, 1792, True, False, 2200), (6, 3, 384, 1152, True, True, 2500),
     (5, 2, 2048, 320, False, True, 4000), (5, 2, 2048, 320, True, False, 6000), (4, 1, 2048, 448, False, False, 8000)])

@@ -625,13 +625,17 @@ __global__ __launch_bounds__(256) void experts_tiles_kernel(
 // chunk (i % 8) ^ (i / 8), so that an operand's sixteen rows come back from different banks), the pairs' rows through
 // the tile's list; NS units lie in LDS, two are on their way.  GATE_UP: the tile's groups of 16 weight rows are gate
 // and up in turn, so a lane holds both sums of its outputs.  k ascends in steps of 32 for every pair as above: the same bits.
-// Unit u + 2 is copied during unit u, into the slot that unit u - 1 has left: its last operands were read, and had arrived
-// (lgkmcnt 0), before the barrier in the middle of unit u - 1.  At that barrier of unit u every wave's copies of unit u + 1 have
-// landed: all but the CP / 2 copies that it issued in the first half of unit u.
+// A unit's operands have all been read, and have arrived (lgkmcnt 0), before the barrier in the middle of its work, and at once the first half of
+// the copies of the unit three behind it goes into its slot, the second half during the first half of the next unit's work.  At
+// the barrier in the middle of unit u every wave's copies of unit u + 1 have landed: all but the CP that it issued since.  So a copy has from one
+// unit's work to two to arrive in (with unit u + 2 copied during unit u, as it was, from a half to one and a half).  us a product of 32
+// experts, 4,096 x 3,072, that / this: 256 pairs an expert 233 / 224, 300 330 / 296, 384 351 / 324; 8,192 pairs of one expert, whose rows the caches
+// hold, 160 / 163.  The last unit's second half issues no copies (the results go through its slot) and stands behind the loop: with a choice
+// between the two inside it, the compiler moved accumulators about right behind MFMAs whose wait states it does not know.
 // A block that works on one pair of tile and column block spends 10 to 15 us of its 40 to 75 on what nothing overlaps: three loads that wait for
 // each other, the first units on their way, the results' way out.  So the launch has a block a CU, and a block goes on to its next
-// pair: that one's list of rows travels during the second unit of the present pair, its first two units of operands during the
-// last two, and the results leave through the third slot while they land.
+// pair: that one's list of rows travels during the first units of the present pair, its first two units of operands during the
+// last three, and the results leave through the third slot while they land.
 // us for both products, a pair a block / now: 32 experts, four a token, 4,096 x 1,536 gated, 2,048 tokens 560 / 537 (576 TFLOP/s; some 720
 // with the tiles' padding), 4,000 tokens 817 / 783; 4,096 x 3,072 without a gate, 2,919 tokens 776 / 739; 2,048 x 1,536 gated, 4,500 tokens
 // 494 / 462; 16 experts, two a token, 2,048 x 1,024, 2,000 tokens 121 / 101; 150 tokens of the first within 2 % (the weight's stream).
@@ -713,12 +717,14 @@ __global__ __launch_bounds__(256) void experts_lines_kernel(
         for (int c = 0; c < CP; ++c) EXL_COPY(c)
         EXL_ISSUED()                                  // (past the end of K the last unit once more)
     }
+#pragma unroll
+    for (int c = 0; c < CP / 2; ++c) EXL_COPY(c)
     // a lane's 16 bytes of an operand: row fr of 16, chunk h * 4 + fg of the row's 8
     unsigned rd[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) rd[h] = (unsigned)(fr >> 3) * 1024u + (unsigned)(((fr & 7) * 8 + ((h * 4 + fg) ^ (fr & 7))) * 16);
     const unsigned a_rd = (unsigned)(wm * WTM) * 2048u, w_rd = A_BYTES + (unsigned)(wn * WTN) * 2048u;
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(CP));
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(CP + CP / 2));
     __syncthreads();
     bf16x8 fw[2][WTN], fa[2][WTM];
 #pragma unroll
@@ -726,11 +732,11 @@ __global__ __launch_bounds__(256) void experts_lines_kernel(
 #pragma unroll
     for (int j = 0; j < WTM; ++j) fa[0][j] = *reinterpret_cast<const bf16x8*>(smem + a_rd + rd[0] + j * 2048);
     unsigned rs = 0;                                  // the slot that the next operands are read from
-#define EXL_TILE(h)                                                                                                 \
+#define EXL_TILE(h, COPIES)                                                                                         \
     {                                                                                                               \
         if (h) {                                                                                                    \
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                                      \
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(CP / 2));                                                          \
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(CP));                                                              \
             asm volatile("s_barrier" ::: "memory");                                                                 \
             rs = rs + UNIT == NS * UNIT ? 0u : rs + UNIT;                                                           \
         }                                                                                                           \
@@ -745,7 +751,7 @@ __global__ __launch_bounds__(256) void experts_lines_kernel(
                     if (x < WTM) fa[(h) ^ 1][x < WTM ? x : 0] = *reinterpret_cast<const bf16x8*>(na + x * 2048);    \
                     else fw[(h) ^ 1][x >= WTM ? x - WTM : 0] = *reinterpret_cast<const bf16x8*>(nw + (x - WTM) * 2048); \
                 }                                                                                                   \
-                if (q % CPM == CPM - 1 && q / CPM < CP / 2) EXL_COPY((h) * (CP / 2) + q / CPM)                      \
+                if ((COPIES) && q % CPM == CPM - 1 && q / CPM < CP / 2) EXL_COPY(((h) ^ 1) * (CP / 2) + q / CPM)     \
             }                                                                                                       \
     }
     floatx4 acc[WTN][WTM];
@@ -765,22 +771,23 @@ __global__ __launch_bounds__(256) void experts_lines_kernel(
                 asm volatile("" : "+a"(acc[i][j]));
             }
         asm volatile("s_nop 7");
-        for (int u = 0; u < nu; ++u) {
-            EXL_TILE(0)
-            EXL_TILE(1)
+        EXL_TILE(0, true)
+        EXL_ISSUED()
+        if (next >= 0) copy_list(tile, list ^ 1024u);                  // here since the barrier of unit 1
+        for (int u = 1; u < nu; ++u) {
+            EXL_TILE(1, true)
+            EXL_TILE(0, true)
             EXL_ISSUED()
-            if (next >= 0) {
-                if (u == 1) copy_list(tile, list ^ 1024u);             // here since the barrier of unit 2
-                if (u == nu - 3) {                                      // the coming copies are the next pair's
-                    const int32_t* in_list = reinterpret_cast<const int32_t*>(smem + LIST + wave * 2048 + (list ^ 1024u));
+            if (next >= 0 && u == nu - 3) {                             // the coming copies are the next pair's
+                const int32_t* in_list = reinterpret_cast<const int32_t*>(smem + LIST + wave * 2048 + (list ^ 1024u));
 #pragma unroll
-                    for (int c = 0; c < LPA; ++c) off[c] = pair_row(in_list[(wave + NW * c) * 8 + (lane >> 3)]);
-                    weight_rows();
-                    u_next = 0;
-                    k_off = 0;
-                }
+                for (int c = 0; c < LPA; ++c) off[c] = pair_row(in_list[(wave + NW * c) * 8 + (lane >> 3)]);
+                weight_rows();
+                u_next = 0;
+                k_off = 0;
             }
         }
+        EXL_TILE(1, false)                                              // (the results go through the last unit's slot)
         // The last MFMAs have written.  The unit that was worked on last has left its slot (its last operands had arrived before the barrier in
         // its middle), and the next pair's first two units are in the other two or on their way: the results go through that slot, a
         // part of it for each wave, so that its stores are whole pieces of a pair's row.
@@ -847,6 +854,8 @@ __global__ __launch_bounds__(256) void experts_lines_kernel(
         if (next < 0) break;
         asm volatile("s_barrier" ::: "memory");       // every wave has left the slot: the next unit's copies go there
         list ^= 1024u;
+#pragma unroll
+        for (int c = 0; c < CP / 2; ++c) EXL_COPY(c)
     }
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));         // the copies past the end must not outlive the block
 #undef EXL_TILE
