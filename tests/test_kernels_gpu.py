@@ -456,6 +456,53 @@ def test_cases_of_128_rows_cover_every_tile_width():
     assert {(128, False), (256, False), (384, False), (128, True), (256, True), (384, True)} <= widths, widths
 
 
+BETWEEN_CASES = [
+    # M, N, K, gated, kept sums: tiles of 192 and 96 rows, six row groups a wave (rows, columns, parts)
+    (900, 512, 1024, False, False, (96, 128, 1)),
+    (768, 512, 1088, True, False, (96, 128, 1)),      # whole tiles, an odd number of units of K
+    (600, 1536, 2048, False, False, (96, 128, 2)),
+    (600, 512, 1088, True, False, (96, 128, 2)),
+    (900, 512, 1088, False, True, (96, 128, 3)),      # parts of six and five units
+    (900, 512, 3072, False, True, (96, 128, 6)),
+    (2100, 1024, 1024, False, True, (96, 128, 1)),    # 22 tile rows
+    (1340, 3072, 1024, False, False, (192, 128, 1)),  # seven tile rows: a band and a rest
+    (700, 6144, 1024, True, False, (192, 128, 1)),
+    (700, 1536, 6144, False, False, (192, 128, 4)),
+    (1340, 1536, 2048, False, True, (192, 128, 2)),
+    (1340, 6144, 1088, False, False, (192, 192, 1)),
+    (768, 12288, 1024, True, False, (192, 192, 1)),
+    (1340, 8192, 1088, False, False, (192, 256, 1)),
+    (1344, 8192, 1088, True, False, (192, 256, 1)),
+    (1340, 4096, 6144, False, True, (192, 256, 2)),
+]
+
+
+@pytest.mark.parametrize("M,N,K,glu,keep,tile", BETWEEN_CASES)
+def test_linear_on_tiles_of_192_and_96_rows(M, N, K, glu, keep, tile):
+    """The four-wave kernel with six row groups a wave: every tile, gated or not, ragged rows, K in one part and split with the sums added
+    or handed on, a row stride beyond K."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(N + K)
+    wide = torch.randn(M, K + 72, generator=g).to(torch.bfloat16).to(DEV)
+    x = wide[:, :K].contiguous()
+    assert _gemm_plan(M, N, K, int(glu), int(keep)) == tile
+    if glu:
+        I = N // 2
+        gate = (torch.randn(I, K, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
+        up = (torch.randn(I, K, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
+        a, b = ops.linear(x.float(), gate.float()), ops.linear(x.float(), up.float())
+        ref, pw = a / (1 + torch.exp(-a)) * b, ops.pack_gate_up(gate, up)
+    else:
+        w = (torch.randn(N, K, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
+        ref, pw = ops.linear(x.float(), w.float()), ops.pack_weight(w)
+    y = ops.linear(x, pw, out_dtype=torch.float32, partials=keep)
+    if keep and tile[2] > 1:
+        assert y.dim() == 3 and y.shape[0] == tile[2]
+    _close(ops.as_tensor(y), ref, 3e-5, f"product on {tile}")
+    if not keep:
+        _close(ops.linear(wide[:, :K], pw), ref, 8e-3, "strided rows, bfloat16 result")
+
+
 FEW_ROWS_CASES = [
     # M, N, K, gated: 17 to 64 rows and K in units of 64, so tiles of 64 or 32 rows on four waves side by side
     (40, 6150, 4096, False),       # 64 x 128, K split; handed on: 64 x 256; rows of the result that are no multiple of 16 bytes

@@ -311,9 +311,9 @@ static int launch_async_g(const bf16_t* A, const bf16_t* Wp, void* C, int M, int
 }
 
 // ------------------------------------------- four waves, whole cache lines ---
-// Block tile 256 x (32 WTN) on 2 x 2 waves (or 128 x (64 WTN) on 1 x 4, for products of few rows,
+// Block tile 256 or 192 x (32 WTN) on 2 x 2 waves (or 128 or 96 x (64 WTN) on 1 x 4, for products of few rows,
 // whose time is the weight's stream: all four waves then read the same rows of A), one wave to a
-// SIMD, each wave 8 x WTN MFMA tiles: half the LDS reads per MFMA of sixteen waves of 64 x 64.  With one wave to a SIMD nothing overlaps unless
+// SIMD, each wave 8 or 6 x WTN MFMA tiles: half the LDS reads per MFMA of sixteen waves of 64 x 64.  With one wave to a SIMD nothing overlaps unless
 // the wave interleaves it itself: the fragments of k-tile t + 1 are read from LDS into a second set
 // of registers, and the copies of later tiles are issued, between the MFMAs of k-tile t.
 //
@@ -422,7 +422,7 @@ __device__ __forceinline__ void w4_store_rows(char* region, F val, TO* out, size
 // read all of A.  us before / now: 7,376 rows of 1,024 x 3,072 on tiles of 256 x 128 55 / 40,
 // 4,700 of 2,048 x 2,048 37.4 / 35.9, 16,384 of 4,096 x 12,288 1,070 / 1,041, of 24,576 x 4,096 2,198 / 2,177.)
 template <int BM>
-constexpr int w4_band() { return BM >= 256 ? 4 : 8; }
+constexpr int w4_band() { return BM >= 192 ? 4 : 8; }
 template <int BM>
 __host__ __device__ inline int w4_rows_together(int TN) {
     const int band = w4_band<BM>() * TN;
@@ -473,10 +473,10 @@ __global__ __launch_bounds__(256) void gemm_bf16_w4_kernel(
     const float* __restrict__ const bias = ex.bias;
     static_assert(!SCALE || WGM == 1, "rows that lack their norm's factor: up to 16, one row tile");
     // WGM: waves along the rows, 2 (a block tile of 256 rows, two waves side by side) or 1 (128 rows, four side by side)
-    // WTM: row groups of 16 a wave, 8, or with the waves side by side 4 or 2 (a block tile of 64 or 32 rows)
+    // WTM: row groups of 16 a wave, 8 or 6 (a block tile of 192 or 96 rows), or with the waves side by side 4 or 2 (of 64 or 32 rows)
     constexpr int NW = 4, NA = 3, WGN = NW / WGM;
     static_assert(WGM == 1 || WGM == 2, "four waves as 2 x 2 or 1 x 4");
-    static_assert(WTM == 8 || (WGM == 1 && (WTM == 4 || WTM == 2)), "fewer rows a wave only with the waves side by side");
+    static_assert(WTM == 8 || WTM == 6 || (WGM == 1 && (WTM == 4 || WTM == 2)), "few rows a wave only with the waves side by side");
     constexpr int BM = WGM * WTM * 16, BN = WGN * WTN * 16;
     constexpr int WF = BN / 16;                       // W fragments a k-tile, 1 KB each
     static_assert(WF % NW == 0, "every wave copies as many fragments of W");
@@ -827,7 +827,7 @@ static int launch_row_tiles(const bf16_t* A, const bf16_t* Wp, void* C, int M, i
 
 // The tiled product's plan for M > 16: which tile, and into how many parts the blocks of a
 // tile split K, by a small cost model (see plan_for).  With K in units of 64: the four-wave
-// kernel's tiles of 256 rows (256, 192 or 128 columns), of 128 rows (384, 256 or 128 columns) and,
+// kernel's tiles of 256 and 192 rows (256, 192 or 128 columns), of 128 (384, 256 or 128 columns) and 96 rows (128) and,
 // up to 64 and 32 rows, of 64 and 32 rows (256 or 128 columns), and from 65 to 512 rows also
 // 64 x 128 with several row tiles; otherwise the sixteen-wave kernel's tiles.
 struct GemmPlan { int tile; int bn; int splits; };   // tile = rows of a block tile
@@ -882,59 +882,83 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
     }
     const int nk = (K + 63) / 64;
     if (K % 64 == 0) {
-        // The four-wave kernel's tiles (256 rows on 2 x 2 waves, 128 rows on 1 x 4) and, up to 512 rows,
+        // The four-wave kernel's tiles (256 or 192 rows on 2 x 2 waves, 128 or 96 rows on 1 x 4) and, up to 512 rows,
         // its 64 x 128, two blocks to a CU.  A block goes through its part of K in
         // units of 64; a unit takes what its MFMAs take at the tile's rate or what its columns of W take
         // to arrive, whichever is longer: a block's share of the HBM stream, at most what one CU pulls.
         // Blocks go round the CUs; each round ends with the pipeline filled and the tile stored.  The constants are
         // fitted to products of the 0.6B to 14B shapes and of the other designs, every tile with
-        // 1 .. 8 parts timed in a graph on an MI355X (weights in turn, none of a launch's host work in the figure), in three pieces:
-        // * Results of one kernel or of the sum over the parts, more than 64 rows: 8,500 products of 65 .. 9,000 rows.  The pick is 1.2 % from the best
-        //   candidate on average (gated 0.5 %), and in 97 of 100 not 3 % slower than what the constants for a slower loop picked.  One
-        //   fit with the kept sums left K in one part where a weight's stream wants more blocks (us, that / these: 110 rows of 6,144 x 2,560
-        //   20.9 / 16.6, gated 78 rows 20.2 / 15.6, 202 of 6,144 x 4,096 29.9 / 26.0, 330 of 4,096 x 4,096 29.2 / 25.8).
-        // * Sums kept for a norm, more than 64 rows: 840 products; 1.1 % from the best with the norm behind it.
+        // 1 .. 8 parts timed on an MI355X (weights in turn that no cache holds, rows from five places), in four pieces:
+        // * Results of one kernel or of the sum over the parts, more than 64 rows: 4,234 products of 65 .. 16,500 rows.  The pick is 0.6 % from the best
+        //   candidate on average; against the tiles of 256, 128 and 64 rows alone 0.979 of the time (513 to 1,040 rows 0.949), and in 3 of 100 slower by
+        //   more than 2 %.
+        // * Sums kept for a norm, more than 64 rows, no more columns than K: 2,832 products; 0.8 % from the best with the norm behind it, 0.962 of the time of
+        //   the tiles and constants before (257 to 2,080 rows 0.943), in 7 of 100 slower by more than 2 %.
+        // * Kept sums of more columns than K, which no model's product into its stream has: constants of an older fit.
         // * Up to 64 rows the four waves side by side take 64 or 32 rows: a product of so few rows is its
         //   weight's stream, and a block that does not work through 128 rows for 32 asks for its next
         //   columns sooner (3 to 10 % less time than the tiles of 128 rows and the sixteen-wave kernel's
         //   64 x 128 on the four products of the three shapes at 17 to 64 rows; their rates fitted to
         //   those 88 cases stand for that, the pick 0.5 % from the best on average, 5 % at worst).
-        // A rate is in flops a microsecond of a CU: of results, of kept sums, up to 64 rows.  ends: us that a block's first fetch and storing its tile take.
-        struct Cand { int bm, bn, slots; double rate, rate_kept, rate_few, ends; };
-        static const Cand cands[11] = {{256, 256, 1, 7.69e6, 6.45e6, 0, 1.42}, {256, 192, 1, 7.02e6, 6.10e6, 0, 1.05}, {256, 128, 1, 6.13e6, 5.42e6, 0, 0.75},
-                                       {128, 384, 1, 6.00e6, 6.49e6, 3.24e6, 1.05}, {128, 256, 1, 5.97e6, 5.38e6, 4.61e6, 0.75}, {128, 128, 1, 4.41e6, 3.56e6, 3.45e6, 0.56},
-                                       {64, 256, 1, 0, 0, 2.4e6, 0}, {64, 128, 1, 0, 0, 2.0e6, 0}, {32, 256, 1, 0, 0, 1.4e6, 0}, {32, 128, 1, 0, 0, 1.3e6, 0},
-                                       {64, 128, 2, 2.72e6, 2.48e6, 0, 0.50}};
-        const bool few = M <= 64, kept = keep && !few;
+        // Tiles of 192 and 96 rows are finer steps between the others: blocks that fill the CUs, or less padding.  They take K from 1,024 on and whole
+        // columns of tiles, which the products they are fitted to have; not one row tile of few rows, whose time is the weight's stream (161 rows of 34,816 x 5,120
+        // gated 91 on 256 x 192, 101 on 192 x 256); up to 384 rows only where they pad less than tiles of 128, if
+        // the sums are not kept; and beyond 2,048 rows K in one part (2,210 of 4,096 x 18,432 257 on 256 x 192, 335 on 192 x 128 in two).
+        // From 1,500 rows on they have to be 2 % ahead: large products are bound by the power the card allows, of which a smaller tile's reads take more
+        // (slower than the tiles before by more than 2 %: 4 of 100 such products without this margin, 0.3 with it).
+        // Three and six parts are for kept sums of 129 to 1,024 rows: beyond, the parts' traffic grows and the rounds are many.
+        // A rate is in flops a microsecond of a CU; ends: us that a block's first fetch and storing its tile take.  Of results, of kept sums, of the older
+        // fit's, up to 64 rows.
+        struct Cand { int bm, bn, slots; double rate, ends, rate_kept, ends_kept, rate_wide, rate_few; };
+        static const Cand cands[15] = {
+            {256, 256, 1, 8.43e6, 1.02, 8.12e6, 1.77, 6.45e6, 0}, {256, 192, 1, 7.65e6, 1.04, 7.50e6, 1.10, 6.10e6, 0},
+            {256, 128, 1, 6.20e6, 0.95, 5.75e6, 1.38, 5.42e6, 0}, {192, 256, 1, 7.80e6, 1.14, 7.63e6, 2.20, 0, 0},
+            {192, 192, 1, 5.90e6, 0.77, 4.48e6, 0.45, 0, 0}, {192, 128, 1, 4.70e6, 0.66, 5.59e6, 0.65, 0, 0},
+            {128, 384, 1, 10.6e6, 1.76, 4.13e6, 1.55, 6.49e6, 3.24e6}, {128, 256, 1, 6.18e6, 0.96, 5.95e6, 0.73, 5.38e6, 4.61e6},
+            {128, 128, 1, 4.41e6, 0.61, 5.04e6, 0.65, 3.56e6, 3.45e6}, {96, 128, 1, 3.71e6, 0.84, 4.30e6, 0.19, 0, 0},
+            {64, 256, 1, 0, 0, 0, 0, 0, 2.4e6}, {64, 128, 1, 0, 0, 0, 0, 0, 2.0e6},
+            {32, 256, 1, 0, 0, 0, 0, 0, 1.4e6}, {32, 128, 1, 0, 0, 0, 0, 0, 1.3e6}, {64, 128, 2, 2.67e6, 0.12, 3.95e6, 0.32, 2.48e6, 0}};
+        const bool few = M <= 64, wide = keep && !few && N > K, kept = keep && !few && !wide;
         // bytes a microsecond of all CUs together and of one alone
-        const double HBM = few ? 7.72e6 : kept ? 8.18e6 : 14.65e6, CU_MAX = few ? 6.0e4 : kept ? 6.54e4 : 5.57e4;
+        const double HBM = few ? 7.72e6 : wide ? 8.18e6 : kept ? 31.57e6 : 9.41e6, CU_MAX = few ? 6.0e4 : wide ? 6.54e4 : kept ? 5.79e4 : 6.04e4;
         GemmPlan best = {128, 128, 1};
         double best_t = 1e30;
         for (const Cand& c : cands) {
+            const bool between = c.bm == 192 || c.bm == 96;
             if (c.bm == 256 && M <= 64) continue;
+            if (between) {
+                if (few || wide || unary || K < 1024 || N % c.bn || M <= (c.bm == 192 ? 192 : 128)) continue;
+                if (!kept && M <= 384 && (M + c.bm - 1) / c.bm * c.bm >= (M + 127) / 128 * 128) continue;
+            }
             if (c.slots == 1 && c.bm <= 64 && M > c.bm) continue;         // (four waves side by side: one row tile)
             if (c.slots == 2 && (M <= 64 || M > 512)) continue;            // (64 x 128 with several row tiles)
             if (plane % c.bn) continue;
-            for (int S = 1; S <= (plane ? 1 : (glu && M > 64) ? 2 : 8); S *= 2) {
+            for (int S = 1; S <= (plane ? 1 : (glu && M > 64) ? 2 : 8); S += S < 4 ? 1 : 2) {
                 if (S > 1 && nk / S < 4) break;
+                if (S % 3 == 0 && !(kept && M > 128 && M <= 1024)) continue;
+                if (S > (between ? 1 : 2) && kept && M > 2048) break;
                 const double blocks = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * S;
                 const double rounds = ceil(blocks / (CUS * c.slots)), at_once = fmin(blocks, CUS * c.slots);
-                double rate = c.rate, ends = c.ends, start = 2.47, streams = ceil((double)N / c.bn) * S;   // (row tiles fetch a column tile's weight once between them)
-                double share = c.slots == 2 && blocks > CUS ? 1.79 : 1.0;       // blocks that share a CU's MFMAs, and each other's waits
-                if (few || kept) {
-                    rate = few ? c.rate_few : c.rate_kept;
+                double rate = kept ? c.rate_kept : c.rate, ends = kept ? c.ends_kept : c.ends, units = (nk + S - 1) / S;
+                double streams = ceil((double)N / c.bn) * S;              // (row tiles fetch a column tile's weight once between them)
+                double share = c.slots == 2 && blocks > CUS ? (kept ? 2.19 : 1.77) : 1.0;     // blocks that share a CU's MFMAs, and each other's waits
+                if (few || wide) {
+                    rate = few ? c.rate_few : c.rate_wide;
                     ends = few ? 3.0 : 1.29 + 2.55 * (c.bm * c.bn / 65536.0);
-                    start = 3.0;
+                    units = (double)nk / S;
                     streams = at_once;
                     share = fmin((double)c.slots, ceil(blocks / CUS));
                 }
                 const double bw = fmin(CU_MAX, HBM / fmin(at_once, streams));
                 const double unit = fmax(2.0 * c.bm * c.bn * 64.0 * share / rate, c.bn * 128.0 / bw);
-                double t = rounds * ((double)nk / S * unit + ends) + start;
+                double t = rounds * (units * unit + ends);
                 // the partial sums: written, read and added by a second kernel, or (kept) read by the
                 // consumer in place of one plane
-                if (S > 1 && keep) t += (S - 1.0) * M * N * 4.0 / (few ? 4e6 : 1.97e6);
-                else if (S > 1 || unary) t += (double)S * M * N * 4.0 / (few ? 2.54e6 : 2.12e6) + (few ? 2.7 : 3.84);
+                // (from the caches as long as they are some 32 MB)
+                const double plane_bytes = (double)M * N * 4.0;
+                if (S > 1 && keep) t += (S - 1.0) * plane_bytes / (few || (kept && S * plane_bytes <= 32e6) ? 4e6 : 1.97e6);
+                else if (S > 1 || unary) t += S * plane_bytes / (few ? 2.54e6 : 2.21e6) + (few ? 2.7 : 2.09);
+                if (between && M >= 1500) t *= 1.02;
                 if (t < best_t) { best_t = t; best = {c.bm, c.bn, S}; }
             }
         }
@@ -1019,9 +1043,9 @@ static int launch_far(const GemmPlan& plan, const bf16_t* A, const bf16_t* Wp, v
                       int n_out, hipStream_t s, float* part, bool reduce) {
     TFF_REQUIRE((size_t)15 * lda * 2 + 128 < (1ull << 32), "gemm: row stride %d too large", lda);
     if (plan.tile <= 64) return launch_async_g<2, 2, 2, 4, 3, GLU>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
-    if (plan.tile == 128 && plan.bn == 128)
+    if (plan.tile <= 128 && plan.bn == 128)
         return launch_async_g<2, 2, 4, 4, 3, GLU>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
-    if (plan.tile == 128) return launch_async_g<2, 4, 4, 4, 3, GLU>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
+    if (plan.tile <= 128) return launch_async_g<2, 4, 4, 4, 3, GLU>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
     return launch_async_g<4, 4, 4, 4, 5, GLU, 1, true>(A, Wp, C, M, N, K, lda, ex, c_dtype, n_out, s, plan.splits, part, reduce);
 }
 
@@ -1048,6 +1072,12 @@ static int run_plan(const GemmPlan& plan, int planned_splits, bool far, const bf
                 if (plan.bn == 256) return launch_w4<4, 5, true, 1>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
                 return launch_w4<6, 4, true, 1>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
             }
+            if (plan.tile == 192) {
+                if (plan.bn == 128) return launch_w4<4, 5, true, 2, false, 6>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
+                if (plan.bn == 192) return launch_w4<6, 5, true, 2, false, 6>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
+                return launch_w4<8, 5, true, 2, false, 6>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
+            }
+            if (plan.tile == 96) return launch_w4<2, 5, true, 1, false, 6>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
             if (plan.bn == 128) return launch_w4<4, 5, true>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
             if (plan.bn == 192) return launch_w4<6, 5, true>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
             return launch_w4<8, 4, true>(A, Wp, C, M, N, K, lda, ex, c_dtype, glu_out, s, S, workspace);
@@ -1082,6 +1112,12 @@ static int run_plan(const GemmPlan& plan, int planned_splits, bool far, const bf
             if (plan.bn == 256) return launch_w4<4, 5, false, 1>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
             return launch_w4<6, 4, false, 1>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
         }
+        if (plan.tile == 192) {
+            if (plan.bn == 128) return launch_w4<4, 5, false, 2, false, 6>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
+            if (plan.bn == 192) return launch_w4<6, 5, false, 2, false, 6>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
+            return launch_w4<8, 5, false, 2, false, 6>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
+        }
+        if (plan.tile == 96) return launch_w4<2, 5, false, 1, false, 6>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
         if (plan.bn == 128) return launch_w4<4, 5>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
         if (plan.bn == 192) return launch_w4<6, 5>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
         return launch_w4<8, 4>(A, Wp, C, M, N, K, lda, ex, c_dtype, 0, s, S, workspace, red);
