@@ -564,3 +564,29 @@ def test_forty_requests_decode_together(disunex_dirs, dtype):
             assert rel_err(row, ref[len(r.prompt) + i - 1]) <= tol(dtype, d), f"request {r.prompt}: output {i}"
             checked += 1
     assert checked > 200
+
+
+@pytest.mark.parametrize("E,I,top,width,ff,T", [(8, 0, 2, 264, 136, 1), (8, 2, 3, 72, 64, 2), (12, 3, 5, 1032, 512, 3), (40, 8, 9, 520, 1032, 1),
+                                                (6, 0, 4, 4096, 1536, 1), (16, 0, 2, 2048, 1024, 2)])
+def test_few_pairs_have_the_bits_of_many(E, I, top, width, ff, T):
+    """Up to 4,096 results a token's experts are dealt to waves of their own, and few gated outputs to more waves: the same bits as the same
+    tokens among many, by an odd number of experts, more than the waves, and with some that hand their input on."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(E + ff)
+    h = torch.randn(T, width, generator=g).bfloat16()
+    mats = [(torch.randn(E, *s, generator=g) * 0.1).bfloat16() for s in ((ff, width), (ff, width), (width, ff))]
+    idx = torch.stack([torch.randperm(E + I, generator=g)[:top] for _ in range(T)]).to(torch.int32)
+    wts = torch.rand(T, top, generator=g)
+    many = max(4097 // (T * width), 18433 // (T * top * ff)) + 1
+    dev = [m.to(DEV) for m in mats]
+    run = lambda n: ops.as_tensor(ops.routed_experts(h.repeat(n, 1).to(DEV), *dev, idx.repeat(n, 1).to(DEV), wts.repeat(n, 1).to(DEV), 0.8, 1.702,   # noqa: E731
+                                                     identity=I, by_tiles=False))
+    few = run(1)
+    assert T * width <= 4096 < many * T * width and many * T * top * ff > 18432
+    assert torch.equal(few.repeat(many, 1), run(many))
+    ref = torch.zeros(T, width, dtype=torch.float64)
+    for t in range(T):
+        for k, e in enumerate(idx[t].tolist()):
+            x = h[t].double()
+            ref[t] += wts[t, k].double() * (plain.expert(x, *(m[e].double() for m in mats), 0.8) if e < E else x)
+    assert _err(few, ref) < 1.5e-2

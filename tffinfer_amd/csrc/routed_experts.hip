@@ -225,6 +225,11 @@ TFF_API int tff_route_by_table(const int32_t* table, const int32_t* ids, int T, 
 
 #define EX_WAVES 4
 #define EX_PER_WAVE 4      // outputs a wave works through
+// Few pairs leave the SIMDs with a wave or two: then a wave takes half as many gated outputs, and a token's experts are dealt to waves of their own
+// (experts_down_shared_kernel).  us, one token, four experts of 4,096 x 1,536 19.1 + 12.7 / 17.5 + 10.6, two of 2,048 x 1,024 6.6 + 5.4 / 5.3 + 4.7,
+// two tokens of the latter 8.0 + 6.2 / 7.2 + 5.6; three tokens of the former 48.2 + 24.7 / 45.4 + 26.4, four 61.7 + 31.8 / 61.1 + 34.0.
+#define EX_FEW_OUTPUTS 18432      // gated outputs up to which it is so
+#define EX_FEW_DOWN 4096          // results
 
 // What bounds a step of one token is how many loads are in flight: a wave asks for two pieces of four weight rows at a time (two
 // outputs' gate and up rows, or four outputs' down rows).  A row after the other on waves of eight outputs, one token of four
@@ -234,7 +239,7 @@ template <typename T>
 __global__ __launch_bounds__(64 * EX_WAVES) void experts_gate_up_kernel(
     const T* __restrict__ h, int h_row, const T* __restrict__ Wg, const T* __restrict__ Wu,
     const int32_t* __restrict__ idx, int top, int width, int ff, int ldw, float limit, float act_alpha, float up_offset,
-    const float* __restrict__ in_wts, T* __restrict__ y, int E) {
+    const float* __restrict__ in_wts, T* __restrict__ y, int E, int per_wave) {
     // Wg null: experts without a gate, y = max(Wu h, 0)^2.  in_wts: the pair's weight multiplies what goes into the
     // expert, W (w h) = w (W h): both products times w before clamps and activation.
     const int pair = blockIdx.x;                  // token * top + k
@@ -248,7 +253,7 @@ __global__ __launch_bounds__(64 * EX_WAVES) void experts_gate_up_kernel(
     const bool vec = sizeof(T) == 2 && width % 8 == 0 && ldw % 8 == 0 && h_row % 8 == 0 && ((uintptr_t)h % 16) == 0 &&
                      ((uintptr_t)Wg % 16) == 0 && ((uintptr_t)Wu % 16) == 0;
     const float win = in_wts ? in_wts[pair] : 1.0f;
-    const int f0 = (blockIdx.y * EX_WAVES + wv) * EX_PER_WAVE, f1 = min(ff, f0 + EX_PER_WAVE);
+    const int f0 = (blockIdx.y * EX_WAVES + wv) * per_wave, f1 = min(ff, f0 + per_wave);
     auto finish = [&](int f, float g, float u) {
         u *= win;
         if (!wg) {
@@ -341,6 +346,60 @@ __global__ __launch_bounds__(64 * EX_WAVES) void experts_down_kernel(
     }
 }
 
+// The same with a wave for every expert of a token: SHARE waves take the experts of the same four outputs in turn, and the first of them adds
+// their sums up, in the order of k as above.
+template <int SHARE>
+__global__ __launch_bounds__(64 * EX_WAVES * SHARE) void experts_down_shared_kernel(
+    const bf16_t* __restrict__ y, const bf16_t* __restrict__ Wd, const int32_t* __restrict__ idx, const float* __restrict__ wts,
+    int top, int width, int ff, int ldw, float* __restrict__ out, int E, const bf16_t* __restrict__ h, int h_row) {
+    __shared__ float4 sums[SHARE][EX_WAVES];
+    __shared__ float weights[SHARE][EX_WAVES];
+    const int t = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = wave % EX_WAVES, share = wave / EX_WAVES;
+    const int n = (blockIdx.y * EX_WAVES + g) * 4;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < top; k0 += SHARE) {
+        const int k = k0 + share;
+        if (k < top && n < width) {
+            const int e = idx[(size_t)t * top + k];
+            const float w = wts ? wts[(size_t)t * top + k] : 1.0f;
+            float d[4];
+            if (e >= E) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[i] = to_f32(h[(size_t)t * h_row + min(n + i, width - 1)]);
+            } else {
+                const bf16_t* const wd = Wd + (size_t)e * width * ldw;
+                const bf16_t* const rows[4] = {wd + (size_t)n * ldw, wd + (size_t)min(n + 1, width - 1) * ldw,
+                                               wd + (size_t)min(n + 2, width - 1) * ldw, wd + (size_t)min(n + 3, width - 1) * ldw};
+                wave_dots8<4, 2>(y + ((size_t)t * top + k) * ff, rows, ff, lane, d);
+            }
+            if (lane == 0) {
+                sums[share][g] = make_float4(d[0], d[1], d[2], d[3]);
+                weights[share][g] = w;
+            }
+        }
+        __syncthreads();
+        if (share == 0) {
+            const int here = min(SHARE, top - k0);
+#pragma unroll
+            for (int s = 0; s < SHARE; ++s)
+                if (s < here) {
+                    const float4 d = sums[s][g];
+                    const float w = weights[s][g];
+                    acc[0] = fmaf(w, d.x, acc[0]), acc[1] = fmaf(w, d.y, acc[1]);
+                    acc[2] = fmaf(w, d.z, acc[2]), acc[3] = fmaf(w, d.w, acc[3]);
+                }
+        }
+        if (k0 + SHARE < top) __syncthreads();
+    }
+    if (share == 0 && lane == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (n + i < width) out[(size_t)t * width + n + i] = acc[i];
+    }
+}
+
 TFF_API int tff_experts_gate_up(const void* h, int h_row, const void* Wg, const void* Wu, const int32_t* idx, int T,
                                 int top, int E, int width, int ff, int ldw, float limit, float act_alpha, float up_offset,
                                 const float* in_wts, void* y,
@@ -350,15 +409,16 @@ TFF_API int tff_experts_gate_up(const void* h, int h_row, const void* Wg, const 
                 "experts_gate_up: bad sizes T=%d top=%d width=%d ff=%d", T, top, width, ff);
     if (T == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid(T * top, (ff + EX_WAVES * EX_PER_WAVE - 1) / (EX_WAVES * EX_PER_WAVE));
+    const int per_wave = Wg && (long)T * top * ff <= EX_FEW_OUTPUTS ? EX_PER_WAVE / 2 : EX_PER_WAVE;
+    const dim3 grid(T * top, (ff + EX_WAVES * per_wave - 1) / (EX_WAVES * per_wave));
     TFF_REQUIRE(grid.y <= 65535, "experts_gate_up: too many outputs");
     if (dtype == TFF_F32)
         experts_gate_up_kernel<float><<<grid, 64 * EX_WAVES, 0, s>>>((const float*)h, h_row, (const float*)Wg, (const float*)Wu,
-                                                                    idx, top, width, ff, ldw, limit, act_alpha, up_offset, in_wts, (float*)y, E);
+                                                                    idx, top, width, ff, ldw, limit, act_alpha, up_offset, in_wts, (float*)y, E, per_wave);
     else if (dtype == TFF_BF16)
         experts_gate_up_kernel<bf16_t><<<grid, 64 * EX_WAVES, 0, s>>>((const bf16_t*)h, h_row, (const bf16_t*)Wg,
                                                                      (const bf16_t*)Wu, idx, top, width, ff, ldw, limit,
-                                                                     act_alpha, up_offset, in_wts, (bf16_t*)y, E);
+                                                                     act_alpha, up_offset, in_wts, (bf16_t*)y, E, per_wave);
     else
         return tff_fail("experts_gate_up: unknown dtype %d", dtype);
     return tff_check_launch("experts_gate_up");
@@ -378,7 +438,12 @@ TFF_API int tff_experts_down(const void* y, const void* Wd, const int32_t* idx, 
     TFF_REQUIRE(grid.y <= 65535, "experts_down: too many outputs");
     if (dtype == TFF_F32)
         experts_down_kernel<float><<<grid, 64 * EX_WAVES, 0, s>>>((const float*)y, (const float*)Wd, idx, wts, top, width, ff, ldw, out, E, (const float*)h, h_row);
-    else if (dtype == TFF_BF16)
+    else if (dtype == TFF_BF16 && top > 1 && (long)T * width <= EX_FEW_DOWN && ff % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)y % 16) == 0 && ((uintptr_t)Wd % 16) == 0) {
+        if (top > 2)
+            experts_down_shared_kernel<4><<<grid, 64 * EX_WAVES * 4, 0, s>>>((const bf16_t*)y, (const bf16_t*)Wd, idx, wts, top, width, ff, ldw, out, E, (const bf16_t*)h, h_row);
+        else
+            experts_down_shared_kernel<2><<<grid, 64 * EX_WAVES * 2, 0, s>>>((const bf16_t*)y, (const bf16_t*)Wd, idx, wts, top, width, ff, ldw, out, E, (const bf16_t*)h, h_row);
+    } else if (dtype == TFF_BF16)
         experts_down_kernel<bf16_t><<<grid, 64 * EX_WAVES, 0, s>>>((const bf16_t*)y, (const bf16_t*)Wd, idx, wts, top, width, ff, ldw, out, E, (const bf16_t*)h, h_row);
     else
         return tff_fail("experts_down: unknown dtype %d", dtype);
