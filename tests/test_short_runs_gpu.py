@@ -46,3 +46,29 @@ def test_short_rows_on_a_block_of_waves(nq, nkv, d, ps, window):
             assert torch.equal(kv.k_cache[page, :, at].cpu(), k_new[r]) and torch.equal(kv.v_cache[page, :, :, at].cpu(), v_new[r]), r
     same = ops.attention_decode_fused(qkv.to(DEV), nq, nkv, d, None, None, 1e-6, None, 0, kv, batch, window, scale)
     _close(out.reshape(R, nq, d)[live], same.reshape(R, nq, d).double().cpu()[live], ATTN_TOL, "against keys split alike")
+
+
+@pytest.mark.parametrize("nq,nkv,d,R", [(16, 8, 128, 13), (8, 2, 32, 24), (6, 3, 256, 9), (32, 32, 64, 11)])
+def test_rows_of_one_run_each_in_any_order(nq, nkv, d, R):
+    """A run's own number says whose it is: runs in another order than the rows', with runs that are not in use in front, between and behind,
+    give the bits of runs in order.  Blocks of eight waves and (more pairs than CUs, heads of 256) single waves."""
+    ops = _ops()
+    ps = 16
+    lengths = [(97 * r + 5) % 700 for r in range(R)]
+    batch, kv, _, _, _, _ = _fake_step([(P, 1) for P in lengths], ps, nkv, d, torch.bfloat16, seed=R)
+    qkv = torch.randn(R, (nq + 2 * nkv) * d, generator=torch.Generator().manual_seed(R)).to(torch.bfloat16).to(DEV)
+    bt = kv.block_tables.cpu()
+    slots = torch.tensor([int(bt[r, P // ps]) * ps + P % ps for r, P in enumerate(lengths)], dtype=torch.int32, device=DEV)
+    start = torch.arange(R + 1, dtype=torch.int32, device=DEV)
+    order = np.random.default_rng(R).permutation(R)
+
+    def run(rows_at):
+        runs = np.full((64, 4), -1, dtype=np.int32)
+        for at, r in rows_at:
+            runs[at] = (r, 0, lengths[r] + 1, lengths[r])
+        return ops.attention_decode_fused(qkv, nq, nkv, d, None, None, 1e-6, None, 0, kv, batch, 0, 1 / math.sqrt(d), slot_mapping=slots,
+                                          key_runs=torch.from_numpy(runs).to(DEV), run_start=start, runs_for_blocks=False, runs_merge=False)
+
+    want = run([(r, r) for r in range(R)])
+    assert torch.equal(run([(i, int(r)) for i, r in enumerate(order)]), want)
+    assert torch.equal(run([(2 * i + 1 + (i > 4) * 9, int(r)) for i, r in enumerate(order)]), want)

@@ -90,8 +90,9 @@ struct AttnFuse {
     const int32_t* pool_tables;
     int pt_stride;
     int pool;
-    // With key_runs: every entry is one run, run r entry r's, and the page numbers are asked for together with the run instead of after it.
-    int run_is_entry;
+    // With key_runs: every entry is one run.  The first page numbers of entry r are asked for together with run r instead of after it; a run that
+    // turns out to be another entry's (or not in use) does not take them.
+    int one_run_each;
 };
 
 // The last block that position pos sees (-1: none).
@@ -219,19 +220,19 @@ __global__ __launch_bounds__(64 * BW, 1) void attn_wave_kernel(
     // waves with work crowded on the other half (a fifth slower at 64 entries of one run each).
     bool by_runs = false;
     if constexpr (SPLIT || (FUSED && BW > 1)) by_runs = fz.key_runs != nullptr;
+    bool early = false;
     int r, col0, g = blockIdx.y, run_index = 0, early_page = 0;
     int4 run = make_int4(0, 0, 0, 0);
     if (by_runs) {
         const int eight = blockIdx.x / (8 * nkv), within = blockIdx.x - eight * (8 * nkv);
         run_index = eight * 8 + (within & 7);
         g = within >> 3;
-        if (fz.run_is_entry) {
-            if (run_index >= T_total) return;
-            early_page = block_tables[(size_t)run_index * bt_stride + min(lane, bt_stride - 1)];
-        }
+        early = FUSED && fz.one_run_each && run_index < T_total;
+        if (early) early_page = block_tables[(size_t)run_index * bt_stride + min(lane, bt_stride - 1)];
         run = reinterpret_cast<const int4*>(fz.key_runs)[run_index];
-        r = fz.run_is_entry ? run_index : run.x;
+        r = run.x;
         if (r < 0) return;
+        early = early && r == run_index;
         col0 = blockIdx.z * 16;
     } else if (work) {
         r = work[2 * blockIdx.x];
@@ -342,7 +343,7 @@ __global__ __launch_bounds__(64 * BW, 1) void attn_wave_kernel(
     if (!POOL && s_begin < s_end) {
         pi0 = page_index(kb0 + s_begin * 32, page_size, page_shift);
         first_count = page_index(min(kmax, kb0 + min(s_end, s_begin + seg_steps) * 32 - 1), page_size, page_shift) - pi0 + 1;
-        if (FUSED && by_runs && fz.run_is_entry && pi0 + first_count <= 64) {     // (the entry's first pages are here already)
+        if (FUSED && early && pi0 + first_count <= 64) {     // (the entry's first pages are here already)
             first_count += pi0;
             pi0 = 0;
             first_page = early_page;
@@ -1607,7 +1608,7 @@ TFF_API int tff_attention_decode_runs(const void* qkv, int qkv_stride, void* out
     if (R == 0 || num_runs == 0) return 0;
     AttnFuse fz{q_weight, k_weight, cos_sin, slot_mapping ? (bf16_t*)k_cache : nullptr,
                 slot_mapping ? (bf16_t*)v_cache : nullptr, slot_mapping, eps, pairing, key_runs};
-    fz.run_is_entry = merge ? 0 : 1;
+    fz.one_run_each = merge ? 0 : 1;
     hipStream_t s = (hipStream_t)stream;
     int rc = -1;
 #define TFF_ATTN_CASE(DTV)                                                                          \
