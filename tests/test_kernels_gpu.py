@@ -2027,3 +2027,26 @@ def test_rows_set_to_zero(sizes):
     ops.zero_rows([b[i % 5:i % 5 + n] for i, (b, n) in enumerate(zip(bufs, sizes))])
     for i, (b, n) in enumerate(zip(bufs, sizes)):
         assert int((b == 0).sum()) == n and float(b[i % 5:i % 5 + n].abs().max()) == 0
+
+
+def test_results_in_bfloat16_are_stored_whole():
+    """K in no units of 64: four neighbouring results of a lane leave in one store, so that a product with half the bytes of results does not take longer
+    than one with float32 results (it took 1.5 to 2 times as long where the compiler had taken the store apart)."""
+    ops = _ops()
+    for M, N, K in ((685, 17256, 120), (1485, 10880, 96)):
+        x = torch.randn(M, K, device=DEV).bfloat16()
+        pw = ops.pack_weight(torch.randn(N, K, device=DEV).bfloat16())
+        outs = {dt: torch.empty(M, N, dtype=dt, device=DEV) for dt in (torch.float32, torch.bfloat16)}
+        best = {}
+        for _ in range(6):
+            for dt, out in outs.items():
+                ops.linear(x, pw, out_dtype=dt, out=out)
+                ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+                ev[0].record()
+                for _ in range(20):
+                    ops.linear(x, pw, out_dtype=dt, out=out)
+                ev[1].record()
+                ev[1].synchronize()
+                best[dt] = min(best.get(dt, 1e9), ev[0].elapsed_time(ev[1]) / 20)
+        assert best[torch.bfloat16] <= 1.25 * best[torch.float32], (M, N, K, best)
+        _close(outs[torch.bfloat16], outs[torch.float32], 8e-3, "the same product in bfloat16")

@@ -22,10 +22,10 @@ __device__ __forceinline__ void store4(TC* dst, const floatx4& v, int n, int N, 
         if constexpr (sizeof(TC) == 4) {
             *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
         } else {
-            union { bf16_t h[4]; uint2 u; } pk;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) pk.h[e] = (bf16_t)v[e];
-            *reinterpret_cast<uint2*>(dst) = pk.u;
+            // (one value of four, not four put together in memory: the compiler took those apart, and joined the last number's store with the one
+            // below, three stores of a lane for one; 685 rows of 17,256 x 120 27.8 us that way, 14.6 this way)
+            typedef __attribute__((__vector_size__(4 * sizeof(bf16_t)))) __bf16 bf16x4;
+            *reinterpret_cast<bf16x4*>(dst) = bf16x4{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
         }
     } else {
 #pragma unroll
