@@ -11,6 +11,12 @@ from tffinfer_amd.kernels.key_runs import (BLOCK_PAIRS, BUSY_WAVES, KEY_STEP, LO
                                           TARGET_WAVES, deal_key_runs, max_key_runs, wants_blocks)
 
 
+def run_lengths(runs, start):
+    """Steps of keys of each run in use."""
+    used = np.asarray(runs)[:int(start[-1])]
+    return (used[:, 2] - used[:, 1] + KEY_STEP - 1) // KEY_STEP
+
+
 def check_runs(runs, start, positions, window):
     runs, start = np.asarray(runs), np.asarray(start)
     R = len(positions)
@@ -140,3 +146,38 @@ def test_short_rows_stay_a_run_each_where_a_block_of_waves_takes_one():
         a, b = deal_key_runs(pos, 0, nkv, short=True), deal_key_runs(pos, 0, nkv)
         assert np.array_equal(a.run_start, b.run_start) and np.array_equal(a.runs[:a.run_start[-1]], b.runs[:b.run_start[-1]])
         assert a.merge == b.merge and a.blocks == b.blocks
+
+
+def test_rows_of_many_pairs_stay_a_run_each_half_as_long_again():
+    from tffinfer_amd.kernels.key_runs import SHORT_PAIRS, SHORT_STEPS, SHORT_STEPS_MANY
+    longest = SHORT_STEPS_MANY * KEY_STEP - 1
+    assert SHORT_STEPS_MANY > SHORT_STEPS
+    for R, one_each in ((SHORT_PAIRS // 8, True), (SHORT_PAIRS // 8 - 1, False)):
+        pos = [longest] + [(61 * i) % longest for i in range(1, R)]
+        dealt = deal_key_runs(pos, 0, 8, short=True)
+        check_runs(dealt.runs, dealt.run_start, pos, 0)
+        assert (dealt.run_start[-1] == R and not dealt.merge) == one_each
+
+
+@pytest.mark.parametrize("short,rows,long,longs", [(90, 20, 1900, 1), (95, 40, 320, 3), (59, 30, 4000, 1), (200, 30, 4000, 2), (300, 40, 2000, 3)])
+def test_short_rows_beside_a_few_long_ones_stay_a_run_each(short, rows, long, longs):
+    """Where the waves' fair share of the keys is a few steps, only the long rows are cut, to half as much again as the short ones have."""
+    pos = [short] * rows + [long] * longs
+    dealt = deal_key_runs(pos, 0, 8)
+    check_runs(dealt.runs, dealt.run_start, pos, 0)
+    n = np.diff(dealt.run_start)
+    assert np.all(n[:rows] == 1) and np.all(n[rows:] > 1)
+    length = run_lengths(dealt.runs, dealt.run_start)
+    measure = -(-3 * (short // KEY_STEP + 1) // 2)
+    assert length.max() <= measure and np.all(n[rows:] == -(-(long // KEY_STEP + 1) // measure))
+
+
+@pytest.mark.parametrize("short,rows,long,longs", [(900, 30, 6000, 2), (700, 24, 2300, 10)])
+def test_rows_are_cut_to_the_fair_share_where_it_is_long(short, rows, long, longs):
+    """A share of FAIR_STEPS steps, or of FAIR_STEPS_MANY with many rows above their measure: no run is longer than the share."""
+    pos = [short] * rows + [long] * longs
+    dealt = deal_key_runs(pos, 0, 8)
+    check_runs(dealt.runs, dealt.run_start, pos, 0)
+    share = -(-sum(p // KEY_STEP + 1 for p in pos) * 8 // TARGET_WAVES)
+    length = run_lengths(dealt.runs, dealt.run_start)
+    assert length.max() <= share and np.all(np.diff(dealt.run_start)[:rows] > 1)

@@ -15,16 +15,18 @@ How many runs: the kernel's waves fill a SIMD's registers alone, so the GPU
 holds RESIDENT_WAVES of them at once, and a wave that streams alone is bound by
 latency, not by bandwidth.  Measured on decode steps of 1 to 128 requests: some
 TARGET_WAVES waves, none beyond what is resident, runs of LONG_STEPS steps and
-more as long as BUSY_WAVES waves have work, never under MIN_STEPS; with so many
-requests that the waves' fair share is most of a request, a run a request.
+more as long as BUSY_WAVES waves have work, never cut under MIN_STEPS; with so
+many requests that the waves' fair share is most of a request, a run a request,
+and a request much longer than the others cut to their measure, or, where many
+are longer, all cut to the fair share.
 
 With as many pairs of request and kv head as BLOCK_PAIRS says (most of a round
 of a block a CU, or of two), and requests of about one length (the longest no
 more than some two times the average, see BLOCK_RATE_SHARE), a block of eight
 waves per request and kv head, which merges its waves' results in LDS, is
 faster than single waves whose results a second kernel merges: every request
-is one run then, and ``blocks`` says so.  So it is for a few short requests (SHORT_STEPS), and whenever rows that are
-a run each have a CU for every pair; the launch sees to that.  A CU holds one such block, and a
+is one run then, and ``blocks`` says so.  So it is for a few short requests (SHORT_STEPS, SHORT_STEPS_MANY), and whenever rows
+that are a run each have a CU for every pair; the launch sees to that.  A CU holds one such block, and a
 block is as slow as its request is long, so uneven lengths go to single waves.
 
 Pure host code (numpy).  The reference has one sequence per forward and no such
@@ -43,7 +45,8 @@ KEY_STEP = 32
 RESIDENT_WAVES = 1024
 #: waves a launch aims at when single waves take the runs
 TARGET_WAVES = 768
-#: no run is shorter than this many steps of keys (a request that has fewer is one run) ...
+#: no request is cut into runs shorter than this many steps of keys (one that has fewer is one run; beside many short
+#: requests a longer one is cut to half as much again as they have, whatever that is) ...
 MIN_STEPS = 4
 #: ... nor shorter than this many while as many waves as BUSY_WAVES are left with work
 LONG_STEPS = 8
@@ -56,10 +59,20 @@ BLOCK_PAIRS = ((160, 256), (448, 512))
 #: longest request has no more than pairs / 111 times the average's keys (per round of blocks)
 BLOCK_RATE_SHARE = 111
 CUS = 256
-#: with no more pairs of row and kv head than CUs, rows of up to so many steps stay a run each: a pair's eight waves, up to three or
-#: four steps each, and no second kernel (us a layer, 8 kv heads, in runs / in one: one row of 250 keys 12.0 / 8.4, of 500 12.2 / 9.0,
-#: of 760 12.1 / 11.3, of 1,000 12.3 / 14.7; eight rows of 500 13.9 / 10.8, sixteen of 760 19.7 / 15.1)
-SHORT_STEPS = 24
+#: with no more pairs of row and kv head than CUs, rows of up to so many steps stay a run each: a pair's eight waves, up to two or three
+#: steps each, and no second kernel; with as many pairs as SHORT_PAIRS, whose runs would be many waves, rows a quarter longer as well.
+#: In one run / in several, us a layer, 8 kv heads, keys that the L2 does not hold: one row of 250 keys 8.1 / 12.4, of 500 11.2 / 12.5, of 760 14.9 / 12.5.
+#: A time over the other: three to eight rows of 500 keys 0.83 to 0.93, of 600 1.0 to 1.1, of 760 1.1 to 1.3; 16 rows of 600 0.89, 24 rows of 111 to 754 1.13
+SHORT_STEPS = 16
+SHORT_STEPS_MANY = 20
+SHORT_PAIRS = 96
+#: rows longer than their measure are cut to the waves' fair share, and all others with them, from a fair share of FAIR_STEPS steps on, or of
+#: FAIR_STEPS_MANY where at least one row in FAIR_ROWS is longer (and merged anyway): a time of cutting to the share over cutting to the measure, by the
+#: share and the rows that are longer, on 5,100 steps of 2 to 64 rows: under 8 steps 1.04 to 1.09 (20 rows of 90 keys beside one of 1,900: 17.9 us, 14.7),
+#: 8 to 12 0.95 to 1.03, 12 to 20 0.97 (more than a fifth of the rows) and 1.02 (fewer), 20 and more 0.94 to 0.97
+FAIR_STEPS = 20
+FAIR_STEPS_MANY = 12
+FAIR_ROWS = 5
 
 
 class KeyRuns(NamedTuple):
@@ -128,7 +141,7 @@ def deal_key_runs(positions, window: int, waves_per_run: int, runs_out: np.ndarr
         if target is not None:
             chunk = max(1 if min_steps is None else int(min_steps), -(-wave_steps // int(target)))
             n = -(-steps // chunk)
-    elif short and R * wps <= CUS and int(steps.max()) <= SHORT_STEPS:
+    elif short and R * wps <= CUS and int(steps.max()) <= (SHORT_STEPS if R * wps < SHORT_PAIRS else SHORT_STEPS_MANY):
         n = np.ones(R, dtype=np.int64)
         chunk = int(steps.max())
     else:
@@ -137,11 +150,12 @@ def deal_key_runs(positions, window: int, waves_per_run: int, runs_out: np.ndarr
         share = -(-wave_steps // max(1, TARGET_WAVES if target is None else int(target)))
         if target is None and share * 5 > typical * 3:
             # so many requests that the waves' fair share is most of a request: requests of about one length stay a run each (nothing
-            # to merge then).  Beside requests much longer than that, which are cut and merged anyway, all are cut to the fair share, so
-            # that no wave is left alone at the end (us, 48 rows of 9 to 256 steps, median 69, share 43: cut to half as much again as the
-            # median 122.6, to the share 103.1; 45 such steps of 21 to 62 rows 0.976 on average, 0.88 to 1.03)
+            # to merge then), and one that is much longer is cut to half as much again as they have.  Where rows are cut and merged anyway, and the
+            # share is long enough, all are cut to it, so that no wave is left alone at the end (48 rows of 9 to 256 steps, median 69,
+            # share 43: cut to half as much again as the median 122.6 us, to the share 103.1)
             chunk = max(share, -(-3 * typical // 2))
-            if int(steps.max()) > chunk:
+            longer = int(np.count_nonzero(mine > chunk))
+            if longer and (share >= FAIR_STEPS or (share >= FAIR_STEPS_MANY and longer * FAIR_ROWS >= mine.shape[0])):
                 chunk = share
             n = -(-steps // chunk)
         elif share >= floor:
