@@ -33,11 +33,18 @@
 
 // MORE: several products in one launch, or an activation of the result (GemmExtra).  Kernels of their own: the tests for them and the registers
 // of the activations cost every plain product 0.2 us.
+// Sixteen rows of a gate and its up group with one unit in flight are at the 256 registers that two waves a SIMD have, on either side of them by what the
+// epilogue takes; the compiler has to stay below (16 rows without factors, 25,728 x 2,056 with one wave a SIMD 29.6 us, with two 24.1; four rows more
+// than eight cost 0.2 us).
+template <int MP, bool GLU, int DEPTH, int KSPLIT>
+constexpr int few_rows_waves() { return MP == 16 && GLU && DEPTH == 1 && KSPLIT <= 4 ? 2 : 1; }
+
 template <int MP, int R, int DEPTH, int KSPLIT, bool GLU, int EPI, bool MORE, bool ONCE>
-__global__ __launch_bounds__(64 * KSPLIT) void gemm_bf16_few_rows_kernel(
+__global__ __launch_bounds__(64 * KSPLIT, (few_rows_waves<MP, GLU, DEPTH, KSPLIT>())) void gemm_bf16_few_rows_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Wp, void* __restrict__ C, int c_float32, int M, int N, int K, int lda, int KB, int n_out,
     const FewRowsFuse fz, const typename std::conditional<MORE, GemmExtra, GemmEpilogue>::type ex) {
     static_assert(MP == 4 || MP == 8 || MP == 16, "rows a load packs");
+    static_assert(DEPTH == 1 || DEPTH == 2, "the ends of the stream are written for one unit in flight and for two");
     static_assert(!GLU || R == 2, "a gate and its up group are a wave's");
     static_assert(EPI < 2 || !GLU, "the product before a norm has a plain float32 result");
     static_assert(!MORE || (EPI == 0 && !GLU), "planes and activations are for plain products");
@@ -209,8 +216,6 @@ __global__ __launch_bounds__(64 * KSPLIT) void gemm_bf16_few_rows_kernel(
         };
         if (more == 0) end(std::integral_constant<int, 0>{});
         if constexpr (DEPTH > 1) { if (more == 1) end(std::integral_constant<int, 1>{}); }
-        if constexpr (DEPTH > 2) { if (more == 2) end(std::integral_constant<int, 2>{}); }
-        if constexpr (DEPTH > 3) { if (more == 3) end(std::integral_constant<int, 3>{}); }
     } else {
         auto all = [&](auto UNITS) {
             constexpr int m = decltype(UNITS)::value;
@@ -222,8 +227,6 @@ __global__ __launch_bounds__(64 * KSPLIT) void gemm_bf16_few_rows_kernel(
         };
         if (count <= 0) factors();
         if constexpr (DEPTH > 1) { if (count == 1) all(std::integral_constant<int, 1>{}); }
-        if constexpr (DEPTH > 2) { if (count == 2) all(std::integral_constant<int, 2>{}); }
-        if constexpr (DEPTH > 3) { if (count == 3) all(std::integral_constant<int, 3>{}); }
     }
 
     // The steps' sums of the columns that hold them, row fr's in lane fr of a row of sixteen lanes.
@@ -348,8 +351,12 @@ static int launch_few_rows(const bf16_t* A, const bf16_t* Wp, void* C, int M, in
     return tff_check_launch("gemm_bf16_few_rows");
 }
 
-// Row groups a block, units in flight and waves, by the columns, K and the rows.  How many waves share K goes by the columns and K alone (but for wide
-// gated weights, see there).  Fitted to 300 products of 192 to 12,288 k and 256 to 34,816 columns, rows 2, 8 and 16; us beside the rules.
+// Row groups a block, units in flight and waves, by the columns, K and the rows.  How many waves share K goes by the columns and K alone (but for
+// wide gated weights, see there).  Fitted to 300 products of 192 to 12,288 k and 256 to 34,816 columns, rows 2, 8 and 16, and, where K is short or the
+// weight gated, to 14,600 of 64 to 12,000 k and 64 to 60,000 columns; us beside the rules.
+// With a short K and many columns the blocks are many and their work little: a CU goes through them as fast as its registers hold waves with work, so
+// that no more waves share K than it has units for (12 rows, 59,520 x 64 on four waves 13.0, on one 5.9; 16 rows, 55,040 x 152 13.7 and 7.5, on four
+// waves and on two 16,384 x 512 7.0 and 5.6).
 template <int MP, int EPI>
 static int few_rows_for(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N, int K, int lda, const GemmCall& ex, int c_dtype, int glu_out, hipStream_t s,
                         const FewRowsFuse& fz) {
@@ -358,11 +365,14 @@ static int few_rows_for(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N
     if (glu_out > 0) {
         if constexpr (EPI < 2) {
             // A pair of groups a CU or less: a block has to keep its CU's share of the stream in flight alone.  (Two units of sixteen rows are
-            // more registers than eight waves have: spilled, 2,560 k took twice as long.)
+            // more registers than eight waves have: spilled, 2,560 k took twice as long.)  With the rows' factors to add up, eight waves also for a short K.
             if (nb <= 2 * cus) {
+                if (EPI == 0 && K <= 512) TFF_FEW(2, 2, 2, true);
                 if constexpr (MP < 16) TFF_FEW(2, 2, 8, true);
                 else TFF_FEW(2, 1, 8, true);
             }
+            // Two waves: 16 rows, 12,800 x 264 gated 5.3 on eight, 4.8 on two; after a norm 7.9 and 7.0.
+            if (nb <= 4 * cus) TFF_FEW(2, 2, 2, true);
             // Eight waves of a short K have a unit or none: 18,432 x 1,024, 2 / 8 / 16 rows, two waves 9.1 / 9.4 / 10.6, eight 9.4 / 9.8 / 13.7.
             if (K < 2048) TFF_FEW(2, 1, 2, true);
             // More, and more than eight rows: blocks of four waves, of which a CU holds more at sixteen rows' registers (34,816 x 5,120, 16 rows,
@@ -374,7 +384,17 @@ static int few_rows_for(const bf16_t* A, const bf16_t* Wp, void* C, int M, int N
         }
     } else {
         // A group a CU or less: as above (2,048 x 12,288, 2 rows, eight waves 12.1, four 12.8).
-        if (nb <= cus) TFF_FEW(1, 2, 8, false);
+        if (nb <= cus) {
+            if (EPI != 1 && K <= 256) TFF_FEW(1, 2, 2, false);
+            TFF_FEW(1, 2, 8, false);
+        }
+        // (up to two groups a CU the rows' factors are what a block of few waves waits for)
+        if (nb <= 4 * cus) {
+            if (K <= 1024 && (EPI != 1 || nb > 2 * cus)) TFF_FEW(1, 2, 2, false);
+        } else if (K <= 896) {
+            if constexpr (EPI == 1) TFF_FEW(1, 2, 2, false);
+            else TFF_FEW(1, 2, 1, false);
+        }
         // A few groups a CU: two groups a block, which then all run at once and fetch the rows for two (6,144 x 12,288, 16 rows, 30.9,
         // one group a block 36.8); up to four rows there is little to fetch, and one group a block begins sooner (25.6 and 26.4).
         if constexpr (MP == 4) {
