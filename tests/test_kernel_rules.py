@@ -251,3 +251,20 @@ def test_an_activation_counts_the_kernel_that_adds_up_the_parts():
     for M, N, K, parts in ((200, 18432, 4096, 2), (128, 12288, 4096, 2), (90, 9216, 2048, 2), (1055, 4096, 4096, 2), (333, 512, 192, 1), (16, 18432, 4096, 0), (2048, 18432, 4096, 0)):
         assert L.tff_gemm_unary_workspace_bytes(M, N, K) == parts * M * N * 4, (M, N, K)
         assert L.tff_gemm_takes_unary(M, N, K) == (parts > 0 or M <= 16)
+
+
+def _plan(M, N, K, glu=0, keep=0):
+    import ctypes
+    r, c, s = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    assert _lib().tff_gemm_plan(M, N, K, glu, keep, ctypes.byref(r), ctypes.byref(c), ctypes.byref(s)) == 0
+    return r.value, c.value, s.value
+
+
+def test_few_gated_rows_go_on_tiles_by_how_these_fill_the_cus():
+    """Not by the number of the weight's elements alone: nine rows and more on tiles that fill three quarters of one round, else the stream."""
+    for N, K in ((28672, 8192), (27648, 5120), (24576, 2048), (24576, 4096), (51200, 5120)):
+        assert _plan(9, N, K, 1)[0] == _plan(16, N, K, 1)[0] == 32, (N, K)
+        assert _plan(8, N, K, 1)[0] == (32 if N * K >= 2.4e8 else 0), (N, K)
+    # half a round of tiles and less, a second round, K in no units of 64
+    for N, K in ((8192, 12288), (22016, 8192), (34816, 5120), (16384, 8192), (73728, 4096), (28672, 8200)):
+        assert _plan(9, N, K, 1) == _plan(16, N, K, 1) == (0, 0, 1), (N, K)

@@ -831,18 +831,10 @@ static int launch_row_tiles(const bf16_t* A, const bf16_t* Wp, void* C, int M, i
 // up to 64 and 32 rows, of 64 and 32 rows (256 or 128 columns), and from 65 to 512 rows also
 // 64 x 128 with several row tiles; otherwise the sixteen-wave kernel's tiles.
 struct GemmPlan { int tile; int bn; int splits; };   // tile = rows of a block tile
-// Up to 16 rows, not gated: more row groups of 16 columns than CUs, but at most 1.6 times as many (see plan_for).
-static bool two_row_groups(int N) {
+// Up to 16 rows, not gated: more groups of 16 columns than CUs, but at most 1.6 times as many.
+static bool little_more_groups_than_cus(int N) {
     const int nb = (N + 15) / 16, cus = tff_device_cus();
     return nb > cus && nb * 10 <= cus * 16;
-}
-// Up to 16 rows, gated: the streaming kernel's time grows with the rows, that of the four-wave kernel's tiles of 32 rows, K in one part, does not.
-// us at 2 / 8 / 12 / 16 rows after a norm, streaming against tiles: the 32B shape's gate and up (2.6e8 elements) 84.8 / 85.8 / 92.7 / 97.3 against 87; the
-// 14B shape's (1.8e8, 272 tiles of 128 columns: a second round for 16 of them) 60.8 / 62.1 / 67.6 / 70.9 against 73 to 75; the 8B shape's (1.0e8, 192
-// tiles) 35.2 / 35.8 / 41.6 / 41.6 against 39 to 41; the 4B shape's (5e7) 18.9 / 19.5 / 21.9 / 22.6 against 23.8.
-static bool few_rows_gated_on_tiles(int M, int N, int K) {
-    const double w = (double)N * K;
-    return K % 64 == 0 && (w >= 2.4e8 || (w >= 0.9e8 && w < 1.6e8 && M >= 12));
 }
 // One row tile of 32 rows, K in one part: the width (128 or 256 columns) that plan_for's model prices lowest.
 static int plan_rows32(int N, int K) {
@@ -861,24 +853,36 @@ static int plan_rows32(int N, int K) {
     return best;
 }
 
+// Up to 16 rows, gated: the streaming kernel's time grows with the rows, from nine on by a tenth; that of the four-wave kernel's tiles of 32 rows, K in
+// one part, does not, and hangs on how their blocks go round the CUs: ahead where they fill three quarters of one round, behind with fewer, and in
+// a second round.  us at 8 / 9 / 16 rows after a norm, streaming against tiles, and the tiles: 51,200 x 5,120 79.5 / 83.4 / 90.3 against 79.5, 200;
+// 28,672 x 8,192 71.3 / 75.2 / 78.7 against 75, 224; 27,648 x 5,120 46.1 / 49.0 / 53.2 against 47.5, 216; 24,576 x 4,096 31.7 / 37.6 / 34.1 against 36,
+// 192; 34,816 x 5,120 56.9 / 60.6 / 65.6 against 65, 136; 22,016 x 8,192 54.3 / 59.9 / 60.2 against 62.5, 172; 8,192 x 12,288 33.4 / 34.3 / 35.9 against
+// 83, 64.  11,000 products of 2e7 to 5e8 elements and 2 to 16 rows: 0.5 % from the better one on average.  (The largest weights are on tiles with any rows:
+// within 2 % there.)
+static bool few_rows_gated_on_tiles(int M, int N, int K) {
+    const double w = (double)N * K;
+    if (K % 64 != 0 || !(w >= 2.4e8 || (M >= 9 && w >= 4e7))) return false;
+    const int bn = plan_rows32(N, K), cus = tff_device_cus(), blocks = (N + bn - 1) / bn;
+    return blocks <= cus && blocks * 4 >= cus * 3;
+}
+
 // plane > 0: the columns of several products, so many each; a tile takes columns of one of them, and K is not split.
 // unary: an activation follows, in the kernel that adds up the parts, which one part then has as well (200 rows of 18,432 x 4,096, a squared relu: in
 // one part, as without it, 63 us, in two 54).
 static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0, bool unary = false) {
     const double CUS = (double)tff_device_cus();
-    // Up to 16 rows: the streaming kernel, a block per 16 columns, unless those blocks go badly
-    // round the 256 CUs (320 of them take as long as 512 would: N = 5120), the caller takes
-    // partial sums anyway and the weight is large enough for the gain (three eighths of its
-    // stream) to pay for the norm's own kernel, which the streaming kernel would have taken into
-    // its epilogue: then the tiles below, whose blocks split K as finely as it takes.
+    // Up to 16 rows: the streaming kernel.  Not where the caller takes partial sums anyway, the groups of 16 columns go badly round the CUs and the
+    // weight is large: those rows are on tiles that split K, with the norm in a kernel of its own.  These lines were drawn beside a streaming
+    // kernel that took a third longer, and are not where the two meet now: with the norm and the next product, streaming against tiles,
+    // us at 9 / 16 rows, 5,120 x 17,408 43 / 49 against 56; 2,560 x 20,480 30 / 37 against 39; 12,800 x 22,528 at 16 rows 149 against 122.
     if (M <= 16 && glu && few_rows_gated_on_tiles(M, N, K)) return {32, plan_rows32(N, K), 1};
     if (M <= 16 && plane) return {0, 0, 1};
     if (M <= 16) {
         const int nb = (N + 15) / 16;
         const double fill = (double)nb / (ceil(nb / CUS) * CUS);
         if (glu || !keep || fill >= 0.8 || (double)N * K < 40e6) return {0, 0, 1};
-        // (two row groups a block: ahead of the tiles up to 8 rows, and up to 16 where K is short)
-        if (two_row_groups(N) && (M <= 8 || (double)N * K < 45e6)) return {0, 0, 1};
+        if (little_more_groups_than_cus(N) && (M <= 8 || (double)N * K < 45e6)) return {0, 0, 1};
     }
     const int nk = (K + 63) / 64;
     if (K % 64 == 0) {
