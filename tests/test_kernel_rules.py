@@ -268,3 +268,12 @@ def test_few_gated_rows_go_on_tiles_by_how_these_fill_the_cus():
     # half a round of tiles and less, a second round, K in no units of 64
     for N, K in ((8192, 12288), (22016, 8192), (34816, 5120), (16384, 8192), (73728, 4096), (28672, 8200)):
         assert _plan(9, N, K, 1) == _plan(16, N, K, 1) == (0, 0, 1), (N, K)
+
+
+def test_parts_of_k_pay_for_the_kernel_that_adds_them_up():
+    """Products of some hundred rows and a short K stay whole; sums kept for a norm are cut as finely as the norm's reads of the parts allow, and few columns
+    of many rows too."""
+    assert _plan(68, 4096, 1024) == _plan(90, 4096, 1024) == (64, 128, 1)
+    assert _plan(107, 512, 768)[2] == _plan(78, 640, 832)[2] == 1
+    assert _plan(116, 2048, 2048, keep=1) == (64, 128, 4)
+    assert _plan(2219, 128, 15424, keep=1)[2] == 8 and _plan(2210, 4096, 18432, keep=1)[2] <= 2

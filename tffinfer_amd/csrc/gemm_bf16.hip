@@ -896,8 +896,9 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
         // * Results of one kernel or of the sum over the parts, more than 64 rows: 4,234 products of 65 .. 16,500 rows.  The pick is 0.6 % from the best
         //   candidate on average; against the tiles of 256, 128 and 64 rows alone 0.979 of the time (513 to 1,040 rows 0.949), and in 3 of 100 slower by
         //   more than 2 %.
-        // * Sums kept for a norm, more than 64 rows, no more columns than K: 2,832 products; 0.8 % from the best with the norm behind it, 0.962 of the time of
-        //   the tiles and constants before (257 to 2,080 rows 0.943), in 7 of 100 slower by more than 2 %.
+        // * Sums kept for a norm, more than 64 rows, no more columns than K: 3,568 products of 65 .. 4,500 rows, each timed with the norm behind it: 0.9 % from the
+        //   best, 0.976 of the time of the tiles of 256, 128 and 64 rows by their constants, in 3 of 100 slower by more than 3 %.  The norm reads the
+        //   parts one after the other, 0.28 us each beside their bytes (116 rows of 2,048 x 2,048: four parts 10.9, eight 12.7).
         // * Kept sums of more columns than K, which no model's product into its stream has: constants of an older fit.
         // * Up to 64 rows the four waves side by side take 64 or 32 rows: a product of so few rows is its
         //   weight's stream, and a block that does not work through 128 rows for 32 asks for its next
@@ -910,21 +911,25 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
         // the sums are not kept; and beyond 2,048 rows K in one part (2,210 of 4,096 x 18,432 257 on 256 x 192, 335 on 192 x 128 in two).
         // From 1,500 rows on they have to be 2 % ahead: large products are bound by the power the card allows, of which a smaller tile's reads take more
         // (slower than the tiles before by more than 2 %: 4 of 100 such products without this margin, 0.3 with it).
-        // Three and six parts are for kept sums of 129 to 1,024 rows: beyond, the parts' traffic grows and the rounds are many.
+        // Three and six parts are for kept sums of 129 to 1,024 rows: beyond, the parts' traffic grows and the rounds are many.  Beyond 2,048 rows kept parts that
+        // are more than the caches hold are not cut further (but few columns are: 2,219 rows of 128 x 15,424 in eight parts 25.9, in two 48.6).
+        // The kernel that adds up results' parts costs 3.0 us beside its bytes, 2.1 where it also joins gate and up (68 rows of 4,096 x 1,024 in one part 7.4,
+        // in four 9.9; 600 gated rows of 512 x 1,088 in two parts rather than one).
         // A rate is in flops a microsecond of a CU; ends: us that a block's first fetch and storing its tile take.  Of results, of kept sums, of the older
         // fit's, up to 64 rows.
         struct Cand { int bm, bn, slots; double rate, ends, rate_kept, ends_kept, rate_wide, rate_few; };
         static const Cand cands[15] = {
-            {256, 256, 1, 8.43e6, 1.02, 8.12e6, 1.77, 6.45e6, 0}, {256, 192, 1, 7.65e6, 1.04, 7.50e6, 1.10, 6.10e6, 0},
-            {256, 128, 1, 6.20e6, 0.95, 5.75e6, 1.38, 5.42e6, 0}, {192, 256, 1, 7.80e6, 1.14, 7.63e6, 2.20, 0, 0},
-            {192, 192, 1, 5.90e6, 0.77, 4.48e6, 0.45, 0, 0}, {192, 128, 1, 4.70e6, 0.66, 5.59e6, 0.65, 0, 0},
-            {128, 384, 1, 10.6e6, 1.76, 4.13e6, 1.55, 6.49e6, 3.24e6}, {128, 256, 1, 6.18e6, 0.96, 5.95e6, 0.73, 5.38e6, 4.61e6},
-            {128, 128, 1, 4.41e6, 0.61, 5.04e6, 0.65, 3.56e6, 3.45e6}, {96, 128, 1, 3.71e6, 0.84, 4.30e6, 0.19, 0, 0},
+            {256, 256, 1, 8.43e6, 1.02, 9.85e6, 0.90, 6.45e6, 0}, {256, 192, 1, 7.65e6, 1.04, 7.58e6, 0.36, 6.10e6, 0},
+            {256, 128, 1, 6.20e6, 0.95, 5.79e6, 1.59, 5.42e6, 0}, {192, 256, 1, 7.80e6, 1.14, 7.63e6, 1.52, 0, 0},
+            {192, 192, 1, 5.90e6, 0.77, 6.92e6, 0.45, 0, 0}, {192, 128, 1, 4.70e6, 0.66, 5.27e6, 0.20, 0, 0},
+            {128, 384, 1, 10.6e6, 1.76, 4.43e6, 1.60, 6.49e6, 3.24e6}, {128, 256, 1, 6.18e6, 0.96, 6.18e6, 0.52, 5.38e6, 4.61e6},
+            {128, 128, 1, 4.41e6, 0.61, 4.87e6, 0.58, 3.56e6, 3.45e6}, {96, 128, 1, 3.71e6, 0.84, 4.12e6, 0.29, 0, 0},
             {64, 256, 1, 0, 0, 0, 0, 0, 2.4e6}, {64, 128, 1, 0, 0, 0, 0, 0, 2.0e6},
-            {32, 256, 1, 0, 0, 0, 0, 0, 1.4e6}, {32, 128, 1, 0, 0, 0, 0, 0, 1.3e6}, {64, 128, 2, 2.67e6, 0.12, 3.95e6, 0.32, 2.48e6, 0}};
+            {32, 256, 1, 0, 0, 0, 0, 0, 1.4e6}, {32, 128, 1, 0, 0, 0, 0, 0, 1.3e6}, {64, 128, 2, 2.67e6, 0.12, 4.62e6, 0.27, 2.48e6, 0}};
         const bool few = M <= 64, wide = keep && !few && N > K, kept = keep && !few && !wide;
-        // bytes a microsecond of all CUs together and of one alone
-        const double HBM = few ? 7.72e6 : wide ? 8.18e6 : kept ? 31.57e6 : 9.41e6, CU_MAX = few ? 6.0e4 : wide ? 6.54e4 : kept ? 5.79e4 : 6.04e4;
+        // bytes a microsecond of all CUs together and of one alone (of kept sums the tiles' rates carry what the stream costs: no bound on all CUs
+        // together improves their fit)
+        const double HBM = few ? 7.72e6 : wide ? 8.18e6 : kept ? INFINITY : 9.41e6, CU_MAX = few ? 6.0e4 : wide ? 6.54e4 : kept ? 4.98e4 : 6.04e4;
         GemmPlan best = {128, 128, 1};
         double best_t = 1e30;
         for (const Cand& c : cands) {
@@ -940,12 +945,13 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
             for (int S = 1; S <= (plane ? 1 : (glu && M > 64) ? 2 : 8); S += S < 4 ? 1 : 2) {
                 if (S > 1 && nk / S < 4) break;
                 if (S % 3 == 0 && !(kept && M > 128 && M <= 1024)) continue;
-                if (S > (between ? 1 : 2) && kept && M > 2048) break;
+                const double plane_bytes = (double)M * N * 4.0;
+                if (S > (between ? 1 : 2) && kept && M > 2048 && S * plane_bytes > 32e6) break;
                 const double blocks = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * S;
                 const double rounds = ceil(blocks / (CUS * c.slots)), at_once = fmin(blocks, CUS * c.slots);
                 double rate = kept ? c.rate_kept : c.rate, ends = kept ? c.ends_kept : c.ends, units = (nk + S - 1) / S;
                 double streams = ceil((double)N / c.bn) * S;              // (row tiles fetch a column tile's weight once between them)
-                double share = c.slots == 2 && blocks > CUS ? (kept ? 2.19 : 1.77) : 1.0;     // blocks that share a CU's MFMAs, and each other's waits
+                double share = c.slots == 2 && blocks > CUS ? (kept ? 2.92 : 1.77) : 1.0;     // blocks that share a CU's MFMAs, and each other's waits
                 if (few || wide) {
                     rate = few ? c.rate_few : c.rate_wide;
                     ends = few ? 3.0 : 1.29 + 2.55 * (c.bm * c.bn / 65536.0);
@@ -959,9 +965,8 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
                 // the partial sums: written, read and added by a second kernel, or (kept) read by the
                 // consumer in place of one plane
                 // (from the caches as long as they are some 32 MB)
-                const double plane_bytes = (double)M * N * 4.0;
-                if (S > 1 && keep) t += (S - 1.0) * plane_bytes / (few || (kept && S * plane_bytes <= 32e6) ? 4e6 : 1.97e6);
-                else if (S > 1 || unary) t += S * plane_bytes / (few ? 2.54e6 : 2.21e6) + (few ? 2.7 : 2.09);
+                if (S > 1 && keep) t += (S - 1.0) * (plane_bytes / (few || (kept && S * plane_bytes <= 32e6) ? 4e6 : 1.97e6) + (kept ? 0.28 : 0.0));
+                else if (S > 1 || unary) t += S * plane_bytes / (few ? 2.54e6 : 2.21e6) + (few ? 2.7 : glu ? 2.09 : 3.0);
                 if (between && M >= 1500) t *= 1.02;
                 if (t < best_t) { best_t = t; best = {c.bm, c.bn, S}; }
             }
