@@ -480,7 +480,7 @@ BETWEEN_CASES = [
 @pytest.mark.parametrize("M,N,K,glu,keep,tile", BETWEEN_CASES)
 def test_linear_on_tiles_of_192_and_96_rows(M, N, K, glu, keep, tile):
     """The four-wave kernel with six row groups a wave: every tile, gated or not, ragged rows, K in one part and split with the sums added
-    or handed on, a row stride beyond K."""
+    or handed on, a row stride beyond K.  Against 64 bits."""
     ops = _ops()
     g = torch.Generator().manual_seed(N + K)
     wide = torch.randn(M, K + 72, generator=g).to(torch.bfloat16).to(DEV)
@@ -490,11 +490,11 @@ def test_linear_on_tiles_of_192_and_96_rows(M, N, K, glu, keep, tile):
         I = N // 2
         gate = (torch.randn(I, K, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
         up = (torch.randn(I, K, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
-        a, b = ops.linear(x.float(), gate.float()), ops.linear(x.float(), up.float())
-        ref, pw = a / (1 + torch.exp(-a)) * b, ops.pack_gate_up(gate, up)
+        a, b = x.double() @ gate.double().T, x.double() @ up.double().T
+        ref, pw = a * torch.sigmoid(a) * b, ops.pack_gate_up(gate, up)
     else:
         w = (torch.randn(N, K, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
-        ref, pw = ops.linear(x.float(), w.float()), ops.pack_weight(w)
+        ref, pw = x.double() @ w.double().T, ops.pack_weight(w)
     y = ops.linear(x, pw, out_dtype=torch.float32, partials=keep)
     if keep and tile[2] > 1:
         assert y.dim() == 3 and y.shape[0] == tile[2]
@@ -1978,6 +1978,27 @@ def test_products_of_several_planes(M, P, N, K):
     ref = torch.stack([x[p].double() @ w[p * N:(p + 1) * N].double().T for p in range(P)])
     assert tuple(out.shape) == (P, M, N)
     assert float((out.double() - ref).abs().max()) < 2.0 ** -20 * K * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("P,M,N,K,tile", [
+    (4, 150, 4096, 1024, (96, 128)), (4, 700, 4096, 1024, (192, 256)), (4, 1500, 4096, 1088, (192, 256)), (4, 601, 2048, 1024, (192, 128)),
+    (3, 1850, 1536, 1024, (192, 192)), (3, 500, 1536, 1088, (96, 128)), (2, 1301, 1536, 1088, (192, 128))])
+def test_products_of_several_planes_on_tiles_of_192_and_96_rows(P, M, N, K, tile):
+    """The four-wave kernel's tiles between the powers of two, K from 1,024 on, ragged rows: each plane against its product in 64 bits, as above."""
+    import ctypes
+    from tffinfer_amd.kernels import lib
+    r, c = ctypes.c_int(), ctypes.c_int()
+    assert lib.load().tff_gemm_planes_plan(P, M, N, K, ctypes.byref(r), ctypes.byref(c)) == 0 and (r.value, c.value) == tile
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(P, M, K, generator=g, device=DEV).bfloat16()
+    w = torch.randn(P * N, K, generator=g, device=DEV).bfloat16()
+    out = ops.linear_planes(x, ops.pack_weight(w))
+    assert tuple(out.shape) == (P, M, N)
+    for p in range(P):
+        ref = x[p].double() @ w[p * N:(p + 1) * N].double().T
+        # K products of two of size one, float32 sums: as many roundings of the largest sum as K has sixteenths, half an ulp each, is far above what shows
+        assert float((out[p].double() - ref).abs().max()) < 2.0 ** -24 * (K / 16) * float(ref.abs().max()), p
 
 
 @pytest.mark.parametrize("act", ["tanh", "gelu", "gelu_tanh", "relu2"])

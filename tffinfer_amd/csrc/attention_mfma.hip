@@ -1568,7 +1568,7 @@ TFF_API int tff_attention_split_reduce(const float* part_o, const float* part_ml
 // equal splits of every entry leave the longest entry's waves at work long after the others.
 // block_waves 8: a block of eight waves per run and kv head instead, which split the run among them
 // and merge in LDS (head sizes up to 128, one column tile).  merge 0: the caller knows that every
-// entry is one run (run_start[r] = r), so nothing is partial and the second kernel is left out.
+// entry is one run, wherever it stands, so nothing is partial and the second kernel is left out.
 // Partial results (part_o [num_runs][nq][d], part_ml [num_runs][nq][2]) of the entries with more
 // than one run are merged by a second kernel.
 TFF_API int tff_attention_decode_runs(const void* qkv, int qkv_stride, void* out, float* part_o,

@@ -1317,6 +1317,15 @@ TFF_API int tff_gemm_planes(const void* A, size_t a_step, const void* W, float* 
     return tff_gemm_bf16((const bf16_t*)A, (const bf16_t*)W, C, M, planes * N, K, lda, GemmCall{{{nullptr, glu_act(__builtin_inff(), 1.0f, 0.0f)}, 0, N, a_step}, w_once},
                          TFF_F32, 0, nullptr, 0, 0, (hipStream_t)stream);
 }
+// Their plan's tile, for tests.
+TFF_API int tff_gemm_planes_plan(int planes, int M, int N, int K, int* tile_rows, int* tile_cols) {
+    TFF_REQUIRE(planes > 0 && M > 0 && N > 0 && K > 0 && (long)planes * N < (1L << 30) && tff_gemm_planes_supported(N, K) && tile_rows && tile_cols,
+                "gemm_planes_plan: bad sizes %d x M=%d N=%d K=%d", planes, M, N, K);
+    const GemmPlan p = plan_for(M, planes * N, K, false, false, N);
+    *tile_rows = p.tile;
+    *tile_cols = p.bn;
+    return 0;
+}
 
 // ------------------------------------------------------------- packing ---
 // Row-major [N, K] -> fragment order, with zero padding to 16 rows and 32 k.

@@ -70,6 +70,7 @@ TFF_API int tff_gemm_unary(const void* A, const void* W, void* C, int M, int N, 
 // C[p] = A[p] . W[p]^T, p < planes, in one launch: A[p] = A + p * a_step, C [planes, M, N] float32, W the weights one after the other in
 // fragment order; N in units of 128, K of 64.
 TFF_API int tff_gemm_planes_supported(int N, int K);
+TFF_API int tff_gemm_planes_plan(int planes, int M, int N, int K, int* tile_rows, int* tile_cols);   // (tff_gemm_plan's tile of them)
 TFF_API int tff_gemm_planes(const void* A, size_t a_step, const void* W, float* C, int planes, int M, int N, int K, int lda, int w_once, tff_stream_t stream);
 
 // resid[M, N] += A . W^T; x_out[M, N] = bfloat16 of tanh(alpha * resid) * norm_w + bias over the new resid: a norm
@@ -215,9 +216,9 @@ TFF_API int tff_attention_split_reduce(const float* part_o, const float* part_ml
 // length keep the waves busy alike however uneven the entries' lengths are.  block_waves 1: a wave
 // per run and kv head; 8: a block of eight waves that split the run among them and merge in LDS
 // (head sizes up to 128, up to 16 query heads a kv head), for runs dealt with that in mind.
-// num_runs is a multiple of eight.  merge 0: the caller knows that every entry is one run, so no
-// result is partial and the merging kernel is not launched (a wrong 0 leaves the entries of
-// several runs without a result).
+// num_runs is a multiple of eight.  merge 0: the caller knows that every entry is one run (the runs
+// in any order; sooner with run r entry r's), so no result is partial and the merging kernel is
+// not launched (a wrong 0 leaves the entries of several runs without a result).
 TFF_API int tff_attention_decode_runs(const void* qkv, int qkv_stride, void* out, float* part_o,
                                       float* part_ml, void* k_cache, void* v_cache,
                                       const int32_t* block_tables, int bt_stride,

@@ -50,6 +50,7 @@ _SIGNATURES = {
     "tff_gemm_unary": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _Z, _I, _P],
     "tff_gemm_planes_supported": [_I, _I],
     "tff_gemm_planes": [_P, _Z, _P, _P, _I, _I, _I, _I, _I, _I, _P],
+    "tff_gemm_planes_plan": [_I, _I, _I, _I, _P, _P],
     "tff_gemm_plan": [_I, _I, _I, _I, _I, _P, _P, _P],
     "tff_gemm_residual_prenorm": [_P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _I, _I, _P],
     "tff_gemm_residual_dyt": [_P, _P, _I, _I, _I, _I, _P, _F, _P, _P, _P, _I, _P],

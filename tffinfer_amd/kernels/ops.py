@@ -1103,7 +1103,8 @@ def attention_decode_fused(qkv: torch.Tensor, nq: int, nkv: int, d: int, q_weigh
     (int32 [runs, 4]: row, first key, end of keys, the row's position) and ``run_start`` (int32
     [R + 1]): the rows' keys dealt into runs by the host, a wave per run and
     kv head (``kernels.key_runs``), or a block of eight waves if they were
-    dealt for that (``runs_for_blocks``) and the head size allows it;
+    dealt for that (``runs_for_blocks``), or are a run a row (``runs_merge`` False)
+    of no more pairs of row and kv head than CUs, and the head size allows it;
     ``runs_merge`` False: the caller knows that every row is one run, and the
     kernel that merges partial results is left out.  Without runs every
     row's keys are split alike (``splits``)."""
