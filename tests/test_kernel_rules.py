@@ -277,3 +277,19 @@ def test_parts_of_k_pay_for_the_kernel_that_adds_them_up():
     assert _plan(107, 512, 768)[2] == _plan(78, 640, 832)[2] == 1
     assert _plan(116, 2048, 2048, keep=1) == (64, 128, 4)
     assert _plan(2219, 128, 15424, keep=1)[2] == 8 and _plan(2210, 4096, 18432, keep=1)[2] <= 2
+
+
+def test_parts_of_k_in_threes_fit_the_cus_of_every_xcd():
+    """An XCD takes an eighth of the tiles in all their parts: blocks that are no more than the CUs may still be more than one XCD's CUs, a second round."""
+    for M, N, K in ((160, 8064, 14144), (303, 3584, 15232), (411, 10496, 13120), (382, 896, 6144)):
+        assert _plan(M, N, K, keep=1)[2] % 3 != 0, (M, N, K)
+    seen = 0
+    for M in range(130, 1025, 37):
+        for N in range(512, 8193, 384):
+            for K in (N, 9728, 14144):
+                rows, cols, parts = _plan(M, N, K, keep=1)
+                tiles = -(-M // rows) * -(-N // cols)
+                if parts % 3 == 0 and rows > 64 and tiles * parts <= 256:
+                    seen += 1
+                    assert -(-tiles // 8) * parts <= 32, (M, N, K, rows, cols, parts)
+    assert seen > 50

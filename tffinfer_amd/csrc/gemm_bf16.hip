@@ -890,15 +890,17 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
         // its 64 x 128, two blocks to a CU.  A block goes through its part of K in
         // units of 64; a unit takes what its MFMAs take at the tile's rate or what its columns of W take
         // to arrive, whichever is longer: a block's share of the HBM stream, at most what one CU pulls.
-        // Blocks go round the CUs; each round ends with the pipeline filled and the tile stored.  The constants are
+        // Blocks go round the CUs of an XCD, which takes an eighth of the tiles in all their parts: 42 tiles in six parts are 252 blocks, but on some
+        // XCDs 36 for 32 CUs, a second round (160 rows of 8,064 x 14,144 104 us, in four parts 69; 411 rows of 10,496 x 13,120, 82 tiles in three parts, 201,
+        // in two 133).  Each round ends with the pipeline filled and the tile stored.  The constants are
         // fitted to products of the 0.6B to 14B shapes and of the other designs, every tile with
         // 1 .. 8 parts timed on an MI355X (weights in turn that no cache holds, rows from five places), in four pieces:
         // * Results of one kernel or of the sum over the parts, more than 64 rows: 4,234 products of 65 .. 16,500 rows.  The pick is 0.6 % from the best
         //   candidate on average; against the tiles of 256, 128 and 64 rows alone 0.979 of the time (513 to 1,040 rows 0.949), and in 3 of 100 slower by
         //   more than 2 %.
-        // * Sums kept for a norm, more than 64 rows, no more columns than K: 3,568 products of 65 .. 4,500 rows, each timed with the norm behind it: 0.9 % from the
-        //   best, 0.976 of the time of the tiles of 256, 128 and 64 rows by their constants, in 3 of 100 slower by more than 3 %.  The norm reads the
-        //   parts one after the other, 0.28 us each beside their bytes (116 rows of 2,048 x 2,048: four parts 10.9, eight 12.7).
+        // * Sums kept for a norm, more than 64 rows, no more columns than K: 3,875 products of 65 .. 16,500 rows, each timed with the norm behind it: 1.0 % from
+        //   the best, 0.972 of the time of the tiles of 256, 128 and 64 rows by their constants, in 2 of 100 slower by more than 3 %.  The norm reads the
+        //   parts one after the other, 0.3 us each beside their bytes (116 rows of 2,048 x 2,048: four parts 10.9, eight 12.7).
         // * Kept sums of more columns than K, which no model's product into its stream has: constants of an older fit.
         // * Up to 64 rows the four waves side by side take 64 or 32 rows: a product of so few rows is its
         //   weight's stream, and a block that does not work through 128 rows for 32 asks for its next
@@ -919,17 +921,16 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
         // fit's, up to 64 rows.
         struct Cand { int bm, bn, slots; double rate, ends, rate_kept, ends_kept, rate_wide, rate_few; };
         static const Cand cands[15] = {
-            {256, 256, 1, 8.43e6, 1.02, 9.85e6, 0.90, 6.45e6, 0}, {256, 192, 1, 7.65e6, 1.04, 7.58e6, 0.36, 6.10e6, 0},
-            {256, 128, 1, 6.20e6, 0.95, 5.79e6, 1.59, 5.42e6, 0}, {192, 256, 1, 7.80e6, 1.14, 7.63e6, 1.52, 0, 0},
-            {192, 192, 1, 5.90e6, 0.77, 6.92e6, 0.45, 0, 0}, {192, 128, 1, 4.70e6, 0.66, 5.27e6, 0.20, 0, 0},
-            {128, 384, 1, 10.6e6, 1.76, 4.43e6, 1.60, 6.49e6, 3.24e6}, {128, 256, 1, 6.18e6, 0.96, 6.18e6, 0.52, 5.38e6, 4.61e6},
-            {128, 128, 1, 4.41e6, 0.61, 4.87e6, 0.58, 3.56e6, 3.45e6}, {96, 128, 1, 3.71e6, 0.84, 4.12e6, 0.29, 0, 0},
+            {256, 256, 1, 8.43e6, 1.02, 8.16e6, 1.72, 6.45e6, 0}, {256, 192, 1, 7.65e6, 1.04, 7.76e6, 2.57, 6.10e6, 0},
+            {256, 128, 1, 6.20e6, 0.95, 6.86e6, 1.45, 5.42e6, 0}, {192, 256, 1, 7.80e6, 1.14, 7.70e6, 1.66, 0, 0},
+            {192, 192, 1, 5.90e6, 0.77, 5.95e6, 1.92, 0, 0}, {192, 128, 1, 4.70e6, 0.66, 5.27e6, 0.67, 0, 0},
+            {128, 384, 1, 10.6e6, 1.76, 7.05e6, 3.67, 6.49e6, 3.24e6}, {128, 256, 1, 6.18e6, 0.96, 7.00e6, 0.40, 5.38e6, 4.61e6},
+            {128, 128, 1, 4.41e6, 0.61, 5.30e6, 0.92, 3.56e6, 3.45e6}, {96, 128, 1, 3.71e6, 0.84, 4.12e6, 0.40, 0, 0},
             {64, 256, 1, 0, 0, 0, 0, 0, 2.4e6}, {64, 128, 1, 0, 0, 0, 0, 0, 2.0e6},
-            {32, 256, 1, 0, 0, 0, 0, 0, 1.4e6}, {32, 128, 1, 0, 0, 0, 0, 0, 1.3e6}, {64, 128, 2, 2.67e6, 0.12, 4.62e6, 0.27, 2.48e6, 0}};
+            {32, 256, 1, 0, 0, 0, 0, 0, 1.4e6}, {32, 128, 1, 0, 0, 0, 0, 0, 1.3e6}, {64, 128, 2, 2.67e6, 0.12, 5.29e6, 0.08, 2.48e6, 0}};
         const bool few = M <= 64, wide = keep && !few && N > K, kept = keep && !few && !wide;
-        // bytes a microsecond of all CUs together and of one alone (of kept sums the tiles' rates carry what the stream costs: no bound on all CUs
-        // together improves their fit)
-        const double HBM = few ? 7.72e6 : wide ? 8.18e6 : kept ? INFINITY : 9.41e6, CU_MAX = few ? 6.0e4 : wide ? 6.54e4 : kept ? 4.98e4 : 6.04e4;
+        // bytes a microsecond of all CUs together (as a bound it is high: what the stream costs beside MFMAs is in the tiles' rates) and of one alone
+        const double HBM = few ? 7.72e6 : wide ? 8.18e6 : kept ? 10.6e6 : 9.41e6, CU_MAX = few ? 6.0e4 : wide ? 6.54e4 : kept ? 4.98e4 : 6.04e4;
         GemmPlan best = {128, 128, 1};
         double best_t = 1e30;
         for (const Cand& c : cands) {
@@ -948,10 +949,11 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
                 const double plane_bytes = (double)M * N * 4.0;
                 if (S > (between ? 1 : 2) && kept && M > 2048 && S * plane_bytes > 32e6) break;
                 const double blocks = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * S;
-                const double rounds = ceil(blocks / (CUS * c.slots)), at_once = fmin(blocks, CUS * c.slots);
+                const double mine = ceil(blocks / S / 8.0) * S, xcd = CUS / 8.0;      // an XCD's blocks, and its CUs
+                const double rounds = ceil(mine / (xcd * c.slots)), at_once = fmin(blocks, CUS * c.slots);
                 double rate = kept ? c.rate_kept : c.rate, ends = kept ? c.ends_kept : c.ends, units = (nk + S - 1) / S;
                 double streams = ceil((double)N / c.bn) * S;              // (row tiles fetch a column tile's weight once between them)
-                double share = c.slots == 2 && blocks > CUS ? (kept ? 2.92 : 1.77) : 1.0;     // blocks that share a CU's MFMAs, and each other's waits
+                double share = c.slots == 2 && mine > xcd ? (kept ? 3.52 : 1.77) : 1.0;     // blocks that share a CU's MFMAs, and each other's waits
                 if (few || wide) {
                     rate = few ? c.rate_few : c.rate_wide;
                     ends = few ? 3.0 : 1.29 + 2.55 * (c.bm * c.bn / 65536.0);
@@ -965,7 +967,7 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
                 // the partial sums: written, read and added by a second kernel, or (kept) read by the
                 // consumer in place of one plane
                 // (from the caches as long as they are some 32 MB)
-                if (S > 1 && keep) t += (S - 1.0) * (plane_bytes / (few || (kept && S * plane_bytes <= 32e6) ? 4e6 : 1.97e6) + (kept ? 0.28 : 0.0));
+                if (S > 1 && keep) t += (S - 1.0) * (plane_bytes / (few || (kept && S * plane_bytes <= 32e6) ? 4e6 : kept ? 2.56e6 : 1.97e6) + (kept ? 0.3 : 0.0));
                 else if (S > 1 || unary) t += S * plane_bytes / (few ? 2.54e6 : 2.21e6) + (few ? 2.7 : glu ? 2.09 : 3.0);
                 if (between && M >= 1500) t *= 1.02;
                 if (t < best_t) { best_t = t; best = {c.bm, c.bn, S}; }
