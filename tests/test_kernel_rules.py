@@ -293,3 +293,16 @@ def test_parts_of_k_in_threes_fit_the_cus_of_every_xcd():
                     seen += 1
                     assert -(-tiles // 8) * parts <= 32, (M, N, K, rows, cols, parts)
     assert seen > 50
+
+
+def test_gated_products_of_some_hundred_rows_are_bound_by_their_weights_stream():
+    """A gated weight of 200 MB is bound by its stream: two parts of K do not make it faster, and cost their sums."""
+    for M in (65, 70, 139, 145, 160, 200):
+        assert _plan(M, 24576, 4096, 1)[2] == 1, M
+
+
+def test_an_activation_keeps_the_float32_sums_that_it_had():
+    """Products in more parts of K before an activation, which would be in one by the constants of products without: plans of their own."""
+    L = _lib()
+    for M, N, K in ((666, 9216, 5120), (1507, 3072, 2048), (523, 9920, 3840), (8651, 6080, 14912), (8941, 512, 2048)):
+        assert L.tff_gemm_takes_unary(M, N, K) == 1, (M, N, K)

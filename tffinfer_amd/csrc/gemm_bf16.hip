@@ -869,7 +869,8 @@ static bool few_rows_gated_on_tiles(int M, int N, int K) {
 
 // plane > 0: the columns of several products, so many each; a tile takes columns of one of them, and K is not split.
 // unary: an activation follows, in the kernel that adds up the parts, which one part then has as well (200 rows of 18,432 x 4,096, a squared relu: in
-// one part, as without it, 63 us, in two 54).
+// one part, as without it, 63 us, in two 54).  Where K is split the activation sees float32 sums: its constants stay as they were when the
+// others were fitted again, so that no size loses them.
 static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0, bool unary = false) {
     const double CUS = (double)tff_device_cus();
     // Up to 16 rows: the streaming kernel.  Not where the caller takes partial sums anyway, the groups of 16 columns go badly round the CUs and the
@@ -894,13 +895,15 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
         // XCDs 36 for 32 CUs, a second round (160 rows of 8,064 x 14,144 104 us, in four parts 69; 411 rows of 10,496 x 13,120, 82 tiles in three parts, 201,
         // in two 133).  Each round ends with the pipeline filled and the tile stored.  The constants are
         // fitted to products of the 0.6B to 14B shapes and of the other designs, every tile with
-        // 1 .. 8 parts timed on an MI355X (weights in turn that no cache holds, rows from five places), in four pieces:
-        // * Results of one kernel or of the sum over the parts, more than 64 rows: 4,234 products of 65 .. 16,500 rows.  The pick is 0.6 % from the best
-        //   candidate on average; against the tiles of 256, 128 and 64 rows alone 0.979 of the time (513 to 1,040 rows 0.949), and in 3 of 100 slower by
-        //   more than 2 %.
+        // 1 .. 8 parts timed on an MI355X (weights in turn that no cache holds, rows from five places), in five pieces:
+        // * Results of one kernel or of the sum over the parts, more than 64 rows: 4,347 products of 65 .. 16,500 rows.  The pick is 0.8 % from the best
+        //   candidate on average; against the tiles of 256, 128 and 64 rows alone 0.988 of the time (513 to 1,500 rows 0.967), and in 2 of 100 slower by
+        //   more than 3 % (in 4 of 100 with constants whose stream's bound was half as high again as a copy's rate: gated, 68 rows of 24,576 x 4,096
+        //   43.4 / 51.2 us, 145 rows 53.0 / 56.1).
         // * Sums kept for a norm, more than 64 rows, no more columns than K: 3,875 products of 65 .. 16,500 rows, each timed with the norm behind it: 1.0 % from
         //   the best, 0.972 of the time of the tiles of 256, 128 and 64 rows by their constants, in 2 of 100 slower by more than 3 %.  The norm reads the
         //   parts one after the other, 0.3 us each beside their bytes (116 rows of 2,048 x 2,048: four parts 10.9, eight 12.7).
+        // * Before an activation, more than 64 rows: an older fit of results (see above).
         // * Kept sums of more columns than K, which no model's product into its stream has: constants of an older fit.
         // * Up to 64 rows the four waves side by side take 64 or 32 rows: a product of so few rows is its
         //   weight's stream, and a block that does not work through 128 rows for 32 asks for its next
@@ -915,22 +918,24 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
         // (slower than the tiles before by more than 2 %: 4 of 100 such products without this margin, 0.3 with it).
         // Three and six parts are for kept sums of 129 to 1,024 rows: beyond, the parts' traffic grows and the rounds are many.  Beyond 2,048 rows kept parts that
         // are more than the caches hold are not cut further (but few columns are: 2,219 rows of 128 x 15,424 in eight parts 25.9, in two 48.6).
-        // The kernel that adds up results' parts costs 3.0 us beside its bytes, 2.1 where it also joins gate and up (68 rows of 4,096 x 1,024 in one part 7.4,
+        // The kernel that adds up results' parts costs 3.5 us beside its bytes, 2.3 where it also joins gate and up (68 rows of 4,096 x 1,024 in one part 7.4,
         // in four 9.9; 600 gated rows of 512 x 1,088 in two parts rather than one).
-        // A rate is in flops a microsecond of a CU; ends: us that a block's first fetch and storing its tile take.  Of results, of kept sums, of the older
-        // fit's, up to 64 rows.
-        struct Cand { int bm, bn, slots; double rate, ends, rate_kept, ends_kept, rate_wide, rate_few; };
+        // A rate is in flops a microsecond of a CU; ends: us that a block's first fetch and storing its tile take.  Of results, of kept sums, before an activation, of the
+        // older fit's, up to 64 rows.
+        struct Cand { int bm, bn, slots; double rate, ends, rate_kept, ends_kept, rate_act, ends_act, rate_wide, rate_few; };
         static const Cand cands[15] = {
-            {256, 256, 1, 8.43e6, 1.02, 8.16e6, 1.72, 6.45e6, 0}, {256, 192, 1, 7.65e6, 1.04, 7.76e6, 2.57, 6.10e6, 0},
-            {256, 128, 1, 6.20e6, 0.95, 6.86e6, 1.45, 5.42e6, 0}, {192, 256, 1, 7.80e6, 1.14, 7.70e6, 1.66, 0, 0},
-            {192, 192, 1, 5.90e6, 0.77, 5.95e6, 1.92, 0, 0}, {192, 128, 1, 4.70e6, 0.66, 5.27e6, 0.67, 0, 0},
-            {128, 384, 1, 10.6e6, 1.76, 7.05e6, 3.67, 6.49e6, 3.24e6}, {128, 256, 1, 6.18e6, 0.96, 7.00e6, 0.40, 5.38e6, 4.61e6},
-            {128, 128, 1, 4.41e6, 0.61, 5.30e6, 0.92, 3.56e6, 3.45e6}, {96, 128, 1, 3.71e6, 0.84, 4.12e6, 0.40, 0, 0},
-            {64, 256, 1, 0, 0, 0, 0, 0, 2.4e6}, {64, 128, 1, 0, 0, 0, 0, 0, 2.0e6},
-            {32, 256, 1, 0, 0, 0, 0, 0, 1.4e6}, {32, 128, 1, 0, 0, 0, 0, 0, 1.3e6}, {64, 128, 2, 2.67e6, 0.12, 5.29e6, 0.08, 2.48e6, 0}};
-        const bool few = M <= 64, wide = keep && !few && N > K, kept = keep && !few && !wide;
+            {256, 256, 1, 7.58e6, 0.93, 8.16e6, 1.72, 8.43e6, 1.02, 6.45e6, 0}, {256, 192, 1, 7.34e6, 1.07, 7.76e6, 2.57, 7.65e6, 1.04, 6.10e6, 0},
+            {256, 128, 1, 6.25e6, 1.10, 6.86e6, 1.45, 6.20e6, 0.95, 5.42e6, 0}, {192, 256, 1, 7.33e6, 0.85, 7.70e6, 1.66, 0, 0, 0, 0},
+            {192, 192, 1, 6.83e6, 1.61, 5.95e6, 1.92, 0, 0, 0, 0}, {192, 128, 1, 5.72e6, 0.48, 5.27e6, 0.67, 0, 0, 0, 0},
+            {128, 384, 1, 6.48e6, 0.98, 7.05e6, 3.67, 10.6e6, 1.76, 6.49e6, 3.24e6}, {128, 256, 1, 6.05e6, 1.38, 7.00e6, 0.40, 6.18e6, 0.96, 5.38e6, 4.61e6},
+            {128, 128, 1, 4.37e6, 0.64, 5.30e6, 0.92, 4.41e6, 0.61, 3.56e6, 3.45e6}, {96, 128, 1, 3.70e6, 1.01, 4.12e6, 0.40, 0, 0, 0, 0},
+            {64, 256, 1, 0, 0, 0, 0, 0, 0, 0, 2.4e6}, {64, 128, 1, 0, 0, 0, 0, 0, 0, 0, 2.0e6},
+            {32, 256, 1, 0, 0, 0, 0, 0, 0, 0, 1.4e6}, {32, 128, 1, 0, 0, 0, 0, 0, 0, 0, 1.3e6},
+            {64, 128, 2, 2.70e6, 0.15, 5.29e6, 0.08, 2.67e6, 0.12, 2.48e6, 0}};
+        const bool few = M <= 64, wide = keep && !few && N > K, kept = keep && !few && !wide, act = unary && !few;
         // bytes a microsecond of all CUs together (as a bound it is high: what the stream costs beside MFMAs is in the tiles' rates) and of one alone
-        const double HBM = few ? 7.72e6 : wide ? 8.18e6 : kept ? 10.6e6 : 9.41e6, CU_MAX = few ? 6.0e4 : wide ? 6.54e4 : kept ? 4.98e4 : 6.04e4;
+        const double HBM = few ? 7.72e6 : wide ? 8.18e6 : kept ? 10.6e6 : act ? 9.41e6 : 6.99e6;
+        const double CU_MAX = few ? 6.0e4 : wide ? 6.54e4 : act ? 6.04e4 : 4.98e4;
         GemmPlan best = {128, 128, 1};
         double best_t = 1e30;
         for (const Cand& c : cands) {
@@ -951,9 +956,9 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
                 const double blocks = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * S;
                 const double mine = ceil(blocks / S / 8.0) * S, xcd = CUS / 8.0;      // an XCD's blocks, and its CUs
                 const double rounds = ceil(mine / (xcd * c.slots)), at_once = fmin(blocks, CUS * c.slots);
-                double rate = kept ? c.rate_kept : c.rate, ends = kept ? c.ends_kept : c.ends, units = (nk + S - 1) / S;
+                double rate = kept ? c.rate_kept : act ? c.rate_act : c.rate, ends = kept ? c.ends_kept : act ? c.ends_act : c.ends, units = (nk + S - 1) / S;
                 double streams = ceil((double)N / c.bn) * S;              // (row tiles fetch a column tile's weight once between them)
-                double share = c.slots == 2 && mine > xcd ? (kept ? 3.52 : 1.77) : 1.0;     // blocks that share a CU's MFMAs, and each other's waits
+                double share = c.slots == 2 && mine > xcd ? (kept ? 3.52 : act ? 1.77 : 1.91) : 1.0;     // blocks that share a CU's MFMAs, and each other's waits
                 if (few || wide) {
                     rate = few ? c.rate_few : c.rate_wide;
                     ends = few ? 3.0 : 1.29 + 2.55 * (c.bm * c.bn / 65536.0);
@@ -968,7 +973,7 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
                 // consumer in place of one plane
                 // (from the caches as long as they are some 32 MB)
                 if (S > 1 && keep) t += (S - 1.0) * (plane_bytes / (few || (kept && S * plane_bytes <= 32e6) ? 4e6 : kept ? 2.56e6 : 1.97e6) + (kept ? 0.3 : 0.0));
-                else if (S > 1 || unary) t += S * plane_bytes / (few ? 2.54e6 : 2.21e6) + (few ? 2.7 : glu ? 2.09 : 3.0);
+                else if (S > 1 || unary) t += S * plane_bytes / (few ? 2.54e6 : act ? 2.21e6 : 2.2e6) + (few ? 2.7 : glu ? 2.28 : act ? 3.0 : 3.45);
                 if (between && M >= 1500) t *= 1.02;
                 if (t < best_t) { best_t = t; best = {c.bm, c.bn, S}; }
             }
