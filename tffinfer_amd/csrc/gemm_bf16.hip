@@ -915,7 +915,7 @@ static GemmPlan plan_for(int M, int N, int K, bool glu, bool keep, int plane = 0
         // gated 91 on 256 x 192, 101 on 192 x 256); up to 384 rows only where they pad less than tiles of 128, if
         // the sums are not kept; and beyond 2,048 rows K in one part (2,210 of 4,096 x 18,432 257 on 256 x 192, 335 on 192 x 128 in two).
         // From 1,500 rows on they have to be 2 % ahead: large products are bound by the power the card allows, of which a smaller tile's reads take more
-        // (slower than the tiles before by more than 2 %: 4 of 100 such products without this margin, 0.3 with it).
+        // (slower than the tiles before by more than 2 %: 2 of 100 such products without this margin, 0.7 with it).
         // Three and six parts are for kept sums of 129 to 1,024 rows: beyond, the parts' traffic grows and the rounds are many.  Beyond 2,048 rows kept parts that
         // are more than the caches hold are not cut further (but few columns are: 2,219 rows of 128 x 15,424 in eight parts 25.9, in two 48.6).
         // The kernel that adds up results' parts costs 3.5 us beside its bytes, 2.3 where it also joins gate and up (68 rows of 4,096 x 1,024 in one part 7.4,
